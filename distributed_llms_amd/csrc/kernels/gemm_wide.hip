@@ -192,21 +192,37 @@ constexpr int PFD = 2;
 template <int BM, int NBUF, int VAR, bool FP8 = false>
 __device__ __forceinline__ void wide_mainloop(bf16* smem, const bf16* const (&srcA)[BM / 64],
                                               const bf16* const (&srcB)[2], int nt, f32x4 (&acc)[BM / 64][4],
-                                              int wv, int lane, const bf16* pfB = nullptr, bf16* pf_lds = nullptr) {
+                                              int wv, int lane, const bf16* pfB = nullptr, bf16* pf_lds = nullptr,
+                                              int rot = 0) {
   constexpr int AEL = BM * WBK, BEL = WBN * WBK, BUF = AEL + BEL;
   constexpr bool PF = (VAR & 128) != 0;
   constexpr int AI = BM / 64, BI = 2, G0 = AI + BI, G = PF ? G0 + 1 : G0, RT = BM / 64;
+  const int wm = wv >> 1, wn = wv & 1;
+  // Rotated K order (VAR & 256): the K loop starts at K-tile `rot`, an eighth of K further on each XCD, and wraps.
+  // Workgroups that start together walk K in step, and their weight rows lie K * 2 bytes apart: at K = 4096 every
+  // line in flight then has the same low 13 address bits, which lands on a part of the memory channels only (the 8B
+  // gate|up, 224 workgroups: 45-51 us in most layers and 38 in the others, by where the weight was allocated).  Eight
+  // starts spread them, and the workgroups of one XCD still share the K-tile of A in its L2 (per-workgroup starts:
+  // 1-3 us slower).  8B gate|up, M = 1 / 64 / 128 / 256: 44.9 / 46.3 / 50.9 / 59.6 -> 36.5 / 39.7 / 45.3 / 56.4 us
+  // (6.4 TB/s at M = 1).
+  constexpr bool ROT = (VAR & 256) != 0;
+  auto kofs = [&](int t) {
+    if constexpr (ROT) {
+      t += rot;
+      t = t >= nt ? t - nt : t;
+    }
+    return t * WBK;
+  };
   // the L2 prefetch of the weight tile staged PFD slots after this one (clamped: counts stay static)
   auto prefetch = [&](int tile) {
     if constexpr (PF)
-      __builtin_amdgcn_global_load_lds((glb_vptr_w)(pfB + min(tile, nt - 1) * WBK), (lds_vptr_w)pf_lds, 4, 0, 0);
+      __builtin_amdgcn_global_load_lds((glb_vptr_w)(pfB + kofs(min(tile, nt - 1))), (lds_vptr_w)pf_lds, 4, 0, 0);
   };
-  const int wm = wv >> 1, wn = wv & 1;
   // cache policy of the staging loads (aux: 2 = nt): VAR 2 streams the weights nt, VAR 3 both operands
   constexpr int BAUX = (VAR & 7) >= 2 ? 2 : 0, AAUX = (VAR & 7) == 3 ? 2 : 0;
   auto stage = [&](int buf, int t) {
     bf16* base = smem + buf * BUF;
-    const int ko = t * WBK;
+    const int ko = kofs(t);
 #pragma unroll
     for (int j = 0; j < AI; ++j)
       __builtin_amdgcn_global_load_lds((glb_vptr_w)(srcA[j] + ko), (lds_vptr_w)(base + (wv * AI + j) * 512), 16, 0,
@@ -403,14 +419,14 @@ __device__ __forceinline__ void wide_mainloop(bf16* smem, const bf16* const (&sr
       // this barrier: refill it with tile t + NBUF - 1
       const int nb = cur == 0 ? NBUF - 1 : cur - 1;
       if constexpr (FP8) {
-        ktile8(cur, smem + nb * BUF, (t + NBUF - 1) * WBK, std::true_type{});
+        ktile8(cur, smem + nb * BUF, kofs(t + NBUF - 1), std::true_type{});
       } else if constexpr (SPLITRD) {
-        ktile_sr(cur, smem + nb * BUF, (t + NBUF - 1) * WBK, std::true_type{});
+        ktile_sr(cur, smem + nb * BUF, kofs(t + NBUF - 1), std::true_type{});
       } else if constexpr ((VAR & 7) == 0) {
         stage(nb, t + NBUF - 1);
         ktile(cur, smem, 0, std::false_type{});
       } else {
-        ktile(cur, smem + nb * BUF, (t + NBUF - 1) * WBK, std::true_type{});
+        ktile(cur, smem + nb * BUF, kofs(t + NBUF - 1), std::true_type{});
       }
       cur = cur == NBUF - 1 ? 0 : cur + 1;
     }
@@ -460,9 +476,7 @@ __global__ void __launch_bounds__(512, 1) gemm_wide_kernel(const bf16* __restric
   }
   const int m0 = m_t * BM;
   const int kt0 = split * kt_per_split;
-  // ablations (timing only, wrong results): VAR & 16 skips the K loop (launch + epilogue cost),
-  // VAR & 8 skips the epilogue stores (kept behind a never-true runtime test so the MFMAs stay)
-  const int nt = (VAR & 16) ? 0 : max(0, min(K / WBK, kt0 + kt_per_split) - kt0);
+  const int nt = max(0, min(K / WBK, kt0 + kt_per_split) - kt0);
 
   // per-lane staging sources: instruction i covers tile rows 8i .. 8i+7, lane -> (row, chunk)
   const bf16* srcA[AI];
@@ -482,8 +496,7 @@ __global__ void __launch_bounds__(512, 1) gemm_wide_kernel(const bf16* __restric
   // PF: lanes l and l + 16k of wave w touch weight row 16 w + (l & 15) of the tile: 128 lines per K-tile
   const bf16* pfB = B + (size_t)wide_b_row<SWIGLU>(16 * wv + (lane & 15), n_t, N / 2) * K + (size_t)kt0 * WBK;
   f32x4 acc[RT][4];
-  wide_mainloop<BM, NBUF, VAR>(smem, srcA, srcB, nt, acc, wv, lane, pfB, smem + NBUF * BUF);
-  if (VAR & 8) return;
+  wide_mainloop<BM, NBUF, VAR>(smem, srcA, srcB, nt, acc, wv, lane, pfB, smem + NBUF * BUF, ((int)(blockIdx.x & 7) * nt) >> 3);
   wide_epilogue<BM, SPLIT, SWIGLU>(acc, C, P, M, N, m0, n_t, split, wm, wn, lane);
 }
 
@@ -535,7 +548,7 @@ __global__ void __launch_bounds__(512, 1) gemm_wide_fp8_kernel(const uint8_t* __
     srcB[j] = B + (size_t)wide_b_row<SWIGLU>(r, n_t, N / 2) * KU + (size_t)kt0 * WBK + wswz(r, lane & 7) * 8;
   }
   f32x4 acc[RT][4];
-  wide_mainloop<BM, NBUF, VAR, true>(smem, srcA, srcB, nt, acc, wv, lane);
+  wide_mainloop<BM, NBUF, VAR, true>(smem, srcA, srcB, nt, acc, wv, lane, nullptr, nullptr, ((int)(blockIdx.x & 7) * nt) >> 3);
   wide_epilogue<BM, SPLIT, SWIGLU, true>(acc, C, P, M, N, m0, n_t, split, wm, wn, lane, sa, sb);
 }
 
@@ -716,31 +729,39 @@ int gemm_wide(uintptr_t c, uintptr_t a, uintptr_t b, uintptr_t ws, long ws_float
   if (S > 1) DLLM_HOST_CHECK(ws != 0 && (long)S * M * N <= ws_floats, "split-K workspace too small");
 
   // weights nt (variant 2) where the grid has no K split: -3..-5 % on the MLP up projection from
-  // cold caches; on the split-K grids nt costs up to +25 % at M = 128 (profiles/wide_gemm.md)
-  // (variant 4 = variant 1 everywhere, for A/B runs)
-  // variant | 32: per-row fragment waits (SPLITRD in wide_mainloop; the engine default);
-  // ablations (A/B timing only): variant | 8 = no epilogue stores, | 16 = no K loop
-  const int abl = variant & 56;
+  // cold caches; variant 4 = variant 1 (default cache policy) everywhere
+  // variant | 32: per-row fragment waits (SPLITRD in wide_mainloop; the engine default)
+  const bool frag = (variant & 32) != 0;
   const bool grp = (variant & 64) != 0 && S == 1;   // grouped row-tile order (large M)
   const bool pf = (variant & 128) != 0;            // L2 prefetch of the weight tile (wide_mainloop PF)
   variant &= 7;
   if (variant == 1 && S == 1) variant = grp ? 1 : 2;
   else if (variant == 4) variant = 1;
-#define DLLM_WIDE_GO3(BM_, SPLIT_, SW_, V_)                                                                      \
-  hipLaunchKernelGGL((gemm_wide_kernel<BM_, SPLIT_, SW_, 3, V_>), dim3((unsigned)grid), dim3(512), 0, s,          \
+  const bool rot = S == 1 && variant == 2;         // rotated K order (wide_mainloop)
+#define DLLM_WIDE_GO3(BM_, SPLIT_, SW_, V_, NB_)                                                                \
+  hipLaunchKernelGGL((gemm_wide_kernel<BM_, SPLIT_, SW_, NB_, V_>), dim3((unsigned)grid), dim3(512), 0, s,       \
                      (const bf16*)a, (const bf16*)b, (bf16*)c, (float*)ws, M, N, K, kts, S)
-#define DLLM_WIDE_GO(BM_, SPLIT_, SW_)                                                                          \
+#define DLLM_WIDE_GO(BM_, SPLIT_, SW_)                                                                         \
   do {                                                                                                         \
-    if (abl == 8) { if (variant == 2) DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 10); else DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 9); } \
-    else if (abl == 16) { if (variant == 2) DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 18); else DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 17); } \
-    else if (pf && abl == 32) { if (variant == 2) DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 162); else DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 161); } \
-    else if (pf) { if (variant == 2) DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 130); else DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 129); } \
-    else if (abl == 32) { if (variant == 2) DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 34); else DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 33); } \
-    else if (grp && !SPLIT_) DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 65);                                              \
-    else if (variant == 0) DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 0);                                                 \
-    else if (variant == 2) DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 2);                                                 \
-    else if (variant == 3) DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 3);                                                 \
-    else DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 1);                                                                   \
+    if (grp && !SPLIT_) DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 65, 3);                                                \
+    else if (rot && !SPLIT_) DLLM_WIDE_ROT(BM_, SW_);                                                          \
+    else if (pf && frag) { if (variant == 2) DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 162, 3); else DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 161, 3); } \
+    else if (pf) { if (variant == 2) DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 130, 3); else DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 129, 3); } \
+    else if (frag) { if (variant == 2) DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 34, 3); else DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 33, 3); } \
+    else if (variant == 0) DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 0, 3);                                              \
+    else if (variant == 2) DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 2, 3);                                              \
+    else if (variant == 3) DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 3, 3);                                              \
+    else DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 1, 3);                                                                \
+  } while (0)
+  // BM = 64 and a grid of one round: the ring as deep as the LDS allows (6 x 24 KiB, five K-tiles in flight: 38.5 vs
+  // 40.0 us for the 8B gate|up at M = 64, 36.5 vs 36.8 at M = 1); with more workgroups than CUs two 3-slot
+  // workgroups per CU are as good, and from 128 rows on the MFMAs hide what the depth would
+#define DLLM_WIDE_ROT(BM_, SW_)                                                                                \
+  do {                                                                                                         \
+    if (BM_ == 64 && grid <= 256 && !pf) { if (frag) DLLM_WIDE_GO3(BM_, false, SW_, 256 + 34, (BM_ == 64 ? 6 : 3)); else DLLM_WIDE_GO3(BM_, false, SW_, 256 + 2, (BM_ == 64 ? 6 : 3)); } \
+    else if (pf) { if (frag) DLLM_WIDE_GO3(BM_, false, SW_, 256 + 162, 3); else DLLM_WIDE_GO3(BM_, false, SW_, 256 + 130, 3); } \
+    else if (frag) DLLM_WIDE_GO3(BM_, false, SW_, 256 + 34, 3);                                                \
+    else DLLM_WIDE_GO3(BM_, false, SW_, 256 + 2, 3);                                                           \
   } while (0)
   if (S == 1) {
     if (BM == 64) { if (swiglu) DLLM_WIDE_GO(64, false, true); else DLLM_WIDE_GO(64, false, false); }
@@ -754,6 +775,7 @@ int gemm_wide(uintptr_t c, uintptr_t a, uintptr_t b, uintptr_t ws, long ws_float
   else if (BM == 128) { if (swiglu) DLLM_WIDE_GO(128, true, true); else DLLM_WIDE_GO(128, true, false); }
   else if (BM == 192) { if (swiglu) DLLM_WIDE_GO(192, true, true); else DLLM_WIDE_GO(192, true, false); }
   else { if (swiglu) DLLM_WIDE_GO(256, true, true); else DLLM_WIDE_GO(256, true, false); }
+#undef DLLM_WIDE_ROT
 #undef DLLM_WIDE_GO
 #undef DLLM_WIDE_GO3
   DLLM_HIP_CHECK(hipGetLastError());
@@ -791,13 +813,15 @@ int gemm_wide_fp8(uintptr_t c, uintptr_t a, uintptr_t a_scale, uintptr_t b, uint
   // row-tile order for large M (no K split)
   const bool nt = (variant & 7) != 4 && S == 1;
   const bool grp = (variant & 64) != 0 && S == 1 && !nt;
+  const bool rot = nt;                             // rotated K order, as in gemm_wide
 #define DLLM_F8_GO3(BM_, SPLIT_, SW_, V_)                                                                   \
   hipLaunchKernelGGL((gemm_wide_fp8_kernel<BM_, SPLIT_, SW_, 3, V_>), dim3((unsigned)grid), dim3(512), 0, s,  \
                      (const uint8_t*)a, (const uint8_t*)b, (const float*)a_scale, (const float*)b_scale,      \
                      (bf16*)c, (float*)ws, M, N, K, kts, S)
 #define DLLM_F8_GO(BM_, SPLIT_, SW_)                                   \
   do {                                                                \
-    if (nt) DLLM_F8_GO3(BM_, SPLIT_, SW_, 2);                          \
+    if (rot && !SPLIT_) DLLM_F8_GO3(BM_, SPLIT_, SW_, 256 + 2);         \
+    else if (nt) DLLM_F8_GO3(BM_, SPLIT_, SW_, 2);                     \
     else if (grp && !SPLIT_) DLLM_F8_GO3(BM_, SPLIT_, SW_, 65);          \
     else DLLM_F8_GO3(BM_, SPLIT_, SW_, 1);                              \
   } while (0)

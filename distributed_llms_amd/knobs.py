@@ -32,9 +32,11 @@ class Knobs:
     # comma list of roles gate_up / down / proj
     wide: str = "auto"
     # gemm_wide variant for unsplit grids (33: LDS-DMA interleaved + asm fragment reads with one
-    # lgkmcnt per MFMA row) and for split-K grids (1); in-engine A/B 27,123 vs 27,014 / 26,896 tok/s
+    # lgkmcnt per MFMA row) and for split-K grids (2: weights nontemporal, each byte is read once per
+    # launch: 8B down 21.7 -> 19.6 us at M = 1, 23.2 -> 21.6 at 64, 34.1 -> 33.4 at 256; qkv 10.9 -> 10.1
+    # at M = 1, 17.8 -> 17.4 at 256; o 8.1 -> 7.7, 15.1 -> 14.6)
     wide_variant: int = 33
-    wide_variant_split: int = 1
+    wide_variant_split: int = 2
     wide_gate_up_max_m: int = 256     # SwiGLU-fused gate|up on gemm_wide up to this M (then split-K gemm_pp / gemm_pf)
     wide_down_max_m: int = 384        # MLP down (K >= 8192, K > N) up to this M (512: split gemm_pp 59 vs 66 us)
     wide_proj_max_m: int = 256        # qkv / LM head up to this M (o: wide_o_max_m; down: wide_down_max_m)

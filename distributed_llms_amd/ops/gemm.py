@@ -236,6 +236,9 @@ def wide_splits(m: int, n: int, k: int, swiglu: bool = False, target_wgs: int = 
     return max(1, min(s, (k // 64) // 8, 16))
 
 
+WIDE_NT_MIN_BYTES = 12 << 20
+
+
 def linear_wide(x: torch.Tensor, w: torch.Tensor, splits: int = 0, swiglu: bool = False, defer: bool = False,
                 variant: int = -1):
     """Wide-M decode GEMM (csrc/kernels/gemm_wide.hip): 256 x 128 x 64 tiles, 3-deep LDS-DMA pipeline,
@@ -255,8 +258,13 @@ def linear_wide(x: torch.Tensor, w: torch.Tensor, splits: int = 0, swiglu: bool 
     if s > 1 and s * m * n > ws.numel():
         s = max(1, ws.numel() // (m * n))
     stream = torch.cuda.current_stream().cuda_stream
-    v = (knobs.K.wide_variant_split if s > 1 else knobs.K.wide_variant) if variant < 0 else variant
     bm = wide_row_tile(m, n, k, swiglu)
+    v = variant if variant >= 0 else knobs.K.wide_variant
+    if s > 1 and variant < 0:
+        # split grids: weights nontemporal where each byte is read from memory once per step -- not below
+        # WIDE_NT_MIN_BYTES (a small model's weights stay in the 256 MiB Infinity Cache from step to step: 1024 x 1024
+        # 5.0 -> 5.9 us with nt), and not on 192-row tiles (8B down at M = 192: 32.0 -> 34.0 us)
+        v = knobs.K.wide_variant_split if n * k * 2 >= WIDE_NT_MIN_BYTES and bm != 192 else 1
     if bm != wide_bm(m):
         v |= bm << 8
     if defer and not swiglu and s > 1:

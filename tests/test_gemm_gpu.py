@@ -142,6 +142,27 @@ def test_wide_l2_prefetch_bit_exact(cuda, m, n, k, splits, swiglu):
         assert torch.equal(a, b), v
 
 
+@pytest.mark.parametrize("m", [1, 64, 65, 256])
+@pytest.mark.parametrize("n,k,swiglu", [(128, 64, False), (256, 192, True), (1152, 320, False), (2176, 448, True),
+                                        (33024, 576, False), (28672, 4096, True)])
+def test_wide_rotated_k_order(cuda, m, n, k, swiglu):
+    """The rotated K order of unsplit grids (start (b % 8) nt / 8, wrapping) at fewer K-tiles than XCDs, than ring
+    slots (6 at 64 rows) and just past both, grids below and above one round of CUs: equal to the same kernel in plain
+    order (variant 4) within what another order of an f32 sum of k products of size |x||w| can change (k 2^-24 of the
+    sum of their magnitudes), plus one bf16 rounding."""
+    x, w = _bf(m, k), _bf(n, k, scale=0.05)
+    a = gemm.linear_wide(x, w, splits=1, swiglu=swiglu, variant=33).float()
+    b = gemm.linear_wide(x, w, splits=1, swiglu=swiglu, variant=4 | 32).float()
+    mag = x.float().abs() @ w.float().abs().t()
+    if swiglu:
+        g, u = mag.chunk(2, -1)
+        # silu(g) u: both factors carry the error of their sums (|silu'| <= 1.1)
+        tol = 2.2 * k * 2.0 ** -24 * g * u
+    else:
+        tol = 2 * k * 2.0 ** -24 * mag
+    assert bool(((a - b).abs() <= tol + 2.0 ** -7 * b.abs() + 1e-30).all())
+
+
 @pytest.mark.parametrize("m,n,k,swiglu", [(4500, 1024, 512, False), (5000, 2048, 256, True), (2048, 256, 128, False)])
 def test_wide_grouped_tile_order_bit_exact(cuda, m, n, k, swiglu):
     """Variant bit 64 (grouped row-tile order for prefill M) only reorders the workgroups: every
