@@ -189,6 +189,8 @@ __device__ __forceinline__ void wide_epilogue(const f32x4 (&acc)[BM / 64][4], bf
 // then in the XCD's L2 when their staging pieces go out, so a tile waits for an L2 hit instead of
 // an HBM round trip.  One more vm op per slot (counted waits use G + 1); results are unchanged.
 constexpr int PFD = 2;
+__device__ __forceinline__ int wide_rot(int xcd, int nt) { return nt >= 16 ? (xcd * nt) >> 3 : 0; }
+
 template <int BM, int NBUF, int VAR, bool FP8 = false>
 __device__ __forceinline__ void wide_mainloop(bf16* smem, const bf16* const (&srcA)[BM / 64],
                                               const bf16* const (&srcB)[2], int nt, f32x4 (&acc)[BM / 64][4],
@@ -204,7 +206,7 @@ __device__ __forceinline__ void wide_mainloop(bf16* smem, const bf16* const (&sr
   // gate|up, 224 workgroups: 45-51 us in most layers and 38 in the others, by where the weight was allocated).  Eight
   // starts spread them, and the workgroups of one XCD still share the K-tile of A in its L2 (per-workgroup starts:
   // 1-3 us slower).  8B gate|up, M = 1 / 64 / 128 / 256: 44.9 / 46.3 / 50.9 / 59.6 -> 36.5 / 39.7 / 45.3 / 56.4 us
-  // (6.4 TB/s at M = 1).
+  // (6.4 TB/s at M = 1).  Below 16 K-tiles the loop is over before the channels matter: plain order (wide_rot).
   constexpr bool ROT = (VAR & 256) != 0;
   auto kofs = [&](int t) {
     if constexpr (ROT) {
@@ -496,7 +498,7 @@ __global__ void __launch_bounds__(512, 1) gemm_wide_kernel(const bf16* __restric
   // PF: lanes l and l + 16k of wave w touch weight row 16 w + (l & 15) of the tile: 128 lines per K-tile
   const bf16* pfB = B + (size_t)wide_b_row<SWIGLU>(16 * wv + (lane & 15), n_t, N / 2) * K + (size_t)kt0 * WBK;
   f32x4 acc[RT][4];
-  wide_mainloop<BM, NBUF, VAR>(smem, srcA, srcB, nt, acc, wv, lane, pfB, smem + NBUF * BUF, ((int)(blockIdx.x & 7) * nt) >> 3);
+  wide_mainloop<BM, NBUF, VAR>(smem, srcA, srcB, nt, acc, wv, lane, pfB, smem + NBUF * BUF, wide_rot((int)(blockIdx.x & 7), nt));
   wide_epilogue<BM, SPLIT, SWIGLU>(acc, C, P, M, N, m0, n_t, split, wm, wn, lane);
 }
 
@@ -548,7 +550,7 @@ __global__ void __launch_bounds__(512, 1) gemm_wide_fp8_kernel(const uint8_t* __
     srcB[j] = B + (size_t)wide_b_row<SWIGLU>(r, n_t, N / 2) * KU + (size_t)kt0 * WBK + wswz(r, lane & 7) * 8;
   }
   f32x4 acc[RT][4];
-  wide_mainloop<BM, NBUF, VAR, true>(smem, srcA, srcB, nt, acc, wv, lane, nullptr, nullptr, ((int)(blockIdx.x & 7) * nt) >> 3);
+  wide_mainloop<BM, NBUF, VAR, true>(smem, srcA, srcB, nt, acc, wv, lane, nullptr, nullptr, wide_rot((int)(blockIdx.x & 7), nt));
   wide_epilogue<BM, SPLIT, SWIGLU, true>(acc, C, P, M, N, m0, n_t, split, wm, wn, lane, sa, sb);
 }
 
@@ -593,7 +595,7 @@ __device__ __forceinline__ void moe_wide_rows(bf16* smem, bf16* __restrict__ Y, 
     // nontemporal weights: rotated K order (wide_mainloop), 16 Mixtral rows: gate|up 300.9 -> 277.3 us, down 148.4 ->
     // 138.3 (6.8 TB/s)
     const int nt = KU / WBK, xcd = (int)((blockIdx.y * gridDim.x + blockIdx.x) & 7);
-    wide_mainloop<BM, NBUF, VAR, FP8>(smem, srcA, srcB, nt, acc, wv, lane, nullptr, nullptr, (xcd * nt) >> 3);
+    wide_mainloop<BM, NBUF, VAR, FP8>(smem, srcA, srcB, nt, acc, wv, lane, nullptr, nullptr, wide_rot(xcd, nt));
     wide_epilogue<BM, false, SWIGLU, FP8, CLIPPED>(acc, Y + (size_t)(off + r0) * ldy, nullptr, rows, N, 0, n_t, 0, wm, wn,
                                           lane, FP8 ? sa + off + r0 : nullptr, sb, limit);
     __syncthreads();   // the next chunk's prologue refills buffers other waves may still read

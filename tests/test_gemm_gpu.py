@@ -144,10 +144,11 @@ def test_wide_l2_prefetch_bit_exact(cuda, m, n, k, splits, swiglu):
 
 @pytest.mark.parametrize("m", [1, 64, 65, 256])
 @pytest.mark.parametrize("n,k,swiglu", [(128, 64, False), (256, 192, True), (1152, 320, False), (2176, 448, True),
-                                        (33024, 576, False), (28672, 4096, True)])
+                                        (33024, 576, False), (256, 1024, True),
+                                        (2176, 1088, False), (28672, 4096, True)])
 def test_wide_rotated_k_order(cuda, m, n, k, swiglu):
-    """The rotated K order of unsplit grids (start (b % 8) nt / 8, wrapping) at fewer K-tiles than XCDs, than ring
-    slots (6 at 64 rows) and just past both, grids below and above one round of CUs: equal to the same kernel in plain
+    """The rotated K order of unsplit grids (start (b % 8) nt / 8, wrapping) from 16 K-tiles on, at fewer K-tiles than
+    that, than XCDs and than ring slots (6 at 64 rows) and just past it, grids below and above one round of CUs: equal to the same kernel in plain
     order (variant 4) within what another order of an f32 sum of k products of size |x||w| can change (k 2^-24 of the
     sum of their magnitudes), plus one bf16 rounding."""
     x, w = _bf(m, k), _bf(n, k, scale=0.05)
