@@ -1,0 +1,214 @@
+// Weight-streaming GEMM for decode batches of up to 64 rows: y[M, N] = x[M, K] . w[N, K]^T, bf16 in, f32 sums, with
+// the bias, the SiLU, clipped or gelu GLU in the epilogue -- one launch where the wide kernel's K-split grid needs a
+// second one to sum its slabs and (behind a bias) a third for the activation.
+//
+// At these sizes a projection of a 1k-4k wide model is a few microseconds of weight bytes, and every further launch
+// costs about 4.6 us (the end of one kernel to the start of the next inside a graph, plus its first load's round trip).
+//
+//  * one workgroup owns RT x 16 weight rows and all of K, so nothing is left to sum in memory; its waves take the
+//    64-deep K-tiles in turn (wave v: tiles v, v + WAVES, ...), so that together they read 512-byte or 1 KiB runs of
+//    every row;
+//  * a wave stages its tiles -- weights and x -- through an LDS ring of its OWN (D slots, global_load_lds_dwordx4 in
+//    whole 128-byte lines, the chunk swizzle c ^ ((row >> 1) & 7) on the source address and on the read): no barrier
+//    in the K loop, the only waits are the wave's counted vmcnt.  x fragments straight from global memory touch 16
+//    half lines per load and took 1.3-2x as long at 16-64 rows (2560 x 2560: 8.1 / 12.4 / 19.2 us at M = 16 / 32 / 64
+//    against 5.9 / 7.4 / 9.7);
+//  * the waves' sums meet in LDS (wave 0 first: the same result on every run), behind the only two barriers.
+// Measured, cold weights, M = 1 / 16 / 32 / 64, us (wide: gemm_wide's K split, without the reduction behind it):
+//   1024 x 1024  3.0 / 3.4 / 4.0 / 5.1 (wide 5.0 / 5.4 / 5.5 / 5.6)    2560 x 2560  4.7 / 5.9 / 7.4 / 9.7 (6.7 / 7.2 / 7.7 / 8.2)
+//   5120 x 2560  7.0 / 8.2 / 9.7 / 12.5 (7.9 / 8.5 / 9.0 / 9.6)        15360 x 2560 + GLU  14.2 / 14.7 / 16.2 / 19.7 (15.8 / 16.5 / 17.5 / 18.5)
+//   4096 x 4096  7.7 / 8.6 / 10.0 / 13.2 (7.8 / 8.1 / 8.5 / 8.9)       2560 x 7680  9.1 / 12.8 / 16.6 / 22.4 (9.3 / 9.6 / 10.1 / 10.6)
+// bound by the weight bytes and the launch below 16 rows, by staging x once per workgroup above.
+#include "common.h"
+#include "launchers.h"
+
+namespace dllm {
+
+namespace {
+typedef __attribute__((address_space(3))) void* lds_vptr_s;
+typedef __attribute__((address_space(1))) void* glb_vptr_s;
+constexpr int SK = 64;                    // K-tile
+
+__device__ __forceinline__ int sswz(int row, int chunk) { return chunk ^ ((row >> 1) & 7); }
+}  // namespace
+
+// GLU 0: y [M, N] (+ bias [N]);  1 / 2 / 3: SiLU / clipped (`limit`) / gelu GLU, w = [gate; up], y [M, N / 2], bias
+// gate | up.  GLU tiles hold RT / 2 16-row tiles of gate rows, then the same output columns' up rows.
+template <int RT, int MT, int D, int GLU, bool NT, int WAVES>
+__global__ void __launch_bounds__(WAVES * 64) gemm_stream_kernel(bf16* __restrict__ Y, const bf16* __restrict__ X,
+                                                                 const bf16* __restrict__ W,
+                                                                 const bf16* __restrict__ bias, int M, int N, int K,
+                                                                 float limit) {
+  static_assert(GLU == 0 || RT % 2 == 0, "gate and up tiles come in pairs");
+  constexpr int SLOT = (RT + MT) * 16 * SK;                     // bf16 elements of one ring slot: weights, then x
+  constexpr int G = 2 * (RT + MT);                              // loads per K-tile
+  constexpr int RING = WAVES * D * SLOT * 2, RED = WAVES * RT * MT * 1024;
+  static_assert((D - 1) * G <= 63, "vmcnt");
+  __shared__ __attribute__((aligned(16))) char smem[RING > RED ? RING : RED];
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int fr = lane & 15, fq = lane >> 4;
+  const int half = N / 2, ncols = GLU ? half : N;
+  constexpr int CT = GLU ? RT / 2 : RT;                         // 16-column tiles of the output
+  const int c0 = blockIdx.x * (CT * 16);
+  bf16* ring = reinterpret_cast<bf16*>(smem) + wv * (D * SLOT);
+
+  // weight row of tile row r (0..15) of 16-row tile t; rows past the matrix repeat its last row
+  auto wrow = [&](int t, int r) {
+    const int c = min(c0 + (t % CT) * 16 + r, ncols - 1);
+    return GLU && t >= CT ? half + c : c;
+  };
+  const bf16* src[RT + MT][2];
+#pragma unroll
+  for (int t = 0; t < RT + MT; ++t)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int r = 8 * j + (lane >> 3);
+      const bf16* row = t < RT ? W + (size_t)wrow(t, r) * K : X + (size_t)min((t - RT) * 16 + r, M - 1) * K;
+      src[t][j] = row + wv * SK + sswz(r, lane & 7) * 8;
+    }
+  const int nk = K / SK, cnt = (nk - wv + WAVES - 1) / WAVES;     // this wave's K-tiles (0 for a short K)
+  f32x4 acc[RT][MT];
+#pragma unroll
+  for (int t = 0; t < RT; ++t)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  auto load = [&](int slot, int i) {
+    const int ko = i * (WAVES * SK);
+#pragma unroll
+    for (int q = 0; q < 2 * RT; ++q)
+      __builtin_amdgcn_global_load_lds((glb_vptr_s)(src[q / 2][q & 1] + ko), (lds_vptr_s)(ring + slot * SLOT + q * 512), 16,
+                                       0, NT ? 2 : 0);
+#pragma unroll
+    for (int q = 2 * RT; q < G; ++q)
+      __builtin_amdgcn_global_load_lds((glb_vptr_s)(src[q / 2][q & 1] + ko), (lds_vptr_s)(ring + slot * SLOT + q * 512), 16,
+                                       0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+#pragma unroll
+  for (int u = 0; u < D; ++u)
+    if (u < cnt) load(u, u);
+  for (int i0 = 0; i0 < cnt; i0 += D) {
+#pragma unroll
+    for (int u = 0; u < D; ++u) {
+      const int i = i0 + u;                                       // wave-uniform
+      if (i < cnt) {
+        // tile i has landed when only the younger tiles' loads are left: min(D - 1, cnt - 1 - i) of them
+        if (D > 1 && cnt - 1 - i >= D - 1) asm volatile("s_waitcnt vmcnt(%0)" ::"i"((D - 1) * G) : "memory");
+        else if (D > 2 && cnt - 1 - i == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(D > 2 ? G : 0) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        const bf16* b = ring + u * SLOT;
+        bf16x8 wa[RT][2], xa[MT][2];
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+#pragma unroll
+          for (int t = 0; t < RT; ++t)
+            wa[t][s] = *reinterpret_cast<const bf16x8*>(b + t * 1024 + fr * SK + sswz(fr, 4 * s + fq) * 8);
+#pragma unroll
+          for (int m = 0; m < MT; ++m)
+            xa[m][s] = *reinterpret_cast<const bf16x8*>(b + (RT + m) * 1024 + fr * SK + sswz(fr, 4 * s + fq) * 8);
+        }
+        // every fragment of the slot is in registers before its refill goes out
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        if (i + D < cnt) load(u, i + D);
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+          for (int t = 0; t < RT; ++t)
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+              acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[t][s], xa[m][s], acc[t][m], 0, 0, 0);
+      }
+    }
+  }
+  __syncthreads();
+  // acc[t][m]: lane holds weight rows 4 fq + v of tile t, x row m 16 + fr
+  f32x4* red = reinterpret_cast<f32x4*>(smem);
+#pragma unroll
+  for (int t = 0; t < RT; ++t)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) red[(wv * RT * MT + t * MT + m) * 64 + lane] = acc[t][m];
+  __syncthreads();
+  for (int e = tid; e < CT * MT * 64; e += WAVES * 64) {
+    const int tile = e >> 6, ln = e & 63, t = tile / MT, m = tile % MT;
+    f32x4 a = red[(t * MT + m) * 64 + ln], b = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) a += red[(w * RT * MT + t * MT + m) * 64 + ln];
+    if constexpr (GLU != 0) {
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) b += red[(w * RT * MT + (t + CT) * MT + m) * 64 + ln];
+    }
+    const int row = m * 16 + (ln & 15), c = c0 + t * 16 + 4 * (ln >> 4);
+    if (row >= M || c >= ncols) continue;
+    bf16x4 o;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int cc = min(c + v, ncols - 1);
+      float z = a[v] + (bias ? bf2f(bias[cc]) : 0.f);
+      if constexpr (GLU != 0) {
+        const float up = b[v] + (bias ? bf2f(bias[half + cc]) : 0.f);
+        z = GLU == 1 ? silu_f(z) * up : GLU == 2 ? clipped_glu_f(z, up, limit) : gelu_glu_f(z, up);
+      }
+      o[v] = f2bf(z);
+    }
+    bf16* dst = Y + (size_t)row * ncols + c;
+    if (c + 4 <= ncols && ncols % 4 == 0) {
+      *reinterpret_cast<bf16x4*>(dst) = o;
+    } else {
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        if (c + v < ncols) dst[v] = o[v];
+    }
+  }
+}
+
+// glu 0: y [M, N] = x w^T (+ bias);  1 / 2 / 3: y [M, N / 2], SiLU / clipped / gelu GLU of w = [gate; up] (+ bias).
+// nt: nontemporal weight loads.
+void gemm_stream(uintptr_t y, uintptr_t x, uintptr_t w, uintptr_t bias, int M, int N, int K, int glu, int nt, float limit,
+                 uintptr_t stream) {
+  DLLM_HOST_CHECK(M >= 1 && M <= 64, "1 <= M <= 64");
+  DLLM_HOST_CHECK(K >= SK && K % SK == 0, "K must be a positive multiple of 64");
+  DLLM_HOST_CHECK(glu >= 0 && glu <= 3, "glu 0..3");
+  DLLM_HOST_CHECK(N >= 1 && (glu == 0 || N % 2 == 0), "N");
+  DLLM_HOST_CHECK(x % 16 == 0 && w % 16 == 0 && y % 8 == 0, "operand alignment");
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  const int ncols = glu ? N / 2 : N;
+  // twice the weight rows per workgroup (half the x staging) once that still leaves a workgroup for most CUs
+  const bool two = (ncols + 15) / 16 > 256;
+  const int per = two ? 32 : 16;
+  const dim3 grid((ncols + per - 1) / per);
+  // single 16-row tiles: 8 waves, the K loop of a small weight is over in one or two rounds; else 4 (several
+  // workgroups per CU)
+#define DLLM_ST_GO(RT_, MT_, GLU_, WV_)                                                                              \
+  do {                                                                                                              \
+    if (nt) hipLaunchKernelGGL((gemm_stream_kernel<RT_, MT_, 2, GLU_, true, WV_>), grid, dim3(WV_ * 64), 0, s,         \
+                               (bf16*)y, (const bf16*)x, (const bf16*)w, (const bf16*)bias, M, N, K, limit);          \
+    else hipLaunchKernelGGL((gemm_stream_kernel<RT_, MT_, 2, GLU_, false, WV_>), grid, dim3(WV_ * 64), 0, s,           \
+                            (bf16*)y, (const bf16*)x, (const bf16*)w, (const bf16*)bias, M, N, K, limit);             \
+  } while (0)
+#define DLLM_ST_M(RT_, GLU_, WV_)                                                                                    \
+  do {                                                                                                              \
+    if (M <= 16) DLLM_ST_GO(RT_, 1, GLU_, WV_);                                                                      \
+    else if (M <= 32) DLLM_ST_GO(RT_, 2, GLU_, WV_);                                                                 \
+    else DLLM_ST_GO(RT_, 4, GLU_, 4);                                                                                \
+  } while (0)
+#define DLLM_ST_GLU(GLU_)                                                                                            \
+  do {                                                                                                              \
+    if (two) DLLM_ST_M(4, GLU_, 4);                                                                                  \
+    else DLLM_ST_M(2, GLU_, 4);                                                                                      \
+  } while (0)
+  if (glu == 0) {
+    if (two) DLLM_ST_M(2, 0, 4);
+    else DLLM_ST_M(1, 0, 8);
+  } else if (glu == 1) DLLM_ST_GLU(1);
+  else if (glu == 2) DLLM_ST_GLU(2);
+  else DLLM_ST_GLU(3);
+#undef DLLM_ST_GLU
+#undef DLLM_ST_M
+#undef DLLM_ST_GO
+  DLLM_HIP_CHECK(hipGetLastError());
+}
+
+}  // namespace dllm

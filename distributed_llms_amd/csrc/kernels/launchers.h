@@ -40,6 +40,8 @@ void gemm_pp_moe(uintptr_t y, uintptr_t x, uintptr_t gather, uintptr_t w, uintpt
                  int N, int K, int xrows, int slots, int mode, uintptr_t stream, float limit);
 void gemm_pf(uintptr_t c, uintptr_t a, uintptr_t b, int M, int N, int K, int mode, int variant, uintptr_t stream,
              float limit);
+void gemm_stream(uintptr_t y, uintptr_t x, uintptr_t w, uintptr_t bias, int M, int N, int K, int glu, int nt, float limit,
+                 uintptr_t stream);
 int gemm_sq(uintptr_t c, uintptr_t a, uintptr_t b, uintptr_t ws, long ws_floats, int M, int N, int K, int splits,
             int mode, int variant, uintptr_t stream);
 

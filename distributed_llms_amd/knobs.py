@@ -31,6 +31,8 @@ class Knobs:
     # which decode-sized GEMMs gemm_wide serves: "auto" (the cutovers below), "all", "none", or a
     # comma list of roles gate_up / down / proj
     wide: str = "auto"
+    # up to 64 rows of a small weight on the weight-streaming kernel (gemm_stream.hip; ops/gemm.stream_fits)
+    stream: bool = True
     # gemm_wide variant for unsplit grids (33: LDS-DMA interleaved + asm fragment reads with one
     # lgkmcnt per MFMA row) and for split-K grids (2: weights nontemporal, each byte is read once per
     # launch: 8B down 21.7 -> 19.6 us at M = 1, 23.2 -> 21.6 at 64, 34.1 -> 33.4 at 256; qkv 10.9 -> 10.1

@@ -255,7 +255,7 @@ class BasopelStage(LayerListStage):
             a = sm.window_attention(q, kc, vc, meta.block_tables, sb, 1 << 30, float(m["scale"]), num_decode=nd,
                                     max_ctx=max_ctx, chunk=size, softcap=float(m.get("softcap") or 0.0), sinks=w["sinks"],
                                     gate=proj, gate_col=hh * d + g * (d + dv))
-        return ops.linear(a.view(a.shape[0], -1), w["wo"], defer=True)
+        return ops.linear_into_norm(a.view(a.shape[0], -1), w["wo"])
 
     def _value_mix(self, i: int, first: Optional[torch.Tensor], tokens: int) -> Optional[sm.ValueMix]:
         if i not in self.mixing:
@@ -294,7 +294,7 @@ class BasopelStage(LayerListStage):
             x, h = sm.post_layer_norm_add(x, o, w["norm1b"], w["norm1b_b"], eps, bias=w.get("bo"), w_next=after[0],
                                           b_next=after[1])
             if spec.get("mlp"):
-                y = ops.linear(sm.linear_gelu_glu(h, w["w_gu"]), w["w_down"], defer=True)
+                y = ops.linear_into_norm(sm.linear_gelu_glu(h, w["w_gu"]), w["w_down"])
                 x, h = sm.post_layer_norm_add(x, y, w["norm2b"], w["norm2b_b"], eps, w_next=nxt[0], b_next=nxt[1])
             if self.taps is not None:
                 self.taps.append(x.clone())

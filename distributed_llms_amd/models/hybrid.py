@@ -371,7 +371,7 @@ class HybridStage(LayerListStage):
             nxt = self.layers[i + 1]["norm1"] if i + 1 < n else None
             x, h = sm.post_norm_add(x, o, w["norm1b"], eps, mult, w_next=w["norm2"] if spec.get("mlp") else nxt)
             if spec.get("mlp"):
-                y = sm.clipped_glu(ops.linear(h, w["w_gu"]), w["b_gu"], spec["mlp"]["limit"])
+                y = sm.linear_clipped_glu(h, w["w_gu"], w["b_gu"], spec["mlp"]["limit"])
                 x, h = sm.post_norm_add(x, ops.linear(y, w["w_down"]), w["norm2b"], eps, mult, bias=w["b_down"],
                                         w_next=nxt)
             if self.taps is not None:

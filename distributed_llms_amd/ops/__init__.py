@@ -21,7 +21,7 @@ from . import gemm, quant
 from . import reference as ref
 
 __all__ = [
-    "embedding", "rms_norm", "fused_add_rms_norm", "layer_norm", "linear", "silu_mul",
+    "embedding", "rms_norm", "fused_add_rms_norm", "layer_norm", "linear", "linear_into_norm", "silu_mul",
     "gelu_tanh", "rope_cache_append", "paged_attention_decode", "paged_attention_prefill",
     "argmax", "add_", "moe_route", "moe_mlp", "decode_split_plan", "paged_attention_decode_rope",
     "paged_attention_prefill_rope",
@@ -144,6 +144,11 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
     if not _gpu(x):
         return ref.linear(x, w, bias)
     return gemm.linear(x, w, bias, defer=defer)
+
+
+def linear_into_norm(x: torch.Tensor, w: torch.Tensor):
+    """:func:`linear` for a consumer that takes a :class:`gemm.SplitKPartial` (the closing norm of a sublayer)."""
+    return gemm.linear_into_norm(x, w) if _gpu(x) else ref.linear(x, w)
 
 
 def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor) -> torch.Tensor:

@@ -1,6 +1,7 @@
 """Dense GEMM dispatch for y = x @ w^T (w is [N, K], nn.Linear layout).
 
-Decode-sized M goes to hand-written gfx950 kernels, per projection role (cutovers measured in
+Up to 64 rows, a small weight goes to the weight-streaming kernel (gemm_stream.hip, :func:`use_stream`): no K split,
+bias and GLU in its epilogue.  Other decode-sized M go to hand-written gfx950 kernels, per projection role (cutovers measured in
 the engine on Llama-3-8B, profiles/wide_gemm.md; each one is a field of :mod:`..knobs`):
 
 * wide-M kernel (gemm_wide.hip: 64/128/192/256-row x 128 tiles, 3-stage LDS-DMA pipeline,
@@ -21,8 +22,8 @@ the engine on Llama-3-8B, profiles/wide_gemm.md; each one is a field of :mod:`..
   256 x 256-tile schedule-2 kernel in its persistent form (gemm_pf in gemm_pp.hip, knobs.pp_persistent)
   -- gate|up with the SwiGLU fused into its epilogue, qkv / o / down plain
   (profiles/round4_gemm_counters.md);
-* what none of them takes (a bias, N not a multiple of 256, fp32 on CPU, operands >= 4 GiB):
-  torch's F.linear.
+* what none of them takes (a bias or N not a multiple of 128 past 64 rows, K not a multiple of 64, fp32 on CPU,
+  operands >= 4 GiB): torch's F.linear.
 
 The role is inferred from the shape: "down" = K >= 8192 and K > N, so the square / widening
 K = 8192 projections of 70B-class models (qkv 8192 -> 10240, o 8192 -> 8192) stay "proj".
@@ -92,6 +93,64 @@ def _use_wide(m: int, n: int, k: int, x: torch.Tensor, w: torch.Tensor, swiglu: 
     return ("down" in roles) if is_down_proj(n, k) else ("proj" in roles and m <= 512)
 
 
+# Weights (elements) up to which gemm_stream serves M <= 64 rows; all sides measured on cold weights, us at M = 1 / 16 /
+# 32 / 64, a split-K reduction or an activation kernel in a launch of its own being 4.6 each (gemm_stream.hip):
+#  * plain: 5120 x 2560 7.0 / 8.2 / 9.7 / 12.5 against 12.5 / 13.1 / 13.6 / 14.2 for the wide kernel and its reduction;
+#    6144 x 4096 10.3 / 12.4 / 13.8 / 17.1 against 14.8 / 15.4 / 15.8 / 16.2;
+#  * the consumer sums the slabs (defer), so the wide kernel pays no reduction: 2560 x 2560 4.7 / 5.9 / 7.4 / 9.7 against
+#    6.7 / 7.2 / 7.7 / 8.2, 1024 x 1024 3.0 / 3.4 / 4.0 / 5.1 against 5.0 / 5.4 / 5.5 / 5.6;
+#  * GLU: 15360 x 2560 14.2 / 14.7 / 16.2 / 19.7 against 20.4 / 21.1 / 22.1 / 23.1; the 8B gate|up (28672 x 4096) 38 / 39 /
+#    44 / 48 against 38 / 38.6 / 40 / 41 for the wide kernel's own SiLU epilogue, which has no other activation.
+STREAM_MAX_M = 64
+STREAM_PLAIN, STREAM_PLAIN_32 = 16 << 20, 32 << 20
+STREAM_DEFER, STREAM_DEFER_16 = 2 << 20, 8 << 20
+STREAM_GLU, STREAM_GLU_32 = 40 << 20, 128 << 20
+
+
+def stream_fits(m: int, n: int, k: int, glu: str = "", defer: bool = False) -> bool:
+    """Does gemm_stream serve an [m, k] x [n, k]^T product?  ``glu``: "" (plain), "silu", "clipped" or "gelu"."""
+    if not 1 <= m <= STREAM_MAX_M or k % 64 or k < 512:
+        return False                                 # K < 512: fewer K-tiles than waves, and no split to save either
+    if glu:
+        return n * k <= (STREAM_GLU_32 if m <= 32 and glu != "silu" else STREAM_GLU)
+    if n > 65536:
+        return False                                 # an LM head fills the chip unsplit on the wide kernel
+    if defer and n % 128 == 0:
+        return n * k <= (STREAM_DEFER_16 if m <= 16 else STREAM_DEFER)
+    return n * k <= (STREAM_PLAIN_32 if m <= 32 else STREAM_PLAIN)
+
+
+def use_stream(m: int, n: int, k: int, x: torch.Tensor, w: torch.Tensor, bias=None, glu: str = "", defer: bool = False) -> bool:
+    return (knobs.K.stream and stream_fits(m, n, k, glu, defer) and x.dtype == w.dtype == torch.bfloat16
+            and x.is_contiguous() and w.is_contiguous() and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and (bias is None or (bias.dtype == torch.bfloat16 and bias.is_contiguous())))
+
+
+def linear_into_norm(x: torch.Tensor, w: torch.Tensor):
+    """``x w^T`` for a consumer that sums split-K slabs itself (post_norm_add, post_layer_norm_add): the finished product
+    where the weight-streaming kernel is faster than the split grid alone, else possibly a :class:`SplitKPartial`."""
+    k = x.shape[-1]
+    if use_stream(x.numel() // k, w.shape[0], k, x, w, defer=True):
+        return linear_stream(x, w)
+    return linear(x, w, defer=True)
+
+
+_STREAM_GLU = {"": 0, "silu": 1, "clipped": 2, "gelu": 3}
+
+
+def linear_stream(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, glu: str = "",
+                  limit: float = 0.0) -> torch.Tensor:
+    """y = x w^T (+ bias), or its GLU with w = [Wg; Wu], for up to 64 rows (csrc/kernels/gemm_stream.hip)."""
+    k = x.shape[-1]
+    n = w.shape[0]
+    m = x.numel() // k
+    y = torch.empty(*x.shape[:-1], n // 2 if glu else n, dtype=x.dtype, device=x.device)
+    _ext.kernels().gemm_stream(y.data_ptr(), x.data_ptr(), w.data_ptr(), 0 if bias is None else bias.data_ptr(), m, n, k,
+                               _STREAM_GLU[glu], 1 if n * k * 2 >= WIDE_NT_MIN_BYTES else 0, float(limit),
+                               torch.cuda.current_stream().cuda_stream)
+    return y
+
+
 class SplitKPartial:
     """Split-K partial sums of ``x @ w.T`` still in the per-stream workspace (not reduced).  Each K
     slice accumulates in f32; the slabs hold it as f16 x 2^-6 by default (csrc/kernels/common.h
@@ -123,6 +182,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
     if w.shape[1] != k:
         raise ValueError(f"linear: x[..., {k}] vs w {tuple(w.shape)}")
     kn = knobs.K
+    if not (defer and n % 128 == 0) and use_stream(m, n, k, x, w, bias):
+        return linear_stream(x, w, bias)
     # decode LM head on gemm_pp with nontemporal weights (236 vs 268 us for gemm_sq at M = 256) --
     # unless comm kernels may hold CUs: beside a 4-workgroup, 20 KiB-LDS receive spinning in
     # another process it took 284 us, gemm_sq 268 either way (bench/debug/lm_head_bench.py,
@@ -402,13 +463,18 @@ def linear_sq(x: torch.Tensor, w: torch.Tensor, splits: int = 0, swiglu: bool = 
     return y
 
 
-def _linear_glu(x: torch.Tensor, w_gate_up: torch.Tensor, limit: Optional[float]) -> Optional[torch.Tensor]:
-    """A GLU of x Wg^T and x Wu^T, W = [Wg; Wu], with the activation in the persistent GEMM's epilogue (prompts) or in
-    the split-K reduction (decode): clipped (``limit``) or gelu_tanh (None); None if the shape takes neither."""
+def _linear_glu(x: torch.Tensor, w_gate_up: torch.Tensor, limit: Optional[float],
+                bias: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+    """A GLU of x Wg^T and x Wu^T, W = [Wg; Wu], with the activation in the weight-streaming GEMM's epilogue (up to 64
+    rows; the only form that takes a ``bias`` [gate | up]), in the persistent GEMM's (prompts) or in the split-K
+    reduction (decode): clipped (``limit``) or gelu_tanh (None); None if the shape takes none of them."""
     k = x.shape[-1]
     n = w_gate_up.shape[0]
     m = x.numel() // k
-    if x.dtype != torch.bfloat16 or n % 256:
+    glu = "gelu" if limit is None else "clipped"
+    if n % 2 == 0 and use_stream(m, n, k, x, w_gate_up, bias, glu):
+        return linear_stream(x, w_gate_up, bias, glu, 0.0 if limit is None else limit)
+    if x.dtype != torch.bfloat16 or n % 256 or bias is not None:
         return None
     if not _use_wide(m, n, k, x, w_gate_up) and _use_pp(m, n, k, x, w_gate_up, knobs.K.pp_swiglu_min_m) \
             and knobs.K.pp_persistent and m * (n // 2) * 2 < (1 << 31) and pf_fills(m, n, x.device):
@@ -426,9 +492,11 @@ def _linear_glu(x: torch.Tensor, w_gate_up: torch.Tensor, limit: Optional[float]
     return gelu_glu(y) if limit is None else clipped_glu(y, None, limit)
 
 
-def linear_clipped_glu(x: torch.Tensor, w_gate_up: torch.Tensor, limit: float) -> Optional[torch.Tensor]:
-    """g sigmoid(1.702 g) (u + 1), g = min(x Wg^T, limit), u = clamp(x Wu^T, -limit, limit), fused (:func:`_linear_glu`)."""
-    return _linear_glu(x, w_gate_up, float(limit))
+def linear_clipped_glu(x: torch.Tensor, w_gate_up: torch.Tensor, limit: float,
+                       bias: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+    """g sigmoid(1.702 g) (u + 1), g = min(x Wg^T, limit), u = clamp(x Wu^T, -limit, limit) (``bias`` [gate | up] added
+    to the products), fused (:func:`_linear_glu`)."""
+    return _linear_glu(x, w_gate_up, float(limit), bias)
 
 
 def linear_gelu_glu(x: torch.Tensor, w_gate_up: torch.Tensor) -> Optional[torch.Tensor]:
@@ -442,6 +510,8 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor) -> Optional[torch.Te
     n = w_gate_up.shape[0]
     m = x.numel() // k
     kn = knobs.K
+    if n % 2 == 0 and use_stream(m, n, k, x, w_gate_up, glu="silu"):
+        return linear_stream(x, w_gate_up, glu="silu")
     if 0 < kn.pp_gate_up_min_m <= m <= 256 and not _comm_cus and _use_pp(m, n, k, x, w_gate_up, 1):
         # decode gate|up on gemm_pp, unsplit, weights nontemporal, on the column tile that gives one
         # round of CUs / 2 .. CUs tiles: 8B (224 x 128 columns) 62.1 vs 64.1 us for gemm_wide, 70B

@@ -185,7 +185,7 @@ def latent_attention(h: torch.Tensor, w: dict, spec: LatentSpec, freqs: Optional
     ``q_norm``, ``c_norm``, ``uq`` [H (dim + rot_dim), q_rank] (``q_norm`` and ``uq`` only with a query latent), ``uk``
     [H, dim, rank], ``uv_t`` [H, rank, vdim], ``o`` [W, H vdim] and optionally ``sinks`` [H] float32.  Returns [T, W] (with
     ``defer`` possibly a :class:`~.gemm.SplitKPartial`)."""
-    from . import linear
+    from . import linear, linear_into_norm
     down = linear(h, w["down"])
     cq = latent_prep(down, spec, w.get("q_norm"), w["c_norm"], freqs, eps, k_cache, v_cache, slot_mapping, sb.positions)
     q = linear(cq, w["uq"]) if spec.q_rank else down[:, :spec.q_cols]
@@ -193,7 +193,7 @@ def latent_attention(h: torch.Tensor, w: dict, spec: LatentSpec, freqs: Optional
     o_lat = sm.window_attention(qf, k_cache, v_cache, block_tables, sb, window, spec.scale, num_decode=num_decode,
                                 sinks=w.get("sinks"), max_ctx=max_ctx)
     o = latent_values(o_lat, w["uv_t"], down if spec.gated else None, spec.gate_col, spec.gate_elements)
-    return linear(o, w["o"], defer=defer)
+    return linear_into_norm(o, w["o"]) if defer else linear(o, w["o"])
 
 
 # ------------------------------------------------------------------ parallel layers on a float32 stream

@@ -450,6 +450,14 @@ def clipped_glu(gu: torch.Tensor, bias_gu: Optional[torch.Tensor], limit: float,
     return out
 
 
+def linear_clipped_glu(x: torch.Tensor, w_gate_up: torch.Tensor, bias_gu: Optional[torch.Tensor], limit: float) -> torch.Tensor:
+    """:func:`clipped_glu` of ``x W^T``, W = [Wg; Wu]: in a GEMM epilogue where one takes the shape and the bias, else the
+    projection followed by the gate kernel."""
+    from . import gemm, linear
+    y = gemm.linear_clipped_glu(x, w_gate_up, limit, bias_gu) if x.is_cuda else None
+    return clipped_glu(linear(x, w_gate_up), bias_gu, limit) if y is None else y
+
+
 def gelu_glu(gu: torch.Tensor) -> torch.Tensor:
     """[T, 2F] = gate | up -> gelu_tanh(gate) * up  [T, F]."""
     t, two_f = gu.shape

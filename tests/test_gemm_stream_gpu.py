@@ -1,0 +1,90 @@
+"""The weight-streaming decode GEMM (csrc/kernels/gemm_stream.hip) against float64, and the rule that picks it."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from distributed_llms_amd import knobs
+from distributed_llms_amd.ops import gemm
+
+
+def _close(y, ref, terms, k):
+    """``ref``: float64 result, ``terms``: the sum of the magnitudes of its products.  An f32 sum of k products in any
+    order is within k 2^-24 of that; the bf16 result rounds by 2^-9."""
+    tol = k * 2.0 ** -24 * terms + 2.0 ** -8 * ref.abs() + 1e-30
+    return bool(((y.double() - ref).abs() <= tol).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [1, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("n,k", [(1, 64), (40, 64), (50, 192), (1024, 1024), (3088, 2560), (4097, 576), (4128, 128)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_stream_linear(cuda, m, n, k, bias):
+    """One 16-row weight tile per workgroup and two (N > 4096), fewer K-tiles than waves, ragged last tiles of N."""
+    x, w = torch.randn(m, k, device="cuda").bfloat16(), (torch.randn(n, k, device="cuda") * 0.05).bfloat16()
+    b = torch.randn(n, device="cuda").bfloat16() if bias else None
+    guard = torch.full((m * n + 64,), 7.0, dtype=torch.bfloat16, device="cuda")
+    y = gemm.linear_stream(x, w, b)
+    ref = F.linear(x.double(), w.double(), None if b is None else b.double())
+    mag = x.double().abs() @ w.double().abs().t() + (0 if b is None else b.double().abs())
+    assert _close(y, ref, mag, k + 1)
+    # nothing outside y: the same launch into a window of a larger buffer
+    from distributed_llms_amd import _ext
+    _ext.kernels().gemm_stream(guard.data_ptr(), x.data_ptr(), w.data_ptr(), 0 if b is None else b.data_ptr(), m, n, k, 0, 1,
+                               0.0, torch.cuda.current_stream().cuda_stream)
+    assert torch.equal(guard[:m * n].view(m, n), y) and bool((guard[m * n:] == 7.0).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [1, 16, 31, 64])
+@pytest.mark.parametrize("half,k", [(24, 64), (1536, 1024), (4112, 640)])
+@pytest.mark.parametrize("glu", ["silu", "clipped", "gelu"])
+@pytest.mark.parametrize("bias", [False, True])
+def test_stream_glu(cuda, m, half, k, glu, bias):
+    x, w = torch.randn(m, k, device="cuda").bfloat16(), (torch.randn(2 * half, k, device="cuda") * k ** -0.5).bfloat16()
+    b = torch.randn(2 * half, device="cuda").bfloat16() if bias else None
+    y = gemm.linear_stream(x, w, b, glu, 0.7)
+    z = F.linear(x.double(), w.double(), None if b is None else b.double())
+    mag = (x.double().abs() @ w.double().abs().t() + (0 if b is None else b.double().abs())) * (k + 1) * 2.0 ** -24
+    g, u = z[:, :half], z[:, half:]
+    if glu == "silu":
+        ref = F.silu(g) * u
+    elif glu == "clipped":
+        g, u = g.clamp(max=0.7), u.clamp(-0.7, 0.7)
+        ref = g * torch.sigmoid(1.702 * g) * (u + 1)
+    else:
+        ref = F.gelu(g, approximate="tanh") * u
+    # |d act / d gate| <= 1.2, act <= |gate|, |u| (+ 1 where clipped): the sums' errors through the product; the hardware
+    # exponential and reciprocal are within 2^-20 of exact; the result rounds to bf16
+    up = u.abs() + (1 if glu == "clipped" else 0)
+    tol = 1.2 * mag[:, :half] * up + (g.abs() + 1e-3) * mag[:, half:] + (2.0 ** -8 + 2.0 ** -18) * ref.abs() + 2.0 ** -22
+    assert bool(((y.double() - ref).abs() <= tol).all())
+
+
+@pytest.mark.gpu
+def test_stream_is_reached_and_matches_the_wide_route(cuda):
+    """ops.linear / linear_swiglu at decode sizes take the kernel by default; knobs.stream off gives the former route."""
+    from distributed_llms_amd import ops
+    x = torch.randn(9, 1024, device="cuda").bfloat16()
+    w = (torch.randn(2048, 1024, device="cuda") * 0.03).bfloat16()
+    for f in (lambda: ops.linear(x, w), lambda: ops.linear_swiglu(x, w), lambda: ops.linear(x[:, None], w)):
+        a = f()
+        with knobs.override(stream=False):
+            b = f()
+        assert a.shape == b.shape
+        torch.testing.assert_close(a.float(), b.float(), atol=2e-2, rtol=2e-2)
+
+
+def test_stream_rule():
+    assert gemm.stream_fits(1, 1024, 1024) and gemm.stream_fits(64, 5120, 2560) and not gemm.stream_fits(65, 1024, 1024)
+    assert not gemm.stream_fits(8, 1024, 1000) and not gemm.stream_fits(8, 128256, 4096)
+    assert gemm.stream_fits(32, 6144, 4096) and not gemm.stream_fits(33, 6144, 4096)
+    assert gemm.stream_fits(16, 2560, 2560, defer=True) and not gemm.stream_fits(17, 2560, 2560, defer=True)
+    assert not gemm.stream_fits(1, 4096, 4096, defer=True)             # the 8B projections stay on the wide kernel
+    assert not gemm.stream_fits(1, 28672, 4096, "silu") and gemm.stream_fits(64, 15360, 2560, "gelu")
+    assert not gemm.stream_fits(8, 1024, 448)
+    x, w = torch.zeros(4, 512, dtype=torch.bfloat16), torch.zeros(256, 512, dtype=torch.bfloat16)
+    assert gemm.use_stream(4, 256, 512, x, w)
+    assert not gemm.use_stream(4, 256, 512, x.float(), w) and not gemm.use_stream(4, 256, 512, x, w.t().contiguous().t())
+    assert not gemm.use_stream(4, 256, 512, x, torch.zeros(256 * 512 + 1, dtype=torch.bfloat16)[1:].view(256, 512))
+    with knobs.override(stream=False):
+        assert not gemm.use_stream(4, 256, 512, x, w)
