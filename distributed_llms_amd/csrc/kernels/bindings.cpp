@@ -54,6 +54,7 @@ PYBIND11_MODULE(_C_kernels, m) {
   m.def("sm_causal_conv", &dllm::sm_causal_conv);
   m.def("sm_rglru_gates", &dllm::sm_rglru_gates);
   m.def("sm_rglru_scan", &dllm::sm_rglru_scan);
+  m.def("sm_rglru_step", &dllm::sm_rglru_step);
   m.def("sm_clipped_glu", &dllm::sm_clipped_glu);
   m.def("sm_softcap", &dllm::sm_softcap);
   m.def("sm_attn_prep", &dllm::sm_attn_prep);

@@ -116,7 +116,7 @@ void hc_step(uintptr_t x, uintptr_t mix, uintptr_t out_w, uintptr_t o, uintptr_t
              uintptr_t stream);
 void sm_rms_norm(uintptr_t y, uintptr_t x, uintptr_t w, int rows, int width, float eps, float offset, int f32,
                  uintptr_t stream);
-void sm_post_norm_add(uintptr_t x, uintptr_t o, uintptr_t bias, uintptr_t w_post, uintptr_t w_next, uintptr_t h,
+void sm_post_norm_add(uintptr_t x, uintptr_t o, int parts, uintptr_t bias, uintptr_t w_post, uintptr_t w_next, uintptr_t h,
                       int rows, int width, float eps, float mult, float offset, uintptr_t o2, float s1, float s2,
                       int f32, uintptr_t stream);
 void sm_causal_conv(uintptr_t y, uintptr_t u, long stride, uintptr_t w, uintptr_t bias, uintptr_t in_bias,
@@ -130,6 +130,10 @@ void sm_rglru_gates(uintptr_t a, uintptr_t g, uintptr_t u, uintptr_t ra_t, uintp
 void sm_rglru_scan(uintptr_t out, uintptr_t a, uintptr_t g, uintptr_t y_raw, long y_stride, uintptr_t y_bias,
                    uintptr_t state, uintptr_t cu, uintptr_t positions, uintptr_t slots, int seqs, int C, int max_q_len,
                    uintptr_t ab, int f32, uintptr_t stream);
+void sm_rglru_step(uintptr_t out, uintptr_t x, uintptr_t y, long ld, uintptr_t conv_w, uintptr_t conv_b, uintptr_t x_b,
+                   uintptr_t conv_state, uintptr_t ra_t, uintptr_t ra_b, uintptr_t ri_t, uintptr_t ri_b, uintptr_t lam,
+                   uintptr_t y_b, uintptr_t state, uintptr_t positions, uintptr_t slots, int seqs, int nb,
+                   int bw, int taps, float scale, uintptr_t arrived, int arrived_len, int f32, uintptr_t stream);
 void sm_clipped_glu(uintptr_t out, uintptr_t gu, uintptr_t bias, int tokens, int F, float limit, float alpha, int f32,
                     uintptr_t stream);
 void sm_softcap(uintptr_t out, uintptr_t x, long n, float cap, float scale, int f32, uintptr_t stream);
@@ -141,7 +145,7 @@ void sm_head_norm_rope(uintptr_t q_out, uintptr_t qkv, long ld, int col0, uintpt
 void sm_attn_prep(uintptr_t q_out, uintptr_t qkv, uintptr_t conv_w, uintptr_t state, uintptr_t q_norm,
                   uintptr_t k_norm, uintptr_t freqs, int nrot, float mag, float eps, uintptr_t k_cache,
                   uintptr_t v_cache, uintptr_t slot_mapping, uintptr_t cu, uintptr_t positions, uintptr_t tok_seq,
-                  uintptr_t slots, int tokens, int seqs, int H, int G, int D, int Dv, int taps, int bs, int f32,
+                  uintptr_t slots, int tokens, int seqs, int H, int G, int D, int Dv, int taps, int bs, int max_q_len, int f32,
                   uintptr_t stream);
 void sm_rownorm_rope(uintptr_t q_out, uintptr_t qkv, long ld, int col0, uintptr_t q_norm, uintptr_t k_norm,
                      uintptr_t freqs, int nrot, float eps, uintptr_t k_cache, uintptr_t v_cache, uintptr_t slot_mapping,

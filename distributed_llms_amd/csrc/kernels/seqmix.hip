@@ -130,7 +130,7 @@ void sm_rms_norm(uintptr_t y, uintptr_t x, uintptr_t w, int rows, int width, flo
                 (const void*)w, width, eps, offset);
 }
 
-// --------------------------------------------------------------------------- close of a sublayer
+// --------------------------------------------------------------------------- close of a sublayer (rows past 16384)
 // x += mult * rms_norm(v) * (offset + w_post) with v = o + bias, or v = s1 o + s2 o2 when a second input is
 // given (two mixers side by side);  h = rms_norm(x) * (offset + w_next) when w_next, else, when h is
 // given, the new stream itself in the activation type (a following sublayer that reads x unnormed)
@@ -206,16 +206,6 @@ __global__ void __launch_bounds__(256) sm_post_norm_add_kernel(float* __restrict
   }
 }
 
-void sm_post_norm_add(uintptr_t x, uintptr_t o, uintptr_t bias, uintptr_t w_post, uintptr_t w_next, uintptr_t h,
-                      int rows, int width, float eps, float mult, float offset, uintptr_t o2, float s1, float s2,
-                      int f32, uintptr_t stream) {
-  if (rows <= 0) return;
-  DLLM_HOST_CHECK(width > 0 && (!w_next || h), "post_norm_add arguments");
-  SM_DISPATCH_V(f32, width % 8 == 0, sm_post_norm_add_kernel, dim3(rows), dim3(256), 0, stream, (float*)x,
-                (const void*)o, (const void*)bias, (const void*)w_post, (const void*)w_next, (void*)h, width, eps, mult,
-                offset, (const void*)o2, s1, s2);
-}
-
 // --------------------------------------------------------------------------- layer norms on the float32 stream
 // One workgroup per row, the row in registers (NV pieces of V consecutive elements per lane): the mean first, then the
 // mean of the squared deviations from it.
@@ -276,6 +266,36 @@ __global__ void __launch_bounds__(256) sm_layer_norm_kernel(void* __restrict__ y
   }
 }
 
+// One row of a product that is still in `parts` split-K slabs (V = 4; common.h part_load): their sum, rounded to bf16 as the
+// reduction of a split product rounds it.  Every load off a clamped place, the slabs eight at a time.
+template <int NV, int V>
+__device__ __forceinline__ void ln_slabs(const float* __restrict__ P, int parts, size_t row, int width, float (&v)[NV][V]) {
+  const size_t slab = (size_t)gridDim.x * width;
+  const int top = width - V;
+  constexpr int CH = NV <= 4 ? 8 : 2;
+  f32x4 a[NV];
+#pragma unroll
+  for (int k = 0; k < NV; ++k) a[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < parts; s0 += CH) {
+    f32x4 l[CH][NV];
+#pragma unroll
+    for (int u = 0; u < CH; ++u)
+#pragma unroll
+      for (int k = 0; k < NV; ++k)
+        l[u][k] = part_load4(P, min(s0 + u, parts - 1) * slab + row + min((k * 256 + (int)threadIdx.x) * V, top));
+#pragma unroll
+    for (int u = 0; u < CH; ++u)
+      if (s0 + u < parts) {
+#pragma unroll
+        for (int k = 0; k < NV; ++k) a[k] += l[u][k];
+      }
+  }
+#pragma unroll
+  for (int k = 0; k < NV; ++k)
+#pragma unroll
+    for (int j = 0; j < V; ++j) v[k][j] = bf2f(f2bf(a[k][j & 3]));
+}
+
 // The close of a sublayer between two layer norms: x += layer_norm(o + bias) (weight wp, bias bp; `bias` null: none), and
 // with wn: h = layer_norm(x) (wn, bn), the next sublayer's input.  parts > 0: o is the sum of that many split-K slabs
 // [rows, width] (common.h part_load; bf16 results, rounded as the reduction of a split product rounds them).
@@ -291,30 +311,7 @@ __global__ void __launch_bounds__(256) sm_post_layer_norm_kernel(
   // every load of the row off a clamped place, so that none waits behind another's guard; the slabs eight at a time
   const int top = width - V;
   if (V == 4 && parts > 0) {
-    const float* P = (const float*)o_;
-    const size_t slab = (size_t)gridDim.x * width;
-    constexpr int CH = NV <= 4 ? 8 : 2;
-    f32x4 a[NV];
-#pragma unroll
-    for (int k = 0; k < NV; ++k) a[k] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int s0 = 0; s0 < parts; s0 += CH) {
-      f32x4 l[CH][NV];
-#pragma unroll
-      for (int u = 0; u < CH; ++u)
-#pragma unroll
-        for (int k = 0; k < NV; ++k)
-          l[u][k] = part_load4(P, min(s0 + u, parts - 1) * slab + row + min((k * 256 + (int)threadIdx.x) * V, top));
-#pragma unroll
-      for (int u = 0; u < CH; ++u)
-        if (s0 + u < parts) {
-#pragma unroll
-          for (int k = 0; k < NV; ++k) a[k] += l[u][k];
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < NV; ++k)
-#pragma unroll
-      for (int j = 0; j < V; ++j) v[k][j] = bf2f(f2bf(a[k][j & 3]));
+    ln_slabs<NV>((const float*)o_, parts, row, width, v);
   } else {
 #pragma unroll
     for (int k = 0; k < NV; ++k) ldv<V>((const T*)o_ + row + min((k * 256 + (int)threadIdx.x) * V, top), v[k]);
@@ -407,6 +404,103 @@ void sm_post_layer_norm_add(uintptr_t x, uintptr_t o, int parts, uintptr_t bias,
   SM_LN_DISPATCH(f32, width, sm_post_layer_norm_kernel, dim3(rows), stream, (float*)x, (const void*)o, parts,
                  (const void*)bias, (const void*)w_post, (const void*)b_post, (const void*)w_next, (const void*)b_next,
                  (void*)h, width, eps);
+}
+
+// The close of a sublayer around RMS norms, the row in registers (NV pieces of V elements per lane): every load -- o or its
+// slabs, the second input, bias, stream and both weights -- goes out before the first use, and nothing is read twice (the
+// three-pass form above re-read o, x and the new x, with each pass's loads behind a block reduction).
+// parts > 0: o is the sum of that many split-K slabs [rows, width], rounded as the reduction of a split product rounds it.
+// 2560 wide, bf16: 16 rows 5.9 -> 4.0 us (bound by the launch and two reductions), 6376 rows 41 -> 37 us (5.2 TB/s).
+template <typename T, int V, int NV>
+__global__ void __launch_bounds__(256) sm_post_norm_row_kernel(float* __restrict__ x, const void* __restrict__ o_, int parts,
+                                                               const void* __restrict__ bias_, const void* __restrict__ wp_,
+                                                               const void* __restrict__ wn_, void* __restrict__ h_, int width,
+                                                               float eps, float mult, float offset,
+                                                               const void* __restrict__ o2_, float s1, float s2) {
+  __shared__ float red[16];
+  const size_t row = (size_t)blockIdx.x * width;
+  float* xr = x + row;
+  float v[NV][V], xv[NV][V], wp[NV][V], wn[NV][V];
+  const int top = width - V;
+  if (V == 4 && parts > 0) {
+    ln_slabs<NV>((const float*)o_, parts, row, width, v);
+  } else {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) ldv<V>((const T*)o_ + row + min((k * 256 + (int)threadIdx.x) * V, top), v[k]);
+  }
+  // what is not given is read from the closing weight and dropped: no load behind a branch (hipcc would wait there)
+  const T* pn = (const T*)(wn_ ? wn_ : wp_);
+  const T* p2 = o2_ ? (const T*)o2_ + row : (const T*)wp_;
+  const T* pb = (const T*)(bias_ ? bias_ : wp_);
+  float c2[NV][V], cb[NV][V];
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+    const int i = min((k * 256 + (int)threadIdx.x) * V, top);
+    ldv<V>(xr + i, xv[k]);
+    ldv<V>((const T*)wp_ + i, wp[k]);
+    ldv<V>(pn + i, wn[k]);
+    ldv<V>(p2 + i, c2[k]);
+    ldv<V>(pb + i, cb[k]);
+  }
+#pragma unroll
+  for (int k = 0; k < NV; ++k)
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+      if (o2_) v[k][j] = s1 * v[k][j] + s2 * c2[k][j];
+      if (bias_) v[k][j] += cb[k][j];
+    }
+  float ss = 0.f;
+#pragma unroll
+  for (int k = 0; k < NV; ++k)
+    if ((k * 256 + (int)threadIdx.x) * V < width) {
+#pragma unroll
+      for (int j = 0; j < V; ++j) ss += v[k][j] * v[k][j];
+    }
+  ss = block_sum(ss, red);
+  const float inv = 1.0f / sqrtf(ss / (float)width + eps);
+  float sq = 0.f;
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+    const int i = (k * 256 + threadIdx.x) * V;
+    if (i < width) {
+#pragma unroll
+      for (int j = 0; j < V; ++j) {
+        xv[k][j] = xv[k][j] + mult * (v[k][j] * inv * (offset + wp[k][j]));
+        sq += xv[k][j] * xv[k][j];
+      }
+      stv<V>(xr + i, xv[k]);
+      if (!wn_ && h_) stv<V>((T*)h_ + row + i, xv[k]);
+    }
+  }
+  if (!wn_) return;
+  sq = block_sum(sq, red);
+  const float inv2 = 1.0f / sqrtf(sq / (float)width + eps);
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+    const int i = (k * 256 + threadIdx.x) * V;
+    if (i < width) {
+#pragma unroll
+      for (int j = 0; j < V; ++j) xv[k][j] = xv[k][j] * inv2 * (offset + wn[k][j]);
+      stv<V>((T*)h_ + row + i, xv[k]);
+    }
+  }
+}
+
+void sm_post_norm_add(uintptr_t x, uintptr_t o, int parts, uintptr_t bias, uintptr_t w_post, uintptr_t w_next, uintptr_t h,
+                      int rows, int width, float eps, float mult, float offset, uintptr_t o2, float s1, float s2,
+                      int f32, uintptr_t stream) {
+  if (rows <= 0) return;
+  DLLM_HOST_CHECK(width > 0 && (!w_next || h), "post_norm_add arguments");
+  DLLM_HOST_CHECK(parts >= 0 && (parts == 0 || (!f32 && width % 4 == 0 && width <= 16384)), "post_norm_add slabs");
+  if (width <= 16384) {
+    SM_LN_DISPATCH(f32, width, sm_post_norm_row_kernel, dim3(rows), stream, (float*)x, (const void*)o, parts,
+                   (const void*)bias, (const void*)w_post, (const void*)w_next, (void*)h, width, eps, mult, offset,
+                   (const void*)o2, s1, s2);
+    return;
+  }
+  SM_DISPATCH_V(f32, width % 8 == 0, sm_post_norm_add_kernel, dim3(rows), dim3(256), 0, stream, (float*)x,
+                (const void*)o, (const void*)bias, (const void*)w_post, (const void*)w_next, (void*)h, width, eps, mult,
+                offset, (const void*)o2, s1, s2);
 }
 
 // --------------------------------------------------------------------------- entry of a looped span
@@ -1103,6 +1197,225 @@ void sm_rglru_scan(uintptr_t out, uintptr_t a, uintptr_t g, uintptr_t y_raw, lon
               (const int32_t*)positions, (const int32_t*)slots, C);
 }
 
+// --------------------------------------------------------------------------- RG-LRU, one token per sequence
+// The whole recurrent branch of a decode step in one launch: the causal convolution of x (with its bias) and its new tail,
+// both gates, the state update and the gelu(y) product -- what the conv, conv tail, gate and scan kernels above do in four.
+// One workgroup per (64 outputs of a block of bw channels, GT_ sequences).  It is bound by round trips and by what one CU
+// can pull in (256 outputs per workgroup: 10.2-10.8 us, of one sequence as of 16), so the outputs are cut small and the
+// loads go out in as few rounds as they can: lane group og = tid % 8 owns 8 consecutive outputs and kg = tid / 8 every 32nd
+// input row of both gate matrices, a block of up to 256 being one round of kRows rows per thread that is sent out before
+// anything waits (the gate kernel had two weight loads in flight per thread: 19-27 us by itself), and each finishing
+// thread has its state, y and biases in registers before the convolution starts.
+// A gate needs all bw convolved inputs of its block, so every workgroup of a block convolves them all, and the tail may
+// move only when all have read it: each counts itself in `arrived` [sequence groups][blocks] once its reads have returned,
+// and the last of them -- nobody waits -- writes the new tail and clears the count.
+// 4 blocks of 256, 4 taps, bf16: one sequence 6.3 us, for 30 in four launches; 10 blocks: 16 sequences 9.1 us (42 before),
+// 64 sequences 20 us.
+constexpr int kRows = 8;       // gate matrix rows in flight per thread
+constexpr int kStepTaps = 8;   // at most
+constexpr int kStepOut = 64;   // outputs per workgroup
+constexpr int kCountStride = 32;
+template <typename T> struct Raw8 { typedef bf16x8 type; };
+template <> struct Raw8<float> { typedef float type __attribute__((ext_vector_type(8))); };
+
+template <typename T, int GT_, int TAPS_>
+__global__ void __launch_bounds__(256) sm_rglru_step_kernel(
+    void* __restrict__ out_, const void* __restrict__ x_, const void* __restrict__ y_, long ld,
+    const void* __restrict__ conv_w_, const void* __restrict__ conv_b_, const void* __restrict__ x_b_, void* conv_state_,
+    const void* __restrict__ ra_t_, const void* __restrict__ ra_b_, const void* __restrict__ ri_t_,
+    const void* __restrict__ ri_b_, const void* __restrict__ lam_, const void* __restrict__ y_b_, float* __restrict__ state,
+    const int32_t* __restrict__ positions, const int32_t* __restrict__ slots, int seqs, int nb, int bw, int taps, float scale,
+    int* __restrict__ arrived) {
+  typedef typename Raw8<T>::type raw8;
+  extern __shared__ float smem[];
+  constexpr int kPitch = 2 * GT_ * kStepOut + 4;      // (+ 4: the groups of a wave write to banks of their own)
+  float* red = smem;                                  // [32 groups][2 gates][GT_][64], kPitch apart
+  float* red2 = red + 32 * kPitch;                    // [2 gates][GT_][64]
+  float* ubs = red2 + 2 * GT_ * kStepOut;             // [GT_][bw] convolved inputs
+  T* tail = (T*)(ubs + GT_ * bw);                     // [GT_][taps - 1][bw] the new tail
+  __shared__ int last;
+  const int nz = (bw + kStepOut - 1) / kStepOut;
+  const int b = blockIdx.x / nz, o0 = (blockIdx.x % nz) * kStepOut;
+  const int s0 = blockIdx.y * GT_, C = nb * bw;
+  const int tid = threadIdx.x, og = tid & 7, kg = tid >> 3;
+  const int ob = min(o0 + 8 * og, bw - 8);            // this lane's 8 outputs (past the block: repeated, never used)
+  const T* ra = (const T*)ra_t_ + (size_t)b * bw * bw + ob;
+  const T* ri = (const T*)ri_t_ + (size_t)b * bw * bw + ob;
+  raw8 wr[kRows], wi[kRows];
+  auto load_rows = [&](int i0) {
+#pragma unroll
+    for (int q = 0; q < kRows; ++q) {
+      const size_t at = (size_t)min(i0 + 32 * q, bw - 1) * bw;
+      wr[q] = *reinterpret_cast<const raw8*>(ra + at);
+      wi[q] = *reinterpret_cast<const raw8*>(ri + at);
+    }
+  };
+  // every load off a clamped place and none behind a branch (hipcc waits out a load inside a branch, uniform or not,
+  // before the next: 15 round trips, 5 us).  A lane's first channel, what the finishing threads (output fo of sequence fk)
+  // need, and the first round of weights go out together
+  const int fk = __builtin_amdgcn_readfirstlane(tid >> 6), fo = o0 + (tid & 63), fq = min(s0 + min(fk, GT_ - 1), seqs - 1);
+  const bool fin = fk < GT_ && s0 + fk < seqs && fo < bw;
+  const int fc = b * bw + min(fo, bw - 1);
+  float* fstate = state + (size_t)slots[fq] * C + fc;
+  int pos[GT_], slot[GT_];
+#pragma unroll
+  for (int k = 0; k < GT_; ++k) {
+    const int q = min(s0 + k, seqs - 1);                        // past the last sequence: repeated, never used
+    pos[k] = positions[q], slot[k] = slots[q];
+  }
+  T w[TAPS_], v[GT_][TAPS_], xb, cb;
+  auto load_taps = [&](int c) {
+    xb = ((const T*)x_b_)[c], cb = ((const T*)conv_b_)[c];
+#pragma unroll
+    for (int j = 0; j < TAPS_; ++j) w[j] = ((const T*)conv_w_)[(size_t)min(j, taps - 1) * C + c];
+#pragma unroll
+    for (int k = 0; k < GT_; ++k) {
+      const T* st = (const T*)conv_state_ + (size_t)slot[k] * (taps - 1) * C + c;
+      const T* xr = (const T*)x_ + (size_t)min(s0 + k, seqs - 1) * ld + c;
+#pragma unroll
+      for (int j = 0; j < TAPS_; ++j) v[k][j] = *(j < taps - 1 ? st + (size_t)j * C : xr);
+    }
+  };
+  load_taps(b * bw + min(tid, bw - 1));
+  const float s_in = *fstate;
+  const T y_in = ((const T*)y_)[(size_t)fq * ld + fc], y_b = ((const T*)y_b_)[fc], lam = ((const T*)lam_)[fc];
+  const T rb = ((const T*)ra_b_)[fc], ib = ((const T*)ri_b_)[fc];
+  const int fpos = positions[fq];
+  load_rows(kg);
+
+  // convolution of the block's channels, a lane per channel; the new tail (the old one a row up, then x) waits in LDS
+  for (int ci = tid; ci < bw; ci += 256) {
+    if (ci != tid) load_taps(b * bw + ci);
+#pragma unroll
+    for (int k = 0; k < GT_; ++k) {
+      float acc = (float)cb;
+#pragma unroll
+      for (int j = 0; j < TAPS_; ++j) {
+        if (j < taps) {
+          const bool live = taps - 1 - j <= pos[k];             // the row lies at or after the sequence's start
+          const T z = live ? v[k][j] : (T)0.f;
+          if (live) acc += (float)w[j] * ((float)z + (float)xb);
+          if (j > 0) tail[(size_t)(k * (taps - 1) + j - 1) * bw + ci] = z;
+        }
+      }
+      ubs[k * bw + ci] = acc;
+    }
+  }
+  __syncthreads();                                    // every read of the old tail in this workgroup has returned
+  // (counters on lines of their own; the answer is not needed before the end)
+  int* count = arrived + (size_t)(blockIdx.y * nb + b) * kCountStride;
+  int before = 0;
+  if (tid == 0) before = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+
+  float ar[GT_][8], ai[GT_][8];
+#pragma unroll
+  for (int k = 0; k < GT_; ++k)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) ar[k][j] = 0.f, ai[k][j] = 0.f;
+  for (int i0 = kg; i0 < bw; i0 += 32 * kRows) {
+    if (i0 > kg) load_rows(i0);
+#pragma unroll
+    for (int q = 0; q < kRows; ++q) {
+      const int base = i0 - kg + 32 * q, i = base + kg;         // base: uniform
+      if (base < bw) {
+        float fr[8], fi[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          fr[j] = (float)wr[q][j], fi[j] = (float)wi[q][j];
+          if (base + 32 > bw) fr[j] = i < bw ? fr[j] : 0.f, fi[j] = i < bw ? fi[j] : 0.f;   // a last, partial round
+        }
+#pragma unroll
+        for (int k = 0; k < GT_; ++k) {
+          const float u = i < bw ? ubs[k * bw + min(i, bw - 1)] : 0.f;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) ar[k][j] = fmaf(fr[j], u, ar[k][j]), ai[k][j] = fmaf(fi[j], u, ai[k][j]);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < GT_; ++k)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      float* r0 = red + kg * kPitch + k * kStepOut + 8 * og + 4 * h;
+      float* r1 = red + kg * kPitch + (GT_ + k) * kStepOut + 8 * og + 4 * h;
+      *reinterpret_cast<f32x4*>(r0) = f32x4{ar[k][4 * h], ar[k][4 * h + 1], ar[k][4 * h + 2], ar[k][4 * h + 3]};
+      *reinterpret_cast<f32x4*>(r1) = f32x4{ai[k][4 * h], ai[k][4 * h + 1], ai[k][4 * h + 2], ai[k][4 * h + 3]};
+    }
+  __syncthreads();
+  for (int e = tid; e < 2 * GT_ * kStepOut; e += 256) {         // (gate, sequence, output): the 32 groups in order
+    float sum = 0.f;
+#pragma unroll
+    for (int g = 0; g < 32; ++g) sum += red[g * kPitch + e];
+    red2[e] = sum;
+  }
+  if (tid == 0) last = before == nz - 1;
+  __syncthreads();
+  if (fin) {
+    const float sr = red2[fk * kStepOut + (tid & 63)], si = red2[(GT_ + fk) * kStepOut + (tid & 63)];
+    const float av = expf(-scale * sigmoid_f(sr + (float)rb) * softplus_f((float)lam));
+    const float gv = sqrtf(1.0f - av * av) * sigmoid_f(si + (float)ib) * ubs[fk * bw + fo];
+    const float s = fmaf(av, fpos > 0 ? s_in : 0.f, gv);
+    *fstate = s;
+    stf((T*)out_ + (size_t)fq * C + b * bw + fo, s * gelu_tanh_f((float)y_in + (float)y_b));
+  }
+  if (last) {                                         // uniform
+    for (int i = tid; i < GT_ * bw; i += 256) {
+      const int k = GT_ == 1 ? 0 : i / bw, ci = i - k * bw, q = s0 + k;
+      if (q < seqs) {
+        T* st = (T*)conv_state_ + (size_t)slots[q] * (taps - 1) * C + b * bw + ci;
+        for (int j = 0; j < taps - 1; ++j) st[(size_t)j * C] = tail[(size_t)(k * (taps - 1) + j) * bw + ci];
+      }
+    }
+    if (tid == 0) *count = 0;
+  }
+}
+
+// Every sequence brings one token, token q of the batch is sequence q's.  x / y: the two halves of the projection (rows
+// ld apart); out [tokens, C]; arrived: sequences x blocks zeroed counters, 32 ints apart, that no other launch uses
+// meanwhile (left zeroed).
+void sm_rglru_step(uintptr_t out, uintptr_t x, uintptr_t y, long ld, uintptr_t conv_w, uintptr_t conv_b, uintptr_t x_b,
+                   uintptr_t conv_state, uintptr_t ra_t, uintptr_t ra_b, uintptr_t ri_t, uintptr_t ri_b, uintptr_t lam,
+                   uintptr_t y_b, uintptr_t state, uintptr_t positions, uintptr_t slots, int seqs, int nb,
+                   int bw, int taps, float scale, uintptr_t arrived, int arrived_len, int f32, uintptr_t stream) {
+  if (seqs <= 0) return;
+  DLLM_HOST_CHECK(nb > 0 && bw >= 8 && bw % 8 == 0 && bw <= 512 && (long)nb * bw <= (1L << 24), "rglru step block sizes");
+  DLLM_HOST_CHECK(taps >= 1 && taps <= kStepTaps && ld >= (long)nb * bw, "rglru step sizes");
+  // sequences per workgroup: two halve the passes over the matrices, which the L2 bears while the grid is small (10 blocks
+  // of 256 at 16 sequences: 9.1 us with one, 10.0 with two; at 64: 20.9 and 20.0)
+  const int gt = seqs <= 32 ? 1 : 2;
+  const int groups = (seqs + gt - 1) / gt;
+  DLLM_HOST_CHECK(arrived != 0 && (long)groups * nb * kCountStride <= arrived_len && groups <= 65535, "rglru step counters");
+  const size_t lds = ((size_t)(33 * 2 * gt * kStepOut + 32 * 4) + (size_t)gt * bw) * sizeof(float) +
+                     (size_t)gt * (taps - 1) * bw * (f32 ? 4 : 2);
+  // consecutive workgroups run on consecutive XCDs: the (block, output) index first, so that with 8 or more of them a
+  // weight tile is read into the L2 of as few XCDs as can be
+  const dim3 grid(nb * ((bw + kStepOut - 1) / kStepOut), groups);
+#define SM_STEP(T, G_, N_)                                                                                                \
+  do {                                                                                                               \
+    if (lds > 64 * 1024)                                                                                             \
+      DLLM_HIP_CHECK(hipFuncSetAttribute((const void*)sm_rglru_step_kernel<T, G_, N_>,                                    \
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));                      \
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(sm_rglru_step_kernel<T, G_, N_>), grid, dim3(256), lds, (hipStream_t)stream,       \
+                       (void*)out, (const void*)x, (const void*)y, ld, (const void*)conv_w, (const void*)conv_b,      \
+                       (const void*)x_b, (void*)conv_state, (const void*)ra_t, (const void*)ra_b, (const void*)ri_t,  \
+                       (const void*)ri_b, (const void*)lam, (const void*)y_b, (float*)state,                          \
+                       (const int32_t*)positions, (const int32_t*)slots, seqs, nb, bw, taps, scale, (int*)arrived);   \
+  } while (0)
+#define SM_STEP_T(T)                                            \
+  do {                                                          \
+    if (gt == 1 && taps <= 4) SM_STEP(T, 1, 4);                 \
+    else if (gt == 1) SM_STEP(T, 1, kStepTaps);                 \
+    else if (taps <= 4) SM_STEP(T, 2, 4);                       \
+    else SM_STEP(T, 2, kStepTaps);                              \
+  } while (0)
+  if (f32) SM_STEP_T(float);
+  else SM_STEP_T(bf16);
+#undef SM_STEP_T
+#undef SM_STEP
+  DLLM_HIP_CHECK(hipGetLastError());
+}
+
 // --------------------------------------------------------------------------- clipped GLU
 template <typename T, int V>
 __global__ void __launch_bounds__(256) sm_clipped_glu_kernel(void* __restrict__ out_, const void* __restrict__ gu_,
@@ -1257,15 +1570,16 @@ __global__ void __launch_bounds__(64) sm_attn_prep_kernel(
 // reads 2-element vectors, the rotation needs no exchange through LDS, and q / k leave as 2-element
 // stores.  Heads up to 512 wide (4 pairs per lane).
 constexpr int kPrepPairs = 4;
+constexpr int kTailTaps = 4;
 
 template <typename T>
 __global__ void __launch_bounds__(256) sm_attn_prep_pair_kernel(
     void* __restrict__ q_out_, const void* __restrict__ qkv_, const void* __restrict__ conv_w_,
-    const void* __restrict__ state_, const void* __restrict__ q_norm_, const void* __restrict__ k_norm_,
+    const void* state_, const void* __restrict__ q_norm_, const void* __restrict__ k_norm_,
     const float* __restrict__ freqs, int nrot, float mag, float eps, void* __restrict__ k_cache_,
     void* __restrict__ v_cache_, const int32_t* __restrict__ slot_mapping, const int32_t* __restrict__ cu,
     const int32_t* __restrict__ positions, const int32_t* __restrict__ tok_seq, const int32_t* __restrict__ slots,
-    int H, int G, int D, int Dv, int taps, int bs) {
+    int H, int G, int D, int Dv, int taps, int bs, void* tail_) {
   const int t = blockIdx.x, head = blockIdx.y * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;   // a wave per head
   if (head >= H + 2 * G) return;
   const int C = H * D + G * (D + Dv);
@@ -1286,6 +1600,25 @@ __global__ void __launch_bounds__(256) sm_attn_prep_pair_kernel(
     x[r][0] = x[r][1] = 0.f;
     if (e < n) {
       const int c = c0 + e;
+      if (tail_) {                                   // one token per sequence, taps <= kTailTaps: the tail moves up here
+        T* sn = (T*)tail_ + (size_t)slots[b] * (taps - 1) * C + c;
+        float xv[kTailTaps][2], wv[kTailTaps][2];
+#pragma unroll
+        for (int j = 0; j < kTailTaps; ++j) {
+          const int jj = min(j, taps - 1);
+          ldv<2>(w + (size_t)jj * C + c, wv[j]);
+          ldv<2>(jj == taps - 1 ? qkv + (size_t)t * C + c : (const T*)sn + (size_t)jj * C, xv[j]);
+        }
+#pragma unroll
+        for (int j = 0; j < kTailTaps; ++j) {
+          if (j < taps) {
+            if (taps - 1 - j > pos) xv[j][0] = xv[j][1] = 0.f;
+            x[r][0] += wv[j][0] * xv[j][0];
+            x[r][1] += wv[j][1] * xv[j][1];
+            if (j > 0) stv<2>(sn + (size_t)(j - 1) * C, xv[j]);
+          }
+        }
+      } else
       for (int j = 0; j < taps; ++j) {
         const int d = taps - 1 - j;
         if (d > pos) continue;
@@ -1343,7 +1676,7 @@ __global__ void __launch_bounds__(256) sm_attn_prep_pair_kernel(
 void sm_attn_prep(uintptr_t q_out, uintptr_t qkv, uintptr_t conv_w, uintptr_t state, uintptr_t q_norm,
                   uintptr_t k_norm, uintptr_t freqs, int nrot, float mag, float eps, uintptr_t k_cache,
                   uintptr_t v_cache, uintptr_t slot_mapping, uintptr_t cu, uintptr_t positions, uintptr_t tok_seq,
-                  uintptr_t slots, int tokens, int seqs, int H, int G, int D, int Dv, int taps, int bs, int f32,
+                  uintptr_t slots, int tokens, int seqs, int H, int G, int D, int Dv, int taps, int bs, int max_q_len, int f32,
                   uintptr_t stream) {
   if (tokens <= 0 || seqs <= 0) return;
   DLLM_HOST_CHECK(H > 0 && G >= 0 && D > 0 && Dv > 0 && taps >= 1 && bs > 0 && 2 * nrot <= D, "attn_prep sizes");
@@ -1351,19 +1684,23 @@ void sm_attn_prep(uintptr_t q_out, uintptr_t qkv, uintptr_t conv_w, uintptr_t st
   DLLM_HOST_CHECK(H + 2 * G <= 65535, "attn_prep heads");
   const int C = H * D + G * (D + Dv);
   const size_t lds = (size_t)std::max(D, Dv) * sizeof(float);
-  if (D % 2 == 0 && Dv % 2 == 0 && std::max(D, Dv) <= 128 * kPrepPairs)
+  const bool pairs = D % 2 == 0 && Dv % 2 == 0 && std::max(D, Dv) <= 128 * kPrepPairs;
+  // one token per sequence: a channel of a sequence's tail is read and moved up by the one lane that convolves it, so the
+  // tail needs no launch of its own (4.6 us)
+  const bool tail = pairs && max_q_len == 1 && taps > 1 && taps <= kTailTaps;
+  if (pairs)
     SM_DISPATCH(f32, sm_attn_prep_pair_kernel, dim3(tokens, (H + 2 * G + 3) / 4), dim3(256), 0, stream, (void*)q_out,
                 (const void*)qkv, (const void*)conv_w, (const void*)state, (const void*)q_norm, (const void*)k_norm,
                 (const float*)freqs, nrot, mag, eps, (void*)k_cache, (void*)v_cache, (const int32_t*)slot_mapping,
                 (const int32_t*)cu, (const int32_t*)positions, (const int32_t*)tok_seq, (const int32_t*)slots, H, G, D,
-                Dv, taps, bs);
+                Dv, taps, bs, tail ? (void*)state : nullptr);
   else
   SM_DISPATCH(f32, sm_attn_prep_kernel, dim3(tokens, H + 2 * G), dim3(64), lds, stream, (void*)q_out, (const void*)qkv,
               (const void*)conv_w, (const void*)state, (const void*)q_norm, (const void*)k_norm, (const float*)freqs,
               nrot, mag, eps, (void*)k_cache, (void*)v_cache, (const int32_t*)slot_mapping, (const int32_t*)cu,
               (const int32_t*)positions, (const int32_t*)tok_seq, (const int32_t*)slots, H, G, D, Dv, taps, bs);
   // the projection's last taps - 1 rows of every sequence become its new tail
-  if (taps > 1)
+  if (taps > 1 && !tail)
     launch_conv_state(state, qkv, (long)C, cu, positions, slots, seqs, C, taps, f32, C % 8 == 0, stream);
 }
 

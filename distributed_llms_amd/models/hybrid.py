@@ -344,17 +344,21 @@ class HybridStage(LayerListStage):
         window = int((m.get("mask") or {}).get("size") or (1 << 30))          # no mask entry: plain causal attention
         scale = float(m["scale"]) if m.get("scale") is not None else m["dim"] ** -0.5
         a = sm.window_attention(q, kc, vc, meta.block_tables, sb, window, scale, num_decode=nd)
-        return ops.linear(a.view(a.shape[0], -1), w["wo"])
+        return ops.linear_into_norm(a.view(a.shape[0], -1), w["wo"])
 
     def _rglru(self, i: int, h: torch.Tensor, w, sb: sm.SeqBatch) -> torch.Tensor:
         m = self.specs[i]["mixer"]
         c = m["width"]
         yx = ops.linear(h, w["w_yx"])
         st = self.state[i]
+        if sm.one_token_each(sb) and sm.rglru_step_fits(m["blocks"], c // m["blocks"], m["conv"]):
+            r = sm.rglru_step(yx, w["conv_w"], w["conv_b"], w["x_b"], st["conv"], w["y_b"], w["ra_t"], w["ra_b"], w["ri_t"],
+                              w["ri_b"], w["lam"], st["s"], sb)
+            return ops.linear_into_norm(r, w["wo"])
         u = sm.causal_conv(yx[:, c:], w["conv_w"], w["conv_b"], st["conv"], sb, in_bias=w["x_b"])
         r = sm.rglru(u, yx[:, :c], w["y_b"], w["ra_t"], w["ra_b"], w["ri_t"], w["ri_b"], w["lam"], st["s"], sb,
                      self.dtype)
-        return ops.linear(r, w["wo"])
+        return ops.linear_into_norm(r, w["wo"])
 
     @torch.inference_mode()
     def forward(self, inp: torch.Tensor, meta: BatchMeta) -> torch.Tensor:
@@ -372,7 +376,7 @@ class HybridStage(LayerListStage):
             x, h = sm.post_norm_add(x, o, w["norm1b"], eps, mult, w_next=w["norm2"] if spec.get("mlp") else nxt)
             if spec.get("mlp"):
                 y = sm.linear_clipped_glu(h, w["w_gu"], w["b_gu"], spec["mlp"]["limit"])
-                x, h = sm.post_norm_add(x, ops.linear(y, w["w_down"]), w["norm2b"], eps, mult, bias=w["b_down"],
+                x, h = sm.post_norm_add(x, ops.linear_into_norm(y, w["w_down"]), w["norm2b"], eps, mult, bias=w["b_down"],
                                         w_next=nxt)
             if self.taps is not None:
                 self.taps.append(x.clone())

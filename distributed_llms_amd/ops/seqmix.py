@@ -138,7 +138,7 @@ def rms_norm_f32(x: torch.Tensor, w: torch.Tensor, eps: float, act_dtype, one_pl
     return y
 
 
-def post_norm_add(x: torch.Tensor, o: torch.Tensor, w_post: torch.Tensor, eps: float, mult: float,
+def post_norm_add(x: torch.Tensor, o, w_post: torch.Tensor, eps: float, mult: float,
                   bias: Optional[torch.Tensor] = None, w_next: Optional[torch.Tensor] = None, one_plus: bool = True,
                   o2: Optional[torch.Tensor] = None, scales=(1.0, 1.0), plain_next: bool = False):
     """The close of a sublayer, fused: ``x += mult * rms_norm(o + bias) * (1 + w_post)`` in place on the
@@ -146,7 +146,9 @@ def post_norm_add(x: torch.Tensor, o: torch.Tensor, w_post: torch.Tensor, eps: f
     ``rms_norm(x) * (1 + w_next)`` in ``o``'s dtype (None otherwise).  ``one_plus`` False: both norm
     weights are plain (``* w``).  ``o2``: the sublayer's output is ``scales[0] * o + scales[1] * o2`` (two
     mixers side by side).  ``plain_next`` (without ``w_next``): the next sublayer reads the stream itself;
-    returns it in ``o``'s dtype (the stream tensor when that is float32)."""
+    returns it in ``o``'s dtype (the stream tensor when that is float32).  ``o`` may be a :class:`~.gemm.SplitKPartial`
+    (without ``o2``): its slabs are then summed in the same launch."""
+    from .gemm import SplitKPartial
     off = 1.0 if one_plus else 0.0
     if not x.is_cuda:
         ob = o.float() if o2 is None else scales[0] * o.float() + scales[1] * o2.float()
@@ -157,16 +159,20 @@ def post_norm_add(x: torch.Tensor, o: torch.Tensor, w_post: torch.Tensor, eps: f
             return x, ((x if o.dtype == torch.float32 else x.to(o.dtype)) if plain_next else None)
         return x, _ref_rms(x, w_next, eps, off).to(o.dtype)
     _ck(x, "x", torch.float32)
-    _ck(o, "o")
     t, width = x.shape
-    if o.shape != x.shape or (o2 is not None and (o2.shape != x.shape or o2.dtype != o.dtype or not o2.is_contiguous())):
+    part = o if isinstance(o, SplitKPartial) else None
+    if part is not None and (o2 is not None or width % 4 or width > 16384):
+        o, part = part.materialize(), None
+    if part is None:
+        _ck(o, "o")
+    if tuple(o.shape) != tuple(x.shape) or (o2 is not None and (o2.shape != x.shape or o2.dtype != o.dtype or not o2.is_contiguous())):
         raise ValueError("post_norm_add: o / x shape mismatch")
     h = None
     if w_next is not None or (plain_next and o.dtype != torch.float32):
-        h = torch.empty_like(o)
-    _k().sm_post_norm_add(x.data_ptr(), o.data_ptr(), _ptr(bias), w_post.data_ptr(), _ptr(w_next), _ptr(h), t, width,
-                          float(eps), float(mult), off, _ptr(o2), float(scales[0]), float(scales[1]), _f32flag(o),
-                          _stream())
+        h = torch.empty(t, width, dtype=o.dtype, device=x.device)
+    _k().sm_post_norm_add(x.data_ptr(), (part.ws if part is not None else o).data_ptr(), 0 if part is None else part.splits, _ptr(bias), w_post.data_ptr(), _ptr(w_next), _ptr(h), t, width,
+                          float(eps), float(mult), off, _ptr(o2), float(scales[0]), float(scales[1]),
+                          1 if o.dtype == torch.float32 else 0, _stream())
     return x, (x if (plain_next and w_next is None and h is None) else h)
 
 
@@ -432,6 +438,59 @@ def rglru(u: torch.Tensor, y_raw: torch.Tensor, y_bias: torch.Tensor, ra_t: torc
     return out
 
 
+def one_token_each(sb: SeqBatch) -> bool:
+    """Every sequence of the batch brings exactly one token (token q is sequence q's)."""
+    return sb.max_q_len == 1 and sb.num_tokens == sb.num_seqs
+
+
+def rglru_step_fits(blocks: int, bw: int, taps: int) -> bool:
+    """Block widths and convolution lengths that :func:`rglru_step` takes."""
+    return 1 <= blocks and bw % 8 == 0 and 8 <= bw <= 512 and blocks * bw <= 1 << 24 and 1 <= taps <= 8
+
+
+_arrived = {}
+
+
+def _arrival_counts(device: torch.device, n: int) -> torch.Tensor:
+    """Zeroed counters of the current stream, which every launch leaves zeroed (launches on one stream follow each other;
+    graphs keep those of the stream they were captured on, as they do the split-K workspace)."""
+    key = (device.index or 0, torch.cuda.current_stream().cuda_stream)
+    t = _arrived.get(key)
+    if t is None or t.numel() < n:
+        t = _arrived[key] = torch.zeros(max(n, 1 << 16), dtype=torch.int32, device=device)
+    return t
+
+
+def rglru_step(yx: torch.Tensor, conv_w: torch.Tensor, conv_b: torch.Tensor, x_b: torch.Tensor, conv_state: torch.Tensor,
+               y_b: torch.Tensor, ra_t: torch.Tensor, ra_b: torch.Tensor, ri_t: torch.Tensor, ri_b: torch.Tensor,
+               lam: torch.Tensor, state: torch.Tensor, sb: SeqBatch, decay_scale: float = 8.0) -> torch.Tensor:
+    """The recurrent branch of a batch with one token per sequence: :func:`causal_conv` of the right half of ``yx`` [T, 2 C]
+    (bias ``x_b``; tail ``conv_state``) and :func:`rglru` of it with the left half as y, in one launch on the GPU."""
+    c = state.shape[1]
+    nb, bw, _ = ra_t.shape
+    taps = conv_w.shape[0]
+    if not one_token_each(sb) or yx.dim() != 2 or yx.shape[1] != 2 * c or nb * bw != c or not rglru_step_fits(nb, bw, taps):
+        raise ValueError("rglru_step: one token per sequence, blocks a multiple of 8 up to 512 wide, up to 8 taps")
+    if not yx.is_cuda:
+        u = causal_conv(yx[:, c:], conv_w, conv_b, conv_state, sb, in_bias=x_b)
+        return rglru(u, yx[:, :c], y_b, ra_t, ra_b, ri_t, ri_b, lam, state, sb, yx.dtype, decay_scale)
+    _ck(yx, "yx")
+    _ck(state, "state", torch.float32)
+    for n, t in (("conv_w", conv_w), ("conv_b", conv_b), ("x_b", x_b), ("conv_state", conv_state), ("y_b", y_b),
+                 ("ra_t", ra_t), ("ra_b", ra_b), ("ri_t", ri_t), ("ri_b", ri_b), ("lam", lam)):
+        _ck(t, n, yx.dtype)
+    if tuple(conv_w.shape) != (taps, c) or tuple(conv_state.shape[1:]) != (taps - 1, c) or tuple(ri_t.shape) != (nb, bw, bw):
+        raise ValueError("rglru_step: shape mismatch")
+    out = torch.empty(yx.shape[0], c, dtype=yx.dtype, device=yx.device)
+    e = yx.element_size()
+    arrived = _arrival_counts(yx.device, sb.num_seqs * nb * 32)
+    _k().sm_rglru_step(out.data_ptr(), yx.data_ptr() + c * e, yx.data_ptr(), yx.stride(0), conv_w.data_ptr(), conv_b.data_ptr(),
+                       x_b.data_ptr(), conv_state.data_ptr(), ra_t.data_ptr(), ra_b.data_ptr(), ri_t.data_ptr(),
+                       ri_b.data_ptr(), lam.data_ptr(), y_b.data_ptr(), state.data_ptr(), sb.positions.data_ptr(), sb.state_slots.data_ptr(), sb.num_seqs, nb, bw, taps, float(decay_scale),
+                       arrived.data_ptr(), arrived.numel(), _f32flag(yx), _stream())
+    return out
+
+
 # ------------------------------------------------------------------ clipped GLU / soft cap
 def clipped_glu(gu: torch.Tensor, bias_gu: Optional[torch.Tensor], limit: float, alpha: float = 1.702) -> torch.Tensor:
     """[T, 2F] = gate | up (+ bias): g = min(gate, limit), u = clamp(up, -limit, limit);
@@ -577,7 +636,7 @@ def attn_prep(qkv: torch.Tensor, conv_w: torch.Tensor, state: torch.Tensor, q_no
                       _ptr(v_cache), slot_mapping.data_ptr(), sb.cu.data_ptr(), sb.positions.data_ptr(),
                       sb.tok_seq.data_ptr(), sb.state_slots.data_ptr(), sb.num_tokens, sb.num_seqs, heads,
                       kv_heads if own_kv else 0, dim, vdim, taps, k_cache.shape[2] if own_kv else 1,
-                      _f32flag(qkv), _stream())
+                      int(sb.max_q_len), _f32flag(qkv), _stream())
     return q
 
 

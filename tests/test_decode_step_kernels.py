@@ -1,0 +1,112 @@
+"""One-launch decode steps of the layer-list models against the same steps done by the general kernels' CPU reference."""
+import numpy as np
+import pytest
+import torch
+
+from distributed_llms_amd.ops import gemm
+from distributed_llms_amd.ops import seqmix as sm
+
+gpu = pytest.mark.gpu
+
+
+def _sb(pos, slots, device):
+    n = len(pos)
+    i32 = lambda a: torch.tensor(a, dtype=torch.int32, device=device)
+    return sm.SeqBatch(i32(list(range(n + 1))), i32(pos), i32(list(range(n))), i32(slots), n, n, 1)
+
+
+@gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("nb,bw,taps", [(1, 8, 1), (3, 40, 2), (4, 256, 4), (2, 264, 8), (10, 256, 4), (1, 512, 3)])
+@pytest.mark.parametrize("seqs", [1, 5, 40, 141])
+def test_rglru_step(cuda, dtype, nb, bw, taps, seqs):
+    """One, two and four sequences per workgroup (an odd last one), blocks narrower and wider than 64 outputs and 256 rows, sequences
+    at positions 0, 1, 2 and later (parts of the tail do not exist yet), slots out of order."""
+    g = torch.Generator().manual_seed(seqs + bw)
+    c = nb * bw
+    r = lambda *s, scale=1.0: (torch.randn(*s, generator=g) * scale).to(dtype)
+    yx, cw, cb, xb, yb = r(seqs, 2 * c), r(taps, c, scale=0.5), r(c, scale=0.1), r(c, scale=0.1), r(c, scale=0.1)
+    ra, ri = r(nb, bw, bw, scale=bw ** -0.5), r(nb, bw, bw, scale=bw ** -0.5)
+    rab, rib, lam = r(nb, bw, scale=0.3), r(nb, bw, scale=0.3), r(c)
+    slots = (torch.randperm(seqs + 3, generator=g)[:seqs]).tolist()
+    pos = [[0, 1, 2, 3, 57][i % 5] for i in range(seqs)]
+    conv, state = r(seqs + 3, taps - 1, c), torch.randn(seqs + 3, c, generator=g)
+    conv_d, state_d = conv.cuda(), state.cuda()
+    d = lambda t: t.cuda()
+    conv_2, state_2 = conv_d.clone(), state_d.clone()            # a second launch finds the counters as the first did
+    again = sm.rglru_step(d(yx), d(cw), d(cb), d(xb), conv_2, d(yb), d(ra), d(rab), d(ri), d(rib), d(lam), state_2,
+                          _sb(pos, slots, "cuda"))
+    out = sm.rglru_step(d(yx), d(cw), d(cb), d(xb), conv_d, d(yb), d(ra), d(rab), d(ri), d(rib), d(lam), state_d,
+                        _sb(pos, slots, "cuda"))
+    ref = sm.rglru_step(yx, cw, cb, xb, conv, yb, ra, rab, ri, rib, lam, state, _sb(pos, slots, "cpu"))
+    assert torch.equal(conv_d, conv_2) and torch.equal(state_d, state_2) and torch.equal(out, again)
+    assert torch.equal(conv_d.cpu(), conv)                       # the tail is moved, not computed
+    # float32 sums of bw products in another order: the gates' arguments within bw 2^-24 of their terms (|u| |w| sum to
+    # a few units), times decay_scale softplus(lam) <= 30 through the exponential; sqrt(1 - a^2) steepens that near a = 1
+    np.testing.assert_allclose(state_d.cpu().numpy(), state.numpy(), atol=2e-4, rtol=2e-4)
+    tol = dict(atol=4e-4, rtol=4e-4) if dtype == torch.float32 else dict(atol=2e-3, rtol=2.0 ** -7)
+    np.testing.assert_allclose(out.float().cpu().numpy(), ref.float().numpy(), **tol)
+
+
+@gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("taps,dim,vdim", [(2, 32, 48), (3, 128, 128), (4, 10, 6), (5, 16, 16)])
+def test_attention_input_moves_the_tail(cuda, dtype, taps, dim, vdim):
+    """One token per sequence: q, caches and the convolution's new tail as the general form leaves them (taps 5: past the
+    one-launch form)."""
+    g = torch.Generator().manual_seed(taps)
+    heads, kvh, bs, pos = 6, 2, 16, [0, 1, 2, 3, 40]
+    c, n = heads * dim + kvh * (dim + vdim), 5
+    r = lambda *s: torch.randn(*s, generator=g).to(dtype)
+    qkv, cw, conv, qn, kn = r(n, c), r(taps, c), r(9, taps - 1, c), r(dim), r(dim)
+    freqs, slot_map = torch.rand(dim // 4, generator=g), torch.tensor([3, 17, 40, 5, 66], dtype=torch.int32)
+    got = []
+    for dev in ("cpu", "cuda"):
+        kc, vc = torch.zeros(5, kvh, bs, dim, dtype=dtype, device=dev), torch.zeros(5, kvh, vdim, bs, dtype=dtype, device=dev)
+        st = conv.to(dev, copy=True)
+        q = sm.attn_prep(qkv.to(dev), cw.to(dev), st, qn.to(dev), kn.to(dev), freqs.to(dev), 1.1, 1e-6, kc, vc, slot_map.to(dev),
+                         _sb(pos, [4, 2, 8, 1, 6], dev), heads, kvh, dim, vdim)
+        got.append([t.float().cpu() for t in (q, kc, vc)] + [st.cpu()])
+    tol = dict(atol=1e-4, rtol=1e-4) if dtype == torch.float32 else dict(atol=1e-2, rtol=2.0 ** -7)
+    for a, b in zip(*[x[:3] for x in got]):
+        torch.testing.assert_close(b, a, **tol)
+    assert torch.equal(got[0][3], got[1][3])
+
+
+@gpu
+@pytest.mark.parametrize("rows", [1, 7, 300])
+@pytest.mark.parametrize("width", [4, 250, 1024, 2560, 4100, 16384, 16392])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("form", ["next", "bias", "two", "plain"])
+def test_post_norm_add_rows(cuda, rows, width, dtype, form):
+    """The register-resident close of a sublayer at partial last pieces, odd widths and past its largest row."""
+    if rows == 300 and width > 4100:
+        return
+    g = torch.Generator().manual_seed(width)
+    r = lambda *s: torch.randn(*s, generator=g)
+    x, o, o2, b, wp, wn = r(rows, width), r(rows, width).to(dtype), r(rows, width).to(dtype), r(width).to(dtype), r(width).to(dtype), r(width).to(dtype)
+    kw = {"next": dict(w_next=wn), "bias": dict(bias=b, w_next=wn), "two": dict(o2=o2, scales=(0.9, 0.7), one_plus=False, w_next=wn),
+          "plain": dict(plain_next=True)}[form]
+    d = lambda v: v.cuda() if isinstance(v, torch.Tensor) else v
+    xr, hr = sm.post_norm_add(x.clone(), o, wp, 1e-6, 0.8, **kw)
+    xg, hg = sm.post_norm_add(x.cuda(), o.cuda(), wp.cuda(), 1e-6, 0.8, **{k: d(v) for k, v in kw.items()})
+    torch.testing.assert_close(xg.cpu(), xr, atol=2e-5, rtol=2e-5)
+    tol = dict(atol=5e-5, rtol=5e-5) if dtype == torch.float32 else dict(atol=1e-3, rtol=2.0 ** -7)
+    torch.testing.assert_close(hg.float().cpu(), hr.float(), **tol)
+
+
+@gpu
+@pytest.mark.parametrize("tokens,width,k", [(1, 256, 1024), (16, 2560, 7680), (40, 4096, 2048)])
+def test_post_norm_add_sums_split_products(cuda, tokens, width, k):
+    """On a split-K product that is not reduced yet, against the same on the reduced one: the slabs are summed in the same
+    order and rounded to bf16 before the norm, so both see the same numbers."""
+    a = torch.randn(tokens, k, device="cuda").bfloat16()
+    w = (torch.randn(width, k, device="cuda") * k ** -0.5).bfloat16()
+    wp, wn, b = (torch.randn(width, device="cuda").bfloat16() for _ in range(3))
+    part = gemm.linear_wide(a, w, defer=True)
+    assert isinstance(part, gemm.SplitKPartial)
+    whole = part.materialize()
+    x0 = torch.randn(tokens, width, device="cuda")
+    got = sm.post_norm_add(x0.clone(), part, wp, 1e-5, 0.7, bias=b, w_next=wn)
+    want = sm.post_norm_add(x0.clone(), whole, wp, 1e-5, 0.7, bias=b, w_next=wn)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
