@@ -169,73 +169,71 @@ struct RopeArgs {
   long slab = 0;
 };
 
-// 8 consecutive qkv elements starting at row offset `off` of sequence b (bf16 or summed partials).
-// NP (0 = bf16 qkv, > 0 = that many slabs, -1 = runtime count) is a compile-time choice: a runtime
-// branch here split the kernel's prologue into blocks
-// with vmcnt(0) waits at every merge (cold B=256: 48 us vs 40 us without the fused part).
-template <int NP>
-__device__ __forceinline__ bf16x8 qkv_load8(const RopeArgs& ra, int b, int width, int off) {
-  if constexpr (NP == 0) return *reinterpret_cast<const bf16x8*>(ra.qkv + (size_t)b * width + off);
-  const size_t p = (size_t)b * width + off;
-  f32x4 a0 = {0.f, 0.f, 0.f, 0.f}, a1 = {0.f, 0.f, 0.f, 0.f};
-  if constexpr (NP > 0) {
-    // compile-time slab count: all 2 * NP loads in flight before the first add (a runtime loop
-    // waits on each slab in turn: NP dependent round trips in front of the KV stream)
-    f32x4 l0[NP], l1[NP];
+// W (8 or 2) consecutive qkv elements of a row in their stored form -- load() -- and as the bf16 values that the rest
+// works with -- value(), slabs summed in slab order as splitk_reduce sums them.  The two are apart so that the prologue
+// has every load under way before it waits for one.  NP: 0 = bf16 qkv, > 0 = that many slabs, -1 = a runtime count
+// (summed as it is loaded), a compile-time choice: a runtime branch split the prologue into blocks with vmcnt(0) waits
+// at every merge (cold B=256: 48 us vs 40 us without the fused part).
+template <int NP, int W>
+struct QkvPiece {
+  typedef bf16 vec __attribute__((ext_vector_type(W)));
+  typedef part_elem raw __attribute__((ext_vector_type(W)));
+  vec q;
+  raw l[NP > 0 ? NP : 1];
+  __device__ __forceinline__ void load(const RopeArgs& ra, size_t p) {
+    if constexpr (NP == 0) {
+      q = *reinterpret_cast<const vec*>(ra.qkv + p);
+    } else if constexpr (NP > 0) {
 #pragma unroll
-    for (int s = 0; s < NP; ++s) {
-      l0[s] = part_load4(ra.part, p + s * ra.slab);
-      l1[s] = part_load4(ra.part, p + s * ra.slab + 4);
-    }
+      for (int s = 0; s < NP; ++s)
+        l[s] = *reinterpret_cast<const raw*>(reinterpret_cast<const part_elem*>(ra.part) + p + s * ra.slab);
+    } else {
+      float a[W] = {};
+      for (int s = 0; s < ra.nparts; ++s) {
+        const raw v = *reinterpret_cast<const raw*>(reinterpret_cast<const part_elem*>(ra.part) + p + s * ra.slab);
 #pragma unroll
-    for (int s = 0; s < NP; ++s) {     // slab order as splitk_reduce: bit-identical sums
-      a0 += l0[s];
-      a1 += l1[s];
-    }
-  } else {
-    for (int s = 0; s < ra.nparts; ++s) {
-      a0 += part_load4(ra.part, p + s * ra.slab);
-      a1 += part_load4(ra.part, p + s * ra.slab + 4);
+        for (int j = 0; j < W; ++j) a[j] += part_value(v[j]);
+      }
+#pragma unroll
+      for (int j = 0; j < W; ++j) q[j] = f2bf(a[j]);
     }
   }
-  bf16x8 o;
+  __device__ __forceinline__ vec value() const {
+    if constexpr (NP <= 0) return q;
+    vec o;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    o[j] = f2bf(a0[j]);
-    o[j + 4] = f2bf(a1[j]);
+    for (int j = 0; j < W; ++j) {
+      float a = 0.f;
+#pragma unroll
+      for (int s = 0; s < NP; ++s) a += part_value(l[s][j]);
+      o[j] = f2bf(a);
+    }
+    return o;
   }
-  return o;
-}
+};
 
-template <int NP>
-__device__ __forceinline__ bf16 qkv_load1(const RopeArgs& ra, int b, int width, int off) {
-  if constexpr (NP == 0) return ra.qkv[(size_t)b * width + off];
-  const size_t p = (size_t)b * width + off;
-  float a = 0.f;
-  if constexpr (NP > 0) {
-    float l[NP];
+// one lane group's cos / sin values of a row
+template <int D>
+struct RopeRow {
+  f32x4 c[D / 64][2], s[D / 64][2];
+  __device__ __forceinline__ void load(const float* cs, int g) {
 #pragma unroll
-    for (int s = 0; s < NP; ++s) l[s] = part_load1(ra.part, p + s * ra.slab);
+    for (int ks = 0; ks < D / 64; ++ks)
 #pragma unroll
-    for (int s = 0; s < NP; ++s) a += l[s];
-  } else {
-    for (int s = 0; s < ra.nparts; ++s) a += part_load1(ra.part, p + s * ra.slab);
+      for (int h = 0; h < 2; ++h) {
+        c[ks][h] = *reinterpret_cast<const f32x4*>(cs + ks * 32 + 8 * g + 4 * h);
+        s[ks][h] = *reinterpret_cast<const f32x4*>(cs + D / 2 + ks * 32 + 8 * g + 4 * h);
+      }
   }
-  return f2bf(a);
-}
+};
 
-template <int D, bool FUSED>
-__device__ __forceinline__ void rope_rotate(bf16x8 (&f)[D / 32], const float* cs, int g) {
-  if (cs == nullptr) return;
+template <int D>
+__device__ __forceinline__ void rope_rotate(bf16x8 (&f)[D / 32], const RopeRow<D>& row) {
 #pragma unroll
   for (int ks = 0; ks < D / 64; ++ks) {
-    const f32x4 c0 = *reinterpret_cast<const f32x4*>(cs + ks * 32 + 8 * g);
-    const f32x4 c1 = *reinterpret_cast<const f32x4*>(cs + ks * 32 + 8 * g + 4);
-    const f32x4 s0 = *reinterpret_cast<const f32x4*>(cs + D / 2 + ks * 32 + 8 * g);
-    const f32x4 s1 = *reinterpret_cast<const f32x4*>(cs + D / 2 + ks * 32 + 8 * g + 4);
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      const float c = j < 4 ? c0[j] : c1[j - 4], s = j < 4 ? s0[j] : s1[j - 4];
+      const float c = row.c[ks][j >> 2][j & 3], s = row.s[ks][j >> 2][j & 3];
       const float a = bf2f(f[ks][j]), b = bf2f(f[ks + D / 64][j]);
       // explicit FMAs: left to hipcc's default contraction, the fused / unfused choice here may
       // differ between kernel instantiations, and the bf16-qkv and split-K-slab forms of the fused
@@ -258,37 +256,106 @@ __global__ void __launch_bounds__(WPB * 64, 2) attn_decode_kernel(   // 2nd arg:
   const int nsplit = gridDim.x;
   const int G = hq / hkv;
   const int r = lane & 15, g = lane >> 4;
-  // the prologue's dependency roots go out first, back to back (vmcnt retires in issue order):
-  // this sequence's position (its cos / sin row), its context length and this split's first 64
-  // block ids -- not guarded by the context, so they need not wait for it -- and one round trip
-  // later every address the prologue loads from is known
+  // Two round trips to memory precede the first MFMA: the sequence's position, its context length, this split's first 64
+  // block ids (not guarded by the context) and the projection's q go out together; what hangs on them -- the first KV
+  // chunk, the cos / sin row and, in the split that owns the new key, its k and v -- follows before anything is summed or
+  // rotated.  (hipcc, left to order the loads, summed q, k and v in four rounds before the first KV load and loaded the
+  // cos / sin row after it; every split read k and v, v as 2-byte pieces.)
   const int pos_b = FUSED ? ra.positions[b] : 0;
   const int ctx = seq_lens[b];
   const int kbeg = split * split_len;
   const int32_t* bt = block_tables + (size_t)b * max_blocks;
-  const int blk_first = lane < min(64, max_blocks - kbeg / kBS) ? bt[kbeg / kBS + lane] : 0;
+  const int blk_first = bt[min(kbeg / kBS + lane, max_blocks - 1)];
   // FUSED: the new key (ctx - 1) is not in the cache yet: its chunk is loaded as usual and the
   // key's K row / V^T column are replaced in registers by the rotated k and v (the split that
   // owns it also appends them to the cache, after its last KV load)
   const bool owns_new = FUSED && ctx > 0 && (ctx - 1) / split_len == split;
   const int kend = min(kbeg + split_len, ctx);     // exclusive
   const int c0 = kbeg / kBS, c1 = kend > kbeg ? (kend + kBS - 1) / kBS : c0;
+  const size_t kv_head_stride = (size_t)kBS * D;
+  const size_t head_off = (size_t)kvh * kv_head_stride;
+  const size_t blk_stride = (size_t)hkv * kv_head_stride;
 
   // Q^T fragments: column r = head kvh*G + r (zero beyond G)
   bf16x8 qf[D / 32];
   const bool col_ok = r < G;
   bf16x8 kn[D / 32];
   bf16 vn[D / 16];
-  if (FUSED) {
-    const int width = (hq + 2 * hkv) * D;
-    const int qo = (kvh * G + (col_ok ? r : 0)) * D, ko = (hq + kvh) * D, vo = (hq + hkv + kvh) * D;
+  KVChunk<D> cur, nxt;
+  auto load_at = [&](KVChunk<D>& c, int blk) {
+    const size_t base = (size_t)blk * blk_stride + head_off;
+    load_chunk<D, true>(c, k_cache + base, v_cache + base, lane);
+  };
+  auto write_out = [&](const WaveState<D>& st, float lt) {
+    if (!col_ok) return;
+    const int h = kvh * G + r;
+    if (nsplit == 1) {
+      // a true division, exactly as the split-reduce computes num / den (bit-identical results
+      // whether a sequence's keys land in one split or in one non-empty split of several)
+      bf16* orow = out + ((size_t)b * hq + h) * D;
 #pragma unroll
-    for (int ks = 0; ks < D / 32; ++ks) {
-      qf[ks] = qkv_load8<PARTS>(ra, b, width, qo + ks * 32 + 8 * g);
-      kn[ks] = qkv_load8<PARTS>(ra, b, width, ko + ks * 32 + 8 * g);
+      for (int dt = 0; dt < D / 16; ++dt) {
+        bf16x4 o;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float v = st.acc[dt][i] / (lt > 0.f ? lt : 1.f);      // divided either way: no branch around each
+          o[i] = f2bf(lt > 0.f ? v : 0.f);
+        }
+        *reinterpret_cast<bf16x4*>(orow + dt * 16 + 4 * g) = o;
+      }
+    } else {
+      const size_t pi = ((size_t)b * hq + h) * nsplit + split;
+      float* po = part_o + pi * D;
+#pragma unroll
+      for (int dt = 0; dt < D / 16; ++dt) *reinterpret_cast<f32x4*>(po + dt * 16 + 4 * g) = st.acc[dt];
+      if (g == 0) { part_ml[pi * 2] = st.m; part_ml[pi * 2 + 1] = lt; }
     }
+  };
+  WaveState<D> st;
+  init_state(st);
+  if (c1 == c0) {                                   // wave-uniform: no key in this split (and not the new one)
+    write_out(st, 0.f);
+    return;
+  }
+  const int blk_0 = __builtin_amdgcn_readlane(blk_first, 0);
+  if constexpr (FUSED) {
+    const size_t row = (size_t)b * (hq + 2 * hkv) * D;
+    QkvPiece<PARTS, 8> qp[D / 32];
+    QkvPiece<PARTS, 2> kp, vp;      // the new key's k and v, two elements per lane
+    RopeRow<D> rr;
 #pragma unroll
-    for (int dt = 0; dt < D / 16; ++dt) vn[dt] = qkv_load1<PARTS>(ra, b, width, vo + dt * 16 + r);
+    for (int ks = 0; ks < D / 32; ++ks) qp[ks].load(ra, row + (size_t)(kvh * G + (col_ok ? r : 0)) * D + ks * 32 + 8 * g);
+    load_at(cur, blk_0);
+    const int pair = 2 * (lane & (D / 2 - 1));
+    kp.load(ra, row + (size_t)(hq + kvh) * D + pair);     // (in every split: under a branch hipcc would wait for it there)
+    vp.load(ra, row + (size_t)(hq + hkv + kvh) * D + pair);
+    if (ra.cos_sin) rr.load(ra.cos_sin + (size_t)pos_b * D, g);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int ks = 0; ks < D / 32; ++ks) qf[ks] = qp[ks].value();
+    if (ra.cos_sin) rope_rotate<D>(qf, rr);
+    if (!col_ok) {
+#pragma unroll
+      for (int ks = 0; ks < D / 32; ++ks) qf[ks] = bf16x8{};
+    }
+    if (owns_new) {                 // wave-uniform; each lane takes its elements from the lanes that hold them
+      const int kw = __builtin_bit_cast(int, kp.value()), vw = __builtin_bit_cast(int, vp.value());
+#pragma unroll
+      for (int ks = 0; ks < D / 32; ++ks) {
+        typedef int i32x4 __attribute__((ext_vector_type(4)));
+        i32x4 w;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) w[i] = __builtin_amdgcn_ds_bpermute(4 * (ks * 16 + 4 * g + i), kw);
+        kn[ks] = __builtin_bit_cast(bf16x8, w);
+      }
+      typedef bf16 bf16x2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+      for (int dt = 0; dt < D / 16; ++dt) {
+        const bf16x2 two = __builtin_bit_cast(bf16x2, __builtin_amdgcn_ds_bpermute(4 * (dt * 8 + (r >> 1)), vw));
+        vn[dt] = r & 1 ? two[1] : two[0];
+      }
+      if (ra.cos_sin) rope_rotate<D>(kn, rr);
+    }
   } else {
     const bf16* qrow = q + ((size_t)b * hq + kvh * G + (col_ok ? r : 0)) * D;
 #pragma unroll
@@ -297,21 +364,8 @@ __global__ void __launch_bounds__(WPB * 64, 2) attn_decode_kernel(   // 2nd arg:
       if (!col_ok) v = bf16x8{};
       qf[ks] = v;
     }
+    load_at(cur, blk_0);
   }
-  // FUSED: rotate q/k and append k/v AFTER the first KV chunk's loads are issued, so the
-  // cos / sin -> rotate dependency overlaps the KV stream instead of preceding it
-  bool rope_done = !FUSED;
-  auto finish_rope = [&]() {
-    if (!FUSED || rope_done) return;
-    rope_done = true;
-    const float* cs = ra.cos_sin ? ra.cos_sin + (size_t)pos_b * D : nullptr;   // pos_b: loaded first
-    rope_rotate<D, FUSED>(qf, cs, g);
-    rope_rotate<D, FUSED>(kn, cs, g);
-    if (!col_ok) {
-#pragma unroll
-      for (int ks = 0; ks < D / 32; ++ks) qf[ks] = bf16x8{};
-    }
-  };
   // FUSED: put the new key into the registers of its chunk (lane masks inside that chunk only)
   const int cnew = FUSED ? (ctx - 1) / kBS : -1;
   const int noff = FUSED ? (ctx - 1) % kBS : 0;
@@ -319,7 +373,7 @@ __global__ void __launch_bounds__(WPB * 64, 2) attn_decode_kernel(   // 2nd arg:
     if (!FUSED) return;
     // wave-uniform (ctx and the chunk index live in SGPRs): every other chunk skips the ~140 lane
     // selects below on a scalar branch instead of running them as no-ops
-    if (!(ctx > 0 && chunk == cnew)) return;
+    if (!(owns_new && chunk == cnew)) return;
     // (two static selects: a runtime choice between ka and kb made hipcc index them through scratch)
     const int prow = krow32(noff);                    // physical K row of the new key
     const bool krow = r == (prow & 15);
@@ -348,42 +402,38 @@ __global__ void __launch_bounds__(WPB * 64, 2) attn_decode_kernel(   // 2nd arg:
       }
     }
   };
-  WaveState<D> st;
-  init_state(st);
   const int kmax = kend - 1;
-  const size_t kv_head_stride = (size_t)kBS * D;
-  const size_t head_off = (size_t)kvh * kv_head_stride;
-  const size_t blk_stride = (size_t)hkv * kv_head_stride;
+  int my_blk = blk_first;
   for (int cb = c0; cb < c1; cb += 64) {            // 64 chunks (2048 keys) of block ids per pass
     const int n = min(64, c1 - cb);
-    const int my_blk = cb == c0 ? blk_first : (lane < n ? bt[cb + lane] : 0);
-    KVChunk<D> cur, nxt;
-    {
-      const size_t base = (size_t)__builtin_amdgcn_readlane(my_blk, 0) * blk_stride + head_off;
-      load_chunk<D, true>(cur, k_cache + base, v_cache + base, lane);
-    }
-    finish_rope();
+    auto block = [&](int j) { return __builtin_amdgcn_readlane(my_blk, j); };
+    // ping-pong, cur <-> nxt (the barriers keep hipcc from strewing a chunk's loads among the other's MFMAs): both loads of a turn unconditional (behind a branch the wait for one chunk, which has to
+    // hold on either path, waits for the other too), and every key of these chunks admissible -- a split's last chunk,
+    // which may be partial and holds the new key, is left for behind the loop
     int j = 0;
-    for (; j + 2 <= n; j += 2) {                    // ping-pong: cur <-> nxt
-      {
-        const size_t base = (size_t)__builtin_amdgcn_readlane(my_blk, j + 1) * blk_stride + head_off;
-        load_chunk<D, true>(nxt, k_cache + base, v_cache + base, lane);
-      }
-      patch(cur, cb + j, (size_t)__builtin_amdgcn_readlane(my_blk, j) * blk_stride + head_off);
-      compute_chunk<D>(st, qf, cur, (cb + j) * kBS, kmax, scale_log2, lane);
-      if (j + 2 < n) {
-        const size_t base = (size_t)__builtin_amdgcn_readlane(my_blk, j + 2) * blk_stride + head_off;
-        load_chunk<D, true>(cur, k_cache + base, v_cache + base, lane);
-      }
-      patch(nxt, cb + j + 1, (size_t)__builtin_amdgcn_readlane(my_blk, j + 1) * blk_stride + head_off);
-      compute_chunk<D>(st, qf, nxt, (cb + j + 1) * kBS, kmax, scale_log2, lane);
+    for (; j + 2 < n; j += 2) {
+      load_at(nxt, block(j + 1));
+      __builtin_amdgcn_sched_barrier(0);
+      compute_chunk<D, false>(st, qf, cur, 0, 0, scale_log2, lane);
+      load_at(cur, block(j + 2));
+      __builtin_amdgcn_sched_barrier(0);
+      compute_chunk<D, false>(st, qf, nxt, 0, 0, scale_log2, lane);
     }
-    if (j < n) {
-      patch(cur, cb + j, (size_t)__builtin_amdgcn_readlane(my_blk, j) * blk_stride + head_off);
+    if (j + 1 < n) {
+      load_at(nxt, block(j + 1));
+      __builtin_amdgcn_sched_barrier(0);
+      compute_chunk<D, false>(st, qf, cur, 0, 0, scale_log2, lane);
+      patch(nxt, cb + j + 1, (size_t)block(j + 1) * blk_stride + head_off);
+      compute_chunk<D>(st, qf, nxt, (cb + j + 1) * kBS, kmax, scale_log2, lane);
+    } else {
+      patch(cur, cb + j, (size_t)block(j) * blk_stride + head_off);
       compute_chunk<D>(st, qf, cur, (cb + j) * kBS, kmax, scale_log2, lane);
+    }
+    if (cb + 64 < c1) {                             // the next pass's first chunk
+      my_blk = bt[min(cb + 64 + lane, max_blocks - 1)];
+      load_at(cur, block(0));
     }
   }
-  finish_rope();   // no cache chunk in this split
   if (owns_new) {
     // append k (row krow32(off)) and v (its [4][D][8] V^T slots) to the paged cache only now, after the
     // last KV load: stores count in vmcnt in issue order, so stores issued before the KV stream
@@ -402,45 +452,47 @@ __global__ void __launch_bounds__(WPB * 64, 2) attn_decode_kernel(   // 2nd arg:
       for (int dt = 0; dt < D / 16; ++dt) v_cache[base + vofs(off, dt * 16 + r, D, kBS)] = vn[dt];
     }
   }
-  float lt = st.lsum;
-  lt = rows_sum(lt);
-  if (!col_ok) return;                              // after the last MFMA: divergence is safe
-  const int h = kvh * G + r;
-  if (nsplit == 1) {
-    // a true division, exactly as the split-reduce computes num / den (bit-identical results
-    // whether a sequence's keys land in one split or in one non-empty split of several)
-    bf16* orow = out + ((size_t)b * hq + h) * D;
-#pragma unroll
-    for (int dt = 0; dt < D / 16; ++dt) {
-      bf16x4 o;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) o[i] = f2bf(lt > 0.f ? st.acc[dt][i] / lt : 0.f);
-      *reinterpret_cast<bf16x4*>(orow + dt * 16 + 4 * g) = o;
-    }
-  } else {
-    const size_t pi = ((size_t)b * hq + h) * nsplit + split;
-    float* po = part_o + pi * D;
-#pragma unroll
-    for (int dt = 0; dt < D / 16; ++dt) *reinterpret_cast<f32x4*>(po + dt * 16 + 4 * g) = st.acc[dt];
-    if (g == 0) { part_ml[pi * 2] = st.m; part_ml[pi * 2 + 1] = lt; }
-  }
+  write_out(st, rows_sum(st.lsum));                 // (after the last MFMA: divergence is safe)
 }
 
-template <int D>
+// Rounds of kRound splits, every load of a round before its first use: one round trip for up to kRound splits (plain loops
+// took two per split: one sequence of 32 heads with 4 splits 4.6 us, of 32 splits 10 us).  An empty split's factor is an
+// exact zero.
+template <int D, int kRound>
 __global__ void __launch_bounds__(D) attn_split_reduce_kernel(bf16* __restrict__ out,
                                                               const float* __restrict__ part_o,
                                                               const float* __restrict__ part_ml,
                                                               int nsplit) {
   const int bh = blockIdx.x, d = threadIdx.x;
   const float* ml = part_ml + (size_t)bh * nsplit * 2;
+  const float* po = part_o + (size_t)bh * nsplit * D + d;
+  float m[kRound], l[kRound], o[kRound];
+  auto load_round = [&](int s0) {
+#pragma unroll
+    for (int k = 0; k < kRound; ++k) {
+      const int s = min(s0 + k, nsplit - 1);        // past the last: repeated, dropped
+      m[k] = ml[2 * s];
+      l[k] = ml[2 * s + 1];
+      o[k] = po[(size_t)s * D];
+    }
+  };
+  load_round(0);
+#pragma unroll
+  for (int k = 0; k < kRound; ++k) asm volatile("" : "+v"(o[k]));   // hipcc would move o's loads behind the maximum
   float M = -INFINITY;
-  for (int s = 0; s < nsplit; ++s) M = fmaxf(M, ml[2 * s]);
+#pragma unroll
+  for (int k = 0; k < kRound; ++k) M = fmaxf(M, m[k]);
+  for (int s = kRound; s < nsplit; ++s) M = fmaxf(M, ml[2 * s]);
+  const float mref = M == -INFINITY ? 0.f : M;      // no key at all: every factor and den are 0
   float num = 0.f, den = 0.f;
-  if (M != -INFINITY) {
-    for (int s = 0; s < nsplit; ++s) {
-      const float f = exp2f(ml[2 * s] - M);
-      num += part_o[((size_t)bh * nsplit + s) * D + d] * f;
-      den += ml[2 * s + 1] * f;
+  for (int s0 = 0; s0 < nsplit; s0 += kRound) {
+    if (s0 > 0) load_round(s0);
+#pragma unroll
+    for (int k = 0; k < kRound; ++k) {
+      const float f = exp2f(m[k] - mref);
+      const float nk = fmaf(o[k], f, num), dk = fmaf(l[k], f, den);
+      num = s0 + k < nsplit ? nk : num;
+      den = s0 + k < nsplit ? dk : den;
     }
   }
   out[(size_t)bh * D + d] = f2bf(den > 0.f ? num / den : 0.f);
@@ -644,7 +696,11 @@ __global__ void __launch_bounds__(WV * 64, NT >= 4 || WV > 4 ? 1 : 2) attn_prefi
       if (!ok) v = bf16x8{};
       qf[t][ks] = v;
     }
-    if (cos_sin != nullptr) rope_rotate<D, true>(qf[t], cos_sin + (size_t)positions[tok] * D, g);
+    if (cos_sin != nullptr) {
+        RopeRow<D> row;
+        row.load(cos_sin + (size_t)positions[tok] * D, g);
+        rope_rotate<D>(qf[t], row);
+      }
     init_state(st[t]);
   }
   const int wg_kmax = qpos0 + min(wg_row0 + WV * R * NT, ql) - 1;
@@ -1523,12 +1579,22 @@ static void decode_launch(uintptr_t out, uintptr_t q, uintptr_t k_cache, uintptr
 #undef DLLM_DEC
   DLLM_HIP_CHECK(hipGetLastError());
   if (num_splits > 1) {
-    if (d == 128)
-      hipLaunchKernelGGL(attn_split_reduce_kernel<128>, dim3(batch * hq), dim3(128), 0, s, (bf16*)out,
-                         (const float*)part_o, (const float*)part_ml, num_splits);
-    else
-      hipLaunchKernelGGL(attn_split_reduce_kernel<64>, dim3(batch * hq), dim3(64), 0, s, (bf16*)out,
-                         (const float*)part_o, (const float*)part_ml, num_splits);
+    // the round that covers the splits with the fewest repeated loads (16 of them for 2 splits: 64 sequences of 64 heads
+    // 3 us slower)
+    auto reduce = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3(batch * hq), dim3(d), 0, s, (bf16*)out, (const float*)part_o, (const float*)part_ml,
+                         num_splits);
+    };
+#define DLLM_REDUCE(DD)                                                 \
+  do {                                                                  \
+    if (num_splits <= 2) reduce(attn_split_reduce_kernel<DD, 2>);       \
+    else if (num_splits <= 4) reduce(attn_split_reduce_kernel<DD, 4>);  \
+    else if (num_splits <= 8) reduce(attn_split_reduce_kernel<DD, 8>);  \
+    else reduce(attn_split_reduce_kernel<DD, 16>);                      \
+  } while (0)
+    if (d == 128) DLLM_REDUCE(128);
+    else DLLM_REDUCE(64);
+#undef DLLM_REDUCE
     DLLM_HIP_CHECK(hipGetLastError());
   }
 }

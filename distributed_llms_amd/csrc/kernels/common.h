@@ -208,6 +208,24 @@ __device__ __forceinline__ float part_load1(const float* P, size_t i) {
   return P[i];
 #endif
 }
+// The stored form of 8 / 2 consecutive elements, for a caller that has several loads under way before it converts any
+// (a conversion next to its load makes hipcc wait there)
+#if DLLM_PART_TYPE == 1
+typedef bf16x8 part_raw8;
+typedef bf16 part_raw2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ float part_value(bf16 v) { return bf2f(v); }
+typedef bf16 part_elem;
+#elif DLLM_PART_TYPE == 2
+typedef _Float16 part_raw8 __attribute__((ext_vector_type(8)));
+typedef _Float16 part_raw2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ float part_value(_Float16 v) { return (float)v * kPartUnscale; }
+typedef _Float16 part_elem;
+#else
+typedef float part_raw8 __attribute__((ext_vector_type(8)));
+typedef float part_raw2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ float part_value(float v) { return v; }
+typedef float part_elem;
+#endif
 // 4 consecutive elements (aligned to 4 elements)
 template <bool NT = false>
 __device__ __forceinline__ f32x4 part_load4(const float* P, size_t i) {

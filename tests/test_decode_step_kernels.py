@@ -3,7 +3,9 @@ import numpy as np
 import pytest
 import torch
 
+from distributed_llms_amd import ops
 from distributed_llms_amd.ops import gemm
+from distributed_llms_amd.ops import reference as ref
 from distributed_llms_amd.ops import seqmix as sm
 
 gpu = pytest.mark.gpu
@@ -20,8 +22,8 @@ def _sb(pos, slots, device):
 @pytest.mark.parametrize("nb,bw,taps", [(1, 8, 1), (3, 40, 2), (4, 256, 4), (2, 264, 8), (10, 256, 4), (1, 512, 3)])
 @pytest.mark.parametrize("seqs", [1, 5, 40, 141])
 def test_rglru_step(cuda, dtype, nb, bw, taps, seqs):
-    """One, two and four sequences per workgroup (an odd last one), blocks narrower and wider than 64 outputs and 256 rows, sequences
-    at positions 0, 1, 2 and later (parts of the tail do not exist yet), slots out of order."""
+    """One and two sequences per workgroup (an odd last one), blocks narrower and wider than 64 outputs and 256 rows,
+    sequences at positions 0, 1, 2 and later (parts of the tail do not exist yet), slots out of order."""
     g = torch.Generator().manual_seed(seqs + bw)
     c = nb * bw
     r = lambda *s, scale=1.0: (torch.randn(*s, generator=g) * scale).to(dtype)
@@ -110,3 +112,44 @@ def test_post_norm_add_sums_split_products(cuda, tokens, width, k):
     got = sm.post_norm_add(x0.clone(), part, wp, 1e-5, 0.7, bias=b, w_next=wn)
     want = sm.post_norm_add(x0.clone(), whole, wp, 1e-5, 0.7, bias=b, w_next=wn)
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+@gpu
+@pytest.mark.parametrize("lens,width,splits", [
+    ([1, 33, 64], 2, 1),                   # one chunk, and the new key alone in its chunk
+    ([65, 64, 1], 4, 2), ([97, 200, 250], 8, 4), ([449, 1], 16, 8), ([1000], 32, 16), ([1025, 3], 33, 17),
+    ([2048], 5120, 1), ([2400, 2049], 5120, 1)])   # splits of 2560 keys: past the 64 chunks of one pass over block ids
+@pytest.mark.parametrize("d,slabs", [(128, 0), (128, 4), (128, 7), (64, 0)])
+def test_decode_attention_rounds_and_passes(cuda, lens, width, splits, d, slabs):
+    """Decode attention at the edges of its split rounds, chunk pairs and block id passes, against float32."""
+    torch.manual_seed(5)
+    b, hq, hkv, used = len(lens), 4, 1, sum(-(-n // 32) for n in lens)
+    k = torch.randn(used, hkv, 32, d).bfloat16().cuda()
+    v = torch.randn(used, hkv, d, 32).bfloat16().cuda()
+    assert ops.decode_split_plan(b, hkv, max(lens), 32, width)[0] == splits
+    bt = torch.zeros(b, width, dtype=torch.int32)
+    at = 0
+    for i, n in enumerate(lens):
+        nb = -(-n // 32)
+        bt[i, :nb] = torch.arange(at, at + nb)
+        at += nb
+    slots = torch.tensor([int(bt[i, (n - 1) // 32]) * 32 + (n - 1) % 32 for i, n in enumerate(lens)], dtype=torch.int32)
+    bt, slots = bt.cuda(), slots.cuda()
+    sl = torch.tensor(lens, dtype=torch.int32).cuda()
+    n = (hq + 2 * hkv) * d
+    qkv = torch.randn(b, n).bfloat16().cuda()
+    arg = qkv
+    if slabs:                               # whole numbers of 2^-6: exact in a slab's 16 bits and in any order of the sum
+        parts = torch.randint(-64, 65, (slabs, b, n)).float() / 64
+        qkv = parts.sum(0).bfloat16().cuda()
+        arg = gemm.SplitKPartial((parts / 64).half().cuda(), slabs, b, n, (b, n), torch.bfloat16, qkv.device)
+    cs = ref.rope_cos_sin(d, 4096, 500000.0, device="cuda")
+    kf, vf = k.float(), v.float()
+    q2 = ref.rope_cache_append(qkv.float(), sl - 1, cs, kf, vf, slots, hq, hkv, d)
+    expect = ref.paged_attention_decode(q2.bfloat16().float(), kf.bfloat16().float(), vf, bt, sl, d ** -0.5)
+    torch.cuda.synchronize()
+    out = ops.paged_attention_decode_rope(arg, sl - 1, cs, k, v, slots, bt, sl, hq, hkv, d, d ** -0.5, max_ctx=max(lens))
+    # probabilities and the result are rounded to bf16 (2^-9 each, of at most max |v|); as much again for a rotated
+    # element that rounds the other way
+    assert (out.float() - expect).abs().max() <= 2.0 ** -7 * vf.abs().max()
+    assert torch.equal(v.float(), vf)
