@@ -30,16 +30,34 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
                                " at " __FILE__ ":" + std::to_string(__LINE__));         \
   } while (0)
 
+// Butterfly over the wave without LDS: the gfx950 row swaps for the xor-32 and xor-16 partners, then rotations inside each
+// row of 16.  After a step that makes a row's lanes equal modulo 2n, a rotation by n hands lane i the value of lane i ^ n,
+// so every sum is bit-identical to the __shfl_xor form, which lowers to six dependent ds_bpermute round trips (about 0.3 us
+// a wave).  Every lane of the wave has to be active, as for the MFMAs.
+template <int N>
+__device__ __forceinline__ float row_rotate(float v) {
+  return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x120 + N, 0xf, 0xf, true));
+}
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, DLLM_WAVE);
-  return v;
+  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(b[0]) + __uint_as_float(b[1]);
+  v += row_rotate<8>(v);
+  v += row_rotate<4>(v);
+  v += row_rotate<2>(v);
+  return v + row_rotate<1>(v);
 }
 
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, DLLM_WAVE));
-  return v;
+  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+  v = fmaxf(v, row_rotate<8>(v));
+  v = fmaxf(v, row_rotate<4>(v));
+  v = fmaxf(v, row_rotate<2>(v));
+  return fmaxf(v, row_rotate<1>(v));
 }
 
 // Reduction over a lane's xor-16 and xor-32 partners (the four 16-lane rows of an MFMA 16x16
@@ -62,13 +80,16 @@ __device__ __forceinline__ float rows_sum(float v) {
   return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
-// Block-wide sum for blockDim.x <= 1024; `red` must hold >= 16 floats.
+// Block-wide sum for blockDim.x <= 1024; `red` must hold >= 16 floats.  NTH: blockDim.x where it is known (0: it is read),
+// so that the waves' sums are read in one LDS round trip.
+template <int NTH = 0>
 __device__ __forceinline__ float block_sum(float v, float* red) {
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = NTH ? NTH / 64 : (blockDim.x + 63) >> 6;
   v = wave_sum(v);
   if (lane == 0) red[wid] = v;
   __syncthreads();
   float t = 0.f;
+#pragma unroll
   for (int i = 0; i < nw; ++i) t += red[i];
   __syncthreads();
   return t;
@@ -100,12 +121,14 @@ __device__ __forceinline__ bf16 f2bf(float x) { return (bf16)x; }
 __device__ __forceinline__ float bf2f(bf16 x) { return (float)x; }
 
 // Block-wide max for blockDim.x <= 1024; `red` must hold >= 16 floats.
+template <int NTH = 0>
 __device__ __forceinline__ float block_max(float v, float* red) {
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = NTH ? NTH / 64 : (blockDim.x + 63) >> 6;
   v = wave_max(v);
   if (lane == 0) red[wid] = v;
   __syncthreads();
   float t = red[0];
+#pragma unroll
   for (int i = 1; i < nw; ++i) t = fmaxf(t, red[i]);
   __syncthreads();
   return t;
@@ -130,9 +153,9 @@ __device__ __forceinline__ void store8_fp8(uint8_t* q, const float (&v)[8], floa
 
 // Norm epilogue with an FP8 consumer: y = bf16(v * inv * g) per element (written when y != null),
 // then the row's e4m3 quantization of those bf16 values (q8 row, scale at *qs).  v [MAXV][8]: the
-// thread's row values, vector idx = threadIdx.x + i * NTH.
+// thread's row values and g [MAXV] its weights, vector idx = threadIdx.x + i * NTH.
 template <int MAXV, int NTH>
-__device__ __forceinline__ void norm_out_fp8(float (&v)[MAXV][8], float inv, const bf16x8* __restrict__ wv, int nvec,
+__device__ __forceinline__ void norm_out_fp8(float (&v)[MAXV][8], float inv, const bf16x8 (&g)[MAXV], int nvec,
                                              bf16* __restrict__ y, uint8_t* __restrict__ q8, float* __restrict__ qs,
                                              float* red) {
   float amax = 0.f;
@@ -140,18 +163,17 @@ __device__ __forceinline__ void norm_out_fp8(float (&v)[MAXV][8], float inv, con
   for (int i = 0; i < MAXV; ++i) {
     const int idx = threadIdx.x + i * NTH;
     if (idx < nvec) {
-      const bf16x8 g = wv[idx];
       bf16x8 o;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        o[j] = f2bf(v[i][j] * inv * bf2f(g[j]));
+        o[j] = f2bf(v[i][j] * inv * bf2f(g[i][j]));
         v[i][j] = bf2f(o[j]);
         amax = fmaxf(amax, fabsf(v[i][j]));
       }
       if (y) reinterpret_cast<bf16x8*>(y)[idx] = o;
     }
   }
-  const float s = fp8_row_scale(block_max(amax, red));
+  const float s = fp8_row_scale(block_max<NTH>(amax, red));
   if (threadIdx.x == 0) *qs = s;
 #pragma unroll
   for (int i = 0; i < MAXV; ++i) {
@@ -208,23 +230,17 @@ __device__ __forceinline__ float part_load1(const float* P, size_t i) {
   return P[i];
 #endif
 }
-// The stored form of 8 / 2 consecutive elements, for a caller that has several loads under way before it converts any
-// (a conversion next to its load makes hipcc wait there)
+// The stored form of an element, for a caller that has several loads under way before it converts any (a conversion next
+// to its load makes hipcc wait there)
 #if DLLM_PART_TYPE == 1
-typedef bf16x8 part_raw8;
-typedef bf16 part_raw2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ float part_value(bf16 v) { return bf2f(v); }
 typedef bf16 part_elem;
+__device__ __forceinline__ float part_value(bf16 v) { return bf2f(v); }
 #elif DLLM_PART_TYPE == 2
-typedef _Float16 part_raw8 __attribute__((ext_vector_type(8)));
-typedef _Float16 part_raw2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ float part_value(_Float16 v) { return (float)v * kPartUnscale; }
 typedef _Float16 part_elem;
+__device__ __forceinline__ float part_value(_Float16 v) { return (float)v * kPartUnscale; }
 #else
-typedef float part_raw8 __attribute__((ext_vector_type(8)));
-typedef float part_raw2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ float part_value(float v) { return v; }
 typedef float part_elem;
+__device__ __forceinline__ float part_value(float v) { return v; }
 #endif
 // 4 consecutive elements (aligned to 4 elements)
 template <bool NT = false>

@@ -25,33 +25,40 @@ __global__ void __launch_bounds__(256) rms_norm_kernel(bf16* __restrict__ y, con
   const int nvec = hidden >> 3;
   const bf16x8* xr = reinterpret_cast<const bf16x8*>(x + (size_t)row * hidden);
   bf16x8* rr = residual ? reinterpret_cast<bf16x8*>(residual + (size_t)row * hidden) : nullptr;
+  const bf16x8* wv = reinterpret_cast<const bf16x8*>(w);
   float v[MAXV][8];
+  bf16x8 a[MAXV], b[MAXV], g[MAXV];
   float ss = 0.f;
+  // every load off a clamped place and before the first use (behind the guards hipcc waited for each vector in turn, and
+  // for the weight behind the block's sum)
+  const bf16x8* rb = rr ? rr : xr;
+#pragma unroll
+  for (int i = 0; i < MAXV; ++i) {
+    const int idx = min((int)threadIdx.x + i * 256, nvec - 1);
+    a[i] = xr[idx];
+    b[i] = rb[idx];
+    g[i] = wv[idx];
+  }
 #pragma unroll
   for (int i = 0; i < MAXV; ++i) {
     const int idx = threadIdx.x + i * 256;
-    if (idx < nvec) {
-      bf16x8 a = xr[idx];
-      if (rr) {
-        bf16x8 b = rr[idx];
-        bf16x8 s;
+    if (rr) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) s[j] = f2bf(bf2f(a[j]) + bf2f(b[j]));
-        rr[idx] = s;
-        a = s;  // normalise the bf16-rounded residual, as the reference does
-      }
+      for (int j = 0; j < 8; ++j) a[i][j] = f2bf(bf2f(a[i][j]) + bf2f(b[i][j]));
+    }
+    if (idx < nvec) {
+      if (rr) rr[idx] = a[i];   // normalise the bf16-rounded residual, as the reference does
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        v[i][j] = bf2f(a[j]);
+        v[i][j] = bf2f(a[i][j]);
         ss += v[i][j] * v[i][j];
       }
     }
   }
-  ss = block_sum(ss, red);
+  ss = block_sum<256>(ss, red);
   const float inv = rsqrtf(ss / (float)hidden + eps);
-  const bf16x8* wv = reinterpret_cast<const bf16x8*>(w);
   if (q8) {   // FP8 consumer (W8A8 GEMM): per-token e4m3 of the bf16-rounded output, y optional
-    norm_out_fp8<MAXV, 256>(v, inv, wv, nvec, y ? y + (size_t)row * hidden : nullptr, q8 + (size_t)row * hidden,
+    norm_out_fp8<MAXV, 256>(v, inv, g, nvec, y ? y + (size_t)row * hidden : nullptr, q8 + (size_t)row * hidden,
                             qs + row, red);
     return;
   }
@@ -60,10 +67,9 @@ __global__ void __launch_bounds__(256) rms_norm_kernel(bf16* __restrict__ y, con
   for (int i = 0; i < MAXV; ++i) {
     const int idx = threadIdx.x + i * 256;
     if (idx < nvec) {
-      bf16x8 g = wv[idx];
       bf16x8 o;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) o[j] = f2bf(v[i][j] * inv * bf2f(g[j]));
+      for (int j = 0; j < 8; ++j) o[j] = f2bf(v[i][j] * inv * bf2f(g[i][j]));
       yr[idx] = o;
     }
   }

@@ -23,19 +23,19 @@ __global__ void __launch_bounds__(256) quant_fp8_rows_kernel(uint8_t* __restrict
   float amax = 0.f;
   if constexpr (MAXV > 0) {
     float v[MAXV][8];
+    bf16x8 a[MAXV];
+    // clamped places, no guard (hipcc would wait for each vector in its branch); a repeated vector leaves the maximum alone
+#pragma unroll
+    for (int i = 0; i < MAXV; ++i) a[i] = xr[min(tid + i * 256, nvec - 1)];
 #pragma unroll
     for (int i = 0; i < MAXV; ++i) {
-      const int idx = tid + i * 256;
-      if (idx < nvec) {
-        const bf16x8 a = xr[idx];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          v[i][j] = bf2f(a[j]);
-          amax = fmaxf(amax, fabsf(v[i][j]));
-        }
+      for (int j = 0; j < 8; ++j) {
+        v[i][j] = bf2f(a[i][j]);
+        amax = fmaxf(amax, fabsf(v[i][j]));
       }
     }
-    const float s = fp8_row_scale(block_max(amax, red));
+    const float s = fp8_row_scale(block_max<256>(amax, red));
     if (tid == 0) scale[m] = s;
 #pragma unroll
     for (int i = 0; i < MAXV; ++i) {

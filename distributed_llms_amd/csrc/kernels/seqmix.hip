@@ -22,24 +22,31 @@
 namespace dllm {
 
 // --------------------------------------------------------------------------- embedding -> f32
-template <typename T>
+// V elements per lane, a row in as many workgroups as it takes (a loop of 2-byte loads waited for each: 16 rows of 2560
+// 2.9 us from cached rows, 2.1 now; cold 7.9 us before)
+template <typename T, int V>
 __global__ void __launch_bounds__(256) sm_embed_kernel(float* __restrict__ out, const int32_t* __restrict__ ids,
                                                        const void* __restrict__ table_, int width, int vocab,
                                                        float scale) {
-  const T* table = (const T*)table_;
+  const int i = (blockIdx.y * 256 + threadIdx.x) * V;
+  if (i >= width) return;
   int id = ids[blockIdx.x];
   id = id < 0 ? 0 : (id >= vocab ? vocab - 1 : id);
-  const T* src = table + (size_t)id * width;
-  float* dst = out + (size_t)blockIdx.x * width;
-  for (int i = threadIdx.x; i < width; i += 256) dst[i] = ldf(src + i) * scale;
+  float v[V];
+  ldv<V>((const T*)table_ + (size_t)id * width + i, v);
+#pragma unroll
+  for (int j = 0; j < V; ++j) v[j] *= scale;
+  stv<V>(out + (size_t)blockIdx.x * width + i, v);
 }
 
 void sm_embed_f32(uintptr_t out, uintptr_t ids, uintptr_t table, int tokens, int width, int vocab, float scale, int f32,
                   uintptr_t stream) {
   if (tokens <= 0) return;
-  DLLM_HOST_CHECK(width > 0 && vocab > 0, "embed sizes");
-  SM_DISPATCH(f32, sm_embed_kernel, dim3(tokens), dim3(256), 0, stream, (float*)out, (const int32_t*)ids,
-              (const void*)table, width, vocab, scale);
+  DLLM_HOST_CHECK(width > 0 && width <= 256 * 65535 && vocab > 0, "embed sizes");
+  const bool vec = width % 8 == 0 && table % 32 == 0 && out % 32 == 0;
+  const dim3 grid(tokens, (width + (vec ? 2047 : 255)) / (vec ? 2048 : 256));
+  SM_DISPATCH_V(f32, vec, sm_embed_kernel, grid, dim3(256), 0, stream, (float*)out, (const int32_t*)ids,
+                (const void*)table, width, vocab, scale);
 }
 
 // --------------------------------------------------------------------------- embedding + RMS norm -> f32 stream
@@ -122,10 +129,63 @@ __global__ void __launch_bounds__(256) sm_rms_norm_kernel(void* __restrict__ y_,
   }
 }
 
+// The same for a row that fits the registers (NV pieces of 8 elements per lane, the same lane for the same elements): x
+// and w loaded once, before the first use, off clamped places.
+template <typename T, int NV>
+__global__ void __launch_bounds__(256) sm_rms_norm_row_kernel(void* __restrict__ y_, const float* __restrict__ x,
+                                                              const void* __restrict__ w_, int width, float eps,
+                                                              float offset) {
+  __shared__ float red[16];
+  T* y = (T*)y_ + (size_t)blockIdx.x * width;
+  const float* xr = x + (size_t)blockIdx.x * width;
+  float v[NV][8], g[NV][8];
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+    const int i = min((k * 256 + (int)threadIdx.x) * 8, width - 8);
+    ldv<8>(xr + i, v[k]);
+    ldv<8>((const T*)w_ + i, g[k]);
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int k = 0; k < NV; ++k)
+    if ((k * 256 + (int)threadIdx.x) * 8 < width) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) ss += v[k][j] * v[k][j];
+    }
+  ss = block_sum<256>(ss, red);
+  const float inv = 1.0f / sqrtf(ss / (float)width + eps);
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+    const int i = (k * 256 + threadIdx.x) * 8;
+    if (i < width) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[k][j] = v[k][j] * inv * (offset + g[k][j]);
+      stv<8>(y + i, v[k]);
+    }
+  }
+}
+
 void sm_rms_norm(uintptr_t y, uintptr_t x, uintptr_t w, int rows, int width, float eps, float offset, int f32,
                  uintptr_t stream) {
   if (rows <= 0) return;
   DLLM_HOST_CHECK(width > 0, "norm width");
+  if (width % 8 == 0 && width <= 8192) {
+    const auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3(rows), dim3(256), 0, (hipStream_t)stream, (void*)y, (const float*)x, (const void*)w,
+                         width, eps, offset);
+    };
+#define SM_RMS_ROW(T)                                                \
+  do {                                                               \
+    if (width <= 2048) go(sm_rms_norm_row_kernel<T, 1>);             \
+    else if (width <= 4096) go(sm_rms_norm_row_kernel<T, 2>);        \
+    else go(sm_rms_norm_row_kernel<T, 4>);                           \
+  } while (0)
+    if (f32) SM_RMS_ROW(float);
+    else SM_RMS_ROW(bf16);
+#undef SM_RMS_ROW
+    DLLM_HIP_CHECK(hipGetLastError());
+    return;
+  }
   SM_DISPATCH_V(f32, width % 8 == 0, sm_rms_norm_kernel, dim3(rows), dim3(256), 0, stream, (void*)y, (const float*)x,
                 (const void*)w, width, eps, offset);
 }
@@ -242,16 +302,18 @@ __global__ void __launch_bounds__(256) sm_layer_norm_kernel(void* __restrict__ y
   const float* xr = x + (size_t)blockIdx.x * width;
   float v[NV][V], w[NV][V], b[NV][V];
 #pragma unroll
-  for (int k = 0; k < NV; ++k) {
-    const int i = (k * 256 + threadIdx.x) * V;
-#pragma unroll
-    for (int j = 0; j < V; ++j) v[k][j] = 0.f;
-    if (i < width) {
-      ldv<V>(xr + i, v[k]);
-      ldv<V>((const T*)w_ + i, w[k]);
-      ldv<V>((const T*)b_ + i, b[k]);
-    }
+  for (int k = 0; k < NV; ++k) {                  // off clamped places: no load waits behind another's guard
+    const int i = min((k * 256 + (int)threadIdx.x) * V, width - V);
+    ldv<V>(xr + i, v[k]);
+    ldv<V>((const T*)w_ + i, w[k]);
+    ldv<V>((const T*)b_ + i, b[k]);
   }
+#pragma unroll
+  for (int k = 0; k < NV; ++k)
+    if ((k * 256 + (int)threadIdx.x) * V >= width) {
+#pragma unroll
+      for (int j = 0; j < V; ++j) v[k][j] = 0.f;
+    }
   float mean, inv;
   ln_stats<V, NV>(v, width, eps, red, mean, inv);
   T* y = (T*)y_ + (size_t)blockIdx.x * width;
@@ -266,91 +328,120 @@ __global__ void __launch_bounds__(256) sm_layer_norm_kernel(void* __restrict__ y
   }
 }
 
-// One row of a product that is still in `parts` split-K slabs (V = 4; common.h part_load): their sum, rounded to bf16 as the
-// reduction of a split product rounds it.  Every load off a clamped place, the slabs eight at a time.
-template <int NV, int V>
-__device__ __forceinline__ void ln_slabs(const float* __restrict__ P, int parts, size_t row, int width, float (&v)[NV][V]) {
+// One row of a product that is still in `parts` split-K slabs (V = 4; common.h part_elem): their sum, rounded to bf16 as the
+// reduction of a split product rounds it.  CH slabs a round, off clamped places, all of a round's loads before its first
+// use (with the adds behind `slab < parts` hipcc moved each load into its branch: ten round trips for 12 slabs).
+template <int CH, int NV, int V>
+__device__ __forceinline__ void ln_slab_rounds(const float* __restrict__ P, int parts, size_t row, int width, float (&v)[NV][V]) {
+  typedef part_elem raw __attribute__((ext_vector_type(4)));
   const size_t slab = (size_t)gridDim.x * width;
-  const int top = width - V;
-  constexpr int CH = NV <= 4 ? 8 : 2;
-  f32x4 a[NV];
+  float a[NV][4];
 #pragma unroll
-  for (int k = 0; k < NV; ++k) a[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int k = 0; k < NV; ++k)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) a[k][j] = 0.f;
   for (int s0 = 0; s0 < parts; s0 += CH) {
-    f32x4 l[CH][NV];
+    raw l[CH][NV];
 #pragma unroll
     for (int u = 0; u < CH; ++u)
 #pragma unroll
       for (int k = 0; k < NV; ++k)
-        l[u][k] = part_load4(P, min(s0 + u, parts - 1) * slab + row + min((k * 256 + (int)threadIdx.x) * V, top));
+        l[u][k] = *reinterpret_cast<const raw*>(reinterpret_cast<const part_elem*>(P) + min(s0 + u, parts - 1) * slab + row +
+                                                min((k * 256 + (int)threadIdx.x) * V, width - V));
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < CH; ++u)
-      if (s0 + u < parts) {
 #pragma unroll
-        for (int k = 0; k < NV; ++k) a[k] += l[u][k];
-      }
+      for (int k = 0; k < NV; ++k)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float t = a[k][j] + part_value(l[u][k][j]);
+          a[k][j] = s0 + u < parts ? t : a[k][j];
+        }
   }
 #pragma unroll
   for (int k = 0; k < NV; ++k)
 #pragma unroll
     for (int j = 0; j < V; ++j) v[k][j] = bf2f(f2bf(a[k][j & 3]));
 }
+template <int NV, int V>
+__device__ __forceinline__ void ln_slabs(const float* __restrict__ P, int parts, size_t row, int width, float (&v)[NV][V]) {
+  if constexpr (NV <= 4) {
+    if (parts <= 4) ln_slab_rounds<4, NV, V>(P, parts, row, width, v);        // uniform
+    else if (parts <= 8) ln_slab_rounds<8, NV, V>(P, parts, row, width, v);
+    else ln_slab_rounds<12, NV, V>(P, parts, row, width, v);
+  } else {
+    ln_slab_rounds<2, NV, V>(P, parts, row, width, v);
+  }
+}
 
 // The close of a sublayer between two layer norms: x += layer_norm(o + bias) (weight wp, bias bp; `bias` null: none), and
 // with wn: h = layer_norm(x) (wn, bn), the next sublayer's input.  parts > 0: o is the sum of that many split-K slabs
 // [rows, width] (common.h part_load; bf16 results, rounded as the reduction of a split product rounds them).
-template <typename T, int V, int NV>
-__global__ void __launch_bounds__(256) sm_post_layer_norm_kernel(
-    float* __restrict__ x, const void* __restrict__ o_, int parts, const void* __restrict__ bias_,
+// Two kernels of one body: the slabs in flight would cost the other form its occupancy (6376 rows: 37 us as one, 30.5 apart).
+template <typename T, int V, int NV, bool SLABS>
+__device__ __forceinline__ void post_layer_norm_row(
+    float* red, float* __restrict__ x, const void* __restrict__ o_, int parts, const void* __restrict__ bias_,
     const void* __restrict__ wp_, const void* __restrict__ bp_, const void* __restrict__ wn_, const void* __restrict__ bn_,
     void* __restrict__ h_, int width, float eps) {
-  __shared__ float red[16];
   const size_t row = (size_t)blockIdx.x * width;
   float* xr = x + row;
-  float v[NV][V], xv[NV][V], w[NV][V], b[NV][V];
-  // every load of the row off a clamped place, so that none waits behind another's guard; the slabs eight at a time
-  const int top = width - V;
-  if (V == 4 && parts > 0) {
+  typedef T vec __attribute__((ext_vector_type(V)));
+  typedef float fvec __attribute__((ext_vector_type(V)));
+  constexpr bool kEarly = NV * V <= 16;           // wider rows do not hold the weights as well
+  float v[NV][V], xv[NV][V];
+  fvec rx[NV];
+  vec rw[NV], rb[NV], rwn[NV], rbn[NV], rc[NV];
+  // every load of the row off a clamped place, in its stored form and before the first use: no load waits behind
+  // another's guard or conversion, and the next norm's weights do not wait for this one's sums (16 rows of 2560: with 12 slabs 8.6 us
+  // before, 5.4 now, without 4.7 and 3.6; 6376 rows 34.2 and 30.5)
+  auto at = [&](int k) { return min((k * 256 + (int)threadIdx.x) * V, width - V); };
+  auto load = [&](vec (&r)[NV], const void* from) {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) r[k] = *reinterpret_cast<const vec*>((const T*)from + at(k));
+  };
+#pragma unroll
+  for (int k = 0; k < NV; ++k) rx[k] = *reinterpret_cast<const fvec*>(xr + at(k));
+  vec ro[NV];
+  if (!SLABS && kEarly) load(ro, (const T*)o_ + row);
+  if (kEarly) load(rw, wp_), load(rb, bp_);
+  if (kEarly && bias_) load(rc, bias_);
+  if (kEarly && wn_) load(rwn, wn_), load(rbn, bn_);
+  if constexpr (SLABS) {
     ln_slabs<NV>((const float*)o_, parts, row, width, v);
   } else {
 #pragma unroll
-    for (int k = 0; k < NV; ++k) ldv<V>((const T*)o_ + row + min((k * 256 + (int)threadIdx.x) * V, top), v[k]);
+    for (int k = 0; k < NV; ++k) {
+      if (!kEarly) ro[k] = *reinterpret_cast<const vec*>((const T*)o_ + row + at(k));
+#pragma unroll
+      for (int j = 0; j < V; ++j) v[k][j] = (float)ro[k][j];
+    }
   }
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
-    const int i = min((k * 256 + (int)threadIdx.x) * V, top);
-    ldv<V>(xr + i, xv[k]);
-    ldv<V>((const T*)wp_ + i, w[k]);
-    ldv<V>((const T*)bp_ + i, b[k]);
-    if (bias_) {
-      float c[V];
-      ldv<V>((const T*)bias_ + i, c);
+    const bool in = (k * 256 + (int)threadIdx.x) * V < width;
+    if (!kEarly && bias_) rc[k] = *reinterpret_cast<const vec*>((const T*)bias_ + at(k));
 #pragma unroll
-      for (int j = 0; j < V; ++j) v[k][j] += c[j];
+    for (int j = 0; j < V; ++j) {
+      if (bias_) v[k][j] += (float)rc[k][j];
+      v[k][j] = in ? v[k][j] : 0.f;
+      xv[k][j] = in ? rx[k][j] : 0.f;
     }
   }
-#pragma unroll
-  for (int k = 0; k < NV; ++k)
-    if ((k * 256 + (int)threadIdx.x) * V >= width) {
-#pragma unroll
-      for (int j = 0; j < V; ++j) v[k][j] = xv[k][j] = 0.f;
-    }
   float mean, inv;
   ln_stats<V, NV>(v, width, eps, red, mean, inv);
+  if (!kEarly) load(rw, wp_), load(rb, bp_);
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
     const int i = (k * 256 + threadIdx.x) * V;
     if (i < width) {
 #pragma unroll
-      for (int j = 0; j < V; ++j) xv[k][j] += (v[k][j] - mean) * inv * w[k][j] + b[k][j];
+      for (int j = 0; j < V; ++j) xv[k][j] += (v[k][j] - mean) * inv * (float)rw[k][j] + (float)rb[k][j];
       stv<V>(xr + i, xv[k]);
-      if (wn_) {
-        ldv<V>((const T*)wn_ + i, w[k]);
-        ldv<V>((const T*)bn_ + i, b[k]);
-      }
     }
   }
   if (!wn_) return;
+  if (!kEarly) load(rwn, wn_), load(rbn, bn_);
   ln_stats<V, NV>(xv, width, eps, red + 8, mean, inv);
   T* h = (T*)h_ + row;
 #pragma unroll
@@ -358,10 +449,27 @@ __global__ void __launch_bounds__(256) sm_post_layer_norm_kernel(
     const int i = (k * 256 + threadIdx.x) * V;
     if (i < width) {
 #pragma unroll
-      for (int j = 0; j < V; ++j) xv[k][j] = (xv[k][j] - mean) * inv * w[k][j] + b[k][j];
+      for (int j = 0; j < V; ++j) xv[k][j] = (xv[k][j] - mean) * inv * (float)rwn[k][j] + (float)rbn[k][j];
       stv<V>(h + i, xv[k]);
     }
   }
+}
+
+template <typename T, int V, int NV>
+__global__ void __launch_bounds__(256) sm_post_layer_norm_kernel(
+    float* __restrict__ x, const void* __restrict__ o, const void* __restrict__ bias, const void* __restrict__ wp,
+    const void* __restrict__ bp, const void* __restrict__ wn, const void* __restrict__ bn, void* __restrict__ h, int width,
+    float eps) {
+  __shared__ float red[16];
+  post_layer_norm_row<T, V, NV, false>(red, x, o, 0, bias, wp, bp, wn, bn, h, width, eps);
+}
+template <typename T, int V, int NV>
+__global__ void __launch_bounds__(256) sm_post_layer_norm_slabs_kernel(
+    float* __restrict__ x, const void* __restrict__ o, int parts, const void* __restrict__ bias, const void* __restrict__ wp,
+    const void* __restrict__ bp, const void* __restrict__ wn, const void* __restrict__ bn, void* __restrict__ h, int width,
+    float eps) {
+  __shared__ float red[16];
+  post_layer_norm_row<T, V, NV, true>(red, x, o, parts, bias, wp, bp, wn, bn, h, width, eps);
 }
 
 // V = 4 elements per lane and piece (width a multiple of 4), else one; the fewest pieces that hold the row
@@ -379,6 +487,20 @@ __global__ void __launch_bounds__(256) sm_post_layer_norm_kernel(
     } else if (np_ <= 4) SM_LN_GO(f32, KERNEL, 1, 4, grid, stream, __VA_ARGS__);                                   \
     else if (np_ <= 16) SM_LN_GO(f32, KERNEL, 1, 16, grid, stream, __VA_ARGS__);                                   \
     else SM_LN_GO(f32, KERNEL, 1, 64, grid, stream, __VA_ARGS__);                                                  \
+    DLLM_HIP_CHECK(hipGetLastError());                                                                             \
+  } while (0)
+// ... of a product in slabs (bf16, width a multiple of 4)
+#define SM_LN_SLABS(width, KERNEL, grid, stream, ...)                                                                \
+  do {                                                                                                             \
+    DLLM_HOST_CHECK((width) > 0 && (width) <= 16384 && (width) % 4 == 0, "layer norm width");                      \
+    const auto go_ = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256), 0, (hipStream_t)(stream), __VA_ARGS__); }; \
+    const int np_ = ((width) + 1023) / 1024;                                                                       \
+    if (np_ <= 1) go_(KERNEL<bf16, 4, 1>);                                                                         \
+    else if (np_ <= 2) go_(KERNEL<bf16, 4, 2>);                                                                    \
+    else if (np_ <= 3) go_(KERNEL<bf16, 4, 3>);                                                                    \
+    else if (np_ <= 4) go_(KERNEL<bf16, 4, 4>);                                                                    \
+    else if (np_ <= 8) go_(KERNEL<bf16, 4, 8>);                                                                    \
+    else go_(KERNEL<bf16, 4, 16>);                                                                                 \
     DLLM_HIP_CHECK(hipGetLastError());                                                                             \
   } while (0)
 #define SM_LN_GO(f32, KERNEL, V, NV, grid, stream, ...)                                                              \
@@ -401,53 +523,62 @@ void sm_post_layer_norm_add(uintptr_t x, uintptr_t o, int parts, uintptr_t bias,
   if (rows <= 0) return;
   DLLM_HOST_CHECK(x && o && w_post && b_post && (!w_next || (b_next && h)), "post_layer_norm_add arguments");
   DLLM_HOST_CHECK(parts >= 0 && (parts == 0 || (!f32 && width % 4 == 0)), "post_layer_norm_add slabs");
-  SM_LN_DISPATCH(f32, width, sm_post_layer_norm_kernel, dim3(rows), stream, (float*)x, (const void*)o, parts,
-                 (const void*)bias, (const void*)w_post, (const void*)b_post, (const void*)w_next, (const void*)b_next,
-                 (void*)h, width, eps);
+  if (parts > 0)
+    SM_LN_SLABS(width, sm_post_layer_norm_slabs_kernel, dim3(rows), stream, (float*)x, (const void*)o, parts,
+                (const void*)bias, (const void*)w_post, (const void*)b_post, (const void*)w_next, (const void*)b_next,
+                (void*)h, width, eps);
+  else
+    SM_LN_DISPATCH(f32, width, sm_post_layer_norm_kernel, dim3(rows), stream, (float*)x, (const void*)o,
+                   (const void*)bias, (const void*)w_post, (const void*)b_post, (const void*)w_next, (const void*)b_next,
+                   (void*)h, width, eps);
 }
 
 // The close of a sublayer around RMS norms, the row in registers (NV pieces of V elements per lane): every load -- o or its
 // slabs, the second input, bias, stream and both weights -- goes out before the first use, and nothing is read twice (the
 // three-pass form above re-read o, x and the new x, with each pass's loads behind a block reduction).
 // parts > 0: o is the sum of that many split-K slabs [rows, width], rounded as the reduction of a split product rounds it.
-// 2560 wide, bf16: 16 rows 5.9 -> 4.0 us (bound by the launch and two reductions), 6376 rows 41 -> 37 us (5.2 TB/s).
-template <typename T, int V, int NV>
-__global__ void __launch_bounds__(256) sm_post_norm_row_kernel(float* __restrict__ x, const void* __restrict__ o_, int parts,
-                                                               const void* __restrict__ bias_, const void* __restrict__ wp_,
-                                                               const void* __restrict__ wn_, void* __restrict__ h_, int width,
-                                                               float eps, float mult, float offset,
-                                                               const void* __restrict__ o2_, float s1, float s2) {
-  __shared__ float red[16];
+// 2560 wide, bf16: 16 rows 4.3 -> 3.2 us (bound by the launch and two reductions), 6376 rows 44 -> 35 us (5.6 TB/s).
+template <typename T, int V, int NV, bool SLABS>
+__device__ __forceinline__ void post_norm_row(float* red, float* __restrict__ x, const void* __restrict__ o_, int parts,
+                                              const void* __restrict__ bias_, const void* __restrict__ wp_,
+                                              const void* __restrict__ wn_, void* __restrict__ h_, int width, float eps,
+                                              float mult, float offset, const void* __restrict__ o2_, float s1, float s2) {
   const size_t row = (size_t)blockIdx.x * width;
   float* xr = x + row;
-  float v[NV][V], xv[NV][V], wp[NV][V], wn[NV][V];
-  const int top = width - V;
-  if (V == 4 && parts > 0) {
+  typedef T vec __attribute__((ext_vector_type(V)));
+  typedef float fvec __attribute__((ext_vector_type(V)));
+  float v[NV][V], xv[NV][V];
+  fvec rx[NV];
+  vec rwp[NV], rwn[NV], r2[NV], rc[NV];
+  // in their stored form: no load behind a conversion (hipcc would wait there)
+  auto at = [&](int k) { return min((k * 256 + (int)threadIdx.x) * V, width - V); };
+  auto load = [&](vec (&r)[NV], const void* from) {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) r[k] = *reinterpret_cast<const vec*>((const T*)from + at(k));
+  };
+#pragma unroll
+  for (int k = 0; k < NV; ++k) rx[k] = *reinterpret_cast<const fvec*>(xr + at(k));
+  vec ro[NV];
+  if (!SLABS) load(ro, (const T*)o_ + row);
+  load(rwp, wp_);
+  if (wn_) load(rwn, wn_);
+  if (o2_) load(r2, (const T*)o2_ + row);
+  if (bias_) load(rc, bias_);
+  if constexpr (SLABS) {
     ln_slabs<NV>((const float*)o_, parts, row, width, v);
   } else {
 #pragma unroll
-    for (int k = 0; k < NV; ++k) ldv<V>((const T*)o_ + row + min((k * 256 + (int)threadIdx.x) * V, top), v[k]);
-  }
-  // what is not given is read from the closing weight and dropped: no load behind a branch (hipcc would wait there)
-  const T* pn = (const T*)(wn_ ? wn_ : wp_);
-  const T* p2 = o2_ ? (const T*)o2_ + row : (const T*)wp_;
-  const T* pb = (const T*)(bias_ ? bias_ : wp_);
-  float c2[NV][V], cb[NV][V];
+    for (int k = 0; k < NV; ++k)
 #pragma unroll
-  for (int k = 0; k < NV; ++k) {
-    const int i = min((k * 256 + (int)threadIdx.x) * V, top);
-    ldv<V>(xr + i, xv[k]);
-    ldv<V>((const T*)wp_ + i, wp[k]);
-    ldv<V>(pn + i, wn[k]);
-    ldv<V>(p2 + i, c2[k]);
-    ldv<V>(pb + i, cb[k]);
+      for (int j = 0; j < V; ++j) v[k][j] = (float)ro[k][j];
   }
 #pragma unroll
   for (int k = 0; k < NV; ++k)
 #pragma unroll
     for (int j = 0; j < V; ++j) {
-      if (o2_) v[k][j] = s1 * v[k][j] + s2 * c2[k][j];
-      if (bias_) v[k][j] += cb[k][j];
+      xv[k][j] = rx[k][j];
+      if (o2_) v[k][j] = s1 * v[k][j] + s2 * (float)r2[k][j];
+      if (bias_) v[k][j] += (float)rc[k][j];
     }
   float ss = 0.f;
 #pragma unroll
@@ -456,7 +587,7 @@ __global__ void __launch_bounds__(256) sm_post_norm_row_kernel(float* __restrict
 #pragma unroll
       for (int j = 0; j < V; ++j) ss += v[k][j] * v[k][j];
     }
-  ss = block_sum(ss, red);
+  ss = block_sum<256>(ss, red);
   const float inv = 1.0f / sqrtf(ss / (float)width + eps);
   float sq = 0.f;
 #pragma unroll
@@ -465,7 +596,7 @@ __global__ void __launch_bounds__(256) sm_post_norm_row_kernel(float* __restrict
     if (i < width) {
 #pragma unroll
       for (int j = 0; j < V; ++j) {
-        xv[k][j] = xv[k][j] + mult * (v[k][j] * inv * (offset + wp[k][j]));
+        xv[k][j] = xv[k][j] + mult * (v[k][j] * inv * (offset + (float)rwp[k][j]));
         sq += xv[k][j] * xv[k][j];
       }
       stv<V>(xr + i, xv[k]);
@@ -473,17 +604,37 @@ __global__ void __launch_bounds__(256) sm_post_norm_row_kernel(float* __restrict
     }
   }
   if (!wn_) return;
-  sq = block_sum(sq, red);
+  sq = block_sum<256>(sq, red);
   const float inv2 = 1.0f / sqrtf(sq / (float)width + eps);
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
     const int i = (k * 256 + threadIdx.x) * V;
     if (i < width) {
 #pragma unroll
-      for (int j = 0; j < V; ++j) xv[k][j] = xv[k][j] * inv2 * (offset + wn[k][j]);
+      for (int j = 0; j < V; ++j) xv[k][j] = xv[k][j] * inv2 * (offset + (float)rwn[k][j]);
       stv<V>((T*)h_ + row + i, xv[k]);
     }
   }
+}
+
+template <typename T, int V, int NV>
+__global__ void __launch_bounds__(256) sm_post_norm_row_kernel(float* __restrict__ x, const void* __restrict__ o,
+                                                               const void* __restrict__ bias, const void* __restrict__ wp,
+                                                               const void* __restrict__ wn, void* __restrict__ h, int width,
+                                                               float eps, float mult, float offset,
+                                                               const void* __restrict__ o2, float s1, float s2) {
+  __shared__ float red[16];
+  post_norm_row<T, V, NV, false>(red, x, o, 0, bias, wp, wn, h, width, eps, mult, offset, o2, s1, s2);
+}
+template <typename T, int V, int NV>
+__global__ void __launch_bounds__(256) sm_post_norm_slabs_kernel(float* __restrict__ x, const void* __restrict__ o,
+                                                                 int parts, const void* __restrict__ bias,
+                                                                 const void* __restrict__ wp, const void* __restrict__ wn,
+                                                                 void* __restrict__ h, int width, float eps, float mult,
+                                                                 float offset, const void* __restrict__ o2, float s1,
+                                                                 float s2) {
+  __shared__ float red[16];
+  post_norm_row<T, V, NV, true>(red, x, o, parts, bias, wp, wn, h, width, eps, mult, offset, o2, s1, s2);
 }
 
 void sm_post_norm_add(uintptr_t x, uintptr_t o, int parts, uintptr_t bias, uintptr_t w_post, uintptr_t w_next, uintptr_t h,
@@ -493,9 +644,14 @@ void sm_post_norm_add(uintptr_t x, uintptr_t o, int parts, uintptr_t bias, uintp
   DLLM_HOST_CHECK(width > 0 && (!w_next || h), "post_norm_add arguments");
   DLLM_HOST_CHECK(parts >= 0 && (parts == 0 || (!f32 && width % 4 == 0 && width <= 16384)), "post_norm_add slabs");
   if (width <= 16384) {
-    SM_LN_DISPATCH(f32, width, sm_post_norm_row_kernel, dim3(rows), stream, (float*)x, (const void*)o, parts,
-                   (const void*)bias, (const void*)w_post, (const void*)w_next, (void*)h, width, eps, mult, offset,
-                   (const void*)o2, s1, s2);
+    if (parts > 0)
+      SM_LN_SLABS(width, sm_post_norm_slabs_kernel, dim3(rows), stream, (float*)x, (const void*)o, parts,
+                  (const void*)bias, (const void*)w_post, (const void*)w_next, (void*)h, width, eps, mult, offset,
+                  (const void*)o2, s1, s2);
+    else
+      SM_LN_DISPATCH(f32, width, sm_post_norm_row_kernel, dim3(rows), stream, (float*)x, (const void*)o,
+                     (const void*)bias, (const void*)w_post, (const void*)w_next, (void*)h, width, eps, mult, offset,
+                     (const void*)o2, s1, s2);
     return;
   }
   SM_DISPATCH_V(f32, width % 8 == 0, sm_post_norm_add_kernel, dim3(rows), dim3(256), 0, stream, (float*)x,

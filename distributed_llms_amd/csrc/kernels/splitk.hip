@@ -124,30 +124,25 @@ __global__ void __launch_bounds__(NTH) splitk_add_rms_norm_kernel(bf16* __restri
     f32x4 a0[CH], a1[CH];
     bf16x8 b[CH];
     if constexpr (SC > 0) {
-      f32x4 l0[CH][SC], l1[CH][SC];
+      typedef part_elem raw __attribute__((ext_vector_type(8)));
+      raw l[CH][SC];
 #pragma unroll
       for (int i = 0; i < CH; ++i) {
         const int idc = min((int)threadIdx.x + (c0 + i) * NTH, nvec - 1);
-        const size_t p = (size_t)row * N + idc * 8;
-#pragma unroll
-        for (int s = 0; s < SC; ++s) {
-          l0[i][s] = part_load4<true>(P, p + s * slab);
-          l1[i][s] = part_load4<true>(P, p + s * slab + 4);
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < CH; ++i) {
-        const int idc = min((int)threadIdx.x + (c0 + i) * NTH, nvec - 1);
+        const part_elem* p = reinterpret_cast<const part_elem*>(P) + (size_t)row * N + idc * 8;
         b[i] = rr[idc];
+#pragma unroll
+        for (int s = 0; s < SC; ++s) l[i][s] = __builtin_nontemporal_load(reinterpret_cast<const raw*>(p + s * slab));
       }
+      __builtin_amdgcn_sched_barrier(0);   // (hipcc kept 8 of the loads back until the first had come in)
 #pragma unroll
       for (int i = 0; i < CH; ++i) {
         a0[i] = f32x4{0.f, 0.f, 0.f, 0.f};
         a1[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int s = 0; s < SC; ++s) {   // same slab order as the runtime loop: bit-identical sums
-          a0[i] += l0[i][s];
-          a1[i] += l1[i][s];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) a0[i][j] += part_value(l[i][s][j]), a1[i][j] += part_value(l[i][s][j + 4]);
         }
       }
     } else {
@@ -183,10 +178,10 @@ __global__ void __launch_bounds__(NTH) splitk_add_rms_norm_kernel(bf16* __restri
       }
     }
   }
-  ss = block_sum(ss, red);
+  ss = block_sum<NTH>(ss, red);
   const float inv = rsqrtf(ss / (float)N + eps);
   if (q8) {   // FP8 consumer: per-token e4m3 of the normalised row (rms_norm_kernel's epilogue)
-    norm_out_fp8<MAXV, NTH>(v, inv, wv, nvec, y ? y + (size_t)row * N : nullptr, q8 + (size_t)row * N, qs + row,
+    norm_out_fp8<MAXV, NTH>(v, inv, g, nvec, y ? y + (size_t)row * N : nullptr, q8 + (size_t)row * N, qs + row,
                             red);
     return;
   }
