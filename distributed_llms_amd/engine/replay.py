@@ -79,9 +79,17 @@ class TraceReplayer:
                 hb.logits_idx = np.arange(hb.num_seqs, dtype=np.int32)
             eng.step_id += 1
             out = eng.runner.execute(hb, slot=0)
-            if wanted:
-                logits = out.float() if hb.is_prefill else out.float().index_select(
-                    0, torch.as_tensor(wanted, dtype=torch.int64, device=out.device))
+            if wanted and hb.is_prefill:
+                logits = out.float()
+            elif wanted and wanted == list(range(hb.num_seqs)):
+                # every row in order, the usual step: no gather, and no upload of its indexes, which -- from pageable
+                # memory -- held the host until the step was done.  A copy: a graph's output is overwritten by the next
+                logits = out.to(torch.float32, copy=True)
+            elif wanted:
+                idx = torch.tensor(wanted, dtype=torch.int64)
+                if out.is_cuda:
+                    idx = idx.pin_memory().to(out.device, non_blocking=True)
+                logits = out.index_select(0, idx).float()
             for _, s, n in order:
                 s.num_cached += n
                 s.chunk = 0
