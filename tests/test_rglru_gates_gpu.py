@@ -1,0 +1,40 @@
+"""The gates of the recurrence over many tokens on the bf16 matrix cores, against 64-bit sums."""
+import pytest
+import torch
+
+from distributed_llms_amd import _ext
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("nb,bw", [(1, 8), (2, 40), (1, 100), (1, 15), (4, 128), (3, 264), (2, 512)])
+@pytest.mark.parametrize("tokens", [65, 128, 129, 300])
+@pytest.mark.parametrize("size", [1e-3, 1.0, 30.0])
+def test_gates_keep_all_bits_of_the_input(cuda, nb, bw, tokens, size):
+    """Partial tiles of tokens, outputs and K chunks; the three bf16 pieces of an input carry all of its 24 bits."""
+    g = torch.Generator().manual_seed(bw + tokens)
+    r = lambda *s, scale=1.0: torch.randn(*s, generator=g) * scale
+    u = r(tokens, nb, bw, scale=size)
+    ra, ri = r(nb, bw, bw, scale=bw ** -0.5).bfloat16(), r(nb, bw, bw, scale=bw ** -0.5).bfloat16()
+    rb, ib, lam = r(nb, bw, scale=0.3).bfloat16(), r(nb, bw, scale=0.3).bfloat16(), r(nb, bw).bfloat16()
+    a, y = (torch.full((tokens, nb * bw), float("nan"), device=cuda) for _ in range(2))
+    d = [x.to(cuda).contiguous() for x in (u, ra, rb, ri, ib, lam)]
+    torch.cuda.synchronize()
+    _ext.kernels().sm_rglru_gates(a.data_ptr(), y.data_ptr(), *(x.data_ptr() for x in d), tokens, nb, bw, 8.0, 0,
+                                  torch.cuda.current_stream().cuda_stream)
+    mul = lambda w: torch.matmul(u.double().transpose(0, 1), w.double()).transpose(0, 1)
+    # the sums: exact products, bw float32 additions of at most the row's absolute sum each, 2^-24 apart
+    bound = lambda w: torch.matmul(u.double().abs().transpose(0, 1), w.double().abs()).transpose(0, 1) * (3 * bw + 8) * 2.0 ** -24
+    zr, zi = mul(ra) + rb.double(), mul(ri) + ib.double()
+    sp = torch.nn.functional.softplus(lam.double())
+    at = lambda z: torch.exp(-8.0 * torch.sigmoid(z) * sp)
+    want = at(zr)
+    # a falls by at most 2 sp = 8 sp / 4 per unit of its sum; as much as 1e-5 of the exponent for the float32 functions
+    slack = want * (2 * sp * bound(ra) + 1e-5 * (1 + 8 * sp)) + 1e-12
+    assert ((a.cpu().double().view(tokens, nb, bw) - want).abs() <= slack).all()
+    x = u.double()
+    mult = lambda v: torch.sqrt((1 - v * v).clamp_min(0))
+    lo, hi = mult((want + slack).clamp_max(1)), mult((want - slack).clamp_min(0))
+    gate, dg = torch.sigmoid(zi), bound(ri) / 4 + 1e-6
+    err = (y.cpu().double().view(tokens, nb, bw) - mult(want) * gate * x).abs()
+    assert (err <= ((hi - lo) * gate + dg + 1e-6) * x.abs() + 1e-12).all()
