@@ -18,7 +18,7 @@ import torch
 
 from distributed_llms_amd.ops import gemm
 
-CASES = [  # name, M, N, K, swiglu, splits, variant (| 64: schedule 2, | 16 / 32: schedule-1 ablations)
+CASES = [  # name, M, N, K, swiglu, splits, variant (| 64: schedule 2)
     ("gate_up dec S2", 256, 28672, 4096, True, 2, 64), ("gate_up dec", 256, 28672, 4096, True, 1, 1),
     ("gate pf S2", 8192, 14336, 4096, False, 1, 68), ("gate pf", 8192, 14336, 4096, False, 1, 4),
     ("gate pf S2 BN128", 8192, 14336, 4096, False, 1, 69),
@@ -49,10 +49,9 @@ def main():
         def run(var):
             return gemm.linear_pp(x, ws_[next(it) % copies], splits=s, swiglu=sw, variant=var)
         for _ in range(10):
-            run((v & 7) | 8 | (v & 112))
+            run((v & 7) | 8 | (v & 64))
         torch.cuda.synchronize()
         bn = 128 if v & 1 else 256
-        # ablations time the diagnostic build itself (their output is garbage)
         grid = (n // bn) * (-(-m // 256)) * s
         full = gemm._workspace(dev)[-grid * 512:].view(grid * 4, 128).cpu()
         rec = full[:, :4]
@@ -63,7 +62,7 @@ def main():
         ideal = 2 * 8 * (bn // 32) * 16
         per = (tot / nt).tolist()
         frac = (bt / tot).tolist()
-        t_real = timed(lambda: run((v & 7) | (v & 64) | (8 | (v & 48) if v & 48 else 0)))
+        t_real = timed(lambda: run((v & 7) | (v & 64)))
         wg_us = (rt_ns / 1e3).view(-1, 4).max(dim=1).values
         print(f"{name:12s} M={m:5d} N={n:5d} K={k:5d} S={s:2d} BN={bn} var={v}: kernel {t_real:7.1f} us "
               f"({2.0 * m * n * k / t_real / 1e6:5.0f} TF) | WG loop median {statistics.median(wg_us.tolist()):6.1f} us, "

@@ -166,8 +166,6 @@ __global__ void __launch_bounds__(256, 1) gemm_pp_kernel(const bf16* __restrict_
   constexpr int G = GA + GB;
   constexpr bool NT = (VAR & 1) != 0, GROUPED = (VAR & 2) != 0;
   constexpr bool PROF = (VAR & 4) != 0;                // diagnostic build: cycle stamps around B_t
-  // diagnostic ablations (wrong results, timing only): no LDS-DMA pieces / no fragment reads in the loop
-  constexpr bool NOLOAD = (VAR & 8) != 0, NOREAD = (VAR & 16) != 0;
   // schedule 2 (VAR 32): a K-tile's fragments are all read into registers early in its first K-half,
   // so its slot is re-staged from then on -- LDS-DMA pieces spread over ~60 % of the K-tile instead
   // of bunched into half of K-half 1 (see the loop)
@@ -384,7 +382,7 @@ __global__ void __launch_bounds__(256, 1) gemm_pp_kernel(const bf16* __restrict_
         else
           acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb1[c], fa1[r], acc[r][c], 0, 0, 0);
         if constexpr (i % 2 == 1 && i / 2 < NR) {
-          if constexpr (!NOREAD) rd1(base1, std::integral_constant<int, i / 2>{});
+          rd1(base1, std::integral_constant<int, i / 2>{});
         }
         if constexpr (i == IB1) {
           if constexpr (PROF) asm volatile("s_memtime %0\n\ts_waitcnt lgkmcnt(0)" : "=s"(sb0) :: "memory");
@@ -400,7 +398,7 @@ __global__ void __launch_bounds__(256, 1) gemm_pp_kernel(const bf16* __restrict_
           }
         }
         if constexpr (i > IB1 && (i - IB1 - 1) % GE == 0 && (i - IB1 - 1) / GE < G) {
-          if constexpr (!NOLOAD) piece(slot, t + NB, (i - IB1 - 1) / GE);
+          piece(slot, t + NB, (i - IB1 - 1) / GE);
         }
         if constexpr (i == IB3) {
           if constexpr (PROF) asm volatile("s_memtime %0\n\ts_waitcnt lgkmcnt(0)" : "=s"(sb0) :: "memory");
@@ -416,7 +414,7 @@ __global__ void __launch_bounds__(256, 1) gemm_pp_kernel(const bf16* __restrict_
           }
         }
         if constexpr (i > IB3 && (i - IB3 - 1) % 2 == 0 && (i - IB3 - 1) / 2 < NR) {
-          if constexpr (!NOREAD) rd0(base0, std::integral_constant<int, (i - IB3 - 1) / 2>{});
+          rd0(base0, std::integral_constant<int, (i - IB3 - 1) / 2>{});
         }
         __builtin_amdgcn_sched_barrier(0);
       });
@@ -488,10 +486,10 @@ __global__ void __launch_bounds__(256, 1) gemm_pp_kernel(const bf16* __restrict_
           acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb0[c], fa0[r], acc[r][c], 0, 0, 0);
 #pragma unroll
           for (int a = 0; a < RT; ++a)
-            if (!NOREAD && SC::pos(0, 0, a) == i) fa1[a] = pp_frag_dyn(base + a_off + a * 16 * 128);
+            if (SC::pos(0, 0, a) == i) fa1[a] = pp_frag_dyn(base + a_off + a * 16 * 128);
 #pragma unroll
           for (int b = 0; b < CT; ++b)
-            if (!NOREAD && SC::pos(0, 1, b) == i) fb1[b] = pp_frag_dyn(base + b_off + b * 16 * 128);
+            if (SC::pos(0, 1, b) == i) fb1[b] = pp_frag_dyn(base + b_off + b * 16 * 128);
           __builtin_amdgcn_sched_barrier(0);
         });
       }
@@ -523,13 +521,13 @@ __global__ void __launch_bounds__(256, 1) gemm_pp_kernel(const bf16* __restrict_
             }
           }
           if constexpr (i >= SC::EB - 1 && (i - SC::EB + 1) % GE == 0 && (i - SC::EB + 1) / GE < G)
-            if constexpr (!NOLOAD) piece(slot, t + NB, (i - SC::EB + 1) / GE);
+            piece(slot, t + NB, (i - SC::EB + 1) / GE);
 #pragma unroll
           for (int a = 0; a < RT; ++a)
-            if (!NOREAD && SC::pos(1, 0, a) == i) fa0[a] = pp_frag_dyn(base + a_off + a * 16 * 128);
+            if (SC::pos(1, 0, a) == i) fa0[a] = pp_frag_dyn(base + a_off + a * 16 * 128);
 #pragma unroll
           for (int b = 0; b < CT; ++b)
-            if (!NOREAD && SC::pos(1, 1, b) == i) fb0[b] = pp_frag_dyn(base + b_off + b * 16 * 128);
+            if (SC::pos(1, 1, b) == i) fb0[b] = pp_frag_dyn(base + b_off + b * 16 * 128);
           __builtin_amdgcn_sched_barrier(0);
         });
       }
@@ -661,9 +659,7 @@ int gemm_pp(uintptr_t c, uintptr_t a, uintptr_t b, uintptr_t ws, long ws_floats,
                      (const int*)nullptr, (const int*)nullptr, 0, 0.f)
   // variant bit 6: schedule 2 (the K-tile's fragments read early, staging spread; weights
   // nontemporal with bit 1 only in the natural tile order).  Bit 3: diagnostic build -- per-wave cycle stamps (loop, B_t waits) into the LAST
-  // grid x 512 floats of ws (after the slabs); output as usual.  With it (schedule 1 only), bit 4:
-  // no LDS-DMA pieces in the loop, bit 5: no fragment reads in the loop (ablations: wrong results,
-  // timing only)
+  // grid x 512 floats of ws (after the slabs); output as usual
   const bool sched2 = (variant & 64) != 0;
   const bool prof = (variant & 8) != 0;
   float* dbg = nullptr;
@@ -680,8 +676,6 @@ int gemm_pp(uintptr_t c, uintptr_t a, uintptr_t b, uintptr_t ws, long ws_floats,
       else DLLM_PP_GO(BN_, MODE_, 32);                               \
     } else if (prof) {                                               \
       if (grp) DLLM_PP_GO(BN_, MODE_, 6);                            \
-      else if (variant & 16) DLLM_PP_GO(BN_, MODE_, 12);             \
-      else if (variant & 32) DLLM_PP_GO(BN_, MODE_, 20);             \
       else DLLM_PP_GO(BN_, MODE_, 4);                                \
     }                                                                \
     else if (grp) { if (nt) DLLM_PP_GO(BN_, MODE_, 3); else DLLM_PP_GO(BN_, MODE_, 2); } \

@@ -90,8 +90,6 @@ __global__ void __launch_bounds__(512, 1) gemm_sq_kernel(const bf16* __restrict_
   // weights streamed nontemporally (read once) where the grid has no K split (VAR 2)
   constexpr int BAUX = (VAR & 3) == 2 ? 2 : 0;
   constexpr bool EARLY = (VAR & 4) != 0;
-  constexpr bool NOSTAGE = (VAR & 8) != 0;      // ablation (wrong results): no staging in the loop
-  constexpr bool NOPIN = (VAR & 16) != 0;       // ablation: no sched_barrier between substeps
   auto piece = [&](bf16* base, int ko, int p) {
     if (p < QAI)
       __builtin_amdgcn_global_load_lds((glb_vptr_q)(A + offA[p] + ko), (lds_vptr_q)(base + (wv * QAI + p) * 512), 16,
@@ -115,7 +113,7 @@ __global__ void __launch_bounds__(512, 1) gemm_sq_kernel(const bf16* __restrict_
     const bf16* sb = sa + QAEL;
     constexpr int NMF = 2 * QRT * QCT;        // 64 MFMAs per wave per K-tile
     constexpr int EVERY = NMF / (QG + 1);     // one staging piece every 7 MFMAs
-    if constexpr (STG && EARLY && !NOSTAGE) {
+    if constexpr (STG && EARLY) {
 #pragma unroll
       for (int p = 0; p < QG; ++p) piece(dst, ko, p);
     }
@@ -137,7 +135,7 @@ __global__ void __launch_bounds__(512, 1) gemm_sq_kernel(const bf16* __restrict_
 #pragma unroll
         for (int ct = 0; ct < QCT; ++ct) {
           acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[rt], fb[ct], acc[rt][ct], 0, 0, 0);
-          if constexpr (STG && !EARLY && !NOSTAGE) {
+          if constexpr (STG && !EARLY) {
             const int i = (s * QRT + rt) * QCT + ct + 1;
             if (i % EVERY == 0 && i / EVERY <= QG) piece(dst, ko, i / EVERY - 1);
           }
@@ -145,7 +143,7 @@ __global__ void __launch_bounds__(512, 1) gemm_sq_kernel(const bf16* __restrict_
       // keep the next substep's 12 fragment reads below this one's MFMAs: hoisting them would
       // need 48 more VGPRs than the 256 a 2-wave-per-SIMD workgroup has (128 go to accumulators);
       // the partner wave on the SIMD covers their latency
-      if constexpr (!NOPIN) __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
 
@@ -226,9 +224,7 @@ int gemm_sq(uintptr_t c, uintptr_t a, uintptr_t b, uintptr_t ws, long ws_floats,
   }
   DLLM_HOST_CHECK(ws != 0 && (long)S * M * N <= ws_floats, "split-K workspace too small");
   // split: natural column order (the SwiGLU, if any, is applied by the reduce)
-  if (variant == 12) DLLM_SQ_GO(true, false, 13);        // ablations (A/B only)
-  else if (variant == 20) DLLM_SQ_GO(true, false, 21);
-  else if (early) DLLM_SQ_GO(true, false, 5);
+  if (early) DLLM_SQ_GO(true, false, 5);
   else DLLM_SQ_GO(true, false, 1);
 #undef DLLM_SQ_GO
   DLLM_HIP_CHECK(hipGetLastError());
