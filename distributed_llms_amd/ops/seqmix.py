@@ -453,12 +453,16 @@ _arrived = {}
 
 def _arrival_counts(device: torch.device, n: int) -> torch.Tensor:
     """Zeroed counters of the current stream, which every launch leaves zeroed (launches on one stream follow each other;
-    graphs keep those of the stream they were captured on, as they do the split-K workspace)."""
+    graphs keep those of the stream they were captured on, as they do the split-K workspace).  Counters that became too
+    few stay allocated, since graphs captured before still count in them; each is twice the last, so their sum is bounded."""
     key = (device.index or 0, torch.cuda.current_stream().cuda_stream)
-    t = _arrived.get(key)
-    if t is None or t.numel() < n:
-        t = _arrived[key] = torch.zeros(max(n, 1 << 16), dtype=torch.int32, device=device)
-    return t
+    kept = _arrived.setdefault(key, [])
+    if not kept or kept[-1].numel() < n:
+        if torch.cuda.is_current_stream_capturing():     # cleared by the graph itself, at every replay, and its own
+            return torch.zeros(n, dtype=torch.int32, device=device)
+        size = max(n, 2 * kept[-1].numel() if kept else 1 << 16)
+        kept.append(torch.zeros(size, dtype=torch.int32, device=device))
+    return kept[-1]
 
 
 def rglru_step(yx: torch.Tensor, conv_w: torch.Tensor, conv_b: torch.Tensor, x_b: torch.Tensor, conv_state: torch.Tensor,
@@ -486,7 +490,8 @@ def rglru_step(yx: torch.Tensor, conv_w: torch.Tensor, conv_b: torch.Tensor, x_b
     arrived = _arrival_counts(yx.device, sb.num_seqs * nb * 32)
     _k().sm_rglru_step(out.data_ptr(), yx.data_ptr() + c * e, yx.data_ptr(), yx.stride(0), conv_w.data_ptr(), conv_b.data_ptr(),
                        x_b.data_ptr(), conv_state.data_ptr(), ra_t.data_ptr(), ra_b.data_ptr(), ri_t.data_ptr(),
-                       ri_b.data_ptr(), lam.data_ptr(), y_b.data_ptr(), state.data_ptr(), sb.positions.data_ptr(), sb.state_slots.data_ptr(), sb.num_seqs, nb, bw, taps, float(decay_scale),
+                       ri_b.data_ptr(), lam.data_ptr(), y_b.data_ptr(), state.data_ptr(), sb.positions.data_ptr(),
+                       sb.state_slots.data_ptr(), sb.num_seqs, nb, bw, taps, float(decay_scale),
                        arrived.data_ptr(), arrived.numel(), _f32flag(yx), _stream())
     return out
 

@@ -76,6 +76,41 @@ def test_attention_input_moves_the_tail(cuda, dtype, taps, dim, vdim):
 
 
 @gpu
+@pytest.mark.parametrize("warm", [True, False])
+def test_rglru_step_graph_outlives_its_counters_successor(cuda, warm):
+    """A graph captured with few sequences still has its arrival counters after a larger batch on the same stream needed
+    more of them, whatever was allocated since; so has one captured on a stream that had none yet."""
+    nb, bw, taps, c = 10, 8, 4, 80
+    r = lambda *s: torch.randn(*s, device=cuda).bfloat16()
+    ops_ = [r(taps, c), r(c), r(c)], [r(c), r(nb, bw, bw), r(nb, bw), r(nb, bw, bw), r(nb, bw), r(c)]
+    state0, conv0, yx = torch.randn(301, c, device=cuda), r(301, taps - 1, c), r(300, 2 * c)
+    run = lambda n, conv, state, sb: sm.rglru_step(yx[:n], *ops_[0], conv, *ops_[1], state, sb)
+    few, many = _sb([5, 9, 7], [1, 2, 3], cuda), _sb([5] * 300, list(range(1, 301)), cuda)
+    conv, state = conv0.clone(), state0.clone()
+    torch.cuda.synchronize()
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        if warm:
+            want = run(3, conv, state, few), conv.clone(), state.clone()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            out = run(3, conv, state, few)
+        run(300, conv0.clone(), state0.clone(), many)            # 300 x 10 counters: more than the first buffer holds
+        s.synchronize()
+        if not warm:
+            want = run(3, conv, state, few), conv.clone(), state.clone()
+        taken = [torch.full((1 << 16,), 7, dtype=torch.int32, device=cuda) for _ in range(8)]
+        for _ in range(3):
+            conv.copy_(conv0)
+            state.copy_(state0)
+            g.replay()
+            s.synchronize()
+            for a, b in zip((out, conv, state), want):
+                assert torch.equal(a, b)
+    del taken
+
+
+@gpu
 @pytest.mark.parametrize("rows", [1, 7, 300])
 @pytest.mark.parametrize("width", [4, 250, 1024, 2560, 4100, 16384, 16392])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
