@@ -58,6 +58,17 @@ def _cus(device) -> int:
 _CUS = {}
 
 
+def _sizes(x: torch.Tensor, w: torch.Tensor, name: str):
+    """(rows, N, K) of ``x w^T``; raises where the kernels, which see pointers and these numbers alone, would read past
+    ``w`` or another device's memory."""
+    k = x.shape[-1]
+    if w.dim() != 2 or w.shape[1] != k:
+        raise ValueError(f"{name}: x[..., {k}] vs w {tuple(w.shape)}")
+    if w.device != x.device:
+        raise ValueError(f"{name}: x on {x.device}, w on {w.device}")
+    return x.numel() // k, w.shape[0], k
+
+
 def pf_fills(m: int, n: int, device) -> bool:
     """gemm_pf (one 256 x 256 tile per CU per round, no split-K) only where its grid fills the chip:
     at least one tile per CU and rounds that are mostly full (knobs.pf_min_eff), or many rounds.
@@ -129,8 +140,8 @@ def use_stream(m: int, n: int, k: int, x: torch.Tensor, w: torch.Tensor, bias=No
 def linear_into_norm(x: torch.Tensor, w: torch.Tensor):
     """``x w^T`` for a consumer that sums split-K slabs itself (post_norm_add, post_layer_norm_add): the finished product
     where the weight-streaming kernel is faster than the split grid alone, else possibly a :class:`SplitKPartial`."""
-    k = x.shape[-1]
-    if use_stream(x.numel() // k, w.shape[0], k, x, w, defer=True):
+    m, n, k = _sizes(x, w, "linear_into_norm")
+    if use_stream(m, n, k, x, w, defer=True):
         return linear_stream(x, w)
     return linear(x, w, defer=True)
 
@@ -141,9 +152,7 @@ _STREAM_GLU = {"": 0, "silu": 1, "clipped": 2, "gelu": 3}
 def linear_stream(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, glu: str = "",
                   limit: float = 0.0) -> torch.Tensor:
     """y = x w^T (+ bias), or its GLU with w = [Wg; Wu], for up to 64 rows (csrc/kernels/gemm_stream.hip)."""
-    k = x.shape[-1]
-    n = w.shape[0]
-    m = x.numel() // k
+    m, n, k = _sizes(x, w, "linear_stream")
     y = torch.empty(*x.shape[:-1], n // 2 if glu else n, dtype=x.dtype, device=x.device)
     _ext.kernels().gemm_stream(y.data_ptr(), x.data_ptr(), w.data_ptr(), 0 if bias is None else bias.data_ptr(), m, n, k,
                                _STREAM_GLU[glu], 1 if n * k * 2 >= WIDE_NT_MIN_BYTES else 0, float(limit),
@@ -176,11 +185,7 @@ class SplitKPartial:
 
 def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, defer: bool = False):
     """y = x w^T (+bias).  ``defer``: may return a :class:`SplitKPartial` (see there)."""
-    k = x.shape[-1]
-    n = w.shape[0]
-    m = x.numel() // k
-    if w.shape[1] != k:
-        raise ValueError(f"linear: x[..., {k}] vs w {tuple(w.shape)}")
+    m, n, k = _sizes(x, w, "linear")
     kn = knobs.K
     if not (defer and n % 128 == 0) and use_stream(m, n, k, x, w, bias):
         return linear_stream(x, w, bias)
@@ -468,9 +473,7 @@ def _linear_glu(x: torch.Tensor, w_gate_up: torch.Tensor, limit: Optional[float]
     """A GLU of x Wg^T and x Wu^T, W = [Wg; Wu], with the activation in the weight-streaming GEMM's epilogue (up to 64
     rows; the only form that takes a ``bias`` [gate | up]), in the persistent GEMM's (prompts) or in the split-K
     reduction (decode): clipped (``limit``) or gelu_tanh (None); None if the shape takes none of them."""
-    k = x.shape[-1]
-    n = w_gate_up.shape[0]
-    m = x.numel() // k
+    m, n, k = _sizes(x, w_gate_up, "linear_glu")
     glu = "gelu" if limit is None else "clipped"
     if n % 2 == 0 and use_stream(m, n, k, x, w_gate_up, bias, glu):
         return linear_stream(x, w_gate_up, bias, glu, 0.0 if limit is None else limit)
@@ -506,9 +509,7 @@ def linear_gelu_glu(x: torch.Tensor, w_gate_up: torch.Tensor) -> Optional[torch.
 
 def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor) -> Optional[torch.Tensor]:
     """silu(x Wg^T) * (x Wu^T) with W = [Wg; Wu] in one launch; None if the shape is not eligible."""
-    k = x.shape[-1]
-    n = w_gate_up.shape[0]
-    m = x.numel() // k
+    m, n, k = _sizes(x, w_gate_up, "linear_swiglu")
     kn = knobs.K
     if n % 2 == 0 and use_stream(m, n, k, x, w_gate_up, glu="silu"):
         return linear_stream(x, w_gate_up, glu="silu")
