@@ -134,7 +134,8 @@ def stream_fits(m: int, n: int, k: int, glu: str = "", defer: bool = False) -> b
 def use_stream(m: int, n: int, k: int, x: torch.Tensor, w: torch.Tensor, bias=None, glu: str = "", defer: bool = False) -> bool:
     return (knobs.K.stream and stream_fits(m, n, k, glu, defer) and x.dtype == w.dtype == torch.bfloat16
             and x.is_contiguous() and w.is_contiguous() and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
-            and (bias is None or (bias.dtype == torch.bfloat16 and bias.is_contiguous())))
+            and (bias is None or (bias.dtype == torch.bfloat16 and tuple(bias.shape) == (n,) and bias.is_contiguous()
+                                  and bias.device == x.device)))
 
 
 def linear_into_norm(x: torch.Tensor, w: torch.Tensor):

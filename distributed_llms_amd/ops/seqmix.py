@@ -518,6 +518,9 @@ def linear_clipped_glu(x: torch.Tensor, w_gate_up: torch.Tensor, bias_gu: Option
     """:func:`clipped_glu` of ``x W^T``, W = [Wg; Wu]: in a GEMM epilogue where one takes the shape and the bias, else the
     projection followed by the gate kernel."""
     from . import gemm, linear
+    if bias_gu is not None and (tuple(bias_gu.shape) != (w_gate_up.shape[0],) or bias_gu.dtype != x.dtype
+                                or bias_gu.device != x.device):
+        raise ValueError(f"linear_clipped_glu: bias [{w_gate_up.shape[0]}] of x's type and device")
     y = gemm.linear_clipped_glu(x, w_gate_up, limit, bias_gu) if x.is_cuda else None
     return clipped_glu(linear(x, w_gate_up), bias_gu, limit) if y is None else y
 

@@ -3,8 +3,11 @@ The kernel entry points are stubbed, so that nothing is launched: the calls run 
 import pytest
 import torch
 
-from distributed_llms_amd import _ext, ops
+import torch.nn.functional as F
+
+from distributed_llms_amd import _ext
 from distributed_llms_amd.ops import gemm
+from distributed_llms_amd.ops import seqmix as sm
 
 
 class _Launches:
@@ -47,4 +50,28 @@ def test_operands_that_do_not_match_are_refused(launches, name, w):
 def test_operands_on_two_devices_are_refused(launches, name):
     with pytest.raises(ValueError):
         GLU[name](_bf(4, 1024), torch.empty(512, 1024, dtype=torch.bfloat16, device="meta"))
+    assert not launches
+
+
+def test_bias_of_another_shape_goes_to_the_general_route(launches):
+    """A bias that is not one element per output: added by its broadcast, or refused, as F.linear has it."""
+    x, w = torch.randn(4, 1024).bfloat16(), torch.randn(512, 1024).bfloat16()
+    for b in (torch.randn(1), torch.randn(4, 512), torch.randn(4, 1), torch.randn(1, 512)):
+        assert torch.equal(gemm.linear(x, w, b.bfloat16()), F.linear(x, w, b.bfloat16()))
+    for n in (0, 511, 513):
+        with pytest.raises(RuntimeError):
+            gemm.linear(x, w, _bf(n))
+    with pytest.raises(RuntimeError):
+        gemm.linear(x, w, torch.empty(512, dtype=torch.bfloat16, device="meta")).sum().item()
+    assert not launches
+    gemm.linear(x, w, _bf(512))
+    assert [n for n, _ in launches] == ["gemm_stream"]
+
+
+@pytest.mark.parametrize("bias", [_bf(1), _bf(511), _bf(1, 512), torch.zeros(512),
+                                  torch.empty(512, dtype=torch.bfloat16, device="meta")])
+def test_glu_bias_that_does_not_fit_is_refused(launches, bias):
+    assert gemm.linear_clipped_glu(_bf(4, 1024), _bf(512, 1024), 7.0, bias) is None
+    with pytest.raises(ValueError):
+        sm.linear_clipped_glu(_bf(4, 1024), _bf(512, 1024), bias, 7.0)
     assert not launches
