@@ -34,6 +34,7 @@ from typing import Optional
 
 import torch
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 
 from .. import _ext
 from .. import knobs
@@ -131,8 +132,18 @@ def stream_fits(m: int, n: int, k: int, glu: str = "", defer: bool = False) -> b
     return n * k <= (STREAM_PLAIN_32 if m <= 32 else STREAM_PLAIN)
 
 
+def _recorded(*tensors) -> bool:
+    """Is the call differentiated or transformed (autograd, forward mode, vmap)?  The kernels leave no trace of it."""
+    for t in tensors:
+        if t is not None and (torch._C._functorch.is_functorch_wrapped_tensor(t)
+                              or (t.requires_grad and torch.is_grad_enabled())
+                              or (forward_ad._current_level >= 0 and forward_ad.unpack_dual(t).tangent is not None)):
+            return True
+    return False
+
+
 def use_stream(m: int, n: int, k: int, x: torch.Tensor, w: torch.Tensor, bias=None, glu: str = "", defer: bool = False) -> bool:
-    return (knobs.K.stream and stream_fits(m, n, k, glu, defer) and x.dtype == w.dtype == torch.bfloat16
+    return (knobs.K.stream and stream_fits(m, n, k, glu, defer) and not _recorded(x, w, bias) and x.dtype == w.dtype == torch.bfloat16
             and x.is_contiguous() and w.is_contiguous() and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
             and (bias is None or (bias.dtype == torch.bfloat16 and tuple(bias.shape) == (n,) and bias.is_contiguous()
                                   and bias.device == x.device)))

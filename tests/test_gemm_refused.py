@@ -75,3 +75,26 @@ def test_glu_bias_that_does_not_fit_is_refused(launches, bias):
     with pytest.raises(ValueError):
         sm.linear_clipped_glu(_bf(4, 1024), _bf(512, 1024), bias, 7.0)
     assert not launches
+
+
+def test_recorded_calls_keep_their_derivatives(launches):
+    """What F.linear differentiates or maps over is not taken from it: autograd, forward mode, vmap (N = 500 or a bias: the
+    shapes of no other kernel)."""
+    from torch.autograd import forward_ad
+    x, w, b = torch.randn(4, 1024).bfloat16(), torch.randn(500, 1024).bfloat16(), torch.randn(500).bfloat16()
+    for which in range(3):
+        t = [x, w, b]
+        t[which] = t[which].clone().requires_grad_()
+        gemm.linear(*t).sum().backward()
+        want = [x, w, b]
+        want[which] = want[which].clone().requires_grad_()
+        F.linear(*want).sum().backward()
+        assert torch.equal(t[which].grad, want[which].grad)
+    with forward_ad.dual_level():
+        y = gemm.linear(forward_ad.make_dual(x, torch.ones_like(x)), w, b)
+        assert torch.equal(forward_ad.unpack_dual(y).tangent, F.linear(torch.ones_like(x), w))
+    assert torch.equal(torch.vmap(lambda v: gemm.linear(v, w, b))(x), torch.vmap(lambda v: F.linear(v, w, b))(x))
+    assert not launches
+    with torch.no_grad():
+        gemm.linear(x.clone().requires_grad_(), w, b)
+    assert [n for n, _ in launches] == ["gemm_stream"]
