@@ -148,6 +148,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
 
 def linear_into_norm(x: torch.Tensor, w: torch.Tensor):
     """:func:`linear` for a consumer that takes a :class:`gemm.SplitKPartial` (the closing norm of a sublayer)."""
+    if isinstance(w, quant.Fp8Weight):
+        return linear(x, w, defer=True)
     return gemm.linear_into_norm(x, w) if _gpu(x) else ref.linear(x, w)
 
 

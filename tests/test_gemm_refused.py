@@ -98,3 +98,11 @@ def test_recorded_calls_keep_their_derivatives(launches):
     with torch.no_grad():
         gemm.linear(x.clone().requires_grad_(), w, b)
     assert [n for n, _ in launches] == ["gemm_stream"]
+
+
+def test_fp8_weight_in_front_of_a_norm():
+    """linear_into_norm takes what linear(defer=True) takes: an fp8 weight too (latent_attention's output projection)."""
+    from distributed_llms_amd import ops
+    from distributed_llms_amd.ops import quant
+    x, w = torch.randn(4, 256).bfloat16(), quant.quantize_weight(torch.randn(128, 256).bfloat16())
+    assert torch.equal(ops.linear_into_norm(x, w), ops.linear(x, w, defer=True))
