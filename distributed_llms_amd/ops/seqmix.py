@@ -57,7 +57,7 @@ def _k():
     return _ext.kernels()
 
 
-def _f32flag(t: torch.Tensor) -> int:
+def _f32flag(t) -> int:
     if t.dtype not in ACT_DTYPES:
         raise TypeError(f"activation dtype {t.dtype} (bfloat16 or float32)")
     return 1 if t.dtype == torch.float32 else 0
@@ -170,9 +170,9 @@ def post_norm_add(x: torch.Tensor, o, w_post: torch.Tensor, eps: float, mult: fl
     h = None
     if w_next is not None or (plain_next and o.dtype != torch.float32):
         h = torch.empty(t, width, dtype=o.dtype, device=x.device)
-    _k().sm_post_norm_add(x.data_ptr(), (part.ws if part is not None else o).data_ptr(), 0 if part is None else part.splits, _ptr(bias), w_post.data_ptr(), _ptr(w_next), _ptr(h), t, width,
-                          float(eps), float(mult), off, _ptr(o2), float(scales[0]), float(scales[1]),
-                          1 if o.dtype == torch.float32 else 0, _stream())
+    _k().sm_post_norm_add(x.data_ptr(), (part.ws if part is not None else o).data_ptr(), 0 if part is None else part.splits,
+                          _ptr(bias), w_post.data_ptr(), _ptr(w_next), _ptr(h), t, width, float(eps), float(mult), off,
+                          _ptr(o2), float(scales[0]), float(scales[1]), _f32flag(o), _stream())
     return x, (x if (plain_next and w_next is None and h is None) else h)
 
 

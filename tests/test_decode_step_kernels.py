@@ -133,6 +133,13 @@ def test_post_norm_add_rows(cuda, rows, width, dtype, form):
 
 
 @gpu
+def test_post_norm_add_refuses_other_types(cuda):
+    x, o, w = torch.zeros(3, 64, device=cuda), torch.zeros(3, 64, device=cuda).half(), torch.zeros(64, device=cuda).half()
+    with pytest.raises(TypeError):
+        sm.post_norm_add(x, o, w, 1e-6, 1.0)
+
+
+@gpu
 @pytest.mark.parametrize("tokens,width,k", [(1, 256, 1024), (16, 2560, 7680), (40, 4096, 2048)])
 def test_post_norm_add_sums_split_products(cuda, tokens, width, k):
     """On a split-K product that is not reduced yet, against the same on the reduced one: the slabs are summed in the same
