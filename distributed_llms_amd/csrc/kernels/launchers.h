@@ -133,7 +133,8 @@ void sm_rglru_scan(uintptr_t out, uintptr_t a, uintptr_t g, uintptr_t y_raw, lon
 void sm_rglru_step(uintptr_t out, uintptr_t x, uintptr_t y, long ld, uintptr_t conv_w, uintptr_t conv_b, uintptr_t x_b,
                    uintptr_t conv_state, uintptr_t ra_t, uintptr_t ra_b, uintptr_t ri_t, uintptr_t ri_b, uintptr_t lam,
                    uintptr_t y_b, uintptr_t state, uintptr_t positions, uintptr_t slots, int seqs, int nb,
-                   int bw, int taps, float scale, uintptr_t arrived, int arrived_len, int f32, uintptr_t stream);
+                   int bw, int taps, float scale, uintptr_t arrived, long arrived_len, int num_slots, int f32,
+                   uintptr_t stream);
 void sm_clipped_glu(uintptr_t out, uintptr_t gu, uintptr_t bias, int tokens, int F, float limit, float alpha, int f32,
                     uintptr_t stream);
 void sm_softcap(uintptr_t out, uintptr_t x, long n, float cap, float scale, int f32, uintptr_t stream);

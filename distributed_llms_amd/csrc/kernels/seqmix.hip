@@ -1467,8 +1467,10 @@ void sm_rglru_scan(uintptr_t out, uintptr_t a, uintptr_t g, uintptr_t y_raw, lon
 // anything waits (the gate kernel had two weight loads in flight per thread: 19-27 us by itself), and each finishing
 // thread has its state, y and biases in registers before the convolution starts.
 // A gate needs all bw convolved inputs of its block, so every workgroup of a block convolves them all, and the tail may
-// move only when all have read it: each counts itself in `arrived` [sequence groups][blocks] once its reads have returned,
-// and the last of them -- nobody waits -- writes the new tail and clears the count.
+// move only when all have read it: each counts itself in `arrived` [state slots][blocks] once its reads have returned, and
+// the last of them -- nobody waits -- writes the new tail.  The count belongs to the slot whose tail it guards, so launches
+// on other slots, on whatever stream or in whatever graph, never meet in it, and it wraps to zero by itself at the last
+// arrival (rows that share the scratch slot leave a whole number of turns).
 // 4 blocks of 256, 4 taps, bf16: one sequence 6.3 us, for 30 in four launches; 10 blocks: 16 sequences 9.1 us (42 before),
 // 64 sequences 20 us.
 constexpr int kRows = 8;       // gate matrix rows in flight per thread
@@ -1485,7 +1487,7 @@ __global__ void __launch_bounds__(256) sm_rglru_step_kernel(
     const void* __restrict__ ra_t_, const void* __restrict__ ra_b_, const void* __restrict__ ri_t_,
     const void* __restrict__ ri_b_, const void* __restrict__ lam_, const void* __restrict__ y_b_, float* __restrict__ state,
     const int32_t* __restrict__ positions, const int32_t* __restrict__ slots, int seqs, int nb, int bw, int taps, float scale,
-    int* __restrict__ arrived) {
+    unsigned* __restrict__ arrived) {
   typedef typename Raw8<T>::type raw8;
   extern __shared__ float smem[];
   constexpr int kPitch = 2 * GT_ * kStepOut + 4;      // (+ 4: the groups of a wave write to banks of their own)
@@ -1493,7 +1495,7 @@ __global__ void __launch_bounds__(256) sm_rglru_step_kernel(
   float* red2 = red + 32 * kPitch;                    // [2 gates][GT_][64]
   float* ubs = red2 + 2 * GT_ * kStepOut;             // [GT_][bw] convolved inputs
   T* tail = (T*)(ubs + GT_ * bw);                     // [GT_][taps - 1][bw] the new tail
-  __shared__ int last;
+  __shared__ int last[GT_];
   const int nz = (bw + kStepOut - 1) / kStepOut;
   const int b = blockIdx.x / nz, o0 = (blockIdx.x % nz) * kStepOut;
   const int s0 = blockIdx.y * GT_, C = nb * bw;
@@ -1563,9 +1565,9 @@ __global__ void __launch_bounds__(256) sm_rglru_step_kernel(
   }
   __syncthreads();                                    // every read of the old tail in this workgroup has returned
   // (counters on lines of their own; the answer is not needed before the end)
-  int* count = arrived + (size_t)(blockIdx.y * nb + b) * kCountStride;
-  int before = 0;
-  if (tid == 0) before = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  unsigned before = 0;
+  if (tid < GT_ && s0 + tid < seqs)
+    before = atomicInc(arrived + ((size_t)(tid == 0 ? slot[0] : slot[GT_ - 1]) * nb + b) * kCountStride, nz - 1);
 
   float ar[GT_][8], ai[GT_][8];
 #pragma unroll
@@ -1609,7 +1611,7 @@ __global__ void __launch_bounds__(256) sm_rglru_step_kernel(
     for (int g = 0; g < 32; ++g) sum += red[g * kPitch + e];
     red2[e] = sum;
   }
-  if (tid == 0) last = before == nz - 1;
+  if (tid < GT_) last[tid] = before == nz - 1;
   __syncthreads();
   if (fin) {
     const float sr = red2[fk * kStepOut + (tid & 63)], si = red2[(GT_ + fk) * kStepOut + (tid & 63)];
@@ -1619,25 +1621,24 @@ __global__ void __launch_bounds__(256) sm_rglru_step_kernel(
     *fstate = s;
     stf((T*)out_ + (size_t)fq * C + b * bw + fo, s * gelu_tanh_f((float)y_in + (float)y_b));
   }
-  if (last) {                                         // uniform
-    for (int i = tid; i < GT_ * bw; i += 256) {
-      const int k = GT_ == 1 ? 0 : i / bw, ci = i - k * bw, q = s0 + k;
-      if (q < seqs) {
-        T* st = (T*)conv_state_ + (size_t)slots[q] * (taps - 1) * C + b * bw + ci;
+#pragma unroll
+  for (int k = 0; k < GT_; ++k) {
+    if (s0 + k < seqs && last[k]) {                   // uniform
+      for (int ci = tid; ci < bw; ci += 256) {
+        T* st = (T*)conv_state_ + (size_t)slot[k] * (taps - 1) * C + b * bw + ci;
         for (int j = 0; j < taps - 1; ++j) st[(size_t)j * C] = tail[(size_t)(k * (taps - 1) + j) * bw + ci];
       }
     }
-    if (tid == 0) *count = 0;
   }
 }
 
 // Every sequence brings one token, token q of the batch is sequence q's.  x / y: the two halves of the projection (rows
-// ld apart); out [tokens, C]; arrived: sequences x blocks zeroed counters, 32 ints apart, that no other launch uses
-// meanwhile (left zeroed).
+// ld apart); out [tokens, C]; arrived: num_slots x blocks counters, 32 ints apart, zero before the first launch.
 void sm_rglru_step(uintptr_t out, uintptr_t x, uintptr_t y, long ld, uintptr_t conv_w, uintptr_t conv_b, uintptr_t x_b,
                    uintptr_t conv_state, uintptr_t ra_t, uintptr_t ra_b, uintptr_t ri_t, uintptr_t ri_b, uintptr_t lam,
                    uintptr_t y_b, uintptr_t state, uintptr_t positions, uintptr_t slots, int seqs, int nb,
-                   int bw, int taps, float scale, uintptr_t arrived, int arrived_len, int f32, uintptr_t stream) {
+                   int bw, int taps, float scale, uintptr_t arrived, long arrived_len, int num_slots, int f32,
+                   uintptr_t stream) {
   if (seqs <= 0) return;
   DLLM_HOST_CHECK(nb > 0 && bw >= 8 && bw % 8 == 0 && bw <= 512 && (long)nb * bw <= (1L << 24), "rglru step block sizes");
   DLLM_HOST_CHECK(taps >= 1 && taps <= kStepTaps && ld >= (long)nb * bw, "rglru step sizes");
@@ -1645,7 +1646,7 @@ void sm_rglru_step(uintptr_t out, uintptr_t x, uintptr_t y, long ld, uintptr_t c
   // of 256 at 16 sequences: 9.1 us with one, 10.0 with two; at 64: 20.9 and 20.0)
   const int gt = seqs <= 32 ? 1 : 2;
   const int groups = (seqs + gt - 1) / gt;
-  DLLM_HOST_CHECK(arrived != 0 && (long)groups * nb * kCountStride <= arrived_len && groups <= 65535, "rglru step counters");
+  DLLM_HOST_CHECK(arrived != 0 && (long)num_slots * nb * kCountStride <= arrived_len && groups <= 65535, "rglru step counters");
   const size_t lds = ((size_t)(33 * 2 * gt * kStepOut + 32 * 4) + (size_t)gt * bw) * sizeof(float) +
                      (size_t)gt * (taps - 1) * bw * (f32 ? 4 : 2);
   // consecutive workgroups run on consecutive XCDs: the (block, output) index first, so that with 8 or more of them a
@@ -1660,7 +1661,7 @@ void sm_rglru_step(uintptr_t out, uintptr_t x, uintptr_t y, long ld, uintptr_t c
                        (void*)out, (const void*)x, (const void*)y, ld, (const void*)conv_w, (const void*)conv_b,      \
                        (const void*)x_b, (void*)conv_state, (const void*)ra_t, (const void*)ra_b, (const void*)ri_t,  \
                        (const void*)ri_b, (const void*)lam, (const void*)y_b, (float*)state,                          \
-                       (const int32_t*)positions, (const int32_t*)slots, seqs, nb, bw, taps, scale, (int*)arrived);   \
+                       (const int32_t*)positions, (const int32_t*)slots, seqs, nb, bw, taps, scale, (unsigned*)arrived);  \
   } while (0)
 #define SM_STEP_T(T)                                            \
   do {                                                          \

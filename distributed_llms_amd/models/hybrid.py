@@ -302,7 +302,8 @@ class HybridStage(LayerListStage):
 
     def allocate_state(self, num_slots: int):
         """State pools, one row per BlockManager state slot: per layer the convolution tail
-        [slots, taps - 1, C] (activation dtype) and per RG-LRU layer the state [slots, C] float32."""
+        [slots, taps - 1, C] (activation dtype) and per RG-LRU layer the state [slots, C] float32 with the counters of
+        its one-launch decode step."""
         self.num_state_slots = num_slots
         self.state = []
         for l in self.specs:
@@ -312,7 +313,8 @@ class HybridStage(LayerListStage):
                 st = {}
             else:
                 c = m["width"]
-                st = {"s": torch.zeros(num_slots, c, dtype=torch.float32, device=self.device)}
+                st = {"s": torch.zeros(num_slots, c, dtype=torch.float32, device=self.device),
+                      "arrived": sm.step_counters(num_slots, m["blocks"], self.device)}
             st["conv"] = torch.zeros(num_slots, max(0, m["conv"] - 1), c, dtype=self.dtype, device=self.device)
             self.state.append(st)
         return self.state
@@ -326,7 +328,7 @@ class HybridStage(LayerListStage):
                 c = m["heads"] * m["dim"] + (0 if "kv_from" in m else m["kv_heads"] * (m["dim"] + m["vdim"]))
             else:
                 c = m["width"]
-                n += 4 * c
+                n += 4 * c + 128 * m["blocks"]
             n += e * c * (m["conv"] - 1)
         return n
 
@@ -353,7 +355,7 @@ class HybridStage(LayerListStage):
         st = self.state[i]
         if sm.one_token_each(sb) and sm.rglru_step_fits(m["blocks"], c // m["blocks"], m["conv"]):
             r = sm.rglru_step(yx, w["conv_w"], w["conv_b"], w["x_b"], st["conv"], w["y_b"], w["ra_t"], w["ra_b"], w["ri_t"],
-                              w["ri_b"], w["lam"], st["s"], sb)
+                              w["ri_b"], w["lam"], st["s"], sb, arrived=st["arrived"])
             return ops.linear_into_norm(r, w["wo"])
         u = sm.causal_conv(yx[:, c:], w["conv_w"], w["conv_b"], st["conv"], sb, in_bias=w["x_b"])
         r = sm.rglru(u, yx[:, :c], w["y_b"], w["ra_t"], w["ra_b"], w["ri_t"], w["ri_b"], w["lam"], st["s"], sb,

@@ -448,28 +448,19 @@ def rglru_step_fits(blocks: int, bw: int, taps: int) -> bool:
     return 1 <= blocks and bw % 8 == 0 and 8 <= bw <= 512 and blocks * bw <= 1 << 24 and 1 <= taps <= 8
 
 
-_arrived = {}
-
-
-def _arrival_counts(device: torch.device, n: int) -> torch.Tensor:
-    """Zeroed counters of the current stream, which every launch leaves zeroed (launches on one stream follow each other;
-    graphs keep those of the stream they were captured on, as they do the split-K workspace).  Counters that became too
-    few stay allocated, since graphs captured before still count in them; each is twice the last, so their sum is bounded."""
-    key = (device.index or 0, torch.cuda.current_stream().cuda_stream)
-    kept = _arrived.setdefault(key, [])
-    if not kept or kept[-1].numel() < n:
-        if torch.cuda.is_current_stream_capturing():     # cleared by the graph itself, at every replay, and its own
-            return torch.zeros(n, dtype=torch.int32, device=device)
-        size = max(n, 2 * kept[-1].numel() if kept else 1 << 16)
-        kept.append(torch.zeros(size, dtype=torch.int32, device=device))
-    return kept[-1]
+def step_counters(num_slots: int, blocks: int, device) -> torch.Tensor:
+    """The arrival counters of :func:`rglru_step` for a state pool of ``num_slots`` rows: zeroed here, once; every launch
+    leaves them zero.  128 bytes apart, so that workgroups on several XCDs count on lines of their own."""
+    return torch.zeros(num_slots * blocks * 32, dtype=torch.int32, device=device)
 
 
 def rglru_step(yx: torch.Tensor, conv_w: torch.Tensor, conv_b: torch.Tensor, x_b: torch.Tensor, conv_state: torch.Tensor,
                y_b: torch.Tensor, ra_t: torch.Tensor, ra_b: torch.Tensor, ri_t: torch.Tensor, ri_b: torch.Tensor,
-               lam: torch.Tensor, state: torch.Tensor, sb: SeqBatch, decay_scale: float = 8.0) -> torch.Tensor:
+               lam: torch.Tensor, state: torch.Tensor, sb: SeqBatch, decay_scale: float = 8.0,
+               arrived: Optional[torch.Tensor] = None) -> torch.Tensor:
     """The recurrent branch of a batch with one token per sequence: :func:`causal_conv` of the right half of ``yx`` [T, 2 C]
-    (bias ``x_b``; tail ``conv_state``) and :func:`rglru` of it with the left half as y, in one launch on the GPU."""
+    (bias ``x_b``; tail ``conv_state``) and :func:`rglru` of it with the left half as y, in one launch on the GPU.
+    ``arrived``: the state pool's :func:`step_counters`, kept beside ``conv_state`` (None: zeroed ones for this call)."""
     c = state.shape[1]
     nb, bw, _ = ra_t.shape
     taps = conv_w.shape[0]
@@ -487,12 +478,15 @@ def rglru_step(yx: torch.Tensor, conv_w: torch.Tensor, conv_b: torch.Tensor, x_b
         raise ValueError("rglru_step: shape mismatch")
     out = torch.empty(yx.shape[0], c, dtype=yx.dtype, device=yx.device)
     e = yx.element_size()
-    arrived = _arrival_counts(yx.device, sb.num_seqs * nb * 32)
+    slots = conv_state.shape[0]
+    if arrived is None:
+        arrived = step_counters(slots, nb, yx.device)
+    _ck(arrived, "arrived", torch.int32)
     _k().sm_rglru_step(out.data_ptr(), yx.data_ptr() + c * e, yx.data_ptr(), yx.stride(0), conv_w.data_ptr(), conv_b.data_ptr(),
                        x_b.data_ptr(), conv_state.data_ptr(), ra_t.data_ptr(), ra_b.data_ptr(), ri_t.data_ptr(),
                        ri_b.data_ptr(), lam.data_ptr(), y_b.data_ptr(), state.data_ptr(), sb.positions.data_ptr(),
                        sb.state_slots.data_ptr(), sb.num_seqs, nb, bw, taps, float(decay_scale),
-                       arrived.data_ptr(), arrived.numel(), _f32flag(yx), _stream())
+                       arrived.data_ptr(), arrived.numel(), slots, _f32flag(yx), _stream())
     return out
 
 

@@ -111,6 +111,57 @@ def test_rglru_step_graph_outlives_its_counters_successor(cuda, warm):
 
 
 @gpu
+@pytest.mark.parametrize("bw", [64, 200])
+def test_rglru_step_counts_by_slot(cuda, bw):
+    """Two graphs captured on one stream, of other slots of one pool, replayed side by side on two others, next to eager
+    launches on the stream of their capture: each slot's count is its own.  Rows that share the scratch slot (padding) and
+    odd last rows of a pair leave every count zero."""
+    nb, taps, c, slots = 3, 4, 3 * bw, 120
+    r = lambda *s: torch.randn(*s, device=cuda).bfloat16()
+    par = [r(taps, c), r(c), r(c)], [r(c), r(nb, bw, bw) * 0.1, r(nb, bw), r(nb, bw, bw) * 0.1, r(nb, bw), r(c)]
+    yx, conv0, state0 = r(41, 2 * c), r(slots, taps - 1, c), torch.randn(slots, c, device=cuda)
+    arrived = sm.step_counters(slots, nb, cuda)
+    parts = [list(range(1, 38)) + [0] * 4, list(range(40, 81)), [100, 101, 0, 0, 0]]
+    sbs = [_sb([7] * len(p), p, cuda) for p in parts]
+
+    def run(i, conv, state, counts):
+        return sm.rglru_step(yx[:len(parts[i])], *par[0], conv, *par[1], state, sbs[i], arrived=counts)
+    want_c, want_s, want = conv0.clone(), state0.clone(), []
+    for i in range(3):
+        want.append(run(i, want_c, want_s, None))
+    conv, state = conv0.clone(), state0.clone()
+    torch.cuda.synchronize()
+    s, a, b = (torch.cuda.Stream() for _ in range(3))
+    graphs, outs = [], []
+    for i in range(2):
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            outs.append(run(i, conv, state, arrived))
+        graphs.append(g)
+    for _ in range(4):
+        conv.copy_(conv0)
+        state.copy_(state0)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(a):
+            graphs[0].replay()
+        with torch.cuda.stream(b):
+            graphs[1].replay()
+        with torch.cuda.stream(s):
+            eager = run(2, conv, state, arrived)
+        torch.cuda.synchronize()
+        live = [37, 41, 2]
+        for got, ref, n in zip(outs + [eager], want, live):
+            assert torch.equal(got[:n], ref[:n])
+        assert torch.equal(conv[1:], want_c[1:]) and torch.equal(state[1:], want_s[1:])
+        assert not arrived.any()
+
+
+def test_rglru_step_keeps_no_process_wide_state():
+    """What the step counts in belongs to the caller's state pool: nothing is kept by stream or device."""
+    assert not [k for k, v in vars(sm).items() if isinstance(v, (dict, list, set)) and not k.startswith("__")]
+
+
+@gpu
 @pytest.mark.parametrize("rows", [1, 7, 300])
 @pytest.mark.parametrize("width", [4, 250, 1024, 2560, 4100, 16384, 16392])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
