@@ -265,7 +265,9 @@ __global__ void __launch_bounds__(WPB * 64, 2) attn_decode_kernel(   // 2nd arg:
   const int ctx = seq_lens[b];
   const int kbeg = split * split_len;
   const int32_t* bt = block_tables + (size_t)b * max_blocks;
-  const int blk_first = bt[min(kbeg / kBS + lane, max_blocks - 1)];
+  // (a table without columns, of contexts that are all 0, has nothing to look up: any word that is there, dropped)
+  const int32_t* first = max_blocks > 0 ? bt + min(kbeg / kBS + lane, max_blocks - 1) : seq_lens + b;
+  const int blk_first = max_blocks > 0 ? *first : 0;
   // FUSED: the new key (ctx - 1) is not in the cache yet: its chunk is loaded as usual and the
   // key's K row / V^T column are replaced in registers by the rotated k and v (the split that
   // owns it also appends them to the cache, after its last KV load)

@@ -246,3 +246,19 @@ def test_decode_attention_rounds_and_passes(cuda, lens, width, splits, d, slabs)
     # element that rounds the other way
     assert (out.float() - expect).abs().max() <= 2.0 ** -7 * vf.abs().max()
     assert torch.equal(v.float(), vf)
+
+
+@gpu
+@pytest.mark.parametrize("fused", [False, True])
+def test_decode_attention_without_block_ids(cuda, fused):
+    """A block table of no columns (every context empty): zeros, and nothing is read through it."""
+    b, hq, hkv, d = 3, 4, 2, 128
+    k, v = torch.randn(2, hkv, 32, d).bfloat16().cuda(), torch.randn(2, hkv, d, 32).bfloat16().cuda()
+    bt, none = torch.zeros(b, 0, dtype=torch.int32, device=cuda), torch.zeros(b, dtype=torch.int32, device=cuda)
+    if fused:
+        qkv, cs = torch.randn(b, (hq + 2 * hkv) * d).bfloat16().cuda(), ref.rope_cos_sin(d, 64, 10000.0, device=cuda)
+        torch.cuda.synchronize()
+        out = ops.paged_attention_decode_rope(qkv, none, cs, k, v, none, bt, none, hq, hkv, d, d ** -0.5)
+    else:
+        out = ops.paged_attention_decode(torch.randn(b, hq, d).bfloat16().cuda(), k, v, bt, none, d ** -0.5)
+    assert torch.equal(out, torch.zeros_like(out))
