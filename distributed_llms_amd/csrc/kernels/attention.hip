@@ -172,30 +172,23 @@ struct RopeArgs {
 // W (8 or 2) consecutive qkv elements of a row in their stored form -- load() -- and as the bf16 values that the rest
 // works with -- value(), slabs summed in slab order as splitk_reduce sums them.  The two are apart so that the prologue
 // has every load under way before it waits for one.  NP: 0 = bf16 qkv, > 0 = that many slabs, -1 = a runtime count
-// (summed as it is loaded), a compile-time choice: a runtime branch split the prologue into blocks with vmcnt(0) waits
-// at every merge (cold B=256: 48 us vs 40 us without the fused part).
+// (q, k and v summed slab by slab by the kernel), a compile-time choice: a runtime branch split the prologue into blocks
+// with vmcnt(0) waits at every merge (cold B=256: 48 us vs 40 us without the fused part).
 template <int NP, int W>
 struct QkvPiece {
   typedef bf16 vec __attribute__((ext_vector_type(W)));
   typedef part_elem raw __attribute__((ext_vector_type(W)));
   vec q;
   raw l[NP > 0 ? NP : 1];
+  static __device__ __forceinline__ raw slab(const RopeArgs& ra, size_t p, int s) {
+    return *reinterpret_cast<const raw*>(reinterpret_cast<const part_elem*>(ra.part) + p + s * ra.slab);
+  }
   __device__ __forceinline__ void load(const RopeArgs& ra, size_t p) {
     if constexpr (NP == 0) {
       q = *reinterpret_cast<const vec*>(ra.qkv + p);
-    } else if constexpr (NP > 0) {
-#pragma unroll
-      for (int s = 0; s < NP; ++s)
-        l[s] = *reinterpret_cast<const raw*>(reinterpret_cast<const part_elem*>(ra.part) + p + s * ra.slab);
     } else {
-      float a[W] = {};
-      for (int s = 0; s < ra.nparts; ++s) {
-        const raw v = *reinterpret_cast<const raw*>(reinterpret_cast<const part_elem*>(ra.part) + p + s * ra.slab);
 #pragma unroll
-        for (int j = 0; j < W; ++j) a[j] += part_value(v[j]);
-      }
-#pragma unroll
-      for (int j = 0; j < W; ++j) q[j] = f2bf(a[j]);
+      for (int s = 0; s < NP; ++s) l[s] = slab(ra, p, s);
     }
   }
   __device__ __forceinline__ vec value() const {
@@ -258,9 +251,9 @@ __global__ void __launch_bounds__(WPB * 64, 2) attn_decode_kernel(   // 2nd arg:
   const int r = lane & 15, g = lane >> 4;
   // Two round trips to memory precede the first MFMA: the sequence's position, its context length, this split's first 64
   // block ids (not guarded by the context) and the projection's q go out together; what hangs on them -- the first KV
-  // chunk, the cos / sin row and, in the split that owns the new key, its k and v -- follows before anything is summed or
-  // rotated.  (hipcc, left to order the loads, summed q, k and v in four rounds before the first KV load and loaded the
-  // cos / sin row after it; every split read k and v, v as 2-byte pieces.)
+  // chunk, the cos / sin row and the new key's k and v (every split loads them, its owner uses them) -- follows before
+  // anything is summed or rotated.  (hipcc, left to order the loads, summed q, k and v in four rounds before the first KV
+  // load and loaded the cos / sin row after it.)
   const int pos_b = FUSED ? ra.positions[b] : 0;
   const int ctx = seq_lens[b];
   const int kbeg = split * split_len;
@@ -325,12 +318,42 @@ __global__ void __launch_bounds__(WPB * 64, 2) attn_decode_kernel(   // 2nd arg:
     QkvPiece<PARTS, 8> qp[D / 32];
     QkvPiece<PARTS, 2> kp, vp;      // the new key's k and v, two elements per lane
     RopeRow<D> rr;
-#pragma unroll
-    for (int ks = 0; ks < D / 32; ++ks) qp[ks].load(ra, row + (size_t)(kvh * G + (col_ok ? r : 0)) * D + ks * 32 + 8 * g);
-    load_at(cur, blk_0);
     const int pair = 2 * (lane & (D / 2 - 1));
-    kp.load(ra, row + (size_t)(hq + kvh) * D + pair);     // (in every split: under a branch hipcc would wait for it there)
-    vp.load(ra, row + (size_t)(hq + hkv + kvh) * D + pair);
+    const size_t q_at = row + (size_t)(kvh * G + (col_ok ? r : 0)) * D + 8 * g;
+    const size_t k_at = row + (size_t)(hq + kvh) * D + pair, v_at = row + (size_t)(hq + hkv + kvh) * D + pair;
+    // (k and v in every split: under a branch hipcc would wait for them there)
+    if constexpr (PARTS >= 0) {
+#pragma unroll
+      for (int ks = 0; ks < D / 32; ++ks) qp[ks].load(ra, q_at + ks * 32);
+      load_at(cur, blk_0);
+      kp.load(ra, k_at);
+      vp.load(ra, v_at);
+    } else {
+      // a runtime count (70B under tensor parallelism: 6, 13 and 16 slabs): all of q, k and v of a slab per round trip.
+      // A loop for each of the six pieces, the KV chunk already in flight, was a round trip per slab and piece and 80
+      // bytes of scratch: 64 rows x 800 keys of 32 / 4 heads, 6 and 16 slabs 34.5 and 48.2 -> 26.6 and 30.8 us, 256 x 300
+      // of 8 / 1 heads 24.8 and 38.3 -> 16.6 and 20.8 us.
+      float aq[D / 32][8] = {}, akv[4] = {};
+      for (int s = 0; s < ra.nparts; ++s) {
+        typename QkvPiece<PARTS, 8>::raw lq[D / 32];
+#pragma unroll
+        for (int ks = 0; ks < D / 32; ++ks) lq[ks] = qp[ks].slab(ra, q_at + ks * 32, s);
+        const auto lk = kp.slab(ra, k_at, s), lv = vp.slab(ra, v_at, s);
+#pragma unroll
+        for (int ks = 0; ks < D / 32; ++ks)
+#pragma unroll
+          for (int j = 0; j < 8; ++j) aq[ks][j] += part_value(lq[ks][j]);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) akv[j] += part_value(lk[j]), akv[2 + j] += part_value(lv[j]);
+      }
+#pragma unroll
+      for (int ks = 0; ks < D / 32; ++ks)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) qp[ks].q[j] = f2bf(aq[ks][j]);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) kp.q[j] = f2bf(akv[j]), vp.q[j] = f2bf(akv[2 + j]);
+      load_at(cur, blk_0);
+    }
     if (ra.cos_sin) rr.load(ra.cos_sin + (size_t)pos_b * D, g);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -409,9 +432,10 @@ __global__ void __launch_bounds__(WPB * 64, 2) attn_decode_kernel(   // 2nd arg:
   for (int cb = c0; cb < c1; cb += 64) {            // 64 chunks (2048 keys) of block ids per pass
     const int n = min(64, c1 - cb);
     auto block = [&](int j) { return __builtin_amdgcn_readlane(my_blk, j); };
-    // ping-pong, cur <-> nxt (the barriers keep hipcc from strewing a chunk's loads among the other's MFMAs): both loads of a turn unconditional (behind a branch the wait for one chunk, which has to
-    // hold on either path, waits for the other too), and every key of these chunks admissible -- a split's last chunk,
-    // which may be partial and holds the new key, is left for behind the loop
+    // ping-pong, cur <-> nxt (the barriers keep hipcc from strewing a chunk's loads among the other's MFMAs): both loads
+    // of a turn unconditional (behind a branch the wait for one chunk, which has to hold on either path, waits for the
+    // other too), and every key of these chunks admissible -- a split's last chunk, which may be partial and holds the new
+    // key, is left for behind the loop
     int j = 0;
     for (; j + 2 < n; j += 2) {
       load_at(nxt, block(j + 1));
