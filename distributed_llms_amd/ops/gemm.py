@@ -133,8 +133,13 @@ def stream_fits(m: int, n: int, k: int, glu: str = "", defer: bool = False) -> b
 
 
 def _recorded(*tensors) -> bool:
-    """Is the call differentiated or transformed (autograd, forward mode, vmap)?  The kernels leave no trace of it."""
+    """Is the call differentiated, transformed or traced (autograd, forward mode, vmap; torch.jit.trace, torch.compile,
+    make_fx and other dispatch modes; tensor subclasses)?  The kernels leave no trace of it."""
+    if torch._C._len_torch_dispatch_stack() or torch._C._get_tracing_state() is not None or torch.compiler.is_compiling():
+        return True
     for t in tensors:
+        if t is not None and type(t) not in (torch.Tensor, torch.nn.Parameter):
+            return True
         if t is not None and (torch._C._functorch.is_functorch_wrapped_tensor(t)
                               or (t.requires_grad and torch.is_grad_enabled())
                               or (forward_ad._current_level >= 0 and forward_ad.unpack_dual(t).tangent is not None)):

@@ -100,6 +100,26 @@ def test_recorded_calls_keep_their_derivatives(launches):
     assert [n for n, _ in launches] == ["gemm_stream"]
 
 
+def test_traced_calls_keep_the_product(launches):
+    """A traced graph holds the product, not the memory that a launch left behind while it was traced; a dispatch mode
+    and a tensor subclass see the call."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.utils.flop_counter import FlopCounterMode
+    x, w, b = torch.randn(4, 1024).bfloat16(), torch.randn(500, 1024).bfloat16(), torch.randn(500).bfloat16()
+    x2 = torch.randn(4, 1024).bfloat16()
+    want = F.linear(x2, w, b)
+    assert torch.equal(torch.jit.trace(lambda v: gemm.linear(v, w, b), x, check_trace=False)(x2), want)
+    assert torch.equal(make_fx(lambda v: gemm.linear(v, w, b))(x)(x2), want)
+    with FakeTensorMode() as mode:
+        fake = [mode.from_tensor(t) for t in (x, w, b)]
+    assert gemm.linear(*fake).shape == (4, 500)                 # (outside the mode: the tensors carry it)
+    with FlopCounterMode(display=False) as flops:
+        gemm.linear(x, w, b)
+    assert flops.get_total_flops() == 2 * 4 * 500 * 1024
+    assert not launches
+
+
 def test_fp8_weight_in_front_of_a_norm():
     """linear_into_norm takes what linear(defer=True) takes: an fp8 weight too (latent_attention's output projection)."""
     from distributed_llms_amd import ops
