@@ -110,6 +110,19 @@ __device__ __forceinline__ float clipped_glu_f(float g, float u, float limit) {
   return g * __builtin_amdgcn_rcpf(1.f + __expf(-kGluAlpha * g)) * (u + 1.0f);
 }
 
+// The same with expf and a true division: the form of the gate kernels (whatever their output type) and of
+// epilogues that took over a gate kernel's calls
+__device__ __forceinline__ float clipped_glu_exact_f(float g, float u, float limit, float alpha) {
+  g = fminf(g, limit);
+  u = fminf(fmaxf(u, -limit), limit);
+  return g * (1.0f / (1.0f + expf(-alpha * g))) * (u + 1.0f);
+}
+__device__ __forceinline__ float gelu_glu_exact_f(float g, float u) {
+  // 0.5 (1 + tanh(z)) = 1 / (1 + e^(-2 z))
+  const float z = 0.7978845608028654f * (g + 0.044715f * g * g * g);
+  return g / (1.0f + expf(-2.0f * z)) * u;
+}
+
 // gelu (tanh form) of the gate times up, 0.5 (1 + tanh(z)) = 1 / (1 + e^(-2 z)): the epilogue form (rounded to bf16)
 __device__ __forceinline__ float gelu_glu_f(float g, float u) {
   const float z2 = 1.5957691216057308f * (g + 0.044715f * g * g * g);

@@ -149,7 +149,8 @@ __global__ void __launch_bounds__(WAVES * 64) gemm_stream_kernel(bf16* __restric
       float z = a[v] + (bias ? bf2f(bias[cc]) : 0.f);
       if constexpr (GLU != 0) {
         const float up = b[v] + (bias ? bf2f(bias[half + cc]) : 0.f);
-        z = GLU == 1 ? silu_f(z) * up : GLU == 2 ? clipped_glu_f(z, up, limit) : gelu_glu_f(z, up);
+        // (a projection, a bias and a gate kernel until they met here: the gate kernels' arithmetic)
+        z = GLU == 1 ? silu_f(z) * up : GLU == 2 ? clipped_glu_exact_f(z, up, limit, kGluAlpha) : gelu_glu_exact_f(z, up);
       }
       o[v] = f2bf(z);
     }

@@ -1696,10 +1696,7 @@ __global__ void __launch_bounds__(256) sm_clipped_glu_kernel(void* __restrict__ 
       for (int j = 0; j < V; ++j) gv[j] += b1[j], uv[j] += b2[j];
     }
 #pragma unroll
-    for (int j = 0; j < V; ++j) {
-      const float g = fminf(gv[j], limit), u = fminf(fmaxf(uv[j], -limit), limit);
-      gv[j] = g * (1.0f / (1.0f + expf(-alpha * g))) * (u + 1.0f);
-    }
+    for (int j = 0; j < V; ++j) gv[j] = clipped_glu_exact_f(gv[j], uv[j], limit, alpha);
     stv<V>(out + c, gv);
   }
 }
@@ -1724,11 +1721,7 @@ __global__ void __launch_bounds__(256) sm_gelu_glu_kernel(void* __restrict__ out
     ldv<V>(gu + c, g);
     ldv<V>(gu + F + c, u);
 #pragma unroll
-    for (int j = 0; j < V; ++j) {
-      // 0.5 (1 + tanh(z)) = 1 / (1 + e^(-2 z))
-      const float z = 0.7978845608028654f * (g[j] + 0.044715f * g[j] * g[j] * g[j]);
-      g[j] = g[j] / (1.0f + expf(-2.0f * z)) * u[j];
-    }
+    for (int j = 0; j < V; ++j) g[j] = gelu_glu_exact_f(g[j], u[j]);
     stv<V>(out + c, g);
   }
 }

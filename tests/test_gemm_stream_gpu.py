@@ -61,6 +61,22 @@ def test_stream_glu(cuda, m, half, k, glu, bias):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("glu", ["clipped", "gelu"])
+def test_stream_glu_keeps_the_gate_kernels_arithmetic(cuda, glu):
+    """Products of one term each are exact in f32, so the epilogue's result is the f32 gate kernel's, rounded once: bit for
+    bit, over gates where the hardware exponential and reciprocal are several f32 ulps off (a million elements)."""
+    from distributed_llms_amd.ops import seqmix as sm
+    m, k, half = 64, 1024, 16384
+    x = torch.linspace(-9, 3, m * k, device="cuda")[torch.randperm(m * k, device="cuda")].view(m, k).bfloat16()
+    w = torch.zeros(2 * half, k, device="cuda", dtype=torch.bfloat16)
+    rows = torch.arange(2 * half, device="cuda")
+    w[rows, torch.randint(0, k, (2 * half,), device="cuda")] = (torch.rand(2 * half, device="cuda") * 2 + 0.5).bfloat16()
+    gu = F.linear(x.double(), w.double()).float()
+    want = sm.clipped_glu(gu, None, 7.0) if glu == "clipped" else sm.gelu_glu(gu)
+    assert torch.equal(gemm.linear_stream(x, w, None, glu, 7.0), want.bfloat16())
+
+
+@pytest.mark.gpu
 def test_stream_is_reached_and_matches_the_wide_route(cuda):
     """ops.linear / linear_swiglu at decode sizes take the kernel by default; knobs.stream off gives the former route."""
     from distributed_llms_amd import ops
