@@ -1180,6 +1180,7 @@ __global__ void __launch_bounds__(256) sm_rglru_gates_kernel(float* __restrict__
 constexpr int kST = 128;      // tokens per workgroup
 constexpr int kSK = 64;       // K chunk in LDS
 constexpr int kSP = kSK + 8;
+constexpr float kBfMax = 0x1.fep+127f;
 
 __global__ void __launch_bounds__(256, 2) sm_rglru_gates_split_kernel(
     float* __restrict__ a_out, float* __restrict__ g_out, const float* __restrict__ u, const bf16* __restrict__ ra_t,
@@ -1216,8 +1217,10 @@ __global__ void __launch_bounds__(256, 2) sm_rglru_gates_split_kernel(
       const bool ok = t0 + r < tokens && kc + k < bw;
       float x = ub[(size_t)min(t0 + r, tokens - 1) * C + min(kc + k, bw - 1)];
       x = ok ? x : 0.f;
-      const bf16 h = f2bf(x);
-      const float xm = __builtin_isfinite(bf2f(h)) ? x - bf2f(h) : 0.f;
+      // (a finite x above the largest bf16 keeps a finite first piece; an infinite or NaN one has no others)
+      const bool fin = __builtin_isfinite(x);
+      const bf16 h = f2bf(fin ? fminf(fmaxf(x, -kBfMax), kBfMax) : x);
+      const float xm = fin ? x - bf2f(h) : 0.f;
       const bf16 m = f2bf(xm);
       us[0][r][k] = h;
       us[1][r][k] = m;

@@ -38,3 +38,33 @@ def test_gates_keep_all_bits_of_the_input(cuda, nb, bw, tokens, size):
     gate, dg = torch.sigmoid(zi), bound(ri) / 4 + 1e-6
     err = (y.cpu().double().view(tokens, nb, bw) - mult(want) * gate * x).abs()
     assert (err <= ((hi - lo) * gate + dg + 1e-6) * x.abs() + 1e-12).all()
+
+
+def _gates(cuda, u, ra, rb, ri, ib, lam):
+    tokens, nb, bw = u.shape
+    a, y = (torch.full((tokens, nb * bw), float("nan"), device=cuda) for _ in range(2))
+    d = [x.to(cuda).contiguous() for x in (u, ra, rb, ri, ib, lam)]
+    torch.cuda.synchronize()
+    _ext.kernels().sm_rglru_gates(a.data_ptr(), y.data_ptr(), *(x.data_ptr() for x in d), tokens, nb, bw, 8.0, 0,
+                                  torch.cuda.current_stream().cuda_stream)
+    return a.cpu().view(tokens, nb, bw), y.cpu().view(tokens, nb, bw)
+
+
+def test_gates_of_the_largest_inputs(cuda):
+    """Finite inputs above the largest bf16 number stay finite (infinity times a zero weight is no number); infinite and
+    NaN inputs reach the sums of their own token alone."""
+    tokens, nb, bw = 70, 2, 64
+    top = torch.finfo(torch.float32).max
+    u = torch.zeros(tokens, nb, bw)
+    u[0, 0, 3], u[1, 1, 5], u[2, 0, 0], u[3, 0, 0] = top, -top, float("inf"), float("nan")
+    w = torch.zeros(nb, bw, bw)
+    w[0, 3, 7] = 2.0 ** -120                                   # the one weight that meets a large input: 256 and -256
+    w[1, 5, 9] = 2.0 ** -120
+    zero = torch.zeros(nb, bw).bfloat16()
+    a, _ = _gates(cuda, u, w.bfloat16(), zero, w.bfloat16(), zero, zero)
+    want = torch.exp(-8.0 * torch.sigmoid(torch.matmul(u.double().transpose(0, 1), w.double()).transpose(0, 1)) *
+                     torch.tensor(2.0).double().log())
+    ok = torch.ones(tokens, dtype=torch.bool)
+    ok[2:4] = False
+    torch.testing.assert_close(a[ok].double(), want[ok], rtol=1e-5, atol=1e-12)
+    assert a[2:4, 0].isnan().all() and (a[2:4, 1] == a[4, 1]).all()
