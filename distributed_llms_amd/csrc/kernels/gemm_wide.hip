@@ -190,6 +190,13 @@ __device__ __forceinline__ void wide_epilogue(const f32x4 (&acc)[BM / 64][4], bf
 // an HBM round trip.  One more vm op per slot (counted waits use G + 1); results are unchanged.
 constexpr int PFD = 2;
 __device__ __forceinline__ int wide_rot(int xcd, int nt) { return nt >= 16 ? (xcd * nt) >> 3 : 0; }
+// The XCD that the first row tile of column tile n_t runs on (the inverse of the XCD remap, no K split): all row tiles of a
+// column start their K loop at the same place, so that equal rows have equal results whichever tile they lie in.
+__device__ __forceinline__ int wide_rot_xcd(int n_t, int mtiles, int total) {
+  if (mtiles == 1) return (int)(blockIdx.x & 7);
+  const int b = n_t * mtiles, q = total >> 3, r = total & 7;
+  return b < r * (q + 1) ? b / (q + 1) : r + (b - r * (q + 1)) / q;
+}
 
 template <int BM, int NBUF, int VAR, bool FP8 = false>
 __device__ __forceinline__ void wide_mainloop(bf16* smem, const bf16* const (&srcA)[BM / 64],
@@ -498,7 +505,8 @@ __global__ void __launch_bounds__(512, 1) gemm_wide_kernel(const bf16* __restric
   // PF: lanes l and l + 16k of wave w touch weight row 16 w + (l & 15) of the tile: 128 lines per K-tile
   const bf16* pfB = B + (size_t)wide_b_row<SWIGLU>(16 * wv + (lane & 15), n_t, N / 2) * K + (size_t)kt0 * WBK;
   f32x4 acc[RT][4];
-  wide_mainloop<BM, NBUF, VAR>(smem, srcA, srcB, nt, acc, wv, lane, pfB, smem + NBUF * BUF, wide_rot((int)(blockIdx.x & 7), nt));
+  const int rot = (VAR & 256) ? wide_rot(wide_rot_xcd(n_t, mtiles, total), nt) : 0;
+  wide_mainloop<BM, NBUF, VAR>(smem, srcA, srcB, nt, acc, wv, lane, pfB, smem + NBUF * BUF, rot);
   wide_epilogue<BM, SPLIT, SWIGLU>(acc, C, P, M, N, m0, n_t, split, wm, wn, lane);
 }
 
@@ -550,7 +558,8 @@ __global__ void __launch_bounds__(512, 1) gemm_wide_fp8_kernel(const uint8_t* __
     srcB[j] = B + (size_t)wide_b_row<SWIGLU>(r, n_t, N / 2) * KU + (size_t)kt0 * WBK + wswz(r, lane & 7) * 8;
   }
   f32x4 acc[RT][4];
-  wide_mainloop<BM, NBUF, VAR, true>(smem, srcA, srcB, nt, acc, wv, lane, nullptr, nullptr, wide_rot((int)(blockIdx.x & 7), nt));
+  const int rot = (VAR & 256) ? wide_rot(wide_rot_xcd(n_t, mtiles, total), nt) : 0;
+  wide_mainloop<BM, NBUF, VAR, true>(smem, srcA, srcB, nt, acc, wv, lane, nullptr, nullptr, rot);
   wide_epilogue<BM, SPLIT, SWIGLU, true>(acc, C, P, M, N, m0, n_t, split, wm, wn, lane, sa, sb);
 }
 

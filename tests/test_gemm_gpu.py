@@ -422,3 +422,17 @@ def test_long_k_down_on_split_gemm_pp(cuda, m):
         d = d.materialize()
     torch.testing.assert_close(y.float(), ref, atol=3e-2, rtol=3e-2)
     torch.testing.assert_close(d.float(), ref, atol=3e-2, rtol=3e-2)
+
+
+@pytest.mark.parametrize("m", [257, 400, 700])
+@pytest.mark.parametrize("n,swiglu", [(11 * 128, False), (13 * 128, True), (40 * 128, False)])
+def test_equal_rows_of_several_row_tiles(cuda, m, n, swiglu):
+    """Row tiles of one column of an unsplit grid on different XCDs sum K in the same order: equal rows, equal results.
+    (11 and 13 columns of 2 or 3 row tiles straddle the XCDs' runs of workgroups.)"""
+    k = 2048
+    x, w = _bf(1, k).expand(m, k).contiguous(), _bf(n, k, scale=0.05)
+    y = gemm.linear_wide(x, w, splits=1, swiglu=swiglu)
+    assert torch.equal(y, y[:1].expand_as(y))
+    from distributed_llms_amd.ops import quant
+    q = quant.linear_fp8(x, quant.quantize_weight(w), swiglu=swiglu, splits=1)
+    assert torch.equal(q, q[:1].expand_as(q))
