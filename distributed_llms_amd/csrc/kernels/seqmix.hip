@@ -28,23 +28,23 @@ template <typename T, int V>
 __global__ void __launch_bounds__(256) sm_embed_kernel(float* __restrict__ out, const int32_t* __restrict__ ids,
                                                        const void* __restrict__ table_, int width, int vocab,
                                                        float scale) {
-  const int i = (blockIdx.y * 256 + threadIdx.x) * V;
-  if (i >= width) return;
   int id = ids[blockIdx.x];
   id = id < 0 ? 0 : (id >= vocab ? vocab - 1 : id);
-  float v[V];
-  ldv<V>((const T*)table_ + (size_t)id * width + i, v);
+  for (long i = (blockIdx.y * 256L + threadIdx.x) * V; i < width; i += gridDim.y * 256L * V) {
+    float v[V];
+    ldv<V>((const T*)table_ + (size_t)id * width + i, v);
 #pragma unroll
-  for (int j = 0; j < V; ++j) v[j] *= scale;
-  stv<V>(out + (size_t)blockIdx.x * width + i, v);
+    for (int j = 0; j < V; ++j) v[j] *= scale;
+    stv<V>(out + (size_t)blockIdx.x * width + i, v);
+  }
 }
 
 void sm_embed_f32(uintptr_t out, uintptr_t ids, uintptr_t table, int tokens, int width, int vocab, float scale, int f32,
                   uintptr_t stream) {
   if (tokens <= 0) return;
-  DLLM_HOST_CHECK(width > 0 && width <= 256 * 65535 && vocab > 0, "embed sizes");
+  DLLM_HOST_CHECK(width > 0 && vocab > 0, "embed sizes");
   const bool vec = width % 8 == 0 && table % 32 == 0 && out % 32 == 0;
-  const dim3 grid(tokens, (width + (vec ? 2047 : 255)) / (vec ? 2048 : 256));
+  const dim3 grid(tokens, std::min(65535, (width - 1) / (vec ? 2048 : 256) + 1));
   SM_DISPATCH_V(f32, vec, sm_embed_kernel, grid, dim3(256), 0, stream, (float*)out, (const int32_t*)ids,
                 (const void*)table, width, vocab, scale);
 }

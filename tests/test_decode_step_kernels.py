@@ -162,6 +162,16 @@ def test_rglru_step_keeps_no_process_wide_state():
 
 
 @gpu
+@pytest.mark.parametrize("width", [1, 2047, 2056, 256 * 65535 + 3])
+def test_embedding_f32_of_any_width(cuda, width):
+    """Vector and scalar pieces, a partial last workgroup, and a row of more pieces than a grid has workgroups."""
+    table = torch.arange(2 * width, device=cuda).view(2, width).remainder(251).bfloat16()
+    ids = torch.tensor([1, 0, 5, -1], dtype=torch.int32, device=cuda)
+    out = sm.embedding_f32(ids, table, 3.0)
+    assert torch.equal(out, table[[1, 0, 1, 0]].float() * 3.0)
+
+
+@gpu
 @pytest.mark.parametrize("rows", [1, 7, 300])
 @pytest.mark.parametrize("width", [4, 250, 1024, 2560, 4100, 16384, 16392])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
