@@ -388,70 +388,86 @@ __device__ __forceinline__ void post_layer_norm_row(
   float* xr = x + row;
   typedef T vec __attribute__((ext_vector_type(V)));
   typedef float fvec __attribute__((ext_vector_type(V)));
-  constexpr bool kEarly = NV * V <= 16;           // wider rows do not hold the weights as well
+  // up to 16 elements per lane are held with all that goes with them; a wider row's stream and weights come in rounds of 16
+  // elements (all at once they took 512 registers and scratch: 4096 rows of 16383, f32, 664 us, of 4097 241)
+  constexpr bool kEarly = NV * V <= 16;
+  constexpr int CH = kEarly ? NV : 16 / V;
   float v[NV][V], xv[NV][V];
   fvec rx[NV];
   vec rw[NV], rb[NV], rwn[NV], rbn[NV], rc[NV];
-  // every load of the row off a clamped place, in its stored form and before the first use: no load waits behind
-  // another's guard or conversion, and the next norm's weights do not wait for this one's sums (16 rows of 2560: with 12 slabs 8.6 us
-  // before, 5.4 now, without 4.7 and 3.6; 6376 rows 34.2 and 30.5)
+  // every load off a clamped place, in its stored form and before the first use: no load waits behind
+  // another's guard or conversion, and the next norm's weights do not wait for this one's sums (16 rows of 2560: with 12
+  // slabs 8.6 us before, 5.4 now, without 4.7 and 3.6; 6376 rows 34.2 and 30.5)
   auto at = [&](int k) { return min((k * 256 + (int)threadIdx.x) * V, width - V); };
-  auto load = [&](vec (&r)[NV], const void* from) {
+  auto load = [&](vec (&r)[NV], const void* from, int k0, int n) {
 #pragma unroll
-    for (int k = 0; k < NV; ++k) r[k] = *reinterpret_cast<const vec*>((const T*)from + at(k));
+    for (int k = k0; k < k0 + n; ++k) r[k] = *reinterpret_cast<const vec*>((const T*)from + at(k));
   };
+  auto load_x = [&](int k0, int n) {
 #pragma unroll
-  for (int k = 0; k < NV; ++k) rx[k] = *reinterpret_cast<const fvec*>(xr + at(k));
+    for (int k = k0; k < k0 + n; ++k) rx[k] = *reinterpret_cast<const fvec*>(xr + at(k));
+  };
   vec ro[NV];
-  if (!SLABS && kEarly) load(ro, (const T*)o_ + row);
-  if (kEarly) load(rw, wp_), load(rb, bp_);
-  if (kEarly && bias_) load(rc, bias_);
-  if (kEarly && wn_) load(rwn, wn_), load(rbn, bn_);
+  if (kEarly) load_x(0, NV);
+  if (!SLABS) load(ro, (const T*)o_ + row, 0, NV);
+  if (kEarly) load(rw, wp_, 0, NV), load(rb, bp_, 0, NV);
+  if (kEarly && bias_) load(rc, bias_, 0, NV);
+  if (kEarly && wn_) load(rwn, wn_, 0, NV), load(rbn, bn_, 0, NV);
   if constexpr (SLABS) {
     ln_slabs<NV>((const float*)o_, parts, row, width, v);
   } else {
 #pragma unroll
-    for (int k = 0; k < NV; ++k) {
-      if (!kEarly) ro[k] = *reinterpret_cast<const vec*>((const T*)o_ + row + at(k));
+    for (int k = 0; k < NV; ++k)
 #pragma unroll
       for (int j = 0; j < V; ++j) v[k][j] = (float)ro[k][j];
-    }
   }
 #pragma unroll
-  for (int k = 0; k < NV; ++k) {
-    const bool in = (k * 256 + (int)threadIdx.x) * V < width;
-    if (!kEarly && bias_) rc[k] = *reinterpret_cast<const vec*>((const T*)bias_ + at(k));
+  for (int k0 = 0; k0 < NV; k0 += CH) {
+    if (!kEarly && bias_) load(rc, bias_, k0, CH);
 #pragma unroll
-    for (int j = 0; j < V; ++j) {
-      if (bias_) v[k][j] += (float)rc[k][j];
-      v[k][j] = in ? v[k][j] : 0.f;
-      xv[k][j] = in ? rx[k][j] : 0.f;
+    for (int k = k0; k < k0 + CH; ++k) {
+      const bool in = (k * 256 + (int)threadIdx.x) * V < width;
+#pragma unroll
+      for (int j = 0; j < V; ++j) {
+        if (bias_) v[k][j] += (float)rc[k][j];
+        v[k][j] = in ? v[k][j] : 0.f;
+      }
     }
   }
   float mean, inv;
   ln_stats<V, NV>(v, width, eps, red, mean, inv);
-  if (!kEarly) load(rw, wp_), load(rb, bp_);
 #pragma unroll
-  for (int k = 0; k < NV; ++k) {
-    const int i = (k * 256 + threadIdx.x) * V;
-    if (i < width) {
+  for (int k0 = 0; k0 < NV; k0 += CH) {
+    if (!kEarly) load_x(k0, CH), load(rw, wp_, k0, CH), load(rb, bp_, k0, CH);
 #pragma unroll
-      for (int j = 0; j < V; ++j) xv[k][j] += (v[k][j] - mean) * inv * (float)rw[k][j] + (float)rb[k][j];
-      stv<V>(xr + i, xv[k]);
+    for (int k = k0; k < k0 + CH; ++k) {
+      const int i = (k * 256 + threadIdx.x) * V;
+#pragma unroll
+      for (int j = 0; j < V; ++j) xv[k][j] = i < width ? rx[k][j] : 0.f;
+      if (i < width) {
+#pragma unroll
+        for (int j = 0; j < V; ++j) xv[k][j] += (v[k][j] - mean) * inv * (float)rw[k][j] + (float)rb[k][j];
+        stv<V>(xr + i, xv[k]);
+      }
     }
+    if (!kEarly) __builtin_amdgcn_sched_barrier(0);
   }
   if (!wn_) return;
-  if (!kEarly) load(rwn, wn_), load(rbn, bn_);
   ln_stats<V, NV>(xv, width, eps, red + 8, mean, inv);
   T* h = (T*)h_ + row;
 #pragma unroll
-  for (int k = 0; k < NV; ++k) {
-    const int i = (k * 256 + threadIdx.x) * V;
-    if (i < width) {
+  for (int k0 = 0; k0 < NV; k0 += CH) {
+    if (!kEarly) load(rwn, wn_, k0, CH), load(rbn, bn_, k0, CH);
 #pragma unroll
-      for (int j = 0; j < V; ++j) xv[k][j] = (xv[k][j] - mean) * inv * (float)rwn[k][j] + (float)rbn[k][j];
-      stv<V>(h + i, xv[k]);
+    for (int k = k0; k < k0 + CH; ++k) {
+      const int i = (k * 256 + threadIdx.x) * V;
+      if (i < width) {
+#pragma unroll
+        for (int j = 0; j < V; ++j) xv[k][j] = (xv[k][j] - mean) * inv * (float)rwn[k][j] + (float)rbn[k][j];
+        stv<V>(h + i, xv[k]);
+      }
     }
+    if (!kEarly) __builtin_amdgcn_sched_barrier(0);
   }
 }
 
@@ -483,9 +499,11 @@ __global__ void __launch_bounds__(256) sm_post_layer_norm_slabs_kernel(
       else if (np_ <= 3) SM_LN_GO(f32, KERNEL, 4, 3, grid, stream, __VA_ARGS__);                                   \
       else if (np_ <= 4) SM_LN_GO(f32, KERNEL, 4, 4, grid, stream, __VA_ARGS__);                                   \
       else if (np_ <= 8) SM_LN_GO(f32, KERNEL, 4, 8, grid, stream, __VA_ARGS__);                                   \
+      else if (np_ <= 12) SM_LN_GO(f32, KERNEL, 4, 12, grid, stream, __VA_ARGS__);                                 \
       else SM_LN_GO(f32, KERNEL, 4, 16, grid, stream, __VA_ARGS__);                                                \
     } else if (np_ <= 4) SM_LN_GO(f32, KERNEL, 1, 4, grid, stream, __VA_ARGS__);                                   \
     else if (np_ <= 16) SM_LN_GO(f32, KERNEL, 1, 16, grid, stream, __VA_ARGS__);                                   \
+    else if (np_ <= 32) SM_LN_GO(f32, KERNEL, 1, 32, grid, stream, __VA_ARGS__);                                   \
     else SM_LN_GO(f32, KERNEL, 1, 64, grid, stream, __VA_ARGS__);                                                  \
     DLLM_HIP_CHECK(hipGetLastError());                                                                             \
   } while (0)

@@ -272,3 +272,40 @@ def test_decode_attention_without_block_ids(cuda, fused):
     else:
         out = ops.paged_attention_decode(torch.randn(b, hq, d).bfloat16().cuda(), k, v, bt, none, d ** -0.5)
     assert torch.equal(out, torch.zeros_like(out))
+
+
+@gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("width", [4097, 8191, 8193, 8200, 12288, 12292, 16383])
+def test_norm_rows_past_4096(cuda, width, dtype):
+    """The closes of a sublayer and the layer norm on rows whose stream and weights come in rounds: partial last pieces of
+    the 12- and 16-piece forms, and odd widths."""
+    g = torch.Generator().manual_seed(width)
+    r = lambda *s: torch.randn(*s, generator=g)
+    x, o, b, wp, bp, wn, bn = (r(3, width), r(3, width).to(dtype)) + tuple(r(width).to(dtype) for _ in range(5))
+    c = lambda *t: [v.cuda() for v in t]
+    tol = dict(atol=5e-5, rtol=5e-5) if dtype == torch.float32 else dict(atol=1e-3, rtol=2.0 ** -7)
+    co, cb, cwp, cbp, cwn, cbn = c(o, b, wp, bp, wn, bn)
+    for gpu_, cpu in ((sm.post_norm_add(x.cuda(), co, cwp, 1e-6, 0.8, bias=cb, w_next=cwn),
+                       sm.post_norm_add(x.clone(), o, wp, 1e-6, 0.8, bias=b, w_next=wn)),
+                      (sm.post_layer_norm_add(x.cuda(), co, cwp, cbp, 1e-6, bias=cb, w_next=cwn, b_next=cbn),
+                       sm.post_layer_norm_add(x.clone(), o, wp, bp, 1e-6, bias=b, w_next=wn, b_next=bn))):
+        torch.testing.assert_close(gpu_[0].cpu(), cpu[0], atol=5e-5, rtol=5e-5)
+        torch.testing.assert_close(gpu_[1].float().cpu(), cpu[1].float(), **tol)
+    torch.testing.assert_close(sm.layer_norm_f32(x.cuda(), cwp, cbp, 1e-6, dtype).float().cpu(),
+                               sm.layer_norm_f32(x, wp, bp, 1e-6, dtype).float(), **tol)
+
+
+@gpu
+@pytest.mark.parametrize("n", [8192, 16384])
+def test_wide_closes_sum_split_products(cuda, n):
+    x, w = torch.randn(3, 1024, device=cuda).bfloat16(), (torch.randn(n, 1024, device=cuda) * 0.03).bfloat16()
+    s, v = torch.randn(3, n, device=cuda), [torch.randn(n, device=cuda).bfloat16() for _ in range(4)]
+    for close in (lambda t, o: sm.post_norm_add(t, o, v[0], 1e-6, 0.8, w_next=v[1]),
+                  lambda t, o: sm.post_layer_norm_add(t, o, v[0], v[1], 1e-6, w_next=v[2], b_next=v[3])):
+        part = gemm.linear_wide(x, w, splits=2, defer=True)
+        assert isinstance(part, gemm.SplitKPartial)
+        got = close(s.clone(), part)
+        want = close(s.clone(), gemm.linear_wide(x, w, splits=2))
+        torch.testing.assert_close(got[0], want[0], atol=1e-5, rtol=1e-5)
+        torch.testing.assert_close(got[1].float(), want[1].float(), atol=1e-3, rtol=2.0 ** -7)
