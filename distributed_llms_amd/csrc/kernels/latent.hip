@@ -191,21 +191,29 @@ __global__ void __launch_bounds__(256) lat_q_fold_kernel(void* __restrict__ out_
 }
 
 // bf16 with 8 | rank: a thread owns 8 consecutive outputs (16-byte weight loads) and every ng-th input
-// row; the ng partial sums of an output meet in LDS.  kFoldRows rows' loads are in flight per thread, the first of them
-// before the inputs are staged (one row at a time it was a round trip each: 32 rows of 16 heads 7.7 -> 6.2 us, the
-// values 6.6 -> 5.6 us).
-constexpr int kFoldRows = 16;
+// row; the ng partial sums of an output meet in LDS.  R rows' loads are in flight per thread (fold_rows), the first of them
+// before the inputs are staged (one row at a time it was a round trip each).
+template <int R>
 struct FoldRows {
-  bf16x8 w[kFoldRows];
+  bf16x8 w[R];
   // rows first, first + ng, .. of w [rows, pitch], the last one repeated past the end
   __device__ __forceinline__ void load(const bf16* __restrict__ wc, int first, int ng, int rows, int pitch) {
 #pragma unroll
-    for (int k = 0; k < kFoldRows; ++k)
+    for (int k = 0; k < R; ++k)
       w[k] = *reinterpret_cast<const bf16x8*>(wc + (size_t)min(first + k * ng, rows - 1) * pitch);
   }
-  __device__ __forceinline__ void add(float (&acc)[8], const float* x, int first, int ng, int rows) const {
+  __device__ __forceinline__ void add(float (&acc)[8], const float* x, int first, int ng, int rows, bool all) const {
+    if (all) {                                               // (uniform) every row of the round exists
 #pragma unroll
-    for (int k = 0; k < kFoldRows; ++k) {
+      for (int k = 0; k < R; ++k) {
+        const float xv = x[first + k * ng];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) acc[i] = fmaf(xv, bf2f(w[k][i]), acc[i]);
+      }
+      return;
+    }
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
       const int r = first + k * ng;
       const float xv = x[min(r, rows - 1)];
 #pragma unroll
@@ -217,6 +225,7 @@ struct FoldRows {
   }
 };
 
+template <int R>
 __global__ void __launch_bounds__(256) lat_q_fold_vec_kernel(bf16* __restrict__ out_, const bf16* __restrict__ q_,
                                                              long ldq, const bf16* __restrict__ wuk, int H, int rank,
                                                              int dim, int rot_dim, int half, const float* __restrict__ freqs, int nfreq,
@@ -230,15 +239,15 @@ __global__ void __launch_bounds__(256) lat_q_fold_vec_kernel(bf16* __restrict__ 
   const bf16* q = q_ + (size_t)t * ldq + h * dq;
   const bf16* w = wuk + (size_t)h * dim * rank;
   const int nc = rank >> 3, c = threadIdx.x % nc, g = threadIdx.x / nc;
-  FoldRows rows;
+  FoldRows<R> rows;
   rows.load(w + 8 * c, g, ng, dim, rank);
   for (int d = threadIdx.x; d < dim; d += 256) qs[d] = bf2f(q[d]);
   __syncthreads();
   if (g < ng) {
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    for (int d = 0; d < dim; d += kFoldRows * ng) {
+    for (int d = 0; d < dim; d += R * ng) {
       if (d > 0) rows.load(w + 8 * c, d + g, ng, dim, rank);
-      rows.add(acc, qs, d + g, ng, dim);
+      rows.add(acc, qs, d + g, ng, dim, d + R * ng <= dim);
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) red[g * rank + 8 * c + i] = acc[i];
@@ -254,6 +263,21 @@ __global__ void __launch_bounds__(256) lat_q_fold_vec_kernel(bf16* __restrict__ 
     rotate_row<bf16>(out + rank, q + dim, i, rot_dim, half, freqs, nfreq, pos);
 }
 
+// Rows in flight per thread (`per`: rows that it adds in all).  16 only while every workgroup has a CU to itself and they
+// are all used; four, a quarter of the registers, are as fast or faster on a larger grid (64 rows of 32 heads, 384 x 96:
+// 11.6 us, 13.2 with 8, 17.2 with 16), and loads that repeat the last row only cost (8 heads of 64 x 32, one row: 3.2 us
+// with one, 3.4 with four, 4.6 with 16; one at a time before 3.2).  16 heads of 512 x 128, 1 / 16 / 64 rows: 16 rows 5.8 / 7.0 /
+// 10.3 us, four 7.3 / 7.9 / 9.7, one at a time 12.5 / 12.7 / 13.9.
+static int fold_rows(int per, long wgs) { return per <= 1 ? 1 : per <= 2 ? 2 : wgs <= 256 && per % 16 == 0 ? 16 : 4; }
+#define FOLD_DISPATCH(KERNEL, per, wgs)                  \
+  do {                                                   \
+    const int r_ = fold_rows(per, wgs);                  \
+    if (r_ == 1) go(KERNEL<1>);                          \
+    else if (r_ == 2) go(KERNEL<2>);                     \
+    else if (r_ == 4) go(KERNEL<4>);                     \
+    else go(KERNEL<16>);                                 \
+  } while (0)
+
 // groups of input rows for the vector forms: as many as 256 threads allow, at most one per input row
 static int fold_groups(int out_width, int in_width) { return std::max(1, std::min(256 / (out_width / 8), in_width)); }
 
@@ -265,9 +289,12 @@ void lat_q_fold(uintptr_t out, uintptr_t q, long ldq, uintptr_t wuk, int tokens,
   DLLM_HOST_CHECK(out && q && wuk && (nfreq == 0 || freqs) && ldq >= (long)H * (dim + rot_dim), "latent query arguments");
   if (!f32 && rank % 8 == 0 && rank <= 2048) {
     const int ng = fold_groups(rank, dim);
-    hipLaunchKernelGGL(lat_q_fold_vec_kernel, dim3(tokens, H), dim3(256), sizeof(float) * ((size_t)dim + (size_t)ng * rank),
-                       (hipStream_t)stream, (bf16*)out, (const bf16*)q, ldq, (const bf16*)wuk, H, rank, dim, rot_dim, half,
-                       (const float*)freqs, nfreq, (const int32_t*)positions, ng);
+    const auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3(tokens, H), dim3(256), sizeof(float) * ((size_t)dim + (size_t)ng * rank),
+                         (hipStream_t)stream, (bf16*)out, (const bf16*)q, ldq, (const bf16*)wuk, H, rank, dim, rot_dim, half,
+                         (const float*)freqs, nfreq, (const int32_t*)positions, ng);
+    };
+    FOLD_DISPATCH(lat_q_fold_vec_kernel, (dim + ng - 1) / ng, (long)tokens * H);
     DLLM_HIP_CHECK(hipGetLastError());
     return;
   }
@@ -300,6 +327,7 @@ __global__ void __launch_bounds__(256) lat_v_unfold_kernel(void* __restrict__ ou
   }
 }
 
+template <int R>
 __global__ void __launch_bounds__(256) lat_v_unfold_vec_kernel(bf16* __restrict__ out_, const bf16* __restrict__ o_,
                                                                const bf16* __restrict__ wuv_t,
                                                                const bf16* __restrict__ gate, long ld, int wide, int H,
@@ -312,15 +340,15 @@ __global__ void __launch_bounds__(256) lat_v_unfold_vec_kernel(bf16* __restrict_
   const bf16* o = o_ + ((size_t)t * H + h) * rank;
   const bf16* w = wuv_t + (size_t)h * rank * vdim;
   const int nc = vdim >> 3, c = threadIdx.x % nc, g = threadIdx.x / nc;
-  FoldRows rows;
+  FoldRows<R> rows;
   rows.load(w + 8 * c, g, ng, rank, vdim);
   for (int r = threadIdx.x; r < rank; r += 256) os[r] = bf2f(o[r]);
   __syncthreads();
   if (g < ng) {
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    for (int r = 0; r < rank; r += kFoldRows * ng) {
+    for (int r = 0; r < rank; r += R * ng) {
       if (r > 0) rows.load(w + 8 * c, r + g, ng, rank, vdim);
-      rows.add(acc, os, r + g, ng, rank);
+      rows.add(acc, os, r + g, ng, rank, r + R * ng <= rank);
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) red[g * vdim + 8 * c + i] = acc[i];
@@ -342,9 +370,12 @@ void lat_v_unfold(uintptr_t out, uintptr_t o, uintptr_t wuv_t, uintptr_t gate, l
                   "latent value arguments");
   if (!f32 && vdim % 8 == 0 && vdim <= 2048) {
     const int ng = fold_groups(vdim, rank);
-    hipLaunchKernelGGL(lat_v_unfold_vec_kernel, dim3(tokens, H), dim3(256),
+    const auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3(tokens, H), dim3(256),
                        sizeof(float) * ((size_t)rank + (size_t)ng * vdim), (hipStream_t)stream, (bf16*)out,
                        (const bf16*)o, (const bf16*)wuv_t, (const bf16*)gate, ld, wide, H, rank, vdim, ng);
+    };
+    FOLD_DISPATCH(lat_v_unfold_vec_kernel, (rank + ng - 1) / ng, (long)tokens * H);
     DLLM_HIP_CHECK(hipGetLastError());
     return;
   }

@@ -309,3 +309,19 @@ def test_wide_closes_sum_split_products(cuda, n):
         want = close(s.clone(), gemm.linear_wide(x, w, splits=2))
         torch.testing.assert_close(got[0], want[0], atol=1e-5, rtol=1e-5)
         torch.testing.assert_close(got[1].float(), want[1].float(), atol=1e-3, rtol=2.0 ** -7)
+
+
+@gpu
+@pytest.mark.parametrize("rows,heads", [(1, 3), (18, 16)])
+@pytest.mark.parametrize("n_in,n_out", [(7, 32), (16, 32), (24, 128), (50, 128), (61, 512), (64, 512), (96, 384), (130, 512), (256, 64)])
+def test_latent_products_by_rows_in_flight(cuda, rows, heads, n_in, n_out):
+    """One, two, four and 16 weight rows in flight per thread, whole and partial rounds; grids of up to 256 workgroups and
+    more (the 16-row form is the small grids')."""
+    from distributed_llms_amd.ops import latent as lat
+    q, uk = torch.randn(rows, heads * n_in, device=cuda).bfloat16(), torch.randn(heads, n_in, n_out, device=cuda).bfloat16()
+    spec = lat.LatentSpec(heads=heads, dim=n_in, vdim=n_out, rank=n_out, q_rank=0, scale=1.0)
+    pos = torch.arange(rows, dtype=torch.int32, device=cuda)
+    q3 = q.view(rows, heads, n_in).double().transpose(0, 1)
+    want, mag = (torch.matmul(a, b).transpose(0, 1) for a, b in ((q3, uk.double()), (q3.abs(), uk.double().abs())))
+    for got in (lat.latent_queries(q, uk, spec, None, pos), lat.latent_values(q.view(rows, heads, n_in), uk).view(rows, heads, n_out)):
+        assert ((got.double() - want).abs() <= n_in * 2.0 ** -24 * mag + 2.0 ** -8 * want.abs()).all()
