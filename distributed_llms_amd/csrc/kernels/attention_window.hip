@@ -875,8 +875,12 @@ void sm_window_attn_decode(uintptr_t out, uintptr_t q, uintptr_t k_cache, uintpt
                                      D, Dv, bs, window, chunk, scale, sinks, splits, ws, softcap, kp, vp, pool, pbs, \
                                      0, 0, keep, gate, gate_ld, stream);                                           \
   } while (0)
-    if (D <= 64 && Dv <= 64) WIN_DEC(2, 4);
+    if (D <= 32 && Dv <= 32) WIN_DEC(1, 2);
+    else if (D <= 64 && Dv <= 64) WIN_DEC(2, 4);
+    else if (D <= 96 && Dv <= 96) WIN_DEC(3, 6);
     else if (D <= 128 && Dv <= 128) WIN_DEC(4, 8);
+    else if (D <= 192 && Dv <= 128) WIN_DEC(6, 8);
+    else if (D <= 192 && Dv <= 192) WIN_DEC(6, 12);
     else WIN_DEC(8, 16);
 #undef WIN_DEC
     return;

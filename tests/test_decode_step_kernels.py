@@ -325,3 +325,29 @@ def test_latent_products_by_rows_in_flight(cuda, rows, heads, n_in, n_out):
     want, mag = (torch.matmul(a, b).transpose(0, 1) for a, b in ((q3, uk.double()), (q3.abs(), uk.double().abs())))
     for got in (lat.latent_queries(q, uk, spec, None, pos), lat.latent_values(q.view(rows, heads, n_in), uk).view(rows, heads, n_out)):
         assert ((got.double() - want).abs() <= n_in * 2.0 ** -24 * mag + 2.0 ** -8 * want.abs()).all()
+
+
+@gpu
+@pytest.mark.parametrize("d,dv", [(8, 8), (32, 32), (40, 24), (64, 64), (72, 96), (96, 96), (104, 128), (136, 128), (192, 128),
+                                  (168, 136), (192, 192), (200, 192), (256, 256)])
+@pytest.mark.parametrize("biased", [False, True])
+def test_window_decode_head_sizes(cuda, d, dv, biased):
+    """Every head size that has a kernel of its own, at its edges: contexts within a tile, past one and past a wave's share."""
+    lens, h, g, bs, size = [1, 31, 33, 100, 700], 6, 2, 16, 300
+    nb = (max(lens) + bs - 1) // bs
+    b = len(lens)
+    kc, vc = torch.randn(b * nb + 1, g, bs, d, device=cuda).bfloat16(), torch.randn(b * nb + 1, g, dv, bs, device=cuda).bfloat16()
+    bt = (torch.randperm(b * nb, device=cuda) + 1).int().view(b, nb)
+    q, bias = torch.randn(b, h, d, device=cuda).bfloat16(), torch.randn(h, 50, device=cuda) if biased else None
+    out = sm.window_attention(q, kc, vc, bt, _sb([n - 1 for n in lens], list(range(b)), cuda), size, d ** -0.5, bias=bias)
+    for i, n in enumerate(lens):
+        at = torch.arange(max(0, n - size), n, device=cuda)
+        blk = bt[i].long()[at // bs]
+        k = kc[blk, :, at % bs].double().repeat_interleave(h // g, 1)                # [keys, h, d]
+        v = vc[blk, :, :, at % bs].double().repeat_interleave(h // g, 1)
+        s = (q[i].double() * k).sum(-1) * d ** -0.5
+        if biased:
+            s = s + bias.double()[:, (n - 1 - at).clamp_max(49)].t()
+        want = (torch.softmax(s, 0)[..., None] * v).sum(0)
+        # scores: d exact products, 2^-24 of their magnitudes (below 2^-15 in all); weights kept to 17 bits; the result in 8
+        assert ((out[i].double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -13 * v.abs().max()).all()
