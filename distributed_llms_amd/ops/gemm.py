@@ -105,31 +105,50 @@ def _use_wide(m: int, n: int, k: int, x: torch.Tensor, w: torch.Tensor, swiglu: 
     return ("down" in roles) if is_down_proj(n, k) else ("proj" in roles and m <= 512)
 
 
-# Weights (elements) up to which gemm_stream serves M <= 64 rows; all sides measured on cold weights, us at M = 1 / 16 /
-# 32 / 64, a split-K reduction or an activation kernel in a launch of its own being 4.6 each (gemm_stream.hip):
-#  * plain: 5120 x 2560 7.0 / 8.2 / 9.7 / 12.5 against 12.5 / 13.1 / 13.6 / 14.2 for the wide kernel and its reduction;
-#    6144 x 4096 10.3 / 12.4 / 13.8 / 17.1 against 14.8 / 15.4 / 15.8 / 16.2;
-#  * the consumer sums the slabs (defer), so the wide kernel pays no reduction: 2560 x 2560 4.7 / 5.9 / 7.4 / 9.7 against
-#    6.7 / 7.2 / 7.7 / 8.2, 1024 x 1024 3.0 / 3.4 / 4.0 / 5.1 against 5.0 / 5.4 / 5.5 / 5.6;
-#  * GLU: 15360 x 2560 14.2 / 14.7 / 16.2 / 19.7 against 20.4 / 21.1 / 22.1 / 23.1; the 8B gate|up (28672 x 4096) 38 / 39 /
-#    44 / 48 against 38 / 38.6 / 40 / 41 for the wide kernel's own SiLU epilogue, which has no other activation.
+# Where gemm_stream serves M <= 64 rows.  A launch and the slab sum that it saves are worth 2-4 us; what it pays is x, staged
+# once per workgroup (so long K and many rows lose), and a last round of workgroups that leaves CUs idle.  Both sides as a
+# caller gets them (reduction, gate kernel or closing norm included), cold weights, us, this kernel / the former route:
+#  * plain, N a multiple of 128 (gemm_wide and its slab sum), M = 1 / 16 / 32 / 64: 1024 x 1024 2.8 / 3.0 / 3.4 / 4.2, 6.8 / 7.3 /
+#    7.5 / 7.5; 4096 x 4096 8.3 / 8.7 / 10.4 / 13.6, 10.6 / 10.8 / 11.8 / 12.8; 2560 x 7680 10.5 / 13.3 / 16.8 / 22.8, 14.2 / 15.2 /
+#    15.5 / 16.3; 1024 x 14336, 16 rows, 19.3, 16.9; 8192 x 4096 16.2 / 15.9 / 16.4, 15.6 / 15.6 / 16.0;
+#  * a bias or another N (F.linear), M = 17 / 33: 4096 x 4096 9-11, 17-24; 500 x 8192 12.3 / 16.5, 11.5 / 11.6; 6144 x 4096, 32
+#    rows, 15.6, 14.8;
+#  * in front of a close that sums the slabs itself, close included, M = 1 / 16 / 32 / 64: 2560 x 2560 7.6 / 9.1 / 10.6 / 13.3,
+#    10.5 / 11.1 / 11.5 / 12.6; 512 x 4096 7.1 / 8.4 / 10.2 / 13.0, 8.6 / 9.1 / 9.2 / 9.5; 1024 x 8192, 16 rows, 13.2, 10.7;
+#  * GLU, M = 1 / 32 / 64: 15360 x 2560 15.8 / 16.9 / 20.4, 18.4 / 19.3 / 20.9; 16384 x 4096 30.2 / 29.7 / 32.0, 34.4 / 33.6 / 34.3;
+#    22016 x 4096 39.8 / 44.0 / 51.3, 34.1 / 35.0 / 39.2; 10240 x 4096 (160 workgroups) 22.0 / 22.6 / 25.7, 18.6 / 19.2 / 20.6;
+#    28672 x 4096 41.8 / 45.0 / 53.4, 41.0 / 39.8 / 42.5; 4096 x 8192 17.8 / 24.0 / 28.7, 16.2 / 18.2 / 19.3.
 STREAM_MAX_M = 64
-STREAM_PLAIN, STREAM_PLAIN_32 = 16 << 20, 32 << 20
-STREAM_DEFER, STREAM_DEFER_16 = 2 << 20, 8 << 20
-STREAM_GLU, STREAM_GLU_32 = 40 << 20, 128 << 20
 
 
-def stream_fits(m: int, n: int, k: int, glu: str = "", defer: bool = False) -> bool:
+def _stream_fill(cols: int) -> float:
+    """Share of the CUs that a round of gemm_stream's workgroups for ``cols`` output columns keeps busy (its launcher's rule:
+    tiles of 16 columns, of 32 once there are more than 256)."""
+    tiles = -(-cols // 16)
+    tiles = -(-cols // 32) if tiles > 256 else tiles
+    return tiles / (256 * -(-tiles // 256))
+
+
+def stream_fits(m: int, n: int, k: int, glu: str = "", defer: bool = False, bias: bool = False) -> bool:
     """Does gemm_stream serve an [m, k] x [n, k]^T product?  ``glu``: "" (plain), "silu", "clipped" or "gelu"."""
     if not 1 <= m <= STREAM_MAX_M or k % 64 or k < 512:
         return False                                 # K < 512: fewer K-tiles than waves, and no split to save either
+    mi = n * k / (1 << 20)
     if glu:
-        return n * k <= (STREAM_GLU_32 if m <= 32 and glu != "silu" else STREAM_GLU)
+        if k > (4096 if m <= 32 else 2560) or (mi > (20 if m <= 32 else 12) and _stream_fill(n // 2) < 0.75):
+            return False
+        return mi <= (64 if m <= 32 and glu != "silu" else 40)
     if n > 65536:
         return False                                 # an LM head fills the chip unsplit on the wide kernel
     if defer and n % 128 == 0:
-        return n * k <= (STREAM_DEFER_16 if m <= 16 else STREAM_DEFER)
-    return n * k <= (STREAM_PLAIN_32 if m <= 32 else STREAM_PLAIN)
+        return (mi <= 8 and k <= 4096) if m <= 16 else (mi <= 2 and k <= 2048)
+    if m <= 16:
+        return mi <= 24 and k <= 8192
+    if m <= 32:
+        return mi <= 24 and k <= 4096
+    if bias or n % 128:
+        return mi <= 16 and k <= 4096
+    return mi <= 12.5 and k <= 2560
 
 
 def _recorded(*tensors) -> bool:
@@ -148,7 +167,7 @@ def _recorded(*tensors) -> bool:
 
 
 def use_stream(m: int, n: int, k: int, x: torch.Tensor, w: torch.Tensor, bias=None, glu: str = "", defer: bool = False) -> bool:
-    return (knobs.K.stream and stream_fits(m, n, k, glu, defer) and not _recorded(x, w, bias) and x.dtype == w.dtype == torch.bfloat16
+    return (knobs.K.stream and stream_fits(m, n, k, glu, defer, bias is not None) and not _recorded(x, w, bias) and x.dtype == w.dtype == torch.bfloat16
             and x.is_contiguous() and w.is_contiguous() and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
             and (bias is None or (bias.dtype == torch.bfloat16 and tuple(bias.shape) == (n,) and bias.is_contiguous()
                                   and bias.device == x.device)))

@@ -98,6 +98,14 @@ def test_stream_rule():
     assert not gemm.stream_fits(1, 4096, 4096, defer=True)             # the 8B projections stay on the wide kernel
     assert not gemm.stream_fits(1, 28672, 4096, "silu") and gemm.stream_fits(64, 15360, 2560, "gelu")
     assert not gemm.stream_fits(8, 1024, 448)
+    # long K and many rows, few columns: staging x once per workgroup costs more than the saved launch
+    assert gemm.stream_fits(16, 2048, 8192) and not gemm.stream_fits(17, 2048, 8192) and not gemm.stream_fits(16, 1024, 14336)
+    assert gemm.stream_fits(32, 1024, 4096) and not gemm.stream_fits(33, 1024, 4096) and gemm.stream_fits(33, 1024, 4096, bias=True)
+    assert not gemm.stream_fits(33, 500, 8192) and gemm.stream_fits(64, 500, 4096)
+    assert not gemm.stream_fits(16, 1024, 8192, defer=True) and not gemm.stream_fits(17, 512, 4096, defer=True)
+    # GLU: a round of workgroups that leaves CUs idle, K past 4096
+    assert gemm.stream_fits(32, 16384, 4096, "gelu") and not gemm.stream_fits(1, 22016, 4096, "gelu")
+    assert not gemm.stream_fits(1, 10240, 4096, "silu") and not gemm.stream_fits(1, 4096, 8192, "clipped")
     x, w = torch.zeros(4, 512, dtype=torch.bfloat16), torch.zeros(256, 512, dtype=torch.bfloat16)
     assert gemm.use_stream(4, 256, 512, x, w)
     assert not gemm.use_stream(4, 256, 512, x.float(), w) and not gemm.use_stream(4, 256, 512, x, w.t().contiguous().t())
