@@ -547,7 +547,7 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor) -> Optional[torch.Te
     """silu(x Wg^T) * (x Wu^T) with W = [Wg; Wu] in one launch; None if the shape is not eligible."""
     m, n, k = _sizes(x, w_gate_up, "linear_swiglu")
     kn = knobs.K
-    if n % 2 == 0 and use_stream(m, n, k, x, w_gate_up, glu="silu"):
+    if n % 16 == 0 and use_stream(m, n, k, x, w_gate_up, glu="silu"):      # (the SiLU kernels' multiples of 8, at any m)
         return linear_stream(x, w_gate_up, glu="silu")
     if 0 < kn.pp_gate_up_min_m <= m <= 256 and not _comm_cus and _use_pp(m, n, k, x, w_gate_up, 1):
         # decode gate|up on gemm_pp, unsplit, weights nontemporal, on the column tile that gives one

@@ -120,6 +120,14 @@ def test_traced_calls_keep_the_product(launches):
     assert not launches
 
 
+def test_swiglu_of_an_odd_width_stays_refused(launches):
+    """The SiLU GLU takes intermediate sizes in multiples of 8, at every number of rows."""
+    for n in (1000, 1002):
+        assert gemm.linear_swiglu(_bf(4, 1024), _bf(n, 1024)) is None and not launches
+    gemm.linear_swiglu(_bf(4, 1024), _bf(1008, 1024))
+    assert [n for n, _ in launches] == ["gemm_stream"]
+
+
 def test_fp8_weight_in_front_of_a_norm():
     """linear_into_norm takes what linear(defer=True) takes: an fp8 weight too (latent_attention's output projection)."""
     from distributed_llms_amd import ops
