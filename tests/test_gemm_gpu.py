@@ -430,9 +430,11 @@ def test_equal_rows_of_several_row_tiles(cuda, m, n, swiglu):
     """Row tiles of one column of an unsplit grid on different XCDs sum K in the same order: equal rows, equal results.
     (11 and 13 columns of 2 or 3 row tiles straddle the XCDs' runs of workgroups.)"""
     k = 2048
-    x, w = _bf(1, k).expand(m, k).contiguous(), _bf(n, k, scale=0.05)
+    # the second half of K cancels the first: what is left is the rounding of the sums, which any other order changes
+    x, w = _bf(1, k // 2).repeat(m, 2), _bf(n, k // 2, scale=2.0)
+    w = torch.cat([w, -w], 1)
     y = gemm.linear_wide(x, w, splits=1, swiglu=swiglu)
-    assert torch.equal(y, y[:1].expand_as(y))
+    assert y.any() and torch.equal(y, y[:1].expand_as(y))
     from distributed_llms_amd.ops import quant
     q = quant.linear_fp8(x, quant.quantize_weight(w), swiglu=swiglu, splits=1)
     assert torch.equal(q, q[:1].expand_as(q))
