@@ -16,7 +16,7 @@ sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.dirname(os.path.abspa
 
 import torch
 
-from distributed_llms_amd import knobs, ops
+from distributed_llms_amd import ops
 from distributed_llms_amd.ops import gemm
 
 SHAPES = {"qkv": (6144, 4096, False), "o": (4096, 4096, False), "gate_up": (28672, 4096, True),
@@ -60,7 +60,7 @@ def main():
                 fns[f"sq{sp}"] = (lambda sp: lambda x, w: gemm.linear_sq(x, w, splits=sp, swiglu=sw))(sp)
             for bm in ([] if a.no_wide else a.bms):
                 for s in a.splits:
-                    v = knobs.K.wide_variant_split if s > 1 else knobs.K.wide_variant
+                    v = gemm.wide_variant(n, k, s, bm)                        # the engine's choice
                     fns[f"w{bm}s{s}"] = (lambda bm, s, v: lambda x, w: gemm.linear_wide(
                         x, w, splits=s, swiglu=sw, variant=v | (bm << 8)))(bm, s, v)
             ok = {}

@@ -341,6 +341,16 @@ def wide_splits(m: int, n: int, k: int, swiglu: bool = False, target_wgs: int = 
 WIDE_NT_MIN_BYTES = 12 << 20
 
 
+def wide_variant(n: int, k: int, splits: int, bm: int) -> int:
+    """gemm_wide's variant for this weight, number of K slices and row tile: knobs.wide_variant on unsplit grids; on split
+    ones knobs.wide_variant_split (weights nontemporal, each byte is read from memory once per step) -- but the default
+    cache policy below WIDE_NT_MIN_BYTES (a small model's weights stay in the 256 MiB Infinity Cache from step to step:
+    1024 x 1024 5.0 -> 5.9 us with nt) and on 192-row tiles (8B down at M = 192: 32.0 -> 34.0 us)."""
+    if splits == 1:
+        return knobs.K.wide_variant
+    return knobs.K.wide_variant_split if n * k * 2 >= WIDE_NT_MIN_BYTES and bm != 192 else 1
+
+
 def linear_wide(x: torch.Tensor, w: torch.Tensor, splits: int = 0, swiglu: bool = False, defer: bool = False,
                 variant: int = -1):
     """Wide-M decode GEMM (csrc/kernels/gemm_wide.hip): 256 x 128 x 64 tiles, 3-deep LDS-DMA pipeline,
@@ -361,12 +371,7 @@ def linear_wide(x: torch.Tensor, w: torch.Tensor, splits: int = 0, swiglu: bool 
         s = max(1, ws.numel() // (m * n))
     stream = torch.cuda.current_stream().cuda_stream
     bm = wide_row_tile(m, n, k, swiglu)
-    v = variant if variant >= 0 else knobs.K.wide_variant
-    if s > 1 and variant < 0:
-        # split grids: weights nontemporal where each byte is read from memory once per step -- not below
-        # WIDE_NT_MIN_BYTES (a small model's weights stay in the 256 MiB Infinity Cache from step to step: 1024 x 1024
-        # 5.0 -> 5.9 us with nt), and not on 192-row tiles (8B down at M = 192: 32.0 -> 34.0 us)
-        v = knobs.K.wide_variant_split if n * k * 2 >= WIDE_NT_MIN_BYTES and bm != 192 else 1
+    v = variant if variant >= 0 else wide_variant(n, k, s, bm)
     if bm != wide_bm(m):
         v |= bm << 8
     if defer and not swiglu and s > 1:

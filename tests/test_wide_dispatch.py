@@ -300,3 +300,11 @@ def test_prefill_attention_auto_version():
     for v in (3, 4, 6, 7, 9):
         with knobs.override(prefill_attn=v):
             assert ops.prefill_attn_version(4096, 128) == v
+
+
+def test_wide_variant_by_weight_and_tile():
+    """Unsplit grids: the knob; split ones: nontemporal weights, but not small ones and not on 192-row tiles."""
+    big, small = (4096, 14336), (1024, 1024)
+    assert gemm.wide_variant(*big, 1, 192) == gemm.wide_variant(*small, 1, 64) == knobs.K.wide_variant
+    assert gemm.wide_variant(*big, 4, 256) == knobs.K.wide_variant_split
+    assert gemm.wide_variant(*big, 4, 192) == gemm.wide_variant(*small, 4, 64) == 1
