@@ -234,15 +234,6 @@ __device__ __forceinline__ void part_store(float* P, size_t i, float v) {
   P[i] = v;
 #endif
 }
-__device__ __forceinline__ float part_load1(const float* P, size_t i) {
-#if DLLM_PART_TYPE == 1
-  return bf2f(reinterpret_cast<const bf16*>(P)[i]);
-#elif DLLM_PART_TYPE == 2
-  return (float)reinterpret_cast<const _Float16*>(P)[i] * kPartUnscale;
-#else
-  return P[i];
-#endif
-}
 // The stored form of an element, for a caller that has several loads under way before it converts any (a conversion next
 // to its load makes hipcc wait there)
 #if DLLM_PART_TYPE == 1

@@ -3,12 +3,13 @@
 // second one to sum its slabs and (behind a bias) a third for the activation.
 //
 // At these sizes a projection of a 1k-4k wide model is a few microseconds of weight bytes, and every further launch
-// costs about 4.6 us (the end of one kernel to the start of the next inside a graph, plus its first load's round trip).
+// (a slab sum, a gate kernel) costs 2-4 us: the end of one kernel to the start of the next inside a graph, plus its first
+// load's round trip.  Where it is the faster route: ops/gemm.stream_fits.
 //
 //  * one workgroup owns RT x 16 weight rows and all of K, so nothing is left to sum in memory; its waves take the
 //    64-deep K-tiles in turn (wave v: tiles v, v + WAVES, ...), so that together they read 512-byte or 1 KiB runs of
 //    every row;
-//  * a wave stages its tiles -- weights and x -- through an LDS ring of its OWN (D slots, global_load_lds_dwordx4 in
+//  * a wave stages its tiles -- weights and x -- through an LDS ring of its OWN (two slots, global_load_lds_dwordx4 in
 //    whole 128-byte lines, the chunk swizzle c ^ ((row >> 1) & 7) on the source address and on the read): no barrier
 //    in the K loop, the only waits are the wave's counted vmcnt.  x fragments straight from global memory touch 16
 //    half lines per load and took 1.3-2x as long at 16-64 rows (2560 x 2560: 8.1 / 12.4 / 19.2 us at M = 16 / 32 / 64
@@ -28,13 +29,14 @@ namespace {
 typedef __attribute__((address_space(3))) void* lds_vptr_s;
 typedef __attribute__((address_space(1))) void* glb_vptr_s;
 constexpr int SK = 64;                    // K-tile
+constexpr int D = 2;                      // slots of a wave's ring
 
 __device__ __forceinline__ int sswz(int row, int chunk) { return chunk ^ ((row >> 1) & 7); }
 }  // namespace
 
 // GLU 0: y [M, N] (+ bias [N]);  1 / 2 / 3: SiLU / clipped (`limit`) / gelu GLU, w = [gate; up], y [M, N / 2], bias
 // gate | up.  GLU tiles hold RT / 2 16-row tiles of gate rows, then the same output columns' up rows.
-template <int RT, int MT, int D, int GLU, bool NT, int WAVES>
+template <int RT, int MT, int GLU, bool NT, int WAVES>
 __global__ void __launch_bounds__(WAVES * 64) gemm_stream_kernel(bf16* __restrict__ Y, const bf16* __restrict__ X,
                                                                  const bf16* __restrict__ W,
                                                                  const bf16* __restrict__ bias, int M, int N, int K,
@@ -43,7 +45,7 @@ __global__ void __launch_bounds__(WAVES * 64) gemm_stream_kernel(bf16* __restric
   constexpr int SLOT = (RT + MT) * 16 * SK;                     // bf16 elements of one ring slot: weights, then x
   constexpr int G = 2 * (RT + MT);                              // loads per K-tile
   constexpr int RING = WAVES * D * SLOT * 2, RED = WAVES * RT * MT * 1024;
-  static_assert((D - 1) * G <= 63, "vmcnt");
+  static_assert(G <= 63, "vmcnt");
   __shared__ __attribute__((aligned(16))) char smem[RING > RED ? RING : RED];
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int fr = lane & 15, fq = lane >> 4;
@@ -93,9 +95,8 @@ __global__ void __launch_bounds__(WAVES * 64) gemm_stream_kernel(bf16* __restric
     for (int u = 0; u < D; ++u) {
       const int i = i0 + u;                                       // wave-uniform
       if (i < cnt) {
-        // tile i has landed when only the younger tiles' loads are left: min(D - 1, cnt - 1 - i) of them
-        if (D > 1 && cnt - 1 - i >= D - 1) asm volatile("s_waitcnt vmcnt(%0)" ::"i"((D - 1) * G) : "memory");
-        else if (D > 2 && cnt - 1 - i == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(D > 2 ? G : 0) : "memory");
+        // tile i has landed when only the younger tile's loads are left, if there is one
+        if (i + 1 < cnt) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(G) : "memory");
         else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
         const bf16* b = ring + u * SLOT;
@@ -184,9 +185,9 @@ void gemm_stream(uintptr_t y, uintptr_t x, uintptr_t w, uintptr_t bias, int M, i
   // workgroups per CU)
 #define DLLM_ST_GO(RT_, MT_, GLU_, WV_)                                                                              \
   do {                                                                                                              \
-    if (nt) hipLaunchKernelGGL((gemm_stream_kernel<RT_, MT_, 2, GLU_, true, WV_>), grid, dim3(WV_ * 64), 0, s,         \
+    if (nt) hipLaunchKernelGGL((gemm_stream_kernel<RT_, MT_, GLU_, true, WV_>), grid, dim3(WV_ * 64), 0, s,         \
                                (bf16*)y, (const bf16*)x, (const bf16*)w, (const bf16*)bias, M, N, K, limit);          \
-    else hipLaunchKernelGGL((gemm_stream_kernel<RT_, MT_, 2, GLU_, false, WV_>), grid, dim3(WV_ * 64), 0, s,           \
+    else hipLaunchKernelGGL((gemm_stream_kernel<RT_, MT_, GLU_, false, WV_>), grid, dim3(WV_ * 64), 0, s,           \
                             (bf16*)y, (const bf16*)x, (const bf16*)w, (const bf16*)bias, M, N, K, limit);             \
   } while (0)
 #define DLLM_ST_M(RT_, GLU_, WV_)                                                                                    \

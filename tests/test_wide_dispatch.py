@@ -304,6 +304,7 @@ def test_prefill_attention_auto_version():
 
 def test_wide_variant_by_weight_and_tile():
     """Unsplit grids: the knob; split ones: nontemporal weights, but not small ones and not on 192-row tiles."""
+    from distributed_llms_amd import knobs
     big, small = (4096, 14336), (1024, 1024)
     assert gemm.wide_variant(*big, 1, 192) == gemm.wide_variant(*small, 1, 64) == knobs.K.wide_variant
     assert gemm.wide_variant(*big, 4, 256) == knobs.K.wide_variant_split
