@@ -76,18 +76,55 @@ def test_stream_glu_keeps_the_gate_kernels_arithmetic(cuda, glu):
     assert torch.equal(gemm.linear_stream(x, w, None, glu, 7.0), want.bfloat16())
 
 
+@pytest.fixture
+def counted(monkeypatch):
+    """The calls that reach the kernel's entry point."""
+    calls, real = [], gemm.linear_stream
+    monkeypatch.setattr(gemm, "linear_stream", lambda *a, **kw: (calls.append(a), real(*a, **kw))[1])
+    return calls
+
+
 @pytest.mark.gpu
-def test_stream_is_reached_and_matches_the_wide_route(cuda):
+def test_stream_is_reached_and_matches_the_wide_route(cuda, counted):
     """ops.linear / linear_swiglu at decode sizes take the kernel by default; knobs.stream off gives the former route."""
     from distributed_llms_amd import ops
     x = torch.randn(9, 1024, device="cuda").bfloat16()
     w = (torch.randn(2048, 1024, device="cuda") * 0.03).bfloat16()
     for f in (lambda: ops.linear(x, w), lambda: ops.linear_swiglu(x, w), lambda: ops.linear(x[:, None], w)):
         a = f()
+        assert len(counted) == 1
         with knobs.override(stream=False):
             b = f()
+        assert len(counted) == 1
+        counted.clear()
         assert a.shape == b.shape
         torch.testing.assert_close(a.float(), b.float(), atol=2e-2, rtol=2e-2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,reached", [(16, 2560, True), (17, 2560, False), (16, 4096, False), (64, 512, True), (65, 512, False)])
+def test_stream_in_front_of_a_close(cuda, counted, m, n, reached):
+    """linear_into_norm on both sides of its cutover: the finished product, or the slabs of a split grid."""
+    from distributed_llms_amd import ops
+    k = 1024 if n == 512 else 2560
+    x, w = torch.randn(m, k, device="cuda").bfloat16(), (torch.randn(n, k, device="cuda") * 0.03).bfloat16()
+    y = ops.linear_into_norm(x, w)
+    assert len(counted) == reached and isinstance(y, torch.Tensor) >= reached
+    y = y if isinstance(y, torch.Tensor) else y.materialize()
+    torch.testing.assert_close(y.float(), x.float() @ w.float().t(), atol=2e-2, rtol=2e-2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,reached", [(1, True), (64, True), (65, False)])
+@pytest.mark.parametrize("biased", [False, True])
+def test_stream_under_the_clipped_glu(cuda, counted, m, reached, biased):
+    from distributed_llms_amd.ops import seqmix as sm
+    x, w = torch.randn(m, 1024, device="cuda").bfloat16(), (torch.randn(3072, 1024, device="cuda") * 0.03).bfloat16()
+    b = torch.randn(3072, device="cuda").bfloat16() if biased else None
+    y = sm.linear_clipped_glu(x, w, b, 0.7)
+    assert len(counted) == reached
+    gu = x.float() @ w.float().t() + (0 if b is None else b.float())
+    torch.testing.assert_close(y.float(), sm.clipped_glu(gu, None, 0.7), atol=2e-2, rtol=2e-2)
 
 
 def test_stream_rule():
