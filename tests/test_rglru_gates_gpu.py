@@ -68,3 +68,33 @@ def test_gates_of_the_largest_inputs(cuda):
     ok[2:4] = False
     torch.testing.assert_close(a[ok].double(), want[ok], rtol=1e-5, atol=1e-12)
     assert a[2:4, 0].isnan().all() and (a[2:4, 1] == a[4, 1]).all()
+
+
+@pytest.mark.parametrize("nb,bw", [(3, 128), (2, 256), (1, 512)])
+def test_gates_see_the_last_bits_of_the_input(cuda, nb, bw):
+    """One product per sum (a permutation for the weights), so that nothing but the input's own bits and the float32 functions
+    round: the third piece shows in every block and every K chunk.  z = -3 .. -6: the gates are open to a change of z."""
+    tokens = 130
+    g = torch.Generator().manual_seed(bw)
+    u = -(3.0 + 3.0 * torch.rand(tokens, nb, bw, generator=g))
+    perm = torch.stack([torch.randperm(bw, generator=g) for _ in range(nb)])          # output o reads input perm[o]
+    w = torch.zeros(nb, bw, bw)
+    w[torch.arange(nb)[:, None], perm, torch.arange(bw)] = 1.0
+    zero, lam = torch.zeros(nb, bw).bfloat16(), torch.full((nb, bw), 3.0).bfloat16()
+    a, _ = _gates(cuda, u, w.bfloat16(), zero, w.bfloat16(), zero, lam)
+    at = perm.expand(tokens, nb, bw)
+
+    def gate(v):
+        z = torch.gather(v.double(), 2, at)
+        return z, 8.0 * torch.sigmoid(z) * torch.nn.functional.softplus(lam.double())
+    z, e = gate(u)
+    want = torch.exp(-e)
+    # the exponent: the three pieces' sum (2^-23 of z at most, which moves it by as much of e |z|), expf, two additions, a
+    # division, softplus and two products at 2^-23 or less each: 12 x 2^-24 of it; the last expf 2^-22
+    tol = want * (e * z.abs() * 2.0 ** -23 + e * 12 * 2.0 ** -24 + 2.0 ** -22)
+    assert ((a.double() - want).abs() <= tol).all()
+    h = u.bfloat16()
+    two = h.double() + (u - h.float()).bfloat16().double()                            # an input of two pieces would be seen
+    seen = (torch.exp(-gate(two)[1]) - want).abs() > tol
+    chunk = torch.nn.functional.one_hot(at // 64, bw // 64).bool()
+    assert ((seen[..., None] & chunk).sum(0).sum(1) > 0.5 * chunk.sum(0).sum(1)).all()
