@@ -237,7 +237,7 @@ class HybridStage(LayerListStage):
             elif m["width"] % m["blocks"]:
                 raise ValueError(f"layer {i}: width is not a multiple of blocks")
         self.kv_layers = [i for i, l in enumerate(self.specs) if kv_width(l)]
-        self.state = None              # per layer {"conv": ..., "s": ...}
+        self.state = None              # per layer {"conv": ..., "s": ..., "arrived": ...}
         self.rot = {}                  # layer -> (freqs [dims/2] f32, magnitude)
         for i, l in enumerate(self.specs):
             if l["type"] == "attention":

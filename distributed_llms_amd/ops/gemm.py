@@ -62,12 +62,12 @@ _CUS = {}
 def _sizes(x: torch.Tensor, w: torch.Tensor, name: str):
     """(rows, N, K) of ``x w^T``; raises where the kernels, which see pointers and these numbers alone, would read past
     ``w`` or another device's memory."""
-    k = x.shape[-1]
-    if w.dim() != 2 or w.shape[1] != k:
+    k = x.size(-1)
+    if w.dim() != 2 or w.size(1) != k:
         raise ValueError(f"{name}: x[..., {k}] vs w {tuple(w.shape)}")
     if w.device != x.device:
         raise ValueError(f"{name}: x on {x.device}, w on {w.device}")
-    return x.numel() // k, w.shape[0], k
+    return x.numel() // k, w.size(0), k
 
 
 def pf_fills(m: int, n: int, device) -> bool:
@@ -151,26 +151,31 @@ def stream_fits(m: int, n: int, k: int, glu: str = "", defer: bool = False, bias
     return mi <= 12.5 and k <= 2560
 
 
-def _recorded(*tensors) -> bool:
+_modes, _tracing, _transforms = (torch._C._len_torch_dispatch_stack, torch._C._get_tracing_state,
+                                 torch._C._functorch.peek_interpreter_stack)
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
+def _recorded(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor]) -> bool:
     """Is the call differentiated, transformed or traced (autograd, forward mode, vmap; torch.jit.trace, torch.compile,
-    make_fx and other dispatch modes; tensor subclasses)?  The kernels leave no trace of it."""
-    if torch._C._len_torch_dispatch_stack() or torch._C._get_tracing_state() is not None or torch.compiler.is_compiling():
+    make_fx and other dispatch modes; tensor subclasses)?  The kernels leave no trace of it.  (Questions to the process
+    first: an eager pass asks this for every product, and per tensor they cost three times as much.)"""
+    if _modes() or _tracing() is not None or _transforms() is not None or forward_ad._current_level >= 0 \
+            or torch.compiler.is_compiling():
         return True
-    for t in tensors:
-        if t is not None and type(t) not in (torch.Tensor, torch.nn.Parameter):
-            return True
-        if t is not None and (torch._C._functorch.is_functorch_wrapped_tensor(t)
-                              or (t.requires_grad and torch.is_grad_enabled())
-                              or (forward_ad._current_level >= 0 and forward_ad.unpack_dual(t).tangent is not None)):
-            return True
-    return False
+    if type(x) not in _PLAIN or type(w) not in _PLAIN or (bias is not None and type(bias) not in _PLAIN):
+        return True
+    return torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or (bias is not None and bias.requires_grad))
 
 
 def use_stream(m: int, n: int, k: int, x: torch.Tensor, w: torch.Tensor, bias=None, glu: str = "", defer: bool = False) -> bool:
-    return (knobs.K.stream and stream_fits(m, n, k, glu, defer, bias is not None) and not _recorded(x, w, bias) and x.dtype == w.dtype == torch.bfloat16
-            and x.is_contiguous() and w.is_contiguous() and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
-            and (bias is None or (bias.dtype == torch.bfloat16 and tuple(bias.shape) == (n,) and bias.is_contiguous()
-                                  and bias.device == x.device)))
+    return (knobs.K.stream and stream_fits(m, n, k, glu, defer, bias is not None) and x.dtype == w.dtype == torch.bfloat16
+            # (a plain product without a bias, N a multiple of 128, and every GLU has kernels on either route)
+            and not (not glu and (bias is not None or n % 128) and _recorded(x, w, bias))
+            and x.is_contiguous() and w.is_contiguous() and x.data_ptr() % 16 == 0
+            and w.data_ptr() % 16 == 0
+            and (bias is None or (bias.dtype == torch.bfloat16 and bias.dim() == 1 and bias.size(0) == n
+                                  and bias.is_contiguous() and bias.device == x.device)))
 
 
 def linear_into_norm(x: torch.Tensor, w: torch.Tensor):
@@ -178,7 +183,7 @@ def linear_into_norm(x: torch.Tensor, w: torch.Tensor):
     where the weight-streaming kernel is faster than the split grid alone, else possibly a :class:`SplitKPartial`."""
     m, n, k = _sizes(x, w, "linear_into_norm")
     if use_stream(m, n, k, x, w, defer=True):
-        return linear_stream(x, w)
+        return _stream(m, n, k, x, w)
     return linear(x, w, defer=True)
 
 
@@ -188,7 +193,12 @@ _STREAM_GLU = {"": 0, "silu": 1, "clipped": 2, "gelu": 3}
 def linear_stream(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, glu: str = "",
                   limit: float = 0.0) -> torch.Tensor:
     """y = x w^T (+ bias), or its GLU with w = [Wg; Wu], for up to 64 rows (csrc/kernels/gemm_stream.hip)."""
-    m, n, k = _sizes(x, w, "linear_stream")
+    return _stream(*_sizes(x, w, "linear_stream"), x, w, bias, glu, limit)
+
+
+def _stream(m: int, n: int, k: int, x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, glu: str = "",
+            limit: float = 0.0) -> torch.Tensor:
+    """:func:`linear_stream` of operands whose sizes the caller has compared."""
     y = torch.empty(*x.shape[:-1], n // 2 if glu else n, dtype=x.dtype, device=x.device)
     _ext.kernels().gemm_stream(y.data_ptr(), x.data_ptr(), w.data_ptr(), 0 if bias is None else bias.data_ptr(), m, n, k,
                                _STREAM_GLU[glu], 1 if n * k * 2 >= WIDE_NT_MIN_BYTES else 0, float(limit),
@@ -224,7 +234,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
     m, n, k = _sizes(x, w, "linear")
     kn = knobs.K
     if not (defer and n % 128 == 0) and use_stream(m, n, k, x, w, bias):
-        return linear_stream(x, w, bias)
+        return _stream(m, n, k, x, w, bias)
     # decode LM head on gemm_pp with nontemporal weights (236 vs 268 us for gemm_sq at M = 256) --
     # unless comm kernels may hold CUs: beside a 4-workgroup, 20 KiB-LDS receive spinning in
     # another process it took 284 us, gemm_sq 268 either way (bench/debug/lm_head_bench.py,
@@ -517,7 +527,7 @@ def _linear_glu(x: torch.Tensor, w_gate_up: torch.Tensor, limit: Optional[float]
     m, n, k = _sizes(x, w_gate_up, "linear_glu")
     glu = "gelu" if limit is None else "clipped"
     if n % 2 == 0 and use_stream(m, n, k, x, w_gate_up, bias, glu):
-        return linear_stream(x, w_gate_up, bias, glu, 0.0 if limit is None else limit)
+        return _stream(m, n, k, x, w_gate_up, bias, glu, 0.0 if limit is None else limit)
     if x.dtype != torch.bfloat16 or n % 256 or bias is not None:
         return None
     if not _use_wide(m, n, k, x, w_gate_up) and _use_pp(m, n, k, x, w_gate_up, knobs.K.pp_swiglu_min_m) \
@@ -553,7 +563,7 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor) -> Optional[torch.Te
     m, n, k = _sizes(x, w_gate_up, "linear_swiglu")
     kn = knobs.K
     if n % 16 == 0 and use_stream(m, n, k, x, w_gate_up, glu="silu"):      # (the SiLU kernels' multiples of 8, at any m)
-        return linear_stream(x, w_gate_up, glu="silu")
+        return _stream(m, n, k, x, w_gate_up, glu="silu")
     if 0 < kn.pp_gate_up_min_m <= m <= 256 and not _comm_cus and _use_pp(m, n, k, x, w_gate_up, 1):
         # decode gate|up on gemm_pp, unsplit, weights nontemporal, on the column tile that gives one
         # round of CUs / 2 .. CUs tiles: 8B (224 x 128 columns) 62.1 vs 64.1 us for gemm_wide, 70B

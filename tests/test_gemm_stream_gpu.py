@@ -79,8 +79,8 @@ def test_stream_glu_keeps_the_gate_kernels_arithmetic(cuda, glu):
 @pytest.fixture
 def counted(monkeypatch):
     """The calls that reach the kernel's entry point."""
-    calls, real = [], gemm.linear_stream
-    monkeypatch.setattr(gemm, "linear_stream", lambda *a, **kw: (calls.append(a), real(*a, **kw))[1])
+    calls, real = [], gemm._stream
+    monkeypatch.setattr(gemm, "_stream", lambda *a, **kw: (calls.append(a), real(*a, **kw))[1])
     return calls
 
 
