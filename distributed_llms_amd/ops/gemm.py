@@ -110,7 +110,8 @@ def _use_wide(m: int, n: int, k: int, x: torch.Tensor, w: torch.Tensor, swiglu: 
 # caller gets them (reduction, gate kernel or closing norm included), cold weights, us, this kernel / the former route:
 #  * plain, N a multiple of 128 (gemm_wide and its slab sum), M = 1 / 16 / 32 / 64: 1024 x 1024 2.8 / 3.0 / 3.4 / 4.2, 6.8 / 7.3 /
 #    7.5 / 7.5; 4096 x 4096 8.3 / 8.7 / 10.4 / 13.6, 10.6 / 10.8 / 11.8 / 12.8; 2560 x 7680 10.5 / 13.3 / 16.8 / 22.8, 14.2 / 15.2 /
-#    15.5 / 16.3; 1024 x 14336, 16 rows, 19.3, 16.9; 8192 x 4096 16.2 / 15.9 / 16.4, 15.6 / 15.6 / 16.0;
+#    15.5 / 16.3; 1024 x 14336, 16 rows, 19.3, 16.9; 8192 x 4096 16.2 / 15.9 / 16.4, 15.6 / 15.6 / 16.0; 32000 x 1024 11.9 / 12.2 /
+#    14.6, 12.6 / 12.6 / 12.8; 5120 x 4096 (160 workgroups), 32 rows, 14.6, 13.6;
 #  * a bias or another N (F.linear), M = 17 / 33: 4096 x 4096 9-11, 17-24; 500 x 8192 12.3 / 16.5, 11.5 / 11.6; 6144 x 4096, 32
 #    rows, 15.6, 14.8;
 #  * in front of a close that sums the slabs itself, close included, M = 1 / 16 / 32 / 64: 2560 x 2560 7.6 / 9.1 / 10.6 / 13.3,
@@ -143,9 +144,9 @@ def stream_fits(m: int, n: int, k: int, glu: str = "", defer: bool = False, bias
     if defer and n % 128 == 0:
         return (mi <= 8 and k <= 4096) if m <= 16 else (mi <= 2 and k <= 2048)
     if m <= 16:
-        return mi <= 24 and k <= 8192
+        return mi <= (32 if k <= 2560 else 24) and k <= 8192
     if m <= 32:
-        return mi <= 24 and k <= 4096
+        return mi <= 24 and k <= 4096 and (mi <= 16 or _stream_fill(n) >= 0.75)
     if bias or n % 128:
         return mi <= 16 and k <= 4096
     return mi <= 12.5 and k <= 2560

@@ -140,6 +140,8 @@ def test_stream_rule():
     assert gemm.stream_fits(32, 1024, 4096) and not gemm.stream_fits(33, 1024, 4096) and gemm.stream_fits(33, 1024, 4096, bias=True)
     assert not gemm.stream_fits(33, 500, 8192) and gemm.stream_fits(64, 500, 4096)
     assert not gemm.stream_fits(16, 1024, 8192, defer=True) and not gemm.stream_fits(17, 512, 4096, defer=True)
+    assert gemm.stream_fits(16, 32000, 1024) and not gemm.stream_fits(17, 32000, 1024) and not gemm.stream_fits(16, 8192, 4096)
+    assert gemm.stream_fits(16, 5120, 4096) and not gemm.stream_fits(32, 5120, 4096)
     # GLU: a round of workgroups that leaves CUs idle, K past 4096
     assert gemm.stream_fits(32, 16384, 4096, "gelu") and not gemm.stream_fits(1, 22016, 4096, "gelu")
     assert not gemm.stream_fits(1, 10240, 4096, "silu") and not gemm.stream_fits(1, 4096, 8192, "clipped")
