@@ -60,7 +60,7 @@ def main():
                 fns[f"sq{sp}"] = (lambda sp: lambda x, w: gemm.linear_sq(x, w, splits=sp, swiglu=sw))(sp)
             for bm in ([] if a.no_wide else a.bms):
                 for s in a.splits:
-                    v = gemm.wide_variant(n, k, s, bm)                        # the engine's choice
+                    v = gemm.wide_variant(m, n, k, s, bm)                        # the engine's choice
                     fns[f"w{bm}s{s}"] = (lambda bm, s, v: lambda x, w: gemm.linear_wide(
                         x, w, splits=s, swiglu=sw, variant=v | (bm << 8)))(bm, s, v)
             ok = {}

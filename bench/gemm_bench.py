@@ -66,7 +66,7 @@ def wide(a):
             x = torch.randn(m, k, device="cuda").to(torch.bfloat16)
             # one HIP graph per implementation: `copies` back-to-back calls, each on its own weight
             # copy (launch overhead out of the measurement, like the engine's captured decode step)
-            wv = gemm.wide_variant(n, k, a.splits or gemm.wide_splits(m, n, k, sw), gemm.wide_row_tile(m, n, k, sw))   # the engine's choice
+            wv = gemm.wide_variant(m, n, k, a.splits or gemm.wide_splits(m, n, k, sw), gemm.wide_row_tile(m, n, k, sw))   # the engine's choice
             impls = {
                 "wide": lambda w: gemm.linear_wide(x, w, splits=a.splits, swiglu=sw, variant=wv),
                 **{f"v{v}": (lambda w, v=v: gemm.linear_wide(x, w, splits=a.splits, swiglu=sw, variant=v))

@@ -34,10 +34,8 @@ class Knobs:
     # up to 64 rows of a small weight on the weight-streaming kernel (gemm_stream.hip; ops/gemm.stream_fits)
     stream: bool = True
     # gemm_wide variant for unsplit grids (33: LDS-DMA interleaved + asm fragment reads with one
-    # lgkmcnt per MFMA row) and for split-K grids (2: weights nontemporal, each byte is read once per
-    # launch: 8B down 21.7 -> 19.6 us at M = 1, 23.2 -> 21.6 at 64, 34.1 -> 33.4 at 256; qkv 10.9 -> 10.1
-    # at M = 1, 17.8 -> 17.4 at 256; o 8.1 -> 7.7, 15.1 -> 14.6; small weights and 192-row tiles take 1
-    # whatever this says: ops/gemm.wide_variant)
+    # lgkmcnt per MFMA row) and for split-K grids of up to 64 rows or long slices (2: weights nontemporal;
+    # the others, small weights and 192-row tiles take 1: ops/gemm.wide_variant)
     wide_variant: int = 33
     wide_variant_split: int = 2
     wide_gate_up_max_m: int = 256     # SwiGLU-fused gate|up on gemm_wide up to this M (then split-K gemm_pp / gemm_pf)

@@ -352,14 +352,20 @@ def wide_splits(m: int, n: int, k: int, swiglu: bool = False, target_wgs: int = 
 WIDE_NT_MIN_BYTES = 12 << 20
 
 
-def wide_variant(n: int, k: int, splits: int, bm: int) -> int:
-    """gemm_wide's variant for this weight, number of K slices and row tile: knobs.wide_variant on unsplit grids; on split
-    ones knobs.wide_variant_split (weights nontemporal, each byte is read from memory once per step) -- but the default
-    cache policy below WIDE_NT_MIN_BYTES (a small model's weights stay in the 256 MiB Infinity Cache from step to step:
-    1024 x 1024 5.0 -> 5.9 us with nt) and on 192-row tiles (8B down at M = 192: 32.0 -> 34.0 us)."""
+def wide_variant(m: int, n: int, k: int, splits: int, bm: int) -> int:
+    """gemm_wide's variant for these sizes, number of K slices and row tile: knobs.wide_variant on unsplit grids; on split
+    ones knobs.wide_variant_split (weights nontemporal, each byte is read from memory once per step) or the default cache
+    policy (1).  Nontemporal weights make the product 2-14 % faster, but from about 64 rows on the launch that sums the slabs
+    loses more than that, unless a slice is long.  With its consumer (add + RMS norm), default -> nontemporal, us, M = 16 / 64 /
+    128 / 256: 4096 x 4096 12.1 / 13.0 / 15.5 / 19.8 -> 11.3 / 13.2 / 16.2 / 20.1; 6144 x 4096 15.6 / 16.7 / 19.3 / 26.6 -> 14.8 /
+    16.8 / 20.0 / 26.9; 4096 x 14336 (28 K-tiles a slice) 25.3 / 26.9 / 31.1 / 41.6 -> 23.4 / 25.9 / 30.5 / 41.5.  Below
+    WIDE_NT_MIN_BYTES a small model's weights stay in the 256 MiB Infinity Cache from step to step (1024 x 1024 5.0 -> 5.9 us
+    with nt), and on 192-row tiles it is slower throughout (8B down at M = 192: 32.0 -> 34.0 us)."""
     if splits == 1:
         return knobs.K.wide_variant
-    return knobs.K.wide_variant_split if n * k * 2 >= WIDE_NT_MIN_BYTES and bm != 192 else 1
+    if n * k * 2 < WIDE_NT_MIN_BYTES or bm == 192 or (m > 64 and k // 64 < 24 * splits):
+        return 1
+    return knobs.K.wide_variant_split
 
 
 def linear_wide(x: torch.Tensor, w: torch.Tensor, splits: int = 0, swiglu: bool = False, defer: bool = False,
@@ -382,7 +388,7 @@ def linear_wide(x: torch.Tensor, w: torch.Tensor, splits: int = 0, swiglu: bool 
         s = max(1, ws.numel() // (m * n))
     stream = torch.cuda.current_stream().cuda_stream
     bm = wide_row_tile(m, n, k, swiglu)
-    v = variant if variant >= 0 else wide_variant(n, k, s, bm)
+    v = variant if variant >= 0 else wide_variant(m, n, k, s, bm)
     if bm != wide_bm(m):
         v |= bm << 8
     if defer and not swiglu and s > 1:

@@ -303,9 +303,10 @@ def test_prefill_attention_auto_version():
 
 
 def test_wide_variant_by_weight_and_tile():
-    """Unsplit grids: the knob; split ones: nontemporal weights, but not small ones and not on 192-row tiles."""
+    """Unsplit grids: the knob; split ones: nontemporal weights, but not small ones, not on 192-row tiles and from 65 rows on
+    only with long slices."""
     from distributed_llms_amd import knobs
-    big, small = (4096, 14336), (1024, 1024)
-    assert gemm.wide_variant(*big, 1, 192) == gemm.wide_variant(*small, 1, 64) == knobs.K.wide_variant
-    assert gemm.wide_variant(*big, 4, 256) == knobs.K.wide_variant_split
-    assert gemm.wide_variant(*big, 4, 192) == gemm.wide_variant(*small, 4, 64) == 1
+    down, o, small = (4096, 14336), (4096, 4096), (1024, 1024)
+    assert gemm.wide_variant(180, *down, 1, 192) == gemm.wide_variant(1, *small, 1, 64) == knobs.K.wide_variant
+    assert gemm.wide_variant(256, *down, 8, 256) == gemm.wide_variant(64, *o, 8, 64) == knobs.K.wide_variant_split
+    assert gemm.wide_variant(180, *down, 8, 192) == gemm.wide_variant(1, *small, 4, 64) == gemm.wide_variant(65, *o, 8, 128) == 1
