@@ -183,9 +183,9 @@ def linear_into_norm(x: torch.Tensor, w: torch.Tensor):
     """``x w^T`` for a consumer that sums split-K slabs itself (post_norm_add, post_layer_norm_add): the finished product
     where the weight-streaming kernel is faster than the split grid alone, else possibly a :class:`SplitKPartial`."""
     m, n, k = _sizes(x, w, "linear_into_norm")
-    if use_stream(m, n, k, x, w, defer=True):
+    if m <= STREAM_MAX_M and use_stream(m, n, k, x, w, defer=True):
         return _stream(m, n, k, x, w)
-    return linear(x, w, defer=True)
+    return _linear(m, n, k, x, w, None, True)
 
 
 _STREAM_GLU = {"": 0, "silu": 1, "clipped": 2, "gelu": 3}
@@ -232,9 +232,13 @@ class SplitKPartial:
 
 def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, defer: bool = False):
     """y = x w^T (+bias).  ``defer``: may return a :class:`SplitKPartial` (see there)."""
-    m, n, k = _sizes(x, w, "linear")
+    return _linear(*_sizes(x, w, "linear"), x, w, bias, defer)
+
+
+def _linear(m: int, n: int, k: int, x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], defer: bool):
+    """:func:`linear` of operands whose sizes the caller has compared."""
     kn = knobs.K
-    if not (defer and n % 128 == 0) and use_stream(m, n, k, x, w, bias):
+    if m <= STREAM_MAX_M and not (defer and n % 128 == 0) and use_stream(m, n, k, x, w, bias):
         return _stream(m, n, k, x, w, bias)
     # decode LM head on gemm_pp with nontemporal weights (236 vs 268 us for gemm_sq at M = 256) --
     # unless comm kernels may hold CUs: beside a 4-workgroup, 20 KiB-LDS receive spinning in
@@ -533,7 +537,7 @@ def _linear_glu(x: torch.Tensor, w_gate_up: torch.Tensor, limit: Optional[float]
     reduction (decode): clipped (``limit``) or gelu_tanh (None); None if the shape takes none of them."""
     m, n, k = _sizes(x, w_gate_up, "linear_glu")
     glu = "gelu" if limit is None else "clipped"
-    if n % 2 == 0 and use_stream(m, n, k, x, w_gate_up, bias, glu):
+    if m <= STREAM_MAX_M and n % 2 == 0 and use_stream(m, n, k, x, w_gate_up, bias, glu):
         return _stream(m, n, k, x, w_gate_up, bias, glu, 0.0 if limit is None else limit)
     if x.dtype != torch.bfloat16 or n % 256 or bias is not None:
         return None
@@ -569,7 +573,7 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor) -> Optional[torch.Te
     """silu(x Wg^T) * (x Wu^T) with W = [Wg; Wu] in one launch; None if the shape is not eligible."""
     m, n, k = _sizes(x, w_gate_up, "linear_swiglu")
     kn = knobs.K
-    if n % 16 == 0 and use_stream(m, n, k, x, w_gate_up, glu="silu"):      # (the SiLU kernels' multiples of 8, at any m)
+    if m <= STREAM_MAX_M and n % 16 == 0 and use_stream(m, n, k, x, w_gate_up, glu="silu"):      # (the SiLU kernels' multiples of 8, at any m)
         return _stream(m, n, k, x, w_gate_up, glu="silu")
     if 0 < kn.pp_gate_up_min_m <= m <= 256 and not _comm_cus and _use_pp(m, n, k, x, w_gate_up, 1):
         # decode gate|up on gemm_pp, unsplit, weights nontemporal, on the column tile that gives one

@@ -512,7 +512,7 @@ def linear_clipped_glu(x: torch.Tensor, w_gate_up: torch.Tensor, bias_gu: Option
     """:func:`clipped_glu` of ``x W^T``, W = [Wg; Wu]: in a GEMM epilogue where one takes the shape and the bias, else the
     projection followed by the gate kernel."""
     from . import gemm, linear
-    if bias_gu is not None and (tuple(bias_gu.shape) != (w_gate_up.shape[0],) or bias_gu.dtype != x.dtype
+    if bias_gu is not None and (bias_gu.dim() != 1 or bias_gu.size(0) != w_gate_up.size(0) or bias_gu.dtype != x.dtype
                                 or bias_gu.device != x.device):
         raise ValueError(f"linear_clipped_glu: bias [{w_gate_up.shape[0]}] of x's type and device")
     y = gemm.linear_clipped_glu(x, w_gate_up, limit, bias_gu) if x.is_cuda else None
