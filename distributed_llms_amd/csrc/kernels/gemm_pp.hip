@@ -751,15 +751,16 @@ void gemm_pp_moe(uintptr_t y, uintptr_t x, uintptr_t gather, uintptr_t w, uintpt
 // tile = w + i P by P = gridDim.x workgroups, w the XCD-aware rank (workgroup b runs on XCD b % 8;
 // w = (b % 8) (P / 8) + b / 8), so each XCD's L2 serves 32 consecutive tiles of the grouped order
 // (8 row tiles x 4 column tiles) at a time.
+// Row tile BM = 32 RT (160 .. 256): a K-tile of 64 takes 1.47 / 1.31 / 1.18 / 1.04 us at 256 / 224 / 192 / 160 rows, the sum
+// of its MFMAs and its LDS traffic, so 256 rows are the most efficient and the shorter tiles are for grids that they fit into
+// fewer or cheaper rounds of the chip (ops/gemm.pf_row_tile has the rule and its figures).  Every row's sum over K is in the
+// same order whatever the tile.
+//
 // MODE 0: C bf16 [M, N];  2: SwiGLU C [M, N / 2] with B = [Bg; Bu] (row groups as pp_b_row);  4: the clipped GLU of
 // `limit` (common.h) in the same layout;  5: its gelu GLU.
 // SCH 8: nontemporal output stores (large SwiGLU outputs), else 0.  The schedule sweeps of rounds 3-5
 // (barrier positions, piece spacing, row-group widths, and the split A / B LDS release of round 5,
 // all within 0.5 % of this schedule: profiles/round5_raw/r5d_pf_sched.txt) were removed.
-struct PfSched {
-  int ib1, ib3, ge, gm;
-};
-
 // ---- gemm_pf's dynamic tile queue (DYN).  The grouped tile order is cut into chunks of PF_CH
 // consecutive tiles (8 row tiles x 4 column tiles); chunk c belongs to XCD c % 8, whose workgroups
 // pull its tiles in order from the XCD's head counter (one 128-byte line each) and, when it is
@@ -813,17 +814,13 @@ __device__ void pf_retire(int* q, int grid) {                      // lane 0, on
     __hip_atomic_store(q + 256, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
-// {barrier after set-1 reads (MFMA), barrier before set-0 reads, MFMAs between pieces (0 = spread
-// over the rest of the K-tile), row tiles per group of the tile order}
-constexpr PfSched kPfSched{40, 88, 0, 8};
-
-template <int MODE, int SCH = 0, bool DYN = false>
+template <int MODE, int SCH = 0, bool DYN = false, int RT = 8>
 __global__ void __launch_bounds__(256, 1) gemm_pf_kernel(const bf16* __restrict__ A, const bf16* __restrict__ B,
                                                          bf16* __restrict__ C, int M, int N, int K,
                                                          int* __restrict__ queue, float limit) {
-  constexpr int NW = 4, NWN = 2, BM = 256, BN = 256, TM = 128, TN = BN / NWN;
-  constexpr int RT = TM / 16, CT = TN / 16;            // 8 x 8 accumulators per wave
-  constexpr int SLOT = (BM + BN) * PBK, NB = 2;        // 2 x 64 KiB ring
+  constexpr int NW = 4, NWN = 2, TM = 16 * RT, BM = 2 * TM, BN = 256, TN = BN / NWN;
+  constexpr int CT = TN / 16;                          // RT x 8 accumulators per wave
+  constexpr int SLOT = (BM + BN) * PBK, NB = 2;        // ring of two K-tiles: 2 x 64 KiB at BM = 256
   constexpr int GA = BM * PBK * 2 / 1024 / NW, GB = BN * PBK * 2 / 1024 / NW, G = GA + GB;
   constexpr bool CLIPPED = MODE == 4, GELU = MODE == 5, SWIGLU = MODE == 2 || CLIPPED || GELU;
   constexpr int OUTW = SWIGLU ? BN / 2 : BN;           // output tile width (elements)
@@ -857,7 +854,7 @@ __global__ void __launch_bounds__(256, 1) gemm_pf_kernel(const bf16* __restrict_
     mine = w < tiles ? (tiles - 1 - w) / P + 1 : 0;
     if (mine == 0) return;                             // uniform: before any load or barrier
   }
-  constexpr int GM = kPfSched.gm;                      // row tiles per group of the tile order
+  constexpr int GM = 8;                                // row tiles per group of the tile order
   const int nt = K / PBK, per = GM * ntn;
   auto tile_of = [&](int i) { return DYN ? tq[i & 3] : w + i * P; };   // my i-th tile (grouped order)
   auto tile_mn = [&](int tau, int& m_t, int& n_t) {
@@ -954,10 +951,11 @@ __global__ void __launch_bounds__(256, 1) gemm_pf_kernel(const bf16* __restrict_
   f32x4 acc[RT][CT];
   bf16x8 fa0[RT], fb0[CT], fa1[RT], fb1[CT];
   constexpr int NMF = RT * CT, NR = RT + CT;
-  constexpr PfSched SC = kPfSched;
-  constexpr int IB1 = SC.ib1;
-  constexpr int GE = SC.ge ? SC.ge : ((2 * NMF - 4 - IB1 - 1) / G > 1 ? (2 * NMF - 4 - IB1 - 1) / G : 1);
-  constexpr int IB3 = SC.ib3;
+  // schedule 2's positions (gemm_pp_kernel): barrier after the set-1 reads, pieces spread over the rest of the K-tile,
+  // barrier before the set-0 reads
+  constexpr int IB1 = 2 * NR + 8 < NMF - 1 ? 2 * NR + 8 : NMF - 1;
+  constexpr int GE = (2 * NMF - 4 - IB1 - 1) / G > 1 ? (2 * NMF - 4 - IB1 - 1) / G : 1;
+  constexpr int IB3 = 2 * NMF - 8 - 2 * NR > NMF ? 2 * NMF - 8 - 2 * NR : NMF;
   static_assert(IB1 > 2 * NR - 1 && IB1 < NMF && IB3 >= NMF, "schedule 2 barriers");
   constexpr int PB3 = (IB3 - IB1 - 1) / GE + 1 < G ? (IB3 - IB1 - 1) / GE + 1 : G;
   constexpr int VC = (NB - 2) * G + PB3;
@@ -1118,11 +1116,11 @@ int* pf_queue(hipStream_t s) {
 }  // namespace
 
 // Persistent prefill GEMM: C = A B^T (mode 0) or SwiGLU (mode 1, C [M, N / 2], B = [Bg; Bu]),
-// 256 x 256 tiles, grid = min(tiles, CUs) rounded up to a multiple of 8.  variant bit 16: the
+// bm x 256 tiles, grid = min(tiles, CUs) rounded up to a multiple of 8.  variant bit 16: the
 // dynamic tile queue (DYN; needs K >= 128) instead of the static tile = w + i P walk; variant 8:
 // nontemporal output stores (by default: SwiGLU outputs > 256 MiB).
 void gemm_pf(uintptr_t c, uintptr_t a, uintptr_t b, int M, int N, int K, int mode, int variant, uintptr_t stream,
-             float limit) {
+             float limit, int bm) {
   const bool dyn = (variant & 16) != 0;
   variant &= ~16;
   DLLM_HOST_CHECK(!dyn || K >= 2 * PBK, "the dynamic tile queue needs K >= 128");
@@ -1147,30 +1145,30 @@ void gemm_pf(uintptr_t c, uintptr_t a, uintptr_t b, int M, int N, int K, int mod
     cus = n > 0 ? n : 256;
     if (dev >= 0 && dev < 64) cus_of[dev].store(cus, std::memory_order_relaxed);
   }
-  const long tiles = (long)(N / 256) * ((M + 255) / 256);
+  DLLM_HOST_CHECK(bm == 256 || bm == 224 || bm == 192 || bm == 160, "row tile 160, 192, 224 or 256");
+  DLLM_HOST_CHECK(bm == 256 || (!dyn && variant == 0), "row tiles below 256: static walk, default stores");
+  const long tiles = (long)(N / 256) * ((M + bm - 1) / bm);
   DLLM_HOST_CHECK(tiles < (1L << 30), "tiles");
   const long grid = ((tiles < cus ? tiles : cus) + 7) / 8 * 8;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   int* q = dyn ? pf_queue(s) : nullptr;
-#define DLLM_PF_GO(MODE_, SCH_, DYN_)                                                                         \
-  hipLaunchKernelGGL((gemm_pf_kernel<MODE_, SCH_, DYN_>), dim3((unsigned)grid), dim3(256), 0, s, (const bf16*)a, \
+#define DLLM_PF_GO(MODE_, SCH_, DYN_, RT_)                                                                         \
+  hipLaunchKernelGGL((gemm_pf_kernel<MODE_, SCH_, DYN_, RT_>), dim3((unsigned)grid), dim3(256), 0, s, (const bf16*)a, \
                      (const bf16*)b, (bf16*)c, M, N, K, q, limit)
-  const bool nt_store = variant == 8 || (mode != 0 && (long)M * (N / 2) * 2 > (256L << 20));
-  if (mode == 4) {
-    if (dyn) { if (nt_store) DLLM_PF_GO(5, 8, true); else DLLM_PF_GO(5, 0, true); }
-    else { if (nt_store) DLLM_PF_GO(5, 8, false); else DLLM_PF_GO(5, 0, false); }
-  } else
-  if (mode == 3) {
-    if (dyn) { if (nt_store) DLLM_PF_GO(4, 8, true); else DLLM_PF_GO(4, 0, true); }
-    else { if (nt_store) DLLM_PF_GO(4, 8, false); else DLLM_PF_GO(4, 0, false); }
-  } else
-  if (mode == 1) {
-    if (dyn) { if (nt_store) DLLM_PF_GO(2, 8, true); else DLLM_PF_GO(2, 0, true); }
-    else { if (nt_store) DLLM_PF_GO(2, 8, false); else DLLM_PF_GO(2, 0, false); }
-  } else {
-    if (dyn) { if (nt_store) DLLM_PF_GO(0, 8, true); else DLLM_PF_GO(0, 0, true); }
-    else { if (nt_store) DLLM_PF_GO(0, 8, false); else DLLM_PF_GO(0, 0, false); }
-  }
+#define DLLM_PF_MODE(MODE_)                                                                              \
+  do {                                                                                                   \
+    if (dyn) { if (nt_store) DLLM_PF_GO(MODE_, 8, true, 8); else DLLM_PF_GO(MODE_, 0, true, 8); }        \
+    else if (bm == 224) DLLM_PF_GO(MODE_, 0, false, 7);                                                  \
+    else if (bm == 192) DLLM_PF_GO(MODE_, 0, false, 6);                                                  \
+    else if (bm == 160) DLLM_PF_GO(MODE_, 0, false, 5);                                                  \
+    else { if (nt_store) DLLM_PF_GO(MODE_, 8, false, 8); else DLLM_PF_GO(MODE_, 0, false, 8); }          \
+  } while (0)
+  const bool nt_store = variant == 8 || (bm == 256 && mode != 0 && (long)M * (N / 2) * 2 > (256L << 20));
+  if (mode == 4) DLLM_PF_MODE(5);
+  else if (mode == 3) DLLM_PF_MODE(4);
+  else if (mode == 1) DLLM_PF_MODE(2);
+  else DLLM_PF_MODE(0);
+#undef DLLM_PF_MODE
 #undef DLLM_PF_GO
   DLLM_HIP_CHECK(hipGetLastError());
 }

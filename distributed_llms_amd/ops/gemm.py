@@ -84,6 +84,42 @@ def pf_fills(m: int, n: int, device) -> bool:
     return rounds >= 4 or tiles / (rounds * cus) >= knobs.K.pf_min_eff
 
 
+# Relative time of a round of gemm_pf's workgroups, by row tile.  A shorter tile does less per byte staged and per LDS read, so
+# it pays only where it saves most of a round: 152 unsplit sizes (7 pairs of N 2560 .. 57344 and K 2560 .. 28672, M 264 ..
+# 8192), each with every row tile, are within 0.3 % of the best tile in the mean under this rule, 5-6 % faster than 256 rows.
+# us, 256 / 224 / 192 / 160 rows: 2560 x 2560, M = 7021 (280 / 320 / 370 / 440 tiles) 108 / 99 / 95 / 84; 4096 x 4096, 6210
+# (400 / 448 / 528 / 624) 183 / 165 / 204 / 187; 6144 x 4096, 3072 (288 / 336 / 384 / 480) 172 / 153 / 146 / 136; 4096 x 14336,
+# 5120 (320 / 368 / 432 / 512) 584 / 554 / 522 / 493; gate|up 28672 x 4096, 384 (224 / 224 / 224 / 336) 97 / 87 / 83 / 140.
+# 128 rows (1.0 us a K-tile against 1.04 for 160) never win where there is no K split.
+_PF_ROUND = {256: 1.0, 224: 0.93, 192: 0.84, 160: 0.76}
+
+
+def pf_row_tile(m: int, n: int, device) -> int:
+    """Row tile with the shortest walk: rounds of the chip times the time of a round.  A single round of 256 rows is
+    gemm_pp's (its epilogue through LDS is 5-7 % faster where no next tile hides the stores), which 224 rows do not beat."""
+    cus = _cus(device)
+    best, at = 256, None
+    for bm, c in _PF_ROUND.items():
+        rounds = -(-(-(-m // bm) * (n // 256)) // cus)
+        t = rounds * (_PF_ROUND[224] if bm == 256 and rounds == 1 else c)
+        if at is None or t < at - 1e-6:
+            best, at = bm, t
+    return best
+
+
+def _pf_plan(m: int, n: int, k: int, out: int, device) -> int:
+    """gemm_pf's row tile for an [m, k] x [n, k]^T product that no decode kernel takes (``out``: output columns), or 0 where
+    gemm_pp serves.  Below 256 rows only where gemm_pp would not split K either -- the sums' order stays the same -- and
+    nothing asks for the dynamic tile queue or nontemporal stores."""
+    if not knobs.K.pp_persistent or m * out * 2 >= 1 << 31:
+        return 0
+    if pp_splits(m, n, k) == 1 and not _comm_cus and not pf_dynamic() and (out == n or m * out * 2 <= 256 << 20):
+        bm = pf_row_tile(m, n, device)
+        if bm != 256:
+            return bm
+    return 256 if pf_fills(m, n, device) else 0
+
+
 def _use_wide(m: int, n: int, k: int, x: torch.Tensor, w: torch.Tensor, swiglu: bool = False) -> bool:
     kn = knobs.K
     roles = {t for t in kn.wide.split(",") if t and t != "none"}
@@ -256,8 +292,9 @@ def _linear(m: int, n: int, k: int, x: torch.Tensor, w: torch.Tensor, bias: Opti
     if bias is None and _use_wide(m, n, k, x, w):
         return linear_wide(x, w, defer=defer)
     if bias is None and _use_pp(m, n, k, x, w, knobs.K.pp_proj_min_m):
-        if kn.pp_persistent and m * n * 2 < (1 << 31) and pf_fills(m, n, x.device):
-            return linear_pf(x, w)
+        bm = _pf_plan(m, n, k, n, x.device)
+        if bm:
+            return linear_pf(x, w, bm=bm)
         # medium M (mixed prefill + decode steps, short prompts): split-K tiles fill the CUs
         return linear_pp(x, w, variant=PP_PREFILL_VARIANT, defer=defer)
     return F.linear(x, w, bias)
@@ -441,12 +478,12 @@ def linear_pp(x: torch.Tensor, w: torch.Tensor, splits: int = 0, swiglu: bool = 
 
 
 def linear_pf(x: torch.Tensor, w: torch.Tensor, swiglu: bool = False, variant: int = 0,
-              limit: Optional[float] = None, gelu: bool = False) -> torch.Tensor:
-    """Persistent prefill GEMM (gemm_pf in csrc/kernels/gemm_pp.hip): schedule 2's 256 x 256 tiles,
+              limit: Optional[float] = None, gelu: bool = False, bm: int = 256) -> torch.Tensor:
+    """Persistent prefill GEMM (gemm_pf in csrc/kernels/gemm_pp.hip): schedule 2's ``bm`` x 256 tiles,
     one workgroup per CU walking its tiles with the LDS-DMA pipeline running across tile
     boundaries; optional fused SwiGLU (``w`` = [Wg; Wu], y [M, N / 2]) or -- ``limit`` -- clipped GLU or -- ``gelu`` --
     gelu_tanh GLU.  ``variant`` 8: nontemporal
-    output stores (the default for SwiGLU outputs > 256 MiB); the tiles come from per-XCD device
+    output stores (the default for SwiGLU outputs > 256 MiB); ``bm``: the row tile (pf_row_tile); the tiles come from per-XCD device
     queues while knobs.pf_dynamic says so (bit 16 of the launcher's variant)."""
     k = x.shape[-1]
     n = w.shape[0]
@@ -457,7 +494,7 @@ def linear_pf(x: torch.Tensor, w: torch.Tensor, swiglu: bool = False, variant: i
         raise ValueError("linear_pf: N % 256 and K % 64")
     glu = swiglu or gelu or limit is not None
     y = torch.empty(*x.shape[:-1], n // 2 if glu else n, dtype=x.dtype, device=x.device)
-    dyn = pf_dynamic() and k >= 128
+    dyn = pf_dynamic() and k >= 128 and bm == 256
     if torch.cuda.is_current_stream_capturing():
         # inside a graph: the static tile walk.  A tile queue is per stream and self-resetting, but
         # a replay may run on another stream beside eager launches that use the same queue
@@ -466,7 +503,7 @@ def linear_pf(x: torch.Tensor, w: torch.Tensor, swiglu: bool = False, variant: i
         variant |= 16                  # per-XCD dynamic tile queues (gemm_pp.hip, DYN)
     _ext.kernels().gemm_pf(y.data_ptr(), x.data_ptr(), w.data_ptr(), m, n, k,
                            4 if gelu else 3 if limit is not None else (1 if swiglu else 0), variant, torch.cuda.current_stream().cuda_stream,
-                           0.0 if limit is None else float(limit))
+                           0.0 if limit is None else float(limit), bm)
     return y
 
 
@@ -541,9 +578,10 @@ def _linear_glu(x: torch.Tensor, w_gate_up: torch.Tensor, limit: Optional[float]
         return _stream(m, n, k, x, w_gate_up, bias, glu, 0.0 if limit is None else limit)
     if x.dtype != torch.bfloat16 or n % 256 or bias is not None:
         return None
-    if not _use_wide(m, n, k, x, w_gate_up) and _use_pp(m, n, k, x, w_gate_up, knobs.K.pp_swiglu_min_m) \
-            and knobs.K.pp_persistent and m * (n // 2) * 2 < (1 << 31) and pf_fills(m, n, x.device):
-        return linear_pf(x, w_gate_up, limit=limit, gelu=limit is None)
+    if not _use_wide(m, n, k, x, w_gate_up) and _use_pp(m, n, k, x, w_gate_up, knobs.K.pp_swiglu_min_m):
+        bm = _pf_plan(m, n, k, n // 2, x.device)
+        if bm:
+            return linear_pf(x, w_gate_up, limit=limit, gelu=limit is None, bm=bm)
     y = linear(x, w_gate_up, defer=True)
     if isinstance(y, SplitKPartial):
         out = torch.empty(*x.shape[:-1], n // 2, dtype=x.dtype, device=x.device)
@@ -587,7 +625,8 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor) -> Optional[torch.Te
     if _use_wide(m, n, k, x, w_gate_up, swiglu=True):
         return linear_wide(x, w_gate_up, swiglu=True)
     if _use_pp(m, n, k, x, w_gate_up, knobs.K.pp_swiglu_min_m):
-        if knobs.K.pp_persistent and m * (n // 2) * 2 < (1 << 31) and pf_fills(m, n, x.device):
-            return linear_pf(x, w_gate_up, swiglu=True)
+        bm = _pf_plan(m, n, k, n // 2, x.device)
+        if bm:
+            return linear_pf(x, w_gate_up, swiglu=True, bm=bm)
         return linear_pp(x, w_gate_up, swiglu=True, variant=PP_PREFILL_VARIANT)
     return None

@@ -355,6 +355,18 @@ def test_pf_matches_pp_schedule2_bit_exact(cuda):
     assert torch.equal(gemm.linear_pf(x, w), gemm.linear_pp(x, w, splits=1, variant=gemm.PP_PREFILL_VARIANT))
 
 
+@pytest.mark.parametrize("bm", [160, 192, 224])
+@pytest.mark.parametrize("m", [1, 161, 447, 1921, 4500])
+@pytest.mark.parametrize("n,k", [(256, 64), (512, 192), (4096, 128)])
+def test_pf_row_tiles_bit_exact(cuda, bm, m, n, k):
+    """Row tiles below 256 (row tails, one K-tile, one and several tiles per workgroup): every sum in the order of the
+    256-row tile, so the same bits, in the plain form and in each GLU."""
+    torch.manual_seed(bm + m + n)
+    x, w = _bf(m, k), _bf(n, k, scale=0.1)
+    for kw in ({}, {"swiglu": True}, {"limit": 0.7}, {"gelu": True}):
+        assert torch.equal(gemm.linear_pf(x, w, bm=bm, **kw), gemm.linear_pf(x, w, **kw)), kw
+
+
 def test_pf_swiglu_output_range_is_the_half_width(cuda):
     """SwiGLU's output is [M, N / 2]: a 70B prefill gate|up (M 32768, 2I 57344) is within the
     kernel's 2 GiB output range although M x 2I x 2 bytes is not (a small-K stand-in shape)."""

@@ -310,3 +310,25 @@ def test_wide_variant_by_weight_and_tile():
     assert gemm.wide_variant(180, *down, 1, 192) == gemm.wide_variant(1, *small, 1, 64) == knobs.K.wide_variant
     assert gemm.wide_variant(256, *down, 8, 256) == gemm.wide_variant(64, *o, 8, 64) == knobs.K.wide_variant_split
     assert gemm.wide_variant(180, *down, 8, 192) == gemm.wide_variant(1, *small, 4, 64) == gemm.wide_variant(65, *o, 8, 128) == 1
+
+
+def test_pf_row_tile_takes_the_cheapest_walk():
+    """The row tile by rounds of the chip: shorter tiles only where they save most of a round, never in front of a K split,
+    the dynamic queue or reserved CUs, and never for a single round that gemm_pp runs as fast."""
+    cpu = torch.device("cpu")
+    assert gemm.pf_row_tile(8192, 4096, cpu) == 256        # 512 tiles: two full rounds
+    assert gemm.pf_row_tile(7021, 2560, cpu) == 160        # 280 tiles of 256 rows: a second round for 24
+    assert gemm.pf_row_tile(6210, 4096, cpu) == 224        # 448 instead of 400 tiles, both two rounds
+    assert gemm.pf_row_tile(448, 28672, cpu) == 256        # one round either way
+    assert gemm._pf_plan(2048, 4096, 4096, 4096, cpu) == 0         # 128 tiles: gemm_pp splits K
+    assert gemm._pf_plan(320, 28672, 4096, 14336, cpu) == 160
+    for m in range(257, 3000, 61):
+        for n in (2560, 4096, 6144, 28672):
+            bm = gemm._pf_plan(m, n, 4096, n, cpu)
+            assert bm in (0, 160, 192, 224, 256)
+            assert bm in (0, 256) or gemm.pp_splits(m, n, 4096) == 1
+    gemm.reserve_cus_for_comm(16)
+    try:
+        assert gemm._pf_plan(7021, 2560, 2560, 2560, cpu) in (0, 256)
+    finally:
+        gemm.release_cus_for_comm()
