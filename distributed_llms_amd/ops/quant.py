@@ -202,9 +202,17 @@ def linear_ref(x, w: Fp8Weight, swiglu: bool = False) -> torch.Tensor:
 
 def fp8_plan(m: int, n: int, k: int, swiglu: bool = False) -> Tuple[int, int]:
     """(K slices, row-tile override or 0) of gemm_wide_fp8 for this shape.  Default: the bf16
-    kernel's rule on the 128-K tiles (a K-tile of fp8 holds the bytes of a 64-K bf16 tile)."""
-    from .gemm import wide_splits
-    s = wide_splits(m, n, k // 2, swiglu)
+    kernel's rule on the 128-K tiles (a K-tile of fp8 holds the bytes of a 64-K bf16 tile); up to 64 rows a split narrow
+    product takes up to 8 slices -- what the reduction loads in one go -- of 4 K-tiles where that is twice as many.  us with
+    the norm behind it, M = 1 / 16 / 64, former -> this: 1024 x 4096 8.9 / 10.0 / 10.4 -> 7.6 / 8.6 / 9.1, 2048 x 2048 9.0 /
+    10.0 / 10.4 -> 7.6 / 8.6 / 9.0 (4 slices), 4096 x 4096 10.0 / 10.8 / 11.5 -> 9.0 / 10.1 / 11.3; 16 slices 10-14, and
+    6144 x 4096 in 5 instead of 4 10.9 / 11.9 / 12.9 -> 11.2 / 12.3 / 13.6."""
+    from . import gemm
+    s = gemm.wide_splits(m, n, k // 2, swiglu)
+    if m <= 64 and not swiglu and s > 1 and not gemm._comm_cus:
+        c = min(8, 256 // (n // 128), (k // 128) // 4)
+        if c >= 2 * s:
+            s = c
     if knobs.K.fp8_bm128 and not swiglu and s > 1 and 128 < m <= 256:
         tiles = (n // 128) * 2
         return max(1, min(256 // tiles, (k // 128) // 4, 16)), 128

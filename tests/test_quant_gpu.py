@@ -70,6 +70,19 @@ def test_fp8_deferred_split_feeds_the_fused_norm():
     torch.testing.assert_close(y.float(), ry.float(), rtol=3e-2, atol=3e-2)
 
 
+@pytest.mark.parametrize("m", [1, 64, 65, 128])
+@pytest.mark.parametrize("n,k,splits", [(1024, 128 * 96, 12), (1024, 128 * 100, 7), (1024, 128 * 104, 16), (4096, 4096, 8),
+                                        (2048, 512, 1), (2048, 1024, 1)])
+def test_fp8_weight_ring_and_policy(m, n, k, splits):
+    """Deep rings and nontemporal weights: slices around the 8, 12 and 14 K-tiles where they set in, a last slice that is
+    shorter or empty, unsplit grids with fewer K-tiles than ring slots.  The sums are f32 of exact products and a split's
+    slabs f16: the same bound as the plain product's test."""
+    w = quant.quantize_weight((torch.randn(n, k) * 0.02).to(DEV))
+    x = _x(m, k, seed=m + k)
+    y = quant.linear_fp8(x, w, splits=splits).float()
+    torch.testing.assert_close(y, _oracle(x, w).to(DEV).to(torch.bfloat16).float(), rtol=2e-2, atol=2e-2)
+
+
 def test_fp8_error_vs_bf16_weights_is_quantization_sized():
     """The W8A8 product against the unquantized bf16 one: a few percent relative error (e4m3
     has 3 mantissa bits), not a layout error."""
