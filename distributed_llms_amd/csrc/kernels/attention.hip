@@ -142,13 +142,13 @@ __device__ __forceinline__ void init_state(WaveState<D>& st) {
 }
 
 // ---------------------------------------------------------------------------
-// Decode: grid (num_splits, Hkv / WPB, B), WPB waves per workgroup, ONE wave per
-// (split, kv-head, sequence).  The wave walks its split's chunks with a depth-2 software
+// Decode: grid (num_splits, Hkv, B), ONE wave per (split, kv-head, sequence) -- JOIN: grid (1, Hkv, B) and a
+// sequence's splits as the waves of one workgroup.  The wave walks its split's chunks with a depth-2 software
 // pipeline -- chunk c+1's K/V loads are in flight while chunk c's MFMAs and softmax run --
 // and the chunk -> block ids come from one lane-parallel load of the block-table row
 // (read back with readlane), so the only dependent HBM latency per chunk is the KV
 // stream itself.  No LDS, no barrier.  num_splits > 1 writes (o, m, l) partials for the
-// split-reduce kernel below.  (The first version used 4 waves per (split, head, seq) with
+// split-reduce kernel below, or (JOIN) to LDS, where the workgroup sums them.  (The first version used 4 waves per (split, head, seq) with
 // chunks round-robin, no cross-chunk prefetch and an LDS combine: 47 us per layer at
 // B=256 / ctx 128-256 on Llama-3-8B, profiles/llama3_8b_b256_kernels_auto.md.)
 // ---------------------------------------------------------------------------
@@ -237,16 +237,17 @@ __device__ __forceinline__ void rope_rotate(bf16x8 (&f)[D / 32], const RopeRow<D
   }
 }
 
-template <int D, int WPB, bool FUSED, int PARTS = 0>
-__global__ void __launch_bounds__(WPB * 64, 2) attn_decode_kernel(   // 2nd arg: min waves per SIMD
+template <int D, bool FUSED, int PARTS = 0, bool JOIN = false>
+__global__ void __launch_bounds__(JOIN ? 512 : 64, 2) attn_decode_kernel(   // 2nd arg: min waves per SIMD
     bf16* __restrict__ out, const bf16* __restrict__ q, bf16* __restrict__ k_cache,
     bf16* __restrict__ v_cache, const int32_t* __restrict__ block_tables,
     const int32_t* __restrict__ seq_lens, float* __restrict__ part_o, float* __restrict__ part_ml,
     int hq, int hkv, int max_blocks, int split_len, float scale_log2, RopeArgs ra) {
-  const int split = blockIdx.x, b = blockIdx.z;
+  extern __shared__ __attribute__((aligned(16))) float join_lds[];   // JOIN: [split][head][D + 4], then [split][head](m, l)
+  const int kvh = blockIdx.y, b = blockIdx.z;
   const int lane = threadIdx.x & 63;
-  const int kvh = blockIdx.y * WPB + (threadIdx.x >> 6);
-  const int nsplit = gridDim.x;
+  const int split = JOIN ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : (int)blockIdx.x;
+  const int nsplit = JOIN ? (int)(blockDim.x >> 6) : (int)gridDim.x;
   const int G = hq / hkv;
   const int r = lane & 15, g = lane >> 4;
   // Two round trips to memory precede the first MFMA: the sequence's position, its context length, this split's first 64
@@ -282,6 +283,38 @@ __global__ void __launch_bounds__(WPB * 64, 2) attn_decode_kernel(   // 2nd arg:
     load_chunk<D, true>(c, k_cache + base, v_cache + base, lane);
   };
   auto write_out = [&](const WaveState<D>& st, float lt) {
+    if constexpr (JOIN) {
+      // the splits meet in LDS and are summed as attn_split_reduce_kernel sums them: the same operations in the same order
+      float2* ml = reinterpret_cast<float2*>(join_lds + nsplit * G * (D + 4));
+      if (col_ok) {
+        float* po = join_lds + (split * G + r) * (D + 4);
+#pragma unroll
+        for (int dt = 0; dt < D / 16; ++dt) *reinterpret_cast<f32x4*>(po + dt * 16 + 4 * g) = st.acc[dt];
+        if (g == 0) ml[split * G + r] = make_float2(st.m, lt);
+      }
+      __syncthreads();
+      for (int i = threadIdx.x; i < G * (D / 4); i += blockDim.x) {
+        const int h = i / (D / 4), e = 4 * (i % (D / 4));
+        float M = -INFINITY;
+        for (int t = 0; t < nsplit; ++t) M = fmaxf(M, ml[t * G + h].x);
+        const float mref = M == -INFINITY ? 0.f : M;
+        f32x4 num = {0.f, 0.f, 0.f, 0.f};
+        float den = 0.f;
+        for (int t = 0; t < nsplit; ++t) {
+          const float2 x = ml[t * G + h];
+          const f32x4 o = *reinterpret_cast<const f32x4*>(join_lds + (t * G + h) * (D + 4) + e);
+          const float f = exp2f(x.x - mref);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) num[j] = fmaf(o[j], f, num[j]);
+          den = fmaf(x.y, f, den);
+        }
+        bf16x4 o;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[j] = f2bf(den > 0.f ? num[j] / den : 0.f);
+        *reinterpret_cast<bf16x4*>(out + ((size_t)b * hq + kvh * G + h) * D + e) = o;
+      }
+      return;
+    }
     if (!col_ok) return;
     const int h = kvh * G + r;
     if (nsplit == 1) {
@@ -309,7 +342,7 @@ __global__ void __launch_bounds__(WPB * 64, 2) attn_decode_kernel(   // 2nd arg:
   WaveState<D> st;
   init_state(st);
   if (c1 == c0) {                                   // wave-uniform: no key in this split (and not the new one)
-    write_out(st, 0.f);
+    write_out(st, 0.f);                             // (JOIN: where this wave meets the others at the barrier)
     return;
   }
   const int blk_0 = __builtin_amdgcn_readlane(blk_first, 0);
@@ -1576,19 +1609,29 @@ static void decode_launch(uintptr_t out, uintptr_t q, uintptr_t k_cache, uintptr
   if (batch == 0) return;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const float sl2 = scale * 1.4426950408889634f;
-  // one wave per kv head; pack up to 4 heads (independent waves) per workgroup
-  const int wpb = hkv % 4 == 0 ? 4 : hkv % 2 == 0 ? 2 : 1;
-  dim3 grid(num_splits, hkv / wpb, batch);
-  auto go = [&](auto kern, int threads) {
-    hipLaunchKernelGGL(kern, grid, dim3(threads), 0, s, (bf16*)out, (const bf16*)q, (bf16*)k_cache, (bf16*)v_cache,
+  // One wave per workgroup: waves that share a CU share its ~64 outstanding cache lines, and a small batch has a CU for
+  // every wave (four heads per workgroup, 32 / 8 heads of 128, us, 4 -> 1 wave a workgroup: 1 sequence of 60 / 500 keys 8.5
+  // -> 6.2 / 11.3 -> 8.0, 8 of 250 11.9 -> 8.8, 192 of 250 46.3 -> 40.0; 256 of 120 the same 31).
+  // The splits of a (sequence, head) as the waves of ONE workgroup (JOIN) save the partials' round trip and the second
+  // launch, some 2 us, and pay 0.6 us per 32 keys of 128 (16 KiB) of every wave that a CU gets on top of an even share: us,
+  // apart -> joined, 16 / 32 / 64 sequences of 120 keys in 2 splits 8.8 / 10.7 / 13.8 -> 8.1 / 8.1 / 10.5, 32 of 1000 in 4 28.4
+  // -> 26.2; not 1 of 250 in 4 (8.0, joined 9.7), 16 of 500 in 8 (14.8, 16.5) or 32 of 1000 keys of 64, 12 heads, in 2
+  // (22.3, 25.0: 384 workgroups of two waves on 256 CUs).
+  const int pairs = batch * hkv;
+  const int surplus = num_splits * ((pairs + 255) / 256) - (num_splits * pairs + 255) / 256;
+  const long join_bytes = (long)num_splits * (hq / hkv) * (d + 6) * 4;
+  const bool join = num_splits > 1 && num_splits <= 8 && join_bytes <= 64 * 1024 &&
+                    (long)surplus * split_len * d < 14000;
+  const dim3 grid(join ? 1 : num_splits, hkv, batch);
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, grid, dim3(join ? num_splits * 64 : 64), join ? join_bytes : 0, s, (bf16*)out, (const bf16*)q, (bf16*)k_cache, (bf16*)v_cache,
                        (const int32_t*)block_tables, (const int32_t*)seq_lens, (float*)part_o, (float*)part_ml, hq,
                        hkv, max_blocks, split_len, sl2, ra);
   };
 #define DLLM_DEC(DD, FF, PP)                                          \
   do {                                                                \
-    if (wpb == 4) go(attn_decode_kernel<DD, 4, FF, PP>, 256);         \
-    else if (wpb == 2) go(attn_decode_kernel<DD, 2, FF, PP>, 128);    \
-    else go(attn_decode_kernel<DD, 1, FF, PP>, 64);                   \
+    if (join) go(attn_decode_kernel<DD, FF, PP, true>);               \
+    else go(attn_decode_kernel<DD, FF, PP>);                          \
   } while (0)
   const bool parts = fused && ra.part != nullptr;
   if (d == 128) {
@@ -1604,7 +1647,7 @@ static void decode_launch(uintptr_t out, uintptr_t q, uintptr_t k_cache, uintptr
   }
 #undef DLLM_DEC
   DLLM_HIP_CHECK(hipGetLastError());
-  if (num_splits > 1) {
+  if (num_splits > 1 && !join) {
     // the round that covers the splits with the fewest repeated loads (16 of them for 2 splits: 64 sequences of 64 heads
     // 3 us slower)
     auto reduce = [&](auto kern) {

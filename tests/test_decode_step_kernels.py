@@ -351,3 +351,39 @@ def test_window_decode_head_sizes(cuda, d, dv, biased):
         want = (torch.softmax(s, 0)[..., None] * v).sum(0)
         # scores: d exact products, 2^-24 of their magnitudes (below 2^-15 in all); weights kept to 17 bits; the result in 8
         assert ((out[i].double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -13 * v.abs().max()).all()
+
+
+@gpu
+@pytest.mark.parametrize("b,hq,hkv,d,ctx", [(2, 4, 1, 128, 128), (3, 16, 1, 128, 100), (5, 2, 2, 64, 250), (64, 16, 4, 128, 129),
+                                            (70, 32, 4, 64, 200), (16, 32, 2, 64, 256), (1, 1, 1, 64, 65)])
+@pytest.mark.parametrize("fused", [False, True])
+def test_decode_attention_joins_splits_in_a_workgroup(cuda, b, hq, hkv, d, ctx, fused):
+    """2 to 4 splits summed in one workgroup: groups of 1 to 16 heads, sequences that leave the last splits (or all but the
+    first) empty, an even and an uneven share of workgroups per CU; against float32."""
+    torch.manual_seed(b + ctx)
+    lens = [max(1, ctx - 37 * (i % 7)) if i else ctx for i in range(b)]
+    width = 1 << (-(-ctx // 32) - 1).bit_length()
+    splits, split_len = ops.decode_split_plan(b, hkv, ctx, 32, width)
+    surplus = splits * -(-b * hkv // 256) - -(-splits * b * hkv // 256)
+    assert 2 <= splits <= 4 and surplus * split_len * d < 14000           # the launcher's rule
+    used = sum(-(-n // 32) for n in lens)
+    k = torch.randn(used, hkv, 32, d).bfloat16().cuda()
+    v = torch.randn(used, hkv, d, 32).bfloat16().cuda()
+    bt, at = torch.zeros(b, width, dtype=torch.int32), 0
+    for i, n in enumerate(lens):
+        bt[i, :-(-n // 32)] = torch.arange(at, at + -(-n // 32))
+        at += -(-n // 32)
+    slots = torch.tensor([int(bt[i, (n - 1) // 32]) * 32 + (n - 1) % 32 for i, n in enumerate(lens)], dtype=torch.int32).cuda()
+    bt, sl = bt.cuda(), torch.tensor(lens, dtype=torch.int32).cuda()
+    kf, vf = k.float(), v.float()
+    if fused:
+        qkv = torch.randn(b, (hq + 2 * hkv) * d).bfloat16().cuda()
+        cs = ref.rope_cos_sin(d, 4096, 500000.0, device="cuda")
+        q = ref.rope_cache_append(qkv.float(), sl - 1, cs, kf, vf, slots, hq, hkv, d).bfloat16()
+        out = ops.paged_attention_decode_rope(qkv, sl - 1, cs, k, v, slots, bt, sl, hq, hkv, d, d ** -0.5, max_ctx=ctx)
+    else:
+        q = torch.randn(b, hq, d).bfloat16().cuda()
+        out = ops.paged_attention_decode(q, k, v, bt, sl, d ** -0.5, max_ctx=ctx)
+    expect = ref.paged_attention_decode(q.float(), kf.bfloat16().float(), vf, bt, sl, d ** -0.5)
+    # as above: bf16 probabilities and result, and as much again for a rotated element that rounds the other way
+    assert (out.float() - expect).abs().max() <= 2.0 ** -7 * vf.abs().max()
