@@ -6,7 +6,7 @@
 // (a slab sum, a gate kernel) costs 2-4 us: the end of one kernel to the start of the next inside a graph, plus its first
 // load's round trip.  Where it is the faster route: ops/gemm.stream_fits.
 //
-//  * one workgroup owns RT x 16 weight rows and all of K, so nothing is left to sum in memory; its waves take the
+//  * one workgroup owns 8 RG weight rows (stream_rows) and all of K, so nothing is left to sum in memory; its waves take the
 //    64-deep K-tiles in turn (wave v: tiles v, v + WAVES, ...), so that together they read 512-byte or 1 KiB runs of
 //    every row;
 //  * a wave stages its tiles -- weights and x -- through an LDS ring of its OWN (two slots, global_load_lds_dwordx4 in
@@ -16,9 +16,9 @@
 //    against 5.9 / 7.4 / 9.7);
 //  * the waves' sums meet in LDS (wave 0 first: the same result on every run), behind the only two barriers.
 // Measured, cold weights, M = 1 / 16 / 32 / 64, us (wide: gemm_wide's K split, without the reduction behind it):
-//   1024 x 1024  3.0 / 3.4 / 4.0 / 5.1 (wide 5.0 / 5.4 / 5.5 / 5.6)    2560 x 2560  4.7 / 5.9 / 7.4 / 9.7 (6.7 / 7.2 / 7.7 / 8.2)
-//   5120 x 2560  7.0 / 8.2 / 9.7 / 12.5 (7.9 / 8.5 / 9.0 / 9.6)        15360 x 2560 + GLU  14.2 / 14.7 / 16.2 / 19.7 (15.8 / 16.5 / 17.5 / 18.5)
-//   4096 x 4096  7.7 / 8.6 / 10.0 / 13.2 (7.8 / 8.1 / 8.5 / 8.9)       2560 x 7680  9.1 / 12.8 / 16.6 / 22.4 (9.3 / 9.6 / 10.1 / 10.6)
+//   1024 x 1024  3.0 / 3.5 / 4.0 / 5.1 (wide 5.0 / 5.4 / 5.5 / 5.6)    2560 x 2560  4.6 / 5.8 / 7.4 / 9.7 (6.7 / 7.2 / 7.7 / 8.2)
+//   5120 x 2560  7.0 / 7.5 / 9.7 / 12.5 (7.9 / 8.5 / 9.0 / 9.6)        15360 x 2560 + GLU  14.6 / 14.8 / 16.2 / 19.7 (15.8 / 16.5 / 17.5 / 18.5)
+//   4096 x 4096  7.6 / 8.6 / 10.0 / 13.2 (7.8 / 8.1 / 8.5 / 8.9)       6144 x 4096  10.4 / 10.1 (10.7 / 11.0)
 // bound by the weight bytes and the launch below 16 rows, by staging x once per workgroup above.
 #include "common.h"
 #include "launchers.h"
@@ -35,39 +35,39 @@ __device__ __forceinline__ int sswz(int row, int chunk) { return chunk ^ ((row >
 }  // namespace
 
 // GLU 0: y [M, N] (+ bias [N]);  1 / 2 / 3: SiLU / clipped (`limit`) / gelu GLU, w = [gate; up], y [M, N / 2], bias
-// gate | up.  GLU tiles hold RT / 2 16-row tiles of gate rows, then the same output columns' up rows.
-template <int RT, int MT, int GLU, bool NT, int WAVES>
+// gate | up.  A workgroup's RG groups of 8 weight rows are its output columns, under a GLU CW gate rows and then the same
+// columns' up rows; XG groups of 8 rows of x.  An odd last group fills half an MFMA tile, its other half repeats it.
+template <int RG, int XG, int GLU, bool NT, int WAVES>
 __global__ void __launch_bounds__(WAVES * 64) gemm_stream_kernel(bf16* __restrict__ Y, const bf16* __restrict__ X,
                                                                  const bf16* __restrict__ W,
                                                                  const bf16* __restrict__ bias, int M, int N, int K,
                                                                  float limit) {
-  static_assert(GLU == 0 || RT % 2 == 0, "gate and up tiles come in pairs");
-  constexpr int SLOT = (RT + MT) * 16 * SK;                     // bf16 elements of one ring slot: weights, then x
-  constexpr int G = 2 * (RT + MT);                              // loads per K-tile
+  static_assert(GLU == 0 || RG % 2 == 0 || RG == 3, "a GLU's CW is a multiple of 4");
+  constexpr int RT = (RG + 1) / 2, MT = (XG + 1) / 2;
+  constexpr int SLOT = (RG + XG) * 8 * SK;                      // bf16 elements of one ring slot: weights, then x
+  constexpr int G = RG + XG;                                    // loads per K-tile
   constexpr int RING = WAVES * D * SLOT * 2, RED = WAVES * RT * MT * 1024;
   static_assert(G <= 63, "vmcnt");
   __shared__ __attribute__((aligned(16))) char smem[RING > RED ? RING : RED];
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int fr = lane & 15, fq = lane >> 4;
   const int half = N / 2, ncols = GLU ? half : N;
-  constexpr int CT = GLU ? RT / 2 : RT;                         // 16-column tiles of the output
-  const int c0 = blockIdx.x * (CT * 16);
+  constexpr int CW = GLU ? RG * 4 : RG * 8;                     // output columns
+  const int c0 = blockIdx.x * CW;
   bf16* ring = reinterpret_cast<bf16*>(smem) + wv * (D * SLOT);
 
-  // weight row of tile row r (0..15) of 16-row tile t; rows past the matrix repeat its last row
-  auto wrow = [&](int t, int r) {
-    const int c = min(c0 + (t % CT) * 16 + r, ncols - 1);
-    return GLU && t >= CT ? half + c : c;
+  // weight row of row r of the workgroup; rows past the matrix repeat its last row
+  auto wrow = [&](int r) {
+    const bool up = GLU && r >= CW;
+    return (up ? half : 0) + min(c0 + (up ? r - CW : r), ncols - 1);
   };
-  const bf16* src[RT + MT][2];
+  const bf16* src[G];
 #pragma unroll
-  for (int t = 0; t < RT + MT; ++t)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int r = 8 * j + (lane >> 3);
-      const bf16* row = t < RT ? W + (size_t)wrow(t, r) * K : X + (size_t)min((t - RT) * 16 + r, M - 1) * K;
-      src[t][j] = row + wv * SK + sswz(r, lane & 7) * 8;
-    }
+  for (int q = 0; q < G; ++q) {
+    const int r = 8 * (q < RG ? q : q - RG) + (lane >> 3);
+    const bf16* row = q < RG ? W + (size_t)wrow(r) * K : X + (size_t)min(r, M - 1) * K;
+    src[q] = row + wv * SK + sswz(r, lane & 7) * 8;
+  }
   const int nk = K / SK, cnt = (nk - wv + WAVES - 1) / WAVES;     // this wave's K-tiles (0 for a short K)
   f32x4 acc[RT][MT];
 #pragma unroll
@@ -78,13 +78,12 @@ __global__ void __launch_bounds__(WAVES * 64) gemm_stream_kernel(bf16* __restric
   auto load = [&](int slot, int i) {
     const int ko = i * (WAVES * SK);
 #pragma unroll
-    for (int q = 0; q < 2 * RT; ++q)
-      __builtin_amdgcn_global_load_lds((glb_vptr_s)(src[q / 2][q & 1] + ko), (lds_vptr_s)(ring + slot * SLOT + q * 512), 16,
-                                       0, NT ? 2 : 0);
+    for (int q = 0; q < RG; ++q)
+      __builtin_amdgcn_global_load_lds((glb_vptr_s)(src[q] + ko), (lds_vptr_s)(ring + slot * SLOT + q * 512), 16, 0,
+                                       NT ? 2 : 0);
 #pragma unroll
-    for (int q = 2 * RT; q < G; ++q)
-      __builtin_amdgcn_global_load_lds((glb_vptr_s)(src[q / 2][q & 1] + ko), (lds_vptr_s)(ring + slot * SLOT + q * 512), 16,
-                                       0, 0);
+    for (int q = RG; q < G; ++q)
+      __builtin_amdgcn_global_load_lds((glb_vptr_s)(src[q] + ko), (lds_vptr_s)(ring + slot * SLOT + q * 512), 16, 0, 0);
     __builtin_amdgcn_sched_barrier(0);
   };
 #pragma unroll
@@ -104,11 +103,15 @@ __global__ void __launch_bounds__(WAVES * 64) gemm_stream_kernel(bf16* __restric
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
 #pragma unroll
-          for (int t = 0; t < RT; ++t)
-            wa[t][s] = *reinterpret_cast<const bf16x8*>(b + t * 1024 + fr * SK + sswz(fr, 4 * s + fq) * 8);
+          for (int t = 0; t < RT; ++t) {
+            const int r = 2 * t + 1 < RG ? fr : fr & 7;
+            wa[t][s] = *reinterpret_cast<const bf16x8*>(b + t * 1024 + r * SK + sswz(r, 4 * s + fq) * 8);
+          }
 #pragma unroll
-          for (int m = 0; m < MT; ++m)
-            xa[m][s] = *reinterpret_cast<const bf16x8*>(b + (RT + m) * 1024 + fr * SK + sswz(fr, 4 * s + fq) * 8);
+          for (int m = 0; m < MT; ++m) {
+            const int r = 2 * m + 1 < XG ? fr : fr & 7;
+            xa[m][s] = *reinterpret_cast<const bf16x8*>(b + RG * 512 + m * 1024 + r * SK + sswz(r, 4 * s + fq) * 8);
+          }
         }
         // every fragment of the slot is in registers before its refill goes out
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -132,16 +135,19 @@ __global__ void __launch_bounds__(WAVES * 64) gemm_stream_kernel(bf16* __restric
 #pragma unroll
     for (int m = 0; m < MT; ++m) red[(wv * RT * MT + t * MT + m) * 64 + lane] = acc[t][m];
   __syncthreads();
-  for (int e = tid; e < CT * MT * 64; e += WAVES * 64) {
-    const int tile = e >> 6, ln = e & 63, t = tile / MT, m = tile % MT;
-    f32x4 a = red[(t * MT + m) * 64 + ln], b = f32x4{0.f, 0.f, 0.f, 0.f};
+  // four columns of one row each: rows R .. R + 3 of the workgroup in tile R / 16, lane group R / 4 % 4
+  for (int e = tid; e < CW / 4 * MT * 16; e += WAVES * 64) {
+    const int m = e / (CW * 4), R = 4 * ((e >> 4) % (CW / 4)), U = CW + R;
+    const int at = ((R >> 4) * MT + m) * 64 + ((R >> 2) & 3) * 16 + (e & 15);
+    f32x4 a = red[at], b = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int w = 1; w < WAVES; ++w) a += red[(w * RT * MT + t * MT + m) * 64 + ln];
+    for (int w = 1; w < WAVES; ++w) a += red[w * RT * MT * 64 + at];
     if constexpr (GLU != 0) {
+      const int up = ((U >> 4) * MT + m) * 64 + ((U >> 2) & 3) * 16 + (e & 15);
 #pragma unroll
-      for (int w = 0; w < WAVES; ++w) b += red[(w * RT * MT + (t + CT) * MT + m) * 64 + ln];
+      for (int w = 0; w < WAVES; ++w) b += red[w * RT * MT * 64 + up];
     }
-    const int row = m * 16 + (ln & 15), c = c0 + t * 16 + 4 * (ln >> 4);
+    const int row = m * 16 + (e & 15), c = c0 + R;
     if (row >= M || c >= ncols) continue;
     bf16x4 o;
 #pragma unroll
@@ -166,6 +172,25 @@ __global__ void __launch_bounds__(WAVES * 64) gemm_stream_kernel(bf16* __restric
   }
 }
 
+// Groups of 8 weight rows per workgroup up to 16 rows of x: the fewest rows (weights and x) that a CU has to stage.  A CU
+// keeps some 64 cache lines in flight whatever the number of its waves, so the time is that of the CU with the most rows:
+// ceil(workgroups / 256) (RG + XG).  Where a weight row is a multiple of 4 KiB the lines of 32 and, more so, 64 rows that walk
+// K in step fall on few memory channels: their rows count 1.24 and 1.6 times.  us, M = 1 / 16, 16-row tiles (32 from 256 tiles
+// on) -> this: 1024 x 3072 4.8 / 6.1 -> 4.4 / 5.3, 2048 x 2048 4.5 / 5.1 -> 4.1 / 4.6, 2048 x 8192 10.5 / 12.0 -> 8.3 / 9.5,
+// 5120 x 2560 8.0 / 8.2 -> 7.0 / 7.5, 6144 x 4096 13.0 / 13.8 -> 10.3 / 10.1; GLU 8192 x 2048 9.0 / 9.3 -> 8.0 / 9.3, 10240 x
+// 2560 11.7 / 12.7 -> 10.9 / 11.3, 16384 x 4096 28.3 / 28.1 -> 23.6 / 25.6, 22016 x 4096 39.9 / 39.6 -> 30.0 / 29.7.
+static int stream_rows(int ncols, int K, bool glu, int xg) {
+  int best = 0;
+  float at = 0.f;
+  for (const int rg : {8, 6, 4, 3, 2, 1}) {
+    if (glu ? rg == 1 : rg > 4) continue;
+    const int cols = glu ? rg * 4 : rg * 8, wgs = (ncols + cols - 1) / cols;
+    const float t = (float)((wgs + 255) / 256) * (float)(rg + xg) * (K % 2048 ? 1.f : rg == 8 ? 1.6f : rg == 4 ? 1.24f : 1.f);
+    if (best == 0 || t < at) best = rg, at = t;
+  }
+  return best;
+}
+
 // glu 0: y [M, N] = x w^T (+ bias);  1 / 2 / 3: y [M, N / 2], SiLU / clipped / gelu GLU of w = [gate; up] (+ bias).
 // nt: nontemporal weight loads.
 void gemm_stream(uintptr_t y, uintptr_t x, uintptr_t w, uintptr_t bias, int M, int N, int K, int glu, int nt, float limit,
@@ -177,38 +202,61 @@ void gemm_stream(uintptr_t y, uintptr_t x, uintptr_t w, uintptr_t bias, int M, i
   DLLM_HOST_CHECK(x % 16 == 0 && w % 16 == 0 && y % 8 == 0, "operand alignment");
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const int ncols = glu ? N / 2 : N;
-  // twice the weight rows per workgroup (half the x staging) once that still leaves a workgroup for most CUs
-  const bool two = (ncols + 15) / 16 > 256;
-  const int per = two ? 32 : 16;
+  const bool one = M <= 16;
+  const int xg = M <= 8 ? 1 : M <= 16 ? 2 : M <= 32 ? 4 : 8;
+  int rg;
+  if (one) {
+    rg = stream_rows(ncols, K, glu != 0, xg);
+  } else {
+    // twice the weight rows per workgroup (half the x staging) once that still leaves a workgroup for most CUs
+    const bool two = (ncols + 15) / 16 > 256;
+    rg = (glu ? 4 : 2) * (two ? 2 : 1);
+  }
+  const int per = glu ? rg * 4 : rg * 8;
   const dim3 grid((ncols + per - 1) / per);
-  // single 16-row tiles: 8 waves, the K loop of a small weight is over in one or two rounds; else 4 (several
-  // workgroups per CU)
-#define DLLM_ST_GO(RT_, MT_, GLU_, WV_)                                                                              \
+  // 8 waves where up to three groups of plain rows have a CU each: their K loop is over in one or two rounds; else 4
+  // (several workgroups per CU)
+  const bool wide = glu == 0 && (one ? rg <= 3 && grid.x <= 256 : rg == 2 && xg == 4);
+#define DLLM_ST_GO(RG_, XG_, GLU_, WV_)                                                                             \
   do {                                                                                                              \
-    if (nt) hipLaunchKernelGGL((gemm_stream_kernel<RT_, MT_, GLU_, true, WV_>), grid, dim3(WV_ * 64), 0, s,         \
+    if (nt) hipLaunchKernelGGL((gemm_stream_kernel<RG_, XG_, GLU_, true, WV_>), grid, dim3(WV_ * 64), 0, s,         \
                                (bf16*)y, (const bf16*)x, (const bf16*)w, (const bf16*)bias, M, N, K, limit);          \
-    else hipLaunchKernelGGL((gemm_stream_kernel<RT_, MT_, GLU_, false, WV_>), grid, dim3(WV_ * 64), 0, s,           \
+    else hipLaunchKernelGGL((gemm_stream_kernel<RG_, XG_, GLU_, false, WV_>), grid, dim3(WV_ * 64), 0, s,           \
                             (bf16*)y, (const bf16*)x, (const bf16*)w, (const bf16*)bias, M, N, K, limit);             \
   } while (0)
-#define DLLM_ST_M(RT_, GLU_, WV_)                                                                                    \
+#define DLLM_ST_P(RG_, XG_)                                                                                         \
   do {                                                                                                              \
-    if (M <= 16) DLLM_ST_GO(RT_, 1, GLU_, WV_);                                                                      \
-    else if (M <= 32) DLLM_ST_GO(RT_, 2, GLU_, WV_);                                                                 \
-    else DLLM_ST_GO(RT_, 4, GLU_, 4);                                                                                \
+    constexpr int W8 = RG_ <= 3 && XG_ <= 4 ? 8 : 4;                                                                  \
+    if (wide) DLLM_ST_GO(RG_, XG_, 0, W8); else DLLM_ST_GO(RG_, XG_, 0, 4);                                            \
   } while (0)
-#define DLLM_ST_GLU(GLU_)                                                                                            \
+#define DLLM_ST_G(RG_, XG_)                                                                                         \
   do {                                                                                                              \
-    if (two) DLLM_ST_M(4, GLU_, 4);                                                                                  \
-    else DLLM_ST_M(2, GLU_, 4);                                                                                      \
+    if (glu == 1) DLLM_ST_GO(RG_, XG_, 1, 4); else if (glu == 2) DLLM_ST_GO(RG_, XG_, 2, 4); else DLLM_ST_GO(RG_, XG_, 3, 4); \
+  } while (0)
+#define DLLM_ST_X(DO_, RG_)                                                                                         \
+  do {                                                                                                              \
+    if (xg == 1) DO_(RG_, 1); else DO_(RG_, 2);                                                                       \
+  } while (0)
+#define DLLM_ST_M(DO_, RG_)                                                                                         \
+  do {                                                                                                              \
+    if (xg == 1) DO_(RG_, 1); else if (xg == 2) DO_(RG_, 2); else if (xg == 4) DO_(RG_, 4); else DO_(RG_, 8);            \
   } while (0)
   if (glu == 0) {
-    if (two) DLLM_ST_M(2, 0, 4);
-    else DLLM_ST_M(1, 0, 8);
-  } else if (glu == 1) DLLM_ST_GLU(1);
-  else if (glu == 2) DLLM_ST_GLU(2);
-  else DLLM_ST_GLU(3);
-#undef DLLM_ST_GLU
+    if (rg == 1) DLLM_ST_X(DLLM_ST_P, 1);
+    else if (rg == 2) DLLM_ST_M(DLLM_ST_P, 2);
+    else if (rg == 3) DLLM_ST_X(DLLM_ST_P, 3);
+    else DLLM_ST_M(DLLM_ST_P, 4);
+  } else {
+    if (rg == 2) DLLM_ST_X(DLLM_ST_G, 2);
+    else if (rg == 3) DLLM_ST_X(DLLM_ST_G, 3);
+    else if (rg == 4) DLLM_ST_M(DLLM_ST_G, 4);
+    else if (rg == 6) DLLM_ST_X(DLLM_ST_G, 6);
+    else DLLM_ST_M(DLLM_ST_G, 8);
+  }
 #undef DLLM_ST_M
+#undef DLLM_ST_X
+#undef DLLM_ST_G
+#undef DLLM_ST_P
 #undef DLLM_ST_GO
   DLLM_HIP_CHECK(hipGetLastError());
 }

@@ -155,6 +155,13 @@ def _use_wide(m: int, n: int, k: int, x: torch.Tensor, w: torch.Tensor, swiglu: 
 #  * GLU, M = 1 / 32 / 64: 15360 x 2560 15.8 / 16.9 / 20.4, 18.4 / 19.3 / 20.9; 16384 x 4096 30.2 / 29.7 / 32.0, 34.4 / 33.6 / 34.3;
 #    22016 x 4096 39.8 / 44.0 / 51.3, 34.1 / 35.0 / 39.2; 10240 x 4096 (160 workgroups) 22.0 / 22.6 / 25.7, 18.6 / 19.2 / 20.6;
 #    28672 x 4096 41.8 / 45.0 / 53.4, 41.0 / 39.8 / 42.5; 4096 x 8192 17.8 / 24.0 / 28.7, 16.2 / 18.2 / 19.3.
+# Up to 16 rows the workgroups are cut by what a CU stages (gemm_stream.hip, stream_rows), which took the line further out, us,
+# M = 1 / 8 / 16:
+#  * plain: 6144 x 4096 11.0 / 10.5 / 10.6, 13.3 / 13.2 / 13.5; 5120 x 5120 11.6 /
+#    11.4 / 12.6, 13.4 / 14.0 / 14.4; 10240 x 8192 28.6 / 29.8 / 32.3, 32.4 / 32.7 / 31.6; 4096 x 8192 16.4 / 16.3, 16.0 / 15.6;
+#  * in front of a close the line stays: 2560 x 7680 at 16 rows in a decode step 12.8 + 4.6 (close), 9.4 + 5.1;
+#  * GLU: 16384 x 4096 24.7 / 23.6 / 25.8, 32.6 / 32.7 / 33.0; 14336 x 5120 25.8 / 24.8 / 26.0, 30.4 / 29.9 / 30.6; 28672 x 4096
+#    38.6 / 37.3 / 42.1, 38.1 / 36.6 / 36.8.
 STREAM_MAX_M = 64
 
 
@@ -172,15 +179,15 @@ def stream_fits(m: int, n: int, k: int, glu: str = "", defer: bool = False, bias
         return False                                 # K < 512: fewer K-tiles than waves, and no split to save either
     mi = n * k / (1 << 20)
     if glu:
-        if k > (4096 if m <= 32 else 2560) or (mi > (20 if m <= 32 else 12) and _stream_fill(n // 2) < 0.75):
+        if k > (5120 if m <= 16 else 4096 if m <= 32 else 2560) or (mi > (20 if m <= 32 else 12) and _stream_fill(n // 2) < 0.75):
             return False
-        return mi <= (64 if m <= 32 and glu != "silu" else 40)
+        return mi <= (96 if m <= 16 else 64 if m <= 32 and glu != "silu" else 40)
     if n > 65536:
         return False                                 # an LM head fills the chip unsplit on the wide kernel
     if defer and n % 128 == 0:
         return (mi <= 8 and k <= 4096) if m <= 16 else (mi <= 2 and k <= 2048)
     if m <= 16:
-        return mi <= (32 if k <= 2560 else 24) and k <= 8192
+        return k <= 8192 and mi <= (32 if k <= 2560 else 80 if m <= 8 and n > 4096 else 28 if n > 4096 else 24)
     if m <= 32:
         return mi <= 24 and k <= 4096 and (mi <= 16 or _stream_fill(n) >= 0.75)
     if bias or n % 128:

@@ -61,6 +61,41 @@ def test_stream_glu(cuda, m, half, k, glu, bias):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("m", [1, 8, 9, 16])
+@pytest.mark.parametrize("n,k", [(2048, 128), (2049, 192), (4096, 128), (4100, 64), (6143, 192), (6145, 128), (10240, 2048),
+                                 (12289, 64), (8, 2048)])
+def test_stream_rows_per_workgroup(cuda, m, n, k):
+    """8, 16, 24 and 32 weight rows per workgroup in one and several rounds, x in one and two groups of 8 rows, last
+    workgroups that hold one row; and the same as a GLU where n has halves."""
+    x, w = torch.randn(m, k, device="cuda").bfloat16(), (torch.randn(n, k, device="cuda") * 0.05).bfloat16()
+    y = gemm.linear_stream(x, w)
+    ref, mag = F.linear(x.double(), w.double()), x.double().abs() @ w.double().abs().t()
+    assert _close(y, ref, mag, k)
+    if n % 2 == 0:
+        h = n // 2
+        g, u = ref[:, :h], ref[:, h:]
+        y = gemm.linear_stream(x, w, None, "silu")
+        # as test_stream_glu: the sums' errors through the product, the activation's 2^-20, the bf16 result
+        e = mag * k * 2.0 ** -24
+        tol = 1.2 * e[:, :h] * u.abs() + (g.abs() + 1e-3) * e[:, h:] + (2.0 ** -8 + 2.0 ** -18) * (F.silu(g) * u).abs() + 2.0 ** -22
+        assert bool(((y.double() - F.silu(g) * u).abs() <= tol).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("half,k,m", [(4096, 64, 16), (5120, 64, 3), (7681, 64, 16), (10240, 64, 16), (3072, 2048, 1), (8192, 2048, 16)])
+def test_stream_glu_rows_per_workgroup(cuda, half, k, m):
+    """Every GLU cut (8, 12, 16, 24 and 32 columns), with biases."""
+    x, w = torch.randn(m, k, device="cuda").bfloat16(), (torch.randn(2 * half, k, device="cuda") * k ** -0.5).bfloat16()
+    b = torch.randn(2 * half, device="cuda").bfloat16()
+    z = F.linear(x.double(), w.double(), b.double())
+    e = (x.double().abs() @ w.double().abs().t() + b.double().abs()) * (k + 1) * 2.0 ** -24
+    g, u = z[:, :half], z[:, half:]
+    ref = F.silu(g) * u
+    tol = 1.2 * e[:, :half] * u.abs() + (g.abs() + 1e-3) * e[:, half:] + (2.0 ** -8 + 2.0 ** -18) * ref.abs() + 2.0 ** -22
+    assert bool(((gemm.linear_stream(x, w, b, "silu").double() - ref).abs() <= tol).all())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("glu", ["clipped", "gelu"])
 def test_stream_glu_keeps_the_gate_kernels_arithmetic(cuda, glu):
     """Products of one term each are exact in f32, so the epilogue's result is the f32 gate kernel's, rounded once: bit for
@@ -151,3 +186,12 @@ def test_stream_rule():
     assert not gemm.use_stream(4, 256, 512, x, torch.zeros(256 * 512 + 1, dtype=torch.bfloat16)[1:].view(256, 512))
     with knobs.override(stream=False):
         assert not gemm.use_stream(4, 256, 512, x, w)
+
+
+def test_stream_rule_up_to_16_rows():
+    """The line where a workgroup's rows follow the CU's share: further out than past 16 rows, on both sides of it."""
+    assert gemm.stream_fits(16, 6144, 4096) and gemm.stream_fits(8, 10240, 8192) and not gemm.stream_fits(9, 10240, 8192)
+    assert gemm.stream_fits(16, 5120, 5120) and not gemm.stream_fits(8, 4096, 8192)
+    assert not gemm.stream_fits(16, 2560, 7680, defer=True)
+    assert gemm.stream_fits(16, 16384, 4096, "silu") and not gemm.stream_fits(17, 16384, 4096, "silu")
+    assert gemm.stream_fits(16, 14336, 5120, "silu") and not gemm.stream_fits(1, 27648, 5120, "silu")
