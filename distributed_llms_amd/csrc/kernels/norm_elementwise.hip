@@ -135,7 +135,7 @@ __global__ void __launch_bounds__(256) rope_cache_kernel(bf16* __restrict__ q_ou
                                                          const float* __restrict__ cos_sin,
                                                          bf16* __restrict__ k_cache, bf16* __restrict__ v_cache,
                                                          const int32_t* __restrict__ slots, int hq, int hkv,
-                                                         int d, int bs, int do_v) {
+                                                         int d, int bs) {
   const int t = blockIdx.x;
   const int half = d >> 1;
   const int qpr = half >> 2;  // threads per head (4 pairs each)
@@ -174,7 +174,6 @@ __global__ void __launch_bounds__(256) rope_cache_kernel(bf16* __restrict__ q_ou
     *reinterpret_cast<bf16x4*>(dst + p) = o1;
     *reinterpret_cast<bf16x4*>(dst + half + p) = o2;
   }
-  if (!do_v) return;  // v_group_kernel appends V
   // v: transposed store into [blk][h][d][bs]
   const bf16* vsrc = row + (hq + hkv) * d;
   for (int i = threadIdx.x; i < hkv * d; i += blockDim.x) {
@@ -183,61 +182,189 @@ __global__ void __launch_bounds__(256) rope_cache_kernel(bf16* __restrict__ q_ou
   }
 }
 
-// V append for a prefill batch, eight tokens per workgroup.  The transposed layouts keep a key's
-// 8-aligned group of 8 contiguous per (head, e) -- vofs(off0 + j) = vofs(off0) + j when
-// off0 % 8 == 0 and bs % 8 == 0 -- so when the group's slots are consecutive and 8-aligned (a
-// prompt's tokens: consecutive slots from a block start) a thread writes one 16-byte vector where
-// the per-token path scatters eight 2-byte stores (whole 64-byte lines instead of partial ones).
-// Loads: for a fixed token j, a wave's 64 consecutive e read 128 contiguous bytes.  Any other group
-// (a prompt boundary inside it, a sequence resuming mid-group, the batch tail) takes the per-token
-// scatter.
-__global__ void __launch_bounds__(256) v_group_kernel(const bf16* __restrict__ qkv, bf16* __restrict__ v_cache,
-                                                      const int32_t* __restrict__ slots, int tokens, int hq,
-                                                      int hkv, int d, int bs) {
+// The same for batches of eight tokens and more, and for a projection still in split-K slabs (any batch): eight tokens and
+// up to 1024 columns of q, k or v per workgroup, all of a thread's loads under way before the first use.
+//
+// V: the transposed layouts keep a key's 8-aligned group of 8 contiguous per (head, e) -- vofs(off0 + j) = vofs(off0) + j
+// when off0 % 8 == 0 and bs % 8 == 0 -- so when the group's slots are consecutive and 8-aligned (a prompt's tokens:
+// consecutive slots from a block start) a thread writes one 16-byte vector, through an LDS tile, where the per-token
+// path scatters eight 2-byte stores (whole 64-byte lines instead of partial ones).  Any other group (a prompt boundary
+// inside it, a sequence resuming mid-group, the batch tail) takes the scatter.
+//
+// Slabs (SC > 0: their number, -1: a runtime number) are summed in slab order and rounded to bf16, as splitk_reduce sums
+// them, on the way: a prompt of 128 tokens of 32 / 8 heads took a launch for the sum (3.7 us), one for K (3.3) and one for V
+// (4.1).  q_out: the rotated q, or (rotate_q 0, slabs only: the attention rotates it) the summed one.
+constexpr int kAppendCols = 1024;
+
+template <int SC>
+__global__ void __launch_bounds__(256) qkv_append_kernel(bf16* __restrict__ q_out, int rotate_q,
+                                                         const bf16* __restrict__ qkv, const float* __restrict__ part,
+                                                         int nparts, long slab, const int32_t* __restrict__ positions,
+                                                         const float* __restrict__ cos_sin, bf16* __restrict__ k_cache,
+                                                         bf16* __restrict__ v_cache, const int32_t* __restrict__ slots,
+                                                         int tokens, int hq, int hkv, int d, int bs) {
+  __shared__ __attribute__((aligned(16))) bf16 tile[8][kAppendCols + 8];
   __shared__ int sl[8];
-  const int t0 = blockIdx.x * 8;
-  const int n = min(8, tokens - t0);
-  if (threadIdx.x < 8) sl[threadIdx.x] = threadIdx.x < n ? slots[t0 + threadIdx.x] : -1;
-  __syncthreads();
-  const int width = (hq + 2 * hkv) * d;
-  const bf16* vsrc = qkv + (size_t)t0 * width + (hq + hkv) * d;
-  bool full = n == 8 && sl[0] >= 0 && sl[0] % 8 == 0;
+  constexpr int R = 4;                                 // four elements or pairs of four per item, R items in flight
+  constexpr int NS = SC > 0 ? SC : 1;
+  const int t0 = blockIdx.x * 8, n = min(8, tokens - t0), tid = threadIdx.x;
+  const int width = (hq + 2 * hkv) * d, half = d >> 1;
+  const int hpc = max(1, kAppendCols / d);             // heads per workgroup
+  const int nkv = (hkv + hpc - 1) / hpc;
+  const int y = blockIdx.y, what = y < nkv ? 2 : y < 2 * nkv ? 1 : 0;          // v, k, q
+  const int h0 = (what == 2 ? y : what == 1 ? y - nkv : y - 2 * nkv) * hpc;
+  const int heads = min(hpc, (what == 0 ? hq : hkv) - h0);
+  const int col0 = ((what == 0 ? 0 : what == 1 ? hq : hq + hkv) + h0) * d;      // first column in a row of qkv
+  // four consecutive values from element p on: in their stored form, and summed
+  typedef part_elem raw4 __attribute__((ext_vector_type(4)));
+  auto load = [&](raw4 (&l)[NS], bf16x4& v, size_t p) {
+    if constexpr (SC == 0) v = *reinterpret_cast<const bf16x4*>(qkv + p);
+    if constexpr (SC > 0) {
 #pragma unroll
-  for (int j = 1; j < 8; ++j) full = full && sl[j] == sl[0] + j;
-  if (full) {
-    const int blk = sl[0] / bs, off0 = sl[0] % bs;
-    for (int i = threadIdx.x; i < hkv * d; i += blockDim.x) {
-      const int h = i / d, e = i % d;
-      bf16x8 o;
+      for (int s = 0; s < NS; ++s)
+        l[s] = __builtin_nontemporal_load(reinterpret_cast<const raw4*>(reinterpret_cast<const part_elem*>(part) + p + s * slab));
+    }
+  };
+  auto finish = [&](const raw4 (&l)[NS], size_t p) {
+    f32x4 a = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (SC == -1) {
+      for (int s = 0; s < nparts; ++s) a += part_load4<true>(part, p + s * slab);
+    } else {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) o[j] = vsrc[(size_t)j * width + i];
-      *reinterpret_cast<bf16x8*>(v_cache + ((size_t)blk * hkv + h) * d * bs + vofs(off0, e, d, bs)) = o;
+      for (int s = 0; s < NS; ++s) a += f32x4{part_value(l[s][0]), part_value(l[s][1]), part_value(l[s][2]), part_value(l[s][3])};
+    }
+    return bf16x4{f2bf(a[0]), f2bf(a[1]), f2bf(a[2]), f2bf(a[3])};
+  };
+  if (what == 2) {
+    const int per = heads * d / 4, total = 8 * per;    // items of a token, of the workgroup
+    if (tid < 8) sl[tid] = tid < n ? slots[t0 + tid] : -1;
+    for (int i0 = tid; i0 < total; i0 += 256 * R) {
+      raw4 l[R][NS];
+      bf16x4 v[R];
+#pragma unroll
+      for (int u = 0; u < R; ++u) {
+        const int i = min(i0 + u * 256, total - 1), j = min(i / per, n - 1);
+        load(l[u], v[u], (size_t)(t0 + j) * width + col0 + (i % per) * 4);
+      }
+#pragma unroll
+      for (int u = 0; u < R; ++u) {
+        const int i = i0 + u * 256;
+        if (i >= total) break;
+        const int j = i / per;
+        if constexpr (SC != 0) v[u] = finish(l[u], (size_t)(t0 + min(j, n - 1)) * width + col0 + (i % per) * 4);
+        *reinterpret_cast<bf16x4*>(&tile[j][(i % per) * 4]) = v[u];
+      }
+    }
+    __syncthreads();
+    bool full = n == 8 && bs % 8 == 0 && sl[0] >= 0 && sl[0] % 8 == 0;
+#pragma unroll
+    for (int j = 1; j < 8; ++j) full = full && sl[j] == sl[0] + j;
+    if (full) {
+      const int blk = sl[0] / bs, off0 = sl[0] % bs;
+      for (int i = tid; i < heads * d; i += 256) {
+        const int h = h0 + i / d, e = i % d;
+        bf16x8 o;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) o[j] = tile[j][i];
+        *reinterpret_cast<bf16x8*>(v_cache + ((size_t)blk * hkv + h) * d * bs + vofs(off0, e, d, bs)) = o;
+      }
+      return;
+    }
+    for (int j = 0; j < n; ++j) {
+      const int blk = sl[j] / bs, off = sl[j] % bs;
+      for (int i = tid; i < heads * d; i += 256)
+        v_cache[((size_t)blk * hkv + h0 + i / d) * d * bs + vofs(off, i % d, d, bs)] = tile[j][i];
     }
     return;
   }
-  for (int j = 0; j < n; ++j) {
-    const int blk = sl[j] / bs, off = sl[j] % bs;
-    for (int i = threadIdx.x; i < hkv * d; i += blockDim.x) {
-      const int h = i / d, e = i % d;
-      v_cache[((size_t)blk * hkv + h) * d * bs + vofs(off, e, d, bs)] = vsrc[(size_t)j * width + i];
+  // q and k: pairs (e, e + d / 2), four of them per item
+  const bool rot = cos_sin != nullptr && (what == 1 || rotate_q);
+  const int qpr = half >> 2, per = heads * qpr, total = n * per;
+  constexpr int RP = 2;
+  for (int i0 = tid; i0 < total; i0 += 256 * RP) {
+    raw4 l1[RP][NS], l2[RP][NS];
+    f32x4 c[RP], s[RP];
+    bf16x4 x1[RP], x2[RP];
+    int pos[RP], slot[RP];
+#pragma unroll
+    for (int u = 0; u < RP; ++u) {
+      const int i = min(i0 + u * 256, total - 1), t = t0 + i / per;
+      pos[u] = positions[t];
+      slot[u] = slots[t];
+      const size_t p = (size_t)t * width + col0 + (i % per) / qpr * d + (i % qpr) * 4;
+      load(l1[u], x1[u], p);
+      load(l2[u], x2[u], p + half);
+    }
+    const float* table = rot ? cos_sin : nullptr;
+    if (table) {
+#pragma unroll
+      for (int u = 0; u < RP; ++u) {
+        const float* cs = table + (size_t)pos[u] * d + (min(i0 + u * 256, total - 1) % qpr) * 4;
+        c[u] = *reinterpret_cast<const f32x4*>(cs);
+        s[u] = *reinterpret_cast<const f32x4*>(cs + half);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < RP; ++u) {
+      const int i = i0 + u * 256;
+      if (i >= total) break;
+      const int t = t0 + i / per, h = h0 + (i % per) / qpr, e = (i % qpr) * 4;
+      if constexpr (SC != 0) {
+        const size_t p = (size_t)t * width + col0 + (h - h0) * d + e;
+        x1[u] = finish(l1[u], p);
+        x2[u] = finish(l2[u], p + half);
+      }
+      bf16x4 o1 = x1[u], o2 = x2[u];
+      if (rot) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float a = bf2f(x1[u][j]), b = bf2f(x2[u][j]);
+          o1[j] = f2bf(a * c[u][j] - b * s[u][j]);
+          o2[j] = f2bf(b * c[u][j] + a * s[u][j]);
+        }
+      }
+      bf16* dst = what == 0 ? q_out + ((size_t)t * hq + h) * d
+                            : k_cache + (((size_t)(slot[u] / bs) * hkv + h) * bs + krow(slot[u] % bs, bs)) * d;
+      *reinterpret_cast<bf16x4*>(dst + e) = o1;
+      *reinterpret_cast<bf16x4*>(dst + half + e) = o2;
     }
   }
 }
 
-void rope_cache_append(uintptr_t q_out, uintptr_t qkv, uintptr_t positions, uintptr_t cos_sin,
-                       uintptr_t k_cache, uintptr_t v_cache, uintptr_t slots, int tokens, int hq, int hkv,
-                       int d, int bs, int v_groups, uintptr_t stream) {
+// part != 0: qkv as nparts split-K slabs, `slab` elements apart (qkv unused); q_out: the rotated q, or the summed one of slabs
+// where rotate_q is 0; 0: neither
+void rope_cache_append(uintptr_t q_out, int rotate_q, uintptr_t qkv, uintptr_t part, int nparts, long slab,
+                       uintptr_t positions, uintptr_t cos_sin, uintptr_t k_cache, uintptr_t v_cache, uintptr_t slots,
+                       int tokens, int hq, int hkv, int d, int bs, int v_groups, uintptr_t stream) {
   DLLM_HOST_CHECK(d % 8 == 0 && d <= 256, "head_dim must be a multiple of 8, <= 256");
   DLLM_HOST_CHECK(hq % hkv == 0, "Hq % Hkv");
+  DLLM_HOST_CHECK(part == 0 || (nparts >= 1 && slab >= (long)tokens * (hq + 2 * hkv) * d), "qkv partial slabs");
+  DLLM_HOST_CHECK(part != 0 || rotate_q || q_out == 0, "an unrotated q is read from qkv itself");
   if (tokens == 0) return;
-  const bool grouped = v_groups && bs % 8 == 0 && tokens >= 8;
-  hipLaunchKernelGGL(rope_cache_kernel, dim3(tokens), dim3(256), 0, reinterpret_cast<hipStream_t>(stream),
-                     (bf16*)q_out, (const bf16*)qkv, (const int32_t*)positions, (const float*)cos_sin,
-                     (bf16*)k_cache, (bf16*)v_cache, (const int32_t*)slots, hq, hkv, d, bs, grouped ? 0 : 1);
-  DLLM_HIP_CHECK(hipGetLastError());
-  if (!grouped) return;
-  hipLaunchKernelGGL(v_group_kernel, dim3((tokens + 7) / 8), dim3(256), 0, reinterpret_cast<hipStream_t>(stream),
-                     (const bf16*)qkv, (bf16*)v_cache, (const int32_t*)slots, tokens, hq, hkv, d, bs);
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  if (part == 0 && !(v_groups && bs % 8 == 0 && tokens >= 8)) {
+    hipLaunchKernelGGL(rope_cache_kernel, dim3(tokens), dim3(256), 0, st, (bf16*)q_out, (const bf16*)qkv,
+                       (const int32_t*)positions, (const float*)cos_sin, (bf16*)k_cache, (bf16*)v_cache,
+                       (const int32_t*)slots, hq, hkv, d, bs);
+    DLLM_HIP_CHECK(hipGetLastError());
+    return;
+  }
+  const int hpc = d > kAppendCols ? 1 : kAppendCols / d;
+  const dim3 grid((tokens + 7) / 8, 2 * ((hkv + hpc - 1) / hpc) + (q_out ? (hq + hpc - 1) / hpc : 0));
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, (bf16*)q_out, rotate_q, (const bf16*)qkv, (const float*)part, nparts,
+                       slab, (const int32_t*)positions, (const float*)cos_sin, (bf16*)k_cache, (bf16*)v_cache,
+                       (const int32_t*)slots, tokens, hq, hkv, d, bs);
+  };
+  switch (part ? nparts : 0) {
+    case 0: go(qkv_append_kernel<0>); break;
+    case 2: go(qkv_append_kernel<2>); break;
+    case 3: go(qkv_append_kernel<3>); break;
+    case 4: go(qkv_append_kernel<4>); break;
+    case 5: go(qkv_append_kernel<5>); break;
+    case 8: go(qkv_append_kernel<8>); break;
+    default: go(qkv_append_kernel<-1>);
+  }
   DLLM_HIP_CHECK(hipGetLastError());
 }
 

@@ -306,24 +306,23 @@ class ModelStage:
 
     def _attention(self, qkv, li: int, meta: BatchMeta) -> torch.Tensor:
         """``qkv``: [T, (Hq + 2 Hkv) D] or, from a split-K projection, a SplitKPartial that the fused
-        decode kernel reduces itself (any other path materialises it)."""
+        decode kernel and the K / V append reduce themselves."""
         cfg = self.cfg
         k_cache, v_cache = self.kv.layer(li)
         fused = not meta.is_prefill and knobs.K.fused_rope and \
             (isinstance(qkv, ops.gemm.SplitKPartial) or qkv.is_cuda)
-        if not fused and isinstance(qkv, ops.gemm.SplitKPartial):
-            qkv = qkv.materialize()
         if fused:
             o = ops.paged_attention_decode_rope(qkv, meta.positions, self.cos_sin, k_cache, v_cache, meta.slot_mapping,
                                                 meta.block_tables, meta.seq_lens, self.hq, self.hkv,
                                                 cfg.head_dim, self.scale, max_ctx=meta.max_ctx or None,
                                                 workspace=meta.attn_workspace)
             return o.view(o.shape[0], self.q_size_local)
-        if meta.is_prefill and not meta.num_decode and qkv.is_cuda and \
+        part = isinstance(qkv, ops.gemm.SplitKPartial)
+        if meta.is_prefill and not meta.num_decode and (part or qkv.is_cuda) and \
                 ops.prefill_rope_in_attention(meta.block_tables.shape[1]):
-            ops.rope_cache_append(qkv, meta.positions, self.cos_sin, k_cache, v_cache, meta.slot_mapping,
-                                  self.hq, self.hkv, cfg.head_dim, write_q=False)
-            o = ops.paged_attention_prefill_rope(qkv, meta.positions, self.cos_sin, k_cache, v_cache,
+            q = ops.rope_cache_append(qkv, meta.positions, self.cos_sin, k_cache, v_cache, meta.slot_mapping,
+                                      self.hq, self.hkv, cfg.head_dim, write_q=False)
+            o = ops.paged_attention_prefill_rope(q if part else qkv, meta.positions, self.cos_sin, k_cache, v_cache,
                                                  meta.block_tables, meta.cu_seqlens_q, meta.seq_lens, self.hq,
                                                  cfg.head_dim, self.scale, max_q_len=meta.max_q_len)
             return o.view(o.shape[0], self.q_size_local)

@@ -193,26 +193,38 @@ def silu_mul(gu: torch.Tensor) -> torch.Tensor:
 def rope_cache_append(qkv, positions, cos_sin, k_cache, v_cache, slot_mapping, num_heads, num_kv_heads,
                       head_dim, write_q: bool = True) -> Optional[torch.Tensor]:
     """Rotate k (and q) and append k / v^T to the paged cache; returns the rotated q [T, Hq, D], or
-    None with ``write_q=False`` (the prefill attention then rotates q itself)."""
-    if not _gpu(qkv):
+    None with ``write_q=False`` (the prefill attention then rotates q itself).
+
+    ``qkv`` may be a :class:`gemm.SplitKPartial`, whose slabs are then summed on the way (bit-identical to reducing
+    first); with ``write_q=False`` the q columns come back summed and unrotated, [T, Hq * D]."""
+    part = qkv if isinstance(qkv, gemm.SplitKPartial) else None
+    if part is None and not _gpu(qkv):
         q = ref.rope_cache_append(qkv, positions, cos_sin, k_cache, v_cache, slot_mapping, num_heads,
                                   num_kv_heads, head_dim)
         return q if write_q else None
-    _ck(qkv, "rope.qkv")
+    if part is None:
+        _ck(qkv, "rope.qkv")
+        t, width = qkv.shape
+    else:
+        t, width = part.m, part.n
     _ck(k_cache, "k_cache")
     _ck(v_cache, "v_cache")
     _ck(positions, "positions", torch.int32)
     _ck(slot_mapping, "slot_mapping", torch.int32)
-    t = qkv.shape[0]
-    if qkv.shape[1] != (num_heads + 2 * num_kv_heads) * head_dim:
+    if width != (num_heads + 2 * num_kv_heads) * head_dim:
         raise ValueError("qkv width mismatch")
     if cos_sin is not None:
         _ck(cos_sin, "cos_sin", torch.float32)
         if cos_sin.shape[1] != head_dim:
             raise ValueError("cos_sin width must equal head_dim")
-    q = torch.empty(t, num_heads, head_dim, dtype=qkv.dtype, device=qkv.device) if write_q else None
-    _ext.kernels().rope_cache_append(q.data_ptr() if write_q else 0, qkv.data_ptr(), positions.data_ptr(),
-                                     0 if cos_sin is None else cos_sin.data_ptr(), k_cache.data_ptr(),
+    q = None
+    if write_q:
+        q = torch.empty(t, num_heads, head_dim, dtype=qkv.dtype, device=qkv.device)
+    elif part is not None:
+        q = torch.empty(t, num_heads * head_dim, dtype=qkv.dtype, device=qkv.device)
+    _ext.kernels().rope_cache_append(0 if q is None else q.data_ptr(), int(write_q), 0 if part is not None else qkv.data_ptr(),
+                                     0 if part is None else part.ws.data_ptr(), 0 if part is None else part.splits, t * width,
+                                     positions.data_ptr(), 0 if cos_sin is None else cos_sin.data_ptr(), k_cache.data_ptr(),
                                      v_cache.data_ptr(), slot_mapping.data_ptr(), t, num_heads, num_kv_heads,
                                      head_dim, k_cache.shape[2], int(knobs.K.v_group_append), _stream())
     return q
@@ -412,8 +424,8 @@ def prefill_rope_in_attention(max_blocks: Optional[int] = None) -> bool:
 def paged_attention_prefill_rope(qkv, positions, cos_sin, k_cache, v_cache, block_tables, cu_seqlens_q, seq_lens,
                                  num_heads: int, head_dim: int, scale: float, max_q_len: Optional[int] = None,
                                  out: Optional[torch.Tensor] = None):
-    """Prefill attention reading q straight from the qkv projection [T, (Hq + 2 Hkv) * D] and rotating it
-    in registers (K / V already appended by ``rope_cache_append(..., write_q=False)``): the rotated q
+    """Prefill attention reading q straight from the qkv projection [T, (Hq + 2 Hkv) * D] (or from its q columns alone,
+    [T, Hq * D]) and rotating it in registers (K / V already appended by ``rope_cache_append(..., write_q=False)``): the rotated q
     never round-trips through HBM.  Returns [T, Hq, D]."""
     hkv = k_cache.shape[1]
     t, width = qkv.shape
@@ -428,7 +440,7 @@ def paged_attention_prefill_rope(qkv, positions, cos_sin, k_cache, v_cache, bloc
     _ck(cu_seqlens_q, "cu_seqlens_q", torch.int32)
     _ck(seq_lens, "seq_lens", torch.int32)
     _ck(positions, "positions", torch.int32)
-    if width != (num_heads + 2 * hkv) * head_dim:
+    if width not in ((num_heads + 2 * hkv) * head_dim, num_heads * head_dim):
         raise ValueError("qkv width mismatch")
     if cos_sin is not None:
         _ck(cos_sin, "cos_sin", torch.float32)

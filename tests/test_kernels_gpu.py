@@ -113,6 +113,42 @@ def test_rope_cache_append_prefill_groups(cuda, grouped):
     torch.testing.assert_close(v1, v2, atol=0, rtol=0)
 
 
+@pytest.mark.parametrize("hq,hkv,d", [(32, 8, 128), (8, 2, 64), (20, 20, 96), (4, 1, 256), (6, 3, 8)])
+@pytest.mark.parametrize("tokens", [1, 8, 45])
+@pytest.mark.parametrize("slabs", [0, 2, 3, 5, 7])
+def test_rope_cache_append_sums_slabs(cuda, hq, hkv, d, tokens, slabs):
+    """The append of a projection in split-K slabs against the append of the reduced one, bit for bit: k, v, the rotated and
+    the plain q; several workgroups of heads, groups of eight tokens that are whole, start mid-group or are short."""
+    from distributed_llms_amd.ops import gemm
+    nb, width = 6, (hq + 2 * hkv) * d
+    first = tokens // 2 + 3
+    slots = torch.tensor([32 + i for i in range(first)][:tokens] + [100 + i for i in range(max(0, tokens - first))],
+                         dtype=torch.int32, device="cuda")
+    pos = torch.randint(0, 500, (tokens,), device="cuda", dtype=torch.int32)
+    cs = ref.rope_cos_sin(d, 1024, 500000.0, device="cuda")
+    if slabs:
+        p = gemm.SplitKPartial((torch.randn(slabs, tokens, width, device="cuda") / 64).half(), slabs, tokens, width,
+                               (tokens, width), torch.bfloat16, torch.device("cuda"))
+        whole = p.materialize()
+    else:
+        p = whole = _bf(tokens, width)
+    k1, v1 = _cache(nb, hkv, d)
+    k2, v2 = _cache(nb, hkv, d)
+    k3, v3 = _cache(nb, hkv, d)
+    q1 = ops.rope_cache_append(p, pos, cs, k1, v1, slots, hq, hkv, d)
+    q3 = ops.rope_cache_append(p, pos, cs, k3, v3, slots, hq, hkv, d, write_q=False)
+    q2 = torch.cat([ops.rope_cache_append(whole[i:i + 1], pos[i:i + 1], cs, k2, v2, slots[i:i + 1], hq, hkv, d)
+                    for i in range(tokens)])
+    assert torch.equal(q1, q2) and torch.equal(k1, k2) and torch.equal(v1, v2)
+    assert torch.equal(k3, k2) and torch.equal(v3, v2)
+    assert q3 is None if not slabs else torch.equal(q3, whole[:, :hq * d])
+    kr, vr = _cache(nb, hkv, d)
+    qr = ref.rope_cache_append(whole.float(), pos, cs, kr, vr, slots, hq, hkv, d)
+    torch.testing.assert_close(q1.float(), qr.float(), atol=2e-2, rtol=2e-2)
+    torch.testing.assert_close(k1.float(), kr.float(), atol=2e-2, rtol=2e-2)
+    assert torch.equal(v1, vr)
+
+
 def _fill_paged(seq_lens, hkv, d, nb_total=None):
     bs = 32
     nblocks = [(n + bs - 1) // bs for n in seq_lens]
