@@ -19,6 +19,7 @@ import torch
 from .. import _ext, knobs
 from . import gemm, quant
 from . import reference as ref
+from .stream import current_stream as _stream
 
 __all__ = [
     "embedding", "rms_norm", "fused_add_rms_norm", "layer_norm", "linear", "linear_into_norm", "silu_mul",
@@ -26,10 +27,6 @@ __all__ = [
     "argmax", "add_", "moe_route", "moe_mlp", "decode_split_plan", "paged_attention_decode_rope",
     "paged_attention_prefill_rope",
 ]
-
-
-def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
 
 
 def _ck(t: torch.Tensor, name: str, dtype=torch.bfloat16):

@@ -38,6 +38,7 @@ from torch.autograd import forward_ad
 
 from .. import _ext
 from .. import knobs
+from .stream import current_stream
 
 
 def is_down_proj(n: int, k: int) -> bool:
@@ -246,7 +247,7 @@ def _stream(m: int, n: int, k: int, x: torch.Tensor, w: torch.Tensor, bias: Opti
     y = torch.empty(*x.shape[:-1], n // 2 if glu else n, dtype=x.dtype, device=x.device)
     _ext.kernels().gemm_stream(y.data_ptr(), x.data_ptr(), w.data_ptr(), 0 if bias is None else bias.data_ptr(), m, n, k,
                                _STREAM_GLU[glu], 1 if n * k * 2 >= WIDE_NT_MIN_BYTES else 0, float(limit),
-                               torch.cuda.current_stream().cuda_stream)
+                               current_stream())
     return y
 
 
@@ -269,7 +270,7 @@ class SplitKPartial:
     def materialize(self) -> torch.Tensor:
         y = torch.empty(self.shape, dtype=self.dtype, device=self.device)
         _ext.kernels().splitk_reduce(y.data_ptr(), self.ws.data_ptr(), 0, self.splits, self.m, self.n,
-                                     torch.cuda.current_stream().cuda_stream)
+                                     current_stream())
         return y
 
 
@@ -323,7 +324,7 @@ _WS_FLOATS = 32 << 20          # 128 MiB of split-K partials per (device, stream
 
 
 def _workspace(device: torch.device) -> torch.Tensor:
-    key = (device.index or 0, torch.cuda.current_stream().cuda_stream)
+    key = (device.index or 0, current_stream())
     t = _ws.get(key)
     if t is None:
         t = _ws[key] = torch.empty(_WS_FLOATS, dtype=torch.float32, device=device)
@@ -434,7 +435,7 @@ def linear_wide(x: torch.Tensor, w: torch.Tensor, splits: int = 0, swiglu: bool 
     ws = _workspace(x.device)
     if s > 1 and s * m * n > ws.numel():
         s = max(1, ws.numel() // (m * n))
-    stream = torch.cuda.current_stream().cuda_stream
+    stream = current_stream()
     bm = wide_row_tile(m, n, k, swiglu)
     v = variant if variant >= 0 else wide_variant(m, n, k, s, bm)
     if bm != wide_bm(m):
@@ -473,7 +474,7 @@ def linear_pp(x: torch.Tensor, w: torch.Tensor, splits: int = 0, swiglu: bool = 
     ws = _workspace(x.device)
     if s > 1 and s * m * n > ws.numel():
         s = max(1, ws.numel() // (m * n))
-    stream = torch.cuda.current_stream().cuda_stream
+    stream = current_stream()
     if defer and not swiglu and s > 1:
         se = _ext.kernels().gemm_pp(0, x.data_ptr(), w.data_ptr(), ws.data_ptr(), ws.numel(), m, n, k, s, 2, variant,
                                     stream)
@@ -509,7 +510,7 @@ def linear_pf(x: torch.Tensor, w: torch.Tensor, swiglu: bool = False, variant: i
     if dyn:
         variant |= 16                  # per-XCD dynamic tile queues (gemm_pp.hip, DYN)
     _ext.kernels().gemm_pf(y.data_ptr(), x.data_ptr(), w.data_ptr(), m, n, k,
-                           4 if gelu else 3 if limit is not None else (1 if swiglu else 0), variant, torch.cuda.current_stream().cuda_stream,
+                           4 if gelu else 3 if limit is not None else (1 if swiglu else 0), variant, current_stream(),
                            0.0 if limit is None else float(limit), bm)
     return y
 
@@ -562,7 +563,7 @@ def linear_sq(x: torch.Tensor, w: torch.Tensor, splits: int = 0, swiglu: bool = 
     ws = _workspace(x.device)
     if s > 1 and s * m * n > ws.numel():
         s = max(1, ws.numel() // (m * n))
-    stream = torch.cuda.current_stream().cuda_stream
+    stream = current_stream()
     v = knobs.K.sq_variant if variant < 0 else variant
     if defer and not swiglu and s > 1:
         se = _ext.kernels().gemm_sq(0, x.data_ptr(), w.data_ptr(), ws.data_ptr(), ws.numel(), m, n, k, s, 2, v,
@@ -592,7 +593,7 @@ def _linear_glu(x: torch.Tensor, w_gate_up: torch.Tensor, limit: Optional[float]
     y = linear(x, w_gate_up, defer=True)
     if isinstance(y, SplitKPartial):
         out = torch.empty(*x.shape[:-1], n // 2, dtype=x.dtype, device=x.device)
-        st = torch.cuda.current_stream().cuda_stream
+        st = current_stream()
         if limit is None:
             _ext.kernels().splitk_reduce_gelu(out.data_ptr(), y.ws.data_ptr(), y.splits, y.m, y.n, st)
         else:

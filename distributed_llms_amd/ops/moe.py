@@ -22,6 +22,7 @@ import torch.nn.functional as F
 
 from .. import _ext, knobs
 from . import reference as ref
+from .stream import current_stream
 
 GROUPED_MAX_TOKENS = 256      # beyond this the per-expert row count makes library GEMMs cheaper
 ROUTER_FUSED_MAX_TOKENS = 64  # up to this many tokens the grouped-choice router product runs inside the selection kernel
@@ -62,7 +63,7 @@ def forward(x: torch.Tensor, w_router: torch.Tensor, w_gate_up: torch.Tensor, w_
         return ref.moe_mlp(x, w_gate_up, w_down, tw, tid - expert_offset)
     from . import linear, linear_swiglu
     k = _ext.kernels()
-    st = torch.cuda.current_stream().cuda_stream
+    st = current_stream()
     t, h = x.shape
     e_loc, two_i, _ = w_gate_up.shape
     e = e_all
@@ -199,7 +200,7 @@ def grouped_choice_ffn(x: torch.Tensor, w_router: torch.Tensor, correction: Opti
         return out.to(x.dtype)
     from . import linear
     k = _ext.kernels()
-    st = torch.cuda.current_stream().cuda_stream
+    st = current_stream()
     dev = x.device
     f32 = 1 if x.dtype == torch.float32 else 0
     if not (x.is_contiguous() and w_up.is_contiguous() and w_down.is_contiguous() and w_router.is_contiguous()):
@@ -280,7 +281,7 @@ def relu_sq_(y: torch.Tensor) -> torch.Tensor:
     if not y.is_contiguous() or y.dtype not in (torch.bfloat16, torch.float32):
         raise ValueError("relu_sq_: contiguous bfloat16 or float32")
     _ext.kernels().relu_sq(y.data_ptr(), y.numel(), 1 if y.dtype == torch.float32 else 0,
-                           torch.cuda.current_stream().cuda_stream)
+                           current_stream())
     return y
 
 
@@ -356,7 +357,7 @@ def softmax_top_ffn(x: torch.Tensor, w_router: torch.Tensor, b_router: Optional[
     from . import linear
     from .latent import linear_swiglu
     k = _ext.kernels()
-    st = torch.cuda.current_stream().cuda_stream
+    st = current_stream()
     dev = x.device
     f32 = 1 if x.dtype == torch.float32 else 0
     if not (x.is_contiguous() and w_gate_up.is_contiguous() and w_down.is_contiguous() and w_router.is_contiguous()):

@@ -27,6 +27,7 @@ from typing import Tuple
 import torch
 
 from .. import _ext, knobs
+from .stream import current_stream
 
 FP8 = torch.float8_e4m3fn
 FP8_MAX = 448.0
@@ -174,7 +175,7 @@ def quantize_rows(x: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
     q = torch.empty(m, k, dtype=FP8, device=x.device)
     s = torch.empty(m, dtype=torch.float32, device=x.device)
     _ext.kernels().quant_fp8_rows(q.data_ptr(), s.data_ptr(), x.data_ptr(), m, k,
-                                  torch.cuda.current_stream().cuda_stream)
+                                  current_stream())
     return q, s
 
 
@@ -253,7 +254,7 @@ def linear_fp8(x: torch.Tensor, w: Fp8Weight, swiglu: bool = False, defer: bool 
         s = max(1, ws.numel() // (m * n))
     # weights streamed non-temporal only where one row tile covers M (each weight byte read once)
     variant = (1 if m <= 256 else (4 | (64 if 0 < knobs.K.fp8_group_m <= m else 0))) | (bm << 8)
-    stream = torch.cuda.current_stream().cuda_stream
+    stream = current_stream()
     kern = _ext.kernels()
     if defer and not swiglu and s > 1:
         se = kern.gemm_wide_fp8(0, xq.data_ptr(), xs.data_ptr(), w.q.data_ptr(), w.scale.data_ptr(), ws.data_ptr(),

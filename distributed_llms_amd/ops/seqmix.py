@@ -31,6 +31,7 @@ from typing import Optional, Tuple
 import torch
 
 from .. import _ext
+from .stream import current_stream as _stream
 
 ACT_DTYPES = (torch.bfloat16, torch.float32)
 SCAN_SEGMENT = 128        # tokens per segment of the segmented RG-LRU scan (kSeg in seqmix.hip)
@@ -47,10 +48,6 @@ class SeqBatch:
     num_seqs: int
     num_tokens: int
     max_q_len: int
-
-
-def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
 
 
 def _k():
