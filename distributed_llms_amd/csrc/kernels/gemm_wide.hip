@@ -763,12 +763,13 @@ int gemm_wide(uintptr_t c, uintptr_t a, uintptr_t b, uintptr_t ws, long ws_float
     else if (pf) { if (variant == 2) DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 130, 3); else DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 129, 3); } \
     else if (frag) { if (variant == 2) DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 34, 3); else DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 33, 3); } \
     else if (variant == 0) DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 0, 3);                                              \
-    else if (variant == 2) DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 2, 3);                                              \
+    else if (variant == 2) { if (BM_ == 64 && grid <= 256) DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 2, (BM_ == 64 ? 6 : 3)); else DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 2, 3); } \
     else if (variant == 3) DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 3, 3);                                              \
     else DLLM_WIDE_GO3(BM_, SPLIT_, SW_, 1, 3);                                                                \
   } while (0)
   // BM = 64 and a grid of one round: the ring as deep as the LDS allows (6 x 24 KiB, five K-tiles in flight: 38.5 vs
-  // 40.0 us for the 8B gate|up at M = 64, 36.5 vs 36.8 at M = 1); with more workgroups than CUs two 3-slot
+  // 40.0 us for the 8B gate|up at M = 64, 36.5 vs 36.8 at M = 1; split with the norm behind it, M = 1 / 32 / 64: 4096 x 14336
+  // 23.1 / 24.4 / 26.0 -> 23.2 / 24.0 / 25.3, 8192 x 8192 34.7 / 34.8 / 36.5 -> 33.0 / 34.3 / 36.0); with more workgroups than CUs two 3-slot
   // workgroups per CU are as good, and from 128 rows on the MFMAs hide what the depth would
 #define DLLM_WIDE_ROT(BM_, SW_)                                                                                \
   do {                                                                                                         \

@@ -209,7 +209,7 @@ def fp8_plan(m: int, n: int, k: int, swiglu: bool = False) -> Tuple[int, int]:
     10.0 / 10.4 -> 7.6 / 8.6 / 9.0 (4 slices), 4096 x 4096 10.0 / 10.8 / 11.5 -> 9.0 / 10.1 / 11.3; 16 slices 10-14, and
     6144 x 4096 in 5 instead of 4 10.9 / 11.9 / 12.9 -> 11.2 / 12.3 / 13.6."""
     from . import gemm
-    s = gemm.wide_splits(m, n, k // 2, swiglu)
+    s = gemm.wide_splits(m, n, k // 2, swiglu, short=False)
     if m <= 64 and not swiglu and s > 1 and not gemm._comm_cus:
         c = min(8, 256 // (n // 128), (k // 128) // 4)
         if c >= 2 * s:

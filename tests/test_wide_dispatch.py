@@ -332,3 +332,12 @@ def test_pf_row_tile_takes_the_cheapest_walk():
         assert gemm._pf_plan(7021, 2560, 2560, 2560, cpu) in (0, 256)
     finally:
         gemm.release_cus_for_comm()
+
+
+def test_wide_splits_take_short_slices_up_to_128_rows():
+    """Up to 8 slices of 4 K-tiles for split products of up to 128 rows; unsplit ones stay unsplit, and nothing else moves."""
+    assert gemm.wide_splits(32, 2560, 2560) == 8 and gemm.wide_splits(128, 2560, 2048) == 8
+    assert gemm.wide_splits(129, 2560, 2560) == 5 and gemm.wide_splits(32, 2560, 2560, short=False) == 5
+    assert gemm.wide_splits(32, 1024, 1024) == 4 and gemm.wide_splits(32, 1024, 512) == 1
+    assert gemm.wide_splits(64, 4096, 4096) == 8 and gemm.wide_splits(64, 6144, 4096) == 5
+    assert gemm.wide_splits(64, 2560, 7680) == 13 and gemm.wide_splits(64, 8192, 28672) == 4
