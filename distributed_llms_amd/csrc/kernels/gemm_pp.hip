@@ -148,28 +148,30 @@ __device__ __forceinline__ int pp_b_row(int r, int n_t, int half) {
 }
 }  // namespace
 
-// MODE 0: C bf16 [M, N];  1: split-K slab P (f16 x 2^-6, common.h) [S, M, N];  2: SwiGLU C [M, N/2];
+// One tile of 32 RT rows.  MODE 0: C bf16 [M, N];  1: split-K slab P (f16 x 2^-6, common.h) [S, M, N];  2: SwiGLU C [M, N/2];
 // 3: C = max(A B^T, 0)^2 (the activation of two-matrix experts, in the epilogue).
 // VAR bit 0: weights nontemporal (read once); bit 1: grouped row-tile order (prefill, no split).
-template <int BN, int MODE, int VAR>
-__global__ void __launch_bounds__(256, 1) gemm_pp_kernel(const bf16* __restrict__ A, const bf16* __restrict__ B,
-                                                         bf16* __restrict__ C, float* __restrict__ P, int M, int N,
-                                                         int K, int ks_per_split, int nsplit, float* __restrict__ D,
-                                                         const int* __restrict__ gather, const int* __restrict__ counts,
-                                                         const int* __restrict__ offsets, int E, float limit = 0.f) {
+// The tile's rows: [r0, min(r0 + BM, rcnt)) of the row range that starts at slot roff (dense: roff 0, rows r0 .. M), off the
+// rows gather[slot] of A where there is a gather.
+template <int BN, int MODE, int VAR, int RT, int SMEM>
+__device__ __forceinline__ void gemm_pp_tile(bf16 (&smem)[SMEM], const bf16* __restrict__ A, const bf16* __restrict__ We,
+                                             bf16* __restrict__ C, float* __restrict__ P, int M, int N, int K, int n_t,
+                                             int r0, int rcnt, int roff, const int* __restrict__ gather, int split,
+                                             int ks0, int nt, float* __restrict__ D, float limit) {
   constexpr int NW = 4, NWN = 2;
-  constexpr int BM = 256, TM = 128, TN = BN / NWN;     // waves as 2 (M) x NWN (N)
-  constexpr int RT = TM / 16, CT = TN / 16;            // 16 x 16 fragments per wave: 8 x 8 or 8 x 4
+  constexpr int TM = 16 * RT, BM = 2 * TM, TN = BN / NWN;      // waves as 2 (M) x NWN (N)
+  constexpr int CT = TN / 16;                          // 16 x 16 fragments per wave: up to 8 x 8 or 8 x 4
   constexpr int SLOT = (BM + BN) * PBK;                // bf16 elements per ring slot (one K-tile)
-  constexpr int NB = BN == 256 ? 2 : 3;                // K-tiles held in LDS
+  constexpr int NB = BN == 256 && RT > 5 ? 2 : 3;      // K-tiles held in LDS
   constexpr int GA = BM * PBK * 2 / 1024 / NW, GB = BN * PBK * 2 / 1024 / NW;  // glds per wave per K-tile
   constexpr int G = GA + GB;
-  constexpr bool NT = (VAR & 1) != 0, GROUPED = (VAR & 2) != 0;
+  constexpr bool NT = (VAR & 1) != 0;
   constexpr bool PROF = (VAR & 4) != 0;                // diagnostic build: cycle stamps around B_t
   // schedule 2 (VAR 32): a K-tile's fragments are all read into registers early in its first K-half,
   // so its slot is re-staged from then on -- LDS-DMA pieces spread over ~60 % of the K-tile instead
   // of bunched into half of K-half 1 (see the loop)
   constexpr bool SCHED2 = (VAR & 32) != 0;
+  static_assert(RT == 8 || SCHED2, "row tiles below 256: schedule 2");
   constexpr bool SWIGLU = MODE == 2;
   // VAR bit 9, with SwiGLU on schedule 2: the clipped GLU of `limit` (common.h) instead of silu(g) * u
   constexpr bool CLIPPED = (VAR & 512) != 0;
@@ -180,62 +182,16 @@ __global__ void __launch_bounds__(256, 1) gemm_pp_kernel(const bf16* __restrict_
   constexpr bool SWI2 = SWIGLU && SCHED2;
   constexpr int IMGW = SWI2 ? BN : OUTW;               // LDS image width (elements)
   constexpr int OPITCH = IMGW + 8;                     // LDS output row pitch (elements): +16 B
-  constexpr int SMEM = NB * SLOT > BM * OPITCH ? NB * SLOT : BM * OPITCH;   // ring, then output image
-  static_assert(SMEM * 2 <= 160 * 1024, "LDS");
-  __shared__ __attribute__((aligned(16))) bf16 smem[SMEM];
+  static_assert(NB * SLOT <= SMEM && BM * OPITCH <= SMEM && SMEM * 2 <= 160 * 1024, "LDS: ring, then output image");
 
+  constexpr bool MOE = (VAR & 128) != 0;
   [[maybe_unused]] unsigned long long rt_entry = 0, rt_loop0 = 0, rt_loop1 = 0;
   if constexpr (PROF) rt_entry = __builtin_amdgcn_s_memrealtime();
-  const int tid = threadIdx.x, lane = tid & 63;
+  int tid = threadIdx.x;
+  if constexpr (MOE) asm volatile("" : "+v"(tid));     // nothing of one row tile's code is hoisted in front of all
+  const int lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wv / NWN, wn = wv % NWN;
-  // MOE (VAR 128): grouped expert GEMM -- the row tiles of every expert's segment of the
-  // expert-sorted slot space, counts / offsets read on the device (no host sync); the grid holds an
-  // upper bound of row tiles (slots / 256 + E), the surplus workgroups exit at once
-  constexpr bool MOE = (VAR & 128) != 0;
-  const int ntiles = N / BN;
-  const int mtiles = MOE ? (int)(gridDim.x / ntiles) : (M + BM - 1) / BM;
-  const int total = gridDim.x;
-  int b = blockIdx.x;
-  {   // bijective XCD remap: consecutive logical blocks share an XCD
-    const int q = total >> 3, r = total & 7, x = b & 7;
-    b = (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + (b >> 3);
-  }
-  int m_t, n_t, split;
-  if constexpr (GROUPED) {
-    const int per = 8 * ntiles, g = b / per, first = g * 8, gsz = min(mtiles - first, 8);
-    m_t = first + (b % per) % gsz;
-    n_t = (b % per) / gsz;
-    split = 0;
-  } else {
-    m_t = b % mtiles;
-    const int rest = b / mtiles;
-    split = rest % nsplit;
-    n_t = rest / nsplit;
-  }
-  const int m0 = m_t * BM;
-  // the tile's rows: [r0, min(r0 + BM, rcnt)) of the row range that starts at slot roff (dense:
-  // roff 0, rows m0 .. M); MOE: expert ex's segment, its weight We = B + ex N K
-  int r0 = m0, rcnt = M, roff = 0;
-  const bf16* We = B;
-  if constexpr (MOE) {
-    int base = 0, ex = -1;
-    for (int x = 0; x < E; ++x) {
-      const int c = counts[x], nx = (c + BM - 1) / BM;
-      if (ex < 0 && m_t < base + nx) {
-        ex = x;
-        r0 = (m_t - base) * BM;
-        rcnt = c;
-      }
-      base += nx;
-    }
-    if (ex < 0) return;                                // past the last real row tile (uniform)
-    roff = offsets[ex];
-    We = B + (size_t)ex * N * K;
-  }
-  const int ks0 = split * ks_per_split;
-  const int nt = max(0, min(K / PBK, ks0 + ks_per_split) - ks0);
-
   // staging sources: wave-instruction i covers 8 slot rows, lane -> (row 8 i + lane / 8,
   // physical chunk lane % 8) <- logical chunk pswz(row, lane % 8) of the source row.  Byte
   // offsets are 32-bit from a wave-uniform base (operands < 4 GiB, checked on the host): one VGPR
@@ -256,7 +212,7 @@ __global__ void __launch_bounds__(256, 1) gemm_pp_kernel(const bf16* __restrict_
       const int slot = roff + min(r0 + r, rcnt - 1);
       srow = gather ? gather[slot] : slot;
     } else {
-      srow = min(m0 + r, M - 1);
+      srow = min(r0 + r, M - 1);
     }
     offA[j] = (uint32_t)srow * (uint32_t)(K * 2) + chunk_q[q & 1];
   }
@@ -548,7 +504,9 @@ __global__ void __launch_bounds__(256, 1) gemm_pp_kernel(const bf16* __restrict_
   // acc[rt][ct] lane l holds C[row wm*TM + rt*16 + (l & 15)][col wn*TN + ct*16 + 4*(l >> 4) + v]
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  const int lr = lane & 15, lq = lane >> 4;
+  // (the lane from the hardware again, so that no register holds it through the loop)
+  const int le = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), te = wv * 64 + le;
+  const int lr = le & 15, lq = le >> 4;
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
     const int row = wm * TM + rt * 16 + lr;
@@ -591,7 +549,7 @@ __global__ void __launch_bounds__(256, 1) gemm_pp_kernel(const bf16* __restrict_
   __syncthreads();
   constexpr int CPR = OUTW / 8;                        // 16-byte chunks per output row
   constexpr int RPI = 64 * NW / CPR;                   // rows per pass
-  const int ch = tid % CPR, rs0 = tid / CPR;
+  const int ch = te % CPR, rs0 = te / CPR;
   const int ldc = SWIGLU ? N / 2 : N;
   const int col0 = n_t * OUTW + ch * 8;
   // SWI2: output columns 8 ch .. 8 ch + 7 sit in 16-column group ch / 2 -> gate at image column
@@ -626,6 +584,83 @@ __global__ void __launch_bounds__(256, 1) gemm_pp_kernel(const bf16* __restrict_
     const double v8[6] = {(double)rt_entry, (double)rt_loop0, (double)rt_loop1, (double)rt_end, (double)hw, (double)xcc};
     double* rec = reinterpret_cast<double*>(D + ((size_t)blockIdx.x * 4 + wv) * 128 + 8);
     if (lane < 6) rec[lane] = v8[lane < 6 ? lane : 0];
+  }
+}
+
+constexpr int pp_smem(int bn, int mode, int var) {      // bf16 elements: ring, then output image
+  const int ring = bn == 256 ? (var & 128 ? 3 * (128 + 256) * PBK : 2 * (256 + 256) * PBK) : 3 * (256 + bn) * PBK;
+  const int image = 256 * ((mode == 2 && (var & 32) == 0 ? bn / 2 : bn) + 8);
+  return ring > image ? ring : image;
+}
+
+template <int BN, int MODE, int VAR>
+__global__ void __launch_bounds__(256, 1) gemm_pp_kernel(const bf16* __restrict__ A, const bf16* __restrict__ B,
+                                                         bf16* __restrict__ C, float* __restrict__ P, int M, int N,
+                                                         int K, int ks_per_split, int nsplit, float* __restrict__ D,
+                                                         const int* __restrict__ gather, const int* __restrict__ counts,
+                                                         const int* __restrict__ offsets, int E, float limit = 0.f) {
+  constexpr int BM = 256;
+  constexpr bool GROUPED = (VAR & 2) != 0;
+  __shared__ __attribute__((aligned(16))) bf16 smem[pp_smem(BN, MODE, VAR)];
+  // MOE (VAR 128): grouped expert GEMM -- the row tiles of every expert's segment of the
+  // expert-sorted slot space, counts / offsets read on the device (no host sync); the grid holds an
+  // upper bound of row tiles (slots / 256 + E), the surplus workgroups exit at once.  The order is that of the real
+  // tiles: dealt over the upper bound, the last XCDs had the surplus and the others half as many tiles again as their share
+  constexpr bool MOE = (VAR & 128) != 0;
+  const int ntiles = N / BN;
+  int mtiles = (M + BM - 1) / BM, total = gridDim.x;
+  if constexpr (MOE) {
+    mtiles = 0;
+    for (int x = 0; x < E; ++x) mtiles += (counts[x] + BM - 1) / BM;
+    total = mtiles * ntiles;
+  }
+  int b = blockIdx.x;
+  {   // bijective XCD remap: consecutive logical blocks share an XCD
+    const int q = total >> 3, r = total & 7, x = b & 7;
+    if (MOE && (b >> 3) >= q + (x < r)) return;        // (uniform) past the real tiles
+    b = (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + (b >> 3);
+  }
+  int m_t, n_t, split;
+  if constexpr (GROUPED) {
+    const int per = 8 * ntiles, g = b / per, first = g * 8, gsz = min(mtiles - first, 8);
+    m_t = first + (b % per) % gsz;
+    n_t = (b % per) / gsz;
+    split = 0;
+  } else {
+    m_t = b % mtiles;
+    const int rest = b / mtiles;
+    split = rest % nsplit;
+    n_t = rest / nsplit;
+  }
+  const int ks0 = split * ks_per_split;
+  const int nt = max(0, min(K / PBK, ks0 + ks_per_split) - ks0);
+  if constexpr (MOE) {
+    int base = 0, ex = 0, r0 = 0, rcnt = 0;
+    for (int x = 0; x < E; ++x) {
+      const int c = counts[x], nx = (c + BM - 1) / BM;
+      if (m_t >= base && m_t < base + nx) {
+        ex = x;
+        r0 = (m_t - base) * BM;
+        rcnt = c;
+      }
+      base += nx;
+    }
+    const int roff = offsets[ex];
+    const bf16* We = B + (size_t)ex * N * K;
+    // a segment's last tile on the row tile that holds what is left (neighbour of the segment's others in the order: put
+    // last, its weight tiles came from memory again).  Both, us, Mixtral gate|up / down, 300 tokens 504 / 282 -> 373 / 250,
+    // 2036 1035 / 604 -> 874 / 605, 8192 3188 / 1695 -> 2861 / 1618; 64 experts 2048 x 1408, 6 a token, 4096 tokens 393 / 215
+    // -> 334 / 183
+    const int left = rcnt - r0;
+    auto go = [&](auto rt) {
+      gemm_pp_tile<BN, MODE, VAR, decltype(rt)::value>(smem, A, We, C, P, M, N, K, n_t, r0, rcnt, roff, gather, split, ks0, nt,
+                                                       D, limit);
+    };
+    if (left <= 128) go(std::integral_constant<int, 4>{});
+    else if (left <= 192) go(std::integral_constant<int, 6>{});
+    else go(std::integral_constant<int, 8>{});
+  } else {
+    gemm_pp_tile<BN, MODE, VAR, 8>(smem, A, B, C, P, M, N, K, n_t, m_t * BM, M, 0, nullptr, split, ks0, nt, D, limit);
   }
 }
 
@@ -715,22 +750,15 @@ void gemm_pp_moe(uintptr_t y, uintptr_t x, uintptr_t gather, uintptr_t w, uintpt
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const long grid = (long)(N / 256) * ((slots + 255) / 256 + E);
   DLLM_HOST_CHECK(grid < (1L << 31), "grid");
-  if (mode == 1)
-    hipLaunchKernelGGL((gemm_pp_kernel<256, 2, 128 | 32 | 2>), dim3((unsigned)grid), dim3(256), 0, s, (const bf16*)x,
-                       (const bf16*)w, (bf16*)y, (float*)nullptr, xrows, N, K, K / PBK, 1, (float*)nullptr,
-                       (const int*)gather, (const int*)counts, (const int*)offsets, E, limit);
-  else if (mode == 3)
-    hipLaunchKernelGGL((gemm_pp_kernel<256, 2, 512 | 128 | 32 | 2>), dim3((unsigned)grid), dim3(256), 0, s, (const bf16*)x,
-                       (const bf16*)w, (bf16*)y, (float*)nullptr, xrows, N, K, K / PBK, 1, (float*)nullptr,
-                       (const int*)gather, (const int*)counts, (const int*)offsets, E, limit);
-  else if (mode == 2)
-    hipLaunchKernelGGL((gemm_pp_kernel<256, 3, 128 | 32 | 2>), dim3((unsigned)grid), dim3(256), 0, s, (const bf16*)x,
-                       (const bf16*)w, (bf16*)y, (float*)nullptr, xrows, N, K, K / PBK, 1, (float*)nullptr,
-                       (const int*)gather, (const int*)counts, (const int*)offsets, E, limit);
-  else
-    hipLaunchKernelGGL((gemm_pp_kernel<256, 0, 128 | 32 | 2>), dim3((unsigned)grid), dim3(256), 0, s, (const bf16*)x,
-                       (const bf16*)w, (bf16*)y, (float*)nullptr, xrows, N, K, K / PBK, 1, (float*)nullptr,
-                       (const int*)gather, (const int*)counts, (const int*)offsets, E, limit);
+#define DLLM_PPM(MODE_, VAR_)                                                                                         \
+  hipLaunchKernelGGL((gemm_pp_kernel<256, MODE_, VAR_>), dim3((unsigned)grid), dim3(256), 0, s, (const bf16*)x,        \
+                     (const bf16*)w, (bf16*)y, (float*)nullptr, xrows, N, K, K / PBK, 1, (float*)nullptr,             \
+                     (const int*)gather, (const int*)counts, (const int*)offsets, E, limit)
+  if (mode == 1) DLLM_PPM(2, 128 | 32 | 2);
+  else if (mode == 3) DLLM_PPM(2, 512 | 128 | 32 | 2);
+  else if (mode == 2) DLLM_PPM(3, 128 | 32 | 2);
+  else DLLM_PPM(0, 128 | 32 | 2);
+#undef DLLM_PPM
   DLLM_HIP_CHECK(hipGetLastError());
 }
 
@@ -751,9 +779,10 @@ void gemm_pp_moe(uintptr_t y, uintptr_t x, uintptr_t gather, uintptr_t w, uintpt
 // tile = w + i P by P = gridDim.x workgroups, w the XCD-aware rank (workgroup b runs on XCD b % 8;
 // w = (b % 8) (P / 8) + b / 8), so each XCD's L2 serves 32 consecutive tiles of the grouped order
 // (8 row tiles x 4 column tiles) at a time.
-// Row tile BM = 32 RT (160 .. 256): a K-tile of 64 takes 1.47 / 1.31 / 1.18 / 1.04 us at 256 / 224 / 192 / 160 rows, the sum
+// Row tile BM = 32 RT (160 .. 256): a K-tile of 64 takes 1.47 / 1.31 / 1.18 / 1.02 us at 256 / 224 / 192 / 160 rows, the sum
 // of its MFMAs and its LDS traffic, so 256 rows are the most efficient and the shorter tiles are for grids that they fit into
-// fewer or cheaper rounds of the chip (ops/gemm.pf_row_tile has the rule and its figures).  Every row's sum over K is in the
+// fewer or cheaper rounds of the chip (ops/gemm.pf_row_tile has the rule and its figures).  160 rows leave room for a third
+// slot, which a shorter K-tile needs (4096 x 14336 at 2560 rows, one round: 253 -> 234 us).  Every row's sum over K is in the
 // same order whatever the tile.
 //
 // MODE 0: C bf16 [M, N];  2: SwiGLU C [M, N / 2] with B = [Bg; Bu] (row groups as pp_b_row);  4: the clipped GLU of
@@ -820,7 +849,7 @@ __global__ void __launch_bounds__(256, 1) gemm_pf_kernel(const bf16* __restrict_
                                                          int* __restrict__ queue, float limit) {
   constexpr int NW = 4, NWN = 2, TM = 16 * RT, BM = 2 * TM, BN = 256, TN = BN / NWN;
   constexpr int CT = TN / 16;                          // RT x 8 accumulators per wave
-  constexpr int SLOT = (BM + BN) * PBK, NB = 2;        // ring of two K-tiles: 2 x 64 KiB at BM = 256
+  constexpr int SLOT = (BM + BN) * PBK, NB = RT > 5 ? 2 : 3;   // ring: 2 x 64 KiB at BM = 256, 3 x 52 KiB at 160
   constexpr int GA = BM * PBK * 2 / 1024 / NW, GB = BN * PBK * 2 / 1024 / NW, G = GA + GB;
   constexpr bool CLIPPED = MODE == 4, GELU = MODE == 5, SWIGLU = MODE == 2 || CLIPPED || GELU;
   constexpr int OUTW = SWIGLU ? BN / 2 : BN;           // output tile width (elements)

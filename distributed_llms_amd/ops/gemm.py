@@ -91,7 +91,7 @@ def pf_fills(m: int, n: int, device) -> bool:
 # us, 256 / 224 / 192 / 160 rows: 2560 x 2560, M = 7021 (280 / 320 / 370 / 440 tiles) 108 / 99 / 95 / 84; 4096 x 4096, 6210
 # (400 / 448 / 528 / 624) 183 / 165 / 204 / 187; 6144 x 4096, 3072 (288 / 336 / 384 / 480) 172 / 153 / 146 / 136; 4096 x 14336,
 # 5120 (320 / 368 / 432 / 512) 584 / 554 / 522 / 493; gate|up 28672 x 4096, 384 (224 / 224 / 224 / 336) 97 / 87 / 83 / 140.
-# 128 rows (1.0 us a K-tile against 1.04 for 160) never win where there is no K split.
+# 128 rows (1.0 us a K-tile against 1.02 for 160) never win where there is no K split.
 _PF_ROUND = {256: 1.0, 224: 0.93, 192: 0.84, 160: 0.76}
 
 

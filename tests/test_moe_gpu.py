@@ -1,6 +1,7 @@
 """Mixtral MoE on the GPU (route + grouped expert GEMMs + combine) vs the fp32 PyTorch reference."""
 import pytest
 import torch
+import torch.nn.functional as F
 
 from distributed_llms_amd import ops
 from distributed_llms_amd.ops import moe
@@ -169,6 +170,41 @@ def test_moe_prefill_grouped_gemm(cuda, t, e, k, h, i, skew):
     expect = ref.moe_mlp(x.float(), wgu.float(), wd.float(), tw, tid)
     tol = 2e-2 * expect.abs().max().item()
     torch.testing.assert_close(out.float(), expect, atol=tol, rtol=3e-2)
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2, 3])
+def test_moe_grouped_gemm_last_tiles(cuda, mode):
+    """Segments whose last row tile holds 1 .. 256 rows, on either side of the 128- and 192-row tiles, with empty experts
+    between, gathered and not: against each segment's own f32 product, nothing written past the segments."""
+    from distributed_llms_amd import _ext
+    counts = [1, 128, 0, 129, 192, 193, 255, 256, 257, 384, 0, 385, 448, 449, 513]
+    e, k, n = len(counts), 192, 512
+    slots, tokens = sum(counts), 700
+    x = _bf(tokens, k)
+    w = _bf(e, n, k, scale=0.1)
+    gather = torch.randint(0, tokens, (slots,), device="cuda", dtype=torch.int32)
+    c = torch.tensor(counts, dtype=torch.int32, device="cuda")
+    off = torch.cumsum(c, 0).to(torch.int32) - c
+    glu = mode in (1, 3)
+    y = torch.full((slots + 8, n // 2 if glu else n), 7.0, dtype=torch.bfloat16, device="cuda")
+    _ext.kernels().gemm_pp_moe(y.data_ptr(), x.data_ptr(), gather.data_ptr(), w.data_ptr(), c.data_ptr(), off.data_ptr(), e, n, k,
+                               tokens, slots, mode, torch.cuda.current_stream().cuda_stream, 0.7)
+    assert bool((y[slots:] == 7.0).all())
+    at = 0
+    for i, m in enumerate(counts):
+        z = x[gather[at:at + m].long()].float() @ w[i].float().t()
+        if mode == 2:
+            z = z.clamp(min=0) ** 2
+        elif glu:                       # gate and up are rounded to bf16 before the activation
+            g, u = z[:, :n // 2].bfloat16().float(), z[:, n // 2:].bfloat16().float()
+            if mode == 1:
+                z = F.silu(g) * u
+            else:
+                g, u = g.clamp(max=0.7), u.clamp(-0.7, 0.7)
+                z = g * torch.sigmoid(1.702 * g) * (u + 1)
+        # bf16 result (and, under a GLU, a gate or up that rounds the other way: as much again, twice)
+        torch.testing.assert_close(y[at:at + m].float(), z, atol=2e-2, rtol=2e-2)
+        at += m
 
 
 def test_moe_prefill_has_no_host_sync(cuda):
