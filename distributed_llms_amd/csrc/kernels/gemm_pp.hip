@@ -786,7 +786,10 @@ void gemm_pp_moe(uintptr_t y, uintptr_t x, uintptr_t gather, uintptr_t w, uintpt
 // same order whatever the tile.
 //
 // MODE 0: C bf16 [M, N];  2: SwiGLU C [M, N / 2] with B = [Bg; Bu] (row groups as pp_b_row);  4: the clipped GLU of
-// `limit` (common.h) in the same layout;  5: its gelu GLU.
+// `limit` (common.h) in the same layout;  5: its gelu GLU;  6: 4 of the products + bias [gate | up], each lane's
+// CT / 2 x 8 bytes per half loaded once per tile.  Mode 6 took the gate kernel's pass over C (read M N, write M N / 2) away: 6376 x
+// 15360 x 2560 434 -> 363 us (mode 0 alone 360); with the gate kernel's expf and division in the epilogue 396, and the
+// error against float64 is the same either way (mean 1.13e-3, 1.71e-3 before, when the product was rounded to bf16 first).
 // SCH 8: nontemporal output stores (large SwiGLU outputs), else 0.  The schedule sweeps of rounds 3-5
 // (barrier positions, piece spacing, row-group widths, and the split A / B LDS release of round 5,
 // all within 0.5 % of this schedule: profiles/round5_raw/r5d_pf_sched.txt) were removed.
@@ -846,12 +849,13 @@ __device__ void pf_retire(int* q, int grid) {                      // lane 0, on
 template <int MODE, int SCH = 0, bool DYN = false, int RT = 8>
 __global__ void __launch_bounds__(256, 1) gemm_pf_kernel(const bf16* __restrict__ A, const bf16* __restrict__ B,
                                                          bf16* __restrict__ C, int M, int N, int K,
-                                                         int* __restrict__ queue, float limit) {
+                                                         int* __restrict__ queue, float limit,
+                                                         const bf16* __restrict__ bias) {
   constexpr int NW = 4, NWN = 2, TM = 16 * RT, BM = 2 * TM, BN = 256, TN = BN / NWN;
   constexpr int CT = TN / 16;                          // RT x 8 accumulators per wave
   constexpr int SLOT = (BM + BN) * PBK, NB = RT > 5 ? 2 : 3;   // ring: 2 x 64 KiB at BM = 256, 3 x 52 KiB at 160
   constexpr int GA = BM * PBK * 2 / 1024 / NW, GB = BN * PBK * 2 / 1024 / NW, G = GA + GB;
-  constexpr bool CLIPPED = MODE == 4, GELU = MODE == 5, SWIGLU = MODE == 2 || CLIPPED || GELU;
+  constexpr bool BIASED = MODE == 6, CLIPPED = MODE == 4 || BIASED, GELU = MODE == 5, SWIGLU = MODE == 2 || CLIPPED || GELU;
   constexpr int OUTW = SWIGLU ? BN / 2 : BN;           // output tile width (elements)
   typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -1071,6 +1075,15 @@ __global__ void __launch_bounds__(256, 1) gemm_pf_kernel(const bf16* __restrict_
     int m_t, n_t;
     tile_mn(tile_of(ti), m_t, n_t);
     const uint32_t colb = (uint32_t)(n_t * OUTW + wn * (OUTW / NWN) + 16 * (lq & 1) + 8 * (lq >> 1)) * 2;
+    [[maybe_unused]] bf16x4 bg[CT / 2], bu[CT / 2];    // biases of this lane's columns
+    if constexpr (BIASED) {
+#pragma unroll
+      for (int i = 0; i < CT / 2; ++i) {
+        const bf16* at = bias + n_t * OUTW + wn * (OUTW / NWN) + 16 * i + 4 * lq;
+        bg[i] = *reinterpret_cast<const bf16x4*>(at);
+        bu[i] = *reinterpret_cast<const bf16x4*>(at + N / 2);
+      }
+    }
 #pragma unroll
     for (int r = 0; r < RT; ++r) {
       // pin row r's accumulators in AGPRs up to here: hipcc would otherwise copy all 256 to VGPRs
@@ -1088,7 +1101,10 @@ __global__ void __launch_bounds__(256, 1) gemm_pf_kernel(const bf16* __restrict_
           const f32x4 g = acc[r][2 * i], u = acc[r][2 * i + 1];
 #pragma unroll
           for (int v = 0; v < 4; ++v)
-            hq[v] = f2bf(GELU ? gelu_glu_f(g[v], u[v]) : CLIPPED ? clipped_glu_f(g[v], u[v], limit) : silu_f(g[v]) * u[v]);
+            hq[v] = f2bf(GELU     ? gelu_glu_f(g[v], u[v])
+                         : BIASED ? clipped_glu_f(g[v] + bf2f(bg[i][v]), u[v] + bf2f(bu[i][v]), limit)
+                         : CLIPPED ? clipped_glu_f(g[v], u[v], limit)
+                                   : silu_f(g[v]) * u[v]);
         } else {
 #pragma unroll
           for (int v = 0; v < 4; ++v) hq[v] = f2bf(acc[r][i][v]);
@@ -1149,7 +1165,7 @@ int* pf_queue(hipStream_t s) {
 // dynamic tile queue (DYN; needs K >= 128) instead of the static tile = w + i P walk; variant 8:
 // nontemporal output stores (by default: SwiGLU outputs > 256 MiB).
 void gemm_pf(uintptr_t c, uintptr_t a, uintptr_t b, int M, int N, int K, int mode, int variant, uintptr_t stream,
-             float limit, int bm) {
+             float limit, int bm, uintptr_t bias) {
   const bool dyn = (variant & 16) != 0;
   variant &= ~16;
   DLLM_HOST_CHECK(!dyn || K >= 2 * PBK, "the dynamic tile queue needs K >= 128");
@@ -1174,6 +1190,7 @@ void gemm_pf(uintptr_t c, uintptr_t a, uintptr_t b, int M, int N, int K, int mod
     cus = n > 0 ? n : 256;
     if (dev >= 0 && dev < 64) cus_of[dev].store(cus, std::memory_order_relaxed);
   }
+  DLLM_HOST_CHECK(bias == 0 || (mode == 3 && bias % 8 == 0), "a bias: clipped GLU, 8-byte aligned");
   DLLM_HOST_CHECK(bm == 256 || bm == 224 || bm == 192 || bm == 160, "row tile 160, 192, 224 or 256");
   DLLM_HOST_CHECK(bm == 256 || (!dyn && variant == 0), "row tiles below 256: static walk, default stores");
   const long tiles = (long)(N / 256) * ((M + bm - 1) / bm);
@@ -1183,7 +1200,7 @@ void gemm_pf(uintptr_t c, uintptr_t a, uintptr_t b, int M, int N, int K, int mod
   int* q = dyn ? pf_queue(s) : nullptr;
 #define DLLM_PF_GO(MODE_, SCH_, DYN_, RT_)                                                                         \
   hipLaunchKernelGGL((gemm_pf_kernel<MODE_, SCH_, DYN_, RT_>), dim3((unsigned)grid), dim3(256), 0, s, (const bf16*)a, \
-                     (const bf16*)b, (bf16*)c, M, N, K, q, limit)
+                     (const bf16*)b, (bf16*)c, M, N, K, q, limit, (const bf16*)bias)
 #define DLLM_PF_MODE(MODE_)                                                                              \
   do {                                                                                                   \
     if (dyn) { if (nt_store) DLLM_PF_GO(MODE_, 8, true, 8); else DLLM_PF_GO(MODE_, 0, true, 8); }        \
@@ -1194,6 +1211,7 @@ void gemm_pf(uintptr_t c, uintptr_t a, uintptr_t b, int M, int N, int K, int mod
   } while (0)
   const bool nt_store = variant == 8 || (bm == 256 && mode != 0 && (long)M * (N / 2) * 2 > (256L << 20));
   if (mode == 4) DLLM_PF_MODE(5);
+  else if (mode == 3 && bias) DLLM_PF_MODE(6);
   else if (mode == 3) DLLM_PF_MODE(4);
   else if (mode == 1) DLLM_PF_MODE(2);
   else DLLM_PF_MODE(0);

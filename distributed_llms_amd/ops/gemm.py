@@ -492,12 +492,13 @@ def linear_pp(x: torch.Tensor, w: torch.Tensor, splits: int = 0, swiglu: bool = 
 
 
 def linear_pf(x: torch.Tensor, w: torch.Tensor, swiglu: bool = False, variant: int = 0,
-              limit: Optional[float] = None, gelu: bool = False, bm: int = 256) -> torch.Tensor:
+              limit: Optional[float] = None, gelu: bool = False, bm: int = 256,
+              bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Persistent prefill GEMM (gemm_pf in csrc/kernels/gemm_pp.hip): schedule 2's ``bm`` x 256 tiles,
     one workgroup per CU walking its tiles with the LDS-DMA pipeline running across tile
     boundaries; optional fused SwiGLU (``w`` = [Wg; Wu], y [M, N / 2]) or -- ``limit`` -- clipped GLU or -- ``gelu`` --
     gelu_tanh GLU.  ``variant`` 8: nontemporal
-    output stores (the default for SwiGLU outputs > 256 MiB); ``bm``: the row tile (pf_row_tile); the tiles come from per-XCD device
+    output stores (the default for SwiGLU outputs > 256 MiB); ``bm``: the row tile (pf_row_tile); ``bias`` [gate | up]: with ``limit``; the tiles come from per-XCD device
     queues while knobs.pf_dynamic says so (bit 16 of the launcher's variant)."""
     k = x.shape[-1]
     n = w.shape[0]
@@ -517,7 +518,7 @@ def linear_pf(x: torch.Tensor, w: torch.Tensor, swiglu: bool = False, variant: i
         variant |= 16                  # per-XCD dynamic tile queues (gemm_pp.hip, DYN)
     _ext.kernels().gemm_pf(y.data_ptr(), x.data_ptr(), w.data_ptr(), m, n, k,
                            4 if gelu else 3 if limit is not None else (1 if swiglu else 0), variant, current_stream(),
-                           0.0 if limit is None else float(limit), bm)
+                           0.0 if limit is None else float(limit), bm, 0 if bias is None else bias.data_ptr())
     return y
 
 
@@ -581,21 +582,31 @@ def linear_sq(x: torch.Tensor, w: torch.Tensor, splits: int = 0, swiglu: bool = 
     return y
 
 
+def _glu_bias(bias: torch.Tensor, n: int, x: torch.Tensor) -> bool:
+    """A bias that gemm_pf's epilogue reads: [gate | up] in bfloat16 on x's device, four columns per load."""
+    return (bias.dtype == torch.bfloat16 and bias.dim() == 1 and bias.size(0) == n and bias.is_contiguous()
+            and bias.device == x.device and bias.data_ptr() % 8 == 0)
+
+
 def _linear_glu(x: torch.Tensor, w_gate_up: torch.Tensor, limit: Optional[float],
                 bias: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """A GLU of x Wg^T and x Wu^T, W = [Wg; Wu], with the activation in the weight-streaming GEMM's epilogue (up to 64
-    rows; the only form that takes a ``bias`` [gate | up]), in the persistent GEMM's (prompts) or in the split-K
-    reduction (decode): clipped (``limit``) or gelu_tanh (None); None if the shape takes none of them."""
+    rows), in the persistent GEMM's (prompts; the forms that take a ``bias`` [gate | up]) or in the split-K
+    reduction (decode): clipped (``limit``) or gelu_tanh (None); None if the shape takes none of them.  The prompt form of a
+    bias, 700 / 3000 / 6376 / 12000 rows x 15360 x 2560: 65 / 211 / 434 / 810 us with the gate kernel behind the product,
+    53 / 185 / 363 / 680 in its epilogue."""
     m, n, k = _sizes(x, w_gate_up, "linear_glu")
     glu = "gelu" if limit is None else "clipped"
     if m <= STREAM_MAX_M and n % 2 == 0 and use_stream(m, n, k, x, w_gate_up, bias, glu):
         return _stream(m, n, k, x, w_gate_up, bias, glu, 0.0 if limit is None else limit)
-    if x.dtype != torch.bfloat16 or n % 256 or bias is not None:
+    if x.dtype != torch.bfloat16 or n % 256 or (bias is not None and not _glu_bias(bias, n, x)):
         return None
     if not _use_wide(m, n, k, x, w_gate_up) and _use_pp(m, n, k, x, w_gate_up, knobs.K.pp_swiglu_min_m):
         bm = _pf_plan(m, n, k, n // 2, x.device)
-        if bm:
-            return linear_pf(x, w_gate_up, limit=limit, gelu=limit is None, bm=bm)
+        if bm and not (bias is not None and (limit is None or _recorded(x, w_gate_up, bias))):
+            return linear_pf(x, w_gate_up, limit=limit, gelu=limit is None, bm=bm, bias=bias)
+    if bias is not None:
+        return None
     y = linear(x, w_gate_up, defer=True)
     if isinstance(y, SplitKPartial):
         out = torch.empty(*x.shape[:-1], n // 2, dtype=x.dtype, device=x.device)

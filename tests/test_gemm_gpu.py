@@ -367,6 +367,38 @@ def test_pf_row_tiles_bit_exact(cuda, bm, m, n, k):
         assert torch.equal(gemm.linear_pf(x, w, bm=bm, **kw), gemm.linear_pf(x, w, **kw)), kw
 
 
+@pytest.mark.parametrize("m,bm", [(1, 256), (300, 256), (161, 160), (900, 192), (449, 224)])
+@pytest.mark.parametrize("f,k", [(128, 64), (640, 192)])
+def test_pf_clipped_glu_bias(cuda, m, bm, f, k):
+    """The clipped GLU of product + bias in the epilogue, every row tile: with a zero bias the unbiased epilogue's bits;
+    else against float64."""
+    torch.manual_seed(m + f)
+    b = torch.randn(2 * f, device="cuda").bfloat16()
+    x, w = _bf(m, k), _bf(2 * f, k, scale=0.1)
+    assert torch.equal(gemm.linear_pf(x, w, limit=0.7, bm=bm, bias=torch.zeros_like(b)), gemm.linear_pf(x, w, limit=0.7, bm=bm))
+    z = x.double() @ w.double().t() + b.double()
+    g, u = z[:, :f].clamp(max=0.7), z[:, f:].clamp(-0.7, 0.7)
+    ref = g * torch.sigmoid(1.702 * g) * (u + 1)
+    e = (x.double().abs() @ w.double().abs().t() + b.double().abs()) * (k + 1) * 2.0 ** -24        # f32 sums, any order
+    tol = 1.2 * e[:, :f] * 1.7 + 0.8 * e[:, f:] + (2.0 ** -8 + 2.0 ** -18) * ref.abs() + 2.0 ** -22
+    assert bool(((gemm.linear_pf(x, w, limit=0.7, bm=bm, bias=b).double() - ref).abs() <= tol).all())
+
+
+def test_clipped_glu_bias_reaches_the_prompt_gemm(cuda, monkeypatch):
+    """A biased clipped GLU over a prompt: in the GEMM's epilogue where its bias can be read there, else behind it."""
+    from distributed_llms_amd.ops import seqmix as sm
+    calls, real = [], gemm.linear_pf
+    monkeypatch.setattr(gemm, "linear_pf", lambda *a, **kw: (calls.append(kw.get("bias")), real(*a, **kw))[1])
+    x, w = _bf(4000, 256), _bf(4096, 256, scale=0.1)   # 256 tiles: a full round of 256 CUs
+    store = torch.randn(4097, device="cuda").bfloat16()
+    for b in (store[:4096], store[1:]):                # aligned, and not
+        calls.clear()
+        y = sm.linear_clipped_glu(x, w, b, 0.7)
+        assert any(c is not None for c in calls) == (b.data_ptr() % 8 == 0)
+        gu = x.float() @ w.float().t()
+        torch.testing.assert_close(y.float(), sm.clipped_glu(gu, b.float(), 0.7), atol=2e-2, rtol=2e-2)
+
+
 def test_pf_swiglu_output_range_is_the_half_width(cuda):
     """SwiGLU's output is [M, N / 2]: a 70B prefill gate|up (M 32768, 2I 57344) is within the
     kernel's 2 GiB output range although M x 2I x 2 bytes is not (a small-K stand-in shape)."""
