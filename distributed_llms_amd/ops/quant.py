@@ -197,19 +197,55 @@ def linear_ref(x, w: Fp8Weight, swiglu: bool = False) -> torch.Tensor:
 # (knobs.fp8_bm128)
 # prefill-sized M (no K split): grouped row-tile order (gemm_wide_fp8 variant bit 64) from this M:
 # at M = 32768 qkv 1018 -> 889 us, o 660 -> 599, gate|up 4509 -> 3924, down 2083 -> 1873 (1.8-2.0
-# PFLOP/s); at M = 2048 it is 1-6 % slower
-# PFLOP/s); at M = 2048 it is 1-6 % slower (knobs.fp8_group_m)
+# PFLOP/s); at M = 2048 it is 1-6 % slower (knobs.fp8_group_m).  Those are 256-row tiles; shorter ones gain from half as
+# many rows: 4096 x 14336 in 192 rows, M = 3072 / 6144, 194 / 397 -> 179 / 363, 128 rows at M = 3072 221 -> 213
+
+
+# Past 256 rows the workgroups of a grid run in rounds of one per CU, so what a launch takes is the number of rounds times
+# what a workgroup of that row tile takes: a K-tile of 128, us, and the workgroup's start and epilogue (measured, one
+# round, K = 2048 ... 14336).  Shorter tiles do less per byte staged.  Two 64-row workgroups share a CU: a further round adds
+# less than the first.  A K split adds the launch that sums the slabs, and their traffic.  Former plan (the decode kernels' K
+# split, 192 / 256-row tiles) -> this, reduction included, us: 4096 x 14336 at M = 448 / 640 / 1536 / 2432 / 2800 43 / 76 / 93 /
+# 188 / 186 -> 39 / 52 / 87 / 164 / 170; 4096 x 4096 at 320 / 640 / 1536 / 2800 19 / 27 / 34 / 63 -> 17 / 21 / 30 / 57; 6144 x 4096 at
+# 320 / 1024 / 1536 22.7 / 32.6 / 61 -> 17.2 / 32.2 / 54; 1024 x 8192 at 320 / 2048 15.6 / 37 -> 12.3 / 28.6; 8192 x 8192 at 640 / 1536
+# 57 / 111 -> 51 / 105; 2048 x 2048 at 768 / 2048 18.2 / 20.1 -> 10.3 / 14.9; where 256 rows fill their rounds (28672 x 4096 at
+# 2432, 302 against 328 in 192 rows; 6144 x 4096 at 2048, 64 against 67 in 128) nothing changes.
+_ROUND_US = {64: (0.435, 3.2), 128: (0.505, 5.0), 192: (0.66, 5.5), 256: (0.745, 6.6)}
+_ROUND_64 = 0.36
+_SLAB_US, _SLAB_US_PER_MB = 3.0, 0.3
+
+
+def _prompt_plan(m: int, n: int, k: int, most: int) -> Tuple[int, int]:
+    """(K slices, row tile) of the cheapest grid past 256 rows.  ``most``: the slabs hold 16 bits, so a product is split no
+    further than the decode rule would split it, and one that this leaves whole stays whole."""
+    from . import gemm
+    best, plan = float("inf"), (1, 256)
+    for bm in (256, 192, 128, 64):
+        tile_us, fixed = _ROUND_US[bm]
+        tiles = (n // 128) * -(-m // bm)
+        for s in range(1, min(most, 8, max(1, k // 128 // 4)) + 1):
+            if s > 1 and (s * m * n > gemm._WS_FLOATS or tiles * s > 256):
+                break
+            rounds, kt = -(-tiles * s // 256), -(-(k // 128) // s)
+            us = ((tile_us + _ROUND_64 * (rounds - 1)) * kt + fixed if bm == 64 else rounds * (tile_us * kt + fixed))
+            if s > 1:
+                us += _SLAB_US + _SLAB_US_PER_MB * s * m * n * 4e-6
+            if us < best:
+                best, plan = us, (s, bm)
+    return plan
 
 
 def fp8_plan(m: int, n: int, k: int, swiglu: bool = False) -> Tuple[int, int]:
-    """(K slices, row-tile override or 0) of gemm_wide_fp8 for this shape.  Default: the bf16
-    kernel's rule on the 128-K tiles (a K-tile of fp8 holds the bytes of a 64-K bf16 tile); up to 64 rows a split narrow
+    """(K slices, row-tile override or 0) of gemm_wide_fp8 for this shape.  Past 256 rows the cheapest
+    grid (:func:`_prompt_plan`; with CUs reserved for communication the decode rule).  Default: the bf16 kernel's rule on the 128-K tiles (a K-tile of fp8 holds the bytes of a 64-K bf16 tile); up to 64 rows a split narrow
     product takes up to 8 slices -- what the reduction loads in one go -- of 4 K-tiles where that is twice as many.  us with
     the norm behind it, M = 1 / 16 / 64, former -> this: 1024 x 4096 8.9 / 10.0 / 10.4 -> 7.6 / 8.6 / 9.1, 2048 x 2048 9.0 /
     10.0 / 10.4 -> 7.6 / 8.6 / 9.0 (4 slices), 4096 x 4096 10.0 / 10.8 / 11.5 -> 9.0 / 10.1 / 11.3; 16 slices 10-14, and
     6144 x 4096 in 5 instead of 4 10.9 / 11.9 / 12.9 -> 11.2 / 12.3 / 13.6."""
     from . import gemm
     s = gemm.wide_splits(m, n, k // 2, swiglu, short=False)
+    if m > 256 and not gemm._comm_cus:
+        return _prompt_plan(m, n, k, s)
     if m <= 64 and not swiglu and s > 1 and not gemm._comm_cus:
         c = min(8, 256 // (n // 128), (k // 128) // 4)
         if c >= 2 * s:
@@ -253,7 +289,8 @@ def linear_fp8(x: torch.Tensor, w: Fp8Weight, swiglu: bool = False, defer: bool 
     if s > 1 and s * m * n > ws.numel():
         s = max(1, ws.numel() // (m * n))
     # weights streamed non-temporal only where one row tile covers M (each weight byte read once)
-    variant = (1 if m <= 256 else (4 | (64 if 0 < knobs.K.fp8_group_m <= m else 0))) | (bm << 8)
+    grouped = 0 < knobs.K.fp8_group_m <= (2 * m if 0 < bm < 256 else m)
+    variant = (1 if m <= 256 else (4 | (64 if grouped else 0))) | (bm << 8)
     stream = current_stream()
     kern = _ext.kernels()
     if defer and not swiglu and s > 1:

@@ -84,3 +84,17 @@ def test_cpu_engine_runs_fp8():
     assert [len(o) for o in out] == [6, 6]
     assert [o[0] for o in out] == [o[0] for o in ref]       # first greedy tokens agree
     assert e8.stage.weight_bytes() < LLMEngine(base).stage.weight_bytes() / 2
+
+
+def test_fp8_prompt_plan_splits_no_further():
+    """Past 256 rows: a product that the decode rule leaves whole stays whole and no other gets more slices (the slabs hold
+    16 bits), the slabs fit the workspace, and one full round of 256-row tiles is left as it is."""
+    from distributed_llms_amd.ops import gemm, quant
+    for m in (257, 300, 449, 640, 1025, 2048, 2817, 5000, 70000):
+        for n in (128, 1024, 4096, 6144, 28672):
+            for k in (128, 640, 4096, 14336):
+                for swiglu in (False, True):
+                    s, bm = quant.fp8_plan(m, n, k, swiglu)
+                    assert 1 <= s <= min(8, gemm.wide_splits(m, n, k // 2, swiglu, short=False))
+                    assert bm in (64, 128, 192, 256) and (s == 1 or s * m * n <= gemm._WS_FLOATS)
+    assert quant.fp8_plan(2048, 4096, 4096) == (1, 256) and quant.fp8_plan(2816, 4096, 4096) == (1, 192)

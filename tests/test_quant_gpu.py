@@ -55,6 +55,35 @@ def test_gemm_wide_fp8_matches_reference(m, n, k, swiglu, splits):
     assert err <= 2e-2 * ref.abs().max().item() + 1e-3, err
 
 
+@pytest.mark.parametrize("m", [257, 449, 2100])
+@pytest.mark.parametrize("n,k,swiglu", [(256, 512, False), (1280, 384, False), (512, 640, True)])
+def test_fp8_row_tiles_bit_exact(monkeypatch, m, n, k, swiglu):
+    """Every row tile past 256 rows, in both tile orders (grouped from 2048 rows below 256): the same sums in the same order."""
+    w, x = quant.quantize_weight((torch.randn(n, k) * 0.02).to(DEV)), _x(m, k, seed=m)
+    out = {}
+    for bm in (256, 192, 128, 64):
+        monkeypatch.setattr(quant, "fp8_plan", lambda *a, bm=bm, **kw: (1, bm))
+        out[bm] = quant.linear_fp8(x, w, swiglu=swiglu)
+    assert all(torch.equal(out[bm], out[256]) for bm in out)
+    err = (out[256].float().cpu() - _oracle(x, w, swiglu)).abs().max().item()
+    assert err <= 2e-2 * out[256].float().abs().max().item() + 1e-3, err
+
+
+@pytest.mark.parametrize("m,n,k,swiglu,plan", [(300, 1024, 8192, False, (6, 64)), (700, 1024, 8192, False, (5, 128)),
+                                               (640, 4096, 14336, False, (2, 192)), (300, 1024, 4096, True, (4, 64))])
+def test_fp8_prompt_plan_splits(m, n, k, swiglu, plan):
+    """The K splits that the prompt rule takes on short row tiles, reduced here or by the norm that follows."""
+    assert quant.fp8_plan(m, n, k, swiglu) == plan
+    w, x = quant.quantize_weight((torch.randn(n, k) * 0.02).to(DEV)), _x(m, k, seed=m)
+    ref = _oracle(x, w, swiglu)
+    y = quant.linear_fp8(x, w, swiglu=swiglu)
+    assert (y.float().cpu() - ref).abs().max().item() <= 2e-2 * ref.abs().max().item() + 1e-3
+    if not swiglu:
+        part = quant.linear_fp8(x, w, defer=True)
+        assert isinstance(part, gemm.SplitKPartial) and part.splits == plan[0]
+        assert torch.equal(part.materialize(), y)
+
+
 def test_fp8_deferred_split_feeds_the_fused_norm():
     m, n, k = 256, 4096, 4096
     w = quant.quantize_weight((torch.randn(n, k) * 0.02).to(DEV))
