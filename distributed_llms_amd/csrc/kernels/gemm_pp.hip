@@ -29,6 +29,7 @@
 #include "common.h"
 #include "launchers.h"
 
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 #include <type_traits>
@@ -162,7 +163,7 @@ __device__ __forceinline__ void gemm_pp_tile(bf16 (&smem)[SMEM], const bf16* __r
   constexpr int TM = 16 * RT, BM = 2 * TM, TN = BN / NWN;      // waves as 2 (M) x NWN (N)
   constexpr int CT = TN / 16;                          // 16 x 16 fragments per wave: up to 8 x 8 or 8 x 4
   constexpr int SLOT = (BM + BN) * PBK;                // bf16 elements per ring slot (one K-tile)
-  constexpr int NB = BN == 256 && RT > 5 ? 2 : 3;      // K-tiles held in LDS
+  constexpr int NB = BN == 256 && RT > 5 ? 2 : BN == 128 && RT == 4 ? 4 : 3;   // K-tiles held in LDS
   constexpr int GA = BM * PBK * 2 / 1024 / NW, GB = BN * PBK * 2 / 1024 / NW;  // glds per wave per K-tile
   constexpr int G = GA + GB;
   constexpr bool NT = (VAR & 1) != 0;
@@ -593,6 +594,8 @@ constexpr int pp_smem(int bn, int mode, int var) {      // bf16 elements: ring, 
   return ring > image ? ring : image;
 }
 
+constexpr int kMoeCus = 256;
+
 template <int BN, int MODE, int VAR>
 __global__ void __launch_bounds__(256, 1) gemm_pp_kernel(const bf16* __restrict__ A, const bf16* __restrict__ B,
                                                          bf16* __restrict__ C, float* __restrict__ P, int M, int N,
@@ -609,9 +612,38 @@ __global__ void __launch_bounds__(256, 1) gemm_pp_kernel(const bf16* __restrict_
   constexpr bool MOE = (VAR & 128) != 0;
   const int ntiles = N / BN;
   int mtiles = (M + BM - 1) / BM, total = gridDim.x;
+  [[maybe_unused]] bool cut = false;
+  // (MOE: an expert per lane, 64 at a time, E <= 256.  Walked one after the other the counts cost every workgroup microseconds:
+  // 64 experts 2048 x 2816, 6 a token, us at 300 / 3000 / 8192 tokens 173 / 348 / 586 -> 157 / 313 / 532, down 90 / 183 / 320 ->
+  // 77 / 159 / 282)
+  [[maybe_unused]] const int lane = threadIdx.x & 63;
+  [[maybe_unused]] int seg[4], end[4];                 // rows of the expert's segment; row tiles up to its end
   if constexpr (MOE) {
+    // Row tiles of up to 128 rows are bound by the weight bytes in flight to one CU, so where there are no others and they leave
+    // half of the CUs idle each is cut into two workgroups of 128 columns (four K-tiles in LDS): us, Mixtral down at 300 / 395
+    // tokens 249 / 255 -> 182 / 191, 8 experts 1024 x 2048 at 300 27 -> 19.  A longer tile in the same round sets its length
+    // anyway (Mixtral down at 1024 tokens, 4 tiles of 12 cut: 344 -> 358), and past one workgroup per CU the rows are staged
+    // twice for nothing (gate|up at 1500 709 -> 816)
+    int shorts = 0;
     mtiles = 0;
-    for (int x = 0; x < E; ++x) mtiles += (counts[x] + BM - 1) / BM;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (64 * q < E) {                                // uniform
+        const int x = 64 * q + lane, c0 = counts[min(x, E - 1)], c = x < E ? c0 : 0;
+        int t = (c + BM - 1) / BM;
+#pragma unroll
+        for (int d = 1; d < 64; d *= 2) {
+          const int below = __shfl_up(t, d);
+          t += lane >= d ? below : 0;
+        }
+        seg[q] = c;
+        end[q] = mtiles + t;
+        mtiles += __builtin_amdgcn_readlane(t, 63);
+        shorts += __popcll(__ballot(c > 0 && c <= 128));
+      }
+    }
+    cut = shorts == mtiles && 2 * mtiles * ntiles <= kMoeCus;
+    if (cut) mtiles *= 2;
     total = mtiles * ntiles;
   }
   int b = blockIdx.x;
@@ -635,16 +667,22 @@ __global__ void __launch_bounds__(256, 1) gemm_pp_kernel(const bf16* __restrict_
   const int ks0 = split * ks_per_split;
   const int nt = max(0, min(K / PBK, ks0 + ks_per_split) - ks0);
   if constexpr (MOE) {
-    int base = 0, ex = 0, r0 = 0, rcnt = 0;
-    for (int x = 0; x < E; ++x) {
-      const int c = counts[x], nx = (c + BM - 1) / BM;
-      if (m_t >= base && m_t < base + nx) {
-        ex = x;
-        r0 = (m_t - base) * BM;
-        rcnt = c;
+    int ex = 0, first = 0, rcnt = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (64 * q < E) {
+        // (cut: every tile is short and a segment's only one is two units; full tiles cannot precede it)
+        const int tiles = (seg[q] + BM - 1) / BM, to = cut ? 2 * end[q] : end[q], from = to - (cut ? 2 * tiles : tiles);
+        const uint64_t owner = __ballot(m_t >= from && m_t < to);
+        if (owner) {                                   // uniform: one lane of one q
+          const int l = __builtin_ctzll(owner);
+          ex = 64 * q + l;
+          first = __builtin_amdgcn_readlane(from, l);
+          rcnt = __builtin_amdgcn_readlane(seg[q], l);
+        }
       }
-      base += nx;
     }
+    const int r0 = cut ? 0 : (m_t - first) * BM;
     const int roff = offsets[ex];
     const bf16* We = B + (size_t)ex * N * K;
     // a segment's last tile on the row tile that holds what is left (neighbour of the segment's others in the order: put
@@ -656,7 +694,9 @@ __global__ void __launch_bounds__(256, 1) gemm_pp_kernel(const bf16* __restrict_
       gemm_pp_tile<BN, MODE, VAR, decltype(rt)::value>(smem, A, We, C, P, M, N, K, n_t, r0, rcnt, roff, gather, split, ks0, nt,
                                                        D, limit);
     };
-    if (left <= 128) go(std::integral_constant<int, 4>{});
+    if (left <= 128 && cut)
+      gemm_pp_tile<128, MODE, VAR, 4>(smem, A, We, C, P, M, N, K, 2 * n_t + m_t - first, r0, rcnt, roff, gather, split, ks0, nt, D, limit);
+    else if (left <= 128) go(std::integral_constant<int, 4>{});
     else if (left <= 192) go(std::integral_constant<int, 6>{});
     else go(std::integral_constant<int, 8>{});
   } else {
@@ -748,7 +788,9 @@ void gemm_pp_moe(uintptr_t y, uintptr_t x, uintptr_t gather, uintptr_t w, uintpt
   DLLM_HOST_CHECK(xrows >= 1 && slots >= 1, "rows");
   DLLM_HOST_CHECK((long)xrows * K * 2 < (1L << 32) && (long)N * K * 2 < (1L << 32), "operands must be < 4 GiB");
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const long grid = (long)(N / 256) * ((slots + 255) / 256 + E);
+  // (up to one workgroup per CU, one row tile per expert may be cut in two)
+  const long most = (long)(N / 256) * ((slots + 255) / 256 + E), cut = (long)(N / 256) * 2 * E;
+  const long grid = std::max(most, std::min(cut, (long)kMoeCus));
   DLLM_HOST_CHECK(grid < (1L << 31), "grid");
 #define DLLM_PPM(MODE_, VAR_)                                                                                         \
   hipLaunchKernelGGL((gemm_pp_kernel<256, MODE_, VAR_>), dim3((unsigned)grid), dim3(256), 0, s, (const bf16*)x,        \

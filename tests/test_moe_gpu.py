@@ -173,6 +173,34 @@ def test_moe_prefill_grouped_gemm(cuda, t, e, k, h, i, skew):
 
 
 @pytest.mark.parametrize("mode", [0, 1, 2, 3])
+@pytest.mark.parametrize("n", [512, 2560])
+@pytest.mark.parametrize("counts", [[0, 1, 128, 0, 129, 300, 384, 385], [3], [128] * 8, [0, 0, 100, 0, 90, 256, 512],
+                                    [0] * 62 + [1, 2, 3, 0, 100] + [0] * 80 + [64] + [0] * 60 + [5]])
+def test_moe_grouped_gemm_cuts_short_tiles(cuda, mode, n, counts):
+    """Row tiles of up to 128 rows, alone and beside longer ones, in two workgroups where they leave half of the CUs idle (2560
+    columns: 8 experts do not): the bits of a launch that is padded past one workgroup per CU with segments of their own."""
+    from distributed_llms_amd import _ext
+    k, tokens, pad = 256, 500, 256 * 9                 # the padding's tiles: 9 x 2 columns x 16 experts > 256
+    w = _bf(len(counts), n, k, scale=0.1)
+    glu = mode in (1, 3)
+
+    def run(c, w, n_pad):
+        c = torch.tensor(c, dtype=torch.int32, device="cuda")
+        slots = int(c.sum())
+        gather = torch.arange(slots, device="cuda", dtype=torch.int32).remainder_(tokens)
+        y = torch.full((slots + 4, n // 2 if glu else n), 7.0, dtype=torch.bfloat16, device="cuda")
+        off = torch.cumsum(c, 0).to(torch.int32) - c
+        _ext.kernels().gemm_pp_moe(y.data_ptr(), x.data_ptr(), gather.data_ptr(), w.data_ptr(), c.data_ptr(), off.data_ptr(),
+                                   len(c), n, k, tokens, slots, mode, torch.cuda.current_stream().cuda_stream, 0.7)
+        assert bool((y[slots:] == 7.0).all())
+        return y[:slots - n_pad]
+
+    x = _bf(tokens, k)
+    more = torch.cat([w, w[:1].expand(16, n, k)]).contiguous()
+    assert torch.equal(run(counts, w, 0), run(counts + [pad] * 16, more, 16 * pad))
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2, 3])
 def test_moe_grouped_gemm_last_tiles(cuda, mode):
     """Segments whose last row tile holds 1 .. 256 rows, on either side of the 128- and 192-row tiles, with empty experts
     between, gathered and not: against each segment's own f32 product, nothing written past the segments."""
