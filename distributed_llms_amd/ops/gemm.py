@@ -391,7 +391,8 @@ def wide_splits(m: int, n: int, k: int, swiglu: bool = False, target_wgs: int = 
     reserved for communication: at most one workgroup per remaining CU).  ``short``: a split product of up to 128
     rows takes up to 8 slices of 4 K-tiles: with the close behind it, M = 8 / 32 / 128, us, 2560 x 2560 in 5 -> 8 slices 11.0 / 11.7 / 15.1 -> 9.7 /
     10.5 / 14.1, 2560 x 2048 in 4 -> 8 10.7 / 11.0 / 13.5 -> 9.7 / 10.1 / 13.2, 1024 x 1024 in 2 -> 4 8.1 / 8.1 / 9.9 -> 6.8 / 7.0 / 8.2;
-    past 128 rows the slabs cost more than the shorter loop saves (2560 x 2560 at 200 rows 15.3 -> 18.8)."""
+    past 128 rows the slabs cost more than the shorter loop saves (2560 x 2560 at 200 rows 15.3 -> 18.8).  A product whose K sets
+    the slices gets as many beside communication: a pipeline's stages round as one engine does."""
     tiles = (n // 128) * (-(-m // wide_row_tile(m, n, k, swiglu)))
     target = target_wgs or knobs.K.wide_target_wgs
     if _comm_cus:
@@ -399,7 +400,7 @@ def wide_splits(m: int, n: int, k: int, swiglu: bool = False, target_wgs: int = 
     else:
         s = max(1, round(target / tiles))
     least = max(1, min(s, (k // 64) // 8, 16))
-    if short and least > 1 and m <= 128 and not swiglu and not _comm_cus:
+    if short and least > 1 and m <= 128 and not swiglu:
         return max(least, min(s, (k // 64) // 4, 8))
     return least
 

@@ -215,7 +215,7 @@ _ROUND_64 = 0.36
 _SLAB_US, _SLAB_US_PER_MB = 3.0, 0.3
 
 
-def _prompt_plan(m: int, n: int, k: int, most: int) -> Tuple[int, int]:
+def _prompt_plan(m: int, n: int, k: int, most: int, cus: int) -> Tuple[int, int]:
     """(K slices, row tile) of the cheapest grid past 256 rows.  ``most``: the slabs hold 16 bits, so a product is split no
     further than the decode rule would split it, and one that this leaves whole stays whole."""
     from . import gemm
@@ -224,9 +224,9 @@ def _prompt_plan(m: int, n: int, k: int, most: int) -> Tuple[int, int]:
         tile_us, fixed = _ROUND_US[bm]
         tiles = (n // 128) * -(-m // bm)
         for s in range(1, min(most, 8, max(1, k // 128 // 4)) + 1):
-            if s > 1 and (s * m * n > gemm._WS_FLOATS or tiles * s > 256):
+            if s > 1 and (s * m * n > gemm._WS_FLOATS or tiles * s > cus):
                 break
-            rounds, kt = -(-tiles * s // 256), -(-(k // 128) // s)
+            rounds, kt = -(-tiles * s // cus), -(-(k // 128) // s)
             us = ((tile_us + _ROUND_64 * (rounds - 1)) * kt + fixed if bm == 64 else rounds * (tile_us * kt + fixed))
             if s > 1:
                 us += _SLAB_US + _SLAB_US_PER_MB * s * m * n * 4e-6
@@ -237,17 +237,18 @@ def _prompt_plan(m: int, n: int, k: int, most: int) -> Tuple[int, int]:
 
 def fp8_plan(m: int, n: int, k: int, swiglu: bool = False) -> Tuple[int, int]:
     """(K slices, row-tile override or 0) of gemm_wide_fp8 for this shape.  Past 256 rows the cheapest
-    grid (:func:`_prompt_plan`; with CUs reserved for communication the decode rule).  Default: the bf16 kernel's rule on the 128-K tiles (a K-tile of fp8 holds the bytes of a 64-K bf16 tile); up to 64 rows a split narrow
+    grid (:func:`_prompt_plan`) of the CUs that communication leaves.  Default: the bf16 kernel's rule on the 128-K tiles (a K-tile of fp8 holds the bytes of a 64-K bf16 tile); up to 64 rows a split narrow
     product takes up to 8 slices -- what the reduction loads in one go -- of 4 K-tiles where that is twice as many.  us with
     the norm behind it, M = 1 / 16 / 64, former -> this: 1024 x 4096 8.9 / 10.0 / 10.4 -> 7.6 / 8.6 / 9.1, 2048 x 2048 9.0 /
     10.0 / 10.4 -> 7.6 / 8.6 / 9.0 (4 slices), 4096 x 4096 10.0 / 10.8 / 11.5 -> 9.0 / 10.1 / 11.3; 16 slices 10-14, and
     6144 x 4096 in 5 instead of 4 10.9 / 11.9 / 12.9 -> 11.2 / 12.3 / 13.6."""
     from . import gemm
     s = gemm.wide_splits(m, n, k // 2, swiglu, short=False)
-    if m > 256 and not gemm._comm_cus:
-        return _prompt_plan(m, n, k, s)
-    if m <= 64 and not swiglu and s > 1 and not gemm._comm_cus:
-        c = min(8, 256 // (n // 128), (k // 128) // 4)
+    cus = 256 - gemm._comm_cus
+    if m > 256:
+        return _prompt_plan(m, n, k, s, cus)
+    if m <= 64 and not swiglu and s > 1:
+        c = min(8, cus // (n // 128), (k // 128) // 4)
         if c >= 2 * s:
             s = c
     if knobs.K.fp8_bm128 and not swiglu and s > 1 and 128 < m <= 256:

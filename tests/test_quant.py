@@ -98,3 +98,19 @@ def test_fp8_prompt_plan_splits_no_further():
                     assert 1 <= s <= min(8, gemm.wide_splits(m, n, k // 2, swiglu, short=False))
                     assert bm in (64, 128, 192, 256) and (s == 1 or s * m * n <= gemm._WS_FLOATS)
     assert quant.fp8_plan(2048, 4096, 4096) == (1, 256) and quant.fp8_plan(2816, 4096, 4096) == (1, 192)
+
+
+@pytest.mark.parametrize("m", [1, 8, 64, 100, 128, 300, 700])
+def test_reserved_cus_leave_small_splits_alone(m):
+    """Products whose K (not the number of CUs) sets the slices are split alike with CUs reserved for communication: the
+    stages of a pipeline sum in the order of a single engine."""
+    from distributed_llms_amd.ops import gemm, quant
+    from distributed_llms_amd.parallel.rccl_transport import comm_cus
+    shapes = [(256, 256), (512, 512), (1024, 1024), (512, 1024), (1024, 2048)]
+    plans = lambda: [(gemm.wide_splits(m, n, k), quant.fp8_plan(m, n, k), quant.fp8_plan(m, n, k, True)) for n, k in shapes]
+    alone = plans()
+    gemm.reserve_cus_for_comm(comm_cus())
+    try:
+        assert plans() == alone
+    finally:
+        gemm.release_cus_for_comm()
