@@ -505,8 +505,9 @@ __device__ __forceinline__ void gemm_pp_tile(bf16 (&smem)[SMEM], const bf16* __r
   // acc[rt][ct] lane l holds C[row wm*TM + rt*16 + (l & 15)][col wn*TN + ct*16 + 4*(l >> 4) + v]
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  // (the lane from the hardware again, so that no register holds it through the loop)
-  const int le = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), te = wv * 64 + le;
+  // (MOE: the lane from the hardware again, so that no register holds it through the loop; the dense forms have one to spare)
+  const int le = MOE ? (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)) : lane;
+  const int te = MOE ? wv * 64 + le : tid;
   const int lr = le & 15, lq = le >> 4;
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
