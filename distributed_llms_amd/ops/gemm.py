@@ -19,9 +19,9 @@ the engine on Llama-3-8B, profiles/wide_gemm.md; each one is a field of :mod:`..
   224 x 256; knobs.pp_gate_up_min_m), and the long-K down projection (K >= knobs.pp_down_min_k,
   70B) at 225 <= M <= 256 on split gemm_pp 128-column tiles (profiles/round6_gate_up_pp.md);
 * prefill (M >= knobs.pp_swiglu_min_m / pp_proj_min_m, above the decode ranges): the 4-wave
-  256 x 256-tile schedule-2 kernel in its persistent form (gemm_pf in gemm_pp.hip, knobs.pp_persistent)
-  -- gate|up with the SwiGLU fused into its epilogue, qkv / o / down plain
-  (profiles/round4_gemm_counters.md);
+  schedule-2 kernel in its persistent form (gemm_pf in gemm_pp.hip, knobs.pp_persistent; 256 x 256 tiles, or row tiles of
+  160, 192 or 224 where they need fewer rounds of the chip, :func:`pf_row_tile`) -- gate|up with the GLU (and a clipped
+  one's bias) in its epilogue, qkv / o / down plain (profiles/round4_gemm_counters.md);
 * what none of them takes (a bias or N not a multiple of 128 past 64 rows, K not a multiple of 64, fp32 on CPU,
   operands >= 4 GiB): torch's F.linear.
 

@@ -5,8 +5,8 @@ GPU path (bf16):
   moe_route      : softmax -> top-k -> renormalise, expert-sorted slots    (HIP, one launch)
   decode-sized T : grouped weight-streaming GEMMs on the sorted slots (gate|up + SwiGLU, then down)
                    entirely on device -- no host sync, so the decode step stays graph-capturable
-  prefill-sized T: grouped 256 x 256-tile GEMMs over the expert-sorted slots (gemm_pp.hip
-                   gemm_pp_moe: one launch per projection, every expert's row tiles in one grid,
+  prefill-sized T: grouped GEMMs over the expert-sorted slots (gemm_pp.hip gemm_pp_moe: 256 x 256 tiles, a
+                   segment's last one of 128, 192 or 256 rows; one launch per projection, every expert's row tiles in one grid,
                    counts / offsets read on the device -- no host sync, no per-expert loop; gate|up
                    with the SwiGLU in its epilogue, the token gather in its A staging)
   W8A8 experts   : the grouped fp8 kernel (moe_wide_gemm_fp8) at every T, also without a host sync
@@ -247,7 +247,7 @@ def grouped_choice_ffn(x: torch.Tensor, w_router: torch.Tensor, correction: Opti
         k.moe_grouped_gemm(ys.data_ptr(), act.data_ptr(), 0, w_down.data_ptr(), counts.data_ptr(), offsets.data_ptr(),
                            e, width, f, 0, rows, knobs.K.moe_variant, st)
     elif bf and f % 256 == 0 and width % 256 == 0 and t * width * 2 < (1 << 32) and slots * f * 2 < (1 << 32):
-        # prompt-sized: one grouped 256 x 256-tile launch per projection over every expert's row tiles
+        # prompt-sized: one grouped launch per projection over every expert's row tiles
         act = torch.empty(slots, f, dtype=x.dtype, device=dev)
         k.gemm_pp_moe(act.data_ptr(), x.data_ptr(), sorted_tok.data_ptr(), w_up.data_ptr(), counts.data_ptr(),
                       offsets.data_ptr(), e, f, width, t, slots, 2, st)                                  # mode 2: relu^2
@@ -404,7 +404,7 @@ def softmax_top_ffn(x: torch.Tensor, w_router: torch.Tensor, b_router: Optional[
                                knobs.K.moe_variant, st)
     elif bf and two_f % 256 == 0 and width % 256 == 0 and f % 64 == 0 and t * width * 2 < (1 << 32) \
             and slots * f * 2 < (1 << 32):
-        # prompt-sized: one grouped 256 x 256-tile launch per projection over every expert's row tiles
+        # prompt-sized: one grouped launch per projection over every expert's row tiles
         act = torch.empty(slots, f, dtype=x.dtype, device=dev)
         k.gemm_pp_moe(act.data_ptr(), x.data_ptr(), sorted_tok.data_ptr(), w_gate_up.data_ptr(), cp, op, e, two_f,
                       width, t, slots, gm, st, lim)
