@@ -386,23 +386,19 @@ def release_cus_for_comm() -> None:
         _comm_cus = 0
 
 
-def wide_splits(m: int, n: int, k: int, swiglu: bool = False, target_wgs: int = 0, short: bool = True) -> int:
+def wide_splits(m: int, n: int, k: int, swiglu: bool = False, target_wgs: int = 0) -> int:
     """K slices for gemm_wide: about one workgroup per CU, >= 8 K-tiles (512) per slice (with CUs
-    reserved for communication: at most one workgroup per remaining CU).  ``short``: a split product of up to 128
-    rows takes up to 8 slices of 4 K-tiles: with the close behind it, M = 8 / 32 / 128, us, 2560 x 2560 in 5 -> 8 slices 11.0 / 11.7 / 15.1 -> 9.7 /
-    10.5 / 14.1, 2560 x 2048 in 4 -> 8 10.7 / 11.0 / 13.5 -> 9.7 / 10.1 / 13.2, 1024 x 1024 in 2 -> 4 8.1 / 8.1 / 9.9 -> 6.8 / 7.0 / 8.2;
-    past 128 rows the slabs cost more than the shorter loop saves (2560 x 2560 at 200 rows 15.3 -> 18.8).  A product whose K sets
-    the slices gets as many beside communication: a pipeline's stages round as one engine does."""
+    reserved for communication: at most one workgroup per remaining CU).  Shorter slices are faster up to 128 rows (2560 x
+    2560 in 8 instead of 5, close included, M = 8 / 128, 11.0 / 15.1 -> 9.7 / 14.1 us), but every slice's sum passes through a
+    16-bit slab: for results around 0.01, whose slabs lose bits to the small end of f16, the error of the slabs' sum against
+    64 bits grew from 2.7e-4 to 3.2e-4 (4 -> 8 slices 2.6e-4 to 3.2e-4)."""
     tiles = (n // 128) * (-(-m // wide_row_tile(m, n, k, swiglu)))
     target = target_wgs or knobs.K.wide_target_wgs
     if _comm_cus:
         s = max(1, (target - _comm_cus) // tiles)
     else:
         s = max(1, round(target / tiles))
-    least = max(1, min(s, (k // 64) // 8, 16))
-    if short and least > 1 and m <= 128 and not swiglu:
-        return max(least, min(s, (k // 64) // 4, 8))
-    return least
+    return max(1, min(s, (k // 64) // 8, 16))
 
 
 WIDE_NT_MIN_BYTES = 12 << 20

@@ -243,7 +243,7 @@ def fp8_plan(m: int, n: int, k: int, swiglu: bool = False) -> Tuple[int, int]:
     10.0 / 10.4 -> 7.6 / 8.6 / 9.0 (4 slices), 4096 x 4096 10.0 / 10.8 / 11.5 -> 9.0 / 10.1 / 11.3; 16 slices 10-14, and
     6144 x 4096 in 5 instead of 4 10.9 / 11.9 / 12.9 -> 11.2 / 12.3 / 13.6."""
     from . import gemm
-    s = gemm.wide_splits(m, n, k // 2, swiglu, short=False)
+    s = gemm.wide_splits(m, n, k // 2, swiglu)
     cus = 256 - gemm._comm_cus
     if m > 256:
         return _prompt_plan(m, n, k, s, cus)

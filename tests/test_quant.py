@@ -95,7 +95,7 @@ def test_fp8_prompt_plan_splits_no_further():
             for k in (128, 640, 4096, 14336):
                 for swiglu in (False, True):
                     s, bm = quant.fp8_plan(m, n, k, swiglu)
-                    assert 1 <= s <= min(8, gemm.wide_splits(m, n, k // 2, swiglu, short=False))
+                    assert 1 <= s <= min(8, gemm.wide_splits(m, n, k // 2, swiglu))
                     assert bm in (64, 128, 192, 256) and (s == 1 or s * m * n <= gemm._WS_FLOATS)
     assert quant.fp8_plan(2048, 4096, 4096) == (1, 256) and quant.fp8_plan(2816, 4096, 4096) == (1, 192)
 

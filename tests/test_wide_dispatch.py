@@ -334,10 +334,17 @@ def test_pf_row_tile_takes_the_cheapest_walk():
         gemm.release_cus_for_comm()
 
 
-def test_wide_splits_take_short_slices_up_to_128_rows():
-    """Up to 8 slices of 4 K-tiles for split products of up to 128 rows; unsplit ones stay unsplit, and nothing else moves."""
-    assert gemm.wide_splits(32, 2560, 2560) == 8 and gemm.wide_splits(128, 2560, 2048) == 8
-    assert gemm.wide_splits(129, 2560, 2560) == 5 and gemm.wide_splits(32, 2560, 2560, short=False) == 5
-    assert gemm.wide_splits(32, 1024, 1024) == 4 and gemm.wide_splits(32, 1024, 512) == 1
-    assert gemm.wide_splits(64, 4096, 4096) == 8 and gemm.wide_splits(64, 6144, 4096) == 5
-    assert gemm.wide_splits(64, 2560, 7680) == 13 and gemm.wide_splits(64, 8192, 28672) == 4
+@pytest.mark.parametrize("m", [1, 8, 64, 128, 129, 256])
+def test_wide_splits_keep_slices_of_8_k_tiles(m):
+    """A slice's sum is handed on in 16 bits, so no slice is shorter than 8 K-tiles, and where the reserved CUs leave room for as
+    many slices as K gives, a pipeline's stages split as one engine does."""
+    shapes = [(512, 512), (1024, 1024), (1024, 3072), (2560, 2048), (2560, 2560), (4096, 2048), (4096, 4096), (2560, 7680)]
+    alone = [gemm.wide_splits(m, n, k) for n, k in shapes]
+    assert all(s == 1 or k // 64 >= 8 * s for (n, k), s in zip(shapes, alone)), alone
+    gemm.reserve_cus_for_comm(16)
+    try:
+        for (n, k), s in zip(shapes, alone):
+            room = (240 // (n // 128 * -(-m // gemm.wide_row_tile(m, n, k)))) >= min(k // 512, 16)
+            assert not room or gemm.wide_splits(m, n, k) == s, (n, k, s)
+    finally:
+        gemm.release_cus_for_comm()
