@@ -237,20 +237,14 @@ def _prompt_plan(m: int, n: int, k: int, most: int, cus: int) -> Tuple[int, int]
 
 def fp8_plan(m: int, n: int, k: int, swiglu: bool = False) -> Tuple[int, int]:
     """(K slices, row-tile override or 0) of gemm_wide_fp8 for this shape.  Past 256 rows the cheapest
-    grid (:func:`_prompt_plan`) of the CUs that communication leaves.  Default: the bf16 kernel's rule on the 128-K tiles (a K-tile of fp8 holds the bytes of a 64-K bf16 tile); up to 64 rows a split narrow
-    product takes up to 8 slices -- what the reduction loads in one go -- of 4 K-tiles where that is twice as many.  us with
-    the norm behind it, M = 1 / 16 / 64, former -> this: 1024 x 4096 8.9 / 10.0 / 10.4 -> 7.6 / 8.6 / 9.1, 2048 x 2048 9.0 /
-    10.0 / 10.4 -> 7.6 / 8.6 / 9.0 (4 slices), 4096 x 4096 10.0 / 10.8 / 11.5 -> 9.0 / 10.1 / 11.3; 16 slices 10-14, and
-    6144 x 4096 in 5 instead of 4 10.9 / 11.9 / 12.9 -> 11.2 / 12.3 / 13.6."""
+    grid (:func:`_prompt_plan`) of the CUs that communication leaves.  Default: the bf16 kernel's rule on the 128-K tiles (a K-tile
+    of fp8 holds the bytes of a 64-K bf16 tile).  Twice the slices of half the K are 1 to 1.5 us of 9 to 10 faster up to 64
+    rows (4096 x 4096 in 8 instead of 4), but a slice's sum is handed on in 16 bits: with 8 the error of the slabs' sum against 64
+    bits was 3.2e-4 instead of 2.6e-4 for results around 0.01."""
     from . import gemm
     s = gemm.wide_splits(m, n, k // 2, swiglu)
-    cus = 256 - gemm._comm_cus
     if m > 256:
-        return _prompt_plan(m, n, k, s, cus)
-    if m <= 64 and not swiglu and s > 1:
-        c = min(8, cus // (n // 128), (k // 128) // 4)
-        if c >= 2 * s:
-            s = c
+        return _prompt_plan(m, n, k, s, 256 - gemm._comm_cus)
     if knobs.K.fp8_bm128 and not swiglu and s > 1 and 128 < m <= 256:
         tiles = (n // 128) * 2
         return max(1, min(256 // tiles, (k // 128) // 4, 16)), 128

@@ -114,3 +114,20 @@ def test_reserved_cus_leave_small_splits_alone(m):
         assert plans() == alone
     finally:
         gemm.release_cus_for_comm()
+
+
+@pytest.mark.parametrize("m", [1, 16, 64, 65, 128])
+def test_fp8_decode_plan_keeps_slices_of_8_k_tiles(m):
+    """A slice's sum is handed on in 16 bits, so no slice is shorter than 8 K-tiles, and where the reserved CUs leave room for
+    as many slices as K gives, a pipeline's stages split as one engine does."""
+    from distributed_llms_amd.ops import gemm, quant
+    shapes = [(1024, 4096), (2048, 2048), (4096, 4096), (8192, 2048), (8192, 2560), (1280, 8192), (4096, 14336)]
+    alone = [quant.fp8_plan(m, n, k) for n, k in shapes]
+    assert all(s == 1 or k // 128 >= 8 * s for (n, k), (s, _) in zip(shapes, alone)), alone
+    gemm.reserve_cus_for_comm(16)
+    try:
+        for (n, k), p in zip(shapes, alone):
+            room = 240 // (n // 128 * -(-m // gemm.wide_row_tile(m, n, k // 2))) >= min(k // 1024, 16)
+            assert not room or quant.fp8_plan(m, n, k) == p, (n, k, p)
+    finally:
+        gemm.release_cus_for_comm()
