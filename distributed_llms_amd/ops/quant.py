@@ -217,22 +217,25 @@ _SLAB_US, _SLAB_US_PER_MB = 3.0, 0.3
 
 def _prompt_plan(m: int, n: int, k: int, most: int, cus: int) -> Tuple[int, int]:
     """(K slices, row tile) of the cheapest grid past 256 rows.  ``most``: the slabs hold 16 bits, so a product is split no
-    further than the decode rule would split it, and one that this leaves whole stays whole."""
+    further than the decode rule would split it, and one that this leaves whole stays whole.  The slices, which set how the
+    result rounds, are those of the whole chip; ``cus`` -- what communication leaves of it -- moves the row tile alone, which
+    changes no bit: a pipeline's stages round as one engine does."""
     from . import gemm
+
+    def us(s, bm, cus):
+        tile_us, fixed = _ROUND_US[bm]
+        rounds, kt = -(-(n // 128) * -(-m // bm) * s // cus), -(-(k // 128) // s)
+        t = (tile_us + _ROUND_64 * (rounds - 1)) * kt + fixed if bm == 64 else rounds * (tile_us * kt + fixed)
+        return t + (_SLAB_US + _SLAB_US_PER_MB * s * m * n * 4e-6 if s > 1 else 0.0)
+
     best, plan = float("inf"), (1, 256)
     for bm in (256, 192, 128, 64):
-        tile_us, fixed = _ROUND_US[bm]
-        tiles = (n // 128) * -(-m // bm)
         for s in range(1, min(most, 8, max(1, k // 128 // 4)) + 1):
-            if s > 1 and (s * m * n > gemm._WS_FLOATS or tiles * s > cus):
+            if s > 1 and (s * m * n > gemm._WS_FLOATS or (n // 128) * -(-m // bm) * s > 256):
                 break
-            rounds, kt = -(-tiles * s // cus), -(-(k // 128) // s)
-            us = ((tile_us + _ROUND_64 * (rounds - 1)) * kt + fixed if bm == 64 else rounds * (tile_us * kt + fixed))
-            if s > 1:
-                us += _SLAB_US + _SLAB_US_PER_MB * s * m * n * 4e-6
-            if us < best:
-                best, plan = us, (s, bm)
-    return plan
+            if us(s, bm, 256) < best:
+                best, plan = us(s, bm, 256), (s, bm)
+    return plan if cus == 256 else (plan[0], min((256, 192, 128, 64), key=lambda bm: us(plan[0], bm, cus)))
 
 
 def fp8_plan(m: int, n: int, k: int, swiglu: bool = False) -> Tuple[int, int]:

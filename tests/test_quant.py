@@ -131,3 +131,21 @@ def test_fp8_decode_plan_keeps_slices_of_8_k_tiles(m):
             assert not room or quant.fp8_plan(m, n, k) == p, (n, k, p)
     finally:
         gemm.release_cus_for_comm()
+
+
+def test_fp8_prompt_plan_splits_alike_beside_communication():
+    """Past 256 rows a product that the decode rule splits alike with and without CUs reserved for communication gets the same
+    number of slices on both sides (the row tile may differ: it changes no bit)."""
+    from distributed_llms_amd.ops import gemm, quant
+    cases = [(m, n, k, sw) for m in (257, 300, 384, 513, 700, 1000, 2048, 4096) for n in (256, 512, 1024, 2560, 4096)
+             for k in (512, 2048, 4096, 7680, 14336) for sw in (False, True)]
+    plans = lambda: [(gemm.wide_splits(m, n, k // 2, sw), quant.fp8_plan(m, n, k, sw)) for m, n, k, sw in cases]
+    alone = plans()
+    gemm.reserve_cus_for_comm(16)
+    try:
+        beside = plans()
+    finally:
+        gemm.release_cus_for_comm()
+    alike = [(c, a, b) for c, (x, a), (y, b) in zip(cases, alone, beside) if x == y]
+    assert len(alike) > len(cases) // 2
+    assert all(a[0] == b[0] and b[1] in (64, 128, 192, 256) for _, a, b in alike), [v for v in alike if v[1][0] != v[2][0]][:5]
