@@ -1204,11 +1204,11 @@ int* pf_queue(hipStream_t s) {
 }  // namespace
 
 // Persistent prefill GEMM: C = A B^T (mode 0) or SwiGLU (mode 1, C [M, N / 2], B = [Bg; Bu]),
-// bm x 256 tiles, grid = min(tiles, CUs) rounded up to a multiple of 8.  variant bit 16: the
+// bm x 256 tiles, grid = min(tiles, CUs or wgs > 0) rounded up to a multiple of 8.  variant bit 16: the
 // dynamic tile queue (DYN; needs K >= 128) instead of the static tile = w + i P walk; variant 8:
 // nontemporal output stores (by default: SwiGLU outputs > 256 MiB).
 void gemm_pf(uintptr_t c, uintptr_t a, uintptr_t b, int M, int N, int K, int mode, int variant, uintptr_t stream,
-             float limit, int bm, uintptr_t bias) {
+             float limit, int bm, uintptr_t bias, int wgs) {
   const bool dyn = (variant & 16) != 0;
   variant &= ~16;
   DLLM_HOST_CHECK(!dyn || K >= 2 * PBK, "the dynamic tile queue needs K >= 128");
@@ -1238,6 +1238,8 @@ void gemm_pf(uintptr_t c, uintptr_t a, uintptr_t b, int M, int N, int K, int mod
   DLLM_HOST_CHECK(bm == 256 || (!dyn && variant == 0), "row tiles below 256: static walk, default stores");
   const long tiles = (long)(N / 256) * ((M + bm - 1) / bm);
   DLLM_HOST_CHECK(tiles < (1L << 30), "tiles");
+  DLLM_HOST_CHECK(wgs >= 0 && wgs % 8 == 0, "workgroups in eights");
+  if (wgs > 0 && wgs < cus) cus = wgs;
   const long grid = ((tiles < cus ? tiles : cus) + 7) / 8 * 8;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   int* q = dyn ? pf_queue(s) : nullptr;

@@ -95,10 +95,11 @@ def pf_fills(m: int, n: int, device) -> bool:
 _PF_ROUND = {256: 1.0, 224: 0.93, 192: 0.84, 160: 0.76}
 
 
-def pf_row_tile(m: int, n: int, device) -> int:
-    """Row tile with the shortest walk: rounds of the chip times the time of a round.  A single round of 256 rows is
-    gemm_pp's (its epilogue through LDS is 5-7 % faster where no next tile hides the stores), which 224 rows do not beat."""
-    cus = _cus(device)
+def pf_row_tile(m: int, n: int, device, cus: int = 0) -> int:
+    """Row tile with the shortest walk (over ``cus`` CUs, else the whole chip): rounds times the time of a round.  A single round
+    of 256 rows is gemm_pp's (its epilogue through LDS is 5-7 % faster where no next tile hides the stores), which 224 rows
+    do not beat."""
+    cus = cus or _cus(device)
     best, at = 256, None
     for bm, c in _PF_ROUND.items():
         rounds = -(-(-(-m // bm) * (n // 256)) // cus)
@@ -111,14 +112,28 @@ def pf_row_tile(m: int, n: int, device) -> int:
 def _pf_plan(m: int, n: int, k: int, out: int, device) -> int:
     """gemm_pf's row tile for an [m, k] x [n, k]^T product that no decode kernel takes (``out``: output columns), or 0 where
     gemm_pp serves.  Below 256 rows only where gemm_pp would not split K either -- the sums' order stays the same -- and
-    nothing asks for the dynamic tile queue or nontemporal stores."""
+    nothing asks for nontemporal stores.  Beside reserved CUs (or with the dynamic tile queue, whose tiles have 256 rows) a
+    plain product, which gemm_pp rounds alike, is left to that.  A GLU does not change kernels there -- gemm_pp's takes a gate
+    and an up rounded to bf16, gemm_pf's the f32 sums -- so that a pipeline's stages round as one engine does: its row
+    tile, which changes no bit, is the one for the CUs that are left.  us beside 16 reserved CUs, gemm_pp -> this: 28672 x
+    4096 at 300 / 640 / 1232 rows 96 / 165 / 259 -> 67 / 122 / 236, 15360 x
+    2560 at 640 / 1232 / 2300 57 / 109 / 171 -> 44 / 82 / 142."""
     if not knobs.K.pp_persistent or m * out * 2 >= 1 << 31:
         return 0
-    if pp_splits(m, n, k) == 1 and not _comm_cus and not pf_dynamic() and (out == n or m * out * 2 <= 256 << 20):
+    if pp_splits(m, n, k) == 1 and (out == n or m * out * 2 <= 256 << 20):
         bm = pf_row_tile(m, n, device)
         if bm != 256:
-            return bm
+            if not pf_dynamic() and not _comm_cus:
+                return bm
+            if out != n:
+                return pf_row_tile(m, n, device, _pf_wgs(_cus(device)))
     return 256 if pf_fills(m, n, device) else 0
+
+
+def _pf_wgs(cus: int) -> int:
+    """Workgroups of gemm_pf's static walk: one per CU that is left (in eights: as many on every XCD).  One that has to wait
+    for a CU would be waited for with its whole share of the tiles."""
+    return max(8, (cus - _comm_cus) // 8 * 8)
 
 
 def _use_wide(m: int, n: int, k: int, x: torch.Tensor, w: torch.Tensor, swiglu: bool = False) -> bool:
@@ -515,7 +530,8 @@ def linear_pf(x: torch.Tensor, w: torch.Tensor, swiglu: bool = False, variant: i
         variant |= 16                  # per-XCD dynamic tile queues (gemm_pp.hip, DYN)
     _ext.kernels().gemm_pf(y.data_ptr(), x.data_ptr(), w.data_ptr(), m, n, k,
                            4 if gelu else 3 if limit is not None else (1 if swiglu else 0), variant, current_stream(),
-                           0.0 if limit is None else float(limit), bm, 0 if bias is None else bias.data_ptr())
+                           0.0 if limit is None else float(limit), bm, 0 if bias is None else bias.data_ptr(),
+                           _pf_wgs(_cus(x.device)) if _comm_cus and bm < 256 else 0)
     return y
 
 

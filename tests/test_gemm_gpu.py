@@ -399,6 +399,23 @@ def test_clipped_glu_bias_reaches_the_prompt_gemm(cuda, monkeypatch):
         torch.testing.assert_close(y.float(), sm.clipped_glu(gu, b.float(), 0.7), atol=2e-2, rtol=2e-2)
 
 
+@pytest.mark.parametrize("m,n,k", [(300, 8192, 128), (1200, 8192, 256), (2900, 4096, 192), (3400, 8192, 64), (5800, 4096, 192)])
+def test_prompt_glu_bits_beside_communication(cuda, m, n, k):
+    """Prompt GLUs whose 256-row tiles would leave the chip idle give the same bits with CUs reserved for communication: as
+    one and several rounds of short tiles over the CUs that are left, and from the tile queue (static for one K-tile)."""
+    from distributed_llms_amd.ops import seqmix as sm
+    x, w, b = _bf(m, k), _bf(n, k, scale=0.1), torch.randn(n, device="cuda").bfloat16()
+    calls = lambda: [ops.linear_swiglu(x, w), sm.linear_clipped_glu(x, w, None, 0.7), sm.linear_clipped_glu(x, w, b, 0.7),
+                     sm.linear_gelu_glu(x, w)]
+    alone = calls()
+    gemm.reserve_cus_for_comm(16)
+    try:
+        beside = calls()
+    finally:
+        gemm.release_cus_for_comm()
+    assert [torch.equal(a, y) for a, y in zip(alone, beside)] == [True] * 4
+
+
 def test_pf_swiglu_output_range_is_the_half_width(cuda):
     """SwiGLU's output is [M, N / 2]: a 70B prefill gate|up (M 32768, 2I 57344) is within the
     kernel's 2 GiB output range although M x 2I x 2 bytes is not (a small-K stand-in shape)."""

@@ -348,3 +348,23 @@ def test_wide_splits_keep_slices_of_8_k_tiles(m):
             assert not room or gemm.wide_splits(m, n, k) == s, (n, k, s)
     finally:
         gemm.release_cus_for_comm()
+
+
+def test_prompt_glu_keeps_its_kernel_beside_communication():
+    """gemm_pp and gemm_pf round a GLU differently, so which of them serves does not hang on reserved CUs or the tile queue; the
+    row tile beside them is the one for the CUs that are left."""
+    from distributed_llms_amd import knobs
+    cpu = torch.device("cpu")
+    sizes = [(m, n, k) for m in range(257, 4200, 37) for n, k in ((28672, 4096), (15360, 2560), (4096, 1024), (57344, 8192))]
+    alone = [gemm._pf_plan(m, n, k, n // 2, cpu) for m, n, k in sizes]
+    assert any(a not in (0, 256) and not gemm.pf_fills(m, n, cpu) for a, (m, n, _) in zip(alone, sizes))
+    gemm.reserve_cus_for_comm(16)
+    try:
+        for (m, n, k), a in zip(sizes, alone):
+            b = gemm._pf_plan(m, n, k, n // 2, cpu)
+            assert (a == 0) == (b == 0), (m, n, k, a, b)
+            assert b == (a if a in (0, 256) else gemm.pf_row_tile(m, n, cpu, 240)), (m, n, k, a, b)
+    finally:
+        gemm.release_cus_for_comm()
+    with knobs.override(pf_dynamic=True):
+        assert all((a == 0) == (gemm._pf_plan(m, n, k, n // 2, cpu) == 0) for (m, n, k), a in zip(sizes, alone))
