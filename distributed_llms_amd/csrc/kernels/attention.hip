@@ -1614,14 +1614,19 @@ static void decode_launch(uintptr_t out, uintptr_t q, uintptr_t k_cache, uintptr
   // -> 6.2 / 11.3 -> 8.0, 8 of 250 11.9 -> 8.8, 192 of 250 46.3 -> 40.0; 256 of 120 the same 31).
   // The splits of a (sequence, head) as the waves of ONE workgroup (JOIN) save the partials' round trip and the second
   // launch, some 2 us, and pay 0.6 us per 32 keys of 128 (16 KiB) of every wave that a CU gets on top of an even share: us,
-  // apart -> joined, 16 / 32 / 64 sequences of 120 keys in 2 splits 8.8 / 10.7 / 13.8 -> 8.1 / 8.1 / 10.5, 32 of 1000 in 4 28.4
-  // -> 26.2; not 1 of 250 in 4 (8.0, joined 9.7), 16 of 500 in 8 (14.8, 16.5) or 32 of 1000 keys of 64, 12 heads, in 2
-  // (22.3, 25.0: 384 workgroups of two waves on 256 CUs).
+  // apart -> joined, 16 / 32 / 64 sequences of 120 keys in 2 splits 8.8 / 10.7 / 13.8 -> 8.1 / 8.1 / 10.5; not 1 of 250 in 4
+  // (8.0, joined 9.7), 16 of 500 in 8 (14.8, 16.5) or 32 of 1000 keys of 64, 12 heads, in 2 (22.3, 25.0: 384 workgroups of
+  // two waves on 256 CUs).
+  // The lengths are not known here (a captured step's are those of its replays), so the worst batch bounds it as well: one
+  // long sequence among short ones, whose waves share one CU while the others idle.  us, apart -> joined, 32 sequences of 60
+  // keys but one of 500 / 1000 / 2000 / 8000, in 4: 11.9 / 13.4 / 17.3 / 40.8 -> 12.9 / 19.5 / 31.9 / 108.5.  Where the keys past
+  // the first split times the head size stay below 40000, no batch of 196, even and ragged, is more than 0.4 us slower joined; the
+  // line gives up 2 us (32 of 1000: 27.4, joined 25.1) to 4 % (32 of 8000: 170, 163) where all are long.
   const int pairs = batch * hkv;
   const int surplus = num_splits * ((pairs + 255) / 256) - (num_splits * pairs + 255) / 256;
   const long join_bytes = (long)num_splits * (hq / hkv) * (d + 6) * 4;
   const bool join = num_splits > 1 && num_splits <= 8 && join_bytes <= 64 * 1024 &&
-                    (long)surplus * split_len * d < 14000;
+                    (long)surplus * split_len * d < 14000 && (long)(num_splits - 1) * split_len * d < 40000;
   const dim3 grid(join ? 1 : num_splits, hkv, batch);
   auto go = [&](auto kern) {
     hipLaunchKernelGGL(kern, grid, dim3(join ? num_splits * 64 : 64), join ? join_bytes : 0, s, (bf16*)out, (const bf16*)q, (bf16*)k_cache, (bf16*)v_cache,

@@ -387,3 +387,42 @@ def test_decode_attention_joins_splits_in_a_workgroup(cuda, b, hq, hkv, d, ctx, 
     expect = ref.paged_attention_decode(q.float(), kf.bfloat16().float(), vf, bt, sl, d ** -0.5)
     # as above: bf16 probabilities and result, and as much again for a rotated element that rounds the other way
     assert (out.float() - expect).abs().max() <= 2.0 ** -7 * vf.abs().max()
+
+
+@gpu
+@pytest.mark.parametrize("b,hq,hkv,d,ctx,rest,splits,joined", [
+    (64, 16, 8, 128, 120, 120, 2, True), (3, 32, 32, 64, 300, 250, 5, True), (3, 32, 32, 64, 384, 1, 6, True),
+    (16, 16, 8, 64, 448, 447, 7, True), (32, 8, 8, 64, 512, 65, 8, True), (32, 32, 8, 128, 300, 60, 3, True),
+    (32, 32, 8, 128, 1000, 60, 4, False), (64, 16, 8, 128, 700, 33, 2, False)])
+@pytest.mark.parametrize("fused", [False, True])
+def test_decode_attention_join_follows_the_longest_sequence(cuda, b, hq, hkv, d, ctx, rest, splits, joined, fused):
+    """One sequence of ``ctx`` keys among ``rest``: 2 to 8 splits as the waves of a workgroup, which leaves the partials'
+    workspace alone, and apart where the waves of one long sequence would wait for each other on a CU; against float32."""
+    from distributed_llms_amd import knobs
+    torch.manual_seed(b + ctx)
+    lens = [ctx] + [rest] * (b - 1)
+    used, width = sum(-(-n // 32) for n in lens), 1 << (-(-ctx // 32) - 1).bit_length()
+    k, v = torch.randn(used, hkv, 32, d).bfloat16().cuda(), torch.randn(used, hkv, d, 32).bfloat16().cuda()
+    bt, at = torch.zeros(b, width, dtype=torch.int32), 0
+    for i, n in enumerate(lens):
+        bt[i, :-(-n // 32)] = torch.arange(at, at + -(-n // 32))
+        at += -(-n // 32)
+    slots = torch.tensor([int(bt[i, (n - 1) // 32]) * 32 + (n - 1) % 32 for i, n in enumerate(lens)], dtype=torch.int32).cuda()
+    bt, sl = bt.cuda(), torch.tensor(lens, dtype=torch.int32).cuda()
+    kf, vf = k.float(), v.float()
+    ws = (torch.full((b * hq * splits * d,), 7.0, device="cuda"), torch.full((b * hq * splits * 2,), 7.0, device="cuda"))
+    with knobs.override(attn_target_waves=2048 if splits == 8 else knobs.K.attn_target_waves):
+        assert ops.decode_split_plan(b, hkv, ctx, 32, width)[0] == splits
+        if fused:
+            qkv = torch.randn(b, (hq + 2 * hkv) * d).bfloat16().cuda()
+            cs = ref.rope_cos_sin(d, 4096, 500000.0, device="cuda")
+            q = ref.rope_cache_append(qkv.float(), sl - 1, cs, kf, vf, slots, hq, hkv, d).bfloat16()
+            out = ops.paged_attention_decode_rope(qkv, sl - 1, cs, k, v, slots, bt, sl, hq, hkv, d, d ** -0.5, max_ctx=ctx,
+                                                  workspace=ws)
+        else:
+            q = torch.randn(b, hq, d).bfloat16().cuda()
+            out = ops.paged_attention_decode(q, k, v, bt, sl, d ** -0.5, max_ctx=ctx, workspace=ws)
+    assert all(bool((t == 7.0).all()) for t in ws) == joined
+    expect = ref.paged_attention_decode(q.float(), kf.bfloat16().float(), vf, bt, sl, d ** -0.5)
+    # as above: bf16 probabilities and result, and as much again for a rotated element that rounds the other way
+    assert (out.float() - expect).abs().max() <= 2.0 ** -7 * vf.abs().max()
