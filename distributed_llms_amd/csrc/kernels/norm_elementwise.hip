@@ -191,15 +191,19 @@ __global__ void __launch_bounds__(256) rope_cache_kernel(bf16* __restrict__ q_ou
 // path scatters eight 2-byte stores (whole 64-byte lines instead of partial ones).  Any other group (a prompt boundary
 // inside it, a sequence resuming mid-group, the batch tail) takes the scatter.
 //
-// Slabs (SC > 0: their number, -1: a runtime number) are summed in slab order and rounded to bf16, as splitk_reduce sums
+// Slabs (SC > 0: their number) are summed in slab order and rounded to bf16, as splitk_reduce sums
 // them, on the way: a prompt of 128 tokens of 32 / 8 heads took a launch for the sum (3.7 us), one for K (3.3) and one for V
-// (4.1).  q_out: the rotated q, or (rotate_q 0, slabs only: the attention rotates it) the summed one.
+// (4.1); 2 / 3 / 4 / 5 / 8 slabs, sum and append 9.4 / 9.7 / 10.0 / 10.2 / 10.8 us -> 8.4 / 8.8 / 9.3 / 9.5 / 10.1.
+// Only the compiled numbers of slabs (rope_cache_append below): a workgroup's eight tokens are one CU's loads, so a
+// loop over more of them is slower than the sum's own launch, which spreads over the chip (128 tokens of 32 / 4 heads, 6 / 13 /
+// 17 slabs, sum and append 8.9 / 11.8 / 13.1 us; summed here one by one 23.6 / 47 / 61, eight at a time 11.3 / 20 / 25).
+// q_out: the rotated q, or (rotate_q 0, slabs only: the attention rotates it) the summed one.
 constexpr int kAppendCols = 1024;
 
 template <int SC>
 __global__ void __launch_bounds__(256) qkv_append_kernel(bf16* __restrict__ q_out, int rotate_q,
                                                          const bf16* __restrict__ qkv, const float* __restrict__ part,
-                                                         int nparts, long slab, const int32_t* __restrict__ positions,
+                                                         long slab, const int32_t* __restrict__ positions,
                                                          const float* __restrict__ cos_sin, bf16* __restrict__ k_cache,
                                                          bf16* __restrict__ v_cache, const int32_t* __restrict__ slots,
                                                          int tokens, int hq, int hkv, int d, int bs) {
@@ -225,14 +229,10 @@ __global__ void __launch_bounds__(256) qkv_append_kernel(bf16* __restrict__ q_ou
         l[s] = __builtin_nontemporal_load(reinterpret_cast<const raw4*>(reinterpret_cast<const part_elem*>(part) + p + s * slab));
     }
   };
-  auto finish = [&](const raw4 (&l)[NS], size_t p) {
+  auto finish = [&](const raw4 (&l)[NS]) {
     f32x4 a = {0.f, 0.f, 0.f, 0.f};
-    if constexpr (SC == -1) {
-      for (int s = 0; s < nparts; ++s) a += part_load4<true>(part, p + s * slab);
-    } else {
 #pragma unroll
-      for (int s = 0; s < NS; ++s) a += f32x4{part_value(l[s][0]), part_value(l[s][1]), part_value(l[s][2]), part_value(l[s][3])};
-    }
+    for (int s = 0; s < NS; ++s) a += f32x4{part_value(l[s][0]), part_value(l[s][1]), part_value(l[s][2]), part_value(l[s][3])};
     return bf16x4{f2bf(a[0]), f2bf(a[1]), f2bf(a[2]), f2bf(a[3])};
   };
   if (what == 2) {
@@ -251,7 +251,7 @@ __global__ void __launch_bounds__(256) qkv_append_kernel(bf16* __restrict__ q_ou
         const int i = i0 + u * 256;
         if (i >= total) break;
         const int j = i / per;
-        if constexpr (SC != 0) v[u] = finish(l[u], (size_t)(t0 + min(j, n - 1)) * width + col0 + (i % per) * 4);
+        if constexpr (SC != 0) v[u] = finish(l[u]);
         *reinterpret_cast<bf16x4*>(&tile[j][(i % per) * 4]) = v[u];
       }
     }
@@ -310,9 +310,8 @@ __global__ void __launch_bounds__(256) qkv_append_kernel(bf16* __restrict__ q_ou
       if (i >= total) break;
       const int t = t0 + i / per, h = h0 + (i % per) / qpr, e = (i % qpr) * 4;
       if constexpr (SC != 0) {
-        const size_t p = (size_t)t * width + col0 + (h - h0) * d + e;
-        x1[u] = finish(l1[u], p);
-        x2[u] = finish(l2[u], p + half);
+        x1[u] = finish(l1[u]);
+        x2[u] = finish(l2[u]);
       }
       bf16x4 o1 = x1[u], o2 = x2[u];
       if (rot) {
@@ -352,8 +351,8 @@ void rope_cache_append(uintptr_t q_out, int rotate_q, uintptr_t qkv, uintptr_t p
   const int hpc = d > kAppendCols ? 1 : kAppendCols / d;
   const dim3 grid((tokens + 7) / 8, 2 * ((hkv + hpc - 1) / hpc) + (q_out ? (hq + hpc - 1) / hpc : 0));
   auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, (bf16*)q_out, rotate_q, (const bf16*)qkv, (const float*)part, nparts,
-                       slab, (const int32_t*)positions, (const float*)cos_sin, (bf16*)k_cache, (bf16*)v_cache,
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, (bf16*)q_out, rotate_q, (const bf16*)qkv, (const float*)part, slab,
+                       (const int32_t*)positions, (const float*)cos_sin, (bf16*)k_cache, (bf16*)v_cache,
                        (const int32_t*)slots, tokens, hq, hkv, d, bs);
   };
   switch (part ? nparts : 0) {
@@ -363,7 +362,7 @@ void rope_cache_append(uintptr_t q_out, int rotate_q, uintptr_t qkv, uintptr_t p
     case 4: go(qkv_append_kernel<4>); break;
     case 5: go(qkv_append_kernel<5>); break;
     case 8: go(qkv_append_kernel<8>); break;
-    default: go(qkv_append_kernel<-1>);
+    default: DLLM_HOST_CHECK(false, "2, 3, 4, 5 or 8 slabs (ops.APPEND_SLABS)");
   }
   DLLM_HIP_CHECK(hipGetLastError());
 }

@@ -306,7 +306,7 @@ class ModelStage:
 
     def _attention(self, qkv, li: int, meta: BatchMeta) -> torch.Tensor:
         """``qkv``: [T, (Hq + 2 Hkv) D] or, from a split-K projection, a SplitKPartial that the fused
-        decode kernel and the K / V append reduce themselves."""
+        decode kernel and (``ops.APPEND_SLABS``) the K / V append reduce themselves."""
         cfg = self.cfg
         k_cache, v_cache = self.kv.layer(li)
         fused = not meta.is_prefill and knobs.K.fused_rope and \
@@ -318,6 +318,8 @@ class ModelStage:
                                                 workspace=meta.attn_workspace)
             return o.view(o.shape[0], self.q_size_local)
         part = isinstance(qkv, ops.gemm.SplitKPartial)
+        if part and qkv.splits not in ops.APPEND_SLABS:
+            qkv, part = qkv.materialize(), False
         if meta.is_prefill and not meta.num_decode and (part or qkv.is_cuda) and \
                 ops.prefill_rope_in_attention(meta.block_tables.shape[1]):
             q = ops.rope_cache_append(qkv, meta.positions, self.cos_sin, k_cache, v_cache, meta.slot_mapping,

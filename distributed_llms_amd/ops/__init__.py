@@ -187,14 +187,23 @@ def silu_mul(gu: torch.Tensor) -> torch.Tensor:
 
 
 # ----------------------------------------------------------- K4 + K5
+APPEND_SLABS = (2, 3, 4, 5, 8)    # numbers of split-K slabs that the K / V append sums itself (norm_elementwise.hip)
+
+
 def rope_cache_append(qkv, positions, cos_sin, k_cache, v_cache, slot_mapping, num_heads, num_kv_heads,
                       head_dim, write_q: bool = True) -> Optional[torch.Tensor]:
     """Rotate k (and q) and append k / v^T to the paged cache; returns the rotated q [T, Hq, D], or
     None with ``write_q=False`` (the prefill attention then rotates q itself).
 
     ``qkv`` may be a :class:`gemm.SplitKPartial`, whose slabs are then summed on the way (bit-identical to reducing
-    first); with ``write_q=False`` the q columns come back summed and unrotated, [T, Hq * D]."""
+    first, which other numbers than ``APPEND_SLABS`` take); with ``write_q=False`` the q columns come back summed and
+    unrotated, [T, Hq * D]."""
     part = qkv if isinstance(qkv, gemm.SplitKPartial) else None
+    if part is not None and part.splits not in APPEND_SLABS:
+        whole = part.materialize()
+        q = rope_cache_append(whole, positions, cos_sin, k_cache, v_cache, slot_mapping, num_heads, num_kv_heads, head_dim,
+                              write_q)
+        return q if write_q else whole[:, :num_heads * head_dim].contiguous()
     if part is None and not _gpu(qkv):
         q = ref.rope_cache_append(qkv, positions, cos_sin, k_cache, v_cache, slot_mapping, num_heads,
                                   num_kv_heads, head_dim)

@@ -149,6 +149,28 @@ def test_rope_cache_append_sums_slabs(cuda, hq, hkv, d, tokens, slabs):
     assert torch.equal(v1, vr)
 
 
+@pytest.mark.parametrize("slabs", [1, 2, 3, 4, 5, 6, 8, 13, 17])
+def test_rope_cache_append_leaves_other_slab_counts_to_the_sum(cuda, monkeypatch, slabs):
+    """Numbers of slabs that the append has no form for are summed by the launch that spreads over the chip, not one slab after
+    the other: the same bits, k, v and q."""
+    from distributed_llms_amd.ops import gemm
+    sums, real = [], gemm.SplitKPartial.materialize
+    monkeypatch.setattr(gemm.SplitKPartial, "materialize", lambda p: (sums.append(p.splits), real(p))[1])
+    t, hq, hkv, d = 45, 8, 1, 128
+    width = (hq + 2 * hkv) * d
+    p = gemm.SplitKPartial((torch.randn(slabs, t, width, device="cuda") / 64).half(), slabs, t, width, (t, width),
+                           torch.bfloat16, torch.device("cuda"))
+    whole = real(p)
+    pos, cs = torch.arange(t, dtype=torch.int32, device="cuda"), ref.rope_cos_sin(d, 1024, 500000.0, device="cuda")
+    caches = [_cache(6, hkv, d) for _ in range(3)]
+    want = ops.rope_cache_append(whole, pos, cs, *caches[0], pos, hq, hkv, d)
+    got = ops.rope_cache_append(p, pos, cs, *caches[1], pos, hq, hkv, d)
+    plain = ops.rope_cache_append(p, pos, cs, *caches[2], pos, hq, hkv, d, write_q=False)
+    assert sums == ([] if slabs in (2, 3, 4, 5, 8) else [slabs] * 2)
+    assert torch.equal(got, want) and torch.equal(plain, whole[:, :hq * d]) and plain.is_contiguous()
+    assert all(torch.equal(a, b) for c in caches[1:] for a, b in zip(c, caches[0]))
+
+
 def _fill_paged(seq_lens, hkv, d, nb_total=None):
     bs = 32
     nblocks = [(n + bs - 1) // bs for n in seq_lens]
