@@ -46,7 +46,7 @@ def gemm_only(xq, xs, w, m, n, k, sw, y, splits=0, bm=0, grp=False):
         s, bm0 = splits, bm
     bm = bm0
     ws = gemm._workspace(xq.device)
-    v = (1 if m <= 256 else (4 | (64 if grp else 0))) | (bm << 8)
+    v = quant.fp8_variant(m, n, k, s, bm) | (64 if grp else 0)
     _ext.kernels().gemm_wide_fp8(y.data_ptr(), xq.data_ptr(), xs.data_ptr(), w.q.data_ptr(), w.scale.data_ptr(),
                                  ws.data_ptr(), ws.numel(), m, n, k, s, 1 if sw else 0, v,
                                  torch.cuda.current_stream().cuda_stream)

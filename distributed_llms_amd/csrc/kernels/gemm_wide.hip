@@ -824,19 +824,16 @@ int gemm_wide_fp8(uintptr_t c, uintptr_t a, uintptr_t a_scale, uintptr_t b, uint
   const long grid = (long)ntiles * mtiles * S;
   DLLM_HOST_CHECK(grid >= 1 && grid < (1L << 31), "grid");
   if (S > 1) DLLM_HOST_CHECK(ws != 0 && (long)S * M * N <= ws_floats, "split-K workspace too small");
-  // weights nt in rotated K order where the grid has no K split (as the bf16 kernel's variant 1); variant | 64: grouped
-  // row-tile order for large M (no K split)
-  const bool rot = (variant & 7) != 4 && S == 1;
+  // variant & 7 == 4: the default cache policy, else weights nontemporal (ops/quant.fp8_variant), in rotated K order where the
+  // grid has no K split (as the bf16 kernel's variant 1); variant | 64: grouped row-tile order for large M (no K split)
+  const bool nt = (variant & 7) != 4, rot = nt && S == 1;
   const bool grp = (variant & 64) != 0 && S == 1 && !rot;
   // Ring: as deep as the LDS allows (6 x 24 KiB at 64 rows, 5 x 32 KiB at 128) for up to one workgroup per CU, where the
-  // K loop waits for weight bytes in flight: gate|up 28672 x 4096, M = 1 / 64 / 128: 24.0 / 26.1 / 30.8 -> 22.7 / 24.3 / 29.5 us.
-  // Split grids (up to one workgroup per CU by their plan): weights nontemporal from 8 K-tiles a slice (12 past 64 rows) of a
-  // matrix that the Infinity Cache does not keep from step to step, and the deep ring from 14, with the norm that sums the
-  // slabs behind it: 4096 x 14336 (14 K-tiles) 16.8 / 18.2 / 21.7 -> 15.5 / 17.9 / 21.2, 6144 x 4096 (8) 11.7 / 13.9 -> 10.9 /
-  // 13.5, 8192 x 28672 (56) 48.8 / 52.1 / 60.6 -> 43.5 / 48.0 / 58.0; 4096 x 4096 in 4 K-tiles 10.9 -> 11.9 at M = 64.
+  // K loop waits for weight bytes in flight: gate|up 28672 x 4096, M = 1 / 64 / 128: 24.0 / 26.1 / 30.8 -> 22.7 / 24.3 / 29.5 us;
+  // on split grids (up to one workgroup per CU by their plan) with nontemporal weights from 14 K-tiles a slice: 4096 x 14336 and
+  // its norm 16.8 / 18.2 -> 15.5 / 17.9 at M = 1 / 64 with both.
   const bool one_round = S == 1 && grid <= 256;
-  const bool nt_split = S > 1 && (long)N * K >= (12L << 20) && kts >= (M <= 64 ? 8 : 12);
-  const bool deep_split = nt_split && BM == 64 && kts >= 14;
+  const bool nt_split = nt && S > 1, deep_split = nt_split && BM == 64 && kts >= 14;
 #define DLLM_F8_GO3(BM_, SPLIT_, SW_, V_, NB_)                                                                   \
   hipLaunchKernelGGL((gemm_wide_fp8_kernel<BM_, SPLIT_, SW_, NB_, V_>), dim3((unsigned)grid), dim3(512), 0, s,    \
                      (const uint8_t*)a, (const uint8_t*)b, (const float*)a_scale, (const float*)b_scale,        \

@@ -258,6 +258,24 @@ def fp8_splits(m: int, n: int, k: int, swiglu: bool = False) -> int:
     return fp8_plan(m, n, k, swiglu)[0]
 
 
+def fp8_variant(m: int, n: int, k: int, splits: int, bm: int) -> int:
+    """gemm_wide_fp8's variant: cache policy of the weights (4: the default one, 1: nontemporal), tile order (64: grouped) and
+    row-tile override.  Nontemporal where a weight byte is read once: up to 256 rows without a K split, and with one where a
+    single row tile covers M, the slices are long (8 K-tiles; past 64 rows 12) and the Infinity Cache does not keep the matrix
+    from step to step.  With the norm that sums the slabs behind it, default -> nontemporal, us: 6144 x 4096 (8 K-tiles) 11.7 /
+    13.9 -> 10.9 / 13.5 at M = 1 / 64, 8192 x 28672 (56) 48.8 / 52.1 / 60.6 -> 43.5 / 48.0 / 58.0 at M = 1 / 64 / 128; but read by
+    several row tiles 4096 x 14336 at M = 200 / 300 34.7 / 41.0 -> 36.2 / 42.8, 5120 x 25600 66.7 / 77.2 -> 69.5 / 81.6 (from 384
+    rows on within 2 % either way) -- unless those are of 64 rows with the deep ring that goes with it (2048 x 8192 at 300, five
+    row tiles, 25.4 -> 24.3)."""
+    order = 64 if 0 < knobs.K.fp8_group_m <= (2 * m if 0 < bm < 256 else m) else 0
+    if splits == 1:
+        return (1 if m <= 256 else 4 | order) | (bm << 8)
+    from . import gemm
+    rows, kt = bm or gemm.wide_bm(m), -(-(k // 128) // splits)
+    nt = n * k >= 12 << 20 and (kt >= (8 if m <= 64 else 12) if m <= rows else rows == 64 and kt >= 14)
+    return (1 if nt else 4) | (bm << 8)
+
+
 def linear_fp8(x: torch.Tensor, w: Fp8Weight, swiglu: bool = False, defer: bool = False, splits: int = 0):
     """y = x w^T (``swiglu``: silu(x Wg^T) * (x Wu^T), w = [Wg; Wu]) with W8A8 e4m3 operands.
     ``defer``: may return a :class:`~distributed_llms_amd.ops.gemm.SplitKPartial` (no SwiGLU)."""
@@ -286,9 +304,7 @@ def linear_fp8(x: torch.Tensor, w: Fp8Weight, swiglu: bool = False, defer: bool 
     ws = _workspace(x.device)
     if s > 1 and s * m * n > ws.numel():
         s = max(1, ws.numel() // (m * n))
-    # weights streamed non-temporal only where one row tile covers M (each weight byte read once)
-    grouped = 0 < knobs.K.fp8_group_m <= (2 * m if 0 < bm < 256 else m)
-    variant = (1 if m <= 256 else (4 | (64 if grouped else 0))) | (bm << 8)
+    variant = fp8_variant(m, n, k, s, bm)
     stream = current_stream()
     kern = _ext.kernels()
     if defer and not swiglu and s > 1:

@@ -149,3 +149,17 @@ def test_fp8_prompt_plan_splits_alike_beside_communication():
     alike = [(c, a, b) for c, (x, a), (y, b) in zip(cases, alone, beside) if x == y]
     assert len(alike) > len(cases) // 2
     assert all(a[0] == b[0] and b[1] in (64, 128, 192, 256) for _, a, b in alike), [v for v in alike if v[1][0] != v[2][0]][:5]
+
+
+def test_fp8_weights_read_by_several_row_tiles_are_cached():
+    """Nontemporal weights only where one row tile reads them (or the deep ring of 64-row tiles goes with it); short slices and
+    small matrices keep the default policy."""
+    from distributed_llms_amd.ops import quant
+    policy = lambda m, n, k: quant.fp8_variant(m, n, k, *quant.fp8_plan(m, n, k)) & 7
+    assert [policy(m, 4096, 14336) for m in (1, 64, 128)] == [1, 1, 1]
+    assert [policy(m, 4096, 14336) for m in (129, 256, 300, 640, 1024)] == [4] * 5
+    assert [policy(m, 8192, 28672) for m in (64, 200, 300)] == [1, 4, 4]
+    assert policy(300, 2048, 8192) == 1 and quant.fp8_plan(300, 2048, 8192) == (3, 64)
+    assert policy(1, 6144, 4096) == 1 and policy(100, 6144, 4096) == 4 and policy(64, 1024, 8192) == 4
+    assert policy(64, 28672, 4096) == 1 and quant.fp8_variant(4096, 28672, 4096, 1, 256) == 4 | 64 | 256 << 8
+    assert quant.fp8_variant(2100, 4096, 4096, 1, 192) == 4 | 64 | 192 << 8 and quant.fp8_variant(2100, 4096, 4096, 1, 0) == 4
