@@ -177,13 +177,16 @@ def _use_wide(m: int, n: int, k: int, x: torch.Tensor, w: torch.Tensor, swiglu: 
 #    11.4 / 12.6, 13.4 / 14.0 / 14.4; 10240 x 8192 28.6 / 29.8 / 32.3, 32.4 / 32.7 / 31.6; 4096 x 8192 16.4 / 16.3, 16.0 / 15.6;
 #  * in front of a close the line stays: 2560 x 7680 at 16 rows in a decode step 12.8 + 4.6 (close), 9.4 + 5.1;
 #  * GLU: 16384 x 4096 24.7 / 23.6 / 25.8, 32.6 / 32.7 / 33.0; 14336 x 5120 25.8 / 24.8 / 26.0, 30.4 / 29.9 / 30.6; 28672 x 4096
-#    38.6 / 37.3 / 42.1, 38.1 / 36.6 / 36.8.
+#    38.6 / 37.3 / 42.1, 38.1 / 36.6 / 36.8; also where a round of the 16- or 32-column workgroups of more rows would leave CUs
+#    idle: 10240 x 4096 16.9 / 16.9 / 17.5, 18.6 / 19.1 / 19.3; 22016 x 4096 30.9 / 31.1 / 31.9, 31.9 / 32.6 / 32.9; 17408 x 2560
+#    17.2 / 17.7 / 19.4, 25.0 / 26.0 / 26.7.  With 4 KiB strides a third round of 24-row workgroups is too much for two groups
+#    of x: 27648 x 2048 21.3 / 21.2 / 23.5, 21.0 / 21.1 / 21.1.
 STREAM_MAX_M = 64
 
 
 def _stream_fill(cols: int) -> float:
-    """Share of the CUs that a round of gemm_stream's workgroups for ``cols`` output columns keeps busy (its launcher's rule:
-    tiles of 16 columns, of 32 once there are more than 256)."""
+    """Share of the CUs that a round of gemm_stream's workgroups for ``cols`` output columns keeps busy past 16 rows (its
+    launcher's rule there: tiles of 16 columns, of 32 once there are more than 256)."""
     tiles = -(-cols // 16)
     tiles = -(-cols // 32) if tiles > 256 else tiles
     return tiles / (256 * -(-tiles // 256))
@@ -194,10 +197,12 @@ def stream_fits(m: int, n: int, k: int, glu: str = "", defer: bool = False, bias
     if not 1 <= m <= STREAM_MAX_M or k % 64 or k < 512:
         return False                                 # K < 512: fewer K-tiles than waves, and no split to save either
     mi = n * k / (1 << 20)
+    if glu and m <= 16:
+        return k <= 5120 and mi <= 96 and (m <= 8 or n <= 24576 or k % 2048 != 0)
     if glu:
-        if k > (5120 if m <= 16 else 4096 if m <= 32 else 2560) or (mi > (20 if m <= 32 else 12) and _stream_fill(n // 2) < 0.75):
+        if k > (4096 if m <= 32 else 2560) or (mi > (20 if m <= 32 else 12) and _stream_fill(n // 2) < 0.75):
             return False
-        return mi <= (96 if m <= 16 else 64 if m <= 32 and glu != "silu" else 40)
+        return mi <= (64 if m <= 32 and glu != "silu" else 40)
     if n > 65536:
         return False                                 # an LM head fills the chip unsplit on the wide kernel
     if defer and n % 128 == 0:

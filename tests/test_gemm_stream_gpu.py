@@ -177,9 +177,9 @@ def test_stream_rule():
     assert not gemm.stream_fits(16, 1024, 8192, defer=True) and not gemm.stream_fits(17, 512, 4096, defer=True)
     assert gemm.stream_fits(16, 32000, 1024) and not gemm.stream_fits(17, 32000, 1024) and not gemm.stream_fits(16, 8192, 4096)
     assert gemm.stream_fits(16, 5120, 4096) and not gemm.stream_fits(32, 5120, 4096)
-    # GLU: a round of workgroups that leaves CUs idle, K past 4096
-    assert gemm.stream_fits(32, 16384, 4096, "gelu") and not gemm.stream_fits(1, 22016, 4096, "gelu")
-    assert not gemm.stream_fits(1, 10240, 4096, "silu") and not gemm.stream_fits(1, 4096, 8192, "clipped")
+    # GLU: past 16 rows a round of workgroups that leaves CUs idle (up to 16 they are cut evenly), K past 4096
+    assert gemm.stream_fits(32, 16384, 4096, "gelu") and not gemm.stream_fits(17, 22016, 4096, "gelu")
+    assert not gemm.stream_fits(17, 10240, 4096, "silu") and not gemm.stream_fits(1, 4096, 8192, "clipped")
     x, w = torch.zeros(4, 512, dtype=torch.bfloat16), torch.zeros(256, 512, dtype=torch.bfloat16)
     assert gemm.use_stream(4, 256, 512, x, w)
     assert not gemm.use_stream(4, 256, 512, x.float(), w) and not gemm.use_stream(4, 256, 512, x, w.t().contiguous().t())
@@ -195,3 +195,13 @@ def test_stream_rule_up_to_16_rows():
     assert not gemm.stream_fits(16, 2560, 7680, defer=True)
     assert gemm.stream_fits(16, 16384, 4096, "silu") and not gemm.stream_fits(17, 16384, 4096, "silu")
     assert gemm.stream_fits(16, 14336, 5120, "silu") and not gemm.stream_fits(1, 27648, 5120, "silu")
+
+
+def test_stream_rule_of_glus_up_to_16_rows_follows_the_cut():
+    """A GLU's workgroups of up to 16 rows are cut evenly, so no size is left out for a round of 16 or 32 columns that they do not
+    have; with 4 KiB strides and two groups of x the line lies at two rounds of 24 rows."""
+    for m in (1, 8, 16):
+        assert all(gemm.stream_fits(m, n, k, "silu") for n, k in ((10240, 4096), (22016, 4096), (17408, 2560), (11008, 5120), (24576, 2048)))
+    assert not gemm.stream_fits(17, 10240, 4096, "silu") and not gemm.stream_fits(32, 22016, 4096, "clipped")
+    assert gemm.stream_fits(8, 27648, 2048, "silu") and not gemm.stream_fits(9, 27648, 2048, "silu")
+    assert gemm.stream_fits(16, 27648, 2560, "silu")
