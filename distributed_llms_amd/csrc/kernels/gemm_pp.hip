@@ -266,11 +266,20 @@ __device__ __forceinline__ void gemm_pp_tile(bf16 (&smem)[SMEM], const bf16* __r
     lane_off[kh] = (uint32_t)((lane & 15) * 128 + ((4 * kh + (lane >> 4)) ^ (((lane & 15) >> 1) & 7)) * 16);
   const uint32_t a_off = (uint32_t)(wm * TM * 128), b_off = (uint32_t)(BM * 128 + wn * TN * 128);
 
+  // Cleared in place behind the first pieces: left to hipcc, the accumulators were cleared in front of the branch on nt and again
+  // behind it, 128 to 256 writes before the first load (256 x 28672 x 4096 with its SwiGLU 59.1 -> 58.6 us, 600 x 4096 x 4096 in 5
+  // slices 35.0 -> 34.4)
   f32x4 acc[RT][CT];
+  auto clear = [&]() {
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int i = 0; i < RT; ++i)
+    for (int i = 0; i < RT; ++i)
 #pragma unroll
-    for (int j = 0; j < CT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < CT; ++j) {
+        acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        asm volatile("" : "+a"(acc[i][j]));
+      }
+  };
 
   // fragments of one K-half: fa[RT] (A rows of the wave tile), fb[CT] (B rows); two sets, so
   // the next K-half's reads are in flight under this one's MFMAs (software pipeline)
@@ -311,6 +320,7 @@ __device__ __forceinline__ void gemm_pp_tile(bf16 (&smem)[SMEM], const bf16* __r
     for (int j = 0; j < NB; ++j)
 #pragma unroll
       for (int p = 0; p < G; ++p) piece(j, j, p);
+    clear();
     pp_vm<(NB - 1) * G>();
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -388,6 +398,8 @@ __device__ __forceinline__ void gemm_pp_tile(bf16 (&smem)[SMEM], const bf16* __r
       float* rec = D + ((size_t)blockIdx.x * 4 + wv) * 128;
       if (lane < 6) rec[lane < 4 ? lane : lane + 16] = vals[lane < 6 ? lane : 0];
     }
+  } else {
+    clear();
   }
   } else {
   if (nt > 0) {
@@ -399,6 +411,7 @@ __device__ __forceinline__ void gemm_pp_tile(bf16 (&smem)[SMEM], const bf16* __r
     for (int j = 0; j < NB; ++j)
 #pragma unroll
       for (int p = 0; p < G; ++p) piece(j, j, p);
+    clear();
     pp_wait_n<G>(NB - 1);
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -499,6 +512,8 @@ __device__ __forceinline__ void gemm_pp_tile(bf16 (&smem)[SMEM], const bf16* __r
       float* rec = D + ((size_t)blockIdx.x * 4 + wv) * 128;
       if (lane < 4) rec[lane] = vals[lane & 3];
     }
+  } else {
+    clear();
   }
   }
   // ---- epilogue: accumulators -> LDS output image (8-byte writes) -> 16-byte row stores.
