@@ -384,6 +384,26 @@ def test_pf_clipped_glu_bias(cuda, m, bm, f, k):
     assert bool(((gemm.linear_pf(x, w, limit=0.7, bm=bm, bias=b).double() - ref).abs() <= tol).all())
 
 
+@pytest.mark.parametrize("bm", [160, 192, 224, 256])
+@pytest.mark.parametrize("k", [64, 192])
+def test_pf_clipped_glu_bias_over_several_tiles(cuda, bm, k):
+    """Workgroups that walk on to tiles of another column tile take that one's bias, beside the next tile's pieces in flight: 18
+    to 29 row tiles of 16 column tiles on 256 CUs, a short last row tile, a bias that moves with the column."""
+    m, f = 4500, 2048
+    assert -(-m // bm) * (2 * f // 256) > 256 and m % bm
+    torch.manual_seed(bm + k)
+    x, w = _bf(m, k), _bf(2 * f, k, scale=0.1)
+    b = (torch.randn(2 * f, device="cuda") * 0.3 + torch.linspace(-0.6, 0.6, 2 * f, device="cuda")).bfloat16()
+    assert torch.equal(gemm.linear_pf(x, w, limit=0.7, bm=bm, bias=torch.zeros_like(b)), gemm.linear_pf(x, w, limit=0.7, bm=bm))
+    y = gemm.linear_pf(x, w, limit=0.7, bm=bm, bias=b)
+    z = x.double() @ w.double().t() + b.double()
+    g, u = z[:, :f].clamp(max=0.7), z[:, f:].clamp(-0.7, 0.7)
+    ref = g * torch.sigmoid(1.702 * g) * (u + 1)
+    e = (x.double().abs() @ w.double().abs().t() + b.double().abs()) * (k + 1) * 2.0 ** -24        # f32 sums, any order
+    tol = 1.2 * e[:, :f] * 1.7 + 0.8 * e[:, f:] + (2.0 ** -8 + 2.0 ** -18) * ref.abs() + 2.0 ** -22
+    assert bool(((y.double() - ref).abs() <= tol).all())
+
+
 def test_clipped_glu_bias_reaches_the_prompt_gemm(cuda, monkeypatch):
     """A biased clipped GLU over a prompt: in the GEMM's epilogue where its bias can be read there, else behind it."""
     from distributed_llms_amd.ops import seqmix as sm

@@ -82,9 +82,10 @@ def test_stream_rows_per_workgroup(cuda, m, n, k):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("half,k,m", [(4096, 64, 16), (5120, 64, 3), (7681, 64, 16), (10240, 64, 16), (3072, 2048, 1), (8192, 2048, 16)])
+@pytest.mark.parametrize("half,k,m", [(1024, 128, 1), (1024, 128, 16), (4096, 64, 16), (5120, 64, 3), (7681, 64, 16), (10240, 64, 16),
+                                      (3072, 2048, 1), (8192, 2048, 16)])
 def test_stream_glu_rows_per_workgroup(cuda, half, k, m):
-    """Every GLU cut (8, 12, 16, 24 and 32 columns), with biases."""
+    """Every GLU cut (8, 8, 16, 24, 32, 24, 12 and 16 columns), with biases."""
     x, w = torch.randn(m, k, device="cuda").bfloat16(), (torch.randn(2 * half, k, device="cuda") * k ** -0.5).bfloat16()
     b = torch.randn(2 * half, device="cuda").bfloat16()
     z = F.linear(x.double(), w.double(), b.double())

@@ -344,6 +344,10 @@ def test_prefill_attention_with_q_rope_in_kernel(cuda, hq, hkv, d, version):
         two_pass = ops.paged_attention_prefill(q, k1, v1, bt, cu, sl, scale)
         assert ops.rope_cache_append(qkv, pos, cs, k2, v2, slots, hq, hkv, d, write_q=False) is None
         fused = ops.paged_attention_prefill_rope(qkv, pos, cs, k2, v2, bt, cu, sl, hq, d, scale, max_q_len=max(qlen))
+        # from rows that hold the q columns alone (what the append of a projection in slabs leaves): the same bits
+        only_q = ops.paged_attention_prefill_rope(qkv[:, :hq * d].contiguous(), pos, cs, k2, v2, bt, cu, sl, hq, d, scale,
+                                                  max_q_len=max(qlen))
+    assert torch.equal(only_q, fused)
     assert torch.equal(k1, k2) and torch.equal(v1, v2)
     torch.testing.assert_close(fused.float(), two_pass.float(), atol=4e-3, rtol=4e-3)
     expect = ref.paged_attention_prefill(ref.rope_q(qkv.float(), pos, cs, hq, d), k1.float(), v1.float(), bt, cu,
