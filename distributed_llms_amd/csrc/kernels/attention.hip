@@ -147,9 +147,9 @@ __device__ __forceinline__ void init_state(WaveState<D>& st) {
 // pipeline -- chunk c+1's K/V loads are in flight while chunk c's MFMAs and softmax run --
 // and the chunk -> block ids come from one lane-parallel load of the block-table row
 // (read back with readlane), so the only dependent HBM latency per chunk is the KV
-// stream itself.  No LDS, no barrier.  num_splits > 1 writes (o, m, l) partials for the
-// split-reduce kernel below, or (JOIN) to LDS, where the workgroup sums them.  (The first version used 4 waves per (split, head, seq) with
-// chunks round-robin, no cross-chunk prefetch and an LDS combine: 47 us per layer at
+// stream itself; no LDS and no barrier on the way.  num_splits > 1 writes (o, m, l) partials for the
+// split-reduce kernel below, or (JOIN) to LDS, where the workgroup sums them behind its one barrier.  (The first version used
+// 4 waves per (split, head, seq) with chunks round-robin, no cross-chunk prefetch and an LDS combine: 47 us per layer at
 // B=256 / ctx 128-256 on Llama-3-8B, profiles/llama3_8b_b256_kernels_auto.md.)
 // ---------------------------------------------------------------------------
 // Fused RoPE + KV append (decode only): the wave reads its q heads and the new token's k / v

@@ -704,7 +704,9 @@ __global__ void __launch_bounds__(256, 1) gemm_pp_kernel(const bf16* __restrict_
     // a segment's last tile on the row tile that holds what is left (neighbour of the segment's others in the order: put
     // last, its weight tiles came from memory again).  Both, us, Mixtral gate|up / down, 300 tokens 504 / 282 -> 373 / 250,
     // 2036 1035 / 604 -> 874 / 605, 8192 3188 / 1695 -> 2861 / 1618; 64 experts 2048 x 1408, 6 a token, 4096 tokens 393 / 215
-    // -> 334 / 183
+    // -> 334 / 183.  56 pairs of even counts and 56 of skewed ones, 257 to 8192 tokens: gate|up and down together 0.54 to 0.99 of
+    // before, one 1.01; Mixtral's down alone is up to 5 % slower where it fills one round or barely a second (400 to 1024
+    // tokens, 2036 with counts to either side of 512: 606 -> 625): every XCD now has its share of the full tiles at once
     const int left = rcnt - r0;
     auto go = [&](auto rt) {
       gemm_pp_tile<BN, MODE, VAR, decltype(rt)::value>(smem, A, We, C, P, M, N, K, n_t, r0, rcnt, roff, gather, split, ks0, nt,
@@ -793,8 +795,10 @@ int gemm_pp(uintptr_t c, uintptr_t a, uintptr_t b, uintptr_t ws, long ws_floats,
 // Grouped expert GEMM over the expert-sorted slot space (MoE prefill): expert e owns
 // slots [offsets[e], offsets[e] + counts[e]) (device arrays, never read on the host); its rows are
 // x[gather[slot]] (gather null: x[slot]) and its weight W[e] ([N, K]; SwiGLU: [2I, K] = [Wg; Wu]).
-// y [slots, N] (SwiGLU: [slots, N / 2]).  Schedule 2, 256 x 256 tiles, grouped row-tile order.
-// xrows: rows of x (buffer range), slots: total slot count (grid bound: slots / 256 + E row tiles).
+// y [slots, N] (SwiGLU: [slots, N / 2]).  Schedule 2, 256 x 256 tiles, a segment's last one of 128, 192 or 256 rows (all short and
+// few: in two workgroups of 128 columns), grouped row-tile order.
+// xrows: rows of x (buffer range), slots: total slot count (grid bound: slots / 256 + E row tiles, or two per expert as far as
+// one workgroup per CU goes).
 void gemm_pp_moe(uintptr_t y, uintptr_t x, uintptr_t gather, uintptr_t w, uintptr_t counts, uintptr_t offsets, int E,
                  int N, int K, int xrows, int slots, int mode, uintptr_t stream, float limit) {
   DLLM_HOST_CHECK(E >= 1 && E <= 256, "1 <= experts <= 256");
@@ -848,6 +852,8 @@ void gemm_pp_moe(uintptr_t y, uintptr_t x, uintptr_t gather, uintptr_t w, uintpt
 // CT / 2 x 8 bytes per half loaded once per tile.  Mode 6 took the gate kernel's pass over C (read M N, write M N / 2) away: 6376 x
 // 15360 x 2560 434 -> 363 us (mode 0 alone 360); with the gate kernel's expf and division in the epilogue 396, and the
 // error against float64 is the same either way (mean 1.13e-3, 1.71e-3 before, when the product was rounded to bf16 first).
+// The unbiased GLUs gain as much where they left gemm_pp and a gate kernel for a row tile below 256: relative error, 640 /
+// 1300 x 15360 x 2560 and 320 x 28672 x 4096, clipped 2.80e-3 -> 1.66e-3, gelu 3.04e-3 -> 1.66e-3, SiLU 3.09e-3 -> 1.66e-3.
 // SCH 8: nontemporal output stores (large SwiGLU outputs), else 0.  The schedule sweeps of rounds 3-5
 // (barrier positions, piece spacing, row-group widths, and the split A / B LDS release of round 5,
 // all within 0.5 % of this schedule: profiles/round5_raw/r5d_pf_sched.txt) were removed.

@@ -123,7 +123,8 @@ class Knobs:
     moe_wide_min_pairs: int = 8       # token-expert pairs per expert from which the tiled GEMM serves
     moe_fused_router: bool = True
     # prefill V append eight tokens per workgroup, 16-byte stores into the transposed V cache
-    # (norm_elementwise.hip qkv_append_kernel); False = the per-token 2-byte scatter.
+    # (norm_elementwise.hip qkv_append_kernel); False = the per-token 2-byte scatter (not of a projection in split-K
+    # slabs, whose append has one form).
     v_group_append: bool = True
     # grouped expert GEMM ring depth: 6 / 5 LDS slots at 64 / 128-row tiles (False: 3 slots)
     moe_deep_ring: bool = True

@@ -513,10 +513,11 @@ def linear_pf(x: torch.Tensor, w: torch.Tensor, swiglu: bool = False, variant: i
               bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Persistent prefill GEMM (gemm_pf in csrc/kernels/gemm_pp.hip): schedule 2's ``bm`` x 256 tiles,
     one workgroup per CU walking its tiles with the LDS-DMA pipeline running across tile
-    boundaries; optional fused SwiGLU (``w`` = [Wg; Wu], y [M, N / 2]) or -- ``limit`` -- clipped GLU or -- ``gelu`` --
-    gelu_tanh GLU.  ``variant`` 8: nontemporal
-    output stores (the default for SwiGLU outputs > 256 MiB); ``bm``: the row tile (pf_row_tile); ``bias`` [gate | up]: with ``limit``; the tiles come from per-XCD device
-    queues while knobs.pf_dynamic says so (bit 16 of the launcher's variant)."""
+    boundaries; optional fused SwiGLU (``w`` = [Wg; Wu], y [M, N / 2]) or -- ``limit`` -- clipped GLU (of the products plus
+    ``bias`` [gate | up], where given) or -- ``gelu`` -- gelu_tanh GLU.  ``variant`` 8: nontemporal
+    output stores (the default for SwiGLU outputs > 256 MiB).  256-row tiles come from per-XCD device queues while
+    knobs.pf_dynamic says so (bit 16 of the launcher's variant); shorter ones (``bm``, pf_row_tile) are walked statically, by
+    the CUs that communication leaves."""
     k = x.shape[-1]
     n = w.shape[0]
     m = x.numel() // k
