@@ -204,29 +204,35 @@ def linear_ref(x, w: Fp8Weight, swiglu: bool = False) -> torch.Tensor:
 # Past 256 rows the workgroups of a grid run in rounds of one per CU, so what a launch takes is the number of rounds times
 # what a workgroup of that row tile takes: a K-tile of 128, us, and the workgroup's start and epilogue (measured, one
 # round, K = 2048 ... 14336).  Shorter tiles do less per byte staged.  Two 64-row workgroups share a CU: a further round adds
-# less than the first.  A K split adds the launch that sums the slabs, and their traffic.  Former plan (the decode kernels' K
-# split, 192 / 256-row tiles) -> this, reduction included, us: 4096 x 14336 at M = 448 / 640 / 1536 / 2432 / 2800 43 / 76 / 93 /
-# 188 / 186 -> 39 / 52 / 87 / 164 / 170; 4096 x 4096 at 320 / 640 / 1536 / 2800 19 / 27 / 34 / 63 -> 17 / 21 / 30 / 57; 6144 x 4096 at
-# 320 / 1024 / 1536 22.7 / 32.6 / 61 -> 17.2 / 32.2 / 54; 1024 x 8192 at 320 / 2048 15.6 / 37 -> 12.3 / 28.6; 8192 x 8192 at 640 / 1536
-# 57 / 111 -> 51 / 105; 2048 x 2048 at 768 / 2048 18.2 / 20.1 -> 10.3 / 14.9; where 256 rows fill their rounds (28672 x 4096 at
-# 2432, 302 against 328 in 192 rows; 6144 x 4096 at 2048, 64 against 67 in 128) nothing changes.
+# less than the first.  A K split adds its slabs: written and read by the consumer, which sums them on its way (the norm behind
+# o and down, the K / V append behind qkv: 0.3 us more than reading the finished product), or, for a GLU, by a launch of their
+# own; us, and us per million slab elements.  Charged with a launch of its own throughout, a plain product went unsplit where that
+# is slower: split as formerly / unsplit / now, 4096 x 4096 at 384 / 640 rows with the norm 25.2 / 28.5 / 25.2 and 33.2 / 34.4 / 30.3,
+# 6144 x 4096 at 384 29.7 / 34.5 / 29.7 and with the append 31.1 / 35.5 / 31.1.  196 sizes (14 weights 512 x 4096 ... 8192 x 28672, 257 to
+# 2800 rows) are within 0.1 % of the best grid in the mean, their norm included, 140 GLUs within 0.4 %, and none is 3 % slower than under
+# the former plan (the decode kernels' K split, 192 / 256-row tiles).  Former -> this, norm included, us: 4096 x 14336 at M =
+# 640 / 1232 89.5 / 130 -> 66.3 / 108; 4096 x 4096 at 500 / 768 31.1 / 44.4 -> 25.9 / 35.4; 6144 x 4096 at 448 / 768 43.7 / 46.5 -> 34.2 /
+# 42.7; 1024 x 4096 at 300 / 1232 19.0 / 30.0 -> 14.9 / 26.0; 2048 x 8192 at 300 / 900 26.2 / 46.5 -> 23.8 / 38.5; where 256 rows
+# fill their rounds (28672 x 4096 at 2432, 302 against 328 in 192 rows; 6144 x 4096 at 2048, 64 against 67 in 128) nothing changes.
 _ROUND_US = {64: (0.435, 3.2), 128: (0.505, 5.0), 192: (0.66, 5.5), 256: (0.745, 6.6)}
 _ROUND_64 = 0.36
-_SLAB_US, _SLAB_US_PER_MB = 3.0, 0.3
+_SLAB_US = {False: (0.3, 0.2), True: (3.0, 0.32)}      # GLU
 
 
-def _prompt_plan(m: int, n: int, k: int, most: int, cus: int) -> Tuple[int, int]:
+def _prompt_plan(m: int, n: int, k: int, most: int, cus: int, swiglu: bool) -> Tuple[int, int]:
     """(K slices, row tile) of the cheapest grid past 256 rows.  ``most``: the slabs hold 16 bits, so a product is split no
     further than the decode rule would split it, and one that this leaves whole stays whole.  The slices, which set how the
-    result rounds, are those of the whole chip; ``cus`` -- what communication leaves of it -- moves the row tile alone, which
-    changes no bit: a pipeline's stages round as one engine does."""
+    result rounds, are those of the whole chip (and of no one consumer: a stage that ends behind the product has another);
+    ``cus`` -- what communication leaves of it -- moves the row tile alone, which changes no bit: a pipeline's stages round as
+    one engine does."""
     from . import gemm
 
     def us(s, bm, cus):
         tile_us, fixed = _ROUND_US[bm]
         rounds, kt = -(-(n // 128) * -(-m // bm) * s // cus), -(-(k // 128) // s)
         t = (tile_us + _ROUND_64 * (rounds - 1)) * kt + fixed if bm == 64 else rounds * (tile_us * kt + fixed)
-        return t + (_SLAB_US + _SLAB_US_PER_MB * s * m * n * 4e-6 if s > 1 else 0.0)
+        slab, per = _SLAB_US[swiglu]
+        return t + (slab + per * s * m * n * 1e-6 if s > 1 else 0.0)
 
     best, plan = float("inf"), (1, 256)
     for bm in (256, 192, 128, 64):
@@ -247,7 +253,7 @@ def fp8_plan(m: int, n: int, k: int, swiglu: bool = False) -> Tuple[int, int]:
     from . import gemm
     s = gemm.wide_splits(m, n, k // 2, swiglu)
     if m > 256:
-        return _prompt_plan(m, n, k, s, 256 - gemm._comm_cus)
+        return _prompt_plan(m, n, k, s, 256 - gemm._comm_cus, swiglu)
     if knobs.K.fp8_bm128 and not swiglu and s > 1 and 128 < m <= 256:
         tiles = (n // 128) * 2
         return max(1, min(256 // tiles, (k // 128) // 4, 16)), 128
@@ -265,8 +271,8 @@ def fp8_variant(m: int, n: int, k: int, splits: int, bm: int) -> int:
     from step to step.  With the norm that sums the slabs behind it, default -> nontemporal, us: 6144 x 4096 (8 K-tiles) 11.7 /
     13.9 -> 10.9 / 13.5 at M = 1 / 64, 8192 x 28672 (56) 48.8 / 52.1 / 60.6 -> 43.5 / 48.0 / 58.0 at M = 1 / 64 / 128; but read by
     several row tiles 4096 x 14336 at M = 200 / 300 34.7 / 41.0 -> 36.2 / 42.8, 5120 x 25600 66.7 / 77.2 -> 69.5 / 81.6 (from 384
-    rows on within 2 % either way) -- unless those are of 64 rows with the deep ring that goes with it (2048 x 8192 at 300, five
-    row tiles, 25.4 -> 24.3)."""
+    rows on within 2 % either way) -- unless those are of 64 rows with the deep ring that goes with it (2048 x 8192 at 300 in 3
+    slices and five row tiles, 25.4 -> 24.3)."""
     order = 64 if 0 < knobs.K.fp8_group_m <= (2 * m if 0 < bm < 256 else m) else 0
     if splits == 1:
         return (1 if m <= 256 else 4 | order) | (bm << 8)

@@ -159,7 +159,17 @@ def test_fp8_weights_read_by_several_row_tiles_are_cached():
     assert [policy(m, 4096, 14336) for m in (1, 64, 128)] == [1, 1, 1]
     assert [policy(m, 4096, 14336) for m in (129, 256, 300, 640, 1024)] == [4] * 5
     assert [policy(m, 8192, 28672) for m in (64, 200, 300)] == [1, 4, 4]
-    assert policy(300, 2048, 8192) == 1 and quant.fp8_plan(300, 2048, 8192) == (3, 64)
+    assert quant.fp8_variant(300, 2048, 8192, 3, 64) & 7 == 1 and policy(300, 2048, 8192) == 4
     assert policy(1, 6144, 4096) == 1 and policy(100, 6144, 4096) == 4 and policy(64, 1024, 8192) == 4
     assert policy(64, 28672, 4096) == 1 and quant.fp8_variant(4096, 28672, 4096, 1, 256) == 4 | 64 | 256 << 8
     assert quant.fp8_variant(2100, 4096, 4096, 1, 192) == 4 | 64 | 192 << 8 and quant.fp8_variant(2100, 4096, 4096, 1, 0) == 4
+
+
+def test_fp8_prompt_plan_splits_where_the_consumer_sums():
+    """A split whose slabs the norm or the append sums costs no launch: narrow products of a few hundred rows are split rather than
+    run as one round of short tiles; a GLU, which pays for the sum, sooner stays whole."""
+    from distributed_llms_amd.ops import quant
+    assert [quant.fp8_plan(m, 4096, 4096) for m in (300, 384, 500, 640)] == [(3, 192), (3, 192), (2, 128), (2, 192)]
+    assert [quant.fp8_plan(m, 6144, 4096) for m in (257, 300, 384)] == [(2, 192)] * 3
+    assert quant.fp8_plan(448, 8192, 8192) == (2, 256) and quant.fp8_plan(300, 2048, 8192) == (5, 128)
+    assert quant.fp8_plan(900, 4096, 4096) == (1, 128) and quant.fp8_plan(448, 4096, 4096, True) == (1, 64)
