@@ -206,16 +206,21 @@ __global__ void __launch_bounds__(256) qkv_append_kernel(bf16* __restrict__ q_ou
                                                          long slab, const int32_t* __restrict__ positions,
                                                          const float* __restrict__ cos_sin, bf16* __restrict__ k_cache,
                                                          bf16* __restrict__ v_cache, const int32_t* __restrict__ slots,
-                                                         int tokens, int hq, int hkv, int d, int bs) {
+                                                         int tokens, int hq, int hkv, int d, int bs, int by_row) {
   __shared__ __attribute__((aligned(16))) bf16 tile[8][kAppendCols + 8];
   __shared__ int sl[8];
   constexpr int R = 4;                                 // four elements or pairs of four per item, R items in flight
   constexpr int NS = SC > 0 ? SC : 1;
-  const int t0 = blockIdx.x * 8, n = min(8, tokens - t0), tid = threadIdx.x;
   const int width = (hq + 2 * hkv) * d, half = d >> 1;
   const int hpc = max(1, kAppendCols / d);             // heads per workgroup
   const int nkv = (hkv + hpc - 1) / hpc;
-  const int y = blockIdx.y, what = y < nkv ? 2 : y < 2 * nkv ? 1 : 0;          // v, k, q
+  int t0 = blockIdx.x * 8, y = blockIdx.y;
+  if (by_row) {
+    t0 = blockIdx.y * 8;
+    y = (blockIdx.x + (blockIdx.y >> 3)) % gridDim.x;
+  }
+  const int n = min(8, tokens - t0), tid = threadIdx.x;
+  const int what = y < nkv ? 2 : y < 2 * nkv ? 1 : 0;          // v, k, q
   const int h0 = (what == 2 ? y : what == 1 ? y - nkv : y - 2 * nkv) * hpc;
   const int heads = min(hpc, (what == 0 ? hq : hkv) - h0);
   const int col0 = ((what == 0 ? 0 : what == 1 ? hq : hq + hkv) + h0) * d;      // first column in a row of qkv
@@ -349,11 +354,18 @@ void rope_cache_append(uintptr_t q_out, int rotate_q, uintptr_t qkv, uintptr_t p
     return;
   }
   const int hpc = d > kAppendCols ? 1 : kAppendCols / d;
-  const dim3 grid((tokens + 7) / 8, 2 * ((hkv + hpc - 1) / hpc) + (q_out ? (hq + hpc - 1) / hpc : 0));
+  const int groups = (tokens + 7) / 8, pieces = 2 * ((hkv + hpc - 1) / hpc) + (q_out ? (hq + hpc - 1) / hpc : 0);
+  // Up to what the caches hold the grid takes all groups of v, then of k, then of q, which have different lengths; past that a
+  // group's pieces are neighbours, so that its rows are read as one stretch of memory, the first piece moving on with the groups
+  // so that every XCD gets every kind.  us, by kind -> by row, q written: 32 / 8 heads of 128, 12000 / 16000 / 32000 tokens (147 /
+  // 197 / 393 MB) 64 / 92 / 182 -> 57 / 79 / 150, 32 / 32 at 4096 / 16000 48 / 178 -> 42 / 151, 16 / 16 of 96 at 12000 / 32000 52.8 / 138
+  // -> 51.2 / 131; but 64 / 8 of 128 at 4096 (84 MB) 31.4 -> 33.6, 32 / 8 of 64 at 4096 (25 MB) 14.6 -> 15.7
+  const int by_row = (long)tokens * (2 * hkv + (q_out ? hq : 0)) * d * 2 >= 100000000 && groups < 65536;
+  const dim3 grid(by_row ? pieces : groups, by_row ? groups : pieces);
   auto go = [&](auto kern) {
     hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, (bf16*)q_out, rotate_q, (const bf16*)qkv, (const float*)part, slab,
                        (const int32_t*)positions, (const float*)cos_sin, (bf16*)k_cache, (bf16*)v_cache,
-                       (const int32_t*)slots, tokens, hq, hkv, d, bs);
+                       (const int32_t*)slots, tokens, hq, hkv, d, bs, by_row);
   };
   switch (part ? nparts : 0) {
     case 0: go(qkv_append_kernel<0>); break;

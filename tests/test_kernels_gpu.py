@@ -149,6 +149,24 @@ def test_rope_cache_append_sums_slabs(cuda, hq, hkv, d, tokens, slabs):
     assert torch.equal(v1, vr)
 
 
+@pytest.mark.parametrize("hq,hkv,d,tokens", [(32, 8, 128, 8201), (32, 8, 64, 16345), (20, 20, 96, 8685), (4, 1, 256, 32555)])
+def test_rope_cache_append_by_row(cuda, hq, hkv, d, tokens):
+    """Grids past 100 MB walk the pieces of a row one after the other: the bits of the append by tokens, 3 to 6 pieces a row, a
+    short last group."""
+    from distributed_llms_amd import knobs
+    assert tokens * (hq + 2 * hkv) * d * 2 >= 100e6 and tokens % 8
+    qkv, cs = _bf(tokens, (hq + 2 * hkv) * d), ref.rope_cos_sin(d, 1024, 500000.0, device="cuda")
+    slots = torch.arange(tokens, dtype=torch.int32, device="cuda") + 32
+    pos = slots % 1000
+    nb = tokens // 32 + 3
+    caches = [(torch.zeros(nb, hkv, 32, d, dtype=torch.bfloat16, device="cuda"),
+               torch.zeros(nb, hkv, d, 32, dtype=torch.bfloat16, device="cuda")) for _ in range(2)]
+    q = ops.rope_cache_append(qkv, pos, cs, *caches[0], slots, hq, hkv, d)
+    with knobs.override(v_group_append=False):
+        want = ops.rope_cache_append(qkv, pos, cs, *caches[1], slots, hq, hkv, d)
+    assert torch.equal(q, want) and all(torch.equal(a, b) for a, b in zip(*caches))
+
+
 @pytest.mark.parametrize("slabs", [1, 2, 3, 4, 5, 6, 8, 13, 17])
 def test_rope_cache_append_leaves_other_slab_counts_to_the_sum(cuda, monkeypatch, slabs):
     """Numbers of slabs that the append has no form for are summed by the launch that spreads over the chip, not one slab after
