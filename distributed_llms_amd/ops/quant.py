@@ -22,6 +22,7 @@ quantization, f32 math), which is also the numerics oracle of the GPU tests.
 """
 from __future__ import annotations
 
+import functools
 from typing import Tuple
 
 import torch
@@ -219,6 +220,7 @@ _ROUND_64 = 0.36
 _SLAB_US = {False: (0.3, 0.2), True: (3.0, 0.32)}      # GLU
 
 
+@functools.lru_cache(maxsize=1024)        # a pass asks for the same few products in every layer, 7 to 29 us each
 def _prompt_plan(m: int, n: int, k: int, most: int, cus: int, swiglu: bool) -> Tuple[int, int]:
     """(K slices, row tile) of the cheapest grid past 256 rows.  ``most``: the slabs hold 16 bits, so a product is split no
     further than the decode rule would split it, and one that this leaves whole stays whole.  The slices, which set how the
