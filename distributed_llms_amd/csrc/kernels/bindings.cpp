@@ -33,6 +33,7 @@ PYBIND11_MODULE(_C_kernels, m) {
   m.def("splitk_add_rms_norm_q8", &dllm::splitk_add_rms_norm_q8);
   m.def("gemm_sq", &dllm::gemm_sq);
   m.def("gemm_stream", &dllm::gemm_stream);
+  m.def("gemm_close", &dllm::gemm_close);
   m.def("gemm_pp_moe", &dllm::gemm_pp_moe, py::arg("y"), py::arg("x"), py::arg("gather"), py::arg("w"), py::arg("counts"), py::arg("offsets"), py::arg("experts"), py::arg("n"), py::arg("k"), py::arg("xrows"), py::arg("slots"), py::arg("mode"), py::arg("stream"),
         py::arg("limit") = 0.f);
   m.def("gemm_pp", &dllm::gemm_pp);

@@ -235,14 +235,14 @@ class BasopelStage(LayerListStage):
         return self.state
 
     # ------------------------------------------------------------------ forward
-    def _softmax_mixer(self, i: int, h: torch.Tensor, w, meta: BatchMeta, sb: sm.SeqBatch, nd: int, max_ctx,
+    def _softmax_mixer(self, i: int, h: sm.Close, w, meta: BatchMeta, sb: sm.SeqBatch, nd: int, max_ctx,
                        v_mix: Optional[sm.ValueMix]):
         spec = self.specs[i]
         m, eps = spec["mixer"], self.cfg.norm_eps
         hh, g, d, dv = m["heads"], m["kv_heads"], m["dim"], m["vdim"]
         kc, vc = self.kv.caches[i]
         size = int((m.get("mask") or {}).get("size") or 0)          # no mask entry: plain causal attention
-        proj = ops.linear(h, w["w_in"])
+        proj = h.linear(w["w_in"])
         if spec["type"] == "attention":
             q = sm.head_norm_rope(proj, 0, w["q_norm"], w["k_norm"], None, eps, kc, vc, meta.slot_mapping, sb.positions, hh, g,
                                   d, dv, bias=w["b_in"], v_mix=v_mix)
@@ -274,7 +274,7 @@ class BasopelStage(LayerListStage):
         nd = meta.num_decode if meta.is_prefill else meta.num_seqs
         max_ctx = meta.max_ctx_d if (meta.is_prefill and nd) else meta.max_ctx
         x = sm.embedding_f32(inp, self.embed["embed"], cfg.embed_scale)
-        h = sm.layer_norm_f32(x, self.layers[0]["norm1"], self.layers[0]["norm1_b"], eps, self.dtype)
+        h = sm.Close.made(x, sm.layer_norm_f32(x, self.layers[0]["norm1"], self.layers[0]["norm1_b"], eps, self.dtype))
         v_first = None                    # the values that later layers read, from the first layer that shares them
         for i, (spec, w) in enumerate(zip(self.specs, self.layers)):
             nxt = (None, None)
@@ -282,7 +282,7 @@ class BasopelStage(LayerListStage):
                 nxt = (self.layers[i + 1]["norm1"], self.layers[i + 1]["norm1_b"])
             if spec["type"] == LATENT:
                 kc, vc = self.kv.caches[i]
-                o = lat.latent_attention(h, w["mix"], self.lspec[i], self.freqs[i], eps, kc, vc, meta.slot_mapping,
+                o = lat.latent_attention(h.input(), w["mix"], self.lspec[i], self.freqs[i], eps, kc, vc, meta.slot_mapping,
                                          meta.block_tables, sb, num_decode=nd, max_ctx=max_ctx, defer=True,
                                          window=int((spec["mixer"].get("mask") or {}).get("size") or 1 << 30))
             else:
@@ -291,13 +291,16 @@ class BasopelStage(LayerListStage):
                     v_first = vm.first
                 o = self._softmax_mixer(i, h, w, meta, sb, nd, max_ctx, vm)
             after = (w["norm2"], w["norm2_b"]) if spec.get("mlp") else nxt
-            x, h = sm.post_layer_norm_add(x, o, w["norm1b"], w["norm1b_b"], eps, bias=w.get("bo"), w_next=after[0],
-                                          b_next=after[1])
+            h = sm.Close("layer", h.x, o, w_post=w["norm1b"], b_post=w["norm1b_b"], eps=eps, bias=w.get("bo"), w_next=after[0],
+                         b_next=after[1])
             if spec.get("mlp"):
-                y = ops.linear_into_norm(sm.linear_gelu_glu(h, w["w_gu"]), w["w_down"])
-                x, h = sm.post_layer_norm_add(x, y, w["norm2b"], w["norm2b_b"], eps, w_next=nxt[0], b_next=nxt[1])
+                y = ops.linear_into_norm(h.gelu_glu(w["w_gu"]), w["w_down"])
+                h = sm.Close("layer", h.x, y, w_post=w["norm2b"], b_post=w["norm2b_b"], eps=eps, w_next=nxt[0], b_next=nxt[1])
             if self.taps is not None:
-                self.taps.append(x.clone())
+                h.input()
+                self.taps.append(h.x.clone())
+        h.input()
+        x = h.x
         if meta.logits_idx is not None:
             x = x.index_select(0, meta.logits_idx)
         hf = sm.layer_norm_f32(x, self.head["final_norm"], self.head["final_norm_b"], eps, self.dtype)

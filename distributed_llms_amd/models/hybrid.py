@@ -333,12 +333,12 @@ class HybridStage(LayerListStage):
         return n
 
     # ------------------------------------------------------------------ forward
-    def _attention(self, i: int, h: torch.Tensor, w, meta: BatchMeta, sb: sm.SeqBatch) -> torch.Tensor:
+    def _attention(self, i: int, h: sm.Close, w, meta: BatchMeta, sb: sm.SeqBatch) -> torch.Tensor:
         m = self.specs[i]["mixer"]
         own = "kv_from" not in m
         kc, vc = self.kv.caches[i if own else m["kv_from"]]
         freqs, mag = self.rot[i]
-        qkv = ops.linear(h, w["wqkv"])
+        qkv = h.linear(w["wqkv"])
         q = sm.attn_prep(qkv, w["conv_w"], self.state[i]["conv"], w["q_norm"], w.get("k_norm"), freqs, mag,
                          self.cfg.norm_eps, kc if own else None, vc if own else None, meta.slot_mapping, sb,
                          m["heads"], m["kv_heads"], m["dim"], m["vdim"])
@@ -348,10 +348,10 @@ class HybridStage(LayerListStage):
         a = sm.window_attention(q, kc, vc, meta.block_tables, sb, window, scale, num_decode=nd)
         return ops.linear_into_norm(a.view(a.shape[0], -1), w["wo"])
 
-    def _rglru(self, i: int, h: torch.Tensor, w, sb: sm.SeqBatch) -> torch.Tensor:
+    def _rglru(self, i: int, h: sm.Close, w, sb: sm.SeqBatch) -> torch.Tensor:
         m = self.specs[i]["mixer"]
         c = m["width"]
-        yx = ops.linear(h, w["w_yx"])
+        yx = h.linear(w["w_yx"])
         st = self.state[i]
         if sm.one_token_each(sb) and sm.rglru_step_fits(m["blocks"], c // m["blocks"], m["conv"]):
             r = sm.rglru_step(yx, w["conv_w"], w["conv_b"], w["x_b"], st["conv"], w["y_b"], w["ra_t"], w["ra_b"], w["ri_t"],
@@ -370,18 +370,21 @@ class HybridStage(LayerListStage):
         eps, mult = cfg.norm_eps, cfg.residual_mult
         sb = self._seq_batch(meta)
         x = sm.embedding_f32(inp, self.embed["embed"])
-        h = sm.rms_norm_f32(x, self.layers[0]["norm1"], eps, self.dtype)
+        h = sm.Close.made(x, sm.rms_norm_f32(x, self.layers[0]["norm1"], eps, self.dtype))
         n = len(self.layers)
         for i, (spec, w) in enumerate(zip(self.specs, self.layers)):
             o = self._attention(i, h, w, meta, sb) if spec["type"] == "attention" else self._rglru(i, h, w, sb)
             nxt = self.layers[i + 1]["norm1"] if i + 1 < n else None
-            x, h = sm.post_norm_add(x, o, w["norm1b"], eps, mult, w_next=w["norm2"] if spec.get("mlp") else nxt)
+            h = sm.Close("rms", h.x, o, w_post=w["norm1b"], eps=eps, mult=mult, w_next=w["norm2"] if spec.get("mlp") else nxt)
             if spec.get("mlp"):
-                y = sm.linear_clipped_glu(h, w["w_gu"], w["b_gu"], spec["mlp"]["limit"])
-                x, h = sm.post_norm_add(x, ops.linear_into_norm(y, w["w_down"]), w["norm2b"], eps, mult, bias=w["b_down"],
-                                        w_next=nxt)
+                y = h.clipped_glu(w["w_gu"], w["b_gu"], spec["mlp"]["limit"])
+                h = sm.Close("rms", h.x, ops.linear_into_norm(y, w["w_down"]), w_post=w["norm2b"], eps=eps, mult=mult,
+                             bias=w["b_down"], w_next=nxt)
             if self.taps is not None:
-                self.taps.append(x.clone())
+                h.input()
+                self.taps.append(h.x.clone())
+        h.input()
+        x = h.x
         if meta.logits_idx is not None:
             x = x.index_select(0, meta.logits_idx)
         hf = sm.rms_norm_f32(x, self.head["final_norm"], eps, self.dtype)

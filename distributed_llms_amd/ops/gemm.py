@@ -245,11 +245,47 @@ def use_stream(m: int, n: int, k: int, x: torch.Tensor, w: torch.Tensor, bias=No
 
 def linear_into_norm(x: torch.Tensor, w: torch.Tensor):
     """``x w^T`` for a consumer that sums split-K slabs itself (post_norm_add, post_layer_norm_add): the finished product
-    where the weight-streaming kernel is faster than the split grid alone, else possibly a :class:`SplitKPartial`."""
+    where the weight-streaming kernel is faster than the split grid alone, else possibly a :class:`SplitKPartial`.  One row
+    that :func:`close_product` can take is finished wherever that kernel serves a plain product (2560 x 7680, the close and a
+    5120 x 2560 product: 19.8 us in three launches of which the second sums slabs, 17.8 in two)."""
     m, n, k = _sizes(x, w, "linear_into_norm")
-    if m <= STREAM_MAX_M and use_stream(m, n, k, x, w, defer=True):
+    if m <= STREAM_MAX_M and use_stream(m, n, k, x, w, defer=m > 1 or n > CLOSE_MAX_WIDTH):
         return _stream(m, n, k, x, w)
     return _linear(m, n, k, x, w, None, True)
+
+
+CLOSE_MAX_WIDTH = 2560             # (csrc/kernels/gemm_close.hip: one row in the registers of four waves)
+
+
+def close_product(kind: str, x: torch.Tensor, o: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], glu: str,
+                  limit: float, w_post, w_next, eps: float, mult: float = 1.0, offset: float = 0.0, o_bias=None, b_post=None,
+                  b_next=None):
+    """(x', y): the close of a sublayer (``kind`` "rms": post_norm_add, "layer": post_layer_norm_add) on a stream ``x`` [1, K]
+    and the product of its output with ``w`` [N, K] (``glu``: "" (plain), "clipped" behind RMS norms or "gelu" behind layer
+    norms) in one launch; None where a call of its own makes it: other numbers of rows (gemm_close.hip), widths, types or
+    layouts, products that another kernel than the weight-streaming one serves."""
+    n, k = w.shape if w.dim() == 2 else (0, 0)
+    if not (knobs.K.stream and x.is_cuda and k <= CLOSE_MAX_WIDTH and x.shape == o.shape == (1, k) and x.dtype == torch.float32
+            and w.dtype == torch.bfloat16 and glu in ("", "clipped" if kind == "rms" else "gelu") and (not glu or n % 2 == 0)
+            and stream_fits(1, n, k, glu, False, bias is not None)
+            # (the builds' cache policy of the weights)
+            and (n * k * 2 >= WIDE_NT_MIN_BYTES) == bool(glu or k > 1024)):
+        return None
+    vecs = [t for t in (o, w_post, w_next, o_bias, b_post, b_next) if t is not None]
+    if any(t.dtype != torch.bfloat16 or t.numel() != k or not t.is_contiguous() or t.device != x.device or t.data_ptr() % 8
+           for t in vecs) or not (x.is_contiguous() and x.data_ptr() % 16 == 0 and w.is_contiguous() and w.device == x.device
+                                  and w.data_ptr() % 16 == 0):
+        return None
+    if bias is not None and not (bias.dtype == torch.bfloat16 and bias.dim() == 1 and bias.size(0) == n and bias.is_contiguous()
+                                 and bias.device == x.device):
+        return None
+    y = torch.empty(1, n // 2 if glu else n, dtype=torch.bfloat16, device=x.device)
+    xo = torch.empty_like(x)
+    p = lambda t: 0 if t is None else t.data_ptr()
+    _ext.kernels().gemm_close(y.data_ptr(), w.data_ptr(), p(bias), n, k, _STREAM_GLU[glu], float(limit), 1 if kind == "rms" else 2,
+                              x.data_ptr(), o.data_ptr(), p(o_bias), w_post.data_ptr(), p(b_post), w_next.data_ptr(), p(b_next),
+                              xo.data_ptr(), float(eps), float(mult), float(offset), current_stream())
+    return xo, y
 
 
 _STREAM_GLU = {"": 0, "silu": 1, "clipped": 2, "gelu": 3}

@@ -228,6 +228,62 @@ def post_layer_norm_add(x: torch.Tensor, o, w_post: torch.Tensor, b_post: torch.
     return x, h
 
 
+class Close:
+    """The close of a sublayer that is still to be made, for the product that reads it: ``kind`` "rms" with the arguments of
+    :func:`post_norm_add` or "layer" with those of :func:`post_layer_norm_add`.  The product makes it in its own launch where
+    that is the faster way (:func:`~.gemm.close_product`: a single row); ``x`` is the new stream from then on (a tensor of its
+    own or the old one, updated in place)."""
+
+    __slots__ = ("kind", "x", "h", "_o", "_kw")
+
+    def __init__(self, kind: str, x: torch.Tensor, o, **kw):
+        self.kind, self.x, self.h, self._o, self._kw = kind, x, None, o, kw
+
+    @classmethod
+    def made(cls, x: torch.Tensor, h: torch.Tensor) -> "Close":
+        """Of a stream whose normed form is at hand (the first sublayer's)."""
+        c = cls("", x, None)
+        c.h = h
+        return c
+
+    def input(self) -> Optional[torch.Tensor]:
+        """The next sublayer's input (None behind the last one), made by a launch of its own unless it is there."""
+        if self._o is not None:
+            self.x, self.h = (post_norm_add if self.kind == "rms" else post_layer_norm_add)(self.x, self._o, **self._kw)
+            self._o = None
+        return self.h
+
+    def _product(self, w: torch.Tensor, bias: Optional[torch.Tensor], glu: str, limit: float) -> Optional[torch.Tensor]:
+        from . import gemm
+        kw, o = self._kw, self._o
+        if type(o) is not torch.Tensor or o.shape[0] != 1 or kw.get("w_next") is None:
+            return None
+        if self.kind == "rms":
+            r = gemm.close_product("rms", self.x, o, w, bias, glu, limit, kw["w_post"], kw["w_next"], kw["eps"], kw["mult"], 1.0,
+                                   kw.get("bias"))
+        else:
+            r = gemm.close_product("layer", self.x, o, w, bias, glu, limit, kw["w_post"], kw["w_next"], kw["eps"],
+                                   o_bias=kw.get("bias"), b_post=kw["b_post"], b_next=kw["b_next"])
+        if r is None:
+            return None
+        self.x, y = r
+        self._o = None
+        return y
+
+    def linear(self, w: torch.Tensor) -> torch.Tensor:
+        from . import linear
+        y = self._product(w, None, "", 0.0)
+        return linear(self.input(), w) if y is None else y
+
+    def clipped_glu(self, w: torch.Tensor, bias: Optional[torch.Tensor], limit: float) -> torch.Tensor:
+        y = self._product(w, bias, "clipped", limit)
+        return linear_clipped_glu(self.input(), w, bias, limit) if y is None else y
+
+    def gelu_glu(self, w: torch.Tensor) -> torch.Tensor:
+        y = self._product(w, None, "gelu", 0.0)
+        return linear_gelu_glu(self.input(), w) if y is None else y
+
+
 def stream_enter(x: torch.Tensor, x0: Optional[torch.Tensor], vec: Optional[torch.Tensor]) -> torch.Tensor:
     """The entry of a pass through a looped span of layers, in place on the float32 stream: x += x0 (a
     second stream, e.g. the embedding output; None: nothing) + vec (one learned row [W] for every token;

@@ -1,0 +1,127 @@
+"""The close of a sublayer in the launch of the product that reads it (csrc/kernels/gemm_close.hip), and the rule for it."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from distributed_llms_amd import knobs, ops
+from distributed_llms_amd.ops import gemm
+from distributed_llms_amd.ops import seqmix as sm
+
+
+def _norm(v, w, b, eps):
+    """RMS norm (no ``b``) around 1 + w, layer norm with one, in float64."""
+    if b is None:
+        return v * torch.rsqrt(v.pow(2).mean(-1, keepdim=True) + eps) * (1.0 + w)
+    c = v - v.mean(-1, keepdim=True)
+    return c * torch.rsqrt(c.pow(2).mean(-1, keepdim=True) + eps) * w + b
+
+
+def _args(kind, k, o_bias, seed, device):
+    g = torch.Generator().manual_seed(seed)
+    r = lambda *s: torch.randn(*s, generator=g).bfloat16().to(device)
+    x, o = torch.randn(1, k, generator=g).to(device), r(1, k)
+    kw = dict(w_post=r(k) * 0.2, w_next=r(k) * 0.2, eps=1e-5, bias=r(k) if o_bias else None)
+    if kind == "rms":
+        kw["mult"] = 0.75
+    else:
+        kw.update(b_post=r(k), b_next=r(k))
+    return x, o, kw
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["rms", "layer"])
+@pytest.mark.parametrize("glu", [False, True])
+@pytest.mark.parametrize("n,k", [(8, 512), (1536, 576), (2048, 1024), (6142, 1024), (6146, 1024), (3072, 1088), (5120, 2560), (15360, 2560)])
+def test_close_product(cuda, kind, glu, n, k):
+    """Widths at and between the edges of the row's pieces, 1 to 8 groups of weight rows, ragged last workgroups, fewer
+    workgroups than CUs and more; the new stream, the product, and nothing outside either."""
+    policy = (n * k * 2 >= gemm.WIDE_NT_MIN_BYTES) == (glu or k > 1024)
+    x, o, kw = _args(kind, k, n % 4 == 0, n + k, "cuda")
+    w = (torch.randn(n, k, device="cuda") * k ** -0.5).bfloat16()
+    b = torch.randn(n, device="cuda").bfloat16() if glu and kind == "rms" and n != 6142 else None
+    act = "" if not glu else "clipped" if kind == "rms" else "gelu"
+    old = x.clone()
+    r = gemm.close_product(kind, x, o, w, b, act, 0.7, kw["w_post"], kw["w_next"], kw["eps"], kw.get("mult", 1.0), 1.0 if kind == "rms" else 0.0,
+                           kw["bias"], kw.get("b_post"), kw.get("b_next"))
+    if not (policy and gemm.stream_fits(1, n, k, act, False, b is not None)):
+        assert r is None
+        return
+    xo, y = r
+    assert torch.equal(x, old)
+    d = lambda t: None if t is None else t.double()
+    v = o.double() + (0 if kw["bias"] is None else kw["bias"].double())
+    s = x.double() + kw.get("mult", 1.0) * _norm(v, d(kw["w_post"]), d(kw.get("b_post")), kw["eps"])
+    # f32 sums of k squares and a handful of roundings, each within 2^-23
+    assert bool(((xo.double() - s).abs() <= (k * 2.0 ** -24 + 2.0 ** -20) * (1.0 + s.abs())).all())
+    h = _norm(xo.double(), d(kw["w_next"]), d(kw.get("b_next")), kw["eps"])
+    z, mag = F.linear(h, w.double(), d(b)), h.abs() @ w.double().abs().t()
+    # h rounds to bf16 (2^-9 each, and the norm's own 2^-20), the product sums k of them in f32
+    e = (2.0 ** -9 + 2.0 ** -18 + k * 2.0 ** -24) * mag + (0 if b is None else 2.0 ** -20 * b.double().abs())
+    if not glu:
+        assert bool(((y.double() - z).abs() <= e + 2.0 ** -8 * z.abs()).all())
+        return
+    half = n // 2
+    g, u = z[:, :half], z[:, half:]
+    if act == "clipped":
+        gc, uc = g.clamp(max=0.7), u.clamp(-0.7, 0.7)
+        ref, up = gc * torch.sigmoid(1.702 * gc) * (uc + 1), uc.abs() + 1
+    else:
+        ref, up = F.gelu(g, approximate="tanh") * u, u.abs()
+    # |d act / d gate| <= 1.2 |up|, act <= |gate| |up|: both sums' errors through the product; the result rounds to bf16
+    tol = 1.2 * e[:, :half] * (up + e[:, half:]) + (g.abs() + 1e-3) * e[:, half:] + (2.0 ** -8 + 2.0 ** -18) * ref.abs() + 2.0 ** -22
+    assert bool(((y.double() - ref).abs() <= tol).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["rms", "layer"])
+def test_close_refused(cuda, kind):
+    """What the launch does not take goes to the close's own: several rows, widths past its registers, K no multiple of 64,
+    float32, a view off its alignment, weights of another cache policy, the switch."""
+    def product(x, o, kw, n=2048, w=None):
+        w = (torch.randn(n, x.shape[1], device="cuda") * 0.05).to(o.dtype) if w is None else w
+        return gemm.close_product(kind, x, o, w, None, "", 0.0, kw["w_post"], kw["w_next"], kw["eps"], 1.0, 1.0, kw["bias"],
+                                  kw.get("b_post"), kw.get("b_next"))
+    x, o, kw = _args(kind, 1024, True, 1, "cuda")
+    assert product(x, o, kw) is not None
+    assert product(x, o, kw, n=8192) is None                                  # (nontemporal weights at this width: GLU builds only)
+    assert product(x.repeat(2, 1), o.repeat(2, 1), kw) is None
+    assert product(x, o.float(), kw) is None
+    pad = torch.zeros(1025, device="cuda")
+    assert product(pad[1:].view(1, -1), o, kw) is None
+    off = torch.zeros(1025, dtype=torch.bfloat16, device="cuda")[1:]
+    assert product(x, o, {**kw, "w_next": off}) is None
+    for k in (2624, 600):
+        assert product(*_args(kind, k, False, 2, "cuda")) is None
+    knobs.K.stream = False
+    try:
+        assert product(x, o, kw) is None
+    finally:
+        knobs.K.stream = True
+
+
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("kind", ["rms", "layer"])
+@pytest.mark.parametrize("rows", [1, 3])
+@pytest.mark.parametrize("last", [False, True])
+def test_close_object(device, kind, rows, last, request):
+    """Close gives the stream and the product that the calls of their own give, whichever way it takes (one rounding of h and
+    one of the product apart at most), once: a second product reads the same input."""
+    if device == "cuda":
+        request.getfixturevalue("cuda")
+    k, n = 1024, 256
+    x, o, kw = _args(kind, k, True, 3, device)
+    x, o = x.repeat(rows, 1), o.repeat(rows, 1)
+    if last:
+        kw.update(w_next=None, **({"b_next": None} if kind == "layer" else {}))
+    w = (torch.randn(n, k, generator=torch.Generator().manual_seed(4)) * k ** -0.5).bfloat16().to(device)
+    c = sm.Close(kind, x.clone(), o, **kw)
+    f = sm.post_norm_add if kind == "rms" else sm.post_layer_norm_add
+    rx, rh = f(x.clone(), o, **kw)
+    if last:
+        assert c.input() is None and torch.equal(c.x, rx)
+        return
+    y, ref = c.linear(w), ops.linear(rh, w)
+    assert (c.x - rx).norm() <= 2.0 ** -18 * rx.norm()
+    assert (y.double() - ref.double()).norm() <= 2.0 ** -7 * ref.double().norm()
+    made = sm.Close.made(x, rh)
+    assert made.input() is rh and torch.equal(made.linear(w), ref) and made.x is x
