@@ -100,6 +100,15 @@ __device__ __forceinline__ void pp_lgkm() {
   }
 }
 
+// One MFMA of accumulator row R.  The rows past the 8th (row tiles of 288) do not fit the 256 accumulation registers and stay in
+// ordinary ones: in asm, since hipcc moves them to accumulation registers and back around each of its own (240 moves a K-tile).
+// (Their operands come from LDS behind counted waits, and the sums are read behind a wait of their own at the end of the loop.)
+template <int R>
+__device__ __forceinline__ void pp_mfma(const bf16x8& b, const bf16x8& a, f32x4& acc) {
+  if constexpr (R < 8) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, a, acc, 0, 0, 0);
+  else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(b), "v"(a));
+}
+
 // Fragment-read schedule of one K-half (RT A-fragments, CT B-fragments; MFMA i uses A r = i / CT,
 // B c = i % CT).  The reads for the OTHER K-half go out after MFMA pos(): A fragment a right after
 // its register's last MFMA in this K-half (a * CT + CT - 1), B fragment b spread over the first
@@ -277,7 +286,8 @@ __device__ __forceinline__ void gemm_pp_tile(bf16 (&smem)[SMEM], const bf16* __r
 #pragma unroll
       for (int j = 0; j < CT; ++j) {
         acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-        asm volatile("" : "+a"(acc[i][j]));
+        if (i * CT + j < 64) asm volatile("" : "+a"(acc[i][j]));
+        else asm volatile("" : "+v"(acc[i][j]));               // (there are 256 accumulation registers)
       }
   };
 
@@ -345,9 +355,9 @@ __device__ __forceinline__ void gemm_pp_tile(bf16 (&smem)[SMEM], const bf16* __r
           pp_lgkm<(w0 > 15 ? 15 : w0)>();
         }
         if constexpr (h == 0)
-          acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb0[c], fa0[r], acc[r][c], 0, 0, 0);
+          pp_mfma<r>(fb0[c], fa0[r], acc[r][c]);
         else
-          acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb1[c], fa1[r], acc[r][c], 0, 0, 0);
+          pp_mfma<r>(fb1[c], fa1[r], acc[r][c]);
         if constexpr (i % 2 == 1 && i / 2 < NR) {
           rd1(base1, std::integral_constant<int, i / 2>{});
         }
@@ -387,6 +397,12 @@ __device__ __forceinline__ void gemm_pp_tile(bf16 (&smem)[SMEM], const bf16* __r
       });
       slot = nslot;
     }
+    if constexpr (RT > 8) {                            // the asm ones' last results
+      static_assert(RT == 9 && CT == 8, "eight accumulators past the 8th row");
+      asm volatile("s_nop 15\n\ts_nop 15" : "+v"(acc[8][0]), "+v"(acc[8][1]), "+v"(acc[8][2]), "+v"(acc[8][3]), "+v"(acc[8][4]),
+                   "+v"(acc[8][5]), "+v"(acc[8][6]), "+v"(acc[8][7]));
+    }
+
     if constexpr (PROF) {
       unsigned long long st1;
       asm volatile("s_memtime %0\n\ts_waitcnt lgkmcnt(0)" : "=s"(st1) :: "memory");
@@ -606,11 +622,23 @@ __device__ __forceinline__ void gemm_pp_tile(bf16 (&smem)[SMEM], const bf16* __r
 
 constexpr int pp_smem(int bn, int mode, int var) {      // bf16 elements: ring, then output image
   const int ring = bn == 256 ? (var & 128 ? 3 * (128 + 256) * PBK : 2 * (256 + 256) * PBK) : 3 * (256 + bn) * PBK;
-  const int image = 256 * ((mode == 2 && (var & 32) == 0 ? bn / 2 : bn) + 8);
+  const int image = (var & 128 ? 288 : 256) * ((mode == 2 && (var & 32) == 0 ? bn / 2 : bn) + 8);
   return ring > image ? ring : image;
 }
 
 constexpr int kMoeCus = 256;
+
+// Segments of a little more than n full row tiles (n <= 4) lie on n tiles of 288 rows, whose ninth accumulator row is in ordinary
+// registers, where that takes a round of the chip away: a tile of 288 rows takes 1.11 of a full one's time, the short one that it
+// saves 0.75 (it is bound by its weights), and the last round of a few of those as much.  us, Mixtral gate|up / down, 2036 tokens
+// (counts to either side of 512) 863 / 611 -> 773 / 380, 2200 1038 / 624 -> 789 / 393, 4096 1448 / 907 -> 1434 / 708; 8 experts 2560 x
+// 2560 at 1100 tokens 113 -> 70; 64 experts 2048 x 1408, 6 a token, 3000 tokens 310 / 153 -> 253 / 129.  In as many rounds a longer
+// tile only sets their length (8 experts of 1040 rows, 2560 x 2560 down, 400 -> 320 tiles: 110 -> 121).
+constexpr int kTall = 288;
+__device__ __forceinline__ bool moe_tall(int rows) {
+  const int n = (rows + kTall - 1) / kTall;
+  return n <= 4 && n < (rows + 255) / 256;
+}
 
 template <int BN, int MODE, int VAR>
 __global__ void __launch_bounds__(256, 1) gemm_pp_kernel(const bf16* __restrict__ A, const bf16* __restrict__ B,
@@ -628,7 +656,7 @@ __global__ void __launch_bounds__(256, 1) gemm_pp_kernel(const bf16* __restrict_
   constexpr bool MOE = (VAR & 128) != 0;
   const int ntiles = N / BN;
   int mtiles = (M + BM - 1) / BM, total = gridDim.x;
-  [[maybe_unused]] bool cut = false;
+  [[maybe_unused]] bool cut = false, tall = false;
   // (MOE: an expert per lane, 64 at a time, E <= 256.  Walked one after the other the counts cost every workgroup microseconds:
   // 64 experts 2048 x 2816, 6 a token, us at 300 / 3000 / 8192 tokens 173 / 348 / 586 -> 157 / 313 / 532, down 90 / 183 / 320 ->
   // 77 / 159 / 282)
@@ -640,7 +668,7 @@ __global__ void __launch_bounds__(256, 1) gemm_pp_kernel(const bf16* __restrict_
     // tokens 249 / 255 -> 182 / 191, 8 experts 1024 x 2048 at 300 27 -> 19.  A longer tile in the same round sets its length
     // anyway (Mixtral down at 1024 tokens, 4 tiles of 12 cut: 344 -> 358), and past one workgroup per CU the rows are staged
     // twice for nothing (gate|up at 1500 709 -> 816)
-    int shorts = 0;
+    int shorts = 0, talls = 0;
     mtiles = 0;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -656,6 +684,21 @@ __global__ void __launch_bounds__(256, 1) gemm_pp_kernel(const bf16* __restrict_
         end[q] = mtiles + t;
         mtiles += __builtin_amdgcn_readlane(t, 63);
         shorts += __popcll(__ballot(c > 0 && c <= 128));
+        talls += __popcll(__ballot(moe_tall(c)));
+      }
+    }
+    // (a tall segment saves one tile)
+    tall = talls > 0 && ((mtiles - talls) * ntiles + kMoeCus - 1) / kMoeCus < (mtiles * ntiles + kMoeCus - 1) / kMoeCus;
+    if (tall) {
+      mtiles -= talls;
+      int before = 0;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        if (64 * q < E) {
+          const uint64_t who = __ballot(moe_tall(seg[q]));
+          end[q] -= before + __popcll(who & (~0ull >> (63 - lane)));
+          before += __popcll(who);
+        }
       }
     }
     cut = shorts == mtiles && 2 * mtiles * ntiles <= kMoeCus;
@@ -688,7 +731,7 @@ __global__ void __launch_bounds__(256, 1) gemm_pp_kernel(const bf16* __restrict_
     for (int q = 0; q < 4; ++q) {
       if (64 * q < E) {
         // (cut: every tile is short and a segment's only one is two units; full tiles cannot precede it)
-        const int tiles = (seg[q] + BM - 1) / BM, to = cut ? 2 * end[q] : end[q], from = to - (cut ? 2 * tiles : tiles);
+        const int rows = tall && moe_tall(seg[q]) ? kTall : BM, tiles = (seg[q] + rows - 1) / rows, to = cut ? 2 * end[q] : end[q], from = to - (cut ? 2 * tiles : tiles);
         const uint64_t owner = __ballot(m_t >= from && m_t < to);
         if (owner) {                                   // uniform: one lane of one q
           const int l = __builtin_ctzll(owner);
@@ -698,7 +741,8 @@ __global__ void __launch_bounds__(256, 1) gemm_pp_kernel(const bf16* __restrict_
         }
       }
     }
-    const int r0 = cut ? 0 : (m_t - first) * BM;
+    tall = tall && moe_tall(rcnt);
+    const int r0 = cut ? 0 : (m_t - first) * (tall ? kTall : BM);
     const int roff = offsets[ex];
     const bf16* We = B + (size_t)ex * N * K;
     // a segment's last tile on the row tile that holds what is left (neighbour of the segment's others in the order: put
@@ -716,6 +760,7 @@ __global__ void __launch_bounds__(256, 1) gemm_pp_kernel(const bf16* __restrict_
       gemm_pp_tile<128, MODE, VAR, 4>(smem, A, We, C, P, M, N, K, 2 * n_t + m_t - first, r0, rcnt, roff, gather, split, ks0, nt, D, limit);
     else if (left <= 128) go(std::integral_constant<int, 4>{});
     else if (left <= 192) go(std::integral_constant<int, 6>{});
+    else if (left > 256 && tall) go(std::integral_constant<int, 9>{});
     else go(std::integral_constant<int, 8>{});
   } else {
     gemm_pp_tile<BN, MODE, VAR, 8>(smem, A, B, C, P, M, N, K, n_t, m_t * BM, M, 0, nullptr, split, ks0, nt, D, limit);

@@ -201,6 +201,32 @@ def test_moe_grouped_gemm_cuts_short_tiles(cuda, mode, n, counts):
 
 
 @pytest.mark.parametrize("mode", [0, 1, 2, 3])
+@pytest.mark.parametrize("counts", [[257, 288, 289, 0, 512, 513, 576, 577, 256], [864, 865, 1, 769, 128],
+                                    [1152, 1153, 1025, 1024], [0] * 70 + [300] + [0] * 70 + [545]])
+def test_moe_grouped_gemm_tall_tiles(cuda, mode, counts):
+    """Segments on either side of 1 to 4 row tiles of 288 rows: past one workgroup per CU (the padding's segments, which are on
+    tiles of 256) the bits of the launch without padding, whose tiles have 256 rows."""
+    from distributed_llms_amd import _ext
+    k, n, tokens, pad = 320, 512, 500, 256 * 9         # the padding's tiles: 9 x 2 columns x 16 experts > 256
+    x, w = _bf(tokens, k), _bf(len(counts), n, k, scale=0.1)
+    more = torch.cat([w, w[:1].expand(16, n, k)]).contiguous()
+
+    def run(c, w, n_pad):
+        c = torch.tensor(c, dtype=torch.int32, device="cuda")
+        slots = int(c.sum())
+        gather = torch.arange(slots, device="cuda", dtype=torch.int32).remainder_(tokens)
+        y = torch.full((slots + 4, n // 2 if mode in (1, 3) else n), 7.0, dtype=torch.bfloat16, device="cuda")
+        off = torch.cumsum(c, 0).to(torch.int32) - c
+        _ext.kernels().gemm_pp_moe(y.data_ptr(), x.data_ptr(), gather.data_ptr(), w.data_ptr(), c.data_ptr(), off.data_ptr(),
+                                   len(c), n, k, tokens, slots, mode, torch.cuda.current_stream().cuda_stream, 0.7)
+        assert bool((y[slots:] == 7.0).all())
+        return y[:slots - n_pad]
+
+    assert 2 * sum(-(-c // 256) for c in counts) <= 256
+    assert torch.equal(run(counts, w, 0), run(counts + [pad] * 16, more, 16 * pad))
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2, 3])
 def test_moe_grouped_gemm_last_tiles(cuda, mode):
     """Segments whose last row tile holds 1 .. 256 rows, on either side of the 128- and 192-row tiles, with empty experts
     between, gathered and not: against each segment's own f32 product, nothing written past the segments."""
