@@ -886,11 +886,12 @@ void gemm_pp_moe(uintptr_t y, uintptr_t x, uintptr_t gather, uintptr_t w, uintpt
 // tile = w + i P by P = gridDim.x workgroups, w the XCD-aware rank (workgroup b runs on XCD b % 8;
 // w = (b % 8) (P / 8) + b / 8), so each XCD's L2 serves 32 consecutive tiles of the grouped order
 // (8 row tiles x 4 column tiles) at a time.
-// Row tile BM = 32 RT (160 .. 256): a K-tile of 64 takes 1.47 / 1.31 / 1.18 / 1.02 us at 256 / 224 / 192 / 160 rows, the sum
-// of its MFMAs and its LDS traffic, so 256 rows are the most efficient and the shorter tiles are for grids that they fit into
-// fewer or cheaper rounds of the chip (ops/gemm.pf_row_tile has the rule and its figures).  160 rows leave room for a third
-// slot, which a shorter K-tile needs (4096 x 14336 at 2560 rows, one round: 253 -> 234 us).  Every row's sum over K is in the
-// same order whatever the tile.
+// Row tile BM = 32 RT (160 .. 320): a K-tile of 64 takes 1.03 / 1.19 / 1.32 / 1.48 / 1.64 / 1.85 us at 160 / 192 / 224 / 256 / 288 / 320
+// rows of full rounds, the sum of its MFMAs and its LDS traffic, at a clock that falls as the matrix cores fill (a longer tile
+// is no faster per row), so that the tiles are there for grids which they fit into fewer or cheaper rounds of the chip
+// (ops/gemm.pf_row_tile and _pf_tall have the rules and their figures).  Past 256 rows the accumulator rows that the 256 accumulation registers
+// do not hold are in ordinary ones (pp_mfma).  160 rows leave room for a third slot, which a shorter K-tile needs (4096 x 14336 at
+// 2560 rows, one round: 253 -> 234 us).  Every row's sum over K is in the same order whatever the tile.
 //
 // MODE 0: C bf16 [M, N];  2: SwiGLU C [M, N / 2] with B = [Bg; Bu] (row groups as pp_b_row);  4: the clipped GLU of
 // `limit` (common.h) in the same layout;  5: its gelu GLU;  6: 4 of the products + bias [gate | up], each lane's
@@ -1135,8 +1136,15 @@ __global__ void __launch_bounds__(256, 1) gemm_pf_kernel(const bf16* __restrict_
     for (int i = 0; i < RT; ++i)
 #pragma unroll
       for (int j = 0; j < CT; ++j) {
-        acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-        asm volatile("" : "+a"(acc[i][j]));            // zeroed in place, in AGPRs
+        if (i < 8) {
+          acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+          asm volatile("" : "+a"(acc[i][j]));          // zeroed in place, in AGPRs as far as these go
+        } else {                                       // (hipcc keeps 48 registers of zeros in scratch for a constant here)
+          float z;
+          asm volatile("v_mov_b32 %0, 0" : "=v"(z));
+          acc[i][j] = f32x4{z, z, z, z};
+          asm volatile("" : "+v"(acc[i][j]));
+        }
       }
     for (int t = 0; t < nt; ++t) {
       // schedule 2's K-tile (gemm_pp_kernel): set-1 reads from the start, barrier after MFMA IB1
@@ -1152,9 +1160,9 @@ __global__ void __launch_bounds__(256, 1) gemm_pf_kernel(const bf16* __restrict_
           pp_lgkm<(w0 > 15 ? 15 : w0)>();
         }
         if constexpr (h == 0)
-          acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb0[c], fa0[r], acc[r][c], 0, 0, 0);
+          pp_mfma<r>(fb0[c], fa0[r], acc[r][c]);
         else
-          acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb1[c], fa1[r], acc[r][c], 0, 0, 0);
+          pp_mfma<r>(fb1[c], fa1[r], acc[r][c]);
         if constexpr (i % 2 == 1 && i / 2 < NR) rd1(base1, std::integral_constant<int, i / 2>{});
         if constexpr (i == IB1) {
           asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -1173,6 +1181,12 @@ __global__ void __launch_bounds__(256, 1) gemm_pf_kernel(const bf16* __restrict_
       });
       advance();
       slot = nslot;
+    }
+    if constexpr (RT > 8) {                            // the asm ones' last results
+#pragma unroll
+      for (int r = 8; r < RT; ++r)
+        asm volatile("s_nop 15\n\ts_nop 15" : "+v"(acc[r][0]), "+v"(acc[r][1]), "+v"(acc[r][2]), "+v"(acc[r][3]), "+v"(acc[r][4]),
+                     "+v"(acc[r][5]), "+v"(acc[r][6]), "+v"(acc[r][7]));
     }
     // epilogue straight from the accumulators: acc[r][c] lane l = C[row wm TM + 16 r + (l & 15)]
     // [col wn TN + 16 c + 4 (l >> 4) + v] (SwiGLU: fragments 2 cp (gate) and 2 cp + 1 (up) hold the
@@ -1198,7 +1212,10 @@ __global__ void __launch_bounds__(256, 1) gemm_pf_kernel(const bf16* __restrict_
       // pin row r's accumulators in AGPRs up to here: hipcc would otherwise copy all 256 to VGPRs
       // at the K loop's exit (and spill, draining the pipeline with vmcnt(0) waits)
 #pragma unroll
-      for (int c = 0; c < CT; ++c) asm volatile("" : "+a"(acc[r][c]));
+      for (int c = 0; c < CT; ++c) {
+        if (r < 8) asm volatile("" : "+a"(acc[r][c]));
+        else asm volatile("" : "+v"(acc[r][c]));
+      }
       const int row = m_t * BM + wm * TM + r * 16 + lr;
       const uint32_t vo = row < M ? (uint32_t)row * (uint32_t)(ldc * 2) + colb : 0x80000000u;
       constexpr int NQ = SWIGLU ? CT / 2 : CT;         // bf16 quads per lane in this row group
@@ -1300,8 +1317,8 @@ void gemm_pf(uintptr_t c, uintptr_t a, uintptr_t b, int M, int N, int K, int mod
     if (dev >= 0 && dev < 64) cus_of[dev].store(cus, std::memory_order_relaxed);
   }
   DLLM_HOST_CHECK(bias == 0 || (mode == 3 && bias % 8 == 0), "a bias: clipped GLU, 8-byte aligned");
-  DLLM_HOST_CHECK(bm == 256 || bm == 224 || bm == 192 || bm == 160, "row tile 160, 192, 224 or 256");
-  DLLM_HOST_CHECK(bm == 256 || (!dyn && variant == 0), "row tiles below 256: static walk, default stores");
+  DLLM_HOST_CHECK(bm == 320 || bm == 288 || bm == 256 || bm == 224 || bm == 192 || bm == 160, "row tile 160, 192, 224, 256, 288 or 320");
+  DLLM_HOST_CHECK(bm == 256 || (!dyn && variant == 0), "row tiles other than 256: static walk, default stores");
   const long tiles = (long)(N / 256) * ((M + bm - 1) / bm);
   DLLM_HOST_CHECK(tiles < (1L << 30), "tiles");
   DLLM_HOST_CHECK(wgs >= 0 && wgs % 8 == 0, "workgroups in eights");
@@ -1315,6 +1332,8 @@ void gemm_pf(uintptr_t c, uintptr_t a, uintptr_t b, int M, int N, int K, int mod
 #define DLLM_PF_MODE(MODE_)                                                                              \
   do {                                                                                                   \
     if (dyn) { if (nt_store) DLLM_PF_GO(MODE_, 8, true, 8); else DLLM_PF_GO(MODE_, 0, true, 8); }        \
+    else if (bm == 320) DLLM_PF_GO(MODE_, 0, false, 10);                                                 \
+    else if (bm == 288) DLLM_PF_GO(MODE_, 0, false, 9);                                                  \
     else if (bm == 224) DLLM_PF_GO(MODE_, 0, false, 7);                                                  \
     else if (bm == 192) DLLM_PF_GO(MODE_, 0, false, 6);                                                  \
     else if (bm == 160) DLLM_PF_GO(MODE_, 0, false, 5);                                                  \

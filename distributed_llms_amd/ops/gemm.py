@@ -20,7 +20,7 @@ the engine on Llama-3-8B, profiles/wide_gemm.md; each one is a field of :mod:`..
   70B) at 225 <= M <= 256 on split gemm_pp 128-column tiles (profiles/round6_gate_up_pp.md);
 * prefill (M >= knobs.pp_swiglu_min_m / pp_proj_min_m, above the decode ranges): the 4-wave
   schedule-2 kernel in its persistent form (gemm_pf in gemm_pp.hip, knobs.pp_persistent; 256 x 256 tiles, or row tiles of
-  160, 192 or 224 where they need fewer rounds of the chip, :func:`pf_row_tile`) -- gate|up with the GLU (and a clipped
+  160 to 320 where they need fewer or cheaper rounds of the chip, :func:`pf_row_tile` and :func:`_pf_tall`) -- gate|up with the GLU (and a clipped
   one's bias) in its epilogue, qkv / o / down plain (profiles/round4_gemm_counters.md);
 * what none of them takes (a bias or N not a multiple of 128 past 64 rows, K not a multiple of 64, fp32 on CPU,
   operands >= 4 GiB): torch's F.linear.
@@ -93,6 +93,12 @@ def pf_fills(m: int, n: int, device) -> bool:
 # 5120 (320 / 368 / 432 / 512) 584 / 554 / 522 / 493; gate|up 28672 x 4096, 384 (224 / 224 / 224 / 336) 97 / 87 / 83 / 140.
 # 128 rows (1.0 us a K-tile against 1.02 for 160) never win where there is no K split.
 _PF_ROUND = {256: 1.0, 224: 0.93, 192: 0.84, 160: 0.76}
+# ... and of the longer ones, which take a round away now and then: 63 unsplit sizes (7 pairs of N 4096 .. 28672 and K 2560 .. 14336,
+# M 1232 .. 16384), each with every row tile, are 1.7 % from the best tile in the mean without them and 0.2 % with them.  us,
+# 320 / 288 rows against the best of the others: 4096 x 14336, M = 4608 (240 / 256 tiles, 464 of 160 rows) 402 / 379, 468; 4096 x 4096,
+# 4608 116 / 105, 127; 28672 x 4096, 1232 (448 / 560, 672 of 224) 226 / 280, 243, 7021 (2464 / 2800, 3584) 1164 / 1178, 1196; 6144 x 4096,
+# 3000 (240 / 264, 456 of 160) 119 / 180, 129; 15360 x 2560, 1232 78 / 119, 87; 28672 x 4096, 16384 (no round less) 2678 / 2645, 2607.
+_PF_ROUND_TALL = {288: 1.12, 320: 1.245}
 
 
 def pf_row_tile(m: int, n: int, device, cus: int = 0) -> int:
@@ -107,6 +113,22 @@ def pf_row_tile(m: int, n: int, device, cus: int = 0) -> int:
         if at is None or t < at - 1e-6:
             best, at = bm, t
     return best
+
+
+def _pf_tall(bm: int, m: int, n: int, out: int, device) -> int:
+    """gemm_pf's row tile where :func:`_pf_plan` gives ``bm``: that, or 288 or 320 rows where their walk is cheaper.  No bit hangs
+    on it; beside reserved CUs, with the dynamic tile queue (256 rows) and for outputs with nontemporal stores (a build of 256
+    rows) the plan's stays."""
+    if _comm_cus or pf_dynamic() or (out != n and m * out * 2 > 256 << 20):
+        return bm
+    cus = _cus(device)
+    rounds = lambda b: -(-(-(-m // b) * (n // 256)) // cus)
+    at = rounds(bm) * _PF_ROUND[bm]
+    for b, c in _PF_ROUND_TALL.items():
+        t = rounds(b) * c
+        if t < at - 1e-6:
+            bm, at = b, t
+    return bm
 
 
 def _pf_plan(m: int, n: int, k: int, out: int, device) -> int:
@@ -358,7 +380,7 @@ def _linear(m: int, n: int, k: int, x: torch.Tensor, w: torch.Tensor, bias: Opti
     if bias is None and _use_pp(m, n, k, x, w, knobs.K.pp_proj_min_m):
         bm = _pf_plan(m, n, k, n, x.device)
         if bm:
-            return linear_pf(x, w, bm=bm)
+            return linear_pf(x, w, bm=_pf_tall(bm, m, n, n, x.device))
         # medium M (mixed prefill + decode steps, short prompts): split-K tiles fill the CUs
         return linear_pp(x, w, variant=PP_PREFILL_VARIANT, defer=defer)
     return F.linear(x, w, bias)
@@ -552,8 +574,8 @@ def linear_pf(x: torch.Tensor, w: torch.Tensor, swiglu: bool = False, variant: i
     boundaries; optional fused SwiGLU (``w`` = [Wg; Wu], y [M, N / 2]) or -- ``limit`` -- clipped GLU (of the products plus
     ``bias`` [gate | up], where given) or -- ``gelu`` -- gelu_tanh GLU.  ``variant`` 8: nontemporal
     output stores (the default for SwiGLU outputs > 256 MiB).  256-row tiles come from per-XCD device queues while
-    knobs.pf_dynamic says so (bit 16 of the launcher's variant); shorter ones (``bm``, pf_row_tile) are walked statically, by
-    the CUs that communication leaves."""
+    knobs.pf_dynamic says so (bit 16 of the launcher's variant); others (``bm``, pf_row_tile) are walked statically, by the CUs
+    that communication leaves."""
     k = x.shape[-1]
     n = w.shape[0]
     m = x.numel() // k
@@ -573,7 +595,7 @@ def linear_pf(x: torch.Tensor, w: torch.Tensor, swiglu: bool = False, variant: i
     _ext.kernels().gemm_pf(y.data_ptr(), x.data_ptr(), w.data_ptr(), m, n, k,
                            4 if gelu else 3 if limit is not None else (1 if swiglu else 0), variant, current_stream(),
                            0.0 if limit is None else float(limit), bm, 0 if bias is None else bias.data_ptr(),
-                           _pf_wgs(_cus(x.device)) if _comm_cus and bm < 256 else 0)
+                           _pf_wgs(_cus(x.device)) if _comm_cus and bm != 256 else 0)
     return y
 
 
@@ -659,7 +681,7 @@ def _linear_glu(x: torch.Tensor, w_gate_up: torch.Tensor, limit: Optional[float]
     if not _use_wide(m, n, k, x, w_gate_up) and _use_pp(m, n, k, x, w_gate_up, knobs.K.pp_swiglu_min_m):
         bm = _pf_plan(m, n, k, n // 2, x.device)
         if bm and not (bias is not None and (limit is None or _recorded(x, w_gate_up, bias))):
-            return linear_pf(x, w_gate_up, limit=limit, gelu=limit is None, bm=bm, bias=bias)
+            return linear_pf(x, w_gate_up, limit=limit, gelu=limit is None, bm=_pf_tall(bm, m, n, n // 2, x.device), bias=bias)
     if bias is not None:
         return None
     y = linear(x, w_gate_up, defer=True)
@@ -707,6 +729,6 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor) -> Optional[torch.Te
     if _use_pp(m, n, k, x, w_gate_up, knobs.K.pp_swiglu_min_m):
         bm = _pf_plan(m, n, k, n // 2, x.device)
         if bm:
-            return linear_pf(x, w_gate_up, swiglu=True, bm=bm)
+            return linear_pf(x, w_gate_up, swiglu=True, bm=_pf_tall(bm, m, n, n // 2, x.device))
         return linear_pp(x, w_gate_up, swiglu=True, variant=PP_PREFILL_VARIANT)
     return None

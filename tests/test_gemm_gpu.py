@@ -367,6 +367,23 @@ def test_pf_row_tiles_bit_exact(cuda, bm, m, n, k):
         assert torch.equal(gemm.linear_pf(x, w, bm=bm, **kw), gemm.linear_pf(x, w, **kw)), kw
 
 
+@pytest.mark.parametrize("bm", [288, 320])
+@pytest.mark.parametrize("m", [1, 289, 577, 1921, 4500])
+@pytest.mark.parametrize("n,k", [(256, 64), (512, 192), (4096, 128), (4096, 1088)])
+def test_pf_tall_row_tiles_bit_exact(cuda, bm, m, n, k):
+    """Row tiles past 256, whose last accumulator rows are in other registers: as test_pf_row_tiles_bit_exact, and the biased
+    GLU; nothing written past the output."""
+    torch.manual_seed(bm + m + n)
+    x, w = _bf(m, k), _bf(n, k, scale=0.1)
+    b = torch.randn(n, device="cuda").bfloat16()
+    for kw in ({}, {"swiglu": True}, {"limit": 0.7}, {"gelu": True}, {"limit": 0.7, "bias": b}):
+        assert torch.equal(gemm.linear_pf(x, w, bm=bm, **kw), gemm.linear_pf(x, w, **kw)), kw
+    from distributed_llms_amd import _ext
+    y = torch.full((m + 2, n), 7.0, dtype=torch.bfloat16, device="cuda")
+    _ext.kernels().gemm_pf(y.data_ptr(), x.data_ptr(), w.data_ptr(), m, n, k, 0, 0, torch.cuda.current_stream().cuda_stream, 0.0, bm, 0, 0)
+    assert bool((y[m:] == 7.0).all()) and torch.equal(y[:m], gemm.linear_pf(x, w))
+
+
 @pytest.mark.parametrize("m,bm", [(1, 256), (300, 256), (161, 160), (900, 192), (449, 224)])
 @pytest.mark.parametrize("f,k", [(128, 64), (640, 192)])
 def test_pf_clipped_glu_bias(cuda, m, bm, f, k):

@@ -334,6 +334,28 @@ def test_pf_row_tile_takes_the_cheapest_walk():
         gemm.release_cus_for_comm()
 
 
+def test_pf_tall_takes_a_round_away():
+    """Row tiles of 288 and 320 rows where their walk is cheaper than the plan's, never dearer; not beside reserved CUs, with the
+    dynamic queue or for outputs that are stored past the caches."""
+    cpu = torch.device("cpu")
+    assert gemm._pf_tall(160, 4608, 4096, 4096, cpu) == 288        # one round instead of two of 160 rows
+    assert gemm._pf_tall(224, 1232, 28672, 14336, cpu) == 320      # two instead of three
+    assert gemm._pf_tall(256, 8192, 4096, 4096, cpu) == 256        # two full ones
+    for m in range(257, 9000, 173):
+        for n in (2560, 4096, 6144, 28672):
+            bm = gemm._pf_plan(m, n, 4096, n, cpu)
+            if bm:
+                tall = gemm._pf_tall(bm, m, n, n, cpu)
+                rounds = [-(-(-(-m // b) * (n // 256)) // 256) for b in (bm, tall)]
+                assert tall == bm or (tall in (288, 320) and rounds[1] < rounds[0])
+    assert gemm._pf_tall(256, 16385, 28672, 14336, cpu) == 256     # more than 256 MiB
+    gemm.reserve_cus_for_comm(16)
+    try:
+        assert gemm._pf_tall(160, 4608, 4096, 4096, cpu) == 160
+    finally:
+        gemm.release_cus_for_comm()
+
+
 @pytest.mark.parametrize("m", [1, 8, 64, 128, 129, 256])
 def test_wide_splits_keep_slices_of_8_k_tiles(m):
     """A slice's sum is handed on in 16 bits, so no slice is shorter than 8 K-tiles, and where the reserved CUs leave room for as
