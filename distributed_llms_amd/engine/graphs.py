@@ -14,11 +14,64 @@ from typing import Dict, Optional, Tuple
 import torch
 
 from ..models.stage import BatchMeta, ModelStage
+from ..ops.stream import current_stream
 from .batch import HostBatch, next_pow2
 
 SCRATCH_SEQ_ID = -1      # owns block 0 (and state slot 0) in the BlockManager
 NROWS = 5                # per-row int32 inputs: ids, positions, slots, seq_lens, state slots
 _CAPTURE_LOCK = threading.Lock()   # one graph capture at a time per process
+
+
+class StagingRing:
+    """Pinned host buffers for the inputs of successive steps, used in turn.  A buffer may be written again once its copy to the
+    device is done; an event behind every copy says so, but holds the stream for 5 us between the copy and the step's graph
+    (195 us a step of a small model for one request), so that one is recorded for half of the ring at a time, and for the copies
+    of a stream that the next step leaves.  ``torch.cuda`` streams live as long as the process; on a caller's own (an
+    ExternalStream, which may be gone by the next step) every copy has its event."""
+
+    BUFFERS = 8
+
+    def __init__(self, size: int):
+        self.buffers = torch.empty(self.BUFFERS, size, dtype=torch.int32)
+        if torch.cuda.is_available():
+            self.buffers = self.buffers.pin_memory()
+        self.arrays = self.buffers.numpy()
+        self.at = 0
+        self.done = ([], [])             # per half of the ring: the events behind its copies
+        self.open = None                 # (handle, stream) of copies that no event covers yet
+        self.known = None                # (handle, stream): of the last step, the object is costly to make
+
+    def take(self) -> int:
+        """Index of the next buffer, free to be written."""
+        half = self.BUFFERS // 2
+        if self.at % half == 0:
+            events = self.done[self.at // half]
+            for e in events:
+                e.synchronize()
+            events.clear()
+        return self.at
+
+    def sent(self):
+        """The copy of the buffer that :meth:`take` gave has been issued on the current stream."""
+        half = self.BUFFERS // 2
+        events = self.done[self.at // half]
+        handle = current_stream()
+        if self.known is None or self.known[0] != handle:
+            self.known = (handle, torch.cuda.current_stream())
+        if self.open is not None and self.open[0] != handle:
+            events.append(self._event(self.open[1]))
+        self.open = self.known
+        own = handle == 0 or self.known[1].stream_id & 1                # (torch's encoding: its own streams are odd)
+        if self.at % half == half - 1 or not own:
+            events.append(self._event(self.known[1]))
+            self.open = None
+        self.at = (self.at + 1) % self.BUFFERS
+
+    @staticmethod
+    def _event(stream):
+        e = torch.cuda.Event()
+        e.record(stream)
+        return e
 
 
 class DecodeGraphRunner:
@@ -55,11 +108,9 @@ class DecodeGraphRunner:
         max_splits = 64
         self.ws = (torch.empty(mb * cfg.num_heads * max_splits * cfg.head_dim, dtype=torch.float32, device=dev),
                    torch.empty(mb * cfg.num_heads * max_splits * 2, dtype=torch.float32, device=dev))
-        self.pinned = torch.empty(NROWS * mb + mb * max_blocks, dtype=torch.int32).pin_memory()
-        self.pinned_np = self.pinned.numpy()
+        self.staging = StagingRing(NROWS * mb + mb * max_blocks)
         self.graphs: Dict[Tuple[int, int], Tuple[torch.cuda.CUDAGraph, torch.Tensor]] = {}
         self.pool = None
-        self.copy_done: Optional[torch.cuda.Event] = None
         self.capture_stream: Optional[torch.cuda.Stream] = None
 
     def bucket(self, b: int, max_ctx: int) -> Tuple[int, int]:
@@ -119,12 +170,11 @@ class DecodeGraphRunner:
         mbk = hb.block_tables.shape[1]
         if mbk > self.max_blocks:
             raise ValueError("block table wider than graph buffers")
-        if self.copy_done is not None:
-            self.copy_done.synchronize()   # previous step's H2D may still read the pinned buffer
-        # numpy views of the pinned staging buffer: a handful of memcpy-sized writes per step
+        # numpy views of a pinned staging buffer: a handful of memcpy-sized writes per step
         # instead of one torch op (~5-10 us of host time each) per field
         n, mb, w = bb, self.max_batch, self.max_blocks
-        p = self.pinned_np
+        buf = self.staging.take()
+        p = self.staging.arrays[buf]
         pv = p[: NROWS * mb].reshape(NROWS, mb)
         pv[0, :b] = hb.ids
         pv[1, :b] = hb.positions
@@ -140,10 +190,8 @@ class DecodeGraphRunner:
         bt[:b, mbk:] = 0
         bt[b:] = 0
         cnt = NROWS * mb + n * w
-        self.dev_in[:cnt].copy_(self.pinned[:cnt], non_blocking=True)
-        if self.copy_done is None:
-            self.copy_done = torch.cuda.Event()
-        self.copy_done.record()
+        self.dev_in[:cnt].copy_(self.staging.buffers[buf, :cnt], non_blocking=True)
+        self.staging.sent()
         if hidden is not None:
             self.hidden[:b].copy_(hidden[:b])
             if bb > b:
