@@ -39,6 +39,7 @@ PYBIND11_MODULE(_C_kernels, m) {
   m.def("gemm_pp", &dllm::gemm_pp);
   m.def("gemm_pf", &dllm::gemm_pf, py::arg("c"), py::arg("a"), py::arg("b"), py::arg("m"), py::arg("n"), py::arg("k"),
         py::arg("mode"), py::arg("variant"), py::arg("stream"), py::arg("limit") = 0.f, py::arg("bm") = 256, py::arg("bias") = 0, py::arg("wgs") = 0);
+  m.def("gemm_pf8", &dllm::gemm_pf8);
   m.def("moe_combine", &dllm::moe_combine);
   m.def("moe_wide_gemm", &dllm::moe_wide_gemm, py::arg("y"), py::arg("x"), py::arg("gather"), py::arg("w"), py::arg("counts"), py::arg("offsets"), py::arg("experts"), py::arg("n"), py::arg("k"), py::arg("mode"), py::arg("stream"),
         py::arg("limit") = 0.f);

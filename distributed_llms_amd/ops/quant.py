@@ -11,7 +11,8 @@ the bf16 ridge at batch 256 -- get both halves of their bound cut:
   (csrc/kernels/quant.hip);
 * GEMM: ``gemm_wide_fp8`` (csrc/kernels/gemm_wide.hip) -- the wide kernel's LDS-DMA pipeline with
   fp8 K-tiles of 128, scales applied in the epilogue (also before SwiGLU and before split-K slabs,
-  so the bf16 path's deferred reductions are reused unchanged).
+  so the bf16 path's deferred reductions are reused unchanged); the larger prompt products on ``gemm_pf8``
+  (csrc/kernels/gemm_pf8.hip), persistent workgroups on 256-column tiles with the same bits.
 
 Mixtral experts take the same scheme through the grouped kernel (``moe_wide_gemm_fp8``: fp8 token
 rows gathered by the expert-sorted slot list, per-(expert, channel) weight scales).
@@ -246,6 +247,34 @@ def _prompt_plan(m: int, n: int, k: int, most: int, cus: int, swiglu: bool) -> T
     return plan if cus == 256 else (plan[0], min((256, 192, 128, 64), key=lambda bm: us(plan[0], bm, cus)))
 
 
+# gemm_pf8 (256-column tiles, persistent) against that: us per K-tile of 128 and round, per K-tile of a full chip's tiles (the clock
+# falls as the matrix cores fill), per round (epilogue, first K-tiles) and once.  Fitted over 17 weights (512 x 2048 ... 57344 x 8192)
+# at 257 ... 4096 rows, 289 sizes, to 4 % where the tile is a likely one; gemm_wide_fp8 takes 1.11 times its model in the mean there.
+# Of the 199 that the plan leaves whole none is slower than it was, and together they take 0.73 of the time (29.6 -> 21.6 ms; the better
+# kernel and tile at each: 21.5).  us at 2560 rows:
+# 28672 x 4096 with its SwiGLU 315 -> 221 (2.7 PFLOP/s; at 8192 rows 956 -> 629, 3.1), 4096 x 14336 169 -> 103, 6144 x 4096 68 -> 48,
+# 4096 x 4096 54 -> 35; 28672 x 4096 at 300 rows 52 -> 35.  A product that the plan splits takes gemm_pf8 a fifth to a half longer.
+_PF8_US = {160: (0.572, 0.28, 3.6, 3.7), 192: (0.643, 0.321, 4.75, 2.8), 224: (0.64, 0.474, 4.9, 3.65), 256: (0.77, 0.484, 6.0, 2.85)}
+
+
+@functools.lru_cache(maxsize=1024)
+def _pf8_plan(m: int, n: int, k: int, bm: int) -> int:
+    """gemm_pf8's row tile for a product past 256 rows that :func:`fp8_plan` leaves whole, on row tiles of ``bm``; 0 where that is
+    cheaper (a small product: half as many columns per tile leave fewer CUs idle).  No bit hangs on it."""
+    if n % 256 or k % 256 or k < 512 or m * k >= 1 << 32 or n * k >= 1 << 32 or m * n * 2 >= 1 << 31:
+        return 0
+    kt, rounds = k // 128, -(-(n // 128) * -(-m // bm) // 256)
+    tile_us, fixed = _ROUND_US[bm]
+    best = 1.04 * ((tile_us + _ROUND_64 * (rounds - 1)) * kt + fixed if bm == 64 else rounds * (tile_us * kt + fixed)) + 1.5
+    plan = 0
+    for rows, (a, b, e, f) in _PF8_US.items():
+        tiles = n // 256 * -(-m // rows)
+        us = kt * (a * -(-tiles // 256) + b * tiles / 256) + e * -(-tiles // 256) + f
+        if us < best:
+            best, plan = us, rows
+    return plan
+
+
 def fp8_plan(m: int, n: int, k: int, swiglu: bool = False) -> Tuple[int, int]:
     """(K slices, row-tile override or 0) of gemm_wide_fp8 for this shape.  Past 256 rows the cheapest
     grid (:func:`_prompt_plan`) of the CUs that communication leaves.  Default: the bf16 kernel's rule on the 128-K tiles (a K-tile
@@ -289,7 +318,7 @@ def linear_fp8(x: torch.Tensor, w: Fp8Weight, swiglu: bool = False, defer: bool 
     ``defer``: may return a :class:`~distributed_llms_amd.ops.gemm.SplitKPartial` (no SwiGLU)."""
     if not x.is_cuda:
         return linear_ref(x, w, swiglu)
-    from .gemm import SplitKPartial, _workspace
+    from . import gemm
     pre = isinstance(x, Fp8Act)
     k = x.shape[-1]
     n, kw = w.shape
@@ -309,7 +338,7 @@ def linear_fp8(x: torch.Tensor, w: Fp8Weight, swiglu: bool = False, defer: bool 
     s, bm = fp8_plan(m, n, k, swiglu)
     if splits:
         s, bm = splits, 0
-    ws = _workspace(x.device)
+    ws = gemm._workspace(x.device)
     if s > 1 and s * m * n > ws.numel():
         s = max(1, ws.numel() // (m * n))
     variant = fp8_variant(m, n, k, s, bm)
@@ -318,8 +347,16 @@ def linear_fp8(x: torch.Tensor, w: Fp8Weight, swiglu: bool = False, defer: bool 
     if defer and not swiglu and s > 1:
         se = kern.gemm_wide_fp8(0, xq.data_ptr(), xs.data_ptr(), w.q.data_ptr(), w.scale.data_ptr(), ws.data_ptr(),
                                 ws.numel(), m, n, k, s, 2, variant, stream)
-        return SplitKPartial(ws, se, m, n, (*x.shape[:-1], n), x.dtype, x.device)
+        return gemm.SplitKPartial(ws, se, m, n, (*x.shape[:-1], n), x.dtype, x.device)
     y = torch.empty(*x.shape[:-1], n // 2 if swiglu else n, dtype=x.dtype, device=x.device)
+    # (beside reserved CUs a persistent workgroup could wait for its CU with a whole share of the tiles)
+    rows = 0
+    if m > 256 and s == 1 and bm and not gemm._comm_cus and (xq.data_ptr() | w.q.data_ptr()) % 16 == 0:
+        rows = _pf8_plan(m, n, k, bm)
+    if rows:
+        kern.gemm_pf8(y.data_ptr(), xq.data_ptr(), xs.data_ptr(), w.q.data_ptr(), w.scale.data_ptr(), m, n, k,
+                      1 if swiglu else 0, rows, stream)
+        return y
     kern.gemm_wide_fp8(y.data_ptr(), xq.data_ptr(), xs.data_ptr(), w.q.data_ptr(), w.scale.data_ptr(), ws.data_ptr(),
                        ws.numel(), m, n, k, s, 1 if swiglu else 0, variant, stream)
     return y

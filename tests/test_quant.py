@@ -151,6 +151,20 @@ def test_fp8_prompt_plan_splits_alike_beside_communication():
     assert all(a[0] == b[0] and b[1] in (64, 128, 192, 256) for _, a, b in alike), [v for v in alike if v[1][0] != v[2][0]][:5]
 
 
+def test_pf8_plan_takes_what_the_kernel_takes():
+    """A row tile that gemm_pf8 is built for, only for sizes that it takes; small products stay on the plan's tiles."""
+    from distributed_llms_amd.ops import quant
+    for m in (257, 449, 1000, 2560, 8192, 100000):
+        for n in (128, 256, 384, 4096, 28672):
+            for k in (128, 256, 384, 512, 640, 4096, 14336):
+                for bm in (64, 128, 192, 256):
+                    rows = quant._pf8_plan(m, n, k, bm)
+                    assert rows in (0, 160, 192, 224, 256)
+                    assert not rows or (n % 256 == 0 and k % 256 == 0 and k >= 512 and m * k < 1 << 32 and m * n * 2 < 1 << 31)
+    assert quant._pf8_plan(300, 512, 512, 64) == 0 and quant._pf8_plan(2560, 4096, 14336, 192) == 160
+    assert quant._pf8_plan(8192, 28672, 4096, 256) == 256 and quant._pf8_plan(70000, 28672, 4096, 256) == 0
+
+
 def test_fp8_weights_read_by_several_row_tiles_are_cached():
     """Nontemporal weights only where one row tile reads them (or the deep ring of 64-row tiles goes with it); short slices and
     small matrices keep the default policy."""

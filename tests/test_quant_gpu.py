@@ -69,6 +69,38 @@ def test_fp8_row_tiles_bit_exact(monkeypatch, m, n, k, swiglu):
     assert err <= 2e-2 * out[256].float().abs().max().item() + 1e-3, err
 
 
+@pytest.mark.parametrize("bm", [160, 192, 224, 256])
+@pytest.mark.parametrize("m,n,k,swiglu", [(1, 256, 512, False), (257, 512, 512, True), (449, 768, 768, False),
+                                          (2817, 512, 1280, True), (2100, 7168, 512, False)])
+def test_gemm_pf8_bit_exact(m, n, k, swiglu, bm):
+    """The persistent prompt kernel on one tile, ragged last row tiles, the fewest K-tiles, several tiles per workgroup and a last
+    group of fewer row tiles: the bits of gemm_wide_fp8 (the same products in the same order), and no write past the output."""
+    from distributed_llms_amd import _ext
+    kern, stream = _ext.kernels(), torch.cuda.current_stream().cuda_stream
+    w, x = quant.quantize_weight((torch.randn(n, k) * 0.02).to(DEV)), _x(m, k, seed=m)
+    xq, xs = quant.quantize_rows(x)
+    out = n // 2 if swiglu else n
+    ref = torch.empty(m, out, dtype=torch.bfloat16, device=DEV)
+    kern.gemm_wide_fp8(ref.data_ptr(), xq.data_ptr(), xs.data_ptr(), w.q.data_ptr(), w.scale.data_ptr(), 0, 0, m, n, k, 1,
+                       1 if swiglu else 0, 4, stream)
+    y = torch.full((m + 1, out), 7.0, dtype=torch.bfloat16, device=DEV)
+    kern.gemm_pf8(y.data_ptr(), xq.data_ptr(), xs.data_ptr(), w.q.data_ptr(), w.scale.data_ptr(), m, n, k,
+                  1 if swiglu else 0, bm, stream)
+    assert torch.equal(y[:m], ref) and bool((y[m] == 7.0).all())
+    want = _oracle(x, w, swiglu)
+    assert (ref.float().cpu() - want).abs().max().item() <= 2e-2 * want.abs().max().item() + 1e-3
+
+
+@pytest.mark.parametrize("m,n,k,swiglu", [(300, 28672, 1024, True), (2100, 4096, 4096, False)])
+def test_fp8_prompt_products_take_the_persistent_kernel(monkeypatch, m, n, k, swiglu):
+    """Through the entry point: the plan's row tile, and the bits of the kernel that it replaces."""
+    assert quant._pf8_plan(m, n, k, quant.fp8_plan(m, n, k, swiglu)[1])
+    w, x = quant.quantize_weight((torch.randn(n, k) * 0.02).to(DEV)), _x(m, k, seed=m)
+    y = quant.linear_fp8(x, w, swiglu=swiglu)
+    monkeypatch.setattr(quant, "_pf8_plan", lambda *a: 0)
+    assert torch.equal(y, quant.linear_fp8(x, w, swiglu=swiglu))
+
+
 @pytest.mark.parametrize("m,n,k,swiglu,plan", [(300, 1024, 8192, False, (6, 64)), (700, 1024, 8192, False, (5, 128)),
                                                (640, 4096, 14336, False, (2, 192)), (300, 1024, 4096, True, (4, 64))])
 def test_fp8_prompt_plan_splits(m, n, k, swiglu, plan):
