@@ -123,25 +123,27 @@ __global__ void __launch_bounds__(256, 1) gemm_pf8_kernel(const uint8_t* __restr
       __builtin_amdgcn_make_buffer_rsrc((void*)C, (short)0, (int)(unsigned)((long)M * ldc * 2), 0x00020000);
   const __amdgpu_buffer_rsrc_t rsSa = __builtin_amdgcn_make_buffer_rsrc((void*)sa, (short)0, M * 4, 0x00020000);
   const __amdgpu_buffer_rsrc_t rsSb = __builtin_amdgcn_make_buffer_rsrc((void*)sb, (short)0, N * 4, 0x00020000);
-  uint32_t chunk_q[2], offB[2], offA[GA];
+  uint32_t chunk_q[2], offB[2], offA[GA], offBv[GB];
 #pragma unroll
   for (int par = 0; par < 2; ++par) {
     chunk_q[par] = (uint32_t)(pswz(8 * par + (lane >> 3), lane & 7) * 16);
     offB[par] = (uint32_t)(lane >> 3) * (uint32_t)K + chunk_q[par];
   }
-  int s_i = 0, s_kt = 0, s_n = 0;
+  int s_i = 0, s_kt = 0;
   // staging side onto my i-th tile: its rows' offsets (past M: the last row again) and its scales, into the buffer that the
   // tile before last has left (nt >= 4: every wave has passed a barrier of the tile in between since)
   auto set_stage = [&](int i) {
     int m_t, n_t;
     tile_mn(w + i * P, m_t, n_t);
-    s_n = n_t;
     const int r0 = m_t * BM;
 #pragma unroll
     for (int j = 0; j < GA; ++j) {
       const int q = wv * GA + j, r = 8 * q + (lane >> 3);
       offA[j] = (uint32_t)min(r0 + r, M - 1) * (uint32_t)K + chunk_q[q & 1];
     }
+#pragma unroll
+    for (int j = 0; j < GB; ++j)
+      offBv[j] = (uint32_t)pp_b_row<BN, SWIGLU>(8 * (wv * GB + j), n_t, N / 2) * (uint32_t)K + offB[j & 1];
     uint8_t* sc = smem + NB * SLOT + (i & 1) * SCALES * 4 + wv * 256;
     const int j = 64 * wv + lane;
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsSa, (lds_vptr_p)sc, 4, min(r0 + j, M - 1) * 4, 0, 0, 0);
@@ -154,10 +156,8 @@ __global__ void __launch_bounds__(256, 1) gemm_pf8_kernel(const uint8_t* __restr
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rsA, (lds_vptr_p)(base + (wv * GA + p) * 1024), 16, (int)offA[p], s_kt * BK, 0,
                                                0);
     } else {
-      const int q = wv * GB + p - GA;
-      const uint32_t brow = (uint32_t)pp_b_row<BN, SWIGLU>(8 * q, s_n, N / 2);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsB, (lds_vptr_p)(base + BM * BK + q * 1024), 16, (int)offB[q & 1],
-                                               (int)(brow * (uint32_t)K + (uint32_t)(s_kt * BK)), 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsB, (lds_vptr_p)(base + BM * BK + (wv * GB + p - GA) * 1024), 16,
+                                               (int)offBv[p - GA], s_kt * BK, 0, 0);
     }
   };
   // next staging K-tile; past my last tile: K-tile nt - 1 of it again (into a slot nobody reads again, so that every K-tile

@@ -186,6 +186,13 @@ __device__ __forceinline__ void gemm_pp_tile(bf16 (&smem)[SMEM], const bf16* __r
   // counts
   // schedule 2 stages through buffer loads: a 32-bit per-lane offset + an SGPR offset per piece
   // (K-tile, B row group), so no 64-bit VGPR address math in the MFMA stream (register pressure)
+  constexpr bool BV = SCHED2 && RT <= 8;               // a register per B piece, its row included (gemm_pf)
+  [[maybe_unused]] uint32_t offBv[BV ? GB : 1];
+  if constexpr (BV) {
+#pragma unroll
+    for (int j = 0; j < GB; ++j)
+      offBv[j] = (uint32_t)pp_b_row<BN, SWIGLU>(8 * (wv * GB + j), n_t, N / 2) * (uint32_t)(K * 2) + offB[j & 1];
+  }
   [[maybe_unused]] __amdgpu_buffer_rsrc_t rsA, rsB;
   if constexpr (SCHED2) {
     rsA = __builtin_amdgcn_make_buffer_rsrc((void*)Ab, (short)0, (int)((long)M * K * 2 - (long)ks0 * 128), 0x00020000);
@@ -198,6 +205,9 @@ __device__ __forceinline__ void gemm_pp_tile(bf16 (&smem)[SMEM], const bf16* __r
       if (p < GA) {
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsA, (lds_vptr_p)(base + (wv * GA + p) * 512), 16, (int)offA[p],
                                                  ks * PBK * 2, 0, 0);
+      } else if constexpr (BV) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsB, (lds_vptr_p)(base + BM * PBK + (wv * GB + p - GA) * 512), 16,
+                                                 (int)offBv[p - GA], ks * PBK * 2, 0, NT ? 2 : 0);
       } else {
         const int q = wv * GB + p - GA;
         const int brow = pp_b_row<BN, SWIGLU>(8 * q, n_t, N / 2);
@@ -837,7 +847,7 @@ void gemm_pp_moe(uintptr_t y, uintptr_t x, uintptr_t gather, uintptr_t w, uintpt
 // tile = w + i P by P = gridDim.x workgroups, w the XCD-aware rank (workgroup b runs on XCD b % 8;
 // w = (b % 8) (P / 8) + b / 8), so each XCD's L2 serves 32 consecutive tiles of the grouped order
 // (8 row tiles x 4 column tiles) at a time.
-// Row tile BM = 32 RT (160 .. 320): a K-tile of 64 takes 1.03 / 1.19 / 1.32 / 1.48 / 1.64 / 1.85 us at 160 / 192 / 224 / 256 / 288 / 320
+// Row tile BM = 32 RT (160 .. 320): a K-tile of 64 takes 1.00 / 1.16 / 1.32 / 1.45 / 1.61 / 1.77 us at 160 / 192 / 224 / 256 / 288 / 320
 // rows of full rounds, the sum of its MFMAs and its LDS traffic, at a clock that falls as the matrix cores fill (a longer tile
 // is no faster per row), so that the tiles are there for grids which they fit into fewer or cheaper rounds of the chip
 // (ops/gemm.pf_row_tile and _pf_tall have the rules and their figures).  Past 256 rows the accumulator rows that the 256 accumulation registers
@@ -971,18 +981,30 @@ __global__ void __launch_bounds__(256, 1) gemm_pf_kernel(const bf16* __restrict_
   uint32_t offB[2];
 #pragma unroll
   for (int par = 0; par < 2; ++par) offB[par] = (uint32_t)(lane >> 3) * (uint32_t)(K * 2) + chunk_q[par];
-  uint32_t offA[GA];
-  int s_i = 0, s_kt = 0, s_n = 0;
+  // A piece is one load and one write of m0: any further instruction is an issue slot of the one wave between two products of 16
+  // cycles (two adds and a multiplication per B piece before: a K-tile of 256 rows took 2540 cycles, now 2400, 2048 of them products).
+  // BV: a register per B piece, its row included; past 256 rows there are none left, and an add makes the scalar offset.
+  // us, 4096 x 14336 at 2560 / 4096 / 5120 rows (160, 256 and 320 a tile) 249 / 342 / 425 -> 231 / 332 / 406, 4096 x 4096 at 8192 193 ->
+  // 186, 8192 x 8192 x 8192 740 -> 720
+  constexpr bool BV = RT <= 8;
+  uint32_t offA[GA], offBv[BV ? GB : 1];
+  int s_i = 0, s_kt = 0;
+  uint32_t s_n = 0, s_b = 0;                           // (not BV) byte offset of the column tile, and of its staging K-tile
   int pend = -1, pend_i = 0;                           // DYN (lane 0): fetch in flight, its ordinal
   auto set_stage = [&](int tau) {
     int m_t, n_t;
     tile_mn(tau, m_t, n_t);
-    s_n = n_t;
+    s_b = s_n = (uint32_t)(n_t * OUTW) * (uint32_t)(K * 2);
     const int r0 = m_t * BM;
 #pragma unroll
     for (int j = 0; j < GA; ++j) {
       const int q = wv * GA + j, r = 8 * q + (lane >> 3);
       offA[j] = (uint32_t)min(r0 + r, M - 1) * (uint32_t)(K * 2) + chunk_q[q & 1];
+    }
+    if constexpr (BV) {
+#pragma unroll
+      for (int j = 0; j < GB; ++j)
+        offBv[j] = (uint32_t)pp_b_row<BN, SWIGLU>(8 * (wv * GB + j), n_t, N / 2) * (uint32_t)(K * 2) + offB[j & 1];
     }
   };
   // piece p of the staging K-tile into ring slot `slot`
@@ -991,12 +1013,13 @@ __global__ void __launch_bounds__(256, 1) gemm_pf_kernel(const bf16* __restrict_
     if (p < GA) {
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rsA, (lds_vptr_p)(base + (wv * GA + p) * 512), 16, (int)offA[p],
                                                s_kt * PBK * 2, 0, 0);
+    } else if constexpr (BV) {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsB, (lds_vptr_p)(base + BM * PBK + (wv * GB + p - GA) * 512), 16,
+                                               (int)offBv[p - GA], s_kt * PBK * 2, 0, 0);
     } else {
-      const int q = wv * GB + p - GA;
-      const uint32_t brow = (uint32_t)pp_b_row<BN, SWIGLU>(8 * q, s_n, N / 2);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsB, (lds_vptr_p)(base + BM * PBK + q * 512), 16, (int)offB[q & 1],
-                                               (int)(brow * (uint32_t)(K * 2) + (uint32_t)(s_kt * PBK * 2)),
-                                               0, 0);
+      const uint32_t row = (uint32_t)pp_b_row<BN, SWIGLU>(8 * (wv * GB + p - GA), 0, N / 2);      // in the first column tile
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsB, (lds_vptr_p)(base + BM * PBK + (wv * GB + p - GA) * 512), 16,
+                                               (int)offB[(p - GA) & 1], (int)(row * (uint32_t)(K * 2) + s_b), 0, 0);
     }
   };
   // next staging K-tile; past my last tile: K-tile nt - 1 of it again (a DUMMY piece into a slot
@@ -1033,6 +1056,7 @@ __global__ void __launch_bounds__(256, 1) gemm_pf_kernel(const bf16* __restrict_
         s_kt = nt - 1;
       }
     }
+    s_b = s_n + (uint32_t)(s_kt * PBK * 2);
   };
 
   const uint32_t lds_base = (uint32_t)(size_t)(lds_vptr_p)smem;
