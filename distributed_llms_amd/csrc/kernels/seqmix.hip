@@ -1188,102 +1188,232 @@ __global__ void __launch_bounds__(256) sm_rglru_gates_kernel(float* __restrict__
   }
 }
 
+// e^x, 1 / (1 + e^-x) and the square root as exact as the library's, in half of its instructions.  e^x = 2^n 2^f, n the nearest integer
+// to x log2(e) and f what is left (log2(e) in two floats); infinities by the clamp, which NaN pass.  The quotient and the root off the
+// hardware's reciprocal and reciprocal root and a Newton step each, without the scaling that hipcc's have.
+__device__ __forceinline__ float exp_near(float x) {
+  x = __builtin_elementwise_minimum(__builtin_elementwise_maximum(x, -1000.f), 1000.f);
+  const float n = rintf(x * 1.44269502f);
+  const float f = fmaf(x, 1.92596300e-8f, fmaf(x, 1.44269502f, -n));
+  return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(f), (int)n);
+}
+__device__ __forceinline__ float sigmoid_near(float x) {
+  const float d = 1.0f + exp_near(-x), q = __builtin_amdgcn_rcpf(d);
+  return d < __builtin_inff() ? fmaf(q, fmaf(-d, q, 1.0f), q) : q;
+}
+__device__ __forceinline__ float sqrt_near(float x) {          // x <= 0: 0
+  const float y = __builtin_amdgcn_rsqf(x), s = x * y;
+  return x > 0.f ? fmaf(fmaf(-s, s, x), 0.5f * y, s) : 0.f * x;
+}
+
 // The same products for bf16 gate matrices on the bf16 matrix cores, as exact as on the float32 ones: u = h + m + l in three
 // bf16 pieces (8 significant bits each, 24 in all: nothing of u is lost), each times the bf16 weight an exact product, the
-// sums in float32.  Three products at 16 times the rate.  One workgroup per (128 tokens, block b, 128 outputs): wave w owns
-// 32 outputs and 4 x 32 tokens of both gates; the pieces of u pass through LDS in K chunks of kSK (rows kSP apart: the 16
-// byte reads of 8 rows fall on banks of their own), the weights come from global memory one k-step of 16 ahead.
-// 6376 tokens, 10 blocks of 256: 275 us on the float32 matrix cores, 133 us here (0.38 PFLOP/s of bf16 products); 168 tokens,
-// 4 blocks: 40 and 39 us.  Error of a and g against 64 bits 1.8e-7 and 1.1e-7 there, 1.1e-7 and 0.8e-7 here.
-constexpr int kST = 128;      // tokens per workgroup
+// sums in float32.  Three products at 16 times the rate: 20 us of them, beside which the vector work (taking u apart, putting
+// the weights' columns together, the gates' functions) bounds it.  One workgroup per (64 tokens, block b, 256 outputs): two waves by
+// tokens, two by outputs, and of a wave's 128 outputs lane n owns 4 n .. 4 n + 3, one in each of four products: u is taken apart once
+// per block, the weights come in 8-byte loads a k-step of 16 ahead (8 rows of them make four fragments in 16 v_perm), u, a and g
+// in 16-byte ones.  The pieces of u pass through LDS in K chunks of kSK, two of them (rows kSP apart: the 16 byte reads of 8
+// rows fall on banks of their own); two workgroups share a CU, one's vector work under the other's products.
+// us, 10 blocks of 256, 6376 / 3000 / 300 tokens: 127 / 65 / 41 with an output per lane (weights two bytes at a time), u taken apart for
+// 128 outputs and the library's functions, 83 / 45 / 24 here (275 on the float32 matrix cores at 6376); 4 blocks, 2000 / 168: 43 / 39 ->
+// 26 / 23.  Largest error of a and g against 64 bits there 5.4e-7 and 8.1e-6, means 1.8e-8 and 2.8e-8, as before.
+// VEC: blocks a multiple of 4 wide and aligned; else elements one by one.
+constexpr int kST = 64;       // tokens per workgroup
+constexpr int kSO = 256;      // outputs
 constexpr int kSK = 64;       // K chunk in LDS
 constexpr int kSP = kSK + 8;
 constexpr float kBfMax = 0x1.fep+127f;
 
-__global__ void __launch_bounds__(256, 2) sm_rglru_gates_split_kernel(
+template <bool VEC>
+__global__ void __launch_bounds__(256, VEC ? 2 : 1) sm_rglru_gates_split_kernel(
     float* __restrict__ a_out, float* __restrict__ g_out, const float* __restrict__ u, const bf16* __restrict__ ra_t,
     const bf16* __restrict__ ra_b, const bf16* __restrict__ ri_t, const bf16* __restrict__ ri_b,
     const bf16* __restrict__ lam, int tokens, int nb, int bw, float scale) {
-  __shared__ __attribute__((aligned(16))) bf16 us[3][kST][kSP];
+  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  __shared__ __attribute__((aligned(16))) bf16 us[2][3][kST][kSP];
   const int t0 = blockIdx.x * kST, b = blockIdx.y, C = nb * bw;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, n = lane & 31, half = lane >> 5;
-  const int o = blockIdx.z * 128 + wave * 32 + n;            // this lane's output channel inside block b
-  const int oc = min(o, bw - 1);
-  const bf16* ra = ra_t + (size_t)b * bw * bw + oc;
-  const bf16* ri = ri_t + (size_t)b * bw * bw + oc;
-  f32x16 cr[4], ci[4];
-#pragma unroll
-  for (int m = 0; m < 4; ++m)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) cr[m][i] = ci[m][i] = 0.f;
-  bf16x8 wr[2], wi[2];
-  auto load_w = [&](int k0, int buf) {                       // rows k0 + 8 half .. of this lane's output column
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const size_t at = (size_t)min(k0 + 8 * half + j, bw - 1) * bw;
-      wr[buf][j] = ra[at];
-      wi[buf][j] = ri[at];
+  const int wm = wave >> 1, wn = wave & 1;
+  const int o = blockIdx.z * kSO + wn * 128 + 4 * n;         // this lane's four output channels inside block b
+  const size_t blk = (size_t)b * bw * bw;
+  // rows of u, a and g through buffers of this workgroup's tokens: nothing is read or written past the last one
+  const size_t row0 = (size_t)t0 * C;
+  const int bytes = min(kST, tokens - t0) * C * 4;
+  const auto ru = __builtin_amdgcn_make_buffer_rsrc((void*)(u + row0), (short)0, bytes, 0x00020000);
+  const auto rsa = __builtin_amdgcn_make_buffer_rsrc((void*)(a_out + row0), (short)0, bytes, 0x00020000);
+  const auto rsg = __builtin_amdgcn_make_buffer_rsrc((void*)(g_out + row0), (short)0, bytes, 0x00020000);
+  auto row4 = [&](int r, int k) -> f32x4 {                   // channels k .. k + 3 of the block in the workgroup's row r
+    if constexpr (VEC) {
+      return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(ru, (r * C + b * bw + k) * 4, 0, 0));
+    } else {
+      const float* row = u + (size_t)min(t0 + r, tokens - 1) * C + b * bw;
+      return f32x4{row[min(k, bw - 1)], row[min(k + 1, bw - 1)], row[min(k + 2, bw - 1)], row[min(k + 3, bw - 1)]};
     }
   };
-  load_w(0, 0);
-  const float* ub = u + (size_t)b * bw;
-  for (int kc = 0; kc < bw; kc += kSK) {
-    __syncthreads();
-#pragma unroll 8
-    for (int i = tid; i < kST * kSK; i += 256) {             // a wave per row of the chunk
-      const int r = i / kSK, k = i - r * kSK;
-      const bool ok = t0 + r < tokens && kc + k < bw;
-      float x = ub[(size_t)min(t0 + r, tokens - 1) * C + min(kc + k, bw - 1)];
-      x = ok ? x : 0.f;
-      // (a finite x above the largest bf16 keeps a finite first piece; an infinite or NaN one has no others)
-      const bool fin = __builtin_isfinite(x);
-      const bf16 h = f2bf(fin ? fminf(fmaxf(x, -kBfMax), kBfMax) : x);
-      const float xm = fin ? x - bf2f(h) : 0.f;
-      const bf16 m = f2bf(xm);
-      us[0][r][k] = h;
-      us[1][r][k] = m;
-      us[2][r][k] = f2bf(xm - bf2f(m));
+
+  // a chunk's values of this thread: four of row (tid >> 4) + 16 q each, zero past the block
+  f32x4 x[4];
+  auto load_u = [&](int kc) {
+    const int k = kc + 4 * (tid & 15);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) x[q] = row4((tid >> 4) + 16 * q, k);
+    if (kc + kSK > bw) {                                     // uniform
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[q][e] = k + e < bw ? x[q][e] : 0.f;
     }
-    __syncthreads();
+  };
+  auto store_u = [&](int buf) {
+    uint32_t top = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float v = x[q][e];                             // (the cast of a vector's element takes its first)
+        top = max(top, __builtin_bit_cast(uint32_t, v) & 0x7fffffffu);
+      }
+    const bool plain = top <= __builtin_bit_cast(uint32_t, kBfMax);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      bf16x4 h, m, l;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float v = x[q][e];
+        h[e] = f2bf(v);
+        const float vm = v - bf2f(h[e]);
+        m[e] = f2bf(vm);
+        l[e] = f2bf(vm - bf2f(m[e]));
+      }
+      if (!plain) {      // (a finite value above the largest bf16 keeps a finite first piece; an infinite or NaN one has no others)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float v = x[q][e];
+          const bool fin = __builtin_isfinite(v);
+          h[e] = f2bf(fin ? fminf(fmaxf(v, -kBfMax), kBfMax) : v);
+          const float vm = fin ? v - bf2f(h[e]) : 0.f;
+          m[e] = f2bf(vm);
+          l[e] = f2bf(vm - bf2f(m[e]));
+        }
+      }
+      const int r = (tid >> 4) + 16 * q, k = 4 * (tid & 15);
+      *reinterpret_cast<bf16x4*>(&us[buf][0][r][k]) = h;
+      *reinterpret_cast<bf16x4*>(&us[buf][1][r][k]) = m;
+      *reinterpret_cast<bf16x4*>(&us[buf][2][r][k]) = l;
+    }
+  };
+  // rows k0 + 8 half .. of this lane's columns of a gate matrix (zero past the block), and the four fragments they make
+  const auto rr = __builtin_amdgcn_make_buffer_rsrc((void*)(ra_t + blk), (short)0, bw * bw * 2, 0x00020000);
+  const auto ri = __builtin_amdgcn_make_buffer_rsrc((void*)(ri_t + blk), (short)0, bw * bw * 2, 0x00020000);
+  const int lane_w = (8 * half * bw + o) * 2;
+  auto load_w = [&](u32x2 (&w)[8], const __amdgpu_buffer_rsrc_t& g, [[maybe_unused]] const bf16* m, int k0) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      if constexpr (VEC) {
+        w[q] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(g, lane_w + (k0 + q) * bw * 2, 0, 0));
+      } else {
+        const int k = k0 + 8 * half + q;
+        const bf16* row = m + blk + (size_t)min(k, bw - 1) * bw;
+        bf16x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = k < bw ? row[min(o + e, bw - 1)] : (bf16)0.f;
+        w[q] = __builtin_bit_cast(u32x2, v);
+      }
+    }
+  };
+  auto fragments = [&](bf16x8 (&f)[4], const u32x2 (&w)[8]) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      u32x4 v;
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        v[q] = __builtin_amdgcn_perm(w[2 * q + 1][j >> 1], w[2 * q][j >> 1], j & 1 ? 0x07060302u : 0x05040100u);
+      f[j] = __builtin_bit_cast(bf16x8, v);
+    }
+  };
+
+  f32x16 cr[4], ci[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) cr[j][i] = ci[j][i] = 0.f;
+  u32x2 wr[8], wi[8];
+  load_u(0);
+  load_w(wr, rr, ra_t, 0);
+  load_w(wi, ri, ri_t, 0);
+  store_u(0);
+  int buf = 0;
+  for (int kc = 0; kc < bw; kc += kSK, buf ^= 1) {
+    __syncthreads();                                         // chunk kc is there; the other buffer's readers are through
+    const bool more = kc + kSK < bw;                         // uniform
+    if (more) load_u(kc + kSK);
 #pragma unroll
     for (int s = 0; s < kSK / 16; ++s) {
-      if (kc + 16 * s < bw) {                                // uniform
-        load_w(kc + 16 * (s + 1), (s + 1) & 1);              // (past the last step: the last row, not used)
-        bf16x8 br = wr[s & 1], bi = wi[s & 1];
-        if (kc + 16 * (s + 1) > bw) {                        // uniform: rows past the block
+      const int k0 = kc + 16 * s;
+      if (k0 < bw) {                                         // uniform
+        bf16x8 a[3], f[4];
 #pragma unroll
-          for (int j = 0; j < 8; ++j)
-            if (kc + 16 * s + 8 * half + j >= bw) br[j] = bi[j] = (bf16)0.f;
-        }
+        for (int p = 0; p < 3; ++p) a[p] = *reinterpret_cast<const bf16x8*>(&us[buf][p][32 * wm + n][16 * s + 8 * half]);
+        fragments(f, wr);
+        load_w(wr, rr, ra_t, k0 + 16);                       // (past the last step: zeros, not used)
+        __builtin_amdgcn_sched_barrier(0);                   // (hipcc moves these loads behind the products)
 #pragma unroll
-        for (int m = 0; m < 4; ++m)
+        for (int j = 0; j < 4; ++j)
 #pragma unroll
-          for (int p = 2; p >= 0; --p) {                     // the small pieces first
-            const bf16x8 a = *reinterpret_cast<const bf16x8*>(&us[p][32 * m + n][16 * s + 8 * half]);
-            cr[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, br, cr[m], 0, 0, 0);
-            ci[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, bi, ci[m], 0, 0, 0);
-          }
+          for (int p = 2; p >= 0; --p)                       // the small pieces first
+            cr[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[p], f[j], cr[j], 0, 0, 0);
+        fragments(f, wi);
+        load_w(wi, ri, ri_t, k0 + 16);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int p = 2; p >= 0; --p) ci[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[p], f[j], ci[j], 0, 0, 0);
       }
     }
+    if (more) store_u(buf ^ 1);
   }
   if (o >= bw) return;
-  const int ch = b * bw + o;
-  const float rb = bf2f(ra_b[ch]), ib = bf2f(ri_b[ch]), sp = softplus_f(bf2f(lam[ch]));
+  f32x4 ux[4];
 #pragma unroll
-  for (int m = 0; m < 4; ++m) {
-    float x[16];
+  for (int i = 0; i < 4; ++i) ux[i] = row4(32 * wm + 4 * half + i, o);
+  float rb[4], ib[4], sp[4];
 #pragma unroll
-    for (int i = 0; i < 16; ++i)
-      x[i] = u[(size_t)min(t0 + 32 * m + 8 * (i >> 2) + 4 * half + (i & 3), tokens - 1) * C + ch];
+  for (int j = 0; j < 4; ++j) {
+    const int ch = b * bw + min(o + j, bw - 1);
+    rb[j] = bf2f(ra_b[ch]), ib[j] = bf2f(ri_b[ch]), sp[j] = softplus_f(bf2f(lam[ch]));
+  }
+#pragma unroll 1
+  for (int i0 = 0; i0 < 16; i0 += 4) {                       // accumulator register i of this lane: row 8 (i / 4) + 4 half + i % 4
+    const int r = 32 * wm + 2 * i0 + 4 * half;
+    f32x4 un[4];                                             // the next four rows' u
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int t = t0 + 32 * m + 8 * (i >> 2) + 4 * half + (i & 3);    // accumulator register i of this lane
-      const float av = expf(-scale * sigmoid_f(cr[m][i] + rb) * sp);
-      const float gv = sqrtf(1.0f - av * av) * sigmoid_f(ci[m][i] + ib) * x[i];
-      if (t < tokens) {
-        a_out[(size_t)t * C + ch] = av;
-        g_out[(size_t)t * C + ch] = gv;
+    for (int i = 0; i < 4; ++i) un[i] = row4(min(r + 8, kST - 4) + i, o);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      f32x4 av, gv;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        av[j] = expf(-scale * sigmoid_near(cr[j][i] + rb[j]) * sp[j]);
+        gv[j] = sqrt_near(1.0f - av[j] * av[j]) * sigmoid_near(ci[j][i] + ib[j]) * ux[i][j];
       }
+      if constexpr (VEC) {
+        const int at = ((r + i) * C + b * bw + o) * 4;
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, av), rsa, at, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, gv), rsg, at, 0, 0);
+      } else if (t0 + r + i < tokens) {
+        const size_t at = (size_t)(t0 + r + i) * C + b * bw + o;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (o + j < bw) a_out[at + j] = av[j], g_out[at + j] = gv[j];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      ux[j] = un[j];
+#pragma unroll
+      for (int i = 0; i < 12; ++i) cr[j][i] = cr[j][i + 4], ci[j][i] = ci[j][i + 4];
     }
   }
 }
@@ -1308,9 +1438,15 @@ void sm_rglru_gates(uintptr_t a, uintptr_t g, uintptr_t u, uintptr_t ra_t, uintp
     return;
   }
   if (!f32) {
-    hipLaunchKernelGGL(sm_rglru_gates_split_kernel, dim3((tokens + kST - 1) / kST, nb, (bw + 127) / 128), dim3(256), 0,
-                       (hipStream_t)stream, (float*)a, (float*)g, (const float*)u, (const bf16*)ra_t, (const bf16*)ra_b,
-                       (const bf16*)ri_t, (const bf16*)ri_b, (const bf16*)lam, tokens, nb, bw, scale);
+    const dim3 grid((tokens + kST - 1) / kST, nb, (bw + kSO - 1) / kSO);
+    const bool vec = bw % 4 == 0 && (u | a | g) % 16 == 0 && (ra_t | ri_t) % 8 == 0;
+#define SM_GATES(VEC_)                                                                                                     \
+  hipLaunchKernelGGL(sm_rglru_gates_split_kernel<VEC_>, grid, dim3(256), 0, (hipStream_t)stream, (float*)a, (float*)g,       \
+                     (const float*)u, (const bf16*)ra_t, (const bf16*)ra_b, (const bf16*)ri_t, (const bf16*)ri_b,            \
+                     (const bf16*)lam, tokens, nb, bw, scale)
+    if (vec) SM_GATES(true);
+    else SM_GATES(false);
+#undef SM_GATES
     DLLM_HIP_CHECK(hipGetLastError());
     return;
   }
