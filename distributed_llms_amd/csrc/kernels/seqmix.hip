@@ -869,6 +869,21 @@ __global__ void __launch_bounds__(256) sm_causal_conv_kernel(void* __restrict__ 
     for (int j = 0; j < V; ++j) acc[j] = 0.f, ib[j] = 0.f;
     if (bias) ldv<V>(bias + c, acc);
     if (in_bias) ldv<V>(in_bias + c, ib);
+    if (taps <= kConvTaps) {                         // (uniform) every load at once, off a place that is always there
+      float xs[kConvTaps][V], ws[kConvTaps][V];
+#pragma unroll
+      for (int j = 0; j < kConvTaps; ++j) {
+        const int jj = min(j, taps - 1), d = taps - 1 - jj;
+        ldv<V>(conv_row(u, stride, st, t, tl, d, taps, C) + c, xs[j]);
+        ldv<V>(w + (size_t)jj * C + c, ws[j]);
+      }
+#pragma unroll
+      for (int j = 0; j < kConvTaps; ++j)
+        if (j < taps && taps - 1 - j <= pos) {       // (uniform)
+#pragma unroll
+          for (int e = 0; e < V; ++e) acc[e] += ws[j][e] * (xs[j][e] + ib[e]);
+        }
+    } else
     for (int j = 0; j < taps; ++j) {
       if (!conv_input_v<T, V>(u, stride, st, t, tl, pos, taps - 1 - j, taps, c, C, xv)) continue;
       ldv<V>(w + (size_t)j * C + c, wv);
@@ -880,6 +895,75 @@ __global__ void __launch_bounds__(256) sm_causal_conv_kernel(void* __restrict__ 
       for (int e = 0; e < V; ++e) acc[e] = acc[e] / (1.0f + expf(-acc[e]));
     }
     stv<V>(y + c, acc);
+  }
+}
+
+// The same over many tokens, up to kConvTaps taps: a thread takes 8 channels of kConvRun tokens, whose rows overlap (7 rows and one
+// read of the weights for 4 tokens, 16 and 4 by themselves), all of them in one round trip where the run lies inside a sequence.
+// 6376 tokens x 2560 to float32: 37 us a token per workgroup and its rows one by one behind branches, 28 here.
+constexpr int kConvRun = 4;
+
+template <typename T, typename OT>
+__global__ void __launch_bounds__(256) sm_causal_conv_run_kernel(
+    void* __restrict__ y_, const void* __restrict__ u_, long stride, const void* __restrict__ w_, const void* __restrict__ bias_,
+    const void* __restrict__ in_bias_, const void* __restrict__ state_, const int32_t* __restrict__ cu,
+    const int32_t* __restrict__ positions, const int32_t* __restrict__ tok_seq, const int32_t* __restrict__ slots, int C, int taps,
+    int act, int tokens) {
+  const long id = (long)blockIdx.x * 256 + threadIdx.x;
+  const int t0 = (int)(id / (C / 8)) * kConvRun, c = (int)(id % (C / 8)) * 8;
+  if (t0 >= tokens) return;
+  const T* u = (const T*)u_ + c;
+  const T* w = (const T*)w_ + c;
+  const int t1 = min(t0 + kConvRun, tokens) - 1, b0 = tok_seq[t0], b1 = tok_seq[t1], tl0 = t0 - cu[b0];
+  float bias[8], ib[8], wv[kConvTaps][8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) bias[e] = ib[e] = 0.f;
+  if (bias_) ldv<8>((const T*)bias_ + c, bias);
+  if (in_bias_) ldv<8>((const T*)in_bias_ + c, ib);
+#pragma unroll
+  for (int j = 0; j < kConvTaps; ++j) ldv<8>(w + (size_t)min(j, taps - 1) * C, wv[j]);
+  auto finish = [&](int t, float (&acc)[8]) {
+    if (act == 1) {                                  // silu, in float32 with the exact exponential
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[e] = acc[e] / (1.0f + expf(-acc[e]));
+    }
+    stv<8>((OT*)y_ + (size_t)t * C + c, acc);
+  };
+  if (b0 == b1 && tl0 >= taps - 1) {
+    float x[kConvRun + kConvTaps - 1][8];            // row i: token t0 - (taps - 1) + i
+#pragma unroll
+    for (int i = 0; i < kConvRun + kConvTaps - 1; ++i) ldv<8>(u + (size_t)min(t0 - (taps - 1) + i, t1) * stride, x[i]);
+#pragma unroll
+    for (int q = 0; q < kConvRun; ++q) {
+      if (t0 + q > t1) break;
+      float acc[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[e] = bias[e];
+#pragma unroll
+      for (int j = 0; j < kConvTaps; ++j)
+        if (j < taps) {                              // (uniform)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) acc[e] += wv[j][e] * (x[q + j][e] + ib[e]);
+        }
+      finish(t0 + q, acc);
+    }
+    return;
+  }
+  for (int t = t0; t <= t1; ++t) {
+    const int b = tok_seq[t], tl = t - cu[b], pos = positions[t];
+    const T* st = (const T*)state_ + (size_t)slots[b] * (taps - 1) * C + c;
+    float acc[8], xs[kConvTaps][8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] = bias[e];
+#pragma unroll
+    for (int j = 0; j < kConvTaps; ++j) ldv<8>(conv_row(u, stride, st, t, tl, taps - 1 - min(j, taps - 1), taps, C), xs[j]);
+#pragma unroll
+    for (int j = 0; j < kConvTaps; ++j)
+      if (j < taps && taps - 1 - j <= pos) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] += wv[j][e] * (xs[j][e] + ib[e]);
+      }
+    finish(t, acc);
   }
 }
 
@@ -942,9 +1026,21 @@ void sm_causal_conv(uintptr_t y, uintptr_t u, long stride, uintptr_t w, uintptr_
   hipLaunchKernelGGL(HIP_KERNEL_NAME(sm_causal_conv_kernel<T, OT, V>), grid, dim3(256), 0, s, (void*)y, (const void*)u, \
                      stride, (const void*)w, (const void*)bias, (const void*)in_bias, (const void*)state,     \
                      (const int32_t*)cu, (const int32_t*)positions, (const int32_t*)tok_seq, (const int32_t*)slots, C, taps, act)
-  if (f32) { if (vec) SM_CONV(float, float, 8); else SM_CONV(float, float, 1); }
+#define SM_CONV_RUN(T, OT)                                                                                           \
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(sm_causal_conv_run_kernel<T, OT>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, \
+                     (void*)y, (const void*)u, stride, (const void*)w, (const void*)bias, (const void*)in_bias,              \
+                     (const void*)state, (const int32_t*)cu, (const int32_t*)positions, (const int32_t*)tok_seq,             \
+                     (const int32_t*)slots, C, taps, act, tokens)
+  // runs of tokens where these by themselves fill the chip (a workgroup on each CU)
+  const long threads = (long)((tokens + kConvRun - 1) / kConvRun) * (C / 8);
+  if (vec && taps <= kConvTaps && threads >= 256 * 256) {
+    if (f32) SM_CONV_RUN(float, float);
+    else if (out_f32) SM_CONV_RUN(bf16, float);
+    else SM_CONV_RUN(bf16, bf16);
+  } else if (f32) { if (vec) SM_CONV(float, float, 8); else SM_CONV(float, float, 1); }
   else if (out_f32) { if (vec) SM_CONV(bf16, float, 8); else SM_CONV(bf16, float, 1); }
   else { if (vec) SM_CONV(bf16, bf16, 8); else SM_CONV(bf16, bf16, 1); }
+#undef SM_CONV_RUN
 #undef SM_CONV
   DLLM_HIP_CHECK(hipGetLastError());
   if (taps > 1) launch_conv_state(state, u, stride, cu, positions, slots, seqs, C, taps, f32, vec, stream);
@@ -1979,11 +2075,15 @@ __global__ void __launch_bounds__(64) sm_attn_prep_kernel(
 
 // The same with even head sizes: a lane owns rotation pairs (channels 2e, 2e + 1), so the convolution
 // reads 2-element vectors, the rotation needs no exchange through LDS, and q / k leave as 2-element
-// stores.  Heads up to 512 wide (4 pairs per lane).
+// stores.  Heads up to 128 R wide, R <= 4.
+// A wave takes every 4 gridDim.y-th head of its token.  On prompts it was bound by round trips (a tap's rows behind a branch each)
+// and by the cosines and sines, the same in all heads: all rows of a head go out at once, and one wave's heads share the angles
+// where the tokens alone fill the chip.  us, 6376 / 21 tokens of the 2B and the small
+// layer list: 90 / 7.1 -> 65 / 4.8.
 constexpr int kPrepPairs = 4;
-constexpr int kTailTaps = 4;
+constexpr int kPrepGroups = 2048;     // workgroups that are resident together: eight on each CU
 
-template <typename T>
+template <typename T, int R, bool MANY>
 __global__ void __launch_bounds__(256) sm_attn_prep_pair_kernel(
     void* __restrict__ q_out_, const void* __restrict__ qkv_, const void* __restrict__ conv_w_,
     const void* state_, const void* __restrict__ q_norm_, const void* __restrict__ k_norm_,
@@ -1991,95 +2091,137 @@ __global__ void __launch_bounds__(256) sm_attn_prep_pair_kernel(
     void* __restrict__ v_cache_, const int32_t* __restrict__ slot_mapping, const int32_t* __restrict__ cu,
     const int32_t* __restrict__ positions, const int32_t* __restrict__ tok_seq, const int32_t* __restrict__ slots,
     int H, int G, int D, int Dv, int taps, int bs, void* tail_) {
-  const int t = blockIdx.x, head = blockIdx.y * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;   // a wave per head
-  if (head >= H + 2 * G) return;
+  const int t = blockIdx.x, lane = threadIdx.x & 63;
   const int C = H * D + G * (D + Dv);
   const int b = tok_seq[t];
   const int tl = t - cu[b], pos = positions[t];
   const T* qkv = (const T*)qkv_;
   const T* w = (const T*)conv_w_;
   const T* st = (const T*)state_ + (size_t)slots[b] * (taps - 1) * C;
-  int c0, n, kind;                                   // kind 0 q, 1 k, 2 v
-  if (head < H) c0 = head * D, n = D, kind = 0;
-  else if (head < H + G) c0 = H * D + (head - H) * D, n = D, kind = 1;
-  else c0 = H * D + G * D + (head - H - G) * Dv, n = Dv, kind = 2;
-  float x[kPrepPairs][2];
-  float ss = 0.f;
+  typedef T pair __attribute__((ext_vector_type(2)));
+  pair xn[R][kConvTaps], wn[R][kConvTaps];             // a head's rows and weights, up to kConvTaps taps
+  auto channels = [&](int head, int& c0, int& n, int& kind) {   // kind 0 q, 1 k, 2 v
+    if (head < H) c0 = head * D, n = D, kind = 0;
+    else if (head < H + G) c0 = H * D + (head - H) * D, n = D, kind = 1;
+    else c0 = H * D + G * D + (head - H - G) * Dv, n = Dv, kind = 2;
+  };
+  auto load = [&](int head) {                          // every load at once, off a place that is always there
+    int c0, n, kind;
+    channels(head, c0, n, kind);
 #pragma unroll
-  for (int r = 0; r < kPrepPairs; ++r) {
-    const int e = 2 * (lane + 64 * r);
-    x[r][0] = x[r][1] = 0.f;
-    if (e < n) {
-      const int c = c0 + e;
-      if (tail_) {                                   // one token per sequence, taps <= kTailTaps: the tail moves up here
-        T* sn = (T*)tail_ + (size_t)slots[b] * (taps - 1) * C + c;
-        float xv[kTailTaps][2], wv[kTailTaps][2];
+    for (int r = 0; r < R; ++r) {
+      const int c = c0 + min(2 * (lane + 64 * r), n - 2);
 #pragma unroll
-        for (int j = 0; j < kTailTaps; ++j) {
-          const int jj = min(j, taps - 1);
-          ldv<2>(w + (size_t)jj * C + c, wv[j]);
-          ldv<2>(jj == taps - 1 ? qkv + (size_t)t * C + c : (const T*)sn + (size_t)jj * C, xv[j]);
-        }
+      for (int j = 0; j < kConvTaps; ++j) {
+        const int jj = min(j, taps - 1);
+        wn[r][j] = *reinterpret_cast<const pair*>(w + (size_t)jj * C + c);
+        xn[r][j] = *reinterpret_cast<const pair*>(conv_row(qkv, (long)C, st, t, tl, taps - 1 - jj, taps, C) + c);
+      }
+    }
+  };
+  const bool few = taps <= kConvTaps;                  // uniform
+  int head = blockIdx.y * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (head >= H + 2 * G) return;
+  if (few) load(head);
+  float cs[R], sn[R];
+  bool angles = false;
+  for (; head < H + 2 * G; head += 4 * gridDim.y) {    // a wave per head
+    int c0, n, kind;
+    channels(head, c0, n, kind);
+    float x[R][2];
+    float ss = 0.f;
+    if (few) {
+      float xv[R][kConvTaps][2], wv[R][kConvTaps][2];
 #pragma unroll
-        for (int j = 0; j < kTailTaps; ++j) {
-          if (j < taps) {
-            if (taps - 1 - j > pos) xv[j][0] = xv[j][1] = 0.f;
-            x[r][0] += wv[j][0] * xv[j][0];
-            x[r][1] += wv[j][1] * xv[j][1];
-            if (j > 0) stv<2>(sn + (size_t)(j - 1) * C, xv[j]);
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int j = 0; j < kConvTaps; ++j)
+#pragma unroll
+          for (int e = 0; e < 2; ++e) xv[r][j][e] = (float)xn[r][j][e], wv[r][j][e] = (float)wn[r][j][e];
+      if constexpr (MANY) load(min(head + 4 * (int)gridDim.y, H + 2 * G - 1));   // the next head's under this one
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int e = 2 * (lane + 64 * r);
+        x[r][0] = x[r][1] = 0.f;
+        if (e < n) {
+#pragma unroll
+          for (int j = 0; j < kConvTaps; ++j) {
+            if (j < taps) {
+              if (taps - 1 - j > pos) xv[r][j][0] = xv[r][j][1] = 0.f;
+              else {
+                x[r][0] = fmaf(wv[r][j][0], xv[r][j][0], x[r][0]);
+                x[r][1] = fmaf(wv[r][j][1], xv[r][j][1], x[r][1]);
+              }
+              // one token per sequence: the tail moves up here
+              if (tail_ && j > 0) stv<2>((T*)tail_ + ((size_t)slots[b] * (taps - 1) + j - 1) * C + c0 + e, xv[r][j]);
+            }
           }
+          ss += fmaf(x[r][0], x[r][0], x[r][1] * x[r][1]);
         }
-      } else
-      for (int j = 0; j < taps; ++j) {
-        const int d = taps - 1 - j;
-        if (d > pos) continue;
-        float xv[2], wv[2];
-        if (d <= tl) ldv<2>(qkv + (size_t)(t - d) * C + c, xv);
-        else ldv<2>(st + (size_t)(tl - d + taps - 1) * C + c, xv);
-        ldv<2>(w + (size_t)j * C + c, wv);
-        x[r][0] += wv[0] * xv[0];
-        x[r][1] += wv[1] * xv[1];
       }
-      ss += x[r][0] * x[r][0] + x[r][1] * x[r][1];
-    }
-  }
-  if (kind == 2) {
-    const int slot = slot_mapping[t];
-    const int blk = slot / bs, off = slot - blk * bs;
-    T* dst = (T*)v_cache_ + ((size_t)blk * G + (head - H - G)) * Dv * bs + off;
+    } else {
 #pragma unroll
-    for (int r = 0; r < kPrepPairs; ++r) {
-      const int e = 2 * (lane + 64 * r);
-      if (e < n) stf(dst + (size_t)e * bs, x[r][0]), stf(dst + (size_t)(e + 1) * bs, x[r][1]);
-    }
-    return;
-  }
-  T* dst;
-  if (kind == 0) dst = (T*)q_out_ + ((size_t)t * H + head) * D;
-  else {
-    const int slot = slot_mapping[t];
-    const int blk = slot / bs, off = slot - blk * bs;
-    dst = (T*)k_cache_ + (((size_t)blk * G + (head - H)) * bs + off) * D;
-  }
-  ss = wave_sum(ss);
-  const float inv = 1.0f / sqrtf(ss / (float)n + eps);
-  const T* nw = (const T*)(kind == 0 ? q_norm_ : k_norm_);
-  const float fpos = (float)pos;
-#pragma unroll
-  for (int r = 0; r < kPrepPairs; ++r) {
-    const int i = lane + 64 * r, e = 2 * i;
-    if (e < n) {
-      float g2[2], o[2];
-      ldv<2>(nw + e, g2);
-      float x0 = x[r][0] * inv * g2[0], x1 = x[r][1] * inv * g2[1];
-      if (i < nrot) {
-        const float ang = fpos * freqs[i];
-        const float cs = cosf(ang) * mag, sn = sinf(ang) * mag;
-        const float r0 = x0 * cs - x1 * sn, r1 = x1 * cs + x0 * sn;
-        x0 = r0, x1 = r1;
+      for (int r = 0; r < R; ++r) {
+        const int e = 2 * (lane + 64 * r);
+        x[r][0] = x[r][1] = 0.f;
+        if (e < n) {
+          for (int j = 0; j < taps; ++j) {
+            float xv[2], wv[2];
+            if (!conv_input_v<T, 2>(qkv, (long)C, st, t, tl, pos, taps - 1 - j, taps, c0 + e, C, xv)) continue;
+            ldv<2>(w + (size_t)j * C + c0 + e, wv);
+            x[r][0] = fmaf(wv[0], xv[0], x[r][0]);
+            x[r][1] = fmaf(wv[1], xv[1], x[r][1]);
+          }
+          ss += fmaf(x[r][0], x[r][0], x[r][1] * x[r][1]);
+        }
       }
-      o[0] = x0, o[1] = x1;
-      stv<2>(dst + e, o);
+    }
+    if (kind == 2) {
+      const int slot = slot_mapping[t];
+      const int blk = slot / bs, off = slot - blk * bs;
+      T* dst = (T*)v_cache_ + ((size_t)blk * G + (head - H - G)) * Dv * bs + off;
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int e = 2 * (lane + 64 * r);
+        if (e < n) stf(dst + (size_t)e * bs, x[r][0]), stf(dst + (size_t)(e + 1) * bs, x[r][1]);
+      }
+      continue;
+    }
+    T* dst;
+    if (kind == 0) dst = (T*)q_out_ + ((size_t)t * H + head) * D;
+    else {
+      const int slot = slot_mapping[t];
+      const int blk = slot / bs, off = slot - blk * bs;
+      dst = (T*)k_cache_ + (((size_t)blk * G + (head - H)) * bs + off) * D;
+    }
+    if (!angles) {                                     // (uniform)
+      angles = true;
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int i = lane + 64 * r;
+        if (i < nrot) {
+          const float ang = (float)pos * freqs[i];
+          cs[r] = cosf(ang) * mag, sn[r] = sinf(ang) * mag;
+        }
+      }
+    }
+    ss = wave_sum(ss);
+    const float inv = 1.0f / sqrtf(ss / (float)n + eps);
+    const T* nw = (const T*)(kind == 0 ? q_norm_ : k_norm_);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int i = lane + 64 * r, e = 2 * i;
+      if (e < n) {
+        float g2[2], o[2];
+        ldv<2>(nw + e, g2);
+        float x0 = x[r][0] * inv * g2[0], x1 = x[r][1] * inv * g2[1];
+        if (i < nrot) {
+          const float r0 = fmaf(x0, cs[r], -(x1 * sn[r])), r1 = fmaf(x1, cs[r], x0 * sn[r]);   // (alike in every form)
+          x0 = r0, x1 = r1;
+        }
+        o[0] = x0, o[1] = x1;
+        stv<2>(dst + e, o);
+      }
     }
   }
 }
@@ -2098,13 +2240,26 @@ void sm_attn_prep(uintptr_t q_out, uintptr_t qkv, uintptr_t conv_w, uintptr_t st
   const bool pairs = D % 2 == 0 && Dv % 2 == 0 && std::max(D, Dv) <= 128 * kPrepPairs;
   // one token per sequence: a channel of a sequence's tail is read and moved up by the one lane that convolves it, so the
   // tail needs no launch of its own (4.6 us)
-  const bool tail = pairs && max_q_len == 1 && taps > 1 && taps <= kTailTaps;
-  if (pairs)
-    SM_DISPATCH(f32, sm_attn_prep_pair_kernel, dim3(tokens, (H + 2 * G + 3) / 4), dim3(256), 0, stream, (void*)q_out,
-                (const void*)qkv, (const void*)conv_w, (const void*)state, (const void*)q_norm, (const void*)k_norm,
-                (const float*)freqs, nrot, mag, eps, (void*)k_cache, (void*)v_cache, (const int32_t*)slot_mapping,
-                (const int32_t*)cu, (const int32_t*)positions, (const int32_t*)tok_seq, (const int32_t*)slots, H, G, D,
-                Dv, taps, bs, tail ? (void*)state : nullptr);
+  const bool tail = pairs && max_q_len == 1 && taps > 1 && taps <= kConvTaps;
+  if (pairs) {
+    // workgroups per token: one per four heads while those fit the chip together, else fewer whose waves take several
+    const int most = (H + 2 * G + 3) / 4, gy = std::max(1, std::min(most, kPrepGroups / tokens));
+    const int r = std::max(D, Dv) <= 128 ? 1 : std::max(D, Dv) <= 256 ? 2 : kPrepPairs;
+#define SM_PREP(T_, R_) do { if (gy < most) SM_PREP_M(T_, R_, true); else SM_PREP_M(T_, R_, false); } while (0)
+#define SM_PREP_M(T_, R_, MANY_)                                                                                                    \
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(sm_attn_prep_pair_kernel<T_, R_, MANY_>), dim3(tokens, gy), dim3(256), 0, (hipStream_t)stream, \
+                     (void*)q_out, (const void*)qkv, (const void*)conv_w, (const void*)state, (const void*)q_norm,           \
+                     (const void*)k_norm, (const float*)freqs, nrot, mag, eps, (void*)k_cache, (void*)v_cache,               \
+                     (const int32_t*)slot_mapping, (const int32_t*)cu, (const int32_t*)positions, (const int32_t*)tok_seq,   \
+                     (const int32_t*)slots, H, G, D, Dv, taps, bs, tail ? (void*)state : nullptr)
+#define SM_PREP_R(T_) do { if (r == 1) SM_PREP(T_, 1); else if (r == 2) SM_PREP(T_, 2); else SM_PREP(T_, kPrepPairs); } while (0)
+    if (f32) SM_PREP_R(float);
+    else SM_PREP_R(bf16);
+#undef SM_PREP_R
+#undef SM_PREP
+#undef SM_PREP_M
+    DLLM_HIP_CHECK(hipGetLastError());
+  }
   else
   SM_DISPATCH(f32, sm_attn_prep_kernel, dim3(tokens, H + 2 * G), dim3(64), lds, stream, (void*)q_out, (const void*)qkv,
               (const void*)conv_w, (const void*)state, (const void*)q_norm, (const void*)k_norm, (const float*)freqs,

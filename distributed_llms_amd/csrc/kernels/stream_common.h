@@ -94,6 +94,13 @@ __device__ __forceinline__ float conv_input(const T* __restrict__ u, long stride
   return ldf(st + (size_t)(tl - d + taps - 1) * C + c);
 }
 
+// That row (of the batch or of the tail) by itself: it is there also where the position lies before the sequence's start.
+template <typename T>
+__device__ __forceinline__ const T* conv_row(const T* u, long stride, const T* st, int t, int tl, int d, int taps, int C) {
+  return d <= tl ? u + (size_t)(t - d) * stride : st + (size_t)(tl - d + taps - 1) * C;
+}
+constexpr int kConvTaps = 4;   // convolutions of up to so many taps load all of their rows at once
+
 template <typename T, int V>
 __device__ __forceinline__ bool conv_input_v(const T* __restrict__ u, long stride, const T* __restrict__ st, int t,
                                              int tl, int pos, int d, int taps, int c, int C, float (&o)[V]) {

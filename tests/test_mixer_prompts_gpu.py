@@ -1,0 +1,75 @@
+"""The input stages of the recurrent and the attention mixers over many tokens, where a thread takes a run of tokens and a wave
+several heads: the bits of the same stages token by token (each chunk of a batch by itself, too short for either)."""
+import pytest
+import torch
+
+from distributed_llms_amd.ops import seqmix as sm
+
+pytestmark = pytest.mark.gpu
+
+
+def _sb(chunks, slots, device):
+    """chunks: (position of the first token, tokens) per sequence."""
+    cu = [0]
+    for _, n in chunks:
+        cu.append(cu[-1] + n)
+    t = lambda v: torch.tensor(v, dtype=torch.int32, device=device)
+    return sm.SeqBatch(t(cu), t([p + i for p, n in chunks for i in range(n)]), t([b for b, (_, n) in enumerate(chunks) for _ in range(n)]),
+                       t(slots), len(chunks), cu[-1], max(n for _, n in chunks))
+
+
+def _chunks(total, g):
+    """Ragged: one token, fewer than the taps, sequences that go on, runs cut by their ends."""
+    out = [(0, 1), (7, 1), (0, 2), (1, 3), (0, 5), (300, 6)]
+    while total > sum(n for _, n in out):
+        n = min(int(torch.randint(9, 700, (1,), generator=g)), total - sum(k for _, k in out))
+        out.append((int(torch.randint(0, 2, (1,), generator=g)) * 50, n))
+    return out
+
+
+@pytest.mark.parametrize("dtype,out", [(torch.bfloat16, torch.float32), (torch.bfloat16, torch.bfloat16), (torch.float32, torch.float32)])
+@pytest.mark.parametrize("c,taps,act", [(2560, 4, None), (264, 3, "silu"), (2560, 1, None), (1024, 2, None), (1024, 5, None)])
+def test_causal_conv_of_runs_bit_exact(cuda, dtype, out, c, taps, act):
+    g = torch.Generator().manual_seed(c + taps)
+    tokens = 4 * 65536 // (c // 8) + 6                              # just past the rule, a last run of fewer tokens
+    chunks = _chunks(tokens, g)
+    r = lambda *s: torch.randn(*s, generator=g).to(dtype).to(cuda)
+    u, w, b, ib = r(tokens, 2 * c)[:, c:], r(taps, c), r(c), r(c)
+    state = r(len(chunks) + 2, taps - 1, c)
+    slots = torch.randperm(len(chunks) + 2, generator=g)[:len(chunks)].tolist()
+    st, st1 = state.clone(), state.clone()
+    conv = lambda rows, to, sb: sm.causal_conv(rows, w, b, to, sb, out_dtype=out, in_bias=ib, act=act)
+    y = conv(u, st, _sb(chunks, slots, cuda))
+    at = 0
+    for (p, n), s in zip(chunks, slots):
+        assert torch.equal(y[at:at + n], conv(u[at:at + n], st1, _sb([(p, n)], [s], cuda))), (p, n)
+        at += n
+    assert torch.equal(st, st1)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("heads,kvh,dim,vdim,taps,nrot", [(20, 2, 128, 128, 4, 32), (3, 1, 64, 96, 3, 32), (9, 1, 192, 320, 2, 10),
+                                                          (6, 1, 30, 16, 1, 0), (5, 2, 64, 64, 5, 8)])
+def test_attention_input_of_many_heads_per_wave_bit_exact(cuda, dtype, heads, kvh, dim, vdim, taps, nrot):
+    g = torch.Generator().manual_seed(heads + dim)
+    tokens, bs, c = 2051, 16, heads * dim + kvh * (dim + vdim)      # fewer workgroups per token than heads / 4
+    chunks = _chunks(tokens, g)
+    r = lambda *s: torch.randn(*s, generator=g).to(dtype).to(cuda)
+    qkv, cw, qn, kn, conv = r(tokens, c), r(taps, c), r(dim), r(dim), r(len(chunks) + 2, taps - 1, c)
+    freqs = torch.rand(nrot, generator=g).to(cuda)
+    slots = torch.randperm(len(chunks) + 2, generator=g)[:len(chunks)].tolist()
+    blocks = -(-tokens // bs)
+    where = torch.randperm(blocks * bs, generator=g)[:tokens].int().to(cuda)
+    pool = lambda: (torch.zeros(blocks, kvh, bs, dim, dtype=dtype, device=cuda), torch.zeros(blocks, kvh, vdim, bs, dtype=dtype, device=cuda),
+                    conv.clone())
+    prep = lambda rows, to, sl, sb: sm.attn_prep(rows, cw, to[2], qn, kn, freqs, 1.1, 1e-6, to[0], to[1], sl, sb, heads, kvh, dim, vdim)
+    a, b = pool(), pool()
+    q = prep(qkv, a, where, _sb(chunks, slots, cuda))
+    at = 0
+    for (p, n), s in zip(chunks, slots):
+        for k in range(0, n, 150):                                  # portions short enough for a wave per head
+            m = min(150, n - k)
+            part = prep(qkv[at + k:at + k + m], b, where[at + k:at + k + m].contiguous(), _sb([(p + k, m)], [s], cuda))
+            assert torch.equal(q[at + k:at + k + m], part), (p, n, k)
+        at += n
+    assert all(torch.equal(x, y) for x, y in zip(a, b))
