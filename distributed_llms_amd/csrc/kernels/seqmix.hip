@@ -1724,8 +1724,11 @@ void sm_rglru_scan(uintptr_t out, uintptr_t a, uintptr_t g, uintptr_t y_raw, lon
 // the last of them -- nobody waits -- writes the new tail.  The count belongs to the slot whose tail it guards, so launches
 // on other slots, on whatever stream or in whatever graph, never meet in it, and it wraps to zero by itself at the last
 // arrival (rows that share the scratch slot leave a whole number of turns).
-// 4 blocks of 256, 4 taps, bf16: one sequence 6.3 us, for 30 in four launches; 10 blocks: 16 sequences 9.1 us (42 before),
-// 64 sequences 20 us.
+// What is then left is a chain in one wave (us of 4.7 behind the launch: 1.1 to send all loads out, 0.3 convolution, 1.5 products,
+// 0.5 sums, 0.7 close): a whole round of rows is multiplied without a branch or select per row (1.5 -> 0.8), and the softplus and
+// the gelu(y), which ask for no gate, are made under the weights' round trip (close 0.7 -> 0.4).
+// 4 blocks of 256, 4 taps, bf16, in a graph: one sequence 6.1 -> 5.5 us (30 in four launches); 10 blocks: 16 sequences 9.6 -> 8.3
+// (42), 64 sequences 19.4 -> 18.
 constexpr int kRows = 8;       // gate matrix rows in flight per thread
 constexpr int kStepTaps = 8;   // at most
 constexpr int kStepOut = 64;   // outputs per workgroup
@@ -1822,6 +1825,12 @@ __global__ void __launch_bounds__(256) sm_rglru_step_kernel(
   if (tid < GT_ && s0 + tid < seqs)
     before = atomicInc(arrived + ((size_t)(tid == 0 ? slot[0] : slot[GT_ - 1]) * nb + b) * kCountStride, nz - 1);
 
+  // what the state's close takes besides the gates, under the weights' round trip (pinned: hipcc sinks it to its use)
+  float sp = 0.f, gy = 0.f;
+  if (fk < GT_) {                                     // uniform
+    sp = softplus_f((float)lam), gy = gelu_tanh_f((float)y_in + (float)y_b);
+    asm volatile("" : "+v"(sp), "+v"(gy));
+  }
   float ar[GT_][8], ai[GT_][8];
 #pragma unroll
   for (int k = 0; k < GT_; ++k)
@@ -1829,6 +1838,22 @@ __global__ void __launch_bounds__(256) sm_rglru_step_kernel(
     for (int j = 0; j < 8; ++j) ar[k][j] = 0.f, ai[k][j] = 0.f;
   for (int i0 = kg; i0 < bw; i0 += 32 * kRows) {
     if (i0 > kg) load_rows(i0);
+    if (i0 - kg + 32 * kRows <= bw) {                           // uniform: a whole round, without a branch or select per row
+      float u[GT_][kRows];
+#pragma unroll
+      for (int k = 0; k < GT_; ++k)
+#pragma unroll
+        for (int q = 0; q < kRows; ++q) u[k][q] = ubs[k * bw + i0 + 32 * q];
+#pragma unroll
+      for (int q = 0; q < kRows; ++q)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const float fr = (float)wr[q][j], fi = (float)wi[q][j];
+#pragma unroll
+          for (int k = 0; k < GT_; ++k) ar[k][j] = fmaf(fr, u[k][q], ar[k][j]), ai[k][j] = fmaf(fi, u[k][q], ai[k][j]);
+        }
+      continue;
+    }
 #pragma unroll
     for (int q = 0; q < kRows; ++q) {
       const int base = i0 - kg + 32 * q, i = base + kg;         // base: uniform
@@ -1868,11 +1893,11 @@ __global__ void __launch_bounds__(256) sm_rglru_step_kernel(
   __syncthreads();
   if (fin) {
     const float sr = red2[fk * kStepOut + (tid & 63)], si = red2[(GT_ + fk) * kStepOut + (tid & 63)];
-    const float av = expf(-scale * sigmoid_f(sr + (float)rb) * softplus_f((float)lam));
+    const float av = expf(-scale * sigmoid_f(sr + (float)rb) * sp);
     const float gv = sqrtf(1.0f - av * av) * sigmoid_f(si + (float)ib) * ubs[fk * bw + fo];
     const float s = fmaf(av, fpos > 0 ? s_in : 0.f, gv);
     *fstate = s;
-    stf((T*)out_ + (size_t)fq * C + b * bw + fo, s * gelu_tanh_f((float)y_in + (float)y_b));
+    stf((T*)out_ + (size_t)fq * C + b * bw + fo, s * gy);
   }
 #pragma unroll
   for (int k = 0; k < GT_; ++k) {
@@ -1896,8 +1921,8 @@ void sm_rglru_step(uintptr_t out, uintptr_t x, uintptr_t y, long ld, uintptr_t c
   DLLM_HOST_CHECK(nb > 0 && bw >= 8 && bw % 8 == 0 && bw <= 512 && (long)nb * bw <= (1L << 24), "rglru step block sizes");
   DLLM_HOST_CHECK(taps >= 1 && taps <= kStepTaps && ld >= (long)nb * bw, "rglru step sizes");
   // sequences per workgroup: two halve the passes over the matrices, which the L2 bears while the grid is small (10 blocks
-  // of 256 at 16 sequences: 9.1 us with one, 10.0 with two; at 64: 20.9 and 20.0)
-  const int gt = seqs <= 32 ? 1 : 2;
+  // of 256 at 16 / 24 sequences: 8.3 / 9.4 us with one, 9.1 / 9.5 with two; at 32 / 64 12.0 / 18.6 and 11.3 / 17.8)
+  const int gt = seqs <= 24 ? 1 : 2;
   const int groups = (seqs + gt - 1) / gt;
   DLLM_HOST_CHECK(arrived != 0 && (long)num_slots * nb * kCountStride <= arrived_len && groups <= 65535, "rglru step counters");
   const size_t lds = ((size_t)(33 * 2 * gt * kStepOut + 32 * 4) + (size_t)gt * bw) * sizeof(float) +
