@@ -581,11 +581,11 @@ constexpr int kDW = 4;
 
 template <int NQK, int NDV, bool BIAS>
 __global__ void __launch_bounds__(64 * kDW) window_attn_decode_kernel(
+    const int32_t* __restrict__ positions, const int32_t* __restrict__ tok_seq, const int32_t* __restrict__ block_tables,
+    int max_blocks, int H, int G, int D, int Dv, int bs, int window, int hpw,   // (14 words: they come with the wave)
     bf16* __restrict__ out, const bf16* __restrict__ q, const bf16* __restrict__ k_cache,
-    const bf16* __restrict__ v_cache, const int32_t* __restrict__ block_tables, int max_blocks,
-    const int32_t* __restrict__ positions, const int32_t* __restrict__ tok_seq, int H, int G, int D, int Dv, int bs,
-    int window, int chunk, float scale, const float* __restrict__ sinks, int hpw, int splits, float* __restrict__ ws,
-    float softcap, const bf16* __restrict__ kp_cache, const bf16* __restrict__ vp_cache, int pool, int pbs,
+    const bf16* __restrict__ v_cache, int chunk, float scale, const float* __restrict__ sinks, int splits,
+    float* __restrict__ ws, float softcap, const bf16* __restrict__ kp_cache, const bf16* __restrict__ vp_cache, int pool, int pbs,
     const float* __restrict__ bias, int nbias, int keep, const bf16* __restrict__ gate, long gate_ld) {
   constexpr int DVP = 16 * NDV;
   __shared__ float so[kDW][16][DVP + 1];
@@ -831,9 +831,9 @@ static void launch_decode(uintptr_t out, uintptr_t q, uintptr_t k_cache, uintptr
   while (hpw > 2 && (long)rows * G * ((R + hpw - 1) / hpw) * splits < 128) hpw = (hpw + 1) / 2;
   hipLaunchKernelGGL(HIP_KERNEL_NAME(window_attn_decode_kernel<NQK, NDV, BIAS>),
                      dim3(rows, G * ((R + hpw - 1) / hpw), splits), dim3(64 * kDW), 0,
-                     (hipStream_t)stream, (bf16*)out, (const bf16*)q, (const bf16*)k_cache, (const bf16*)v_cache,
-                     (const int32_t*)block_tables, max_blocks, (const int32_t*)positions, (const int32_t*)tok_seq, H, G,
-                     D, Dv, bs, window, chunk, scale, (const float*)sinks, hpw, splits, (float*)ws, softcap, (const bf16*)kp,
+                     (hipStream_t)stream, (const int32_t*)positions, (const int32_t*)tok_seq, (const int32_t*)block_tables,
+                     max_blocks, H, G, D, Dv, bs, window, hpw, (bf16*)out, (const bf16*)q, (const bf16*)k_cache,
+                     (const bf16*)v_cache, chunk, scale, (const float*)sinks, splits, (float*)ws, softcap, (const bf16*)kp,
                      (const bf16*)vp, pool, pbs, (const float*)bias, nbias, keep, (const bf16*)gate, gate_ld);
   DLLM_HIP_CHECK(hipGetLastError());
   if (splits > 1) {

@@ -481,9 +481,9 @@ __global__ void __launch_bounds__(256) sm_post_layer_norm_kernel(
 }
 template <typename T, int V, int NV>
 __global__ void __launch_bounds__(256) sm_post_layer_norm_slabs_kernel(
-    float* __restrict__ x, const void* __restrict__ o, int parts, const void* __restrict__ bias, const void* __restrict__ wp,
-    const void* __restrict__ bp, const void* __restrict__ wn, const void* __restrict__ bn, void* __restrict__ h, int width,
-    float eps) {
+    float* __restrict__ x, const void* __restrict__ o, int parts, int width, const void* __restrict__ bias,
+    const void* __restrict__ wp, const void* __restrict__ bp, const void* __restrict__ wn, const void* __restrict__ bn,
+    void* __restrict__ h, float eps) {              // (sizes among the first 14 words: those come with the wave)
   __shared__ float red[16];
   post_layer_norm_row<T, V, NV, true>(red, x, o, parts, bias, wp, bp, wn, bn, h, width, eps);
 }
@@ -543,8 +543,8 @@ void sm_post_layer_norm_add(uintptr_t x, uintptr_t o, int parts, uintptr_t bias,
   DLLM_HOST_CHECK(parts >= 0 && (parts == 0 || (!f32 && width % 4 == 0)), "post_layer_norm_add slabs");
   if (parts > 0)
     SM_LN_SLABS(width, sm_post_layer_norm_slabs_kernel, dim3(rows), stream, (float*)x, (const void*)o, parts,
-                (const void*)bias, (const void*)w_post, (const void*)b_post, (const void*)w_next, (const void*)b_next,
-                (void*)h, width, eps);
+                width, (const void*)bias, (const void*)w_post, (const void*)b_post, (const void*)w_next, (const void*)b_next,
+                (void*)h, eps);
   else
     SM_LN_DISPATCH(f32, width, sm_post_layer_norm_kernel, dim3(rows), stream, (float*)x, (const void*)o,
                    (const void*)bias, (const void*)w_post, (const void*)b_post, (const void*)w_next, (const void*)b_next,
@@ -1738,12 +1738,12 @@ template <> struct Raw8<float> { typedef float type __attribute__((ext_vector_ty
 
 template <typename T, int GT_, int TAPS_>
 __global__ void __launch_bounds__(256) sm_rglru_step_kernel(
+    const int32_t* __restrict__ slots, const int32_t* __restrict__ positions, const void* __restrict__ ra_t_,
+    const void* __restrict__ ri_t_, int seqs, int nb, int bw, int taps, void* conv_state_,   // (14 words: they come with the wave)
     void* __restrict__ out_, const void* __restrict__ x_, const void* __restrict__ y_, long ld,
-    const void* __restrict__ conv_w_, const void* __restrict__ conv_b_, const void* __restrict__ x_b_, void* conv_state_,
-    const void* __restrict__ ra_t_, const void* __restrict__ ra_b_, const void* __restrict__ ri_t_,
-    const void* __restrict__ ri_b_, const void* __restrict__ lam_, const void* __restrict__ y_b_, float* __restrict__ state,
-    const int32_t* __restrict__ positions, const int32_t* __restrict__ slots, int seqs, int nb, int bw, int taps, float scale,
-    unsigned* __restrict__ arrived) {
+    const void* __restrict__ conv_w_, const void* __restrict__ conv_b_, const void* __restrict__ x_b_,
+    const void* __restrict__ ra_b_, const void* __restrict__ ri_b_, const void* __restrict__ lam_, const void* __restrict__ y_b_,
+    float* __restrict__ state, float scale, unsigned* __restrict__ arrived) {
   typedef typename Raw8<T>::type raw8;
   extern __shared__ float smem[];
   constexpr int kPitch = 2 * GT_ * kStepOut + 4;      // (+ 4: the groups of a wave write to banks of their own)
@@ -1936,10 +1936,10 @@ void sm_rglru_step(uintptr_t out, uintptr_t x, uintptr_t y, long ld, uintptr_t c
       DLLM_HIP_CHECK(hipFuncSetAttribute((const void*)sm_rglru_step_kernel<T, G_, N_>,                                    \
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));                      \
     hipLaunchKernelGGL(HIP_KERNEL_NAME(sm_rglru_step_kernel<T, G_, N_>), grid, dim3(256), lds, (hipStream_t)stream,       \
-                       (void*)out, (const void*)x, (const void*)y, ld, (const void*)conv_w, (const void*)conv_b,      \
-                       (const void*)x_b, (void*)conv_state, (const void*)ra_t, (const void*)ra_b, (const void*)ri_t,  \
-                       (const void*)ri_b, (const void*)lam, (const void*)y_b, (float*)state,                          \
-                       (const int32_t*)positions, (const int32_t*)slots, seqs, nb, bw, taps, scale, (unsigned*)arrived);  \
+                       (const int32_t*)slots, (const int32_t*)positions, (const void*)ra_t, (const void*)ri_t, seqs, nb, bw,  \
+                       taps, (void*)conv_state, (void*)out, (const void*)x, (const void*)y, ld, (const void*)conv_w,          \
+                       (const void*)conv_b, (const void*)x_b, (const void*)ra_b, (const void*)ri_b, (const void*)lam,         \
+                       (const void*)y_b, (float*)state, scale, (unsigned*)arrived);                                          \
   } while (0)
 #define SM_STEP_T(T)                                            \
   do {                                                          \
@@ -2110,12 +2110,11 @@ constexpr int kPrepGroups = 2048;     // workgroups that are resident together: 
 
 template <typename T, int R, bool MANY>
 __global__ void __launch_bounds__(256) sm_attn_prep_pair_kernel(
-    void* __restrict__ q_out_, const void* __restrict__ qkv_, const void* __restrict__ conv_w_,
-    const void* state_, const void* __restrict__ q_norm_, const void* __restrict__ k_norm_,
-    const float* __restrict__ freqs, int nrot, float mag, float eps, void* __restrict__ k_cache_,
-    void* __restrict__ v_cache_, const int32_t* __restrict__ slot_mapping, const int32_t* __restrict__ cu,
-    const int32_t* __restrict__ positions, const int32_t* __restrict__ tok_seq, const int32_t* __restrict__ slots,
-    int H, int G, int D, int Dv, int taps, int bs, void* tail_) {
+    const int32_t* __restrict__ tok_seq, const int32_t* __restrict__ cu, const int32_t* __restrict__ positions,
+    const int32_t* __restrict__ slots, int H, int G, int D, int Dv, int taps, int bs,   // (14 words: they come with the wave)
+    void* __restrict__ q_out_, const void* __restrict__ qkv_, const void* __restrict__ conv_w_, const void* state_,
+    const void* __restrict__ q_norm_, const void* __restrict__ k_norm_, const float* __restrict__ freqs, int nrot, float mag,
+    float eps, void* __restrict__ k_cache_, void* __restrict__ v_cache_, const int32_t* __restrict__ slot_mapping, void* tail_) {
   const int t = blockIdx.x, lane = threadIdx.x & 63;
   const int C = H * D + G * (D + Dv);
   const int b = tok_seq[t];
@@ -2272,11 +2271,11 @@ void sm_attn_prep(uintptr_t q_out, uintptr_t qkv, uintptr_t conv_w, uintptr_t st
     const int r = std::max(D, Dv) <= 128 ? 1 : std::max(D, Dv) <= 256 ? 2 : kPrepPairs;
 #define SM_PREP(T_, R_) do { if (gy < most) SM_PREP_M(T_, R_, true); else SM_PREP_M(T_, R_, false); } while (0)
 #define SM_PREP_M(T_, R_, MANY_)                                                                                                    \
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(sm_attn_prep_pair_kernel<T_, R_, MANY_>), dim3(tokens, gy), dim3(256), 0, (hipStream_t)stream, \
-                     (void*)q_out, (const void*)qkv, (const void*)conv_w, (const void*)state, (const void*)q_norm,           \
-                     (const void*)k_norm, (const float*)freqs, nrot, mag, eps, (void*)k_cache, (void*)v_cache,               \
-                     (const int32_t*)slot_mapping, (const int32_t*)cu, (const int32_t*)positions, (const int32_t*)tok_seq,   \
-                     (const int32_t*)slots, H, G, D, Dv, taps, bs, tail ? (void*)state : nullptr)
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(sm_attn_prep_pair_kernel<T_, R_, MANY_>), dim3(tokens, gy), dim3(256), 0,             \
+                     (hipStream_t)stream, (const int32_t*)tok_seq, (const int32_t*)cu, (const int32_t*)positions,            \
+                     (const int32_t*)slots, H, G, D, Dv, taps, bs, (void*)q_out, (const void*)qkv, (const void*)conv_w,      \
+                     (const void*)state, (const void*)q_norm, (const void*)k_norm, (const float*)freqs, nrot, mag, eps,      \
+                     (void*)k_cache, (void*)v_cache, (const int32_t*)slot_mapping, tail ? (void*)state : nullptr)
 #define SM_PREP_R(T_) do { if (r == 1) SM_PREP(T_, 1); else if (r == 2) SM_PREP(T_, 2); else SM_PREP(T_, kPrepPairs); } while (0)
     if (f32) SM_PREP_R(float);
     else SM_PREP_R(bf16);
