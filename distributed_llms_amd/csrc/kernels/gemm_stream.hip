@@ -33,8 +33,8 @@ __global__ void __launch_bounds__(WAVES * 64) gemm_stream_kernel(bf16* __restric
   gemm_stream_body<RG, XG, GLU, NT, WAVES, kNoClose, 64>(Y, X, W, bias, M, N, K, limit, CloseArgs{});
 }
 
-// Groups of 8 weight rows per workgroup up to 16 rows of x: the fewest rows (weights and x) that a CU has to stage.  A CU
-// keeps some 64 cache lines in flight whatever the number of its waves, so the time is that of the CU with the most rows:
+// Groups of 8 weight rows per workgroup up to 16 rows of x: the fewest rows (weights and x) that a CU has to stage.  What a CU
+// takes in does not grow with its waves, so the time is that of the CU with the most rows:
 // ceil(workgroups / 256) (RG + XG).  Where a weight row is a multiple of 4 KiB the lines of 32 and, more so, 64 rows that walk
 // K in step fall on few memory channels: their rows count 1.24 and 1.6 times.  us, M = 1 / 16, 16-row tiles (32 from 256 tiles
 // on) -> this: 1024 x 3072 4.8 / 6.1 -> 4.4 / 5.3, 2048 x 2048 4.5 / 5.1 -> 4.1 / 4.6, 2048 x 8192 10.5 / 12.0 -> 8.3 / 9.5,
