@@ -50,6 +50,8 @@ PYBIND11_MODULE(_C_kernels, m) {
   m.def("sm_embed_f32", &dllm::sm_embed_f32);
   m.def("sm_rms_norm", &dllm::sm_rms_norm);
   m.def("sm_layer_norm", &dllm::sm_layer_norm);
+  m.def("sm_embed_first_norm", &dllm::sm_embed_first_norm);
+  m.def("sm_embed_first_norm_fits", &dllm::sm_embed_first_norm_fits);
   m.def("sm_post_layer_norm_add", &dllm::sm_post_layer_norm_add);
   m.def("sm_gelu_glu", &dllm::sm_gelu_glu);
   m.def("sm_post_norm_add", &dllm::sm_post_norm_add);

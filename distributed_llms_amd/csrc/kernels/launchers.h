@@ -81,6 +81,9 @@ void paged_attention_prefill(uintptr_t out, uintptr_t q, uintptr_t k_cache, uint
 // are float (else bf16)
 void sm_embed_f32(uintptr_t out, uintptr_t ids, uintptr_t table, int tokens, int width, int vocab, float scale, int f32,
                   uintptr_t stream);
+bool sm_embed_first_norm_fits(int width, bool layer);
+void sm_embed_first_norm(uintptr_t x, uintptr_t y, uintptr_t ids, uintptr_t table, uintptr_t w, uintptr_t b, int tokens, int width,
+                         int vocab, float scale, float eps, float offset, int f32, uintptr_t stream);
 void sm_layer_norm(uintptr_t y, uintptr_t x, uintptr_t w, uintptr_t b, int rows, int width, float eps, int f32,
                    uintptr_t stream);
 void sm_post_layer_norm_add(uintptr_t x, uintptr_t o, int parts, uintptr_t bias, uintptr_t w_post, uintptr_t b_post,

@@ -273,11 +273,13 @@ class BasopelStage(LayerListStage):
         sb = self._seq_batch(meta)
         nd = meta.num_decode if meta.is_prefill else meta.num_seqs
         max_ctx = meta.max_ctx_d if (meta.is_prefill and nd) else meta.max_ctx
-        x = sm.embedding_f32(inp, self.embed["embed"], cfg.embed_scale)
-        h = sm.Close.made(x, sm.layer_norm_f32(x, self.layers[0]["norm1"], self.layers[0]["norm1_b"], eps, self.dtype))
+        h = sm.Close.made(*sm.embedding_first_norm(inp, self.embed["embed"], self.layers[0]["norm1"], eps, self.dtype,
+                                                   cfg.embed_scale, self.layers[0]["norm1_b"]))
+        # (every row's logits: the last close makes their norm)
+        last = (self.head["final_norm"], self.head["final_norm_b"]) if meta.logits_idx is None else (None, None)
         v_first = None                    # the values that later layers read, from the first layer that shares them
         for i, (spec, w) in enumerate(zip(self.specs, self.layers)):
-            nxt = (None, None)
+            nxt = last
             if i + 1 < len(self.layers):
                 nxt = (self.layers[i + 1]["norm1"], self.layers[i + 1]["norm1_b"])
             if spec["type"] == LATENT:
@@ -299,9 +301,8 @@ class BasopelStage(LayerListStage):
             if self.taps is not None:
                 h.input()
                 self.taps.append(h.x.clone())
-        h.input()
-        x = h.x
+        hf = h.input()
         if meta.logits_idx is not None:
-            x = x.index_select(0, meta.logits_idx)
-        hf = sm.layer_norm_f32(x, self.head["final_norm"], self.head["final_norm_b"], eps, self.dtype)
+            hf = sm.layer_norm_f32(h.x.index_select(0, meta.logits_idx), self.head["final_norm"], self.head["final_norm_b"], eps,
+                                   self.dtype)
         return sm.softcap_f32(ops.linear(hf, self.embed["embed"]), 0.0)

@@ -369,12 +369,12 @@ class HybridStage(LayerListStage):
         cfg = self.cfg
         eps, mult = cfg.norm_eps, cfg.residual_mult
         sb = self._seq_batch(meta)
-        x = sm.embedding_f32(inp, self.embed["embed"])
-        h = sm.Close.made(x, sm.rms_norm_f32(x, self.layers[0]["norm1"], eps, self.dtype))
+        h = sm.Close.made(*sm.embedding_first_norm(inp, self.embed["embed"], self.layers[0]["norm1"], eps, self.dtype))
         n = len(self.layers)
+        last = self.head["final_norm"] if meta.logits_idx is None else None     # every row's logits: the last close makes their norm
         for i, (spec, w) in enumerate(zip(self.specs, self.layers)):
             o = self._attention(i, h, w, meta, sb) if spec["type"] == "attention" else self._rglru(i, h, w, sb)
-            nxt = self.layers[i + 1]["norm1"] if i + 1 < n else None
+            nxt = self.layers[i + 1]["norm1"] if i + 1 < n else last
             h = sm.Close("rms", h.x, o, w_post=w["norm1b"], eps=eps, mult=mult, w_next=w["norm2"] if spec.get("mlp") else nxt)
             if spec.get("mlp"):
                 y = h.clipped_glu(w["w_gu"], w["b_gu"], spec["mlp"]["limit"])
@@ -383,11 +383,9 @@ class HybridStage(LayerListStage):
             if self.taps is not None:
                 h.input()
                 self.taps.append(h.x.clone())
-        h.input()
-        x = h.x
+        hf = h.input()
         if meta.logits_idx is not None:
-            x = x.index_select(0, meta.logits_idx)
-        hf = sm.rms_norm_f32(x, self.head["final_norm"], eps, self.dtype)
+            hf = sm.rms_norm_f32(h.x.index_select(0, meta.logits_idx), self.head["final_norm"], eps, self.dtype)
         return sm.softcap_f32(ops.linear(hf, self.head["lm_head"]), cfg.logit_softcap)
 
 

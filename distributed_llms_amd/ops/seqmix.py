@@ -197,6 +197,30 @@ def layer_norm_f32(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor, eps: float
     return y
 
 
+def embedding_first_norm(ids: torch.Tensor, table: torch.Tensor, w: torch.Tensor, eps: float, act_dtype, scale: float = 1.0,
+                         b: Optional[torch.Tensor] = None):
+    """:func:`embedding_f32` and, of its rows, :func:`layer_norm_f32` (with a bias ``b``) or :func:`rms_norm_f32`: the stream and
+    the first sublayer's input, in one launch where the rows fit its registers."""
+    ptrs = (table, w) if b is None else (table, w, b)
+    if (table.is_cuda and table.dtype == act_dtype and all(t.data_ptr() % 32 == 0 for t in ptrs)
+            and _k().sm_embed_first_norm_fits(table.shape[1], b is not None)):
+        _ck(ids, "ids", torch.int32)
+        _ck(table, "table")
+        _ck(w, "w", act_dtype)
+        if b is not None:
+            _ck(b, "b", act_dtype)
+        t, (vocab, width) = ids.numel(), table.shape
+        if w.numel() != width or (b is not None and b.numel() != width):
+            raise ValueError("embedding_first_norm: weight / bias width")
+        x = torch.empty(t, width, dtype=torch.float32, device=table.device)
+        y = torch.empty(t, width, dtype=act_dtype, device=table.device)
+        _k().sm_embed_first_norm(x.data_ptr(), y.data_ptr(), ids.data_ptr(), table.data_ptr(), w.data_ptr(), _ptr(b), t, width, vocab,
+                                 float(scale), float(eps), 1.0, _f32flag(table), _stream())
+        return x, y
+    x = embedding_f32(ids, table, scale)
+    return x, rms_norm_f32(x, w, eps, act_dtype) if b is None else layer_norm_f32(x, w, b, eps, act_dtype)
+
+
 def post_layer_norm_add(x: torch.Tensor, o, w_post: torch.Tensor, b_post: torch.Tensor, eps: float,
                         bias: Optional[torch.Tensor] = None, w_next: Optional[torch.Tensor] = None,
                         b_next: Optional[torch.Tensor] = None):
