@@ -105,14 +105,15 @@ struct CloseRow {
 }  // namespace
 
 // GLU 0: y [M, N] (+ bias [N]);  1 / 2 / 3: SiLU / clipped (`limit`) / gelu GLU, w = [gate; up], y [M, N / 2], bias
-// gate | up.  A workgroup's RG groups of 8 weight rows are its output columns, under a GLU CW gate rows and then the same
-// columns' up rows; XG groups of 8 rows of x.  An odd last group fills half an MFMA tile, its other half repeats it.
+// gate | up;  4: y [M, N] in float32, soft-capped by `limit` where that is positive (logits).  A workgroup's RG groups of
+// 8 weight rows are its output columns, under a GLU CW gate rows and then the same columns' up rows; XG groups of 8 rows of x.  An odd last group fills half an MFMA tile, its other half repeats it.
 // CLOSE (M == 1): x is not read but made (CloseRow, K <= KMAX) by CV further waves, and stays in LDS.
 template <int RG, int XG, int GLU, bool NT, int WAVES, int CLOSE, int KMAX>
 __device__ __forceinline__ void gemm_stream_body(bf16* __restrict__ Y, const bf16* __restrict__ X, const bf16* __restrict__ W,
                                                  const bf16* __restrict__ bias, int M, int N, int K, float limit,
                                                  const CloseArgs& close) {
-  static_assert(GLU == 0 || RG % 2 == 0 || RG == 3, "a GLU's CW is a multiple of 4");
+  constexpr bool PAIR = GLU >= 1 && GLU <= 3, CAPPED = GLU == 4;
+  static_assert(!PAIR || RG % 2 == 0 || RG == 3, "a GLU's CW is a multiple of 4");
   constexpr int RT = (RG + 1) / 2, MT = (XG + 1) / 2;
   constexpr int G = CLOSE ? RG : RG + XG;                       // loads per K-tile
   constexpr int SLOT = G * 8 * SK;                              // bf16 elements of one ring slot: weights, then x
@@ -124,14 +125,14 @@ __device__ __forceinline__ void gemm_stream_body(bf16* __restrict__ Y, const bf1
   __shared__ __attribute__((aligned(16))) bf16 made[CLOSE ? KMAX : 8];
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int fr = lane & 15, fq = lane >> 4;
-  const int half = N / 2, ncols = GLU ? half : N;
-  constexpr int CW = GLU ? RG * 4 : RG * 8;                     // output columns
+  const int half = N / 2, ncols = PAIR ? half : N;
+  constexpr int CW = PAIR ? RG * 4 : RG * 8;                    // output columns
   const int c0 = blockIdx.x * CW;
   bf16* ring = reinterpret_cast<bf16*>(smem) + wv * (D * SLOT);
 
   // weight row of row r of the workgroup; rows past the matrix repeat its last row
   auto wrow = [&](int r) {
-    const bool up = GLU && r >= CW;
+    const bool up = PAIR && r >= CW;
     return (up ? half : 0) + min(c0 + (up ? r - CW : r), ncols - 1);
   };
   typedef CloseRow<CLOSE, CLOSE ? (KMAX + 256 * CV - 1) / (256 * CV) : 1> Row;
@@ -143,13 +144,13 @@ __device__ __forceinline__ void gemm_stream_body(bf16* __restrict__ Y, const bf1
   // for each of a thread's eight loads -> this, M = 1 / 16: 6144 x 1024 + clipped GLU 5.18 / 5.55 -> 4.79 / 5.18, 15360 x 2560
   // 16.5 / 15.9 -> 16.2 / 15.6; 2560 x 2560 plain 4.96 / 6.15 -> 4.80 / 5.92.
   constexpr int EL = CW / 4 * MT * 16, NE = (EL + TH - 1) / TH;
-  bf16 eb[NE][GLU ? 8 : 4] = {};
+  bf16 eb[NE][PAIR ? 8 : 4] = {};
   auto load_bias = [&](const bf16* bs, int n) {
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const int cc = min(c0 + 4 * (((tid + n * TH) >> 4) % (CW / 4)) + v, ncols - 1);
       eb[n][v] = bs[bias ? cc : 0];
-      if constexpr (GLU != 0) eb[n][4 + v] = bs[bias ? half + cc : 0];
+      if constexpr (PAIR) eb[n][4 + v] = bs[bias ? half + cc : 0];
     }
   };
   if constexpr (GLU == 2) {
@@ -258,7 +259,7 @@ __device__ __forceinline__ void gemm_stream_body(bf16* __restrict__ Y, const bf1
     f32x4 a = red[at], b = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 1; w < WAVES; ++w) a += red[w * RT * MT * 64 + at];
-    if constexpr (GLU != 0) {
+    if constexpr (PAIR) {
       const int up = ((U >> 4) * MT + m) * 64 + ((U >> 2) & 3) * 16 + (e & 15);
 #pragma unroll
       for (int w = 0; w < WAVES; ++w) b += red[w * RT * MT * 64 + up];
@@ -270,12 +271,29 @@ __device__ __forceinline__ void gemm_stream_body(bf16* __restrict__ Y, const bf1
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       float z = a[v] + (bias ? bf2f(eb[n][v]) : 0.f);
-      if constexpr (GLU != 0) {
+      if constexpr (PAIR) {
         const float up = b[v] + (bias ? bf2f(eb[n][4 + v]) : 0.f);
         // (a projection, a bias and a gate kernel until they met here: the gate kernels' arithmetic)
         z = GLU == 1 ? silu_f(z) * up : GLU == 2 ? clipped_glu_exact_f(z, up, limit, kGluAlpha) : gelu_glu_exact_f(z, up);
       }
       o[v] = f2bf(z);
+    }
+    if constexpr (CAPPED) {                          // logits: of the product's bf16, as a launch of their own made them
+      f32x4 l;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const float z = bf2f(o[v]);
+        l[v] = limit > 0.f ? limit * tanhf(z / limit) : z;
+      }
+      float* dst = reinterpret_cast<float*>(Y) + (size_t)row * ncols + c;
+      if (c + 4 <= ncols && ncols % 4 == 0) {
+        *reinterpret_cast<f32x4*>(dst) = l;
+      } else {
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          if (c + v < ncols) dst[v] = l[v];
+      }
+      continue;
     }
     bf16* dst = Y + (size_t)row * ncols + c;
     if (c + 4 <= ncols && ncols % 4 == 0) {

@@ -53,31 +53,35 @@ int stream_rows(int ncols, int K, bool glu, int xg) {
 }
 
 // glu 0: y [M, N] = x w^T (+ bias);  1 / 2 / 3: y [M, N / 2], SiLU / clipped / gelu GLU of w = [gate; up] (+ bias).
+// 4: y [M, N] in float32, cap tanh(z / cap) of the rounded product z with cap = limit, z itself where that is not positive.
+// (A launch of their own read the rounded logits back and wrote 4 bytes each: 1.6 to 2 us of a step whose head's product takes
+// 12.4; the epilogue's threads have them in registers.  The sums keep their order, so the logits their bits.)
 // nt: nontemporal weight loads.
 void gemm_stream(uintptr_t y, uintptr_t x, uintptr_t w, uintptr_t bias, int M, int N, int K, int glu, int nt, float limit,
                  uintptr_t stream) {
   DLLM_HOST_CHECK(M >= 1 && M <= 64, "1 <= M <= 64");
   DLLM_HOST_CHECK(K >= SK && K % SK == 0, "K must be a positive multiple of 64");
-  DLLM_HOST_CHECK(glu >= 0 && glu <= 3, "glu 0..3");
-  DLLM_HOST_CHECK(N >= 1 && (glu == 0 || N % 2 == 0), "N");
-  DLLM_HOST_CHECK(x % 16 == 0 && w % 16 == 0 && y % 8 == 0, "operand alignment");
+  DLLM_HOST_CHECK(glu >= 0 && glu <= 4, "glu 0..4");
+  const bool pair = glu >= 1 && glu <= 3;
+  DLLM_HOST_CHECK(N >= 1 && (!pair || N % 2 == 0), "N");
+  DLLM_HOST_CHECK(x % 16 == 0 && w % 16 == 0 && y % (glu == 4 ? 16 : 8) == 0, "operand alignment");
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const int ncols = glu ? N / 2 : N;
+  const int ncols = pair ? N / 2 : N;
   const bool one = M <= 16;
   const int xg = M <= 8 ? 1 : M <= 16 ? 2 : M <= 32 ? 4 : 8;
   int rg;
   if (one) {
-    rg = stream_rows(ncols, K, glu != 0, xg);
+    rg = stream_rows(ncols, K, pair, xg);
   } else {
     // twice the weight rows per workgroup (half the x staging) once that still leaves a workgroup for most CUs
     const bool two = (ncols + 15) / 16 > 256;
-    rg = (glu ? 4 : 2) * (two ? 2 : 1);
+    rg = (pair ? 4 : 2) * (two ? 2 : 1);
   }
-  const int per = glu ? rg * 4 : rg * 8;
+  const int per = pair ? rg * 4 : rg * 8;
   const dim3 grid((ncols + per - 1) / per);
   // 8 waves where up to three groups of plain rows have a CU each: their K loop is over in one or two rounds; else 4
   // (several workgroups per CU)
-  const bool wide = glu == 0 && (one ? rg <= 3 && grid.x <= 256 : rg == 2 && xg == 4);
+  const bool wide = !pair && (one ? rg <= 3 && grid.x <= 256 : rg == 2 && xg == 4);
 #define DLLM_ST_GO(RG_, XG_, GLU_, WV_)                                                                             \
   do {                                                                                                              \
     if (nt) hipLaunchKernelGGL((gemm_stream_kernel<RG_, XG_, GLU_, true, WV_>), grid, dim3(WV_ * 64), 0, s,         \
@@ -89,6 +93,11 @@ void gemm_stream(uintptr_t y, uintptr_t x, uintptr_t w, uintptr_t bias, int M, i
   do {                                                                                                              \
     constexpr int W8 = RG_ <= 3 && XG_ <= 4 ? 8 : 4;                                                                  \
     if (wide) DLLM_ST_GO(RG_, XG_, 0, W8); else DLLM_ST_GO(RG_, XG_, 0, 4);                                            \
+  } while (0)
+#define DLLM_ST_C(RG_, XG_)                                                                                         \
+  do {                                                                                                              \
+    constexpr int W8 = RG_ <= 3 && XG_ <= 4 ? 8 : 4;                                                                  \
+    if (wide) DLLM_ST_GO(RG_, XG_, 4, W8); else DLLM_ST_GO(RG_, XG_, 4, 4);                                            \
   } while (0)
 #define DLLM_ST_G(RG_, XG_)                                                                                         \
   do {                                                                                                              \
@@ -107,6 +116,11 @@ void gemm_stream(uintptr_t y, uintptr_t x, uintptr_t w, uintptr_t bias, int M, i
     else if (rg == 2) DLLM_ST_M(DLLM_ST_P, 2);
     else if (rg == 3) DLLM_ST_X(DLLM_ST_P, 3);
     else DLLM_ST_M(DLLM_ST_P, 4);
+  } else if (glu == 4) {
+    if (rg == 1) DLLM_ST_X(DLLM_ST_C, 1);
+    else if (rg == 2) DLLM_ST_M(DLLM_ST_C, 2);
+    else if (rg == 3) DLLM_ST_X(DLLM_ST_C, 3);
+    else DLLM_ST_M(DLLM_ST_C, 4);
   } else {
     if (rg == 2) DLLM_ST_X(DLLM_ST_G, 2);
     else if (rg == 3) DLLM_ST_X(DLLM_ST_G, 3);
@@ -117,6 +131,7 @@ void gemm_stream(uintptr_t y, uintptr_t x, uintptr_t w, uintptr_t bias, int M, i
 #undef DLLM_ST_M
 #undef DLLM_ST_X
 #undef DLLM_ST_G
+#undef DLLM_ST_C
 #undef DLLM_ST_P
 #undef DLLM_ST_GO
   DLLM_HIP_CHECK(hipGetLastError());

@@ -305,4 +305,4 @@ class BasopelStage(LayerListStage):
         if meta.logits_idx is not None:
             hf = sm.layer_norm_f32(h.x.index_select(0, meta.logits_idx), self.head["final_norm"], self.head["final_norm_b"], eps,
                                    self.dtype)
-        return sm.softcap_f32(ops.linear(hf, self.embed["embed"]), 0.0)
+        return sm.logits_f32(hf, self.embed["embed"])

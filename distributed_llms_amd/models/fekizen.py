@@ -353,4 +353,4 @@ class FekizenStage(LayerListStage):
         if meta.logits_idx is not None:
             x = x.index_select(0, meta.logits_idx)
         hf = sm.rms_norm_f32(x, self.head["final_norm"], eps, self.dtype, one_plus=False)
-        return sm.softcap_f32(ops.linear(hf, self.head["lm_head"]), 0.0)
+        return sm.logits_f32(hf, self.head["lm_head"])

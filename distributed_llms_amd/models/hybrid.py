@@ -386,7 +386,7 @@ class HybridStage(LayerListStage):
         hf = h.input()
         if meta.logits_idx is not None:
             hf = sm.rms_norm_f32(h.x.index_select(0, meta.logits_idx), self.head["final_norm"], eps, self.dtype)
-        return sm.softcap_f32(ops.linear(hf, self.head["lm_head"]), cfg.logit_softcap)
+        return sm.logits_f32(hf, self.head["lm_head"], cfg.logit_softcap)
 
 
 class _PagedCaches:

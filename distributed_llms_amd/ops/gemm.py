@@ -329,6 +329,15 @@ def _stream(m: int, n: int, k: int, x: torch.Tensor, w: torch.Tensor, bias: Opti
     return y
 
 
+def stream_logits(x: torch.Tensor, w: torch.Tensor, cap: float) -> torch.Tensor:
+    """float32 cap tanh(z / cap) of z = x w^T rounded to bf16 (cap <= 0: z) of sizes that :func:`use_stream` takes."""
+    (m, k), n = x.shape, w.shape[0]
+    y = torch.empty(m, n, dtype=torch.float32, device=x.device)
+    _ext.kernels().gemm_stream(y.data_ptr(), x.data_ptr(), w.data_ptr(), 0, m, n, k, 4, 1 if n * k * 2 >= WIDE_NT_MIN_BYTES else 0,
+                               float(cap), current_stream())
+    return y
+
+
 class SplitKPartial:
     """Split-K partial sums of ``x @ w.T`` still in the per-stream workspace (not reduced).  Each K
     slice accumulates in f32; the slabs hold it as f16 x 2^-6 by default (csrc/kernels/common.h

@@ -627,6 +627,17 @@ def softcap_f32(logits: torch.Tensor, cap: float, scale: float = 1.0) -> torch.T
     return out
 
 
+def logits_f32(x: torch.Tensor, w: torch.Tensor, cap: float = 0.0) -> torch.Tensor:
+    """:func:`softcap_f32` of the product ``x w^T``: in the product's own launch where that is the weight-streaming one (32000
+    columns of K = 1024, 1 / 8 / 16 rows: 13.9 / 14.2 / 15.1 us in two launches, 12.3 / 12.4 / 13.1 in one)."""
+    from . import gemm, linear
+    if (type(x) is torch.Tensor and type(w) in (torch.Tensor, torch.nn.Parameter) and x.is_cuda and x.dim() == 2
+            and x.shape[0] <= gemm.STREAM_MAX_M and x.device == w.device and w.dim() == 2 and w.shape[1] == x.shape[1]
+            and not gemm._recorded(x, w, None) and gemm.use_stream(x.shape[0], w.shape[0], x.shape[1], x, w)):
+        return gemm.stream_logits(x, w, cap)
+    return softcap_f32(linear(x, w), cap)
+
+
 # ------------------------------------------------------------------ rotary tables
 def yarn_frequencies(dims: int, base: float, scaling: Optional[dict]) -> Tuple[torch.Tensor, float]:
     """(f [dims / 2] float32, magnitude): rotary frequencies f_i = base^(-2i/dims), blended by YaRN
