@@ -106,7 +106,8 @@ struct CloseRow {
 
 // GLU 0: y [M, N] (+ bias [N]);  1 / 2 / 3: SiLU / clipped (`limit`) / gelu GLU, w = [gate; up], y [M, N / 2], bias
 // gate | up;  4: y [M, N] in float32, soft-capped by `limit` where that is positive (logits).  A workgroup's RG groups of
-// 8 weight rows are its output columns, under a GLU CW gate rows and then the same columns' up rows; XG groups of 8 rows of x.  An odd last group fills half an MFMA tile, its other half repeats it.
+// 8 weight rows are its output columns, under a GLU CW gate rows and then the same columns' up rows; XG groups of 8 rows of
+// x.  An odd last group fills half an MFMA tile, its other half repeats it.
 // CLOSE (M == 1): x is not read but made (CloseRow, K <= KMAX) by CV further waves, and stays in LDS.
 template <int RG, int XG, int GLU, bool NT, int WAVES, int CLOSE, int KMAX>
 __device__ __forceinline__ void gemm_stream_body(bf16* __restrict__ Y, const bf16* __restrict__ X, const bf16* __restrict__ W,

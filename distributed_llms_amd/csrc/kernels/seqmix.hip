@@ -1395,15 +1395,14 @@ __device__ __forceinline__ float sqrt_near(float x) {          // x <= 0: 0
 // us, 10 blocks of 256, 6376 / 3000 / 300 tokens: 127 / 65 / 41 with an output per lane (weights two bytes at a time), u taken apart for
 // 128 outputs and the library's functions, 83 / 45 / 24 here (275 on the float32 matrix cores at 6376); 4 blocks, 2000 / 168: 43 / 39 ->
 // 26 / 23.  Largest error of a and g against 64 bits there 5.4e-7 and 8.1e-6, means 1.8e-8 and 2.8e-8, as before.
-// VEC: blocks a multiple of 4 wide and aligned; else elements one by one.
+// Blocks a multiple of 4 wide, 16-byte aligned.
 constexpr int kST = 64;       // tokens per workgroup
 constexpr int kSO = 256;      // outputs
 constexpr int kSK = 64;       // K chunk in LDS
 constexpr int kSP = kSK + 8;
 constexpr float kBfMax = 0x1.fep+127f;
 
-template <bool VEC>
-__global__ void __launch_bounds__(256, VEC ? 2 : 1) sm_rglru_gates_split_kernel(
+__global__ void __launch_bounds__(256, 2) sm_rglru_gates_split_kernel(
     float* __restrict__ a_out, float* __restrict__ g_out, const float* __restrict__ u, const bf16* __restrict__ ra_t,
     const bf16* __restrict__ ra_b, const bf16* __restrict__ ri_t, const bf16* __restrict__ ri_b,
     const bf16* __restrict__ lam, int tokens, int nb, int bw, float scale) {
@@ -1422,12 +1421,7 @@ __global__ void __launch_bounds__(256, VEC ? 2 : 1) sm_rglru_gates_split_kernel(
   const auto rsa = __builtin_amdgcn_make_buffer_rsrc((void*)(a_out + row0), (short)0, bytes, 0x00020000);
   const auto rsg = __builtin_amdgcn_make_buffer_rsrc((void*)(g_out + row0), (short)0, bytes, 0x00020000);
   auto row4 = [&](int r, int k) -> f32x4 {                   // channels k .. k + 3 of the block in the workgroup's row r
-    if constexpr (VEC) {
-      return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(ru, (r * C + b * bw + k) * 4, 0, 0));
-    } else {
-      const float* row = u + (size_t)min(t0 + r, tokens - 1) * C + b * bw;
-      return f32x4{row[min(k, bw - 1)], row[min(k + 1, bw - 1)], row[min(k + 2, bw - 1)], row[min(k + 3, bw - 1)]};
-    }
+    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(ru, (r * C + b * bw + k) * 4, 0, 0));
   };
 
   // a chunk's values of this thread: four of row (tid >> 4) + 16 q each, zero past the block
@@ -1485,20 +1479,10 @@ __global__ void __launch_bounds__(256, VEC ? 2 : 1) sm_rglru_gates_split_kernel(
   const auto rr = __builtin_amdgcn_make_buffer_rsrc((void*)(ra_t + blk), (short)0, bw * bw * 2, 0x00020000);
   const auto ri = __builtin_amdgcn_make_buffer_rsrc((void*)(ri_t + blk), (short)0, bw * bw * 2, 0x00020000);
   const int lane_w = (8 * half * bw + o) * 2;
-  auto load_w = [&](u32x2 (&w)[8], const __amdgpu_buffer_rsrc_t& g, [[maybe_unused]] const bf16* m, int k0) {
+  auto load_w = [&](u32x2 (&w)[8], const __amdgpu_buffer_rsrc_t& g, int k0) {
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      if constexpr (VEC) {
-        w[q] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(g, lane_w + (k0 + q) * bw * 2, 0, 0));
-      } else {
-        const int k = k0 + 8 * half + q;
-        const bf16* row = m + blk + (size_t)min(k, bw - 1) * bw;
-        bf16x4 v;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = k < bw ? row[min(o + e, bw - 1)] : (bf16)0.f;
-        w[q] = __builtin_bit_cast(u32x2, v);
-      }
-    }
+    for (int q = 0; q < 8; ++q)
+      w[q] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(g, lane_w + (k0 + q) * bw * 2, 0, 0));
   };
   auto fragments = [&](bf16x8 (&f)[4], const u32x2 (&w)[8]) {
 #pragma unroll
@@ -1518,8 +1502,8 @@ __global__ void __launch_bounds__(256, VEC ? 2 : 1) sm_rglru_gates_split_kernel(
     for (int i = 0; i < 16; ++i) cr[j][i] = ci[j][i] = 0.f;
   u32x2 wr[8], wi[8];
   load_u(0);
-  load_w(wr, rr, ra_t, 0);
-  load_w(wi, ri, ri_t, 0);
+  load_w(wr, rr, 0);
+  load_w(wi, ri, 0);
   store_u(0);
   int buf = 0;
   for (int kc = 0; kc < bw; kc += kSK, buf ^= 1) {
@@ -1534,7 +1518,7 @@ __global__ void __launch_bounds__(256, VEC ? 2 : 1) sm_rglru_gates_split_kernel(
 #pragma unroll
         for (int p = 0; p < 3; ++p) a[p] = *reinterpret_cast<const bf16x8*>(&us[buf][p][32 * wm + n][16 * s + 8 * half]);
         fragments(f, wr);
-        load_w(wr, rr, ra_t, k0 + 16);                       // (past the last step: zeros, not used)
+        load_w(wr, rr, k0 + 16);                             // (past the last step: zeros, not used)
         __builtin_amdgcn_sched_barrier(0);                   // (hipcc moves these loads behind the products)
 #pragma unroll
         for (int j = 0; j < 4; ++j)
@@ -1542,7 +1526,7 @@ __global__ void __launch_bounds__(256, VEC ? 2 : 1) sm_rglru_gates_split_kernel(
           for (int p = 2; p >= 0; --p)                       // the small pieces first
             cr[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[p], f[j], cr[j], 0, 0, 0);
         fragments(f, wi);
-        load_w(wi, ri, ri_t, k0 + 16);
+        load_w(wi, ri, k0 + 16);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int j = 0; j < 4; ++j)
@@ -1576,22 +1560,111 @@ __global__ void __launch_bounds__(256, VEC ? 2 : 1) sm_rglru_gates_split_kernel(
         av[j] = expf(-scale * sigmoid_near(cr[j][i] + rb[j]) * sp[j]);
         gv[j] = sqrt_near(1.0f - av[j] * av[j]) * sigmoid_near(ci[j][i] + ib[j]) * ux[i][j];
       }
-      if constexpr (VEC) {
-        const int at = ((r + i) * C + b * bw + o) * 4;
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, av), rsa, at, 0, 0);
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, gv), rsg, at, 0, 0);
-      } else if (t0 + r + i < tokens) {
-        const size_t at = (size_t)(t0 + r + i) * C + b * bw + o;
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          if (o + j < bw) a_out[at + j] = av[j], g_out[at + j] = gv[j];
-      }
+      const int at = ((r + i) * C + b * bw + o) * 4;
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, av), rsa, at, 0, 0);
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, gv), rsg, at, 0, 0);
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       ux[j] = un[j];
 #pragma unroll
       for (int i = 0; i < 12; ++i) cr[j][i] = cr[j][i + 4], ci[j][i] = ci[j][i + 4];
+    }
+  }
+}
+
+// The same sums with an output per lane and 32 per wave, 128 tokens by 128 outputs per workgroup, u and the weights element by
+// element: any width and alignment, and no lane idle from blocks of 128 on.  Bound by its vector work and by two-byte loads.
+// Which kernel, us, this / the one above: widths that are no multiple of 4 this (8 blocks of 255, 300 / 16000 tokens 41 / 266
+// against 59 / 503 element by element there); 8 blocks of 64, 128, 256: 2000 tokens 26 / 18, 32 / 22, 45 / 29; 8000 tokens 36 / 41,
+// 49 / 55, 116 / 85: blocks up to 128 leave half of the other's waves idle, which counts once the CUs hold two workgroups each;
+// 3 blocks of 24, 300 / 16000 tokens: 23 / 28, 27 / 44.
+constexpr int kCT = 128;      // tokens per workgroup
+
+__global__ void __launch_bounds__(256, 2) sm_rglru_gates_column_kernel(
+    float* __restrict__ a_out, float* __restrict__ g_out, const float* __restrict__ u, const bf16* __restrict__ ra_t,
+    const bf16* __restrict__ ra_b, const bf16* __restrict__ ri_t, const bf16* __restrict__ ri_b,
+    const bf16* __restrict__ lam, int tokens, int nb, int bw, float scale) {
+  __shared__ __attribute__((aligned(16))) bf16 us[3][kCT][kSP];
+  const int t0 = blockIdx.x * kCT, b = blockIdx.y, C = nb * bw;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, n = lane & 31, half = lane >> 5;
+  const int o = blockIdx.z * 128 + wave * 32 + n;            // this lane's output channel inside block b
+  const int oc = min(o, bw - 1);
+  const bf16* ra = ra_t + (size_t)b * bw * bw + oc;
+  const bf16* ri = ri_t + (size_t)b * bw * bw + oc;
+  f32x16 cr[4], ci[4];
+#pragma unroll
+  for (int m = 0; m < 4; ++m)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) cr[m][i] = ci[m][i] = 0.f;
+  bf16x8 wr[2], wi[2];
+  auto load_w = [&](int k0, int buf) {                       // rows k0 + 8 half .. of this lane's output column
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const size_t at = (size_t)min(k0 + 8 * half + j, bw - 1) * bw;
+      wr[buf][j] = ra[at];
+      wi[buf][j] = ri[at];
+    }
+  };
+  load_w(0, 0);
+  const float* ub = u + (size_t)b * bw;
+  for (int kc = 0; kc < bw; kc += kSK) {
+    __syncthreads();
+#pragma unroll 8
+    for (int i = tid; i < kCT * kSK; i += 256) {             // a wave per row of the chunk
+      const int r = i / kSK, k = i - r * kSK;
+      const bool ok = t0 + r < tokens && kc + k < bw;
+      float x = ub[(size_t)min(t0 + r, tokens - 1) * C + min(kc + k, bw - 1)];
+      x = ok ? x : 0.f;
+      // (a finite x above the largest bf16 keeps a finite first piece; an infinite or NaN one has no others)
+      const bool fin = __builtin_isfinite(x);
+      const bf16 h = f2bf(fin ? fminf(fmaxf(x, -kBfMax), kBfMax) : x);
+      const float xm = fin ? x - bf2f(h) : 0.f;
+      const bf16 m = f2bf(xm);
+      us[0][r][k] = h;
+      us[1][r][k] = m;
+      us[2][r][k] = f2bf(xm - bf2f(m));
+    }
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < kSK / 16; ++s) {
+      if (kc + 16 * s < bw) {                                // uniform
+        load_w(kc + 16 * (s + 1), (s + 1) & 1);              // (past the last step: the last row, not used)
+        bf16x8 br = wr[s & 1], bi = wi[s & 1];
+        if (kc + 16 * (s + 1) > bw) {                        // uniform: rows past the block
+#pragma unroll
+          for (int j = 0; j < 8; ++j)
+            if (kc + 16 * s + 8 * half + j >= bw) br[j] = bi[j] = (bf16)0.f;
+        }
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+#pragma unroll
+          for (int p = 2; p >= 0; --p) {                     // the small pieces first
+            const bf16x8 a = *reinterpret_cast<const bf16x8*>(&us[p][32 * m + n][16 * s + 8 * half]);
+            cr[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, br, cr[m], 0, 0, 0);
+            ci[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, bi, ci[m], 0, 0, 0);
+          }
+      }
+    }
+  }
+  if (o >= bw) return;
+  const int ch = b * bw + o;
+  const float rb = bf2f(ra_b[ch]), ib = bf2f(ri_b[ch]), sp = softplus_f(bf2f(lam[ch]));
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+    float x[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      x[i] = u[(size_t)min(t0 + 32 * m + 8 * (i >> 2) + 4 * half + (i & 3), tokens - 1) * C + ch];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int t = t0 + 32 * m + 8 * (i >> 2) + 4 * half + (i & 3);    // accumulator register i of this lane
+      const float av = expf(-scale * sigmoid_f(cr[m][i] + rb) * sp);
+      const float gv = sqrtf(1.0f - av * av) * sigmoid_f(ci[m][i] + ib) * x[i];
+      if (t < tokens) {
+        a_out[(size_t)t * C + ch] = av;
+        g_out[(size_t)t * C + ch] = gv;
+      }
     }
   }
 }
@@ -1616,14 +1689,15 @@ void sm_rglru_gates(uintptr_t a, uintptr_t g, uintptr_t u, uintptr_t ra_t, uintp
     return;
   }
   if (!f32) {
-    const dim3 grid((tokens + kST - 1) / kST, nb, (bw + kSO - 1) / kSO);
+    const dim3 grid((tokens + kST - 1) / kST, nb, (bw + kSO - 1) / kSO), cols((tokens + kCT - 1) / kCT, nb, (bw + 127) / 128);
     const bool vec = bw % 4 == 0 && (u | a | g) % 16 == 0 && (ra_t | ri_t) % 8 == 0;
-#define SM_GATES(VEC_)                                                                                                     \
-  hipLaunchKernelGGL(sm_rglru_gates_split_kernel<VEC_>, grid, dim3(256), 0, (hipStream_t)stream, (float*)a, (float*)g,       \
-                     (const float*)u, (const bf16*)ra_t, (const bf16*)ra_b, (const bf16*)ri_t, (const bf16*)ri_b,            \
-                     (const bf16*)lam, tokens, nb, bw, scale)
-    if (vec) SM_GATES(true);
-    else SM_GATES(false);
+    const bool split = vec && bw >= 48 && (bw > 128 || (size_t)grid.x * nb <= 512);
+#define SM_GATES(KERNEL_, GRID_)                                                                                           \
+  hipLaunchKernelGGL(KERNEL_, GRID_, dim3(256), 0, (hipStream_t)stream, (float*)a, (float*)g, (const float*)u,               \
+                     (const bf16*)ra_t, (const bf16*)ra_b, (const bf16*)ri_t, (const bf16*)ri_b, (const bf16*)lam, tokens,   \
+                     nb, bw, scale)
+    if (split) SM_GATES(sm_rglru_gates_split_kernel, grid);
+    else SM_GATES(sm_rglru_gates_column_kernel, cols);
 #undef SM_GATES
     DLLM_HIP_CHECK(hipGetLastError());
     return;

@@ -40,6 +40,13 @@ def test_gates_keep_all_bits_of_the_input(cuda, nb, bw, tokens, size):
     assert (err <= ((hi - lo) * gate + dg + 1e-6) * x.abs() + 1e-12).all()
 
 
+@pytest.mark.parametrize("nb,bw,tokens", [(8, 48, 4096), (8, 48, 4097), (8, 128, 4096), (8, 128, 4097), (8, 132, 4097), (3, 44, 200),
+                                          (2, 257, 130)])
+def test_gates_on_both_sides_of_the_rule(cuda, nb, bw, tokens):
+    """Narrow blocks, many workgroups of blocks up to 128, widths that are no multiple of 4: an output per lane; else four."""
+    test_gates_keep_all_bits_of_the_input(cuda, nb, bw, tokens, 1.0)
+
+
 def _gates(cuda, u, ra, rb, ri, ib, lam):
     tokens, nb, bw = u.shape
     a, y = (torch.full((tokens, nb * bw), float("nan"), device=cuda) for _ in range(2))
