@@ -1366,24 +1366,6 @@ __global__ void __launch_bounds__(256) sm_rglru_gates_kernel(float* __restrict__
   }
 }
 
-// e^x, 1 / (1 + e^-x) and the square root as exact as the library's, in half of its instructions.  e^x = 2^n 2^f, n the nearest integer
-// to x log2(e) and f what is left (log2(e) in two floats); infinities by the clamp, which NaN pass.  The quotient and the root off the
-// hardware's reciprocal and reciprocal root and a Newton step each, without the scaling that hipcc's have.
-__device__ __forceinline__ float exp_near(float x) {
-  x = __builtin_elementwise_minimum(__builtin_elementwise_maximum(x, -1000.f), 1000.f);
-  const float n = rintf(x * 1.44269502f);
-  const float f = fmaf(x, 1.92596300e-8f, fmaf(x, 1.44269502f, -n));
-  return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(f), (int)n);
-}
-__device__ __forceinline__ float sigmoid_near(float x) {
-  const float d = 1.0f + exp_near(-x), q = __builtin_amdgcn_rcpf(d);
-  return d < __builtin_inff() ? fmaf(q, fmaf(-d, q, 1.0f), q) : q;
-}
-__device__ __forceinline__ float sqrt_near(float x) {          // x <= 0: 0
-  const float y = __builtin_amdgcn_rsqf(x), s = x * y;
-  return x > 0.f ? fmaf(fmaf(-s, s, x), 0.5f * y, s) : 0.f * x;
-}
-
 // The same products for bf16 gate matrices on the bf16 matrix cores, as exact as on the float32 ones: u = h + m + l in three
 // bf16 pieces (8 significant bits each, 24 in all: nothing of u is lost), each times the bf16 weight an exact product, the
 // sums in float32.  Three products at 16 times the rate: 20 us of them, beside which the vector work (taking u apart, putting
@@ -1392,9 +1374,12 @@ __device__ __forceinline__ float sqrt_near(float x) {          // x <= 0: 0
 // per block, the weights come in 8-byte loads a k-step of 16 ahead (8 rows of them make four fragments in 16 v_perm), u, a and g
 // in 16-byte ones.  The pieces of u pass through LDS in K chunks of kSK, two of them (rows kSP apart: the 16 byte reads of 8
 // rows fall on banks of their own); two workgroups share a CU, one's vector work under the other's products.
-// us, 10 blocks of 256, 6376 / 3000 / 300 tokens: 127 / 65 / 41 with an output per lane (weights two bytes at a time), u taken apart for
-// 128 outputs and the library's functions, 83 / 45 / 24 here (275 on the float32 matrix cores at 6376); 4 blocks, 2000 / 168: 43 / 39 ->
-// 26 / 23.  Largest error of a and g against 64 bits there 5.4e-7 and 8.1e-6, means 1.8e-8 and 2.8e-8, as before.
+// The gates' functions are those of the other kernels (sigmoid_f, sqrtf): a and g have the same bits whichever kernel the alignment
+// and the rule below choose.  (Quotient and root off the hardware's approximations and a Newton step each: 83 us for 94, but 1 % of
+// a and 2 % of g another last bit.  With a second step and the remainder all bits were there, in 93 us.)
+// us, 10 blocks of 256, 6376 / 3000 / 300 tokens: 126 / 64 / 40 with an output per lane (weights two bytes at a time) and u taken apart
+// for 128 outputs, 94 / 50 / 27 here (275 on the float32 matrix cores at 6376); 4 blocks, 2000 / 168: 42 / 39 -> 28 / 26.  Largest
+// error of a and g against 64 bits there 5.4e-7 and 8.1e-6, means 1.8e-8 and 2.8e-8, as before.
 // Blocks a multiple of 4 wide, 16-byte aligned.
 constexpr int kST = 64;       // tokens per workgroup
 constexpr int kSO = 256;      // outputs
@@ -1557,8 +1542,8 @@ __global__ void __launch_bounds__(256, 2) sm_rglru_gates_split_kernel(
       f32x4 av, gv;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        av[j] = expf(-scale * sigmoid_near(cr[j][i] + rb[j]) * sp[j]);
-        gv[j] = sqrt_near(1.0f - av[j] * av[j]) * sigmoid_near(ci[j][i] + ib[j]) * ux[i][j];
+        av[j] = expf(-scale * sigmoid_f(cr[j][i] + rb[j]) * sp[j]);
+        gv[j] = sqrtf(1.0f - av[j] * av[j]) * sigmoid_f(ci[j][i] + ib[j]) * ux[i][j];
       }
       const int at = ((r + i) * C + b * bw + o) * 4;
       __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, av), rsa, at, 0, 0);
@@ -1575,10 +1560,10 @@ __global__ void __launch_bounds__(256, 2) sm_rglru_gates_split_kernel(
 
 // The same sums with an output per lane and 32 per wave, 128 tokens by 128 outputs per workgroup, u and the weights element by
 // element: any width and alignment, and no lane idle from blocks of 128 on.  Bound by its vector work and by two-byte loads.
-// Which kernel, us, this / the one above: widths that are no multiple of 4 this (8 blocks of 255, 300 / 16000 tokens 41 / 266
-// against 59 / 503 element by element there); 8 blocks of 64, 128, 256: 2000 tokens 26 / 18, 32 / 22, 45 / 29; 8000 tokens 36 / 41,
-// 49 / 55, 116 / 85: blocks up to 128 leave half of the other's waves idle, which counts once the CUs hold two workgroups each;
-// 3 blocks of 24, 300 / 16000 tokens: 23 / 28, 27 / 44.
+// Which kernel, us, this / the one above: widths that are no multiple of 4 this (8 blocks of 255, 300 / 16000 tokens 41 / 257
+// against 59 / 503 element by element there); 8 blocks of 64, 128, 256: 2000 tokens 27 / 20, 31 / 23, 47 / 30; 4500 tokens 34 / 38,
+// 43 / 47, 94 / 66; 8000 36 / 47, 49 / 58, 115 / 86: blocks up to 128 leave half of the other's waves idle, which counts once the CUs
+// hold two workgroups each; 3 blocks of 24, 300 / 16000 tokens: 23 / 34, 27 / 52.
 constexpr int kCT = 128;      // tokens per workgroup
 
 __global__ void __launch_bounds__(256, 2) sm_rglru_gates_column_kernel(

@@ -105,3 +105,24 @@ def test_gates_see_the_last_bits_of_the_input(cuda, nb, bw):
     seen = (torch.exp(-gate(two)[1]) - want).abs() > tol
     chunk = torch.nn.functional.one_hot(at // 64, bw // 64).bool()
     assert ((seen[..., None] & chunk).sum(0).sum(1) > 0.5 * chunk.sum(0).sum(1)).all()
+
+
+@pytest.mark.parametrize("nb,bw,tokens", [(10, 256, 300), (4, 256, 168), (2, 132, 1001), (3, 48, 65), (1, 700, 130), (8, 128, 4096)])
+def test_gates_have_the_same_bits_on_either_kernel(cuda, nb, bw, tokens):
+    """Four outputs per lane, and an output per lane (which an input off its 16 bytes takes): the same products in the same order,
+    and the same functions of them, over gates that are nearly shut, half open and nearly open."""
+    g = torch.Generator().manual_seed(bw)
+    r = lambda *s, scale=1.0: (torch.randn(*s, generator=g) * scale).to(cuda)
+    u = r(tokens * nb * bw, scale=8.0)
+    off = torch.empty(u.numel() + 1, device=cuda)[1:].copy_(u)
+    assert u.data_ptr() % 16 == 0 and off.data_ptr() % 16 == 4
+    w = [r(nb, bw, bw, scale=bw ** -0.5).bfloat16() for _ in range(2)]
+    b = [r(nb, bw).bfloat16() for _ in range(3)]
+    out = []
+    for x in (u, off):
+        a, y = (torch.full((tokens, nb * bw), float("nan"), device=cuda) for _ in range(2))
+        _ext.kernels().sm_rglru_gates(a.data_ptr(), y.data_ptr(), x.data_ptr(), w[0].data_ptr(), b[0].data_ptr(), w[1].data_ptr(),
+                                      b[1].data_ptr(), b[2].data_ptr(), tokens, nb, bw, 8.0, 0, torch.cuda.current_stream().cuda_stream)
+        out.append((a, y))
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+    assert not out[0][0].isnan().any() and not out[0][1].isnan().any()
