@@ -47,23 +47,24 @@ struct CloseRow {
     }
   }
 
-  // Sum (SQ: centred sum of squares) of the row, places past K left out; `red`: CV floats of LDS, other ones every time.
+  // Sum (SQ: centred sum of squares) of the row, places past K left out, in the order of the launch of its own (seqmix.hip:
+  // the same four waves, the same places, wave 0 first); `red`: CV floats of LDS, other ones every time.
   template <bool SQ>
   static __device__ __forceinline__ float sum(const float (&v)[PV][4], float mean, int K, int wv, int lane, float* red) {
     float s = 0.f;
 #pragma unroll
     for (int k = 0; k < PV; ++k) {
-      float t = 0.f;
+      if (place(k, wv, lane) < K) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) t += SQ ? (v[k][j] - mean) * (v[k][j] - mean) : v[k][j];
-      s += place(k, wv, lane) < K ? t : 0.f;
+        for (int j = 0; j < 4; ++j) s += SQ ? (v[k][j] - mean) * (v[k][j] - mean) : v[k][j];
+      }
     }
     s = wave_sum(s);
     if (lane == 0) red[wv] = s;
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     const f32x4 r = *reinterpret_cast<const f32x4*>(red);
-    return (r[0] + r[1]) + (r[2] + r[3]);
+    return ((r[0] + r[1]) + r[2]) + r[3];
   }
 
   // The normed row into `h`; the new stream to memory from one workgroup.  `red`: 4 CV floats.

@@ -52,6 +52,12 @@ int stream_rows(int ncols, int K, bool glu, int xg) {
   return best;
 }
 
+// 8 waves for a plain product where up to three groups of its rows have a CU each: their K loop is over in one or two rounds; else
+// 4 (several workgroups per CU).  Which wave has which K-tiles is the order of the sums.
+bool stream_wide(int m, int ncols, int rg) {
+  return m <= 16 ? rg <= 3 && (ncols + rg * 8 - 1) / (rg * 8) <= 256 : rg == 2 && m <= 32;
+}
+
 // glu 0: y [M, N] = x w^T (+ bias);  1 / 2 / 3: y [M, N / 2], SiLU / clipped / gelu GLU of w = [gate; up] (+ bias).
 // 4: y [M, N] in float32, cap tanh(z / cap) of the rounded product z with cap = limit, z itself where that is not positive.
 // (A launch of their own read the rounded logits back and wrote 4 bytes each: 1.6 to 2 us of a step whose head's product takes
@@ -79,9 +85,7 @@ void gemm_stream(uintptr_t y, uintptr_t x, uintptr_t w, uintptr_t bias, int M, i
   }
   const int per = pair ? rg * 4 : rg * 8;
   const dim3 grid((ncols + per - 1) / per);
-  // 8 waves where up to three groups of plain rows have a CU each: their K loop is over in one or two rounds; else 4
-  // (several workgroups per CU)
-  const bool wide = !pair && (one ? rg <= 3 && grid.x <= 256 : rg == 2 && xg == 4);
+  const bool wide = !pair && stream_wide(M, ncols, rg);
 #define DLLM_ST_GO(RG_, XG_, GLU_, WV_)                                                                             \
   do {                                                                                                              \
     if (nt) hipLaunchKernelGGL((gemm_stream_kernel<RG_, XG_, GLU_, true, WV_>), grid, dim3(WV_ * 64), 0, s,         \

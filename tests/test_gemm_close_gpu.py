@@ -72,6 +72,32 @@ def test_close_product(cuda, kind, glu, n, k):
     assert bool(((y.double() - ref).abs() <= tol).all())
 
 
+# weight rows of a workgroup / 8 -> sizes of the plain product (with 8 waves, with 4) and of the GLU
+PLAIN = [(8, 512), (1528, 576), (2560, 2560), (2056, 1024), (6152, 2048), (4104, 1024), (4610, 2112), (8200, 1536), (6152, 2560)]
+GLUS = [(4096, 2048), (4096, 2560), (6146, 1024), (4104, 2560), (8192, 1024), (6152, 2560), (8200, 1088), (8206, 2560), (12296, 1024),
+        (15360, 2560)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["rms", "layer"])
+@pytest.mark.parametrize("n,k,glu", [(*s, False) for s in PLAIN] + [(*s, True) for s in GLUS])
+def test_close_product_has_the_bits_of_two_launches(cuda, kind, n, k, glu):
+    """Every split of the weight rows, both numbers of waves of a plain product, rows of one and of three pieces per lane: the
+    stream and the product of the close's own launch and the product's."""
+    x, o, kw = _args(kind, k, n % 16 == 0, n + k, "cuda")
+    g = torch.Generator("cuda").manual_seed(n)
+    w = (torch.randn(n, k, device="cuda", generator=g) * k ** -0.5).bfloat16()
+    b = torch.randn(n, device="cuda", generator=g).bfloat16() if glu and kind == "rms" else None
+    act = "" if not glu else "clipped" if kind == "rms" else "gelu"
+    r = gemm.close_product(kind, x, o, w, b, act, 0.7, kw["w_post"], kw["w_next"], kw["eps"], kw.get("mult", 1.0), 1.0 if kind == "rms" else 0.0,
+                           kw["bias"], kw.get("b_post"), kw.get("b_next"))
+    assert r is not None
+    f = sm.post_norm_add if kind == "rms" else sm.post_layer_norm_add
+    xr, h = f(x.clone(), o, **kw)
+    y = ops.linear(h, w) if not glu else sm.linear_clipped_glu(h, w, b, 0.7) if kind == "rms" else sm.linear_gelu_glu(h, w)
+    assert torch.equal(r[0], xr) and torch.equal(r[1], y)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind", ["rms", "layer"])
 def test_close_refused(cuda, kind):
