@@ -55,6 +55,8 @@ PYBIND11_MODULE(_C_kernels, m) {
   m.def("sm_post_layer_norm_add", &dllm::sm_post_layer_norm_add);
   m.def("sm_gelu_glu", &dllm::sm_gelu_glu);
   m.def("sm_post_norm_add", &dllm::sm_post_norm_add);
+  m.def("sm_post_norm_last", &dllm::sm_post_norm_last);
+  m.def("sm_post_norm_last_fits", &dllm::sm_post_norm_last_fits);
   m.def("sm_causal_conv", &dllm::sm_causal_conv);
   m.def("sm_rglru_gates", &dllm::sm_rglru_gates);
   m.def("sm_rglru_scan", &dllm::sm_rglru_scan);

@@ -127,6 +127,9 @@ void sm_rms_norm(uintptr_t y, uintptr_t x, uintptr_t w, int rows, int width, flo
 void sm_post_norm_add(uintptr_t x, uintptr_t o, int parts, uintptr_t bias, uintptr_t w_post, uintptr_t w_next, uintptr_t h,
                       int rows, int width, float eps, float mult, float offset, uintptr_t o2, float s1, float s2,
                       int f32, uintptr_t stream);
+bool sm_post_norm_last_fits(int width);
+void sm_post_norm_last(uintptr_t x, uintptr_t o, int parts, uintptr_t bias, uintptr_t w_post, uintptr_t w_next, uintptr_t h, int rows,
+                       int width, float eps, float mult, float offset, int f32, uintptr_t stream);
 void sm_causal_conv(uintptr_t y, uintptr_t u, long stride, uintptr_t w, uintptr_t bias, uintptr_t in_bias,
                     uintptr_t state, uintptr_t cu, uintptr_t positions, uintptr_t tok_seq, uintptr_t slots,
                     int tokens, int seqs, int C, int taps, int f32, int out_f32, int act, uintptr_t stream);

@@ -638,11 +638,15 @@ void sm_post_layer_norm_add(uintptr_t x, uintptr_t o, int parts, uintptr_t bias,
 // three-pass form above re-read o, x and the new x, with each pass's loads behind a block reduction).
 // parts > 0: o is the sum of that many split-K slabs [rows, width], rounded as the reduction of a split product rounds it.
 // 2560 wide, bf16: 16 rows 4.3 -> 3.2 us (bound by the launch and two reductions), 6376 rows 44 -> 35 us (5.6 TB/s).
-template <typename T, int V, int NV, bool SLABS>
+// LAST: h is the norm of the whole stack's output, which else is a launch of sm_rms_norm: the row passes through LDS (`row_s`,
+// width floats) into that kernel's lanes, so that its sum has the same order and h the same bits (a step of the small layer list takes
+// as long as with the close's own order).
+template <typename T, int V, int NV, bool SLABS, bool LAST = false>
 __device__ __forceinline__ void post_norm_row(float* red, float* __restrict__ x, const void* __restrict__ o_, int parts,
                                               const void* __restrict__ bias_, const void* __restrict__ wp_,
                                               const void* __restrict__ wn_, void* __restrict__ h_, int width, float eps,
-                                              float mult, float offset, const void* __restrict__ o2_, float s1, float s2) {
+                                              float mult, float offset, const void* __restrict__ o2_, float s1, float s2,
+                                              float* row_s = nullptr) {
   const size_t row = (size_t)blockIdx.x * width;
   float* xr = x + row;
   typedef T vec __attribute__((ext_vector_type(V)));
@@ -661,7 +665,16 @@ __device__ __forceinline__ void post_norm_row(float* red, float* __restrict__ x,
   vec ro[NV];
   if (!SLABS) load(ro, (const T*)o_ + row);
   load(rwp, wp_);
-  if (wn_) load(rwn, wn_);
+  typedef T vec8 __attribute__((ext_vector_type(8)));
+  constexpr int N8 = LAST ? (NV * V + 7) / 8 : 1;
+  vec8 rw8[N8];
+  auto at8 = [&](int k) { return min((k * 256 + (int)threadIdx.x) * 8, width - 8); };
+  if constexpr (LAST) {
+#pragma unroll
+    for (int k = 0; k < N8; ++k) rw8[k] = *reinterpret_cast<const vec8*>((const T*)wn_ + at8(k));
+  } else {
+    if (wn_) load(rwn, wn_);
+  }
   if (o2_) load(r2, (const T*)o2_ + row);
   if (bias_) load(rc, bias_);
   if constexpr (SLABS) {
@@ -700,8 +713,34 @@ __device__ __forceinline__ void post_norm_row(float* red, float* __restrict__ x,
         sq += xv[k][j] * xv[k][j];
       }
       stv<V>(xr + i, xv[k]);
-      if (!wn_ && h_) stv<V>((T*)h_ + row + i, xv[k]);
+      if constexpr (LAST) stv<V>(row_s + i, xv[k]);
+      else if (!wn_ && h_) stv<V>((T*)h_ + row + i, xv[k]);
     }
+  }
+  if constexpr (LAST) {
+    __syncthreads();
+    float y[N8][8];
+    float s8 = 0.f;
+#pragma unroll
+    for (int k = 0; k < N8; ++k) {
+      ldv<8>(row_s + at8(k), y[k]);
+      if ((k * 256 + (int)threadIdx.x) * 8 < width) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) s8 += y[k][j] * y[k][j];
+      }
+    }
+    s8 = block_sum<256>(s8, red);
+    const float inv8 = 1.0f / sqrtf(s8 / (float)width + eps);
+#pragma unroll
+    for (int k = 0; k < N8; ++k) {
+      const int i = (k * 256 + threadIdx.x) * 8;
+      if (i < width) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) y[k][j] = y[k][j] * inv8 * (offset + (float)rw8[k][j]);
+        stv<8>((T*)h_ + row + i, y[k]);
+      }
+    }
+    return;
   }
   if (!wn_) return;
   sq = block_sum<256>(sq, red);
@@ -735,6 +774,43 @@ __global__ void __launch_bounds__(256) sm_post_norm_slabs_kernel(float* __restri
                                                                  float s2) {
   __shared__ float red[16];
   post_norm_row<T, V, NV, true>(red, x, o, parts, bias, wp, wn, h, width, eps, mult, offset, o2, s1, s2);
+}
+
+template <typename T, int NV, bool SLABS>
+__global__ void __launch_bounds__(256) sm_post_norm_last_kernel(float* __restrict__ x, const void* __restrict__ o, int parts,
+                                                                int width, const void* __restrict__ bias,
+                                                                const void* __restrict__ wp, const void* __restrict__ wn,
+                                                                void* __restrict__ h, float eps, float mult, float offset) {
+  __shared__ float red[16];
+  __shared__ __attribute__((aligned(16))) float row_s[NV * 1024];
+  post_norm_row<T, 4, NV, SLABS, true>(red, x, o, parts, bias, wp, wn, h, width, eps, mult, offset, nullptr, 0.f, 0.f, row_s);
+}
+
+// The close of the last sublayer with the norm behind it, h in the bits of sm_rms_norm (widths of its row kernel).
+bool sm_post_norm_last_fits(int width) { return width % 8 == 0 && width <= 8192; }
+
+void sm_post_norm_last(uintptr_t x, uintptr_t o, int parts, uintptr_t bias, uintptr_t w_post, uintptr_t w_next, uintptr_t h, int rows,
+                       int width, float eps, float mult, float offset, int f32, uintptr_t stream) {
+  if (rows <= 0) return;
+  DLLM_HOST_CHECK(x && o && w_post && w_next && h && width > 0 && sm_post_norm_last_fits(width), "post_norm_last arguments");
+  DLLM_HOST_CHECK(parts >= 0 && (parts == 0 || !f32), "post_norm_last slabs");
+  const auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(rows), dim3(256), 0, (hipStream_t)stream, (float*)x, (const void*)o, parts, width,
+                       (const void*)bias, (const void*)w_post, (const void*)w_next, (void*)h, eps, mult, offset);
+  };
+#define SM_LAST(T, SLABS_)                                                    \
+  do {                                                                        \
+    if (width <= 1024) go(sm_post_norm_last_kernel<T, 1, SLABS_>);            \
+    else if (width <= 2048) go(sm_post_norm_last_kernel<T, 2, SLABS_>);       \
+    else if (width <= 3072) go(sm_post_norm_last_kernel<T, 3, SLABS_>);       \
+    else if (width <= 4096) go(sm_post_norm_last_kernel<T, 4, SLABS_>);       \
+    else go(sm_post_norm_last_kernel<T, 8, SLABS_>);                          \
+  } while (0)
+  if (f32) SM_LAST(float, false);
+  else if (parts > 0) SM_LAST(bf16, true);
+  else SM_LAST(bf16, false);
+#undef SM_LAST
+  DLLM_HIP_CHECK(hipGetLastError());
 }
 
 void sm_post_norm_add(uintptr_t x, uintptr_t o, int parts, uintptr_t bias, uintptr_t w_post, uintptr_t w_next, uintptr_t h,

@@ -374,12 +374,13 @@ class HybridStage(LayerListStage):
         last = self.head["final_norm"] if meta.logits_idx is None else None     # every row's logits: the last close makes their norm
         for i, (spec, w) in enumerate(zip(self.specs, self.layers)):
             o = self._attention(i, h, w, meta, sb) if spec["type"] == "attention" else self._rglru(i, h, w, sb)
-            nxt = self.layers[i + 1]["norm1"] if i + 1 < n else last
-            h = sm.Close("rms", h.x, o, w_post=w["norm1b"], eps=eps, mult=mult, w_next=w["norm2"] if spec.get("mlp") else nxt)
+            nxt, final = (self.layers[i + 1]["norm1"], False) if i + 1 < n else (last, True)
+            h = sm.Close("rms", h.x, o, w_post=w["norm1b"], eps=eps, mult=mult, w_next=w["norm2"] if spec.get("mlp") else nxt,
+                         final=final and not spec.get("mlp"))
             if spec.get("mlp"):
                 y = h.clipped_glu(w["w_gu"], w["b_gu"], spec["mlp"]["limit"])
                 h = sm.Close("rms", h.x, ops.linear_into_norm(y, w["w_down"]), w_post=w["norm2b"], eps=eps, mult=mult,
-                             bias=w["b_down"], w_next=nxt)
+                             bias=w["b_down"], w_next=nxt, final=final)
             if self.taps is not None:
                 h.input()
                 self.taps.append(h.x.clone())

@@ -137,14 +137,15 @@ def rms_norm_f32(x: torch.Tensor, w: torch.Tensor, eps: float, act_dtype, one_pl
 
 def post_norm_add(x: torch.Tensor, o, w_post: torch.Tensor, eps: float, mult: float,
                   bias: Optional[torch.Tensor] = None, w_next: Optional[torch.Tensor] = None, one_plus: bool = True,
-                  o2: Optional[torch.Tensor] = None, scales=(1.0, 1.0), plain_next: bool = False):
+                  o2: Optional[torch.Tensor] = None, scales=(1.0, 1.0), plain_next: bool = False, final: bool = False):
     """The close of a sublayer, fused: ``x += mult * rms_norm(o + bias) * (1 + w_post)`` in place on the
     float32 residual stream; with ``w_next`` also returns the next sublayer's input
     ``rms_norm(x) * (1 + w_next)`` in ``o``'s dtype (None otherwise).  ``one_plus`` False: both norm
     weights are plain (``* w``).  ``o2``: the sublayer's output is ``scales[0] * o + scales[1] * o2`` (two
     mixers side by side).  ``plain_next`` (without ``w_next``): the next sublayer reads the stream itself;
     returns it in ``o``'s dtype (the stream tensor when that is float32).  ``o`` may be a :class:`~.gemm.SplitKPartial`
-    (without ``o2``): its slabs are then summed in the same launch."""
+    (without ``o2``): its slabs are then summed in the same launch.  ``final``: ``w_next`` is the norm behind the last sublayer
+    and h has the bits of :func:`rms_norm_f32` (whose sum has another order than a close's)."""
     from .gemm import SplitKPartial
     off = 1.0 if one_plus else 0.0
     if not x.is_cuda:
@@ -164,6 +165,15 @@ def post_norm_add(x: torch.Tensor, o, w_post: torch.Tensor, eps: float, mult: fl
         _ck(o, "o")
     if tuple(o.shape) != tuple(x.shape) or (o2 is not None and (o2.shape != x.shape or o2.dtype != o.dtype or not o2.is_contiguous())):
         raise ValueError("post_norm_add: o / x shape mismatch")
+    if final and w_next is not None:
+        if o2 is None and _k().sm_post_norm_last_fits(width) and w_next.data_ptr() % 16 == 0:
+            h = torch.empty(t, width, dtype=o.dtype, device=x.device)
+            _k().sm_post_norm_last(x.data_ptr(), (part.ws if part is not None else o).data_ptr(), 0 if part is None else part.splits,
+                                   _ptr(bias), w_post.data_ptr(), w_next.data_ptr(), h.data_ptr(), t, width, float(eps), float(mult),
+                                   off, _f32flag(o), _stream())
+            return x, h
+        x, _ = post_norm_add(x, o if part is None else part, w_post, eps, mult, bias, None, one_plus, o2, scales)
+        return x, rms_norm_f32(x, w_next, eps, o.dtype, one_plus)
     h = None
     if w_next is not None or (plain_next and o.dtype != torch.float32):
         h = torch.empty(t, width, dtype=o.dtype, device=x.device)
@@ -280,7 +290,7 @@ class Close:
     def _product(self, w: torch.Tensor, bias: Optional[torch.Tensor], glu: str, limit: float) -> Optional[torch.Tensor]:
         from . import gemm
         kw, o = self._kw, self._o
-        if type(o) is not torch.Tensor or o.shape[0] != 1 or kw.get("w_next") is None:
+        if type(o) is not torch.Tensor or o.shape[0] != 1 or kw.get("w_next") is None or kw.get("final"):
             return None
         if self.kind == "rms":
             r = gemm.close_product("rms", self.x, o, w, bias, glu, limit, kw["w_post"], kw["w_next"], kw["eps"], kw["mult"], 1.0,
