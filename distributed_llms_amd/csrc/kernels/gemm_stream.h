@@ -63,6 +63,7 @@ struct CloseRow {
     if (lane == 0) red[wv] = s;
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");                             // (the barrier by itself keeps no load behind it)
     const f32x4 r = *reinterpret_cast<const f32x4*>(red);
     return ((r[0] + r[1]) + r[2]) + r[3];
   }
@@ -198,6 +199,7 @@ __device__ __forceinline__ void gemm_stream_body(bf16* __restrict__ Y, const bf1
       for (int b = 0; b < Row::kBarriers; ++b) __builtin_amdgcn_s_barrier();
     }
     __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
   }
   for (int i0 = 0; i0 < cnt; i0 += D) {
 #pragma unroll

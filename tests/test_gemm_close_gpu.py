@@ -151,3 +151,15 @@ def test_close_object(device, kind, rows, last, request):
     assert (y.double() - ref.double()).norm() <= 2.0 ** -7 * ref.double().norm()
     made = sm.Close.made(x, rh)
     assert made.input() is rh and torch.equal(made.linear(w), ref) and made.x is x
+
+
+def test_no_load_of_a_close_can_move_in_front_of_its_barrier():
+    """The barrier builtin orders nothing for the compiler: behind each one that ordinary LDS loads follow stands a clobber."""
+    import os
+    import re
+    import distributed_llms_amd
+    path = os.path.join(os.path.dirname(distributed_llms_amd.__file__), "csrc", "kernels", "gemm_stream.h")
+    with open(path) as f:
+        code = re.sub(r"//[^\n]*", "", f.read())
+    behind = [code[m.end():].split(";")[0].strip() for m in re.finditer(r"^\s*__builtin_amdgcn_s_barrier\(\);", code, re.M)]
+    assert len(behind) == 2 and all(b == 'asm volatile("" ::: "memory")' for b in behind)
