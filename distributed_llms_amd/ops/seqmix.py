@@ -266,12 +266,13 @@ class Close:
     """The close of a sublayer that is still to be made, for the product that reads it: ``kind`` "rms" with the arguments of
     :func:`post_norm_add` or "layer" with those of :func:`post_layer_norm_add`.  The product makes it in its own launch where
     that is the faster way (:func:`~.gemm.close_product`: a single row); ``x`` is the new stream from then on (a tensor of its
-    own or the old one, updated in place)."""
+    own or the old one, updated in place).  One product reads a Close: inside its launch the normed rows never reach memory, so
+    that a second one, or :meth:`input`, is refused then.  What several read asks for :meth:`input` first."""
 
-    __slots__ = ("kind", "x", "h", "_o", "_kw")
+    __slots__ = ("kind", "x", "h", "_o", "_kw", "_taken")
 
     def __init__(self, kind: str, x: torch.Tensor, o, **kw):
-        self.kind, self.x, self.h, self._o, self._kw = kind, x, None, o, kw
+        self.kind, self.x, self.h, self._o, self._kw, self._taken = kind, x, None, o, kw, False
 
     @classmethod
     def made(cls, x: torch.Tensor, h: torch.Tensor) -> "Close":
@@ -282,6 +283,8 @@ class Close:
 
     def input(self) -> Optional[torch.Tensor]:
         """The next sublayer's input (None behind the last one), made by a launch of its own unless it is there."""
+        if self._taken:
+            raise RuntimeError("Close: a product has made this sublayer's input in its own launch; ask for input() before it")
         if self._o is not None:
             self.x, self.h = (post_norm_add if self.kind == "rms" else post_layer_norm_add)(self.x, self._o, **self._kw)
             self._o = None
@@ -301,7 +304,7 @@ class Close:
         if r is None:
             return None
         self.x, y = r
-        self._o = None
+        self._o, self._taken = None, True
         return y
 
     def linear(self, w: torch.Tensor) -> torch.Tensor:

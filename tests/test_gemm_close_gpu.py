@@ -131,7 +131,7 @@ def test_close_refused(cuda, kind):
 @pytest.mark.parametrize("last", [False, True])
 def test_close_object(device, kind, rows, last, request):
     """Close gives the stream and the product that the calls of their own give, whichever way it takes (one rounding of h and
-    one of the product apart at most), once: a second product reads the same input."""
+    one of the product apart at most)."""
     if device == "cuda":
         request.getfixturevalue("cuda")
     k, n = 1024, 256
@@ -163,3 +163,25 @@ def test_no_load_of_a_close_can_move_in_front_of_its_barrier():
         code = re.sub(r"//[^\n]*", "", f.read())
     behind = [code[m.end():].split(";")[0].strip() for m in re.finditer(r"^\s*__builtin_amdgcn_s_barrier\(\);", code, re.M)]
     assert len(behind) == 2 and all(b == 'asm volatile("" ::: "memory")' for b in behind)
+
+
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("kind", ["rms", "layer"])
+def test_close_is_read_by_one_product(monkeypatch, device, kind, request):
+    """Behind a product that made the row in its launch there is no input to read: an error, not a product of nothing.  With
+    the input asked for first any number of products read it."""
+    if device == "cuda":
+        request.getfixturevalue("cuda")
+    x, o, kw = _args(kind, 1024, True, 5, device)
+    w = (torch.randn(256, 1024, generator=torch.Generator().manual_seed(6)) / 32).bfloat16().to(device)
+    if device == "cpu":
+        monkeypatch.setattr(gemm, "close_product", lambda kind, x, o, w, *a, **k: (x + 1, o @ w.t()))
+    c = sm.Close(kind, x.clone(), o, **kw)
+    c.linear(w)
+    for again in (c.input, lambda: c.linear(w)):
+        with pytest.raises(RuntimeError, match="input"):
+            again()
+    c = sm.Close(kind, x.clone(), o, **kw)
+    h = c.input()
+    y = c.linear(w)
+    assert c.input() is h and torch.equal(y, ops.linear(h, w)) and torch.equal(c.linear(w), y)
