@@ -293,11 +293,12 @@ class Close:
     def _product(self, w: torch.Tensor, bias: Optional[torch.Tensor], glu: str, limit: float) -> Optional[torch.Tensor]:
         from . import gemm
         kw, o = self._kw, self._o
-        if type(o) is not torch.Tensor or o.shape[0] != 1 or kw.get("w_next") is None or kw.get("final"):
+        if (type(o) is not torch.Tensor or o.shape[0] != 1 or kw.get("w_next") is None or kw.get("final")
+                or kw.get("o2") is not None):
             return None
         if self.kind == "rms":
-            r = gemm.close_product("rms", self.x, o, w, bias, glu, limit, kw["w_post"], kw["w_next"], kw["eps"], kw["mult"], 1.0,
-                                   kw.get("bias"))
+            r = gemm.close_product("rms", self.x, o, w, bias, glu, limit, kw["w_post"], kw["w_next"], kw["eps"], kw["mult"],
+                                   1.0 if kw.get("one_plus", True) else 0.0, kw.get("bias"))
         else:
             r = gemm.close_product("layer", self.x, o, w, bias, glu, limit, kw["w_post"], kw["w_next"], kw["eps"],
                                    o_bias=kw.get("bias"), b_post=kw["b_post"], b_next=kw["b_next"])

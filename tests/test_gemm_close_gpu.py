@@ -185,3 +185,15 @@ def test_close_is_read_by_one_product(monkeypatch, device, kind, request):
     h = c.input()
     y = c.linear(w)
     assert c.input() is h and torch.equal(y, ops.linear(h, w)) and torch.equal(c.linear(w), y)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("more", [{"one_plus": False}, {"o2": True, "scales": (0.5, 2.0)}, {"plain_next": True}, {"final": True}])
+def test_close_takes_every_argument_of_its_function(cuda, more):
+    """Plain norm weights in either launch; what only the function makes is left to it."""
+    x, o, kw = _args("rms", 1024, True, 7, "cuda")
+    w = (torch.randn(256, 1024, generator=torch.Generator().manual_seed(8)) / 32).bfloat16().cuda()
+    kw.update({k: o.flip(1).contiguous() if k == "o2" else v for k, v in more.items()})
+    xr, h = sm.post_norm_add(x.clone(), o, **kw)
+    c = sm.Close("rms", x.clone(), o, **kw)
+    assert torch.equal(c.linear(w), ops.linear(h, w)) and torch.equal(c.x, xr)
