@@ -8,9 +8,16 @@
 // The sums are in the order of the two launches (the row's places, and as many product waves with the same K-tiles as gemm_stream
 // has), so that the new stream and the product have their bits.  (Twice the product waves under a GLU of up to 128 rows a workgroup:
 // other bits, 4096 x 2560 8.3 for 8.9, but 8192 and 16384 x 2048 14.2 and 22.9 for 10.4 and 15.3.)
-// us, close + product -> this, cold weights: RMS norms 2048 x 1024 5.3 -> 4.0, 6144 x 1024 + clipped GLU 7.5 -> 6.1, 5120 x 2560
-// 9.9 -> 8.8, 15360 x 2560 + GLU 19.5 -> 18.1; layer norms 1536 x 1024 5.4 -> 4.2, 6144 x 1024 + gelu GLU 7.2 -> 6.3, 15360 x
-// 2560 19.4 -> 18.5.  More rows cost each workgroup as many times the arithmetic: 4 rows at best equal (6144 x 1024 7.1 / 7.1),
+// us, close + product -> this, cold weights, RMS norms with a clipped GLU or without, layer norms with a gelu GLU or without:
+//   K  512:  512 / 2048 4.4 / 4.7 -> 3.1 / 3.7, + GLU 3072 5.4 -> 4.3;  4.8 / 5.1 -> 3.5 / 4.0, 5.5 -> 4.5
+//   K 1024:  2048 / 8192 5.1 / 7.1 -> 4.0 / 6.3, + GLU 6144 7.0 -> 6.0;  1536 5.4 -> 4.2, 7.1 -> 6.3
+//   K 1536:  1536 / 4608 5.5 / 7.4 -> 4.8 / 6.5, + GLU 9216 10.5 -> 9.8;  6.0 / 7.7 -> 5.3 / 7.2, 10.7 -> 10.3
+//   K 2048:  2048 / 6144 6.6 / 9.2 -> 5.8 / 8.7, + GLU 16384 17.3 -> 15.7;  7.0 / 9.6 -> 6.4 / 9.4, 17.4 -> 15.2
+//   K 2560:  2560 / 5120 7.7 / 9.8 -> 6.5 / 8.8, + GLU 15360 19.0 -> 18.1;  8.2 / 10.2 -> 7.2 / 9.5, 19.2 -> 18.5
+//   K 3072:  3072 / 9216 8.4 / 15.1 -> 7.4 / 13.7, + GLU 8192 / 16384 13.7 / 22.3 -> 12.8 / 21.4;  8.9 / 15.5 -> 8.0 / 14.5, 22.5 -> 21.9
+// and every size between and past them that was tried (160, to 96 Mi weights) as fast at least.  Wider rows, in four pieces, win as
+// much in most products (4096 x 4096 10.9 -> 10.3, 22016 x 4096 + GLU 35.7 -> 33.4), but some GLUs, where a few CUs have a second
+// workgroup, lose: 18432 x 3584 26.7 -> 29.5, 14336 / 16384 / 18432 x 4096 27.0 / 28.9 / 31.0 -> 29.3 / 31.3 / 32.2.  More rows cost each workgroup as many times the arithmetic: 4 rows at best equal (6144 x 1024 7.1 / 7.1),
 // 2560 wide slower (15360 19.3 / 19.8), so that the launch of its own is kept for them.
 #include "gemm_stream.h"
 #include "launchers.h"
@@ -27,12 +34,13 @@ __global__ void __launch_bounds__((WAVES + CV) * 64) gemm_close_kernel(bf16* __r
 int stream_rows(int ncols, int K, bool glu, int xg);
 bool stream_wide(int m, int ncols, int rg);
 
-// kind 1: RMS norms * (offset + w) (glu 0 or 2), 2: layer norms * w + b (glu 0 or 3); ob, bias: may be 0
-void gemm_close(uintptr_t y, uintptr_t w, uintptr_t bias, int N, int K, int glu, float limit, int kind, uintptr_t x, uintptr_t o,
+// kind 1: RMS norms * (offset + w) (glu 0 or 2), 2: layer norms * w + b (glu 0 or 3); ob, bias: may be 0; nt: nontemporal weight
+// loads.  Rows of one piece of 4 elements per lane (K <= 1024) or of up to three (3072).
+void gemm_close(uintptr_t y, uintptr_t w, uintptr_t bias, int N, int K, int glu, int nt, float limit, int kind, uintptr_t x, uintptr_t o,
                 uintptr_t ob, uintptr_t wp, uintptr_t bp, uintptr_t wn, uintptr_t bn, uintptr_t xo, float eps, float mult,
                 float offset, uintptr_t stream) {
   DLLM_HOST_CHECK(kind == kRmsClose || kind == kLayerClose, "kind 1 or 2");
-  DLLM_HOST_CHECK(K >= SK && K % SK == 0 && K <= 2560, "K: multiples of 64 up to 2560");
+  DLLM_HOST_CHECK(K >= SK && K % SK == 0 && K <= 3072, "K: multiples of 64 up to 3072");
   DLLM_HOST_CHECK(glu == 0 || glu == (kind == kRmsClose ? 2 : 3), "a clipped GLU behind RMS norms, a gelu GLU behind layer norms");
   DLLM_HOST_CHECK(N >= 1 && (glu == 0 || N % 2 == 0), "N");
   DLLM_HOST_CHECK(x && o && wp && wn && xo && x != xo && (kind != kLayerClose || (bp && bn)), "close operands");
@@ -46,8 +54,11 @@ void gemm_close(uintptr_t y, uintptr_t w, uintptr_t bias, int N, int K, int glu,
     hipLaunchKernelGGL(kern, dim3((ncols + per - 1) / per), dim3((waves + CV) * 64), 0, s, (bf16*)y, (const bf16*)w,
                        (const bf16*)bias, N, K, limit, c);
   };
-  // nontemporal weights as ops/gemm asks for them elsewhere: not where the whole of a model's stays in the Infinity Cache
-#define DLLM_CL_R(RG_, GLU_, CL_, KM_, WV_)                                                                                  go(gemm_close_kernel<RG_, GLU_, (GLU_ != 0 || KM_ > 1024), WV_, CL_, KM_>, GLU_ ? RG_ * 4 : RG_ * 8, WV_)
+#define DLLM_CL_R(RG_, GLU_, CL_, KM_, WV_)                                                                               \
+  do {                                                                                                                    \
+    if (nt) go(gemm_close_kernel<RG_, GLU_, true, WV_, CL_, KM_>, GLU_ ? RG_ * 4 : RG_ * 8, WV_);                         \
+    else go(gemm_close_kernel<RG_, GLU_, false, WV_, CL_, KM_>, GLU_ ? RG_ * 4 : RG_ * 8, WV_);                           \
+  } while (0)
 #define DLLM_CL_P(CL_, KM_)                                                                                               \
   do {                                                                                                                    \
     if (rg == 1) DLLM_CL_R(1, 0, CL_, KM_, 8);                       /* (a second round is never worth eight rows) */     \
@@ -59,18 +70,18 @@ void gemm_close(uintptr_t y, uintptr_t w, uintptr_t bias, int N, int K, int glu,
   } while (0)
 #define DLLM_CL_G(GLU_, CL_, KM_)                                                                                         \
   do {                                                                                                                    \
-    if (rg == 2) DLLM_CL_R(2, GLU_, CL_, KM_, 4);                                                                            \
-    else if (rg == 3) DLLM_CL_R(3, GLU_, CL_, KM_, 4);                                                                       \
-    else if (rg == 4) DLLM_CL_R(4, GLU_, CL_, KM_, 4);                                                                       \
-    else if (rg == 6) DLLM_CL_R(6, GLU_, CL_, KM_, 4);                                                                       \
-    else DLLM_CL_R(8, GLU_, CL_, KM_, 4);                                                                                    \
+    if (rg == 2) DLLM_CL_R(2, GLU_, CL_, KM_, 4);                                                                         \
+    else if (rg == 3) DLLM_CL_R(3, GLU_, CL_, KM_, 4);                                                                    \
+    else if (rg == 4) DLLM_CL_R(4, GLU_, CL_, KM_, 4);                                                                    \
+    else if (rg == 6) DLLM_CL_R(6, GLU_, CL_, KM_, 4);                                                                    \
+    else DLLM_CL_R(8, GLU_, CL_, KM_, 4);                                                                                 \
   } while (0)
 #define DLLM_CL_K(CL_, GLU_)                                                                                              \
   do {                                                                                                                    \
     if (glu == 0 && K <= 1024) DLLM_CL_P(CL_, 1024);                                                                      \
-    else if (glu == 0) DLLM_CL_P(CL_, 2560);                                                                              \
+    else if (glu == 0) DLLM_CL_P(CL_, 3072);                                                                              \
     else if (K <= 1024) DLLM_CL_G(GLU_, CL_, 1024);                                                                       \
-    else DLLM_CL_G(GLU_, CL_, 2560);                                                                                      \
+    else DLLM_CL_G(GLU_, CL_, 3072);                                                                                      \
   } while (0)
   if (kind == kRmsClose) DLLM_CL_K(kRmsClose, 2);
   else DLLM_CL_K(kLayerClose, 3);

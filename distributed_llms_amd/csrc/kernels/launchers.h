@@ -42,7 +42,7 @@ void gemm_pf(uintptr_t c, uintptr_t a, uintptr_t b, int M, int N, int K, int mod
              float limit, int bm, uintptr_t bias, int wgs);
 void gemm_pf8(uintptr_t c, uintptr_t a, uintptr_t a_scale, uintptr_t b, uintptr_t b_scale, int M, int N, int K, int mode, int bm,
               uintptr_t stream);
-void gemm_close(uintptr_t y, uintptr_t w, uintptr_t bias, int N, int K, int glu, float limit, int kind, uintptr_t x, uintptr_t o,
+void gemm_close(uintptr_t y, uintptr_t w, uintptr_t bias, int N, int K, int glu, int nt, float limit, int kind, uintptr_t x, uintptr_t o,
                 uintptr_t ob, uintptr_t wp, uintptr_t bp, uintptr_t wn, uintptr_t bn, uintptr_t xo, float eps, float mult,
                 float offset, uintptr_t stream);
 void gemm_stream(uintptr_t y, uintptr_t x, uintptr_t w, uintptr_t bias, int M, int N, int K, int glu, int nt, float limit,

@@ -276,7 +276,7 @@ def linear_into_norm(x: torch.Tensor, w: torch.Tensor):
     return _linear(m, n, k, x, w, None, True)
 
 
-CLOSE_MAX_WIDTH = 2560             # (csrc/kernels/gemm_close.hip: one row in the registers of four waves)
+CLOSE_MAX_WIDTH = 3072             # (csrc/kernels/gemm_close.hip: one row in the registers of four waves, and what more would cost)
 
 
 def close_product(kind: str, x: torch.Tensor, o: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], glu: str,
@@ -289,9 +289,7 @@ def close_product(kind: str, x: torch.Tensor, o: torch.Tensor, w: torch.Tensor, 
     n, k = w.shape if w.dim() == 2 else (0, 0)
     if not (knobs.K.stream and x.is_cuda and k <= CLOSE_MAX_WIDTH and x.shape == o.shape == (1, k) and x.dtype == torch.float32
             and w.dtype == torch.bfloat16 and glu in ("", "clipped" if kind == "rms" else "gelu") and (not glu or n % 2 == 0)
-            and stream_fits(1, n, k, glu, False, bias is not None)
-            # (the builds' cache policy of the weights)
-            and (n * k * 2 >= WIDE_NT_MIN_BYTES) == bool(glu or k > 1024)):
+            and stream_fits(1, n, k, glu, False, bias is not None)):
         return None
     vecs = [t for t in (o, w_post, w_next, o_bias, b_post, b_next) if t is not None]
     if any(t.dtype != torch.bfloat16 or t.numel() != k or not t.is_contiguous() or t.device != x.device or t.data_ptr() % 8
@@ -304,7 +302,7 @@ def close_product(kind: str, x: torch.Tensor, o: torch.Tensor, w: torch.Tensor, 
     y = torch.empty(1, n // 2 if glu else n, dtype=torch.bfloat16, device=x.device)
     xo = torch.empty_like(x)
     p = lambda t: 0 if t is None else t.data_ptr()
-    _ext.kernels().gemm_close(y.data_ptr(), w.data_ptr(), p(bias), n, k, _STREAM_GLU[glu], float(limit), 1 if kind == "rms" else 2,
+    _ext.kernels().gemm_close(y.data_ptr(), w.data_ptr(), p(bias), n, k, _STREAM_GLU[glu], 1 if n * k * 2 >= WIDE_NT_MIN_BYTES else 0, float(limit), 1 if kind == "rms" else 2,
                               x.data_ptr(), o.data_ptr(), p(o_bias), w_post.data_ptr(), p(b_post), w_next.data_ptr(), p(b_next),
                               xo.data_ptr(), float(eps), float(mult), float(offset), current_stream())
     return xo, y
