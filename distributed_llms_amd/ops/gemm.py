@@ -267,9 +267,12 @@ def use_stream(m: int, n: int, k: int, x: torch.Tensor, w: torch.Tensor, bias=No
 
 def linear_into_norm(x: torch.Tensor, w: torch.Tensor):
     """``x w^T`` for a consumer that sums split-K slabs itself (post_norm_add, post_layer_norm_add): the finished product
-    where the weight-streaming kernel is faster than the split grid alone, else possibly a :class:`SplitKPartial`.  One row
-    that :func:`close_product` can take is finished wherever that kernel serves a plain product (2560 x 7680, the close and a
-    5120 x 2560 product: 19.8 us in three launches of which the second sums slabs, 17.8 in two)."""
+    where the weight-streaming kernel is faster than the split grid alone, else possibly a :class:`SplitKPartial`.  One row of
+    a width that :func:`close_product` takes is finished wherever that kernel serves a plain product, also where the close then
+    has a launch of its own (a latent layer's, the last one, one behind a product that is not fused).  us, with slabs / finished
+    / finished and the close in the next product: 2560 x 7680 and 5120 x 2560 behind it 20.1 / 18.7 / 17.7, 2560 x 4096 17.7 /
+    15.9 / 15.0, 2048 x 8192 and 4096 x 2048 18.5 / 16.3 / 16.0, 1536 x 6144 and 3072 x 1536 14.0 / 12.8 / 12.2, 1024 x 8192 and
+    2048 x 1024 12.8 / 12.2 / 11.1, 3072 x 3072 and 4608 x 3072 18.1 / 15.3 / 14.5, 3072 x 8192 and 9216 x 3072 28.5 / 27.5 / 26.2."""
     m, n, k = _sizes(x, w, "linear_into_norm")
     if m <= STREAM_MAX_M and use_stream(m, n, k, x, w, defer=m > 1 or n > CLOSE_MAX_WIDTH):
         return _stream(m, n, k, x, w)
