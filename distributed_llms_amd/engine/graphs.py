@@ -26,8 +26,8 @@ class StagingRing:
     """Pinned host buffers for the inputs of successive steps, used in turn.  A buffer may be written again once its copy to the
     device is done; an event behind every copy says so, but holds the stream for 5 us between the copy and the step's graph
     (195 us a step of a small model for one request), so that one is recorded for half of the ring at a time, and for the copies
-    of a stream that the next step leaves.  ``torch.cuda`` streams live as long as the process; on a caller's own (an
-    ExternalStream, which may be gone by the next step) every copy has its event."""
+    of a stream that the next step leaves.  Only the default stream and those that the runner's owner keeps as long as the runner
+    (:meth:`keep`) are known to be there then; on any other, which may be gone by the next step, every copy has its event."""
 
     BUFFERS = 8
 
@@ -38,8 +38,12 @@ class StagingRing:
         self.arrays = self.buffers.numpy()
         self.at = 0
         self.done = ([], [])             # per half of the ring: the events behind its copies
-        self.open = None                 # (handle, stream) of copies that no event covers yet
-        self.known = None                # (handle, stream): of the last step, the object is costly to make
+        self.lasting = {}                # handle -> stream: the default one and the owner's
+        self.open = None                 # the lasting stream with copies that no event covers yet
+
+    def keep(self, stream):
+        """``stream`` outlives this ring (the engine's own)."""
+        self.lasting[stream.cuda_stream] = stream
 
     def take(self) -> int:
         """Index of the next buffer, free to be written."""
@@ -56,14 +60,14 @@ class StagingRing:
         half = self.BUFFERS // 2
         events = self.done[self.at // half]
         handle = current_stream()
-        if self.known is None or self.known[0] != handle:
-            self.known = (handle, torch.cuda.current_stream())
-        if self.open is not None and self.open[0] != handle:
-            events.append(self._event(self.open[1]))
-        self.open = self.known
-        own = handle == 0 or self.known[1].stream_id & 1                # (torch's encoding: its own streams are odd)
-        if self.at % half == half - 1 or not own:
-            events.append(self._event(self.known[1]))
+        if handle == 0 and 0 not in self.lasting:
+            self.lasting[0] = torch.cuda.current_stream()
+        stream = self.lasting.get(handle)
+        if self.open is not None and self.open is not stream:
+            events.append(self._event(self.open))
+        self.open = stream
+        if self.at % half == half - 1 or stream is None:
+            events.append(self._event(torch.cuda.current_stream() if stream is None else stream))
             self.open = None
         self.at = (self.at + 1) % self.BUFFERS
 

@@ -90,6 +90,8 @@ class LLMEngine:
         if gpu:
             dev = self.stage.device
             self.streams = [torch.cuda.Stream(dev) for _ in range(self.num_slots)]
+            for graphs, s in zip(self.runner.graph_sets, self.streams):
+                graphs.staging.keep(s)
             # two pinned token buffers + events per slot: with lookahead two steps of a slot are in flight
             self.tok_host = [[torch.empty(max(ecfg.max_batch, 1), dtype=torch.int32).pin_memory() for _ in range(2)]
                              for _ in range(self.num_slots)]

@@ -10,7 +10,7 @@ from distributed_llms_amd.engine import graphs
 
 class _Stream:
     def __init__(self, handle, sid):
-        self.handle, self.stream_id, self.issued = handle, sid, []
+        self.cuda_stream, self.stream_id, self.issued = handle, sid, []
 
 
 class _Event:
@@ -24,33 +24,36 @@ class _Event:
         self.log |= self.covers
 
 
+@pytest.mark.parametrize("ids", [(0, 3, 5, 8), (0, 4, 6, 9)])               # (whatever a stream's id says about its kind)
 @pytest.mark.parametrize("seed", range(6))
-def test_buffers_are_reused_behind_their_copies(monkeypatch, seed):
-    """Random walks over the default stream, two of torch's and an external one (never recorded on after its step)."""
+def test_buffers_are_reused_behind_their_copies(monkeypatch, seed, ids):
+    """Random walks over the default stream, two that the owner keeps and a caller's (never recorded on after its step)."""
     rng, done, events = random.Random(seed), set(), []
-    streams = [_Stream(0, 0), _Stream(11, 3), _Stream(12, 5), _Stream(13, 8)]
-    now = [streams[0]]
-    monkeypatch.setattr(graphs, "current_stream", lambda: now[0].handle)
+    streams = [_Stream(h, i) for h, i in zip((0, 11, 12, 13), ids)]
+    now = [streams[seed % 3]]
+    monkeypatch.setattr(graphs, "current_stream", lambda: now[0].cuda_stream)
     monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: now[0])
 
     def event(stream):
-        assert stream is now[0] or stream.stream_id != 8
+        assert stream is now[0] or stream is not streams[3]
         e = _Event(done)
         e.record(stream)
         events.append(e)
         return e
     monkeypatch.setattr(graphs.StagingRing, "_event", staticmethod(event))
     ring, last = graphs.StagingRing(4), {}
+    for s in streams[1:3]:
+        ring.keep(s)
     steps = 400
     for step in range(steps):
-        if rng.random() < (0.0, 0.02, 0.1, 0.3, 0.9, 0.5)[seed]:
+        if rng.random() < (0.0, 0.0, 0.1, 0.3, 0.9, 0.02)[seed]:
             now[0] = rng.choice(streams)
         buf = ring.take()
         assert buf not in last or last[buf] in done, (step, buf)
         last[buf] = step
         now[0].issued.append(step)
         ring.sent()
-    if seed == 0:
+    if seed < 2:
         assert len(events) == steps // (ring.BUFFERS // 2)
 
 
@@ -69,6 +72,7 @@ def test_host_runs_ahead_of_replays(cuda):
     eng = LLMEngine(EngineConfig(model=name, dtype="bfloat16", device="cuda", max_batch=2, max_seq_len=256, num_kv_blocks=64,
                                  graph_batch_sizes=(2,)), stage)
     steps, other = 3 * graphs.StagingRing.BUFFERS + 1, torch.cuda.Stream()
+    assert eng.streams[0].cuda_stream in eng.runner.graphs.staging.lasting
 
     def run(ahead):
         rp = TraceReplayer(eng)
