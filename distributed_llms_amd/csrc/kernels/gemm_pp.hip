@@ -61,7 +61,8 @@ __device__ __forceinline__ void pp_wait_n(int younger) {   // younger: compile-t
 
 // One MFMA of accumulator row R.  The rows past the 8th (row tiles of 288) do not fit the 256 accumulation registers and stay in
 // ordinary ones: in asm, since hipcc moves them to accumulation registers and back around each of its own (240 moves a K-tile).
-// (Their operands come from LDS behind counted waits, and the sums are read behind a wait of their own at the end of the loop.)
+// (Their operands come from LDS behind counted waits, and the sums are read behind a wait of their own at the end of the loop.  A copy
+// that hipcc put in between would have none: tests/test_asm_mfma_waits.py reads the built code for one.)
 template <int R>
 __device__ __forceinline__ void pp_mfma(const bf16x8& b, const bf16x8& a, f32x4& acc) {
   if constexpr (R < 8) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, a, acc, 0, 0, 0);
