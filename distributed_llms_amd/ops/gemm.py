@@ -20,7 +20,7 @@ the engine on Llama-3-8B, profiles/wide_gemm.md; each one is a field of :mod:`..
   70B) at 225 <= M <= 256 on split gemm_pp 128-column tiles (profiles/round6_gate_up_pp.md);
 * prefill (M >= knobs.pp_swiglu_min_m / pp_proj_min_m, above the decode ranges): the 4-wave
   schedule-2 kernel in its persistent form (gemm_pf in gemm_pp.hip, knobs.pp_persistent; 256 x 256 tiles, or row tiles of
-  160 to 320 where they need fewer or cheaper rounds of the chip, :func:`pf_row_tile` and :func:`_pf_tall`) -- gate|up with the GLU (and a clipped
+  160 to 320 where they need fewer or cheaper rounds of the chip, :func:`_pf_tile`) -- gate|up with the GLU (and a clipped
   one's bias) in its epilogue, qkv / o / down plain (profiles/round4_gemm_counters.md);
 * what none of them takes (a bias or N not a multiple of 128 past 64 rows, K not a multiple of 64, fp32 on CPU,
   operands >= 4 GiB): torch's F.linear.
@@ -150,6 +150,12 @@ def _pf_plan(m: int, n: int, k: int, out: int, device) -> int:
             if out != n:
                 return pf_row_tile(m, n, device, _pf_wgs(_cus(device)))
     return 256 if pf_fills(m, n, device) else 0
+
+
+def _pf_tile(m: int, n: int, k: int, out: int, device) -> int:
+    """Row tile of the prompt products: :func:`_pf_plan`'s kernel, with the longer tile where :func:`_pf_tall` finds its walk cheaper."""
+    bm = _pf_plan(m, n, k, out, device)
+    return _pf_tall(bm, m, n, out, device) if bm else 0
 
 
 def _pf_wgs(cus: int) -> int:
@@ -388,9 +394,9 @@ def _linear(m: int, n: int, k: int, x: torch.Tensor, w: torch.Tensor, bias: Opti
     if bias is None and _use_wide(m, n, k, x, w):
         return linear_wide(x, w, defer=defer)
     if bias is None and _use_pp(m, n, k, x, w, knobs.K.pp_proj_min_m):
-        bm = _pf_plan(m, n, k, n, x.device)
+        bm = _pf_tile(m, n, k, n, x.device)
         if bm:
-            return linear_pf(x, w, bm=_pf_tall(bm, m, n, n, x.device))
+            return linear_pf(x, w, bm=bm)
         # medium M (mixed prefill + decode steps, short prompts): split-K tiles fill the CUs
         return linear_pp(x, w, variant=PP_PREFILL_VARIANT, defer=defer)
     return F.linear(x, w, bias)
@@ -689,9 +695,9 @@ def _linear_glu(x: torch.Tensor, w_gate_up: torch.Tensor, limit: Optional[float]
     if x.dtype != torch.bfloat16 or n % 256 or (bias is not None and not _glu_bias(bias, n, x)):
         return None
     if not _use_wide(m, n, k, x, w_gate_up) and _use_pp(m, n, k, x, w_gate_up, knobs.K.pp_swiglu_min_m):
-        bm = _pf_plan(m, n, k, n // 2, x.device)
+        bm = _pf_tile(m, n, k, n // 2, x.device)
         if bm and not (bias is not None and (limit is None or _recorded(x, w_gate_up, bias))):
-            return linear_pf(x, w_gate_up, limit=limit, gelu=limit is None, bm=_pf_tall(bm, m, n, n // 2, x.device), bias=bias)
+            return linear_pf(x, w_gate_up, limit=limit, gelu=limit is None, bm=bm, bias=bias)
     if bias is not None:
         return None
     y = linear(x, w_gate_up, defer=True)
@@ -737,8 +743,8 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor) -> Optional[torch.Te
     if _use_wide(m, n, k, x, w_gate_up, swiglu=True):
         return linear_wide(x, w_gate_up, swiglu=True)
     if _use_pp(m, n, k, x, w_gate_up, knobs.K.pp_swiglu_min_m):
-        bm = _pf_plan(m, n, k, n // 2, x.device)
+        bm = _pf_tile(m, n, k, n // 2, x.device)
         if bm:
-            return linear_pf(x, w_gate_up, swiglu=True, bm=_pf_tall(bm, m, n, n // 2, x.device))
+            return linear_pf(x, w_gate_up, swiglu=True, bm=bm)
         return linear_pp(x, w_gate_up, swiglu=True, variant=PP_PREFILL_VARIANT)
     return None
