@@ -2137,9 +2137,11 @@ void sm_rglru_step(uintptr_t out, uintptr_t x, uintptr_t y, long ld, uintptr_t c
   if (seqs <= 0) return;
   DLLM_HOST_CHECK(nb > 0 && bw >= 8 && bw % 8 == 0 && bw <= 512 && (long)nb * bw <= (1L << 24), "rglru step block sizes");
   DLLM_HOST_CHECK(taps >= 1 && taps <= kStepTaps && ld >= (long)nb * bw, "rglru step sizes");
-  // sequences per workgroup: two halve the passes over the matrices, which the L2 bears while the grid is small (10 blocks
-  // of 256 at 16 / 24 sequences: 8.3 / 9.4 us with one, 9.1 / 9.5 with two; at 32 / 64 12.0 / 18.6 and 11.3 / 17.8)
-  const int gt = seqs <= 24 ? 1 : 2;
+  // sequences per workgroup: two halve the passes over the matrices, which the L2 bears while the grid is small.  us, one / two:
+  // 10 blocks of 256 at 16 / 28 / 32 sequences 7.3 / 9.8 / 10.7 and 8.4 / 10.2 / 10.4, 4 blocks of 256 at 32 6.5 and 7.0, 8 blocks of
+  // 64 5.0 and 6.2, 20 of 128 10.6 and 10.1; at 64 16.6, 8.2, 6.2, 16.0 and 16.8, 8.6, 6.2, 16.1; at 128 10 and 16 of 256 28.3, 41.9 and
+  // 26.4, 38.7
+  const int gt = seqs <= 32 ? 1 : 2;
   const int groups = (seqs + gt - 1) / gt;
   DLLM_HOST_CHECK(arrived != 0 && (long)num_slots * nb * kCountStride <= arrived_len && groups <= 65535, "rglru step counters");
   const size_t lds = ((size_t)(33 * 2 * gt * kStepOut + 32 * 4) + (size_t)gt * bw) * sizeof(float) +
