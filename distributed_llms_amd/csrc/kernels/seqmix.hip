@@ -1001,7 +1001,7 @@ void sm_token_shift(uintptr_t y, uintptr_t h, uintptr_t w, uintptr_t state, uint
 
 // --------------------------------------------------------------------------- causal convolution with state
 // (conv_input / conv_input_v, the reads of a token's earlier inputs, are in stream_common.h)
-template <typename T, typename OT, int V>
+template <typename T, typename OT, int V, int TAPS>
 __global__ void __launch_bounds__(256) sm_causal_conv_kernel(void* __restrict__ y_, const void* __restrict__ u_,
                                                              long stride, const void* __restrict__ w_,
                                                              const void* __restrict__ bias_,
@@ -1010,8 +1010,9 @@ __global__ void __launch_bounds__(256) sm_causal_conv_kernel(void* __restrict__ 
                                                              const int32_t* __restrict__ cu,
                                                              const int32_t* __restrict__ positions,
                                                              const int32_t* __restrict__ tok_seq,
-                                                             const int32_t* __restrict__ slots, int C, int taps,
+                                                             const int32_t* __restrict__ slots, int C, int taps_,
                                                              int act) {
+  const int taps = TAPS > 0 ? TAPS : taps_;
   const int t = blockIdx.x;
   const int b = tok_seq[t];
   const int tl = t - cu[b], pos = positions[t];
@@ -1027,26 +1028,26 @@ __global__ void __launch_bounds__(256) sm_causal_conv_kernel(void* __restrict__ 
     for (int j = 0; j < V; ++j) acc[j] = 0.f, ib[j] = 0.f;
     if (bias) ldv<V>(bias + c, acc);
     if (in_bias) ldv<V>(in_bias + c, ib);
-    if (taps <= kConvTaps) {                         // (uniform) every load at once, off a place that is always there
-      float xs[kConvTaps][V], ws[kConvTaps][V];
+    if constexpr (TAPS > 0) {                        // every load at once, off a place that is always there
+      float xs[TAPS][V], ws[TAPS][V];
 #pragma unroll
-      for (int j = 0; j < kConvTaps; ++j) {
-        const int jj = min(j, taps - 1), d = taps - 1 - jj;
-        ldv<V>(conv_row(u, stride, st, t, tl, d, taps, C) + c, xs[j]);
-        ldv<V>(w + (size_t)jj * C + c, ws[j]);
+      for (int j = 0; j < TAPS; ++j) {
+        ldv<V>(conv_row(u, stride, st, t, tl, TAPS - 1 - j, TAPS, C) + c, xs[j]);
+        ldv<V>(w + (size_t)j * C + c, ws[j]);
       }
 #pragma unroll
-      for (int j = 0; j < kConvTaps; ++j)
-        if (j < taps && taps - 1 - j <= pos) {       // (uniform)
+      for (int j = 0; j < TAPS; ++j)
+        if (TAPS - 1 - j <= pos) {                   // (uniform)
 #pragma unroll
           for (int e = 0; e < V; ++e) acc[e] += ws[j][e] * (xs[j][e] + ib[e]);
         }
-    } else
-    for (int j = 0; j < taps; ++j) {
-      if (!conv_input_v<T, V>(u, stride, st, t, tl, pos, taps - 1 - j, taps, c, C, xv)) continue;
-      ldv<V>(w + (size_t)j * C + c, wv);
+    } else {
+      for (int j = 0; j < taps; ++j) {
+        if (!conv_input_v<T, V>(u, stride, st, t, tl, pos, taps - 1 - j, taps, c, C, xv)) continue;
+        ldv<V>(w + (size_t)j * C + c, wv);
 #pragma unroll
-      for (int e = 0; e < V; ++e) acc[e] += wv[e] * (xv[e] + ib[e]);
+        for (int e = 0; e < V; ++e) acc[e] += wv[e] * (xv[e] + ib[e]);
+      }
     }
     if (act == 1) {                                  // silu, in float32 with the exact exponential
 #pragma unroll
@@ -1056,30 +1057,34 @@ __global__ void __launch_bounds__(256) sm_causal_conv_kernel(void* __restrict__ 
   }
 }
 
-// The same over many tokens, up to kConvTaps taps: a thread takes 8 channels of kConvRun tokens, whose rows overlap (7 rows and one
-// read of the weights for 4 tokens, 16 and 4 by themselves), all of them in one round trip where the run lies inside a sequence.
-// 6376 tokens x 2560 to float32: 37 us a token per workgroup and its rows one by one behind branches, 28 here.
+// The same over many tokens, 3 or 4 taps: a thread takes 8 channels of kConvRun tokens, whose rows overlap (7 rows and one read of the
+// weights for 4 tokens, 16 and 4 by themselves), all of them in one round trip where the run lies inside a sequence.
+// us with the state's launch, bf16 to float32: rows one by one behind branches / all at once (above) / runs.  4 taps: 8000 tokens x 2560
+// 46 / 41 / 31, 1000 x 5120 17.5 / 15.8 / 13.8, 4000 x 1024 15.6 / 13.9 / 12.8, but 1000 x 2560 11.4 / 10.6 / 10.2 (to bf16 9.9 / 9.1 /
+// 10.2), 500 x 5120 10.5 / 9.9 / 10.2 (9.6 / 9.2 / 10.2), 2000 x 1024 8.8 / 8.5 / 9.0: runs from some 100000 threads on, three
+// workgroups for two CUs.  3 taps 8000 x 5120 67 / 64 / 52.  2 taps share too little: 55 / 51 / 53, 1000 x 5120 to bf16 11.0 / 11.1 / 11.8.
 constexpr int kConvRun = 4;
+constexpr long kConvRunThreads = 256 * 384;
 
-template <typename T, typename OT>
+template <typename T, typename OT, int TAPS>
 __global__ void __launch_bounds__(256) sm_causal_conv_run_kernel(
     void* __restrict__ y_, const void* __restrict__ u_, long stride, const void* __restrict__ w_, const void* __restrict__ bias_,
     const void* __restrict__ in_bias_, const void* __restrict__ state_, const int32_t* __restrict__ cu,
-    const int32_t* __restrict__ positions, const int32_t* __restrict__ tok_seq, const int32_t* __restrict__ slots, int C, int taps,
-    int act, int tokens) {
+    const int32_t* __restrict__ positions, const int32_t* __restrict__ tok_seq, const int32_t* __restrict__ slots, int C, int act,
+    int tokens) {
   const long id = (long)blockIdx.x * 256 + threadIdx.x;
   const int t0 = (int)(id / (C / 8)) * kConvRun, c = (int)(id % (C / 8)) * 8;
   if (t0 >= tokens) return;
   const T* u = (const T*)u_ + c;
   const T* w = (const T*)w_ + c;
   const int t1 = min(t0 + kConvRun, tokens) - 1, b0 = tok_seq[t0], b1 = tok_seq[t1], tl0 = t0 - cu[b0];
-  float bias[8], ib[8], wv[kConvTaps][8];
+  float bias[8], ib[8], wv[TAPS][8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) bias[e] = ib[e] = 0.f;
   if (bias_) ldv<8>((const T*)bias_ + c, bias);
   if (in_bias_) ldv<8>((const T*)in_bias_ + c, ib);
 #pragma unroll
-  for (int j = 0; j < kConvTaps; ++j) ldv<8>(w + (size_t)min(j, taps - 1) * C, wv[j]);
+  for (int j = 0; j < TAPS; ++j) ldv<8>(w + (size_t)j * C, wv[j]);
   auto finish = [&](int t, float (&acc)[8]) {
     if (act == 1) {                                  // silu, in float32 with the exact exponential
 #pragma unroll
@@ -1087,10 +1092,10 @@ __global__ void __launch_bounds__(256) sm_causal_conv_run_kernel(
     }
     stv<8>((OT*)y_ + (size_t)t * C + c, acc);
   };
-  if (b0 == b1 && tl0 >= taps - 1) {
-    float x[kConvRun + kConvTaps - 1][8];            // row i: token t0 - (taps - 1) + i
+  if (b0 == b1 && tl0 >= TAPS - 1) {
+    float x[kConvRun + TAPS - 1][8];                 // row i: token t0 - (TAPS - 1) + i
 #pragma unroll
-    for (int i = 0; i < kConvRun + kConvTaps - 1; ++i) ldv<8>(u + (size_t)min(t0 - (taps - 1) + i, t1) * stride, x[i]);
+    for (int i = 0; i < kConvRun + TAPS - 1; ++i) ldv<8>(u + (size_t)min(t0 - (TAPS - 1) + i, t1) * stride, x[i]);
 #pragma unroll
     for (int q = 0; q < kConvRun; ++q) {
       if (t0 + q > t1) break;
@@ -1098,26 +1103,24 @@ __global__ void __launch_bounds__(256) sm_causal_conv_run_kernel(
 #pragma unroll
       for (int e = 0; e < 8; ++e) acc[e] = bias[e];
 #pragma unroll
-      for (int j = 0; j < kConvTaps; ++j)
-        if (j < taps) {                              // (uniform)
+      for (int j = 0; j < TAPS; ++j)
 #pragma unroll
-          for (int e = 0; e < 8; ++e) acc[e] += wv[j][e] * (x[q + j][e] + ib[e]);
-        }
+        for (int e = 0; e < 8; ++e) acc[e] += wv[j][e] * (x[q + j][e] + ib[e]);
       finish(t0 + q, acc);
     }
     return;
   }
   for (int t = t0; t <= t1; ++t) {
     const int b = tok_seq[t], tl = t - cu[b], pos = positions[t];
-    const T* st = (const T*)state_ + (size_t)slots[b] * (taps - 1) * C + c;
-    float acc[8], xs[kConvTaps][8];
+    const T* st = (const T*)state_ + (size_t)slots[b] * (TAPS - 1) * C + c;
+    float acc[8], xs[TAPS][8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc[e] = bias[e];
 #pragma unroll
-    for (int j = 0; j < kConvTaps; ++j) ldv<8>(conv_row(u, stride, st, t, tl, taps - 1 - min(j, taps - 1), taps, C), xs[j]);
+    for (int j = 0; j < TAPS; ++j) ldv<8>(conv_row(u, stride, st, t, tl, TAPS - 1 - j, TAPS, C), xs[j]);
 #pragma unroll
-    for (int j = 0; j < kConvTaps; ++j)
-      if (j < taps && taps - 1 - j <= pos) {
+    for (int j = 0; j < TAPS; ++j)
+      if (TAPS - 1 - j <= pos) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) acc[e] += wv[j][e] * (xs[j][e] + ib[e]);
       }
@@ -1180,25 +1183,37 @@ void sm_causal_conv(uintptr_t y, uintptr_t u, long stride, uintptr_t w, uintptr_
   const int per = 256 * (vec ? 8 : 1);
   const dim3 grid(tokens, std::min(8, (C + per - 1) / per));
   hipStream_t s = (hipStream_t)stream;
-#define SM_CONV(T, OT, V)                                                                                    \
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(sm_causal_conv_kernel<T, OT, V>), grid, dim3(256), 0, s, (void*)y, (const void*)u, \
+#define SM_CONV_N(T, OT, V, N)                                                                                         \
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(sm_causal_conv_kernel<T, OT, V, N>), grid, dim3(256), 0, s, (void*)y, (const void*)u, \
                      stride, (const void*)w, (const void*)bias, (const void*)in_bias, (const void*)state,     \
                      (const int32_t*)cu, (const int32_t*)positions, (const int32_t*)tok_seq, (const int32_t*)slots, C, taps, act)
-#define SM_CONV_RUN(T, OT)                                                                                           \
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(sm_causal_conv_run_kernel<T, OT>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, \
+#define SM_CONV_RUN(T, OT, N)                                                                                        \
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(sm_causal_conv_run_kernel<T, OT, N>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, \
                      (void*)y, (const void*)u, stride, (const void*)w, (const void*)bias, (const void*)in_bias,              \
                      (const void*)state, (const int32_t*)cu, (const int32_t*)positions, (const int32_t*)tok_seq,             \
-                     (const int32_t*)slots, C, taps, act, tokens)
-  // runs of tokens where these by themselves fill the chip (a workgroup on each CU)
+                     (const int32_t*)slots, C, act, tokens)
+#define SM_CONV_T(T, OT, N)                                                                                            \
+  do {                                                                                                                 \
+    if (N > 2 && runs) SM_CONV_RUN(T, OT, (N > 2 ? N : 3));                                                            \
+    else if (vec) SM_CONV_N(T, OT, 8, N);                                                                              \
+    else SM_CONV_N(T, OT, 1, N);                                                                                       \
+  } while (0)
+#define SM_CONV(T, OT)                                                                                                 \
+  do {                                                                                                                 \
+    if (taps == 2) SM_CONV_T(T, OT, 2);                                                                                \
+    else if (taps == 3) SM_CONV_T(T, OT, 3);                                                                           \
+    else if (taps == 4) SM_CONV_T(T, OT, 4);                                                                           \
+    else if (vec) SM_CONV_N(T, OT, 8, 0);                                                                              \
+    else SM_CONV_N(T, OT, 1, 0);                                                                                       \
+  } while (0)
   const long threads = (long)((tokens + kConvRun - 1) / kConvRun) * (C / 8);
-  if (vec && taps <= kConvTaps && threads >= 256 * 256) {
-    if (f32) SM_CONV_RUN(float, float);
-    else if (out_f32) SM_CONV_RUN(bf16, float);
-    else SM_CONV_RUN(bf16, bf16);
-  } else if (f32) { if (vec) SM_CONV(float, float, 8); else SM_CONV(float, float, 1); }
-  else if (out_f32) { if (vec) SM_CONV(bf16, float, 8); else SM_CONV(bf16, float, 1); }
-  else { if (vec) SM_CONV(bf16, bf16, 8); else SM_CONV(bf16, bf16, 1); }
+  const bool runs = vec && threads >= kConvRunThreads;
+  if (f32) SM_CONV(float, float);
+  else if (out_f32) SM_CONV(bf16, float);
+  else SM_CONV(bf16, bf16);
 #undef SM_CONV_RUN
+#undef SM_CONV_N
+#undef SM_CONV_T
 #undef SM_CONV
   DLLM_HIP_CHECK(hipGetLastError());
   if (taps > 1) launch_conv_state(state, u, stride, cu, positions, slots, seqs, C, taps, f32, vec, stream);

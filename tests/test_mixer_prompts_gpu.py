@@ -28,10 +28,11 @@ def _chunks(total, g):
 
 
 @pytest.mark.parametrize("dtype,out", [(torch.bfloat16, torch.float32), (torch.bfloat16, torch.bfloat16), (torch.float32, torch.float32)])
-@pytest.mark.parametrize("c,taps,act", [(2560, 4, None), (264, 3, "silu"), (2560, 1, None), (1024, 2, None), (1024, 5, None)])
+@pytest.mark.parametrize("c,taps,act", [(2560, 4, None), (264, 3, "silu"), (1024, 3, None), (2560, 1, None), (1024, 2, None), (1024, 5, None),
+                                        (37, 4, "silu"), (37, 2, None)])
 def test_causal_conv_of_runs_bit_exact(cuda, dtype, out, c, taps, act):
     g = torch.Generator().manual_seed(c + taps)
-    tokens = 4 * 65536 // (c // 8) + 6                              # just past the rule, a last run of fewer tokens
+    tokens = 4 * 98304 // (c // 8) + 6 if c % 8 == 0 else 600       # just past the rule, a last run of fewer tokens
     chunks = _chunks(tokens, g)
     r = lambda *s: torch.randn(*s, generator=g).to(dtype).to(cuda)
     u, w, b, ib = r(tokens, 2 * c)[:, c:], r(taps, c), r(c), r(c)
