@@ -2335,20 +2335,27 @@ __global__ void __launch_bounds__(64) sm_attn_prep_kernel(
 // The same with even head sizes: a lane owns rotation pairs (channels 2e, 2e + 1), so the convolution
 // reads 2-element vectors, the rotation needs no exchange through LDS, and q / k leave as 2-element
 // stores.  Heads up to 128 R wide, R <= 4.
-// A wave takes every 4 gridDim.y-th head of its token.  On prompts it was bound by round trips (a tap's rows behind a branch each)
-// and by the cosines and sines, the same in all heads: all rows of a head go out at once, and one wave's heads share the angles
-// where the tokens alone fill the chip.  us, 6376 / 21 tokens of the 2B and the small
-// layer list: 90 / 7.1 -> 65 / 4.8.
+// On prompts it was bound by round trips (a tap's rows behind a branch each) and by the cosines and sines, the same in all heads: all
+// rows of a head go out at once (TAPS 2 .. 4, known to the compiler: as a number up to 4 they cost 14 registers and 3 to 28 % of
+// the prompts of 100 to 1000 tokens), and in MANY a wave takes every 4 gridDim.y-th head of its token, which share the angles.
+// TAPS 0: any number, one after the other.
+// us with the state's launch, a tap at a time behind branches -> this, q + k + v heads x width, 100 / 500 / 2048 / 8000 tokens:
+//   24 x 128, 4 taps    7.2 / 10.9 / 29 / 92  ->  7.0 / 10.8 / 23 / 61       80 x 64, 4 taps  8.7 / 21.1 / 72 / 260  ->  8.7 / 17.9 / 49 / 145
+//   10 x 256, 4 taps    7.6 / 9.8 / 24 / 68   ->  6.9 / 9.1 / 20 / 50        9 x 64, 5 taps   6.9 / 7.5 / 13.3 / 43  ->  6.6 / 7.4 / 13.5 / 40
+//   6 x 512, 2 taps     7.7 / 9.9 / 23 / 58   ->  6.9 / 9.0 / 19 / 47 (a wave per head: MANY's registers leave too few waves, 51 at 8000)
 constexpr int kPrepPairs = 4;
 constexpr int kPrepGroups = 2048;     // workgroups that are resident together: eight on each CU
 
-template <typename T, int R, bool MANY>
+template <typename T, int R, int TAPS, bool MANY>
 __global__ void __launch_bounds__(256) sm_attn_prep_pair_kernel(
     const int32_t* __restrict__ tok_seq, const int32_t* __restrict__ cu, const int32_t* __restrict__ positions,
-    const int32_t* __restrict__ slots, int H, int G, int D, int Dv, int taps, int bs,   // (14 words: they come with the wave)
+    const int32_t* __restrict__ slots, int H, int G, int D, int Dv, int taps_, int bs,   // (14 words: they come with the wave)
     void* __restrict__ q_out_, const void* __restrict__ qkv_, const void* __restrict__ conv_w_, const void* state_,
     const void* __restrict__ q_norm_, const void* __restrict__ k_norm_, const float* __restrict__ freqs, int nrot, float mag,
     float eps, void* __restrict__ k_cache_, void* __restrict__ v_cache_, const int32_t* __restrict__ slot_mapping, void* tail_) {
+  static_assert(TAPS > 0 || !MANY, "the next head's rows are read ahead");
+  constexpr int NT = TAPS > 0 ? TAPS : 1;
+  const int taps = TAPS > 0 ? TAPS : taps_;
   const int t = blockIdx.x, lane = threadIdx.x & 63;
   const int C = H * D + G * (D + Dv);
   const int b = tok_seq[t];
@@ -2357,7 +2364,7 @@ __global__ void __launch_bounds__(256) sm_attn_prep_pair_kernel(
   const T* w = (const T*)conv_w_;
   const T* st = (const T*)state_ + (size_t)slots[b] * (taps - 1) * C;
   typedef T pair __attribute__((ext_vector_type(2)));
-  pair xn[R][kConvTaps], wn[R][kConvTaps];             // a head's rows and weights, up to kConvTaps taps
+  pair xn[R][NT], wn[R][NT];                           // a head's rows and weights
   auto channels = [&](int head, int& c0, int& n, int& kind) {   // kind 0 q, 1 k, 2 v
     if (head < H) c0 = head * D, n = D, kind = 0;
     else if (head < H + G) c0 = H * D + (head - H) * D, n = D, kind = 1;
@@ -2370,30 +2377,32 @@ __global__ void __launch_bounds__(256) sm_attn_prep_pair_kernel(
     for (int r = 0; r < R; ++r) {
       const int c = c0 + min(2 * (lane + 64 * r), n - 2);
 #pragma unroll
-      for (int j = 0; j < kConvTaps; ++j) {
-        const int jj = min(j, taps - 1);
-        wn[r][j] = *reinterpret_cast<const pair*>(w + (size_t)jj * C + c);
-        xn[r][j] = *reinterpret_cast<const pair*>(conv_row(qkv, (long)C, st, t, tl, taps - 1 - jj, taps, C) + c);
+      for (int j = 0; j < NT; ++j) {
+        wn[r][j] = *reinterpret_cast<const pair*>(w + (size_t)j * C + c);
+        xn[r][j] = *reinterpret_cast<const pair*>(conv_row(qkv, (long)C, st, t, tl, taps - 1 - j, taps, C) + c);
       }
     }
   };
-  const bool few = taps <= kConvTaps;                  // uniform
   int head = blockIdx.y * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (head >= H + 2 * G) return;
-  if (few) load(head);
-  float cs[R], sn[R];
+  if constexpr (TAPS > 0) load(head);
+  float cs[MANY ? R : 1], sn[MANY ? R : 1];            // one wave's heads share the angles
   bool angles = false;
-  for (; head < H + 2 * G; head += 4 * gridDim.y) {    // a wave per head
+  auto angle = [&](int i, float& c, float& s) {
+    const float ang = (float)pos * freqs[i];
+    c = cosf(ang) * mag, s = sinf(ang) * mag;
+  };
+  for (bool more = true; more; more = MANY && (head += 4 * (int)gridDim.y) < H + 2 * G) {
     int c0, n, kind;
     channels(head, c0, n, kind);
     float x[R][2];
     float ss = 0.f;
-    if (few) {
-      float xv[R][kConvTaps][2], wv[R][kConvTaps][2];
+    if constexpr (TAPS > 0) {
+      float xv[R][NT][2], wv[R][NT][2];
 #pragma unroll
       for (int r = 0; r < R; ++r)
 #pragma unroll
-        for (int j = 0; j < kConvTaps; ++j)
+        for (int j = 0; j < NT; ++j)
 #pragma unroll
           for (int e = 0; e < 2; ++e) xv[r][j][e] = (float)xn[r][j][e], wv[r][j][e] = (float)wn[r][j][e];
       if constexpr (MANY) load(min(head + 4 * (int)gridDim.y, H + 2 * G - 1));   // the next head's under this one
@@ -2403,16 +2412,14 @@ __global__ void __launch_bounds__(256) sm_attn_prep_pair_kernel(
         x[r][0] = x[r][1] = 0.f;
         if (e < n) {
 #pragma unroll
-          for (int j = 0; j < kConvTaps; ++j) {
-            if (j < taps) {
-              if (taps - 1 - j > pos) xv[r][j][0] = xv[r][j][1] = 0.f;
-              else {
-                x[r][0] = fmaf(wv[r][j][0], xv[r][j][0], x[r][0]);
-                x[r][1] = fmaf(wv[r][j][1], xv[r][j][1], x[r][1]);
-              }
-              // one token per sequence: the tail moves up here
-              if (tail_ && j > 0) stv<2>((T*)tail_ + ((size_t)slots[b] * (taps - 1) + j - 1) * C + c0 + e, xv[r][j]);
+          for (int j = 0; j < NT; ++j) {
+            if (taps - 1 - j > pos) xv[r][j][0] = xv[r][j][1] = 0.f;
+            else {
+              x[r][0] = fmaf(wv[r][j][0], xv[r][j][0], x[r][0]);
+              x[r][1] = fmaf(wv[r][j][1], xv[r][j][1], x[r][1]);
             }
+            // one token per sequence: the tail moves up here
+            if (tail_ && j > 0) stv<2>((T*)tail_ + ((size_t)slots[b] * (taps - 1) + j - 1) * C + c0 + e, xv[r][j]);
           }
           ss += fmaf(x[r][0], x[r][0], x[r][1] * x[r][1]);
         }
@@ -2423,12 +2430,11 @@ __global__ void __launch_bounds__(256) sm_attn_prep_pair_kernel(
         const int e = 2 * (lane + 64 * r);
         x[r][0] = x[r][1] = 0.f;
         if (e < n) {
-          for (int j = 0; j < taps; ++j) {
-            float xv[2], wv[2];
-            if (!conv_input_v<T, 2>(qkv, (long)C, st, t, tl, pos, taps - 1 - j, taps, c0 + e, C, xv)) continue;
-            ldv<2>(w + (size_t)j * C + c0 + e, wv);
-            x[r][0] = fmaf(wv[0], xv[0], x[r][0]);
-            x[r][1] = fmaf(wv[1], xv[1], x[r][1]);
+          for (int j = max(0, taps - 1 - pos); j < taps; ++j) {
+            const pair xv = *reinterpret_cast<const pair*>(conv_row(qkv, (long)C, st, t, tl, taps - 1 - j, taps, C) + c0 + e);
+            const pair wv = *reinterpret_cast<const pair*>(w + (size_t)j * C + c0 + e);
+            x[r][0] = fmaf((float)wv[0], (float)xv[0], x[r][0]);
+            x[r][1] = fmaf((float)wv[1], (float)xv[1], x[r][1]);
           }
           ss += fmaf(x[r][0], x[r][0], x[r][1] * x[r][1]);
         }
@@ -2452,16 +2458,11 @@ __global__ void __launch_bounds__(256) sm_attn_prep_pair_kernel(
       const int blk = slot / bs, off = slot - blk * bs;
       dst = (T*)k_cache_ + (((size_t)blk * G + (head - H)) * bs + off) * D;
     }
-    if (!angles) {                                     // (uniform)
+    if (MANY && !angles) {                             // (uniform)
       angles = true;
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const int i = lane + 64 * r;
-        if (i < nrot) {
-          const float ang = (float)pos * freqs[i];
-          cs[r] = cosf(ang) * mag, sn[r] = sinf(ang) * mag;
-        }
-      }
+      for (int r = 0; r < R; ++r)
+        if (lane + 64 * r < nrot) angle(lane + 64 * r, cs[MANY ? r : 0], sn[MANY ? r : 0]);
     }
     ss = wave_sum(ss);
     const float inv = 1.0f / sqrtf(ss / (float)n + eps);
@@ -2474,7 +2475,9 @@ __global__ void __launch_bounds__(256) sm_attn_prep_pair_kernel(
         ldv<2>(nw + e, g2);
         float x0 = x[r][0] * inv * g2[0], x1 = x[r][1] * inv * g2[1];
         if (i < nrot) {
-          const float r0 = fmaf(x0, cs[r], -(x1 * sn[r])), r1 = fmaf(x1, cs[r], x0 * sn[r]);   // (alike in every form)
+          if (!MANY) angle(i, cs[0], sn[0]);
+          const float c = cs[MANY ? r : 0], s = sn[MANY ? r : 0];
+          const float r0 = fmaf(x0, c, -(x1 * s)), r1 = fmaf(x1, c, x0 * s);   // (alike in every form)
           x0 = r0, x1 = r1;
         }
         o[0] = x0, o[1] = x1;
@@ -2500,21 +2503,35 @@ void sm_attn_prep(uintptr_t q_out, uintptr_t qkv, uintptr_t conv_w, uintptr_t st
   // tail needs no launch of its own (4.6 us)
   const bool tail = pairs && max_q_len == 1 && taps > 1 && taps <= kConvTaps;
   if (pairs) {
-    // workgroups per token: one per four heads while those fit the chip together, else fewer whose waves take several
-    const int most = (H + 2 * G + 3) / 4, gy = std::max(1, std::min(most, kPrepGroups / tokens));
-    const int r = std::max(D, Dv) <= 128 ? 1 : std::max(D, Dv) <= 256 ? 2 : kPrepPairs;
-#define SM_PREP(T_, R_) do { if (gy < most) SM_PREP_M(T_, R_, true); else SM_PREP_M(T_, R_, false); } while (0)
-#define SM_PREP_M(T_, R_, MANY_)                                                                                                    \
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(sm_attn_prep_pair_kernel<T_, R_, MANY_>), dim3(tokens, gy), dim3(256), 0,             \
+    const int most = (H + 2 * G + 3) / 4, r = std::max(D, Dv) <= 128 ? 1 : std::max(D, Dv) <= 256 ? 2 : kPrepPairs;
+    const bool exact = taps >= 2 && taps <= kConvTaps;
+    // workgroups per token: one per four heads while those fit the chip together, else fewer whose waves take as many heads each
+    // (18 heads of 64 at 500 tokens: 5 workgroups 9.1 us, 4 whose first wave takes two heads each 9.3, 3 8.6)
+    int gy = most;
+    if (exact && r <= 2) {
+      const int fit = std::max(1, kPrepGroups / tokens), each = (most + fit - 1) / fit;
+      gy = (most + each - 1) / each;
+    }
+#define SM_PREP_M(T_, R_, N_, MANY_)                                                                                                \
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(sm_attn_prep_pair_kernel<T_, R_, N_, MANY_>), dim3(tokens, gy), dim3(256), 0,         \
                      (hipStream_t)stream, (const int32_t*)tok_seq, (const int32_t*)cu, (const int32_t*)positions,            \
                      (const int32_t*)slots, H, G, D, Dv, taps, bs, (void*)q_out, (const void*)qkv, (const void*)conv_w,      \
                      (const void*)state, (const void*)q_norm, (const void*)k_norm, (const float*)freqs, nrot, mag, eps,      \
                      (void*)k_cache, (void*)v_cache, (const int32_t*)slot_mapping, tail ? (void*)state : nullptr)
+#define SM_PREP_N(T_, R_, N_) do { if (R_ <= 2 && gy < most) SM_PREP_M(T_, R_, N_, (R_ <= 2)); else SM_PREP_M(T_, R_, N_, false); } while (0)
+#define SM_PREP(T_, R_)                                                                                                      \
+  do {                                                                                                                       \
+    if (!exact) SM_PREP_M(T_, R_, 0, false);                                                                                 \
+    else if (taps == 2) SM_PREP_N(T_, R_, 2);                                                                                \
+    else if (taps == 3) SM_PREP_N(T_, R_, 3);                                                                                \
+    else SM_PREP_N(T_, R_, 4);                                                                                               \
+  } while (0)
 #define SM_PREP_R(T_) do { if (r == 1) SM_PREP(T_, 1); else if (r == 2) SM_PREP(T_, 2); else SM_PREP(T_, kPrepPairs); } while (0)
     if (f32) SM_PREP_R(float);
     else SM_PREP_R(bf16);
 #undef SM_PREP_R
 #undef SM_PREP
+#undef SM_PREP_N
 #undef SM_PREP_M
     DLLM_HIP_CHECK(hipGetLastError());
   }

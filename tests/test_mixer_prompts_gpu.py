@@ -49,11 +49,14 @@ def test_causal_conv_of_runs_bit_exact(cuda, dtype, out, c, taps, act):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("heads,kvh,dim,vdim,taps,nrot", [(20, 2, 128, 128, 4, 32), (3, 1, 64, 96, 3, 32), (9, 1, 192, 320, 2, 10),
-                                                          (6, 1, 30, 16, 1, 0), (5, 2, 64, 64, 5, 8)])
-def test_attention_input_of_many_heads_per_wave_bit_exact(cuda, dtype, heads, kvh, dim, vdim, taps, nrot):
+@pytest.mark.parametrize("tokens,heads,kvh,dim,vdim,taps,nrot", [
+    (2051, 20, 2, 128, 128, 4, 32), (2051, 3, 1, 64, 96, 3, 32), (2051, 9, 1, 192, 256, 2, 10), (700, 40, 4, 64, 64, 4, 16),
+    (500, 18, 1, 64, 64, 3, 20), (2051, 9, 1, 192, 320, 2, 10), (2051, 6, 1, 30, 16, 1, 0), (2051, 5, 2, 64, 64, 5, 8)])
+def test_attention_input_of_many_heads_per_wave_bit_exact(cuda, dtype, tokens, heads, kvh, dim, vdim, taps, nrot):
+    """All heads of a token in one workgroup, in two or three of as many each (the first five); a wave per head with every number
+    of taps."""
     g = torch.Generator().manual_seed(heads + dim)
-    tokens, bs, c = 2051, 16, heads * dim + kvh * (dim + vdim)      # fewer workgroups per token than heads / 4
+    bs, c = 16, heads * dim + kvh * (dim + vdim)
     chunks = _chunks(tokens, g)
     r = lambda *s: torch.randn(*s, generator=g).to(dtype).to(cuda)
     qkv, cw, qn, kn, conv = r(tokens, c), r(taps, c), r(dim), r(dim), r(len(chunks) + 2, taps - 1, c)
