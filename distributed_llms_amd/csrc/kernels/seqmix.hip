@@ -1651,16 +1651,28 @@ __global__ void __launch_bounds__(256, 2) sm_rglru_gates_split_kernel(
 
 // The same sums with an output per lane and 32 per wave, 128 tokens by 128 outputs per workgroup, u and the weights element by
 // element: any width and alignment, and no lane idle from blocks of 128 on.  Bound by its vector work and by two-byte loads.
-// Which kernel, us, this / the one above: widths that are no multiple of 4 this (8 blocks of 255, 300 / 16000 tokens 41 / 257
+// Which kernel, us, this / the one above: widths that are no multiple of 4 this (8 blocks of 255, 300 / 16000 tokens 40 / 257
 // against 59 / 503 element by element there); 8 blocks of 64, 128, 256: 2000 tokens 27 / 20, 31 / 23, 47 / 30; 4500 tokens 34 / 38,
 // 43 / 47, 94 / 66; 8000 36 / 47, 49 / 58, 115 / 86: blocks up to 128 leave half of the other's waves idle, which counts once the CUs
 // hold two workgroups each; 3 blocks of 24, 300 / 16000 tokens: 23 / 34, 27 / 52.
 constexpr int kCT = 128;      // tokens per workgroup
 
-__global__ void __launch_bounds__(256, 2) sm_rglru_gates_column_kernel(
-    float* __restrict__ a_out, float* __restrict__ g_out, const float* __restrict__ u, const bf16* __restrict__ ra_t,
-    const bf16* __restrict__ ra_b, const bf16* __restrict__ ri_t, const bf16* __restrict__ ri_b,
-    const bf16* __restrict__ lam, int tokens, int nb, int bw, float scale) {
+// (The arguments come in one piece, which is loaded.  Preloaded into the waves' registers as the other kernels' are, they cost it 2 % at
+// few tokens, 8 blocks of 255 at 300 / 1000 / 8000 us 39.9 / 42.8 / 118 -> 40.5 / 43.3 / 118, 8 blocks of 129 at 500 33.0 -> 33.4.)
+struct GateArgs {
+  float *a, *g;
+  const float* u;
+  const bf16 *ra_t, *ra_b, *ri_t, *ri_b, *lam;
+  int tokens, nb, bw;
+  float scale;
+};
+__global__ void __launch_bounds__(256, 2) sm_rglru_gates_column_kernel(const GateArgs p) {
+  float *__restrict__ a_out = p.a, *__restrict__ g_out = p.g;
+  const float* __restrict__ u = p.u;
+  const bf16 *__restrict__ ra_t = p.ra_t, *__restrict__ ri_t = p.ri_t;
+  const bf16 *ra_b = p.ra_b, *ri_b = p.ri_b, *lam = p.lam;
+  const int tokens = p.tokens, nb = p.nb, bw = p.bw;
+  const float scale = p.scale;
   __shared__ __attribute__((aligned(16))) bf16 us[3][kCT][kSP];
   const int t0 = blockIdx.x * kCT, b = blockIdx.y, C = nb * bw;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, n = lane & 31, half = lane >> 5;
@@ -1773,7 +1785,10 @@ void sm_rglru_gates(uintptr_t a, uintptr_t g, uintptr_t u, uintptr_t ra_t, uintp
                      (const bf16*)ra_t, (const bf16*)ra_b, (const bf16*)ri_t, (const bf16*)ri_b, (const bf16*)lam, tokens,   \
                      nb, bw, scale)
     if (split) SM_GATES(sm_rglru_gates_split_kernel, grid);
-    else SM_GATES(sm_rglru_gates_column_kernel, cols);
+    else
+      hipLaunchKernelGGL(sm_rglru_gates_column_kernel, cols, dim3(256), 0, (hipStream_t)stream,
+                         GateArgs{(float*)a, (float*)g, (const float*)u, (const bf16*)ra_t, (const bf16*)ra_b, (const bf16*)ri_t,
+                                  (const bf16*)ri_b, (const bf16*)lam, tokens, nb, bw, scale});
 #undef SM_GATES
     DLLM_HIP_CHECK(hipGetLastError());
     return;
