@@ -10,7 +10,12 @@ from distributed_llms_amd.engine import graphs
 
 class _Stream:
     def __init__(self, handle, sid):
-        self.cuda_stream, self.stream_id, self.issued = handle, sid, []
+        self.handle, self.stream_id, self.issued, self.made = handle, sid, [], False
+
+    @property
+    def cuda_stream(self):                       # (torch makes a stream when its handle is first asked for)
+        self.made = True
+        return self.handle
 
 
 class _Event:
@@ -44,15 +49,17 @@ def test_buffers_are_reused_behind_their_copies(monkeypatch, seed, ids):
     ring, last = graphs.StagingRing(4), {}
     for s in streams[1:3]:
         ring.keep(s)
-    steps = 400
+    used, steps = {now[0]}, 400
     for step in range(steps):
         if rng.random() < (0.0, 0.0, 0.1, 0.3, 0.9, 0.02)[seed]:
             now[0] = rng.choice(streams)
+            used.add(now[0])
         buf = ring.take()
         assert buf not in last or last[buf] in done, (step, buf)
         last[buf] = step
         now[0].issued.append(step)
         ring.sent()
+    assert {s for s in streams if s.made} == used
     if seed < 2:
         assert len(events) == steps // (ring.BUFFERS // 2)
 
@@ -72,7 +79,7 @@ def test_host_runs_ahead_of_replays(cuda):
     eng = LLMEngine(EngineConfig(model=name, dtype="bfloat16", device="cuda", max_batch=2, max_seq_len=256, num_kv_blocks=64,
                                  graph_batch_sizes=(2,)), stage)
     steps, other = 3 * graphs.StagingRing.BUFFERS + 1, torch.cuda.Stream()
-    assert eng.streams[0].cuda_stream in eng.runner.graphs.staging.lasting
+    assert eng.streams[0] in eng.runner.graphs.staging.kept
 
     def run(ahead):
         rp = TraceReplayer(eng)
