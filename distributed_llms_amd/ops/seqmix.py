@@ -31,6 +31,8 @@ from typing import Optional, Tuple
 import torch
 
 from .. import _ext
+from . import gemm, linear            # (at the top: an import inside a function is 1 us of host time per call)
+from .gemm import SplitKPartial
 from .stream import current_stream as _stream
 
 ACT_DTYPES = (torch.bfloat16, torch.float32)
@@ -146,7 +148,6 @@ def post_norm_add(x: torch.Tensor, o, w_post: torch.Tensor, eps: float, mult: fl
     returns it in ``o``'s dtype (the stream tensor when that is float32).  ``o`` may be a :class:`~.gemm.SplitKPartial`
     (without ``o2``): its slabs are then summed in the same launch.  ``final``: ``w_next`` is the norm behind the last sublayer
     and h has the bits of :func:`rms_norm_f32` (whose sum has another order than a close's)."""
-    from .gemm import SplitKPartial
     off = 1.0 if one_plus else 0.0
     if not x.is_cuda:
         ob = o.float() if o2 is None else scales[0] * o.float() + scales[1] * o2.float()
@@ -238,7 +239,6 @@ def post_layer_norm_add(x: torch.Tensor, o, w_post: torch.Tensor, b_post: torch.
     ``b_post``) in place on the float32 residual stream; with ``w_next`` / ``b_next`` also returns the next sublayer's input
     layer_norm(x) in the activation type (None otherwise).  ``o`` may be a :class:`~.gemm.SplitKPartial` (the output of a
     split-K product that is not reduced yet): its slabs are then summed in the same launch."""
-    from .gemm import SplitKPartial
     if tuple(o.shape) != tuple(x.shape) or (w_next is None) != (b_next is None):
         raise ValueError("post_layer_norm_add: o / x shape mismatch, or half a next norm")
     if not x.is_cuda:
@@ -297,7 +297,6 @@ class Close:
         return self.h
 
     def _product(self, w: torch.Tensor, bias: Optional[torch.Tensor], glu: str, limit: float) -> Optional[torch.Tensor]:
-        from . import gemm
         kw, o = self._kw, self._o
         if kw.get("w_next") is None or kw.get("final") or kw.get("o2") is not None:
             return None
@@ -314,7 +313,6 @@ class Close:
         return y
 
     def linear(self, w: torch.Tensor) -> torch.Tensor:
-        from . import linear
         y = None if self._o is None else self._product(w, None, "", 0.0)
         return linear(self.input(), w) if y is None else y
 
@@ -607,7 +605,6 @@ def clipped_glu(gu: torch.Tensor, bias_gu: Optional[torch.Tensor], limit: float,
 def linear_clipped_glu(x: torch.Tensor, w_gate_up: torch.Tensor, bias_gu: Optional[torch.Tensor], limit: float) -> torch.Tensor:
     """:func:`clipped_glu` of ``x W^T``, W = [Wg; Wu]: in a GEMM epilogue where one takes the shape and the bias, else the
     projection followed by the gate kernel."""
-    from . import gemm, linear
     if bias_gu is not None and (bias_gu.dim() != 1 or bias_gu.size(0) != w_gate_up.size(0) or bias_gu.dtype != x.dtype
                                 or bias_gu.device != x.device):
         raise ValueError(f"linear_clipped_glu: bias [{w_gate_up.shape[0]}] of x's type and device")
@@ -630,7 +627,6 @@ def gelu_glu(gu: torch.Tensor) -> torch.Tensor:
 def linear_gelu_glu(x: torch.Tensor, w_gate_up: torch.Tensor) -> torch.Tensor:
     """gelu_tanh(x Wg^T) * (x Wu^T), W = [Wg; Wu]: in a GEMM epilogue or the split-K reduction where the framework's
     bf16 GEMMs take the shape, else the projection followed by the gate kernel (float32, odd sizes)."""
-    from . import gemm, linear
     y = gemm.linear_gelu_glu(x, w_gate_up) if x.is_cuda else None
     return gelu_glu(linear(x, w_gate_up)) if y is None else y
 
@@ -649,7 +645,6 @@ def softcap_f32(logits: torch.Tensor, cap: float, scale: float = 1.0) -> torch.T
 def logits_f32(x: torch.Tensor, w: torch.Tensor, cap: float = 0.0) -> torch.Tensor:
     """:func:`softcap_f32` of the product ``x w^T``: in the product's own launch where that is the weight-streaming one (32000
     columns of K = 1024, 1 / 8 / 16 rows: 13.9 / 14.2 / 15.1 us in two launches, 12.3 / 12.4 / 13.1 in one)."""
-    from . import gemm, linear
     if (type(x) is torch.Tensor and type(w) in (torch.Tensor, torch.nn.Parameter) and x.is_cuda and x.dim() == 2
             and x.shape[0] <= gemm.STREAM_MAX_M and x.device == w.device and w.dim() == 2 and w.shape[1] == x.shape[1]
             and not gemm._recorded(x, w, None) and gemm.use_stream(x.shape[0], w.shape[0], x.shape[1], x, w)):
