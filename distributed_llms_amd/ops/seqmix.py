@@ -266,9 +266,10 @@ class Close:
     """The close of a sublayer that is still to be made, for the product that reads it: ``kind`` "rms" with the arguments of
     :func:`post_norm_add` or "layer" with those of :func:`post_layer_norm_add`.  The product makes it in its own launch where
     that is the faster way (:func:`~.gemm.close_product`: a single row); ``x`` is the new stream from then on (a tensor of its
-    own or the old one, updated in place).  Several rows, or slabs, are closed at once (the host issues a prompt of 40 tokens on
-    the small layer list in 551 us, 567 where each product asks, 540 with the functions alone).  One product reads a Close: inside its launch the normed rows never reach memory, so
-    that a second one, or :meth:`input`, is refused then.  What several read asks for :meth:`input` first."""
+    own or the old one, updated in place).  Several rows, or slabs, are closed at once: kept until each product had asked, they cost
+    a prompt of 40 tokens on the small layer list 16 us of the host time that bounds it (551 -> 567 us).  One product reads a
+    Close: inside its launch the normed rows never reach memory, so that a second one, or :meth:`input`, is refused then.  What
+    several read asks for :meth:`input` first."""
 
     __slots__ = ("kind", "x", "h", "_o", "_kw", "_taken")
 
