@@ -302,7 +302,10 @@ def run_loopback_pipeline(ecfg: EngineConfig, num_stages: int, prompts, params: 
         try:
             dev = runners[s].stage.device
             if dev.type == "cuda":
-                with torch.cuda.stream(torch.cuda.Stream(dev)):
+                own = torch.cuda.Stream(dev)
+                if runners[s].graphs is not None:
+                    runners[s].graphs.staging.keep(own)
+                with torch.cuda.stream(own):
                     stage_worker_loop(runners[s], hub.transport(s), stop_on_round_end=False)
             else:
                 stage_worker_loop(runners[s], hub.transport(s), stop_on_round_end=False)
