@@ -17,8 +17,9 @@
 //   K 3072:  3072 / 9216 8.4 / 15.1 -> 7.4 / 13.7, + GLU 8192 / 16384 13.7 / 22.3 -> 12.8 / 21.4;  8.9 / 15.5 -> 8.0 / 14.5, 22.5 -> 21.9
 // and every size between and past them that was tried (160, to 96 Mi weights) as fast at least.  Wider rows, in four pieces, win as
 // much in most products (4096 x 4096 10.9 -> 10.3, 22016 x 4096 + GLU 35.7 -> 33.4), but some GLUs, where a few CUs have a second
-// workgroup, lose: 18432 x 3584 26.7 -> 29.5, 14336 / 16384 / 18432 x 4096 27.0 / 28.9 / 31.0 -> 29.3 / 31.3 / 32.2.  More rows cost each workgroup as many times the arithmetic: 4 rows at best equal (6144 x 1024 7.1 / 7.1),
-// 2560 wide slower (15360 19.3 / 19.8), so that the launch of its own is kept for them.
+// workgroup, lose: 18432 x 3584 26.7 -> 29.5, 14336 / 16384 / 18432 x 4096 27.0 / 28.9 / 31.0 -> 29.3 / 31.3 / 32.2.
+// More rows cost each workgroup as many times the arithmetic: 4 rows at best equal (6144 x 1024 7.1 / 7.1), 2560 wide slower (15360
+// 19.3 / 19.8), so that the launch of its own is kept for them.
 #include "gemm_stream.h"
 #include "launchers.h"
 

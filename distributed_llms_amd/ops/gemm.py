@@ -311,9 +311,10 @@ def close_product(kind: str, x: torch.Tensor, o: torch.Tensor, w: torch.Tensor, 
     y = torch.empty(1, n // 2 if glu else n, dtype=torch.bfloat16, device=x.device)
     xo = torch.empty_like(x)
     p = lambda t: 0 if t is None else t.data_ptr()
-    _ext.kernels().gemm_close(y.data_ptr(), w.data_ptr(), p(bias), n, k, _STREAM_GLU[glu], 1 if n * k * 2 >= WIDE_NT_MIN_BYTES else 0, float(limit), 1 if kind == "rms" else 2,
-                              x.data_ptr(), o.data_ptr(), p(o_bias), w_post.data_ptr(), p(b_post), w_next.data_ptr(), p(b_next),
-                              xo.data_ptr(), float(eps), float(mult), float(offset), current_stream())
+    _ext.kernels().gemm_close(y.data_ptr(), w.data_ptr(), p(bias), n, k, _STREAM_GLU[glu], 1 if n * k * 2 >= WIDE_NT_MIN_BYTES else 0,
+                              float(limit), 1 if kind == "rms" else 2, x.data_ptr(), o.data_ptr(), p(o_bias), w_post.data_ptr(),
+                              p(b_post), w_next.data_ptr(), p(b_next), xo.data_ptr(), float(eps), float(mult), float(offset),
+                              current_stream())
     return xo, y
 
 
