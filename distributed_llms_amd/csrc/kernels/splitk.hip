@@ -107,7 +107,9 @@ __global__ void __launch_bounds__(NTH) splitk_add_rms_norm_kernel(bf16* __restri
   // dependent memory round trips instead of one.
   const int S = SC > 0 ? SC : S_;
   constexpr int SE = SC > 0 ? SC : 1;
-  constexpr int CH = MAXV * SE <= 16 ? MAXV : (16 / SE > 0 ? 16 / SE : 1);
+  // (a divisor of MAXV: chunks of 3 vectors of 4, 8192 wide in 5 slabs, went past the row)
+  constexpr int CH = MAXV * SE <= 16 ? MAXV : SE <= 2 ? 8 : SE <= 4 ? 4 : SE <= 8 ? 2 : 1;
+  static_assert(MAXV % CH == 0, "whole chunks");
   __shared__ float red[16];
   const int row = blockIdx.x;
   const int nvec = N >> 3;

@@ -218,6 +218,21 @@ def test_post_norm_add_sums_split_products(cuda, tokens, width, k):
 
 
 @gpu
+@pytest.mark.parametrize("n,slabs", [(4096, 5), (6144, 5), (8192, 3), (8192, 5), (8192, 8), (16384, 2), (16384, 3), (16384, 5), (16384, 7)])
+def test_add_rms_norm_sums_slabs_inside_its_rows(cuda, n, slabs):
+    """Every split of a row's vectors into chunks of loads: the sum of the slabs as the plain reduction makes it, and nothing
+    written past the rows (5 slabs of 8192 were taken in chunks of three vectors of four)."""
+    g = torch.Generator("cuda").manual_seed(n + slabs)
+    ws = torch.randn(slabs * 2 * n, generator=g, device="cuda").half().view(torch.float32)
+    part = gemm.SplitKPartial(ws, slabs, 2, n, (2, n), torch.bfloat16, ws.device)
+    room = torch.randn(4, n, generator=g, device="cuda").bfloat16()
+    w, before = torch.randn(n, generator=g, device="cuda").bfloat16(), room.clone()
+    want, r = ops.fused_add_rms_norm(part.materialize(), room[:2].clone(), w, 1e-5)
+    y, res = ops.fused_add_rms_norm(part, room[:2], w, 1e-5)
+    assert torch.equal(y, want) and torch.equal(res, r) and torch.equal(room[2:], before[2:])
+
+
+@gpu
 @pytest.mark.parametrize("lens,width,splits", [
     ([1, 33, 64], 2, 1),                   # one chunk, and the new key alone in its chunk
     ([65, 64, 1], 4, 2), ([97, 200, 250], 8, 4), ([449, 1], 16, 8), ([1000], 32, 16), ([1025, 3], 33, 17),
