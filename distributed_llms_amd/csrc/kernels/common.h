@@ -235,6 +235,17 @@ __device__ __forceinline__ void part_store(float* P, size_t i, float v) {
   P[i] = v;
 #endif
 }
+// 4 consecutive elements (aligned to 4 elements)
+__device__ __forceinline__ void part_store4(float* P, size_t i, const f32x4& v) {
+#if DLLM_PART_TYPE == 1
+  *reinterpret_cast<bf16x4*>(reinterpret_cast<bf16*>(P) + i) = bf16x4{f2bf(v[0]), f2bf(v[1]), f2bf(v[2]), f2bf(v[3])};
+#elif DLLM_PART_TYPE == 2
+  const f32x4 s = v * kPartScale;
+  *reinterpret_cast<f16x4*>(reinterpret_cast<_Float16*>(P) + i) = f16x4{(_Float16)s[0], (_Float16)s[1], (_Float16)s[2], (_Float16)s[3]};
+#else
+  *reinterpret_cast<f32x4*>(P + i) = v;
+#endif
+}
 // The stored form of an element, for a caller that has several loads under way before it converts any (a conversion next
 // to its load makes hipcc wait there)
 #if DLLM_PART_TYPE == 1

@@ -348,14 +348,17 @@ class ModelStage:
                                            max_ctx=meta.max_ctx or None, workspace=meta.attn_workspace)
         return o.view(o.shape[0], self.q_size_local)
 
-    def _mlp(self, h: torch.Tensor, lw: Dict[str, torch.Tensor]) -> torch.Tensor:
+    def _mlp(self, h: Optional[torch.Tensor], lw: Dict[str, torch.Tensor], gated: Optional[torch.Tensor] = None) -> torch.Tensor:
+        """``gated``: the dense MLP's activation, where the launch of its norm has made it already (``h`` is None then)."""
         if self.cfg.is_moe:
             out = ops.moe_forward(h, lw["router"], lw["experts_gate_up"], lw["experts_down"],
                                   self.cfg.experts_per_token, self.tp.expert_offset(self.cfg.num_experts))
             return self.tp.all_reduce_(out) if self.tp.enabled else out
         # defer: the down projection's split-K reduce is fused into the next residual-add + RMSNorm
         # (under TP the partial [T, H] is all-reduced first, so it is materialised)
-        out = ops.linear(ops.linear_swiglu(h, lw["w_gate_up"]), lw["w_down"], defer=not self.tp.enabled)
+        if gated is None:
+            gated = ops.linear_swiglu(h, lw["w_gate_up"])
+        out = ops.linear(gated, lw["w_down"], defer=not self.tp.enabled)
         return self.tp.all_reduce_(out) if self.tp.enabled else out
 
     def _units(self):
@@ -394,14 +397,20 @@ class ModelStage:
             if self.has(l, 0) or self.has(l, 1) or self.has(l, 2):
                 a = qkv = None
                 if self.has(l, 0):
-                    # W8A8 projection next (quant="fp8"): the norm kernel emits the per-token e4m3 input
-                    q8 = isinstance(lw.get("wqkv"), ops.quant.Fp8Weight)
-                    if h is None:
-                        x = ops.rms_norm(residual, lw["attn_norm"], eps, quant_out=q8)
+                    # one row: the add and the norm in the projection's launch
+                    defer = knobs.K.defer_qkv and self.has(l, 1)
+                    one = ops.norm_linear(h, residual, lw["attn_norm"], eps, lw["wqkv"]) if defer else None
+                    if one is not None:
+                        qkv, residual = one
                     else:
-                        x, residual = ops.fused_add_rms_norm(h, residual, lw["attn_norm"], eps, quant_out=q8)
+                        # W8A8 projection next (quant="fp8"): the norm kernel emits the per-token e4m3 input
+                        q8 = isinstance(lw.get("wqkv"), ops.quant.Fp8Weight)
+                        if h is None:
+                            x = ops.rms_norm(residual, lw["attn_norm"], eps, quant_out=q8)
+                        else:
+                            x, residual = ops.fused_add_rms_norm(h, residual, lw["attn_norm"], eps, quant_out=q8)
+                        qkv = ops.linear(x, lw["wqkv"], defer=defer)
                     h = None
-                    qkv = ops.linear(x, lw["wqkv"], defer=knobs.K.defer_qkv and self.has(l, 1))
                     if not self.has(l, 1):
                         out_aux = self._dense(qkv)
                         break
@@ -420,19 +429,24 @@ class ModelStage:
                         h = ops.linear(a, lw["wo"], defer=knobs.K.defer_o)
             # ---- MLP half: atoms 3 / 4 (first / second half of the intermediate columns)
             if self.has(l, 3) or self.has(l, 4):
-                q8 = isinstance(lw.get("w_gate_up"), ops.quant.Fp8Weight)
-                if h is None:
-                    x = ops.rms_norm(residual, lw["mlp_norm"], eps, quant_out=q8)
+                one = None if cfg.is_moe else ops.norm_linear(h, residual, lw["mlp_norm"], eps, lw["w_gate_up"], swiglu=True)
+                x = gated = None
+                if one is not None:
+                    gated, residual = one
                 else:
-                    x, residual = ops.fused_add_rms_norm(h, residual, lw["mlp_norm"], eps, quant_out=q8)
+                    q8 = isinstance(lw.get("w_gate_up"), ops.quant.Fp8Weight)
+                    if h is None:
+                        x = ops.rms_norm(residual, lw["mlp_norm"], eps, quant_out=q8)
+                    else:
+                        x, residual = ops.fused_add_rms_norm(h, residual, lw["mlp_norm"], eps, quant_out=q8)
                 if self.has(l, 3) and self.has(l, 4):
-                    h = self._mlp(x, lw)
+                    h = self._mlp(x, lw, gated)
                 elif self.has(l, 3):                  # cut between the MLP halves: hand over the partial sum
-                    out_aux = self._dense(self._mlp(x, lw))
+                    out_aux = self._dense(self._mlp(x, lw, gated))
                     h = None
                     break
                 else:                                 # second half: add the first half's partial sum
-                    h = ops.add_(self._dense(self._mlp(x, lw)), carry)
+                    h = ops.add_(self._dense(self._mlp(x, lw, gated)), carry)
         if out_aux is not None:
             return torch.cat([residual, out_aux.view(out_aux.shape[0], -1)], dim=1)
         if not self.is_last:

@@ -162,6 +162,14 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor) -> torch.Tensor:
     return silu_mul(linear(x, w_gate_up))
 
 
+def norm_linear(h, residual: torch.Tensor, norm_w: torch.Tensor, eps: float, w, swiglu: bool = False):
+    """:func:`fused_add_rms_norm` (``h`` None: :func:`rms_norm`) and :func:`linear` (deferred) or :func:`linear_swiglu` behind it in
+    one launch: (product, new residual), or None where they have launches of their own (:func:`gemm.norm_linear`)."""
+    if isinstance(w, quant.Fp8Weight) or not _gpu(residual):
+        return None
+    return gemm.norm_linear(h, residual, norm_w, eps, w, swiglu)
+
+
 def add_(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     """a <- a + b (in place)."""
     if not _gpu(a):

@@ -530,6 +530,9 @@ def linear_wide(x: torch.Tensor, w: torch.Tensor, splits: int = 0, swiglu: bool 
     if n % 128 or k % 64:
         raise ValueError("linear_wide: N % 128 and K % 64")
     s = splits or wide_splits(m, n, k, swiglu)
+    if m == 1 and not splits and variant < 0 and (s == 1 or (defer and not swiglu)) and one_fits(n, k, s, swiglu) \
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0:
+        return _one(x, w, s, swiglu, x.shape[:-1], x=x)
     ws = _workspace(x.device)
     if s > 1 and s * m * n > ws.numel():
         s = max(1, ws.numel() // (m * n))
@@ -545,6 +548,68 @@ def linear_wide(x: torch.Tensor, w: torch.Tensor, splits: int = 0, swiglu: bool 
     _ext.kernels().gemm_wide(y.data_ptr(), x.data_ptr(), w.data_ptr(), ws.data_ptr(), ws.numel(), m, n, k, s,
                              1 if swiglu else 0, v, stream)
     return y
+
+
+ONE_MAX_WIDTH = 8192               # (csrc/kernels/gemm_one.hip: a row, or its slice, in the registers of four waves)
+ONE_MAX_SLABS = 8
+
+
+def one_fits(n: int, k: int, s: int, swiglu: bool = False) -> bool:
+    """Does gemm_one serve one row's [1, k] x [n, k]^T product in ``s`` K slices?  It has gemm_wide's bits and is as fast or faster
+    wherever that would run (figures there).  GLUs unsplit: below 171 column tiles the weight-streaming kernel's shorter ones keep more
+    CUs busy, us with the add + norm in front, apart / in one launch: 22016 x 4096 (172 tiles) 33.5 / 30.0, 16384 x 3072 (128) 20.6 /
+    22.0, 13824 x 2560 (108) 17.1 / 19.1-21.6, 8192 x 2048 (64) 9.6 / 12.6."""
+    return (knobs.K.one and n % 128 == 0 and k % 64 == 0 and n * k * 2 < 1 << 32 and -(-(k // 64) // s) * 64 <= ONE_MAX_WIDTH
+            and (not swiglu or (s == 1 and n // 128 >= 171)))
+
+
+def _one(like: torch.Tensor, w: torch.Tensor, s: int, swiglu: bool, lead, x=None, residual=None, part=None, norm_w=None,
+         res_out=None, eps: float = 0.0):
+    """gemm_one's launch: the finished product of one row, or its :class:`SplitKPartial` (``s`` > 1).  Slabs that are read lie at the
+    start of the workspace or in its second half, and those that are written in the other."""
+    n, k = w.shape
+    p = lambda t: 0 if t is None else t.data_ptr()
+    nt = 1 if n * k * 2 >= WIDE_NT_MIN_BYTES else 0
+    args = (p(x), p(residual), 0 if part is None else part.ws.data_ptr(), 0 if part is None else part.splits, p(norm_w), p(res_out),
+            float(eps), current_stream())
+    if s > 1:
+        ws = _workspace(like.device)
+        if part is not None and part.ws.data_ptr() == ws.data_ptr():
+            ws = ws[ws.numel() // 2:]
+        se = _ext.kernels().gemm_one(0, ws.data_ptr(), w.data_ptr(), n, k, s, 2, nt, *args)
+        return SplitKPartial(ws, se, 1, n, (*lead, n), like.dtype, like.device)
+    y = torch.empty(*lead, n // 2 if swiglu else n, dtype=like.dtype, device=like.device)
+    _ext.kernels().gemm_one(y.data_ptr(), 0, w.data_ptr(), n, k, 1, 1 if swiglu else 0, nt, *args)
+    return y
+
+
+def norm_linear(h, residual: torch.Tensor, norm_w: torch.Tensor, eps: float, w: torch.Tensor, swiglu: bool = False):
+    """(y, r): r = ``residual`` + ``h`` (None: ``residual``; a :class:`SplitKPartial`: its sum), y = rms_norm(r) * ``norm_w`` times
+    w^T (a :class:`SplitKPartial`) or its SwiGLU, in one launch -- one row of a weight that gemm_wide or gemm_one would serve behind a
+    norm of its own, with the bits of the two; else None.  ``residual`` is left as it is."""
+    k = residual.shape[-1]
+    if not (residual.is_cuda and residual.numel() == k and w.dim() == 2 and w.size(1) == k and norm_w.numel() == k
+            and k <= ONE_MAX_WIDTH and residual.dtype == w.dtype == norm_w.dtype == torch.bfloat16):
+        return None
+    n = w.size(0)
+    if not _use_wide(1, n, k, residual, w, swiglu):
+        return None
+    s = wide_splits(1, n, k, swiglu)
+    if not one_fits(n, k, s, swiglu) or (s == 1 and not swiglu):
+        return None
+    part = h if isinstance(h, SplitKPartial) else None
+    if part is not None:
+        if part.splits > ONE_MAX_SLABS or part.m != 1 or part.n != k or part.device != residual.device:
+            return None
+    elif h is not None and not (h.shape == residual.shape and h.dtype == residual.dtype and h.is_contiguous() and h.device == residual.device):
+        return None
+    if w.device != residual.device or norm_w.device != residual.device or not norm_w.is_contiguous() \
+            or any(t.data_ptr() % 16 for t in (residual, norm_w, w)) or (part is None and h is not None and h.data_ptr() % 16):
+        return None
+    res_out = residual if h is None else torch.empty_like(residual)
+    y = _one(residual, w, s, swiglu, residual.shape[:-1], None if part is not None else h, residual, part, norm_w,
+             None if h is None else res_out, eps)
+    return y, res_out
 
 
 def pp_splits(m: int, n: int, k: int, bn: int = 256, target_wgs: int = 256) -> int:
