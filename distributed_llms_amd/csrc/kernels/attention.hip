@@ -237,17 +237,15 @@ __device__ __forceinline__ void rope_rotate(bf16x8 (&f)[D / 32], const RopeRow<D
   }
 }
 
-template <int D, bool FUSED, int PARTS = 0, bool JOIN = false>
-__global__ void __launch_bounds__(JOIN ? 512 : 64, 2) attn_decode_kernel(   // 2nd arg: min waves per SIMD
-    bf16* __restrict__ out, const bf16* __restrict__ q, bf16* __restrict__ k_cache,
-    bf16* __restrict__ v_cache, const int32_t* __restrict__ block_tables,
-    const int32_t* __restrict__ seq_lens, float* __restrict__ part_o, float* __restrict__ part_ml,
-    int hq, int hkv, int max_blocks, int split_len, float scale_log2, RopeArgs ra) {
-  extern __shared__ __attribute__((aligned(16))) float join_lds[];   // JOIN: [split][head][D + 4], then [split][head](m, l)
-  const int kvh = blockIdx.y, b = blockIdx.z;
-  const int lane = threadIdx.x & 63;
-  const int split = JOIN ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : (int)blockIdx.x;
-  const int nsplit = JOIN ? (int)(blockDim.x >> 6) : (int)gridDim.x;
+// One wave's part of a decode: sequence b, kv head kvh, keys [split * split_len, + split_len).  write_out(state, denominator)
+// takes the wave's partial result.  append: does this wave write the new key and value (FUSED, where the split owns them)?  NT:
+// K/V lines that nobody else reads.
+template <int D, bool FUSED, int PARTS, bool NT, class WriteOut>
+__device__ __forceinline__ void attn_decode_wave(const bf16* __restrict__ q, bf16* __restrict__ k_cache,
+                                                 bf16* __restrict__ v_cache, const int32_t* __restrict__ block_tables,
+                                                 const int32_t* __restrict__ seq_lens, int hq, int hkv, int max_blocks,
+                                                 int split_len, float scale_log2, const RopeArgs& ra, int b, int kvh, int split,
+                                                 int lane, bool append, WriteOut&& write_out) {
   const int G = hq / hkv;
   const int r = lane & 15, g = lane >> 4;
   // Two round trips to memory precede the first MFMA: the sequence's position, its context length, this split's first 64
@@ -280,69 +278,12 @@ __global__ void __launch_bounds__(JOIN ? 512 : 64, 2) attn_decode_kernel(   // 2
   KVChunk<D> cur, nxt;
   auto load_at = [&](KVChunk<D>& c, int blk) {
     const size_t base = (size_t)blk * blk_stride + head_off;
-    load_chunk<D, true>(c, k_cache + base, v_cache + base, lane);
-  };
-  auto write_out = [&](const WaveState<D>& st, float lt) {
-    if constexpr (JOIN) {
-      // the splits meet in LDS and are summed as attn_split_reduce_kernel sums them: the same operations in the same order
-      float2* ml = reinterpret_cast<float2*>(join_lds + nsplit * G * (D + 4));
-      if (col_ok) {
-        float* po = join_lds + (split * G + r) * (D + 4);
-#pragma unroll
-        for (int dt = 0; dt < D / 16; ++dt) *reinterpret_cast<f32x4*>(po + dt * 16 + 4 * g) = st.acc[dt];
-        if (g == 0) ml[split * G + r] = make_float2(st.m, lt);
-      }
-      __syncthreads();
-      for (int i = threadIdx.x; i < G * (D / 4); i += blockDim.x) {
-        const int h = i / (D / 4), e = 4 * (i % (D / 4));
-        float M = -INFINITY;
-        for (int t = 0; t < nsplit; ++t) M = fmaxf(M, ml[t * G + h].x);
-        const float mref = M == -INFINITY ? 0.f : M;
-        f32x4 num = {0.f, 0.f, 0.f, 0.f};
-        float den = 0.f;
-        for (int t = 0; t < nsplit; ++t) {
-          const float2 x = ml[t * G + h];
-          const f32x4 o = *reinterpret_cast<const f32x4*>(join_lds + (t * G + h) * (D + 4) + e);
-          const float f = exp2f(x.x - mref);
-#pragma unroll
-          for (int j = 0; j < 4; ++j) num[j] = fmaf(o[j], f, num[j]);
-          den = fmaf(x.y, f, den);
-        }
-        bf16x4 o;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) o[j] = f2bf(den > 0.f ? num[j] / den : 0.f);
-        *reinterpret_cast<bf16x4*>(out + ((size_t)b * hq + kvh * G + h) * D + e) = o;
-      }
-      return;
-    }
-    if (!col_ok) return;
-    const int h = kvh * G + r;
-    if (nsplit == 1) {
-      // a true division, exactly as the split-reduce computes num / den (bit-identical results
-      // whether a sequence's keys land in one split or in one non-empty split of several)
-      bf16* orow = out + ((size_t)b * hq + h) * D;
-#pragma unroll
-      for (int dt = 0; dt < D / 16; ++dt) {
-        bf16x4 o;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float v = st.acc[dt][i] / (lt > 0.f ? lt : 1.f);      // divided either way: no branch around each
-          o[i] = f2bf(lt > 0.f ? v : 0.f);
-        }
-        *reinterpret_cast<bf16x4*>(orow + dt * 16 + 4 * g) = o;
-      }
-    } else {
-      const size_t pi = ((size_t)b * hq + h) * nsplit + split;
-      float* po = part_o + pi * D;
-#pragma unroll
-      for (int dt = 0; dt < D / 16; ++dt) *reinterpret_cast<f32x4*>(po + dt * 16 + 4 * g) = st.acc[dt];
-      if (g == 0) { part_ml[pi * 2] = st.m; part_ml[pi * 2 + 1] = lt; }
-    }
+    load_chunk<D, NT>(c, k_cache + base, v_cache + base, lane);
   };
   WaveState<D> st;
   init_state(st);
   if (c1 == c0) {                                   // wave-uniform: no key in this split (and not the new one)
-    write_out(st, 0.f);                             // (JOIN: where this wave meets the others at the barrier)
+    write_out(st, 0.f);                             // (joined: where this wave meets the others at the barrier)
     return;
   }
   const int blk_0 = __builtin_amdgcn_readlane(blk_first, 0);
@@ -453,7 +394,7 @@ __global__ void __launch_bounds__(JOIN ? 512 : 64, 2) attn_decode_kernel(   // 2
       // [D][8] V^T tile (2 KiB, 16 full 128-B lines) with the new key patched in -- no partially
       // written lines to read-modify-write.  This is the sequence's last chunk: no KV load follows
       // whose vmcnt wait would include these stores.
-      if (vcol && owns_new) {
+      if (vcol && append) {
 #pragma unroll
         for (int dt = 0; dt < D / 16; ++dt)
           *reinterpret_cast<bf16x8*>(v_cache + cbase + g * 8 * D + (dt * 16 + r) * 8) = c.v[dt];
@@ -493,7 +434,7 @@ __global__ void __launch_bounds__(JOIN ? 512 : 64, 2) attn_decode_kernel(   // 2
       load_at(cur, block(0));
     }
   }
-  if (owns_new) {
+  if (owns_new && append) {
     // append k (row krow32(off)) and v (its [4][D][8] V^T slots) to the paged cache only now, after the
     // last KV load: stores count in vmcnt in issue order, so stores issued before the KV stream
     // made every later chunk wait for their (scattered 2-byte V^T) write acknowledgements
@@ -512,6 +453,212 @@ __global__ void __launch_bounds__(JOIN ? 512 : 64, 2) attn_decode_kernel(   // 2
     }
   }
   write_out(st, rows_sum(st.lsum));                 // (after the last MFMA: divergence is safe)
+}
+
+template <int D, bool FUSED, int PARTS = 0, bool JOIN = false>
+__global__ void __launch_bounds__(JOIN ? 512 : 64, 2) attn_decode_kernel(   // 2nd arg: min waves per SIMD
+    bf16* __restrict__ out, const bf16* __restrict__ q, bf16* __restrict__ k_cache,
+    bf16* __restrict__ v_cache, const int32_t* __restrict__ block_tables,
+    const int32_t* __restrict__ seq_lens, float* __restrict__ part_o, float* __restrict__ part_ml,
+    int hq, int hkv, int max_blocks, int split_len, float scale_log2, RopeArgs ra) {
+  extern __shared__ __attribute__((aligned(16))) float join_lds[];   // JOIN: [split][head][D + 4], then [split][head](m, l)
+  const int kvh = blockIdx.y, b = blockIdx.z;
+  const int lane = threadIdx.x & 63;
+  const int split = JOIN ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : (int)blockIdx.x;
+  const int nsplit = JOIN ? (int)(blockDim.x >> 6) : (int)gridDim.x;
+  const int G = hq / hkv;
+  const int r = lane & 15, g = lane >> 4;
+  const bool col_ok = r < G;
+  auto write_out = [&](const WaveState<D>& st, float lt) {
+    if constexpr (JOIN) {
+      // the splits meet in LDS and are summed as attn_split_reduce_kernel sums them: the same operations in the same order
+      float2* ml = reinterpret_cast<float2*>(join_lds + nsplit * G * (D + 4));
+      if (col_ok) {
+        float* po = join_lds + (split * G + r) * (D + 4);
+#pragma unroll
+        for (int dt = 0; dt < D / 16; ++dt) *reinterpret_cast<f32x4*>(po + dt * 16 + 4 * g) = st.acc[dt];
+        if (g == 0) ml[split * G + r] = make_float2(st.m, lt);
+      }
+      __syncthreads();
+      for (int i = threadIdx.x; i < G * (D / 4); i += blockDim.x) {
+        const int h = i / (D / 4), e = 4 * (i % (D / 4));
+        float M = -INFINITY;
+        for (int t = 0; t < nsplit; ++t) M = fmaxf(M, ml[t * G + h].x);
+        const float mref = M == -INFINITY ? 0.f : M;
+        f32x4 num = {0.f, 0.f, 0.f, 0.f};
+        float den = 0.f;
+        for (int t = 0; t < nsplit; ++t) {
+          const float2 x = ml[t * G + h];
+          const f32x4 o = *reinterpret_cast<const f32x4*>(join_lds + (t * G + h) * (D + 4) + e);
+          const float f = exp2f(x.x - mref);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) num[j] = fmaf(o[j], f, num[j]);
+          den = fmaf(x.y, f, den);
+        }
+        bf16x4 o;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[j] = f2bf(den > 0.f ? num[j] / den : 0.f);
+        *reinterpret_cast<bf16x4*>(out + ((size_t)b * hq + kvh * G + h) * D + e) = o;
+      }
+      return;
+    }
+    if (!col_ok) return;
+    const int h = kvh * G + r;
+    if (nsplit == 1) {
+      // a true division, exactly as the split-reduce computes num / den (bit-identical results
+      // whether a sequence's keys land in one split or in one non-empty split of several)
+      bf16* orow = out + ((size_t)b * hq + h) * D;
+#pragma unroll
+      for (int dt = 0; dt < D / 16; ++dt) {
+        bf16x4 o;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float v = st.acc[dt][i] / (lt > 0.f ? lt : 1.f);      // divided either way: no branch around each
+          o[i] = f2bf(lt > 0.f ? v : 0.f);
+        }
+        *reinterpret_cast<bf16x4*>(orow + dt * 16 + 4 * g) = o;
+      }
+    } else {
+      const size_t pi = ((size_t)b * hq + h) * nsplit + split;
+      float* po = part_o + pi * D;
+#pragma unroll
+      for (int dt = 0; dt < D / 16; ++dt) *reinterpret_cast<f32x4*>(po + dt * 16 + 4 * g) = st.acc[dt];
+      if (g == 0) { part_ml[pi * 2] = st.m; part_ml[pi * 2 + 1] = lt; }
+    }
+  };
+  attn_decode_wave<D, FUSED, PARTS, true>(q, k_cache, v_cache, block_tables, seq_lens, hq, hkv, max_blocks, split_len, scale_log2,
+                                          ra, b, kvh, split, lane, true, write_out);
+}
+
+// ---------------------------------------------------------------------------
+// Decode attention and the o-projection behind it in one launch, for one or two short sequences.  Bound by round trips: attention of one
+// sequence is 8 workgroups (of 8 kv heads) that wait 5 us for four of them while the other CUs idle, and the projection behind it waits 2 us
+// for its first weights.  K slice kvh of the projection is what kv head kvh's query heads give, so a workgroup of (128 columns, kvh) makes
+// that part of its input itself -- as the 31 other workgroups of the head do, out of the same XCD's L2 -- while its whole weight
+// slice is on its way into LDS.  Four waves attend, a (sequence, split of its keys) at a time, and four fetch the weights (loads
+// return in order: a wave that waits for keys would wait for its weights too), 0.9 us later, so that the first round trips of the
+// others are not behind 128 KiB (at once 11.3 us, 0.4 us later 10.5, now 10.2); all eight multiply.  The slices are left as split-K
+// slabs for the next norm.
+// us, attention and projection / this, 32 / 8 heads of 128, 4096 x 4096: one sequence of 37 / 69 / 150 / 256 / 400 / 500 keys 14.6 / 14.1 /
+// 14.0 / 14.7 / 14.3 / 14.9 -> 10.2 / 9.7 / 10.5 / 12.9 / 13.8 / 15.0, two of 30 / 60 / 120 / 200 15.2 / 15.8 / 15.6 / 14.9 -> 10.0 / 11.1 / 12.2 /
+// 14.6.  Every CU reads all keys and values of its head at some 16 KiB per 0.3 us, so that is where it ends: one of 1000 16.0 ->
+// 19.2, four of 200 15.2 -> 19.2, eight of 220 16.2 -> 27.6.
+// ---------------------------------------------------------------------------
+constexpr int kAoFront = 4;               // waves that attend
+constexpr int kAoD = 128;
+
+template <int PARTS>
+__global__ void __launch_bounds__(512, 2) attn_o_kernel(const bf16* __restrict__ W, bf16* __restrict__ k_cache,
+                                                        bf16* __restrict__ v_cache, const int32_t* __restrict__ block_tables,
+                                                        const int32_t* __restrict__ seq_lens, int M, int N, int hq, int hkv,
+                                                        int max_blocks, int split_len, int ns, float scale_log2, RopeArgs ra,
+                                                        float* __restrict__ P) {
+  extern __shared__ __attribute__((aligned(16))) char ao_lds[];   // weights | rows | partial results of split sequences
+  constexpr int D = kAoD;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int G = hq / hkv, K = hq * D, tiles = G * (D / 64);       // K-tiles of 64 in the slice
+  // the workgroups of a kv head on one XCD, as far as they divide
+  int b = blockIdx.x;
+  {
+    const int q = gridDim.x >> 3, r = gridDim.x & 7, x = b & 7;
+    b = (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + (b >> 3);
+  }
+  const int ntiles = N / 128, kvh = b / ntiles, n_t = b - kvh * ntiles;
+  const int wbytes = tiles * 16384, pitch = G * D * 2;
+  char* rows = ao_lds + wbytes;
+  float* part = reinterpret_cast<float*>(rows + ((M * pitch + 15) & ~15));      // [task][head][D + 4]
+  float2* ml = reinterpret_cast<float2*>(part + (ns > 1 ? M * ns * G * (D + 4) : 0));
+  const int r = lane & 15, g = lane >> 4;
+  // element e (a multiple of 4) of row m: 16-byte chunks swizzled in each 128 bytes
+  auto row_at = [&](int m, int e) {
+    const int c = e >> 3;
+    return reinterpret_cast<bf16x4*>(rows + m * pitch + ((c & ~7) | ((c ^ m) & 7)) * 16 + (e & 4) * 2);
+  };
+  if (wv >= kAoFront) {
+    const int w = wv - kAoFront;
+    const char* src[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int q = w * 4 + j, row = 8 * q + (lane >> 3);
+      src[j] = reinterpret_cast<const char*>(W) + ((size_t)(n_t * 128 + row) * K + (size_t)kvh * G * D) * 2 +
+               ((lane & 7) ^ ((row >> 1) & 7)) * 16;
+    }
+    __builtin_amdgcn_s_sleep(32);                    // (0.9 us: see above)
+    for (int t = 0; t < tiles; ++t)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        __builtin_amdgcn_global_load_lds((glb_vptr_a)(src[j] + t * 128), (lds_vptr_a)(ao_lds + t * 16384 + (w * 4 + j) * 1024), 16, 0, 2);
+    if (ns > 1) __builtin_amdgcn_s_barrier();
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  } else {
+    for (int task = wv; task < M * ns; task += kAoFront) {
+      const int m = task / ns, split = task - m * ns;
+      auto write_out = [&](const WaveState<D>& st, float lt) {
+        if (r >= G) return;
+        if (ns > 1) {
+          float* po = part + (task * G + r) * (D + 4);
+#pragma unroll
+          for (int dt = 0; dt < D / 16; ++dt) *reinterpret_cast<f32x4*>(po + dt * 16 + 4 * g) = st.acc[dt];
+          if (g == 0) ml[task * G + r] = make_float2(st.m, lt);
+          return;
+        }
+#pragma unroll
+        for (int dt = 0; dt < D / 16; ++dt) {
+          bf16x4 o;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float v = st.acc[dt][i] / (lt > 0.f ? lt : 1.f);
+            o[i] = f2bf(lt > 0.f ? v : 0.f);
+          }
+          *row_at(m, r * D + dt * 16 + 4 * g) = o;
+        }
+      };
+      attn_decode_wave<D, true, PARTS, false>(nullptr, k_cache, v_cache, block_tables, seq_lens, hq, hkv, max_blocks, split_len,
+                                              scale_log2, ra, m, kvh, split, lane, n_t == 0, write_out);
+    }
+    if (ns > 1) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      for (int i = threadIdx.x; i < M * G * (D / 4); i += kAoFront * 64) {
+        const int e = 4 * (i % (D / 4)), mh = i / (D / 4), m = mh / G, h = mh - m * G;
+        float top = -INFINITY;
+        for (int t = 0; t < ns; ++t) top = fmaxf(top, ml[(m * ns + t) * G + h].x);
+        const float mref = top == -INFINITY ? 0.f : top;
+        f32x4 num = {0.f, 0.f, 0.f, 0.f};
+        float den = 0.f;
+        for (int t = 0; t < ns; ++t) {
+          const float2 x = ml[(m * ns + t) * G + h];
+          const f32x4 o = *reinterpret_cast<const f32x4*>(part + ((m * ns + t) * G + h) * (D + 4) + e);
+          const float f = exp2f(x.x - mref);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) num[j] = fmaf(o[j], f, num[j]);
+          den = fmaf(x.y, f, den);
+        }
+        bf16x4 o;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[j] = f2bf(den > 0.f ? num[j] / den : 0.f);
+        *row_at(m, h * D + e) = o;
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  }
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  const int wrow = wv * 16 + r, ar = min(r, M - 1);
+  const char* pb = ao_lds + wrow * 128;
+  const char* pa = rows + ar * pitch;
+  const int bo0 = (g ^ ((r >> 1) & 7)) * 16, bo1 = ((4 + g) ^ ((r >> 1) & 7)) * 16;
+  const int ao0 = ((g ^ ar) & 7) * 16, ao1 = (((4 + g) ^ ar) & 7) * 16;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int t = 0; t < tiles; ++t) {
+    const bf16x8 b0 = *reinterpret_cast<const bf16x8*>(pb + t * 16384 + bo0), b1 = *reinterpret_cast<const bf16x8*>(pb + t * 16384 + bo1);
+    const bf16x8 a0 = *reinterpret_cast<const bf16x8*>(pa + t * 128 + ao0), a1 = *reinterpret_cast<const bf16x8*>(pa + t * 128 + ao1);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b0, a0, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b1, a1, acc, 0, 0, 0);
+  }
+  if (r < M) part_store4(P, ((size_t)kvh * M + r) * N + n_t * 128 + wv * 16 + 4 * g, acc);
 }
 
 // Rounds of kRound splits, every load of a round before its first use: one round trip for up to kRound splits (plain loops
@@ -1691,6 +1838,40 @@ void paged_attention_decode_rope(uintptr_t out, uintptr_t qkv, uintptr_t positio
               (const float*)qkv_part, qkv_nparts, qkv_slab};
   decode_launch(out, 0, k_cache, v_cache, block_tables, seq_lens, part_o, part_ml, batch, hq, hkv, d, block_size,
                 max_blocks, num_splits, split_len, scale, ra, true, stream);
+}
+
+// LDS of attn_o_kernel
+static long attn_o_bytes(int batch, int hq, int hkv, int ns) {
+  const int g = hq / hkv;
+  return (long)g * (kAoD / 64) * 16384 + (((long)batch * g * kAoD * 2 + 15) & ~15L) + (ns > 1 ? (long)batch * ns * g * (kAoD + 6) * 4 : 0);
+}
+
+// paged_attention_decode_rope of heads of 128 and slab kvh of [hkv, batch, n] at `slabs` = its heads' part of the product with wo [n, hq * 128]
+void attn_o(uintptr_t slabs, uintptr_t wo, int n, uintptr_t qkv, uintptr_t positions, uintptr_t cos_sin, uintptr_t slots,
+            uintptr_t k_cache, uintptr_t v_cache, uintptr_t block_tables, uintptr_t seq_lens, int batch, int hq, int hkv,
+            int block_size, int max_blocks, int num_splits, int split_len, float scale, uintptr_t qkv_part, int qkv_nparts,
+            long qkv_slab, uintptr_t stream) {
+  DLLM_HOST_CHECK(block_size == kBS, "paged attention requires block_size 32");
+  DLLM_HOST_CHECK(hq % hkv == 0 && hq / hkv <= 16 && batch >= 1 && batch <= 16 && n % 128 == 0, "sizes");
+  DLLM_HOST_CHECK(num_splits >= 1 && split_len % kBS == 0 && split_len > 0, "split_len multiple of 32");
+  DLLM_HOST_CHECK((qkv || qkv_part) && positions && slots, "fused decode needs qkv, positions, slots");
+  DLLM_HOST_CHECK(qkv_part == 0 || (qkv_nparts >= 1 && qkv_slab >= (long)batch * (hq + 2 * hkv) * kAoD), "qkv partial slabs");
+  const long lds = attn_o_bytes(batch, hq, hkv, num_splits);
+  DLLM_HOST_CHECK(lds <= 160 * 1024, "LDS");
+  RopeArgs ra{(const bf16*)qkv, (const int32_t*)positions, (const float*)cos_sin, (const int32_t*)slots,
+              (const float*)qkv_part, qkv_nparts, qkv_slab};
+  auto go = [&](auto kern) {
+    DLLM_HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+    hipLaunchKernelGGL(kern, dim3((unsigned)(n / 128 * hkv)), dim3(512), lds, reinterpret_cast<hipStream_t>(stream), (const bf16*)wo,
+                       (bf16*)k_cache, (bf16*)v_cache, (const int32_t*)block_tables, (const int32_t*)seq_lens, batch, n, hq, hkv,
+                       max_blocks, split_len, num_splits, scale * 1.4426950408889634f, ra, (float*)slabs);
+  };
+  if (qkv_part == 0) go(attn_o_kernel<0>);
+  else if (qkv_nparts == 5) go(attn_o_kernel<5>);
+  else if (qkv_nparts == 4) go(attn_o_kernel<4>);
+  else if (qkv_nparts == 8) go(attn_o_kernel<8>);
+  else go(attn_o_kernel<-1>);
+  DLLM_HIP_CHECK(hipGetLastError());
 }
 
 template <int D>

@@ -348,6 +348,15 @@ class ModelStage:
                                            max_ctx=meta.max_ctx or None, workspace=meta.attn_workspace)
         return o.view(o.shape[0], self.q_size_local)
 
+    def _attention_o(self, qkv, li: int, meta: BatchMeta, wo):
+        """Decode attention and the o-projection in one launch (one or two short sequences), or None."""
+        if meta.is_prefill or not knobs.K.fused_rope or not knobs.K.defer_o:
+            return None
+        k_cache, v_cache = self.kv.layer(li)
+        return ops.paged_attention_decode_o(qkv, meta.positions, self.cos_sin, k_cache, v_cache, meta.slot_mapping,
+                                            meta.block_tables, meta.seq_lens, self.hq, self.hkv, self.cfg.head_dim, self.scale,
+                                            wo, max_ctx=meta.max_ctx or None)
+
     def _mlp(self, h: Optional[torch.Tensor], lw: Dict[str, torch.Tensor], gated: Optional[torch.Tensor] = None) -> torch.Tensor:
         """``gated``: the dense MLP's activation, where the launch of its norm has made it already (``h`` is None then)."""
         if self.cfg.is_moe:
@@ -415,11 +424,14 @@ class ModelStage:
                         out_aux = self._dense(qkv)
                         break
                 if self.has(l, 1):
-                    a = self._attention(qkv if qkv is not None else carry, self.kv_index[l], meta)
+                    if self.has(l, 2) and not self.tp.enabled:
+                        h = self._attention_o(qkv if qkv is not None else carry, self.kv_index[l], meta, lw["wo"])
+                    if h is None:
+                        a = self._attention(qkv if qkv is not None else carry, self.kv_index[l], meta)
                     if not self.has(l, 2):
                         out_aux = a
                         break
-                if self.has(l, 2):
+                if self.has(l, 2) and h is None:
                     a = a if a is not None else carry
                     # defer: a split-K o-projection's reduce is fused into the MLP half's add + RMSNorm
                     # (TP: row-parallel partial sums, all-reduced over the group)

@@ -378,6 +378,57 @@ def paged_attention_decode_rope(qkv, positions, cos_sin, k_cache, v_cache, slot_
     return out
 
 
+def attn_o_splits(batch: int, max_ctx: int, hq: int, hkv: int, d: int, n: int) -> int:
+    """Splits of a sequence's keys in :func:`paged_attention_decode_o`, 0 where it does not serve the call: one or two sequences of up to
+    512 keys together (longer ones, and more, are slower than two launches: csrc/kernels/attention.hip, attn_o_kernel), a slice of at most
+    512 projection inputs per kv head (its weights fill the LDS), one round of workgroups that keeps three quarters of the CUs busy.  On the
+    context's bucket, as the decode graphs have it, so that a graph and the eager path take the same way."""
+    bucket = max(256, 1 << max(0, max_ctx - 1).bit_length())
+    if not (knobs.K.one and d == 128 and hq % hkv == 0 and hq // hkv <= 4 and n % 128 == 0 and 192 <= n // 128 * hkv <= 256
+            and batch <= 2 and batch * bucket <= 512) or gemm._comm_cus:
+        return 0
+    return 4 if batch * bucket == 256 else 2
+
+
+def paged_attention_decode_o(qkv, positions, cos_sin, k_cache, v_cache, slot_mapping, block_tables, seq_lens, num_heads: int,
+                             num_kv_heads: int, head_dim: int, scale: float, wo, max_ctx: Optional[int] = None):
+    """:func:`paged_attention_decode_rope` and the deferred :func:`linear` with ``wo`` [N, Hq * D] behind it in one launch: a
+    :class:`gemm.SplitKPartial` with a slab per kv head, or None where they have launches of their own (:func:`attn_o_splits`)."""
+    part = qkv if isinstance(qkv, gemm.SplitKPartial) else None
+    if isinstance(wo, quant.Fp8Weight) or not k_cache.is_cuda or block_tables.dim() != 2 or not block_tables.shape[1]:
+        return None
+    b, width = (part.m, part.n) if part is not None else (qkv.shape[0], qkv.shape[-1])
+    hq, hkv, d, bs, max_blocks = num_heads, num_kv_heads, head_dim, k_cache.shape[2], block_tables.shape[1]
+    max_ctx = max_ctx or max_blocks * bs
+    n = wo.shape[0]
+    ns = attn_o_splits(b, max_ctx, hq, hkv, d, n)
+    if not ns or b < 1 or bs != 32 or max_ctx > max_blocks * bs or width != (hq + 2 * hkv) * d:
+        return None
+    if not (wo.dim() == 2 and wo.shape[1] == hq * d and wo.dtype == torch.bfloat16 and wo.is_contiguous() and wo.data_ptr() % 16 == 0
+            and wo.device == k_cache.device):
+        return None
+    if part is None:
+        _ck(qkv, "attn.qkv")
+    elif len(part.shape) != 2:
+        return None
+    _ck(k_cache, "k_cache")
+    _ck(v_cache, "v_cache")
+    for t, name in ((positions, "positions"), (slot_mapping, "slot_mapping"), (block_tables, "block_tables"), (seq_lens, "seq_lens")):
+        _ck(t, name, torch.int32)
+    if cos_sin is not None:
+        _ck(cos_sin, "cos_sin", torch.float32)
+        if cos_sin.shape[1] != d:
+            raise ValueError("cos_sin width must equal head_dim")
+    bucket = max(256, 1 << (max_ctx - 1).bit_length())
+    ws = gemm.slab_space(k_cache.device, part)
+    _ext.kernels().attn_o(ws.data_ptr(), wo.data_ptr(), n, 0 if part is not None else qkv.data_ptr(), positions.data_ptr(),
+                          0 if cos_sin is None else cos_sin.data_ptr(), slot_mapping.data_ptr(), k_cache.data_ptr(),
+                          v_cache.data_ptr(), block_tables.data_ptr(), seq_lens.data_ptr(), b, hq, hkv, bs, max_blocks, ns,
+                          -(-bucket // (bs * ns)) * bs, float(scale), 0 if part is None else part.ws.data_ptr(),
+                          0 if part is None else part.splits, 0 if part is None else part.m * part.n, _stream())
+    return gemm.SplitKPartial(ws, hkv, b, n, (b, n), torch.bfloat16, k_cache.device)
+
+
 def prefill_attn_version(max_q_len: int, head_dim: int) -> int:
     """The prefill attention kernel for a batch: knobs.prefill_attn, or with 0 (auto) from
     knobs.prefill_w32_min_q query rows at head_dim 128 the persistent 32x32x16 kernel (9: 1.1x v4 at

@@ -426,6 +426,13 @@ def _workspace(device: torch.device) -> torch.Tensor:
     return t
 
 
+def slab_space(device: torch.device, read: Optional[SplitKPartial]) -> torch.Tensor:
+    """Where a launch that reads ``read`` may leave its own slabs (of up to half the workspace): the start of the workspace, or its
+    second half where ``read`` lies at the start."""
+    ws = _workspace(device)
+    return ws[ws.numel() // 2:] if read is not None and read.ws.data_ptr() == ws.data_ptr() else ws
+
+
 def wide_bm(m: int) -> int:
     """Row tile of gemm_wide for M rows (mirrors wide_bm in csrc/kernels/gemm_wide.hip)."""
     if m <= 64:
@@ -565,17 +572,14 @@ def one_fits(n: int, k: int, s: int, swiglu: bool = False) -> bool:
 
 def _one(like: torch.Tensor, w: torch.Tensor, s: int, swiglu: bool, lead, x=None, residual=None, part=None, norm_w=None,
          res_out=None, eps: float = 0.0):
-    """gemm_one's launch: the finished product of one row, or its :class:`SplitKPartial` (``s`` > 1).  Slabs that are read lie at the
-    start of the workspace or in its second half, and those that are written in the other."""
+    """gemm_one's launch: the finished product of one row, or its :class:`SplitKPartial` (``s`` > 1)."""
     n, k = w.shape
     p = lambda t: 0 if t is None else t.data_ptr()
     nt = 1 if n * k * 2 >= WIDE_NT_MIN_BYTES else 0
     args = (p(x), p(residual), 0 if part is None else part.ws.data_ptr(), 0 if part is None else part.splits, p(norm_w), p(res_out),
             float(eps), current_stream())
     if s > 1:
-        ws = _workspace(like.device)
-        if part is not None and part.ws.data_ptr() == ws.data_ptr():
-            ws = ws[ws.numel() // 2:]
+        ws = slab_space(like.device, part)
         se = _ext.kernels().gemm_one(0, ws.data_ptr(), w.data_ptr(), n, k, s, 2, nt, *args)
         return SplitKPartial(ws, se, 1, n, (*lead, n), like.dtype, like.device)
     y = torch.empty(*lead, n // 2 if swiglu else n, dtype=like.dtype, device=like.device)
