@@ -450,7 +450,7 @@ def wide_row_tile(m: int, n: int, k: int, swiglu: bool = False) -> int:
     """Row tile gemm_wide uses for this shape (knobs.wide_small_bm for small split grids, else
     wide_bm): e.g. 128 runs an M = 256 o-projection as 2 row tiles x 4 K slices instead of 1 x 8."""
     kn = knobs.K
-    if kn.wide_small_bm and not swiglu and n * k <= kn.wide_small_bm_maxw and kn.wide_small_bm < wide_bm(m):
+    if kn.wide_small_bm and not swiglu and n * k <= kn.wide_small_bm_maxw and kn.wide_small_bm < wide_bm(m) and m <= 256:
         return kn.wide_small_bm
     return wide_bm(m)
 
@@ -545,6 +545,8 @@ def linear_wide(x: torch.Tensor, w: torch.Tensor, splits: int = 0, swiglu: bool 
         s = max(1, ws.numel() // (m * n))
     stream = current_stream()
     bm = wide_row_tile(m, n, k, swiglu)
+    if not splits and variant < 0 and duo_fits(m, n, k, s, bm, swiglu) and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0:
+        return _duo(x, w, m, n, k, s, bm, swiglu, defer)
     v = variant if variant >= 0 else wide_variant(m, n, k, s, bm)
     if bm != wide_bm(m):
         v |= bm << 8
@@ -555,6 +557,29 @@ def linear_wide(x: torch.Tensor, w: torch.Tensor, splits: int = 0, swiglu: bool 
     _ext.kernels().gemm_wide(y.data_ptr(), x.data_ptr(), w.data_ptr(), ws.data_ptr(), ws.numel(), m, n, k, s,
                              1 if swiglu else 0, v, stream)
     return y
+
+
+def duo_fits(m: int, n: int, k: int, s: int, bm: int, swiglu: bool = False) -> bool:
+    """Does gemm_duo serve an [m, k] x [n, k]^T product in ``s`` K slices on row tiles of ``bm`` (gemm_wide's plan, whose bits it has)?  GLUs from 65
+    rows on, slabs from 129 (up to 128 rows they are equal: 4096 x 14336 with its norm 29.8 / 29.8 us, 6144 x 4096 16.6 / 16.6), where
+    the workgroups keep three quarters of the CUs busy: its four waves take twice as long over a K-tile as gemm_wide's eight where
+    nothing else bounds them.  us, gemm_wide / this at 256 rows: 2048 x 2048 (64 workgroups) 12.0 / 14.1, 2560 x 2560 (100) 13.8 / 15.6,
+    4096 x 2048 (128) 15.0 / 15.5, 8192 x 8192 (256) 45.4 / 43.6."""
+    rows = 64 < m <= 256 and s == 1 if swiglu else 128 < m <= 512 and s > 1
+    return (knobs.K.duo and rows and bm in (128, 192, 256) and n % 128 == 0 and k % 64 == 0 and n // 128 * s * -(-m // bm) >= 192
+            and m * k * 2 < 1 << 32 and n * k * 2 < 1 << 32)
+
+
+def _duo(x: torch.Tensor, w: torch.Tensor, m: int, n: int, k: int, s: int, bm: int, swiglu: bool, defer: bool):
+    """gemm_duo's launch: the SwiGLU, or the slabs' :class:`SplitKPartial` (summed without ``defer``)."""
+    ws = _workspace(x.device)
+    y = torch.empty(*x.shape[:-1], n // 2, dtype=x.dtype, device=x.device) if swiglu else None
+    se = _ext.kernels().gemm_duo(y.data_ptr() if swiglu else 0, x.data_ptr(), w.data_ptr(), ws.data_ptr(), ws.numel(), m, n, k, s,
+                                 swiglu, bm, current_stream())
+    if swiglu:
+        return y
+    part = SplitKPartial(ws, se, m, n, (*x.shape[:-1], n), x.dtype, x.device)
+    return part if defer else part.materialize()
 
 
 ONE_MAX_WIDTH = 8192               # (csrc/kernels/gemm_one.hip: a row, or its slice, in the registers of four waves)
@@ -641,6 +666,9 @@ def linear_pp(x: torch.Tensor, w: torch.Tensor, splits: int = 0, swiglu: bool = 
     ws = _workspace(x.device)
     if s > 1 and s * m * n > ws.numel():
         s = max(1, ws.numel() // (m * n))
+    if swiglu and variant == PP_GATE_UP_VARIANT and s == 1 and duo_fits(m, n, k, s, wide_bm(m), True) and x.data_ptr() % 16 == 0 \
+            and w.data_ptr() % 16 == 0:
+        return _duo(x, w, m, n, k, s, wide_bm(m), True, False)
     stream = current_stream()
     if defer and not swiglu and s > 1:
         se = _ext.kernels().gemm_pp(0, x.data_ptr(), w.data_ptr(), ws.data_ptr(), ws.numel(), m, n, k, s, 2, variant,
@@ -803,8 +831,8 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor) -> Optional[torch.Te
         return _stream(m, n, k, x, w_gate_up, glu="silu")
     if 0 < kn.pp_gate_up_min_m <= m <= 256 and not _comm_cus and _use_pp(m, n, k, x, w_gate_up, 1):
         # decode gate|up on gemm_pp, unsplit, weights nontemporal, on the column tile that gives one
-        # round of CUs / 2 .. CUs tiles: 8B (224 x 128 columns) 62.1 vs 64.1 us for gemm_wide, 70B
-        # (224 x 256 columns) 204 vs 259 us for gemm_sq (bench/debug/medium_m_sweep.py --pp)
+        # round of CUs / 2 .. CUs tiles: 8B (224 x 128 columns) 62.1 vs 64.1 us for gemm_wide (57.5 on gemm_duo, which
+        # linear_pp takes for these), 70B (224 x 256 columns) 204 vs 259 us for gemm_sq (bench/debug/medium_m_sweep.py --pp)
         cus = _cus(x.device)
         if n % 128 == 0 and cus // 2 <= n // 128 <= cus:
             return linear_pp(x, w_gate_up, splits=1, swiglu=True, variant=PP_GATE_UP_VARIANT)
