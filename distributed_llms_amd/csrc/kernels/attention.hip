@@ -544,8 +544,61 @@ __global__ void __launch_bounds__(JOIN ? 512 : 64, 2) attn_decode_kernel(   // 2
 // 14.6.  Every CU reads all keys and values of its head at some 16 KiB per 0.3 us, so that is where it ends: one of 1000 16.0 ->
 // 19.2, four of 200 15.2 -> 19.2, eight of 220 16.2 -> 27.6.
 // ---------------------------------------------------------------------------
-constexpr int kAoFront = 4;               // waves that attend
+constexpr int kAoFront = 4;               // waves that make the input
 constexpr int kAoD = 128;
+
+// A workgroup's place: (128 columns, kv head), the workgroups of a head on one XCD as far as they divide
+__device__ __forceinline__ void ao_place(int ntiles, int& kvh, int& n_t) {
+  const int q = gridDim.x >> 3, r = gridDim.x & 7, x = blockIdx.x & 7;
+  const int b = (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + (int)(blockIdx.x >> 3);
+  kvh = b / ntiles;
+  n_t = b - kvh * ntiles;
+}
+
+// The weight slice W[128 n_t .. + 127][G D kvh .. + G D - 1] to LDS, K-tiles of 64 with chunks swizzled, by wave w of the four that fetch
+__device__ __forceinline__ void ao_weights(const bf16* __restrict__ W, char* lds, int K, int slice, int kvh, int n_t, int w, int lane) {
+  const char* src[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int row = 8 * (w * 4 + j) + (lane >> 3);
+    src[j] = reinterpret_cast<const char*>(W) + ((size_t)(n_t * 128 + row) * K + (size_t)kvh * slice) * 2 + ((lane & 7) ^ ((row >> 1) & 7)) * 16;
+  }
+  for (int t = 0; t < slice / 64; ++t)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      __builtin_amdgcn_global_load_lds((glb_vptr_a)(src[j] + t * 128), (lds_vptr_a)(lds + t * 16384 + (w * 4 + j) * 1024), 16, 0, 2);
+}
+
+// Element e (a multiple of 4) of input row m in LDS: 16-byte chunks swizzled in each 128 bytes
+__device__ __forceinline__ bf16x4* ao_row(char* rows, int pitch, int m, int e) {
+  const int c = e >> 3;
+  return reinterpret_cast<bf16x4*>(rows + m * pitch + ((c & ~7) | ((c ^ m) & 7)) * 16 + (e & 4) * 2);
+}
+
+// Slab kvh of the M rows, by all eight waves
+__device__ __forceinline__ void ao_product(const char* lds, const char* rows, float* __restrict__ P, int M, int N, int slice, int kvh, int n_t,
+                                           int wv, int lane) {
+  const int r = lane & 15, g = lane >> 4, ar = min(r, M - 1);
+  const char* pb = lds + (wv * 16 + r) * 128;
+  const char* pa = rows + ar * slice * 2;
+  const int bo0 = (g ^ ((r >> 1) & 7)) * 16, bo1 = ((4 + g) ^ ((r >> 1) & 7)) * 16;
+  const int ao0 = ((g ^ ar) & 7) * 16, ao1 = (((4 + g) ^ ar) & 7) * 16;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int t = 0; t < slice / 64; ++t) {
+    const bf16x8 b0 = *reinterpret_cast<const bf16x8*>(pb + t * 16384 + bo0), b1 = *reinterpret_cast<const bf16x8*>(pb + t * 16384 + bo1);
+    const bf16x8 a0 = *reinterpret_cast<const bf16x8*>(pa + t * 128 + ao0), a1 = *reinterpret_cast<const bf16x8*>(pa + t * 128 + ao1);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b0, a0, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b1, a1, acc, 0, 0, 0);
+  }
+  if (r < M) part_store4(P, ((size_t)kvh * M + r) * N + n_t * 128 + wv * 16 + 4 * g, acc);
+}
+
+__device__ __forceinline__ void ao_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
 
 template <int PARTS>
 __global__ void __launch_bounds__(512, 2) attn_o_kernel(const bf16* __restrict__ W, bf16* __restrict__ k_cache,
@@ -556,41 +609,19 @@ __global__ void __launch_bounds__(512, 2) attn_o_kernel(const bf16* __restrict__
   extern __shared__ __attribute__((aligned(16))) char ao_lds[];   // weights | rows | partial results of split sequences
   constexpr int D = kAoD;
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int G = hq / hkv, K = hq * D, tiles = G * (D / 64);       // K-tiles of 64 in the slice
-  // the workgroups of a kv head on one XCD, as far as they divide
-  int b = blockIdx.x;
-  {
-    const int q = gridDim.x >> 3, r = gridDim.x & 7, x = b & 7;
-    b = (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + (b >> 3);
-  }
-  const int ntiles = N / 128, kvh = b / ntiles, n_t = b - kvh * ntiles;
-  const int wbytes = tiles * 16384, pitch = G * D * 2;
-  char* rows = ao_lds + wbytes;
-  float* part = reinterpret_cast<float*>(rows + ((M * pitch + 15) & ~15));      // [task][head][D + 4]
+  const int G = hq / hkv, slice = G * D, pitch = slice * 2;
+  int kvh, n_t;
+  ao_place(N / 128, kvh, n_t);
+  char* rows = ao_lds + slice * 256;
+  float* part = reinterpret_cast<float*>(rows + M * pitch);       // [task][head][D + 4]
   float2* ml = reinterpret_cast<float2*>(part + (ns > 1 ? M * ns * G * (D + 4) : 0));
-  const int r = lane & 15, g = lane >> 4;
-  // element e (a multiple of 4) of row m: 16-byte chunks swizzled in each 128 bytes
-  auto row_at = [&](int m, int e) {
-    const int c = e >> 3;
-    return reinterpret_cast<bf16x4*>(rows + m * pitch + ((c & ~7) | ((c ^ m) & 7)) * 16 + (e & 4) * 2);
-  };
   if (wv >= kAoFront) {
-    const int w = wv - kAoFront;
-    const char* src[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int q = w * 4 + j, row = 8 * q + (lane >> 3);
-      src[j] = reinterpret_cast<const char*>(W) + ((size_t)(n_t * 128 + row) * K + (size_t)kvh * G * D) * 2 +
-               ((lane & 7) ^ ((row >> 1) & 7)) * 16;
-    }
-    __builtin_amdgcn_s_sleep(32);                    // (0.9 us: see above)
-    for (int t = 0; t < tiles; ++t)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        __builtin_amdgcn_global_load_lds((glb_vptr_a)(src[j] + t * 128), (lds_vptr_a)(ao_lds + t * 16384 + (w * 4 + j) * 1024), 16, 0, 2);
+    __builtin_amdgcn_s_sleep(32);                      // (0.9 us: see above)
+    ao_weights(W, ao_lds, hq * D, slice, kvh, n_t, wv - kAoFront, lane);
     if (ns > 1) __builtin_amdgcn_s_barrier();
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   } else {
+    const int r = lane & 15, g = lane >> 4;
     for (int task = wv; task < M * ns; task += kAoFront) {
       const int m = task / ns, split = task - m * ns;
       auto write_out = [&](const WaveState<D>& st, float lt) {
@@ -610,16 +641,14 @@ __global__ void __launch_bounds__(512, 2) attn_o_kernel(const bf16* __restrict__
             const float v = st.acc[dt][i] / (lt > 0.f ? lt : 1.f);
             o[i] = f2bf(lt > 0.f ? v : 0.f);
           }
-          *row_at(m, r * D + dt * 16 + 4 * g) = o;
+          *ao_row(rows, pitch, m, r * D + dt * 16 + 4 * g) = o;
         }
       };
       attn_decode_wave<D, true, PARTS, false>(nullptr, k_cache, v_cache, block_tables, seq_lens, hq, hkv, max_blocks, split_len,
                                               scale_log2, ra, m, kvh, split, lane, n_t == 0, write_out);
     }
     if (ns > 1) {
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      __builtin_amdgcn_s_barrier();
-      asm volatile("" ::: "memory");
+      ao_barrier();
       for (int i = threadIdx.x; i < M * G * (D / 4); i += kAoFront * 64) {
         const int e = 4 * (i % (D / 4)), mh = i / (D / 4), m = mh / G, h = mh - m * G;
         float top = -INFINITY;
@@ -638,27 +667,74 @@ __global__ void __launch_bounds__(512, 2) attn_o_kernel(const bf16* __restrict__
         bf16x4 o;
 #pragma unroll
         for (int j = 0; j < 4; ++j) o[j] = f2bf(den > 0.f ? num[j] / den : 0.f);
-        *row_at(m, h * D + e) = o;
+        *ao_row(rows, pitch, m, h * D + e) = o;
       }
     }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   }
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-  const int wrow = wv * 16 + r, ar = min(r, M - 1);
-  const char* pb = ao_lds + wrow * 128;
-  const char* pa = rows + ar * pitch;
-  const int bo0 = (g ^ ((r >> 1) & 7)) * 16, bo1 = ((4 + g) ^ ((r >> 1) & 7)) * 16;
-  const int ao0 = ((g ^ ar) & 7) * 16, ao1 = (((4 + g) ^ ar) & 7) * 16;
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-  for (int t = 0; t < tiles; ++t) {
-    const bf16x8 b0 = *reinterpret_cast<const bf16x8*>(pb + t * 16384 + bo0), b1 = *reinterpret_cast<const bf16x8*>(pb + t * 16384 + bo1);
-    const bf16x8 a0 = *reinterpret_cast<const bf16x8*>(pa + t * 128 + ao0), a1 = *reinterpret_cast<const bf16x8*>(pa + t * 128 + ao1);
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b0, a0, acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b1, a1, acc, 0, 0, 0);
+  ao_barrier();
+  ao_product(ao_lds, rows, P, M, N, slice, kvh, n_t, wv, lane);
+}
+
+// The join of split sequences and the o-projection in one launch, the same way: four waves join a kv head's heads (with the operations of
+// attn_split_reduce_kernel in their order) while four fetch the weight slice.  us, attention, join and projection in three launches / in
+// two, 32 / 8 heads of 128, 4096 x 4096: 3 / 4 / 6 / 8 sequences in 4 splits 15.6 / 15.7 / 15.6 / 16.2 -> 13.9 / 14.1 / 14.2 / 15.5, 4 in 8 15.5 -> 14.8, 1 and 2 in 16
+// 15.6 / 16.2 -> 14.0 / 14.9.  Past 32 splits in all every CU reads too much of them: 12 in 4 17.2 -> 18.2, 8 in 8 17.4 -> 18.8.
+template <int NS>
+__global__ void __launch_bounds__(512, 2) join_o_kernel(const bf16* __restrict__ W, const float* __restrict__ part_o,
+                                                        const float* __restrict__ part_ml, int M, int N, int hq, int hkv, int ns,
+                                                        float* __restrict__ P) {
+  extern __shared__ __attribute__((aligned(16))) char jo_lds[];   // weights | rows
+  constexpr int D = kAoD, U = NS <= 4 ? 4 : NS <= 8 ? 2 : 1;      // pieces of 4 elements whose loads are under way together
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int G = hq / hkv, slice = G * D;
+  int kvh, n_t;
+  ao_place(N / 128, kvh, n_t);
+  char* rows = jo_lds + slice * 256;
+  if (wv >= kAoFront) {
+    ao_weights(W, jo_lds, hq * D, slice, kvh, n_t, wv - kAoFront, lane);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  } else {
+    const int items = M * G * (D / 4);
+    for (int i0 = threadIdx.x; i0 < items; i0 += U * kAoFront * 64) {
+      f32x4 o[U][NS];
+      f32x2 x[U][NS];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {                    // past the last piece and the last split: those again, dropped
+        const int i = min(i0 + u * kAoFront * 64, items - 1), mh = i / (D / 4), m = mh / G;
+        const size_t at = ((size_t)m * hq + kvh * G + mh - m * G) * ns;
+#pragma unroll
+        for (int t = 0; t < NS; ++t) {
+          const size_t p = at + min(t, ns - 1);
+          x[u][t] = *reinterpret_cast<const f32x2*>(part_ml + 2 * p);
+          o[u][t] = *reinterpret_cast<const f32x4*>(part_o + p * D + 4 * (i % (D / 4)));
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int i = i0 + u * kAoFront * 64, mh = i / (D / 4), m = mh / G;
+        float top = -INFINITY;
+#pragma unroll
+        for (int t = 0; t < NS; ++t) top = fmaxf(top, x[u][t][0]);
+        const float mref = top == -INFINITY ? 0.f : top;
+        f32x4 num = {0.f, 0.f, 0.f, 0.f};
+        float den = 0.f;
+#pragma unroll
+        for (int t = 0; t < NS; ++t) {
+          const float f = exp2f(x[u][t][0] - mref);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) num[j] = t < ns ? fmaf(o[u][t][j], f, num[j]) : num[j];
+          den = t < ns ? fmaf(x[u][t][1], f, den) : den;
+        }
+        bf16x4 r;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) r[j] = f2bf(den > 0.f ? num[j] / den : 0.f);
+        if (i < items) *ao_row(rows, slice * 2, m, (mh - m * G) * D + 4 * (i % (D / 4))) = r;
+      }
+    }
   }
-  if (r < M) part_store4(P, ((size_t)kvh * M + r) * N + n_t * 128 + wv * 16 + 4 * g, acc);
+  ao_barrier();
+  ao_product(jo_lds, rows, P, M, N, slice, kvh, n_t, wv, lane);
 }
 
 // Rounds of kRound splits, every load of a round before its first use: one round trip for up to kRound splits (plain loops
@@ -1740,10 +1816,11 @@ __global__ void __launch_bounds__(kW32Waves * 64, 1) attn_prefill_w32p_kernel(
 }
 
 // ------------------------------------------------------------------ launchers
-static void decode_launch(uintptr_t out, uintptr_t q, uintptr_t k_cache, uintptr_t v_cache, uintptr_t block_tables,
+// Returns whether the splits' partial results are left for the caller to join (only where `leave` allows it)
+static bool decode_launch(uintptr_t out, uintptr_t q, uintptr_t k_cache, uintptr_t v_cache, uintptr_t block_tables,
                           uintptr_t seq_lens, uintptr_t part_o, uintptr_t part_ml, int batch, int hq, int hkv, int d,
                           int block_size, int max_blocks, int num_splits, int split_len, float scale, RopeArgs ra,
-                          bool fused, uintptr_t stream) {
+                          bool fused, uintptr_t stream, bool leave = false) {
   DLLM_HOST_CHECK(block_size == kBS, "paged attention requires block_size 32");
   DLLM_HOST_CHECK(hq % hkv == 0 && hq / hkv <= 16, "GQA group size must be <= 16");
   DLLM_HOST_CHECK(d == 64 || d == 128, "head_dim must be 64 or 128");
@@ -1753,7 +1830,7 @@ static void decode_launch(uintptr_t out, uintptr_t q, uintptr_t k_cache, uintptr
                   "fused decode needs qkv, positions, slots");
   DLLM_HOST_CHECK(ra.part == nullptr || (ra.nparts >= 1 && ra.slab >= (long)batch * (hq + 2 * hkv) * d),
                   "qkv partial slabs");
-  if (batch == 0) return;
+  if (batch == 0) return false;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const float sl2 = scale * 1.4426950408889634f;
   // One wave per workgroup: waves that share a CU share its ~64 outstanding cache lines, and a small batch has a CU for
@@ -1799,6 +1876,7 @@ static void decode_launch(uintptr_t out, uintptr_t q, uintptr_t k_cache, uintptr
   }
 #undef DLLM_DEC
   DLLM_HIP_CHECK(hipGetLastError());
+  if (leave && num_splits > 1 && !join) return true;
   if (num_splits > 1 && !join) {
     // the round that covers the splits with the fewest repeated loads (16 of them for 2 splits: 64 sequences of 64 heads
     // 3 us slower)
@@ -1818,6 +1896,7 @@ static void decode_launch(uintptr_t out, uintptr_t q, uintptr_t k_cache, uintptr
 #undef DLLM_REDUCE
     DLLM_HIP_CHECK(hipGetLastError());
   }
+  return false;
 }
 
 void paged_attention_decode(uintptr_t out, uintptr_t q, uintptr_t k_cache, uintptr_t v_cache,
@@ -1829,21 +1908,22 @@ void paged_attention_decode(uintptr_t out, uintptr_t q, uintptr_t k_cache, uintp
 }
 
 // decode with RoPE + KV append fused in: reads the raw qkv projection [B, (hq + 2 hkv) * d]
-void paged_attention_decode_rope(uintptr_t out, uintptr_t qkv, uintptr_t positions, uintptr_t cos_sin, uintptr_t slots,
+bool paged_attention_decode_rope(uintptr_t out, uintptr_t qkv, uintptr_t positions, uintptr_t cos_sin, uintptr_t slots,
                                  uintptr_t k_cache, uintptr_t v_cache, uintptr_t block_tables, uintptr_t seq_lens,
                                  uintptr_t part_o, uintptr_t part_ml, int batch, int hq, int hkv, int d,
                                  int block_size, int max_blocks, int num_splits, int split_len, float scale,
-                                 uintptr_t qkv_part, int qkv_nparts, long qkv_slab, uintptr_t stream) {
+                                 uintptr_t qkv_part, int qkv_nparts, long qkv_slab, uintptr_t stream,
+                                 bool leave) {
   RopeArgs ra{(const bf16*)qkv, (const int32_t*)positions, (const float*)cos_sin, (const int32_t*)slots,
               (const float*)qkv_part, qkv_nparts, qkv_slab};
-  decode_launch(out, 0, k_cache, v_cache, block_tables, seq_lens, part_o, part_ml, batch, hq, hkv, d, block_size,
-                max_blocks, num_splits, split_len, scale, ra, true, stream);
+  return decode_launch(out, 0, k_cache, v_cache, block_tables, seq_lens, part_o, part_ml, batch, hq, hkv, d, block_size,
+                max_blocks, num_splits, split_len, scale, ra, true, stream, leave);
 }
 
 // LDS of attn_o_kernel
 static long attn_o_bytes(int batch, int hq, int hkv, int ns) {
   const int g = hq / hkv;
-  return (long)g * (kAoD / 64) * 16384 + (((long)batch * g * kAoD * 2 + 15) & ~15L) + (ns > 1 ? (long)batch * ns * g * (kAoD + 6) * 4 : 0);
+  return (long)g * (kAoD / 64) * 16384 + (long)batch * g * kAoD * 2 + (ns > 1 ? (long)batch * ns * g * (kAoD + 6) * 4 : 0);
 }
 
 // paged_attention_decode_rope of heads of 128 and slab kvh of [hkv, batch, n] at `slabs` = its heads' part of the product with wo [n, hq * 128]
@@ -1871,6 +1951,24 @@ void attn_o(uintptr_t slabs, uintptr_t wo, int n, uintptr_t qkv, uintptr_t posit
   else if (qkv_nparts == 4) go(attn_o_kernel<4>);
   else if (qkv_nparts == 8) go(attn_o_kernel<8>);
   else go(attn_o_kernel<-1>);
+  DLLM_HIP_CHECK(hipGetLastError());
+}
+
+// The partial results of `ns` splits (part_o [batch, hq, ns, 128], part_ml [batch, hq, ns, 2]) joined, and slab kvh of [hkv, batch, n] at `slabs` =
+// the part of their product with wo [n, hq * 128] that kv head kvh's heads give
+void join_o(uintptr_t slabs, uintptr_t wo, int n, uintptr_t part_o, uintptr_t part_ml, int batch, int hq, int hkv, int ns, uintptr_t stream) {
+  DLLM_HOST_CHECK(hq % hkv == 0 && hq / hkv <= 16 && batch >= 1 && batch <= 16 && n % 128 == 0, "sizes");
+  DLLM_HOST_CHECK(ns >= 1 && ns <= 16 && part_o && part_ml, "up to 16 splits");
+  const long lds = attn_o_bytes(batch, hq, hkv, 1);
+  DLLM_HOST_CHECK(lds <= 160 * 1024, "LDS");
+  auto go = [&](auto kern) {
+    DLLM_HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+    hipLaunchKernelGGL(kern, dim3((unsigned)(n / 128 * hkv)), dim3(512), lds, reinterpret_cast<hipStream_t>(stream), (const bf16*)wo,
+                       (const float*)part_o, (const float*)part_ml, batch, n, hq, hkv, ns, (float*)slabs);
+  };
+  if (ns <= 4) go(join_o_kernel<4>);
+  else if (ns <= 8) go(join_o_kernel<8>);
+  else go(join_o_kernel<16>);
   DLLM_HIP_CHECK(hipGetLastError());
 }
 

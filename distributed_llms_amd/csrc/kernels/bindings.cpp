@@ -49,6 +49,7 @@ PYBIND11_MODULE(_C_kernels, m) {
   m.def("paged_attention_decode", &dllm::paged_attention_decode);
   m.def("paged_attention_decode_rope", &dllm::paged_attention_decode_rope);
   m.def("attn_o", &dllm::attn_o);
+  m.def("join_o", &dllm::join_o);
   m.def("paged_attention_prefill", &dllm::paged_attention_prefill);
   m.def("sm_embed_f32", &dllm::sm_embed_f32);
   m.def("sm_rms_norm", &dllm::sm_rms_norm);

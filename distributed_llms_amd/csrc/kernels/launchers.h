@@ -75,11 +75,12 @@ void attn_o(uintptr_t slabs, uintptr_t wo, int n, uintptr_t qkv, uintptr_t posit
             uintptr_t k_cache, uintptr_t v_cache, uintptr_t block_tables, uintptr_t seq_lens, int batch, int hq, int hkv,
             int block_size, int max_blocks, int num_splits, int split_len, float scale, uintptr_t qkv_part, int qkv_nparts,
             long qkv_slab, uintptr_t stream);
-void paged_attention_decode_rope(uintptr_t out, uintptr_t qkv, uintptr_t positions, uintptr_t cos_sin, uintptr_t slots,
+bool paged_attention_decode_rope(uintptr_t out, uintptr_t qkv, uintptr_t positions, uintptr_t cos_sin, uintptr_t slots,
                                  uintptr_t k_cache, uintptr_t v_cache, uintptr_t block_tables, uintptr_t seq_lens,
                                  uintptr_t part_o, uintptr_t part_ml, int batch, int hq, int hkv, int d,
                                  int block_size, int max_blocks, int num_splits, int split_len, float scale,
-                                 uintptr_t qkv_part, int qkv_nparts, long qkv_slab, uintptr_t stream);
+                                 uintptr_t qkv_part, int qkv_nparts, long qkv_slab, uintptr_t stream, bool leave);
+void join_o(uintptr_t slabs, uintptr_t wo, int n, uintptr_t part_o, uintptr_t part_ml, int batch, int hq, int hkv, int ns, uintptr_t stream);
 void paged_attention_prefill(uintptr_t out, uintptr_t q, uintptr_t k_cache, uintptr_t v_cache,
                              uintptr_t block_tables, uintptr_t cu_seqlens_q, uintptr_t seq_lens, int batch,
                              int hq, int hkv, int d, int block_size, int max_blocks, int max_q_len, float scale,

@@ -349,13 +349,13 @@ class ModelStage:
         return o.view(o.shape[0], self.q_size_local)
 
     def _attention_o(self, qkv, li: int, meta: BatchMeta, wo):
-        """Decode attention and the o-projection in one launch (one or two short sequences), or None."""
+        """Decode attention and the o-projection behind it where they share a launch (few sequences), or None."""
         if meta.is_prefill or not knobs.K.fused_rope or not knobs.K.defer_o:
             return None
         k_cache, v_cache = self.kv.layer(li)
         return ops.paged_attention_decode_o(qkv, meta.positions, self.cos_sin, k_cache, v_cache, meta.slot_mapping,
                                             meta.block_tables, meta.seq_lens, self.hq, self.hkv, self.cfg.head_dim, self.scale,
-                                            wo, max_ctx=meta.max_ctx or None)
+                                            wo, max_ctx=meta.max_ctx or None, workspace=meta.attn_workspace)
 
     def _mlp(self, h: Optional[torch.Tensor], lw: Dict[str, torch.Tensor], gated: Optional[torch.Tensor] = None) -> torch.Tensor:
         """``gated``: the dense MLP's activation, where the launch of its norm has made it already (``h`` is None then)."""

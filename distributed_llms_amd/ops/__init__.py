@@ -323,6 +323,14 @@ def paged_attention_decode_rope(qkv, positions, cos_sin, k_cache, v_cache, slot_
 
     ``qkv`` may be a :class:`gemm.SplitKPartial`: the kernel then sums the split-K slabs (f32 sums of f16 x 2^-6 slices) itself
     (bit-identical to reducing first), which removes the reduce launch and the bf16 round trip."""
+    return _decode_rope(qkv, positions, cos_sin, k_cache, v_cache, slot_mapping, block_tables, seq_lens, num_heads, num_kv_heads,
+                        head_dim, scale, max_ctx, workspace)[0]
+
+
+def _decode_rope(qkv, positions, cos_sin, k_cache, v_cache, slot_mapping, block_tables, seq_lens, num_heads: int, num_kv_heads: int,
+                 head_dim: int, scale: float, max_ctx: Optional[int], workspace: Optional[tuple], leave: bool = False):
+    """:func:`paged_attention_decode_rope`, and None -- or, with ``leave``, where its splits would be joined by a launch of their own, what
+    that reads instead: (partial sums, maxima and denominators, number of splits)."""
     part = None
     if isinstance(qkv, gemm.SplitKPartial):
         part = qkv
@@ -334,7 +342,7 @@ def paged_attention_decode_rope(qkv, positions, cos_sin, k_cache, v_cache, slot_
     if part is None and not _gpu(qkv):
         q = ref.rope_cache_append(qkv, positions, cos_sin, k_cache, v_cache, slot_mapping, num_heads, num_kv_heads,
                                   head_dim)
-        return ref.paged_attention_decode(q, k_cache, v_cache, block_tables, seq_lens, scale)
+        return ref.paged_attention_decode(q, k_cache, v_cache, block_tables, seq_lens, scale), None
     if part is None:
         _ck(qkv, "attn.qkv")
     _ck(k_cache, "k_cache")
@@ -368,32 +376,42 @@ def paged_attention_decode_rope(qkv, positions, cos_sin, k_cache, v_cache, slot_
             if po_t.numel() < b * hq * splits * d or pml_t.numel() < b * hq * splits * 2:
                 raise ValueError("attention workspace too small")
         po, pml = po_t.data_ptr(), pml_t.data_ptr()
-    _ext.kernels().paged_attention_decode_rope(
+    left = _ext.kernels().paged_attention_decode_rope(
         out.data_ptr(), 0 if part is not None else qkv.data_ptr(), positions.data_ptr(),
         0 if cos_sin is None else cos_sin.data_ptr(),
         slot_mapping.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), block_tables.data_ptr(), seq_lens.data_ptr(),
         po, pml, b, hq, hkv, d, bs, max_blocks, splits, split_len, float(scale),
         0 if part is None else part.ws.data_ptr(), 0 if part is None else part.splits,
-        0 if part is None else part.m * part.n, _stream())
-    return out
+        0 if part is None else part.m * part.n, _stream(), leave)
+    return out, (po_t, pml_t, splits) if left else None
+
+
+def _o_by_heads(hq: int, hkv: int, d: int, n: int) -> bool:
+    """Can the o-projection's K slices be the kv heads' (csrc/kernels/attention.hip, attn_o_kernel and join_o_kernel)?  Slices of at most 512 inputs,
+    whose weights fill the LDS, and one round of workgroups that keeps three quarters of the CUs busy."""
+    return (knobs.K.one and d == 128 and hq % hkv == 0 and hq // hkv <= 4 and n % 128 == 0 and 192 <= n // 128 * hkv <= 256
+            and not gemm._comm_cus)
 
 
 def attn_o_splits(batch: int, max_ctx: int, hq: int, hkv: int, d: int, n: int) -> int:
-    """Splits of a sequence's keys in :func:`paged_attention_decode_o`, 0 where it does not serve the call: one or two sequences of up to
-    512 keys together (longer ones, and more, are slower than two launches: csrc/kernels/attention.hip, attn_o_kernel), a slice of at most
-    512 projection inputs per kv head (its weights fill the LDS), one round of workgroups that keeps three quarters of the CUs busy.  On the
-    context's bucket, as the decode graphs have it, so that a graph and the eager path take the same way."""
+    """Splits of a sequence's keys where :func:`paged_attention_decode_o` is one launch, else 0: one or two sequences of up to 512 keys
+    together (longer ones, and more, are slower than two launches: figures there).  On the context's bucket, as the decode graphs have
+    it, so that a graph and the eager path take the same way."""
     bucket = max(256, 1 << max(0, max_ctx - 1).bit_length())
-    if not (knobs.K.one and d == 128 and hq % hkv == 0 and hq // hkv <= 4 and n % 128 == 0 and 192 <= n // 128 * hkv <= 256
-            and batch <= 2 and batch * bucket <= 512) or gemm._comm_cus:
+    if not _o_by_heads(hq, hkv, d, n) or batch > 2 or batch * bucket > 512:
         return 0
     return 4 if batch * bucket == 256 else 2
 
 
+JOIN_O_MAX_SPLITS = 32              # (of all sequences together: csrc/kernels/attention.hip, join_o_kernel)
+
+
 def paged_attention_decode_o(qkv, positions, cos_sin, k_cache, v_cache, slot_mapping, block_tables, seq_lens, num_heads: int,
-                             num_kv_heads: int, head_dim: int, scale: float, wo, max_ctx: Optional[int] = None):
-    """:func:`paged_attention_decode_rope` and the deferred :func:`linear` with ``wo`` [N, Hq * D] behind it in one launch: a
-    :class:`gemm.SplitKPartial` with a slab per kv head, or None where they have launches of their own (:func:`attn_o_splits`)."""
+                             num_kv_heads: int, head_dim: int, scale: float, wo, max_ctx: Optional[int] = None,
+                             workspace: Optional[tuple] = None):
+    """:func:`paged_attention_decode_rope` and the deferred :func:`linear` with ``wo`` [N, Hq * D] behind it, in one launch
+    (:func:`attn_o_splits`) or with the join of the attention's splits in the projection's launch (up to 32 splits of the
+    sequences' keys together): what :func:`linear` returns, or None where the two functions are as good."""
     part = qkv if isinstance(qkv, gemm.SplitKPartial) else None
     if isinstance(wo, quant.Fp8Weight) or not k_cache.is_cuda or block_tables.dim() != 2 or not block_tables.shape[1]:
         return None
@@ -401,16 +419,27 @@ def paged_attention_decode_o(qkv, positions, cos_sin, k_cache, v_cache, slot_map
     hq, hkv, d, bs, max_blocks = num_heads, num_kv_heads, head_dim, k_cache.shape[2], block_tables.shape[1]
     max_ctx = max_ctx or max_blocks * bs
     n = wo.shape[0]
-    ns = attn_o_splits(b, max_ctx, hq, hkv, d, n)
-    if not ns or b < 1 or bs != 32 or max_ctx > max_blocks * bs or width != (hq + 2 * hkv) * d:
+    if not _o_by_heads(hq, hkv, d, n) or not 1 <= b <= JOIN_O_MAX_SPLITS // 2 or bs != 32 or max_ctx > max_blocks * bs \
+            or width != (hq + 2 * hkv) * d or (part is not None and len(part.shape) != 2):
         return None
     if not (wo.dim() == 2 and wo.shape[1] == hq * d and wo.dtype == torch.bfloat16 and wo.is_contiguous() and wo.data_ptr() % 16 == 0
             and wo.device == k_cache.device):
         return None
+    ns = attn_o_splits(b, max_ctx, hq, hkv, d, n)
+    ws = gemm.slab_space(k_cache.device, part)
+    out = gemm.SplitKPartial(ws, hkv, b, n, (b, n), torch.bfloat16, k_cache.device)
+    if not ns:
+        splits = decode_split_plan(b, hkv, max_ctx, bs, max_blocks)[0]
+        if not 1 < splits <= 16 or b * splits > JOIN_O_MAX_SPLITS:
+            return None
+        a, left = _decode_rope(qkv, positions, cos_sin, k_cache, v_cache, slot_mapping, block_tables, seq_lens, hq, hkv, d, scale,
+                               max_ctx, workspace, leave=True)
+        if left is None:
+            return gemm.linear(a.view(b, hq * d), wo, defer=True)
+        _ext.kernels().join_o(ws.data_ptr(), wo.data_ptr(), n, left[0].data_ptr(), left[1].data_ptr(), b, hq, hkv, left[2], _stream())
+        return out
     if part is None:
         _ck(qkv, "attn.qkv")
-    elif len(part.shape) != 2:
-        return None
     _ck(k_cache, "k_cache")
     _ck(v_cache, "v_cache")
     for t, name in ((positions, "positions"), (slot_mapping, "slot_mapping"), (block_tables, "block_tables"), (seq_lens, "seq_lens")):
@@ -420,13 +449,12 @@ def paged_attention_decode_o(qkv, positions, cos_sin, k_cache, v_cache, slot_map
         if cos_sin.shape[1] != d:
             raise ValueError("cos_sin width must equal head_dim")
     bucket = max(256, 1 << (max_ctx - 1).bit_length())
-    ws = gemm.slab_space(k_cache.device, part)
     _ext.kernels().attn_o(ws.data_ptr(), wo.data_ptr(), n, 0 if part is not None else qkv.data_ptr(), positions.data_ptr(),
                           0 if cos_sin is None else cos_sin.data_ptr(), slot_mapping.data_ptr(), k_cache.data_ptr(),
                           v_cache.data_ptr(), block_tables.data_ptr(), seq_lens.data_ptr(), b, hq, hkv, bs, max_blocks, ns,
                           -(-bucket // (bs * ns)) * bs, float(scale), 0 if part is None else part.ws.data_ptr(),
                           0 if part is None else part.splits, 0 if part is None else part.m * part.n, _stream())
-    return gemm.SplitKPartial(ws, hkv, b, n, (b, n), torch.bfloat16, k_cache.device)
+    return out
 
 
 def prefill_attn_version(max_q_len: int, head_dim: int) -> int:

@@ -63,6 +63,32 @@ def test_equal_bits_where_the_splits_are(cuda, ctx):
     assert torch.equal(got.materialize(), ops.linear(a.view(1, -1), wo, defer=True).materialize())
 
 
+# every number of splits that has a build of its own and those between, with empty ones (short sequences in a wide table) and none of a
+# sequence's at all; one to sixteen sequences, also where the attention joins its splits itself
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens,width", [([600], 0), ([1000, 30], 0), ([513], 32), ([200, 90, 1], 0), ([33, 64, 0, 250], 8), ([90, 80, 70, 60, 50, 40], 0),
+                                        ([250] * 8, 8), ([40, 33] * 4, 8), ([300, 10, 20, 500], 16), ([100] * 16, 4), ([900, 900], 32)])
+@pytest.mark.parametrize("hq,hkv,n,parts", [(32, 8, 4096, 5), (16, 8, 3072, 0)])
+def test_joined_in_the_projection(cuda, lens, width, hq, hkv, n, parts):
+    qkv, pos, cs, kc, vc, slots, table, sl, wo = _case(lens, hq, hkv, n, parts, sum(lens) + len(lens))
+    table = torch.cat([table, table.new_zeros(len(lens), max(0, width - table.shape[1]))], 1)
+    ctx = max(max(lens), 32 * width)
+    k1, v1 = kc.clone(), vc.clone()
+    got = ops.paged_attention_decode_o(qkv, pos, cs, k1, v1, slots, table, sl, hq, hkv, D, D ** -0.5, wo, max_ctx=ctx)
+    dense = lambda t: t.materialize() if isinstance(t, gemm.SplitKPartial) else t
+    got = dense(got)
+    a = ops.paged_attention_decode_rope(qkv, pos, cs, kc, vc, slots, table, sl, hq, hkv, D, D ** -0.5, max_ctx=ctx)
+    splits = ops.decode_split_plan(len(lens), hkv, ctx, BS, table.shape[1])[0]
+    assert (got is not None) == (1 < splits <= 16 and len(lens) * splits <= 32), splits
+    if got is None:
+        return
+    assert torch.equal(k1, kc) and torch.equal(v1, vc)
+    # a slice per kv head, or -- where the attention joined its splits itself -- the projection's own plan
+    own = dense(ops.linear(a.view(len(lens), -1), wo, defer=True))
+    by_heads = dense(gemm.linear_wide(a.view(len(lens), -1), wo, splits=hkv, defer=True))
+    assert torch.equal(got, by_heads) or torch.equal(got, own)
+
+
 @pytest.mark.gpu
 def test_replays(cuda):
     """A captured step, replayed with other lengths and keys between eager work, against the eager call."""
