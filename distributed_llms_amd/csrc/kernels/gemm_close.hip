@@ -8,16 +8,23 @@
 // The sums are in the order of the two launches (the row's places, and as many product waves with the same K-tiles as gemm_stream
 // has), so that the new stream and the product have their bits.  (Twice the product waves under a GLU of up to 128 rows a workgroup:
 // other bits, 4096 x 2560 8.3 for 8.9, but 8192 and 16384 x 2048 14.2 and 22.9 for 10.4 and 15.3.)
-// us, close + product -> this, cold weights, RMS norms with a clipped GLU or without, layer norms with a gelu GLU or without:
-//   K  512:  512 / 2048 4.4 / 4.7 -> 3.1 / 3.7, + GLU 3072 5.4 -> 4.3;  4.8 / 5.1 -> 3.5 / 4.0, 5.5 -> 4.5
-//   K 1024:  2048 / 8192 5.1 / 7.1 -> 4.0 / 6.3, + GLU 6144 7.0 -> 6.0;  1536 5.4 -> 4.2, 7.1 -> 6.3
-//   K 1536:  1536 / 4608 5.5 / 7.4 -> 4.8 / 6.5, + GLU 9216 10.5 -> 9.8;  6.0 / 7.7 -> 5.3 / 7.2, 10.7 -> 10.3
-//   K 2048:  2048 / 6144 6.6 / 9.2 -> 5.8 / 8.7, + GLU 16384 17.3 -> 15.7;  7.0 / 9.6 -> 6.4 / 9.4, 17.4 -> 15.2
-//   K 2560:  2560 / 5120 7.7 / 9.8 -> 6.5 / 8.8, + GLU 15360 19.0 -> 18.1;  8.2 / 10.2 -> 7.2 / 9.5, 19.2 -> 18.5
-//   K 3072:  3072 / 9216 8.4 / 15.1 -> 7.4 / 13.7, + GLU 8192 / 16384 13.7 / 22.3 -> 12.8 / 21.4;  8.9 / 15.5 -> 8.0 / 14.5, 22.5 -> 21.9
-// and every size between and past them that was tried (160, to 96 Mi weights) as fast at least.  Wider rows, in four pieces, win as
+// The product's waves wait (a barrier) until the row's loads are issued: a CU's requests for lines are served in their order, and the row
+// came behind the first weights, 0.4 to 1.2 us later.
+// us, close + product -> this with weights and row issued together -> as it is, cold weights, RMS norms with a clipped GLU or without,
+// layer norms with a gelu GLU or without:
+//   K  512:  512 / 2048 4.4 / 4.7 -> 3.2 / 3.5 -> 3.0 / 3.1, + GLU 3072 5.4 -> 4.1 -> 3.7;  4.8 / 5.1 -> 3.6 / 3.9 -> 3.4 / 3.6, 5.5 -> 4.4 -> 3.8
+//   K 1024:  2048 / 8192 5.1 / 7.1 -> 3.9 / 6.1 -> 3.3 / 5.4, + GLU 6144 7.0 -> 5.9 -> 5.2;  1536 5.4 -> 4.1 -> 3.6, 7.1 -> 6.2 -> 5.1
+//   K 1536:  1536 / 4608 5.5 / 7.4 -> 5.1 / 6.4 -> 4.4 / 5.3, + GLU 9216 10.5 -> 9.7 -> 8.9;  6.0 / 7.7 -> 5.7 / 7.1 -> 5.0 / 5.9, 10.7 -> 10.1 -> 8.9
+//   K 2048:  2048 / 6144 6.6 / 9.2 -> 5.8 / 8.3 -> 4.8 / 7.0;  7.0 / 9.6 -> 6.3 / 8.9 -> 5.4 / 7.3
+//   K 2560:  2560 / 5120 7.7 / 9.8 -> 6.3 / 8.4 -> 5.5 / 7.4, + GLU 15360 19.0 -> 17.3 -> 16.6;  8.2 / 10.2 -> 7.0 / 9.1 -> 6.0 / 8.0, 19.2 -> 17.9 -> 16.6
+//   K 3072:  3072 / 9216 8.4 / 15.1 -> 7.1 / 13.1 -> 6.2 / 12.7, + GLU 8192 / 16384 13.7 / 22.3 -> 12.2 / 20.6 -> 11.4 / 19.6;  8.9 / 15.5 -> 7.8 /
+//   14.0 -> 6.8 / 13.0, 22.5 -> 21.0 -> 19.5
+// A GLU with rows of 4 KiB is the exception: waves that start together ask a part of the memory channels (16384 x 2048 17.3 -> 14.6 -> 14.8,
+// 17.4 -> 14.7 -> 15.4).
+// Before that barrier every size between and past these that was tried (160, to 96 Mi weights) was as fast as the two launches at least.  Wider
+// rows, in four pieces, won as
 // much in most products (4096 x 4096 10.9 -> 10.3, 22016 x 4096 + GLU 35.7 -> 33.4), but some GLUs, where a few CUs have a second
-// workgroup, lose: 18432 x 3584 26.7 -> 29.5, 14336 / 16384 / 18432 x 4096 27.0 / 28.9 / 31.0 -> 29.3 / 31.3 / 32.2.
+// workgroup, lost: 18432 x 3584 26.7 -> 29.5, 14336 / 16384 / 18432 x 4096 27.0 / 28.9 / 31.0 -> 29.3 / 31.3 / 32.2.
 // More rows cost each workgroup as many times the arithmetic: 4 rows at best equal (6144 x 1024 7.1 / 7.1), 2560 wide slower (15360
 // 19.3 / 19.8), so that the launch of its own is kept for them.
 #include "gemm_stream.h"

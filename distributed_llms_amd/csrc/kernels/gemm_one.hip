@@ -5,9 +5,10 @@
 // every launch pays 2-3 us to start, to get its first weights and to drain.  So
 //  * the norm has no launch of its own: every workgroup makes the row it multiplies (K times slabs + 2 values, 72 KiB for 4096 in 8
 //    slabs, out of its XCD's L2) in four waves of its own while eight others have the first weights under way.  (Loads return in
-//    order: a wave that has both under way would wait for its weights with its row.)  The weights start half a microsecond later, so
-//    that the row's requests are not behind them: a CU has some 256 lines under way.  us, add + norm and product / in one launch:
-//    6144 x 4096 12.8 / 10.0, 28672 x 4096 with its SwiGLU 42.4 / 36.5, 10240 x 8192 34.0 / 32.6, 57344 x 8192 152 / 148, 3072 x 2048 9.0 / 5.9;
+//    order: a wave that has both under way would wait for its weights with its row.)  The weights wait until the row's loads are issued (a
+//    barrier): a CU has some 256 lines under way, in their order.  us, add + norm and product / in one launch, weights at once / as it is:
+//    6144 x 4096 12.8 / 10.4 / 10.0, 28672 x 4096 with its SwiGLU 42.4 / 38.3 / 36.5, 10240 x 8192 34.0 / 33.0 / 32.6, 57344 x 8192 152 / 150 / 149, 3072 x
+//    2048 9.0 / 6.6 / 6.0;
 //  * the row is whole in LDS and each wave streams 16 weight rows through a ring of its own: no staging of x, no barriers.  us,
 //    gemm_wide / this: 4096 x 14336 20.0 / 19.2, 4096 x 4096 7.6 / 7.1, 8192 x 8192 31.3 / 27.2, 128256 x 4096 160 / 155;
 //  * the ring: D K-tiles of 64.  3 are enough for slices under 32 K-tiles (4096 x 14336 in 8 of 28: 19.2, with 5 19.6); longer ones
@@ -61,7 +62,7 @@ __device__ __forceinline__ void one_row(const OneRow& in, int K, int ks0, int nt
     return;
   } else {
     typedef part_elem raw __attribute__((ext_vector_type(8)));
-    constexpr int CH = 2;                                // pieces whose slabs are under way together
+    constexpr int CH = IN == kRowSlabsNorm ? 2 : MAXV;   // pieces whose loads are under way together
     bf16x8 g[MAXV], r[MAXV];
     float ss = 0.f;
 #pragma unroll
@@ -83,6 +84,8 @@ __device__ __forceinline__ void one_row(const OneRow& in, int K, int ks0, int nt
 #pragma unroll
         for (int i = 0; i < MAXV; ++i) g[i] = reinterpret_cast<const bf16x8*>(in.w)[min(place(i), nvec - 1)];
       }
+      __builtin_amdgcn_sched_barrier(0);
+      if (c0 == 0) __builtin_amdgcn_s_barrier();         // the row's requests are out: now the weights'
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int i = 0; i < CH; ++i) {
@@ -169,7 +172,8 @@ __global__ void __launch_bounds__((OF + OW) * 64, 1) gemm_one_kernel(const bf16*
     for (int j = 0; j < 2; ++j)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_vptr_p)(ring + slot * 2048 + j * 1024), 16, (int)offB[j], k * 128, 0, NT ? 2 : 0);
   };
-  if constexpr (IN != kRowAsIs) __builtin_amdgcn_s_sleep(8);
+  if constexpr (IN != kRowAsIs) __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int j = 0; j < D; ++j) stage(j, j);
   const uint32_t lds0 = (uint32_t)(size_t)(lds_vptr_p)smem;
