@@ -577,9 +577,16 @@ static void launch_tile(uintptr_t out, uintptr_t q, uintptr_t k_cache, uintptr_t
 // the A operand of S^T = K Q^T (row r of a 16-key half holds the key that makes the accumulator hand
 // each lane 8 consecutive keys), V^T pieces (8 keys of one channel, 16 bytes) as the A operand of
 // O^T = V^T P^T.  Each wave keeps an online softmax; the waves' partial results meet in LDS.
+//
+// What bounds it: a CU's requests (300 keys of 128 + 128 channels are 150 KiB, 5 us of them) behind the round trips of position, block and
+// first keys, then the end.  So a tile that a wave does not have is one line and not a tile read again, and the end has no round trip, four
+// channels a thread and the sinks and gates at hand.  us before / now: 32 rows of 300 keys, 16 / 4 heads of 128 11.6 / 10.4, with biases 13.0 /
+// 11.6, latent 256 + 192 14.8 / 12.1; 64 of 120 7.4 / 6.6; 64 of 300, 256 + 256 22.6 / 17.4; 64 of 77, 32 / 8 of 128 gated 9.6 / 8.3; one row of
+// 50 4.9 / 4.6 (four of 30, 8 / 8 of 64 and gated 4.5 / 4.65).  Two whole tiles under way per wave were slower (32 of 300 12.7).
 constexpr int kDW = 4;
 
-template <int NQK, int NDV, bool BIAS>
+// END: sinks or a gate (and one run: with more the merge applies them).
+template <int NQK, int NDV, bool BIAS, bool END>
 __global__ void __launch_bounds__(64 * kDW) window_attn_decode_kernel(
     const int32_t* __restrict__ positions, const int32_t* __restrict__ tok_seq, const int32_t* __restrict__ block_tables,
     int max_blocks, int H, int G, int D, int Dv, int bs, int window, int hpw,   // (14 words: they come with the wave)
@@ -588,8 +595,8 @@ __global__ void __launch_bounds__(64 * kDW) window_attn_decode_kernel(
     float* __restrict__ ws, float softcap, const bf16* __restrict__ kp_cache, const bf16* __restrict__ vp_cache, int pool, int pbs,
     const float* __restrict__ bias, int nbias, int keep, const bf16* __restrict__ gate, long gate_ld) {
   constexpr int DVP = 16 * NDV;
-  __shared__ float so[kDW][16][DVP + 1];
-  __shared__ float sml[kDW][2][16];
+  __shared__ __attribute__((aligned(16))) float so[kDW][16][DVP + 4];
+  __shared__ float sml[kDW][2][16], sfin[2][16];     // per head: the waves' maxima and weight sums; sinks, gates
   // the query heads of a K/V head are dealt to workgroups hpw (<= 16) at a time: part p runs heads
   // hpw p .. of the group (fewer heads per workgroup when few rows would leave most CUs idle)
   const int t = blockIdx.x;
@@ -601,6 +608,14 @@ __global__ void __launch_bounds__(64 * kDW) window_attn_decode_kernel(
   const int lo = win_lo(pos, window, chunk);
   const int bsh = __ffs(bs) - 1;                     // bs is a power of two here
   const int32_t* bt = block_tables + (size_t)b * max_blocks;
+  // what the end needs, here beside the position: there it was a round trip of its own.  (Off a place that is there, not behind a
+  // branch, whose wait would cover the loads behind it.)
+  float sink = 0.f;
+  bf16 gated = (bf16)0.f;
+  if constexpr (END) {
+    sink = *(sinks ? sinks + hb + min(col, nh - 1) : reinterpret_cast<const float*>(positions));
+    gated = *(gate ? gate + (size_t)t * gate_ld + hb + min(col, nh - 1) : q);
+  }
   bf16x8 qf[NQK];
   {
     const bf16* qrow = q + ((size_t)t * H + hb + min(col, nh - 1)) * D;
@@ -643,13 +658,13 @@ __global__ void __launch_bounds__(64 * kDW) window_attn_decode_kernel(
     const int sh = ti < ptile ? pbsh : bsh;
     return Blocks{bt[min(k0 + jr, hi) >> sh], bt[min(k0 + jr + 4, hi) >> sh], bt[min(k0 + 8 * grp, hi & ~7) >> sh]};
   };
-  auto load_k = [&](int ti, const Blocks& at) {
+  auto load_k = [&](int ti, const Blocks& at, bool real) {
     int k0, hi;
     edges(ti, k0, hi);
     const bf16* kc = ti < ptile ? fk_cache : k_cache;
     const int cb = ti < ptile ? fbs : bs;
-    const bf16* r1 = kc + (((size_t)at.k1 * G + g) * cb + (min(k0 + jr, hi) & (cb - 1))) * D;
-    const bf16* r2 = kc + (((size_t)at.k2 * G + g) * cb + (min(k0 + jr + 4, hi) & (cb - 1))) * D;
+    const bf16* r1 = kc + (real ? (((size_t)at.k1 * G + g) * cb + (min(k0 + jr, hi) & (cb - 1))) * D : 0);
+    const bf16* r2 = kc + (real ? (((size_t)at.k2 * G + g) * cb + (min(k0 + jr + 4, hi) & (cb - 1))) * D : 0);
 #pragma unroll
     for (int s2 = 0; s2 < NQK; ++s2) {
       const int d0 = min(32 * s2 + 8 * grp, D - 8);
@@ -683,7 +698,7 @@ __global__ void __launch_bounds__(64 * kDW) window_attn_decode_kernel(
   if (tbeg < tstop) {
     now = blocks_of(tbeg);
     next = blocks_of(min(tbeg + kDW, tlast));
-    load_k(tbeg, now);
+    load_k(tbeg, now, true);
   }
   for (int ti = tbeg; ti < tstop; ti += kDW) {
     int k0, rhi;
@@ -709,7 +724,7 @@ __global__ void __launch_bounds__(64 * kDW) window_attn_decode_kernel(
         s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kb[s2], qf[s2], s1, 0, 0, 0);
       }
     }
-    load_k(tn, next);
+    load_k(tn, next, ti + kDW < tstop);
     now = next;
     next = after;
     float p[8];
@@ -748,44 +763,48 @@ __global__ void __launch_bounds__(64 * kDW) window_attn_decode_kernel(
     }
   }
   // partial results: lane (col, grp) holds channels 16 dt + 4 grp + i of head col
-  if (grp == 0) sml[wave][0][col] = m, sml[wave][1][col] = l;
+  if (grp == 0) {
+    sml[wave][0][col] = m, sml[wave][1][col] = l;
+    if (END && wave == 0) sfin[0][col] = sink, sfin[1][col] = gate_f(bf2f(gated));
+  }
 #pragma unroll
-  for (int dt = 0; dt < NDV; ++dt)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) so[wave][col][16 * dt + 4 * grp + i] = acc[dt][i];
+  for (int dt = 0; dt < NDV; ++dt) *reinterpret_cast<f32x4*>(&so[wave][col][16 * dt + 4 * grp]) = acc[dt];
   __syncthreads();
-  for (int idx = tid; idx < nh * Dv; idx += 64 * kDW) {
-    const int hh = idx / Dv, e = idx - hh * Dv;
-    float mm = -INFINITY;
+  const int pieces = Dv >> 2;                        // of four channels (Dv is a multiple of 8)
+  for (int idx = tid; idx < nh * pieces; idx += 64 * kDW) {
+    const int hh = idx / pieces, e = 4 * (idx - hh * pieces);
+    float mm = -INFINITY, ll = 0.f;
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < kDW; ++w) mm = fmaxf(mm, sml[w][0][hh]);
-    float ll = 0.f, o = 0.f;
-    if (splits > 1) {                              // unnormalised partial: Dv sums, then their maximum and weight
-#pragma unroll
-      for (int w = 0; w < kDW; ++w) {
-        const float f = sml[w][0][hh] == -INFINITY ? 0.f : expf(sml[w][0][hh] - mm);
-        ll += sml[w][1][hh] * f;
-        o += so[w][hh][e] * f;
-      }
-      float* part = ws + (((size_t)t * H + hb + hh) * splits + blockIdx.z) * (Dv + 2);
-      part[e] = o;
-      if (e == 0) part[Dv] = mm, part[Dv + 1] = ll;
-      continue;
-    }
-    if (sinks) {                                   // exp(sink) joins the denominator
-      const float sk = sinks[hb + hh];
-      mm = fmaxf(mm, sk);
-      ll = expf(sk - mm);
+    if (END && sinks && splits == 1) {               // exp(sink) joins the denominator
+      mm = fmaxf(mm, sfin[0][hh]);
+      ll = expf(sfin[0][hh] - mm);
     }
 #pragma unroll
     for (int w = 0; w < kDW; ++w) {
       const float f = sml[w][0][hh] == -INFINITY ? 0.f : expf(sml[w][0][hh] - mm);
+      const f32x4 part = *reinterpret_cast<const f32x4*>(&so[w][hh][e]);
       ll += sml[w][1][hh] * f;
-      o += so[w][hh][e] * f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[i] += part[i] * f;
     }
-    o /= ll;
-    if (gate) o *= gate_f(bf2f(gate[(size_t)t * gate_ld + hb + hh]));
-    out[((size_t)t * H + hb + hh) * Dv + e] = (bf16)o;
+    const size_t row = (size_t)t * H + hb + hh;
+    if (splits > 1) {                                // unnormalised partial: Dv sums, then their maximum and weight
+      float* part = ws + (row * splits + blockIdx.z) * (Dv + 2);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) part[e + i] = o[i];
+      if (e == 0) part[Dv] = mm, part[Dv + 1] = ll;
+      continue;
+    }
+    bf16x4 o4;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      o[i] /= ll;
+      if (END && gate) o[i] *= sfin[1][hh];
+      o4[i] = (bf16)o[i];
+    }
+    *reinterpret_cast<bf16x4*>(out + row * Dv + e) = o4;
   }
 }
 
@@ -829,8 +848,8 @@ static void launch_decode(uintptr_t out, uintptr_t q, uintptr_t k_cache, uintptr
   splits = ws ? std::max(1, std::min(splits, 64)) : 1;
   int hpw = std::min(16, R);
   while (hpw > 2 && (long)rows * G * ((R + hpw - 1) / hpw) * splits < 128) hpw = (hpw + 1) / 2;
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(window_attn_decode_kernel<NQK, NDV, BIAS>),
-                     dim3(rows, G * ((R + hpw - 1) / hpw), splits), dim3(64 * kDW), 0,
+  auto kernel = splits == 1 && (sinks || gate) ? window_attn_decode_kernel<NQK, NDV, BIAS, true> : window_attn_decode_kernel<NQK, NDV, BIAS, false>;
+  hipLaunchKernelGGL(kernel, dim3(rows, G * ((R + hpw - 1) / hpw), splits), dim3(64 * kDW), 0,
                      (hipStream_t)stream, (const int32_t*)positions, (const int32_t*)tok_seq, (const int32_t*)block_tables,
                      max_blocks, H, G, D, Dv, bs, window, hpw, (bf16*)out, (const bf16*)q, (const bf16*)k_cache,
                      (const bf16*)v_cache, chunk, scale, (const float*)sinks, splits, (float*)ws, softcap, (const bf16*)kp,
@@ -881,6 +900,7 @@ void sm_window_attn_decode(uintptr_t out, uintptr_t q, uintptr_t k_cache, uintpt
     else if (D <= 128 && Dv <= 128) WIN_DEC(4, 8);
     else if (D <= 192 && Dv <= 128) WIN_DEC(6, 8);
     else if (D <= 192 && Dv <= 192) WIN_DEC(6, 12);
+    else if (Dv <= 192) WIN_DEC(8, 12);
     else WIN_DEC(8, 16);
 #undef WIN_DEC
     return;

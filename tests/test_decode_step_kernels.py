@@ -369,6 +369,36 @@ def test_window_decode_head_sizes(cuda, d, dv, biased):
 
 
 @gpu
+@pytest.mark.parametrize("sunk,gated", [(True, False), (False, True), (True, True)])
+@pytest.mark.parametrize("h,g,d,dv", [(3, 3, 64, 40), (6, 2, 128, 128), (34, 2, 72, 96), (16, 1, 256, 192)])
+def test_window_decode_sinks_and_gates(cuda, h, g, d, dv, sunk, gated):
+    """The end of a row: sinks and gates apart and together, 1 to 16 heads a workgroup and a group in two of them (17), channels that
+    are no multiple of 16, waves without a tile, keys whole and (long contexts of few rows) in runs."""
+    lens, bs = [1, 40, 129, 900], 32
+    b, nb = len(lens), -(-max(lens) // 32)
+    kc, vc = torch.randn(b * nb + 1, g, bs, d, device=cuda).bfloat16(), torch.randn(b * nb + 1, g, dv, bs, device=cuda).bfloat16()
+    bt = (torch.randperm(b * nb, device=cuda) + 1).int().view(b, nb)
+    q = torch.randn(b, h, d, device=cuda).bfloat16()
+    sinks = torch.randn(h, device=cuda) if sunk else None
+    gate = torch.randn(b, h + 3, device=cuda).bfloat16() if gated else None
+    sb = _sb([n - 1 for n in lens], list(range(b)), cuda)
+    for max_ctx in (None, max(lens)):
+        out = sm.window_attention(q, kc, vc, bt, sb, 1 << 30, d ** -0.5, sinks=sinks, gate=gate, gate_col=2 if gated else 0, max_ctx=max_ctx)
+        for i, n in enumerate(lens):
+            at = torch.arange(n, device=cuda)
+            blk = bt[i].long()[at // bs]
+            k = kc[blk, :, at % bs].double().repeat_interleave(h // g, 1)
+            v = vc[blk, :, :, at % bs].double().repeat_interleave(h // g, 1)
+            s = (q[i].double() * k).sum(-1) * d ** -0.5
+            w = torch.softmax(torch.cat([s, sinks.double()[None]]) if sunk else s, 0)[:n]
+            want = (w[..., None] * v).sum(0)
+            if gated:
+                want = want * torch.sigmoid(gate[i, 2:2 + h].double())[:, None]
+            # as above: scores within 2^-15, weights to 17 bits, the result in 8
+            assert ((out[i].double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -13 * v.abs().max()).all()
+
+
+@gpu
 @pytest.mark.parametrize("b,hq,hkv,d,ctx", [(2, 4, 1, 128, 128), (3, 16, 1, 128, 100), (5, 2, 2, 64, 250), (64, 16, 4, 128, 129),
                                             (70, 32, 4, 64, 200), (16, 32, 2, 64, 256), (1, 1, 1, 64, 65)])
 @pytest.mark.parametrize("fused", [False, True])
