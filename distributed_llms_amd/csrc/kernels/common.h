@@ -213,6 +213,13 @@ __host__ __device__ __forceinline__ int vofs(int off, int e, int d, int bs) {
   return bs == 32 ? (off >> 3) * 8 * d + e * 8 + (off & 7) : e * bs + off;
 }
 
+// A barrier that only orders the issue of loads between the waves: what is in front of it has been issued, nothing has to have landed.
+__device__ __forceinline__ void issue_barrier() {
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+}
+
 // ---- split-K partial slabs (the workspace the split GEMMs leave for the next op).
 // DLLM_PART_TYPE selects the slab element (indices are in elements of that type):
 //   0  f32

@@ -190,9 +190,7 @@ __device__ __forceinline__ void gemm_stream_body(bf16* __restrict__ Y, const bf1
   if constexpr (CLOSE != kNoClose) {
     // The weights' requests behind the row's: a CU has some 256 lines under way, in their order, so that without this barrier the row came
     // behind the first weights (gemm_close.hip has the figures).  It waits for nothing but that the loads are issued.
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_sched_barrier(0);
+    issue_barrier();
   }
 #pragma unroll
   for (int u = 0; u < D; ++u)
