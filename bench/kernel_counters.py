@@ -41,6 +41,7 @@ def main():
                 ops.fused_add_rms_norm(p, res, g, 1e-5)
             else:
                 p.materialize()
+            gemm.linear_wide(x[:m // 2].contiguous(), w)          # (128 rows: gemm_wide, where 256 run on gemm_duo)
         if want("gate_up"):
             gemm.linear_wide(bf(m, h, sc=0.5), bf(2 * inter, h, sc=0.02), swiglu=True)
         if want("lm_head"):
