@@ -450,7 +450,7 @@ def wide_row_tile(m: int, n: int, k: int, swiglu: bool = False) -> int:
     """Row tile gemm_wide uses for this shape (knobs.wide_small_bm for small split grids, else
     wide_bm): e.g. 128 runs an M = 256 o-projection as 2 row tiles x 4 K slices instead of 1 x 8."""
     kn = knobs.K
-    if kn.wide_small_bm and not swiglu and n * k <= kn.wide_small_bm_maxw and kn.wide_small_bm < wide_bm(m) and m <= 256:
+    if kn.wide_small_bm and not swiglu and n * k <= kn.wide_small_bm_maxw and kn.wide_small_bm < wide_bm(m):
         return kn.wide_small_bm
     return wide_bm(m)
 
@@ -545,8 +545,9 @@ def linear_wide(x: torch.Tensor, w: torch.Tensor, splits: int = 0, swiglu: bool 
         s = max(1, ws.numel() // (m * n))
     stream = current_stream()
     bm = wide_row_tile(m, n, k, swiglu)
-    if not splits and variant < 0 and duo_fits(m, n, k, s, bm, swiglu) and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0:
-        return _duo(x, w, m, n, k, s, bm, swiglu, defer)
+    tall = duo_row_tile(m, n, k, s, bm, swiglu) if not splits and variant < 0 else 0
+    if tall and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0:
+        return _duo(x, w, m, n, k, s, tall, swiglu, defer)
     v = variant if variant >= 0 else wide_variant(m, n, k, s, bm)
     if bm != wide_bm(m):
         v |= bm << 8
@@ -568,6 +569,21 @@ def duo_fits(m: int, n: int, k: int, s: int, bm: int, swiglu: bool = False) -> b
     rows = 64 < m <= 256 and s == 1 if swiglu else 128 < m <= 512 and s > 1
     return (knobs.K.duo and rows and bm in (128, 192, 256) and n % 128 == 0 and k % 64 == 0 and n // 128 * s * -(-m // bm) >= 192
             and m * k * 2 < 1 << 32 and n * k * 2 < 1 << 32)
+
+
+def duo_row_tile(m: int, n: int, k: int, s: int, bm: int, swiglu: bool = False) -> int:
+    """gemm_duo's row tile for a product that gemm_wide would run in ``s`` K slices on row tiles of ``bm``, or 0.  Past 256 rows ``bm`` itself or the
+    next taller one whose tiles are one round of the CUs; the slices stay, and with them every bit.  us with the sum and norm
+    behind them, gemm_wide on ``bm`` / this, 300 and 512 rows: 4096 x 4096 31.9 / 23.6 (192-row tiles in 3 slices), 28.5 / 27.4 (128, 2); 3072 x 2048 19.4 /
+    14.1, 22.6 / 16.5 (192); 3072 x 3072 23.3 / 17.0, 29.8 / 20.4 (192); 2048 x 4096 14.8 / 14.1, 18.1 / 16.6; 2048 x 2048 11.9 / 11.3, 14.6 / 12.7 (192
+    and 256 workgroups of 128).  Four row tiles of 128 that leave CUs idle stay there: 2560 x 2560 (240) at 400 / 512 15.8 / 17.5, here 16.4 / 18.8."""
+    def ok(t):
+        wgs = n // 128 * s * -(-m // t)
+        return duo_fits(m, n, k, s, t, swiglu) and not (t == 128 and m > 384 and wgs < 256)
+
+    fits = [t for t in (128, 192, 256) if t >= bm and (t == bm or m > 256) and ok(t)]
+    one = [t for t in fits if n // 128 * s * -(-m // t) <= 256]
+    return (one or fits or [0])[0]
 
 
 def _duo(x: torch.Tensor, w: torch.Tensor, m: int, n: int, k: int, s: int, bm: int, swiglu: bool, defer: bool):

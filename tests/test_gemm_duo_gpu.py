@@ -107,5 +107,8 @@ def test_rule():
     assert not f(256, 2048, 2048, 4, 256) and not f(256, 65536, 4096, 1, 256)
     with knobs.override(duo=False):
         assert not f(256, 4096, 14336, 8, 256)
-    assert gemm.wide_row_tile(320, 4096, 4096) == 192 and gemm.wide_splits(320, 4096, 4096) == 4
-    assert gemm.wide_row_tile(512, 4096, 4096) == 256 and gemm.wide_splits(512, 4096, 4096) == 4
+    # past 256 rows: the slices that gemm_wide takes, on the row tile that makes one round of them
+    for m, n, k, tile in ((320, 4096, 4096, 192), (400, 4096, 4096, 128), (512, 4096, 4096, 128), (300, 3072, 2048, 192), (512, 3072, 3072, 192),
+                          (300, 2560, 2560, 128), (512, 2560, 2560, 0), (512, 2048, 2048, 128), (400, 4096, 14336, 256), (256, 4096, 4096, 128)):
+        s, bm = gemm.wide_splits(m, n, k), gemm.wide_row_tile(m, n, k)
+        assert gemm.duo_row_tile(m, n, k, s, bm) == tile
