@@ -10,7 +10,7 @@
 // the K-tile's one barrier: 57-62 us.  us, gemm_wide (or gemm_pp) / this, slabs with the sum and norm behind them:
 //   28672 x 4096, SwiGLU   M = 96 / 128 / 192 / 256   46.3 / 46.8 / 53.6 / 61.9 -> 44.5 / 45.8 / 52.8 / 57.5
 //   4096 x 14336           192 / 256                  35.3 / 40.1 -> 34.4 / 38.6
-//   4096 x 4096            160 / 256 / 320 / 512      16.0 / 18.4 / 32.2 / 27.9 -> 15.1 / 17.6 / 19.5 / 24.6
+//   4096 x 4096            160 / 256 / 300 / 512      16.0 / 18.4 / 31.9 / 28.5 -> 15.1 / 17.6 / 23.6 / 27.4
 //   6144 x 4096            160 / 200 / 256            18.5 / 22.2 / 23.4 -> 18.2 / 19.7 / 21.5
 //   8192 x 8192            160 / 256                  40.3 / 45.4 -> 39.5 / 43.6
 // It needs the CUs: 2048 x 2048 in 64 workgroups, 256 rows 12.0 -> 14.1 (ops/gemm.duo_fits has the rule).
@@ -25,6 +25,11 @@
 // the weights in the caches' default policy; in longer ones the stores are a smaller part and nontemporal weights gain more (4096 x 14336
 // 41.4 -> 38.6).
 // The sums have gemm_wide's order: equal bits.
+//
+// An XCD has the column tiles of a slice next to each other: its L2 then holds one slice of the activations, where the slices of a column tile
+// beside each other had every XCD fetch all of them (7 MiB of 4096 x 14336 at 256 rows, eight times, beside 112 MiB of weights).  With the sum
+// and norm behind them, 4096 x 14336 at 256 / 384 / 512 rows 42.4 / 56.5 / 64.8 -> 41.2 / 54.3 / 60.2 us, 1024 x 8192 at 512 in 8 slices 19.9 ->
+// 17.8, 2560 x 7680 at 400 27.6 -> 26.4; in a decode step of 256 requests on 8B the down projection 40.7 -> 35.8.
 #include "gemm_pp_common.h"
 #include "launchers.h"
 
@@ -41,12 +46,12 @@ __global__ void __launch_bounds__(512, 1) gemm_duo_kernel(const bf16* __restrict
   __shared__ __attribute__((aligned(16))) bf16 smem[NB * SLOT];
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int b = blockIdx.x;
-  {   // row tiles, then slices of a column tile on one XCD
+  {   // row tiles of a column tile, then column tiles of a slice on one XCD
     const int q = gridDim.x >> 3, r = gridDim.x & 7, x = b & 7;
     b = (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + (b >> 3);
   }
   const int mtiles = (M + BM - 1) / BM;
-  const int m_t = b % mtiles, rest = b / mtiles, split = rest % nsplit, n_t = rest / nsplit;
+  const int m_t = b % mtiles, rest = b / mtiles, ntiles = N / BN, split = rest / ntiles, n_t = rest - split * ntiles;
   const int m0 = m_t * BM;
   const int ks0 = split * kts, nt = min(K / PBK, ks0 + kts) - ks0;               // >= 1 (host)
   if (wv >= 4) {

@@ -680,10 +680,20 @@ __global__ void __launch_bounds__(256, 1) gemm_pp_kernel(const bf16* __restrict_
     n_t = (b % per) / gsz;
     split = 0;
   } else {
+    // Row tiles of a column tile, then the column tiles of a slice: an XCD's workgroups share their slice of A in its L2, 1 / 8 of A where
+    // every XCD read all of it (tiles of 2560 x 7680, 900 rows, with the sum and norm behind them 45.3 -> 43.7 us; 4096 x 14336,
+    // 500 / 900 / 1232 rows 64.8 / 100 / 123 -> 60.2 / 96.7 / 118.5).  Slices of 3 to 5 K-tiles are measured faster the other way, slices
+    // of a column tile next to each other: 1024 x 3072 at 700 rows in 16 of 3 22.4, in the order above 25.4, 1024 x 4096 at 900 in 16 of
+    // 4 26.0 / 27.5, 2560 x 2560 at 600 in 8 of 5 24.4 / 25.7; in 10 of 6 1024 x 4096 at 1100 26.5 / 25.7.
     m_t = b % mtiles;
     const int rest = b / mtiles;
-    split = rest % nsplit;
-    n_t = rest / nsplit;
+    if (ks_per_split >= 6) {
+      split = rest / ntiles;
+      n_t = rest - split * ntiles;
+    } else {
+      split = rest % nsplit;
+      n_t = rest / nsplit;
+    }
   }
   const int ks0 = split * ks_per_split;
   const int nt = max(0, min(K / PBK, ks0 + ks_per_split) - ks0);

@@ -536,3 +536,20 @@ def test_equal_rows_of_several_row_tiles(cuda, m, n, swiglu):
     from distributed_llms_amd.ops import quant
     q = quant.linear_fp8(x, quant.quantize_weight(w), swiglu=swiglu, splits=1)
     assert torch.equal(q, q[:1].expand_as(q))
+
+
+# slices on either side of six K-tiles (where the order of the workgroups changes), the last one shorter, one to three row and column tiles
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [1, 256, 257, 700])
+@pytest.mark.parametrize("n,k,s", [(256, 640, 2), (512, 640, 2), (768, 704, 2), (256, 1088, 3), (512, 1216, 3), (768, 2112, 8)])
+def test_pp_slices(cuda, m, n, k, s):
+    from distributed_llms_amd.ops import gemm
+    g = torch.Generator("cuda").manual_seed(m + n + k)
+    x = torch.randn(m, k, generator=g, device="cuda").bfloat16()
+    w = (torch.randn(n, k, generator=g, device="cuda") * k ** -0.5).bfloat16()
+    part = gemm.linear_pp(x, w, splits=s, variant=gemm.PP_PREFILL_VARIANT, defer=True)
+    kts = -(-(k // 64) // s) * 64
+    slabs = part.ws.view(torch.float16)[:part.splits * m * n].view(part.splits, m, n)
+    for i in range(part.splits):
+        want = x[:, i * kts:(i + 1) * kts].double() @ w[:, i * kts:(i + 1) * kts].double().T * 2.0 ** -6
+        assert (slabs[i].double() - want).norm() <= 2.0 ** -10 * want.norm()    # (one rounding to f16 and f32 sums)
