@@ -43,10 +43,14 @@ struct KVChunk {
   bf16x8 v[D / 16];
 };
 
+// last: the last of the chunk's keys that is of use (31: all of them).  Lanes of later keys read key 0's K row and group 0's V^T tile again,
+// lines that other lanes ask for anyway: a chunk of a few keys is as few requests, of which a CU has some 256 under way.
 template <int D, bool NT = false>
 __device__ __forceinline__ void load_chunk(KVChunk<D>& c, const bf16* __restrict__ kblk,
-                                           const bf16* __restrict__ vblk, int lane) {
+                                           const bf16* __restrict__ vblk, int lane, int last = kBS - 1) {
   const int r = lane & 15, g = lane >> 4;
+  const int key = 8 * (r >> 2) + (r & 3);              // of K row r; row 16 + r holds key + 4 (krow32)
+  const int ra = key <= last ? r : 0, rb = key + 4 <= last ? 16 + r : 0, gv = 8 * g <= last ? g : 0;
 // NT: the decode wave reads each K/V line once per step (cold, HBM): nontemporal loads cut the
 // attention alone 41.4 -> 35.3 us at B=256 / ctx 192 (profiles/attn_fused_ablation.md); prefill
 // re-reads a sequence's K/V for every q tile and keeps the default policy
@@ -54,12 +58,12 @@ __device__ __forceinline__ void load_chunk(KVChunk<D>& c, const bf16* __restrict
                          : *reinterpret_cast<const bf16x8*>(p))
 #pragma unroll
   for (int ks = 0; ks < D / 32; ++ks) {
-    c.ka[ks] = DLLM_KVLD(kblk + r * D + ks * 32 + 8 * g);
-    c.kb[ks] = DLLM_KVLD(kblk + (16 + r) * D + ks * 32 + 8 * g);
+    c.ka[ks] = DLLM_KVLD(kblk + ra * D + ks * 32 + 8 * g);
+    c.kb[ks] = DLLM_KVLD(kblk + rb * D + ks * 32 + 8 * g);
   }
 #pragma unroll
   for (int dt = 0; dt < D / 16; ++dt)
-    c.v[dt] = DLLM_KVLD(vblk + g * 8 * D + (dt * 16 + r) * 8);
+    c.v[dt] = DLLM_KVLD(vblk + gv * 8 * D + (dt * 16 + r) * 8);
 #undef DLLM_KVLD
 }
 
@@ -276,9 +280,9 @@ __device__ __forceinline__ void attn_decode_wave(const bf16* __restrict__ q, bf1
   bf16x8 kn[D / 32];
   bf16 vn[D / 16];
   KVChunk<D> cur, nxt;
-  auto load_at = [&](KVChunk<D>& c, int blk) {
+  auto load_at = [&](KVChunk<D>& c, int blk, int chunk) {
     const size_t base = (size_t)blk * blk_stride + head_off;
-    load_chunk<D, NT>(c, k_cache + base, v_cache + base, lane);
+    load_chunk<D, NT>(c, k_cache + base, v_cache + base, lane, kend - 1 - chunk * kBS);
   };
   WaveState<D> st;
   init_state(st);
@@ -299,7 +303,7 @@ __device__ __forceinline__ void attn_decode_wave(const bf16* __restrict__ q, bf1
     if constexpr (PARTS >= 0) {
 #pragma unroll
       for (int ks = 0; ks < D / 32; ++ks) qp[ks].load(ra, q_at + ks * 32);
-      load_at(cur, blk_0);
+      load_at(cur, blk_0, c0);
       kp.load(ra, k_at);
       vp.load(ra, v_at);
     } else {
@@ -326,7 +330,7 @@ __device__ __forceinline__ void attn_decode_wave(const bf16* __restrict__ q, bf1
         for (int j = 0; j < 8; ++j) qp[ks].q[j] = f2bf(aq[ks][j]);
 #pragma unroll
       for (int j = 0; j < 2; ++j) kp.q[j] = f2bf(akv[j]), vp.q[j] = f2bf(akv[2 + j]);
-      load_at(cur, blk_0);
+      load_at(cur, blk_0, c0);
     }
     if (ra.cos_sin) rr.load(ra.cos_sin + (size_t)pos_b * D, g);
     __builtin_amdgcn_sched_barrier(0);
@@ -363,7 +367,7 @@ __device__ __forceinline__ void attn_decode_wave(const bf16* __restrict__ q, bf1
       if (!col_ok) v = bf16x8{};
       qf[ks] = v;
     }
-    load_at(cur, blk_0);
+    load_at(cur, blk_0, c0);
   }
   // FUSED: put the new key into the registers of its chunk (lane masks inside that chunk only)
   const int cnew = FUSED ? (ctx - 1) / kBS : -1;
@@ -412,15 +416,15 @@ __device__ __forceinline__ void attn_decode_wave(const bf16* __restrict__ q, bf1
     // key, is left for behind the loop
     int j = 0;
     for (; j + 2 < n; j += 2) {
-      load_at(nxt, block(j + 1));
+      load_at(nxt, block(j + 1), cb + j + 1);
       __builtin_amdgcn_sched_barrier(0);
       compute_chunk<D, false>(st, qf, cur, 0, 0, scale_log2, lane);
-      load_at(cur, block(j + 2));
+      load_at(cur, block(j + 2), cb + j + 2);
       __builtin_amdgcn_sched_barrier(0);
       compute_chunk<D, false>(st, qf, nxt, 0, 0, scale_log2, lane);
     }
     if (j + 1 < n) {
-      load_at(nxt, block(j + 1));
+      load_at(nxt, block(j + 1), cb + j + 1);
       __builtin_amdgcn_sched_barrier(0);
       compute_chunk<D, false>(st, qf, cur, 0, 0, scale_log2, lane);
       patch(nxt, cb + j + 1, (size_t)block(j + 1) * blk_stride + head_off);
@@ -431,7 +435,7 @@ __device__ __forceinline__ void attn_decode_wave(const bf16* __restrict__ q, bf1
     }
     if (cb + 64 < c1) {                             // the next pass's first chunk
       my_blk = bt[min(cb + 64 + lane, max_blocks - 1)];
-      load_at(cur, block(0));
+      load_at(cur, block(0), cb + 64);
     }
   }
   if (owns_new && append) {

@@ -243,6 +243,38 @@ def test_paged_attention_decode_fused_rope(cuda, hq, hkv, d, lens, rope):
     torch.testing.assert_close(v1.float(), v2, atol=0, rtol=0)
 
 
+@pytest.mark.parametrize("hq,hkv,d", [(32, 8, 128), (12, 12, 64), (4, 1, 128)])
+@pytest.mark.parametrize("most", [66, 70 * 32])
+def test_decode_reads_no_key_behind_the_last(cuda, hq, hkv, d, most):
+    """Lanes of a last chunk's later keys read lines of earlier ones: K rows behind the last key and V^T tiles behind its group of eight
+    may hold anything (contexts of every length within three chunks; with a long one beside them, behind split keys)."""
+    lens = list(range(1, 67)) + ([most - 3, most - 31] if most > 66 else [])
+    k, v, bt = _fill_paged(lens, hkv, d)
+    b, sl = len(lens), torch.tensor(lens, dtype=torch.int32, device="cuda")
+    q, qkv, scale = _bf(b, hq, d), _bf(b, (hq + 2 * hkv) * d), 1 / math.sqrt(d)
+    slots = torch.stack([bt[i, (n - 1) // 32] * 32 + (n - 1) % 32 for i, n in enumerate(lens)]).to(torch.int32)
+    cs = ref.rope_cos_sin(d, 4096, 500000.0, device="cuda")
+    outs = []
+    for fill in (0.0, float("nan")):
+        k1, v1 = k.clone(), v.clone()
+        for i, n in enumerate(lens):
+            blk = bt[i, (n - 1) // 32].item()
+            v1[blk].view(hkv, 4, d, 8)[:, ((n - 1) % 32) // 8 + 1:] = fill
+            for j in range((n - 1) % 32 + 1, 32):
+                k1[blk, :, ((j & 4) << 2) + ((j >> 3) << 2) + (j & 3)] = fill
+        kr, vr = k1.clone(), v1.clone()
+        outs.append((ops.paged_attention_decode(q, k1, v1, bt, sl, scale),
+                     ops.paged_attention_decode_rope(qkv, sl - 1, cs, kr, vr, slots, bt, sl, hq, hkv, d, scale)))
+        if fill == 0.0:
+            kf, vf = k1.float(), v1.float()
+            want = ref.paged_attention_decode(q.float(), kf, vf, bt, sl, scale)
+            q2 = ref.rope_cache_append(qkv.float(), sl - 1, cs, kf, vf, slots, hq, hkv, d)
+            for got, expect in zip(outs[0], (want, ref.paged_attention_decode(q2, kf, vf, bt, sl, scale))):
+                torch.testing.assert_close(got.float(), expect, atol=2e-2, rtol=2e-2)
+    for x, y in zip(*outs):
+        assert torch.equal(x, y)
+
+
 @pytest.mark.parametrize("version", ["3", "4", "6", "7", "9"])
 @pytest.mark.parametrize("hq,hkv,d", [(32, 8, 128), (64, 8, 128), (12, 12, 64), (8, 4, 64), (16, 16, 128),
                                       (32, 2, 128)])
