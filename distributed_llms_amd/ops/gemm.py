@@ -30,6 +30,8 @@ K = 8192 projections of 70B-class models (qkv 8192 -> 10240, o 8192 -> 8192) sta
 """
 from __future__ import annotations
 
+import functools
+import operator
 from typing import Optional
 
 import torch
@@ -164,9 +166,14 @@ def _pf_wgs(cus: int) -> int:
     return max(8, (cus - _comm_cus) // 8 * 8)
 
 
+@functools.lru_cache(maxsize=64)
+def _roles(names: str) -> frozenset:
+    return frozenset(t for t in names.split(",") if t and t != "none")
+
+
 def _use_wide(m: int, n: int, k: int, x: torch.Tensor, w: torch.Tensor, swiglu: bool = False) -> bool:
     kn = knobs.K
-    roles = {t for t in kn.wide.split(",") if t and t != "none"}
+    roles = _roles(kn.wide)
     if not roles or m < 1 or n % 128 or k % 64:
         return False
     if not (x.dtype == w.dtype == torch.bfloat16 and x.is_contiguous() and w.is_contiguous()):
@@ -530,34 +537,48 @@ def linear_wide(x: torch.Tensor, w: torch.Tensor, splits: int = 0, swiglu: bool 
     k = x.shape[-1]
     n = w.shape[0]
     m = x.numel() // k
-    if splits == 0 and variant < 0 and use_sq(m, n, k, swiglu):
+    own = splits == 0 and variant < 0
+    sq, s, tall, v = _wide_plan(m, n, k, swiglu, splits, variant, _comm_cus, _WIDE_KNOBS(knobs.K))
+    if sq:
         return linear_sq(x, w, swiglu=swiglu, defer=defer)
     if not (x.dtype == w.dtype == torch.bfloat16 and x.is_contiguous() and w.is_contiguous()):
         raise ValueError("linear_wide: bf16 contiguous operands")
     if n % 128 or k % 64:
         raise ValueError("linear_wide: N % 128 and K % 64")
-    s = splits or wide_splits(m, n, k, swiglu)
-    if m == 1 and not splits and variant < 0 and (s == 1 or (defer and not swiglu)) and one_fits(n, k, s, swiglu) \
-            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0:
+    xp, wp = x.data_ptr(), w.data_ptr()
+    if m == 1 and own and (s == 1 or (defer and not swiglu)) and one_fits(n, k, s, swiglu) and not (xp | wp) % 16:
         return _one(x, w, s, swiglu, x.shape[:-1], x=x)
-    ws = _workspace(x.device)
-    if s > 1 and s * m * n > ws.numel():
-        s = max(1, ws.numel() // (m * n))
-    stream = current_stream()
-    bm = wide_row_tile(m, n, k, swiglu)
-    tall = duo_row_tile(m, n, k, s, bm, swiglu) if not splits and variant < 0 else 0
-    if tall and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0:
+    if tall and not (xp | wp) % 16:
         return _duo(x, w, m, n, k, s, tall, swiglu, defer)
-    v = variant if variant >= 0 else wide_variant(m, n, k, s, bm)
-    if bm != wide_bm(m):
-        v |= bm << 8
+    ws = _workspace(x.device)
+    stream = current_stream()
     if defer and not swiglu and s > 1:
-        se = _ext.kernels().gemm_wide(0, x.data_ptr(), w.data_ptr(), ws.data_ptr(), ws.numel(), m, n, k, s, 2, v, stream)
+        se = _ext.kernels().gemm_wide(0, xp, wp, ws.data_ptr(), _WS_FLOATS, m, n, k, s, 2, v, stream)
         return SplitKPartial(ws, se, m, n, (*x.shape[:-1], n), x.dtype, x.device)
     y = torch.empty(*x.shape[:-1], n // 2 if swiglu else n, dtype=x.dtype, device=x.device)
-    _ext.kernels().gemm_wide(y.data_ptr(), x.data_ptr(), w.data_ptr(), ws.data_ptr(), ws.numel(), m, n, k, s,
-                             1 if swiglu else 0, v, stream)
+    _ext.kernels().gemm_wide(y.data_ptr(), xp, wp, ws.data_ptr(), _WS_FLOATS, m, n, k, s, 1 if swiglu else 0, v, stream)
     return y
+
+
+_WIDE_KNOBS = operator.attrgetter("sq", "sq_min_m", "sq_split", "wide_target_wgs", "wide_small_bm", "wide_small_bm_maxw", "wide_variant",
+                                  "wide_variant_split", "duo")
+
+
+@functools.lru_cache(maxsize=1024)         # a pass asks for the same few products in every layer, 6 us each
+def _wide_plan(m: int, n: int, k: int, swiglu: bool, splits: int, variant: int, comm_cus: int, kn: tuple):
+    """linear_wide's (does gemm_sq take it, K slices, gemm_duo's row tile or 0, variant word) for sizes, a caller's own slices and
+    variant, the CUs reserved for communication and what is read of the knobs."""
+    own = splits == 0 and variant < 0
+    if own and use_sq(m, n, k, swiglu):
+        return True, 0, 0, 0
+    if n % 128 or k % 64:
+        return False, 0, 0, 0
+    s = splits or wide_splits(m, n, k, swiglu)
+    if s > 1 and s * m * n > _WS_FLOATS and not (m == 1 and own):
+        s = max(1, _WS_FLOATS // (m * n))
+    bm = wide_row_tile(m, n, k, swiglu)
+    v = variant if variant >= 0 else wide_variant(m, n, k, s, bm)
+    return False, s, duo_row_tile(m, n, k, s, bm, swiglu) if own else 0, v | bm << 8 if bm != wide_bm(m) else v
 
 
 def duo_fits(m: int, n: int, k: int, s: int, bm: int, swiglu: bool = False) -> bool:
@@ -747,7 +768,7 @@ def sq_role(n: int, k: int, swiglu: bool) -> str:
 
 def use_sq(m: int, n: int, k: int, swiglu: bool = False) -> bool:
     kn = knobs.K
-    roles = {t for t in kn.sq.split(",") if t and t != "none"}
+    roles = _roles(kn.sq)
     if not roles or not (kn.sq_min_m <= m <= 256) or n % 256 or k % 64:
         return False
     if not kn.sq_split and sq_splits(m, n, k) > 1:
