@@ -43,6 +43,9 @@ PYBIND11_MODULE(_C_kernels, m) {
         py::arg("mode"), py::arg("variant"), py::arg("stream"), py::arg("limit") = 0.f, py::arg("bm") = 256, py::arg("bias") = 0, py::arg("wgs") = 0);
   m.def("gemm_pf8", &dllm::gemm_pf8);
   m.def("moe_combine", &dllm::moe_combine);
+  m.def("moe_combine_norm", &dllm::moe_combine_norm);
+  m.def("moe_scatter", &dllm::moe_scatter);
+  m.def("splitk_norm_route", &dllm::splitk_norm_route);
   m.def("moe_wide_gemm", &dllm::moe_wide_gemm, py::arg("y"), py::arg("x"), py::arg("gather"), py::arg("w"), py::arg("counts"), py::arg("offsets"), py::arg("experts"), py::arg("n"), py::arg("k"), py::arg("mode"), py::arg("stream"),
         py::arg("limit") = 0.f);
   m.def("moe_router_route", &dllm::moe_router_route);

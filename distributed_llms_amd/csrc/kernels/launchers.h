@@ -64,6 +64,12 @@ void moe_wide_gemm(uintptr_t y, uintptr_t x, uintptr_t gather, uintptr_t w, uint
                    int E, int N, int K, int mode, uintptr_t stream, float limit);
 void moe_wide_gemm_fp8(uintptr_t y, uintptr_t x, uintptr_t gather, uintptr_t w, uintptr_t counts, uintptr_t offsets,
                        int E, int N, int K, int mode, uintptr_t sa, uintptr_t wscale, uintptr_t stream);
+void moe_scatter(uintptr_t topk_ids, int T, int E, int k, uintptr_t counts, uintptr_t offsets, uintptr_t sorted_tok, uintptr_t inv,
+                 uintptr_t stream);
+void moe_combine_norm(uintptr_t y, uintptr_t residual, uintptr_t ysorted, uintptr_t topk_w, uintptr_t inv, uintptr_t w, int T, int H, int k,
+                      float eps, uintptr_t stream);
+void splitk_norm_route(uintptr_t y, uintptr_t residual, uintptr_t ws, int S, int M, int N, uintptr_t w, float eps, uintptr_t router, int E,
+                       int k, uintptr_t topk_w, uintptr_t topk_ids, uintptr_t stream);
 void moe_combine(uintptr_t out, uintptr_t ysorted, uintptr_t topk_w, uintptr_t inv, int T, int H, int k,
                  uintptr_t stream);
 

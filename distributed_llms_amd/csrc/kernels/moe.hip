@@ -12,6 +12,7 @@
 #include "skinny_common.h"
 #include "launchers.h"
 #include "stream_common.h"
+#include "moe_top.h"
 
 namespace dllm {
 
@@ -116,36 +117,9 @@ __global__ void __launch_bounds__(256) moe_router_kernel(const bf16* __restrict_
   __syncthreads();
   if (threadIdx.x != 0) return;
   float p[E];
-  float mx = -INFINITY;
 #pragma unroll
-  for (int e = 0; e < E; ++e) {
-    p[e] = bf2f(f2bf(((part[0][e] + part[1][e]) + part[2][e]) + part[3][e]));
-    mx = fmaxf(mx, p[e]);
-  }
-  float sum = 0.f;
-#pragma unroll
-  for (int e = 0; e < E; ++e) {
-    p[e] = __expf(p[e] - mx);
-    sum += p[e];
-  }
-  int ids[8];
-  float ws[8];
-  float tot = 0.f;
-  for (int j = 0; j < k; ++j) {
-    int best = 0;
-    float bv = -1.f;
-#pragma unroll
-    for (int e = 0; e < E; ++e)
-      if (p[e] > bv) { bv = p[e]; best = e; }
-    ids[j] = best;
-    ws[j] = bv / sum;
-    tot += ws[j];
-    p[best] = -2.f;
-  }
-  for (int j = 0; j < k; ++j) {
-    topk_ids[t * k + j] = ids[j];
-    topk_w[t * k + j] = ws[j] / tot;
-  }
+  for (int e = 0; e < E; ++e) p[e] = ((part[0][e] + part[1][e]) + part[2][e]) + part[3][e];
+  moe_top<E>(p, t, k, topk_w, topk_ids);
 }
 
 __global__ void __launch_bounds__(1024) moe_scatter_kernel(const int* __restrict__ topk_ids, int T, int E, int k,
@@ -279,6 +253,79 @@ __global__ void __launch_bounds__(256) moe_combine_kernel(bf16* __restrict__ out
   }
 }
 
+// The combine in the launch of the add and RMS norm behind it: h = the combine's bf16 row, r = bf16(h + residual), residual <- r, y = rmsnorm(r) w, with
+// moe_combine_kernel's and rms_norm_kernel's bits (the same sums per element, the same vectors per thread).  Bound by the round trips of a short launch
+// (slots and weights, then the experts' rows; the residual and the norm's weight are loaded beside the former); apart they were two such launches:
+// 16 rows of 4096, two experts a token, traced in a decode step 5.3 + 5.3 -> 5.3 us.
+template <int MAXV>
+__global__ void __launch_bounds__(256) moe_combine_norm_kernel(bf16* __restrict__ y, bf16* __restrict__ residual,
+                                                               const bf16* __restrict__ ysorted, const float* __restrict__ topk_w,
+                                                               const int* __restrict__ inv_slot, const bf16* __restrict__ w, int H, int k,
+                                                               float eps) {
+  __shared__ float red[16];
+  const int t = blockIdx.x, nvec = H >> 3;
+  bf16x8* rr = reinterpret_cast<bf16x8*>(residual + (size_t)t * H);
+  bf16x8 b[MAXV], g[MAXV], a[MAXV];
+  float v[MAXV][8];
+#pragma unroll
+  for (int i = 0; i < MAXV; ++i) {
+    const int at = min((int)threadIdx.x + i * 256, nvec - 1);
+    b[i] = rr[at];
+    g[i] = reinterpret_cast<const bf16x8*>(w)[at];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[i][j] = 0.f;
+  }
+  for (int j = 0; j < k; j += 2) {                       // two experts' rows under way
+    const int j1 = min(j + 1, k - 1);
+    const float w0 = topk_w[t * k + j], w1 = topk_w[t * k + j1];
+    const bf16x8* y0 = reinterpret_cast<const bf16x8*>(ysorted + (size_t)inv_slot[t * k + j] * H);
+    const bf16x8* y1 = reinterpret_cast<const bf16x8*>(ysorted + (size_t)inv_slot[t * k + j1] * H);
+    bf16x8 e0[MAXV], e1[MAXV];
+#pragma unroll
+    for (int i = 0; i < MAXV; ++i) {
+      const int at = min((int)threadIdx.x + i * 256, nvec - 1);
+      e0[i] = y0[at];
+      e1[i] = y1[at];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < MAXV; ++i)
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        v[i][q] = fmaf(w0, bf2f(e0[i][q]), v[i][q]);
+        if (j + 1 < k) v[i][q] = fmaf(w1, bf2f(e1[i][q]), v[i][q]);
+      }
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < MAXV; ++i) {
+    const int at = threadIdx.x + i * 256;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) a[i][q] = f2bf(bf2f(f2bf(v[i][q])) + bf2f(b[i][q]));
+    if (at < nvec) {
+      rr[at] = a[i];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        v[i][q] = bf2f(a[i][q]);
+        ss += v[i][q] * v[i][q];
+      }
+    }
+  }
+  ss = block_sum<256>(ss, red);
+  const float inv = rsqrtf(ss / (float)H + eps);
+  bf16x8* yr = reinterpret_cast<bf16x8*>(y + (size_t)t * H);
+#pragma unroll
+  for (int i = 0; i < MAXV; ++i) {
+    const int at = threadIdx.x + i * 256;
+    if (at < nvec) {
+      bf16x8 o;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) o[q] = f2bf(v[i][q] * inv * bf2f(g[i][q]));
+      yr[at] = o;
+    }
+  }
+}
+
 // ------------------------------------------------------------------ launchers
 void moe_route(uintptr_t logits, int T, int E, int k, uintptr_t topk_w, uintptr_t topk_ids, uintptr_t counts,
                uintptr_t offsets, uintptr_t sorted_tok, uintptr_t inv, uintptr_t stream) {
@@ -309,6 +356,35 @@ void moe_router_route(uintptr_t x, uintptr_t w, int T, int H, int E, int k, uint
   DLLM_HIP_CHECK(hipGetLastError());
   hipLaunchKernelGGL(moe_scatter_kernel, dim3(1), dim3(1024), 0, s, (const int*)topk_ids, T, E, k, (int*)counts,
                      (int*)offsets, (int*)sorted_tok, (int*)inv);
+  DLLM_HIP_CHECK(hipGetLastError());
+}
+
+// the counts, offsets and slot lists of choices that are made already
+void moe_scatter(uintptr_t topk_ids, int T, int E, int k, uintptr_t counts, uintptr_t offsets, uintptr_t sorted_tok, uintptr_t inv,
+                 uintptr_t stream) {
+  DLLM_HOST_CHECK(E >= 1 && E <= kMaxExperts && k >= 1 && k <= E && T >= 0, "1 <= experts <= 64");
+  if (T == 0) return;
+  hipLaunchKernelGGL(moe_scatter_kernel, dim3(1), dim3(1024), 0, reinterpret_cast<hipStream_t>(stream), (const int*)topk_ids, T, E, k,
+                     (int*)counts, (int*)offsets, (int*)sorted_tok, (int*)inv);
+  DLLM_HIP_CHECK(hipGetLastError());
+}
+
+// y [T, H], residual [T, H] (updated), ysorted [T k, H], topk_w / inv [T, k], w [H]
+void moe_combine_norm(uintptr_t y, uintptr_t residual, uintptr_t ysorted, uintptr_t topk_w, uintptr_t inv, uintptr_t w, int T, int H, int k,
+                      float eps, uintptr_t stream) {
+  DLLM_HOST_CHECK(H % 8 == 0 && H > 0 && H <= 8 * 256 * 8, "hidden must be a multiple of 8 and <= 16384");
+  DLLM_HOST_CHECK(T >= 0 && k >= 1 && k <= 8, "1 <= top_k <= 8");
+  DLLM_HOST_CHECK((y | residual | ysorted | w) % 16 == 0, "alignment");
+  if (T == 0) return;
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(T), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), (bf16*)y, (bf16*)residual, (const bf16*)ysorted,
+                       (const float*)topk_w, (const int*)inv, (const bf16*)w, H, k, eps);
+  };
+  const int nvec = H / 8;
+  if (nvec <= 256) go(moe_combine_norm_kernel<1>);
+  else if (nvec <= 512) go(moe_combine_norm_kernel<2>);
+  else if (nvec <= 1024) go(moe_combine_norm_kernel<4>);
+  else go(moe_combine_norm_kernel<8>);
   DLLM_HIP_CHECK(hipGetLastError());
 }
 

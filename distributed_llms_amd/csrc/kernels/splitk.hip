@@ -8,6 +8,7 @@
 // before the first add (nontemporal: slabs are read once).
 #include "common.h"
 #include "launchers.h"
+#include "moe_top.h"
 
 namespace dllm {
 
@@ -91,11 +92,22 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(bf16* __restrict__ o
 // Bit-identical to splitk_reduce_kernel followed by rms_norm_kernel with a residual (same
 // per-element summation order, same thread -> vector mapping for the sum of squares), minus one
 // launch and the bf16 h round trip through HBM.  One 256-thread workgroup per row.
-template <int MAXV, int SC, bool EX, int NTH = 256>
+//
+// E > 0 (EX): also the router of E experts behind it, moe_router_kernel's logits of the row and the choice of k experts, with its bits.  Its
+// weights, 64 KiB of E = 8, are asked for with the slabs; as a launch of its own it was another three round trips (16 rows of 4096 in 8 slabs,
+// traced in a decode step, norm + router 5.5 + 5.2 -> 5.7 us).  Where its weights are more than that (8192 wide, 16 experts) the launch stays.
+struct RouteArgs {
+  const bf16* w;            // [E, N]
+  float* topk_w;            // [M, k]
+  int* topk_ids;
+  int k;
+};
+template <int MAXV, int SC, bool EX, int NTH = 256, int E = 0>
 __global__ void __launch_bounds__(NTH) splitk_add_rms_norm_kernel(bf16* __restrict__ y, bf16* __restrict__ residual,
                                                                   const float* __restrict__ P, int S_, int M, int N,
                                                                   const bf16* __restrict__ w, float eps,
-                                                                  uint8_t* __restrict__ q8, float* __restrict__ qs) {
+                                                                  uint8_t* __restrict__ q8, float* __restrict__ qs,
+                                                                  RouteArgs ro) {
   // SC > 0: the slab count is a compile-time constant, so all of a vector's 2*SC slab loads are
   // issued before the first add (the runtime-S loop waited on each slab in turn)
   //
@@ -121,6 +133,10 @@ __global__ void __launch_bounds__(NTH) splitk_add_rms_norm_kernel(bf16* __restri
   float ss = 0.f;
 #pragma unroll
   for (int k = 0; k < MAXV; ++k) g[k] = wv[min((int)threadIdx.x + k * NTH, nvec - 1)];
+  // (moe_router_kernel's places: a quarter of the row per wave, 64 vectors at a time)
+  static_assert(E == 0 || (EX && NTH == 256 && CH == MAXV), "whole rows of 256 threads");
+  const int lane = threadIdx.x & 63, rv = (threadIdx.x >> 6) * 64 * MAXV + lane;
+  [[maybe_unused]] bf16x8 rw[E > 0 ? MAXV : 1][E > 0 ? E : 1];
 #pragma unroll
   for (int c0 = 0; c0 < MAXV; c0 += CH) {
     f32x4 a0[CH], a1[CH];
@@ -135,6 +151,12 @@ __global__ void __launch_bounds__(NTH) splitk_add_rms_norm_kernel(bf16* __restri
         b[i] = rr[idc];
 #pragma unroll
         for (int s = 0; s < SC; ++s) l[i][s] = __builtin_nontemporal_load(reinterpret_cast<const raw*>(p + s * slab));
+      }
+      if constexpr (E > 0) {
+#pragma unroll
+        for (int u = 0; u < MAXV; ++u)
+#pragma unroll
+          for (int e = 0; e < E; ++e) rw[u][e] = reinterpret_cast<const bf16x8*>(ro.w)[e * nvec + rv + 64 * u];
       }
       __builtin_amdgcn_sched_barrier(0);   // (hipcc kept 8 of the loads back until the first had come in)
 #pragma unroll
@@ -187,6 +209,7 @@ __global__ void __launch_bounds__(NTH) splitk_add_rms_norm_kernel(bf16* __restri
                             red);
     return;
   }
+  __shared__ bf16x8 line[E > 0 ? MAXV * NTH : 1];
   bf16x8* yr = reinterpret_cast<bf16x8*>(y + (size_t)row * N);
 #pragma unroll
   for (int i = 0; i < MAXV; ++i) {
@@ -196,7 +219,35 @@ __global__ void __launch_bounds__(NTH) splitk_add_rms_norm_kernel(bf16* __restri
 #pragma unroll
       for (int j = 0; j < 8; ++j) o[j] = f2bf(v[i][j] * inv * bf2f(g[i][j]));
       yr[idx] = o;
+      if constexpr (E > 0) line[idx] = o;
     }
+  }
+  if constexpr (E > 0) {
+    __shared__ float sums[4][E > 0 ? E : 1];
+    float acc[E > 0 ? E : 1];
+#pragma unroll
+    for (int e = 0; e < E; ++e) acc[e] = 0.f;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < MAXV; ++u) {
+      const bf16x8 xv = line[rv + 64 * u];
+#pragma unroll
+      for (int e = 0; e < E; ++e)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) acc[e] = fmaf(bf2f(xv[i]), bf2f(rw[u][e][i]), acc[e]);
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e) acc[e] = wave_sum(acc[e]);
+    if (lane == 0) {
+#pragma unroll
+      for (int e = 0; e < E; ++e) sums[threadIdx.x >> 6][e] = acc[e];
+    }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    float p[E > 0 ? E : 1];
+#pragma unroll
+    for (int e = 0; e < E; ++e) p[e] = ((sums[0][e] + sums[1][e]) + sums[2][e]) + sums[3][e];
+    moe_top<E>(p, row, ro.k, ro.topk_w, ro.topk_ids);
   }
 }
 
@@ -215,7 +266,7 @@ void splitk_add_rms_norm_q8(uintptr_t y, uintptr_t residual, uintptr_t ws, int S
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   auto go = [&](auto kern) {
     hipLaunchKernelGGL(kern, dim3(M), dim3(256), 0, s, (bf16*)y, (bf16*)residual, (const float*)ws, S, M, N,
-                       (const bf16*)w, eps, (uint8_t*)q8, (float*)qs);
+                       (const bf16*)w, eps, (uint8_t*)q8, (float*)qs, RouteArgs{});
   };
   const int nvec = N / 8;
 #define DLLM_SKN2(MV, EX)                                              \
@@ -240,6 +291,27 @@ void splitk_add_rms_norm_q8(uintptr_t y, uintptr_t residual, uintptr_t ws, int S
   else DLLM_SKN(8);
 #undef DLLM_SKN
 #undef DLLM_SKN2
+  DLLM_HIP_CHECK(hipGetLastError());
+}
+
+// splitk_add_rms_norm and the choice of k of 8 experts by the normed rows (router [8, N]): 4 or 8 slabs of rows of 2048 or 4096
+void splitk_norm_route(uintptr_t y, uintptr_t residual, uintptr_t ws, int S, int M, int N, uintptr_t w, float eps, uintptr_t router, int E,
+                       int k, uintptr_t topk_w, uintptr_t topk_ids, uintptr_t stream) {
+  DLLM_HOST_CHECK(E == 8 && (N == 2048 || N == 4096) && (S == 4 || S == 8), "8 experts, rows of 2048 or 4096, 4 or 8 slabs");
+  DLLM_HOST_CHECK(k >= 1 && k <= E && M >= 0, "1 <= top_k <= 8");
+  DLLM_HOST_CHECK((y | residual | ws | w | router) % 16 == 0, "alignment");
+  if (M == 0) return;
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(M), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), (bf16*)y, (bf16*)residual, (const float*)ws, S, M,
+                       N, (const bf16*)w, eps, nullptr, nullptr, RouteArgs{(const bf16*)router, (float*)topk_w, (int*)topk_ids, k});
+  };
+  if (N == 2048) {
+    if (S == 8) go(splitk_add_rms_norm_kernel<1, 8, true, 256, 8>);
+    else go(splitk_add_rms_norm_kernel<1, 4, true, 256, 8>);
+  } else {
+    if (S == 8) go(splitk_add_rms_norm_kernel<2, 8, true, 256, 8>);
+    else go(splitk_add_rms_norm_kernel<2, 4, true, 256, 8>);
+  }
   DLLM_HIP_CHECK(hipGetLastError());
 }
 

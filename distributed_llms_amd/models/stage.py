@@ -357,11 +357,13 @@ class ModelStage:
                                             meta.block_tables, meta.seq_lens, self.hq, self.hkv, self.cfg.head_dim, self.scale,
                                             wo, max_ctx=meta.max_ctx or None, workspace=meta.attn_workspace)
 
-    def _mlp(self, h: Optional[torch.Tensor], lw: Dict[str, torch.Tensor], gated: Optional[torch.Tensor] = None) -> torch.Tensor:
-        """``gated``: the dense MLP's activation, where the launch of its norm has made it already (``h`` is None then)."""
+    def _mlp(self, h: Optional[torch.Tensor], lw: Dict[str, torch.Tensor], gated: Optional[torch.Tensor] = None, choice=None):
+        """``gated``: the dense MLP's activation, where the launch of its norm has made it already (``h`` is None then).  ``choice``: the choice of
+        experts that the norm's launch has made (ops.moe.norm_route)."""
         if self.cfg.is_moe:
             out = ops.moe_forward(h, lw["router"], lw["experts_gate_up"], lw["experts_down"],
-                                  self.cfg.experts_per_token, self.tp.expert_offset(self.cfg.num_experts))
+                                  self.cfg.experts_per_token, self.tp.expert_offset(self.cfg.num_experts), choice,
+                                  defer=not self.tp.enabled)
             return self.tp.all_reduce_(out) if self.tp.enabled else out
         # defer: the down projection's split-K reduce is fused into the next residual-add + RMSNorm
         # (under TP the partial [T, H] is all-reduced first, so it is materialised)
@@ -381,7 +383,7 @@ class ModelStage:
 
     @staticmethod
     def _dense(t):
-        return t.materialize() if isinstance(t, ops.gemm.SplitKPartial) else t
+        return t.materialize() if isinstance(t, (ops.gemm.SplitKPartial, ops.moe.Combine)) else t
 
     def _forward_llama(self, inp: torch.Tensor, meta: BatchMeta) -> torch.Tensor:
         cfg = self.cfg
@@ -408,6 +410,8 @@ class ModelStage:
                 if self.has(l, 0):
                     # one row: the add and the norm in the projection's launch
                     defer = knobs.K.defer_qkv and self.has(l, 1)
+                    if residual.shape[0] == 1 and isinstance(h, ops.moe.Combine):
+                        h = h.materialize()
                     one = ops.norm_linear(h, residual, lw["attn_norm"], eps, lw["wqkv"]) if defer else None
                     if one is not None:
                         qkv, residual = one
@@ -442,9 +446,12 @@ class ModelStage:
             # ---- MLP half: atoms 3 / 4 (first / second half of the intermediate columns)
             if self.has(l, 3) or self.has(l, 4):
                 one = None if cfg.is_moe else ops.norm_linear(h, residual, lw["mlp_norm"], eps, lw["w_gate_up"], swiglu=True)
-                x = gated = None
+                route = ops.moe.norm_route(h, residual, lw["mlp_norm"], eps, lw["router"], cfg.experts_per_token) if cfg.is_moe else None
+                x = gated = choice = None
                 if one is not None:
                     gated, residual = one
+                elif route is not None:
+                    x, residual, choice = route
                 else:
                     q8 = isinstance(lw.get("w_gate_up"), ops.quant.Fp8Weight)
                     if h is None:
@@ -452,13 +459,13 @@ class ModelStage:
                     else:
                         x, residual = ops.fused_add_rms_norm(h, residual, lw["mlp_norm"], eps, quant_out=q8)
                 if self.has(l, 3) and self.has(l, 4):
-                    h = self._mlp(x, lw, gated)
+                    h = self._mlp(x, lw, gated, choice)
                 elif self.has(l, 3):                  # cut between the MLP halves: hand over the partial sum
-                    out_aux = self._dense(self._mlp(x, lw, gated))
+                    out_aux = self._dense(self._mlp(x, lw, gated, choice))
                     h = None
                     break
                 else:                                 # second half: add the first half's partial sum
-                    h = ops.add_(self._dense(self._mlp(x, lw, gated)), carry)
+                    h = ops.add_(self._dense(self._mlp(x, lw, gated, choice)), carry)
         if out_aux is not None:
             return torch.cat([residual, out_aux.view(out_aux.shape[0], -1)], dim=1)
         if not self.is_last:

@@ -17,7 +17,7 @@ from typing import Optional, Tuple
 import torch
 
 from .. import _ext, knobs
-from . import gemm, quant
+from . import gemm, moe, quant
 from . import reference as ref
 from .stream import current_stream as _stream
 
@@ -86,6 +86,15 @@ def fused_add_rms_norm(x: torch.Tensor, residual: torch.Tensor, w: torch.Tensor,
     ``x`` may be a :class:`gemm.SplitKPartial` (split-K GEMM output not yet reduced): the
     reduction then happens inside the same kernel (splitk_add_rms_norm).  ``quant_out``: the
     normalised output comes back as a :class:`quant.Fp8Act` (see :func:`rms_norm`)."""
+    if isinstance(x, moe.Combine):
+        if quant_out or w.data_ptr() % 16 or residual.data_ptr() % 16:
+            x = x.materialize()
+        else:
+            _ck(residual, "fused_add_rms_norm.residual")
+            _ck(w, "fused_add_rms_norm.w")
+            if tuple(x.shape) != tuple(residual.shape):
+                raise ValueError("x/residual shape mismatch")
+            return x.add_norm(residual, w, eps), residual
     if isinstance(x, gemm.SplitKPartial):
         _ck(residual, "fused_add_rms_norm.residual")
         _ck(w, "fused_add_rms_norm.w")
@@ -570,17 +579,14 @@ def argmax(logits: torch.Tensor) -> torch.Tensor:
 
 # ------------------------------------------------------------ K11/K12
 def moe_route(router_logits: torch.Tensor, top_k: int):
-    from . import moe
     return moe.route(router_logits, top_k)
 
 
 def moe_mlp(x, w_gate_up, w_down, topk_w, topk_ids):
-    from . import moe
     return moe.mlp(x, w_gate_up, w_down, topk_w, topk_ids)
 
 
-def moe_forward(x, w_router, w_gate_up, w_down, top_k: int, expert_offset: int = 0):
+def moe_forward(x, w_router, w_gate_up, w_down, top_k: int, expert_offset: int = 0, choice=None, defer: bool = False):
     """Full Mixtral sparse MLP: route + expert SwiGLU MLPs + weighted combine (``expert_offset``:
     the weights hold experts [offset, offset + E_local) -- expert parallelism, ops/moe.py)."""
-    from . import moe
-    return moe.forward(x, w_router, w_gate_up, w_down, top_k, expert_offset)
+    return moe.forward(x, w_router, w_gate_up, w_down, top_k, expert_offset, choice, defer)

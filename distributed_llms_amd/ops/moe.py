@@ -43,12 +43,58 @@ def mlp(x, w_gate_up, w_down, topk_w, topk_ids):
     return ref.moe_mlp(x, w_gate_up, w_down, topk_w, topk_ids)
 
 
+class Combine:
+    """A mixture's output whose experts' rows are not summed yet (``forward(..., defer=True)``): for ``ops.fused_add_rms_norm``, which sums them
+    in its launch, or :meth:`materialize`."""
+
+    __slots__ = ("ys", "topk_w", "inv", "top_k", "shape", "dtype", "device")
+
+    def __init__(self, ys, topk_w, inv, top_k, like):
+        self.ys, self.topk_w, self.inv, self.top_k = ys, topk_w, inv, top_k
+        self.shape, self.dtype, self.device = like.shape, like.dtype, like.device
+
+    def materialize(self) -> torch.Tensor:
+        t, h = self.shape
+        out = torch.empty(t, h, dtype=self.dtype, device=self.device)
+        _ext.kernels().moe_combine(out.data_ptr(), self.ys.data_ptr(), self.topk_w.data_ptr(), self.inv.data_ptr(), t, h, self.top_k,
+                                   current_stream())
+        return out
+
+    def add_norm(self, residual: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
+        """residual <- residual + output; rms_norm(residual) * w."""
+        t, h = self.shape
+        y = torch.empty_like(residual)
+        _ext.kernels().moe_combine_norm(y.data_ptr(), residual.data_ptr(), self.ys.data_ptr(), self.topk_w.data_ptr(), self.inv.data_ptr(),
+                                        w.data_ptr(), t, h, self.top_k, float(eps), current_stream())
+        return y
+
+
+def norm_route(h, residual: torch.Tensor, norm_w: torch.Tensor, eps: float, w_router: torch.Tensor, top_k: int):
+    """(y, residual, choice): residual <- residual + ``h`` (a split product's slabs), y = rms_norm(residual) * ``norm_w`` and the choice of experts
+    by y that :func:`forward` takes, in one launch with the bits of the two; None for what that kernel does not serve (other inputs
+    than 4 or 8 slabs of rows of 2048 or 4096, other numbers of experts than 8)."""
+    from .gemm import SplitKPartial
+    if not (isinstance(h, SplitKPartial) and h.splits in (4, 8) and h.n in (2048, 4096) and w_router.shape == (8, h.n) and 1 <= top_k <= 8
+            and knobs.K.moe_fused_router and residual.dtype == norm_w.dtype == w_router.dtype == torch.bfloat16
+            and tuple(h.shape) == tuple(residual.shape) and norm_w.numel() == h.n and residual.is_contiguous() and norm_w.is_contiguous()
+            and w_router.is_contiguous() and h.device == residual.device == norm_w.device == w_router.device
+            and not (residual.data_ptr() | norm_w.data_ptr() | w_router.data_ptr()) % 16):
+        return None
+    y = torch.empty_like(residual)
+    topk_w = torch.empty(h.m, top_k, dtype=torch.float32, device=residual.device)
+    topk_ids = torch.empty(h.m, top_k, dtype=torch.int32, device=residual.device)
+    _ext.kernels().splitk_norm_route(y.data_ptr(), residual.data_ptr(), h.ws.data_ptr(), h.splits, h.m, h.n, norm_w.data_ptr(), float(eps),
+                                     w_router.data_ptr(), 8, top_k, topk_w.data_ptr(), topk_ids.data_ptr(), current_stream())
+    return y, residual, (topk_w, topk_ids)
+
+
 def forward(x: torch.Tensor, w_router: torch.Tensor, w_gate_up: torch.Tensor, w_down: torch.Tensor,
-            top_k: int, expert_offset: int = 0) -> torch.Tensor:
+            top_k: int, expert_offset: int = 0, choice=None, defer: bool = False):
     """``w_gate_up`` / ``w_down`` may hold a contiguous range of the experts (expert parallelism):
     experts ``[expert_offset, expert_offset + w_gate_up.shape[0])`` of the router's E.  Routing is
     always over all E; tokens routed elsewhere contribute zero here, so the expert-parallel
-    group's sum (an all-reduce) is the full MoE output."""
+    group's sum (an all-reduce) is the full MoE output.  ``choice``: :func:`norm_route`'s, made already.  ``defer``: the output may
+    come back as a :class:`Combine`."""
     e_all = w_router.shape[0]
     if not (0 <= expert_offset and expert_offset + w_gate_up.shape[0] <= e_all):
         raise ValueError(f"experts [{expert_offset}, {expert_offset + w_gate_up.shape[0]}) outside the router's {e_all}")
@@ -72,13 +118,15 @@ def forward(x: torch.Tensor, w_router: torch.Tensor, w_gate_up: torch.Tensor, w_
     if not (x.is_contiguous() and w_gate_up.is_contiguous() and w_down.is_contiguous()):
         raise ValueError("moe: operands must be contiguous")
     dev = x.device
-    topk_w = torch.empty(t, top_k, dtype=torch.float32, device=dev)
-    topk_ids = torch.empty(t, top_k, dtype=torch.int32, device=dev)
+    topk_w, topk_ids = choice or (torch.empty(t, top_k, dtype=torch.float32, device=dev),
+                                  torch.empty(t, top_k, dtype=torch.int32, device=dev))
     counts = torch.empty(e, dtype=torch.int32, device=dev)
     offsets = torch.empty(e + 1, dtype=torch.int32, device=dev)
     sorted_tok = torch.empty(t * top_k, dtype=torch.int32, device=dev)
     inv = torch.empty(t * top_k, dtype=torch.int32, device=dev)
-    if knobs.K.moe_fused_router and e in (8, 16) and h % 32 == 0 and x.dtype == w_router.dtype == torch.bfloat16 \
+    if choice:
+        k.moe_scatter(topk_ids.data_ptr(), t, e, top_k, counts.data_ptr(), offsets.data_ptr(), sorted_tok.data_ptr(), inv.data_ptr(), st)
+    elif knobs.K.moe_fused_router and e in (8, 16) and h % 32 == 0 and x.dtype == w_router.dtype == torch.bfloat16 \
             and w_router.is_contiguous():
         # router GEMV + softmax/top-k + scatter in two launches (no [T, E] logits round trip), at
         # decode and prefill T alike
@@ -141,9 +189,8 @@ def forward(x: torch.Tensor, w_router: torch.Tensor, w_gate_up: torch.Tensor, w_
             a, b = off[expert_offset + j], off[expert_offset + j + 1]
             if b > a:
                 ys[a:b] = F.linear(linear_swiglu(xs[a:b], w_gate_up[j]), w_down[j])
-    out = torch.empty_like(x)
-    k.moe_combine(out.data_ptr(), ys.data_ptr(), topk_w.data_ptr(), inv.data_ptr(), t, h, top_k, st)
-    return out
+    out = Combine(ys, topk_w, inv, top_k, x)
+    return out if defer and x.dtype == torch.bfloat16 and h % 8 == 0 and h <= 16384 else out.materialize()
 
 
 # ------------------------------------------------------------------ grouped-choice router, squared-ReLU experts

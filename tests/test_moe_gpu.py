@@ -304,3 +304,60 @@ def test_moe_fp8_prefill_grouped_no_host_sync(cuda):
     tw, tid = ref.moe_route(ref.linear(x, wr).float(), k)
     expect = quant.moe_mlp_ref(x, wgu, wd, tw, tid)
     torch.testing.assert_close(out.float(), expect.float(), atol=3e-2 * expect.abs().max().item(), rtol=5e-2)
+
+
+@pytest.mark.parametrize("t", [1, 2, 7, 64, 129, 200])
+@pytest.mark.parametrize("n,k,s", [(4096, 4096, 8), (4096, 4096, 4), (2048, 2048, 4), (2048, 4096, 8)])
+@pytest.mark.parametrize("top", [1, 2, 8])
+def test_norm_and_choice_in_one_launch(cuda, t, n, k, s, top):
+    """The add + norm of a split product's slabs with the choice of experts behind it: the bits of the two launches."""
+    from distributed_llms_amd import _ext
+    from distributed_llms_amd.ops import gemm
+    x, w, wr = _bf(t, k), _bf(n, k, scale=k ** -0.5), _bf(8, n, scale=n ** -0.5)
+    res, nw = _bf(t, n), _bf(n)
+    r0, r1 = res.clone(), res.clone()
+    part = gemm.linear_wide(x, w, splits=s, defer=True)
+    assert part.splits == s
+    y0, _ = ops.fused_add_rms_norm(part, r0, nw, 1e-5)
+    got = moe.norm_route(part, r1, nw, 1e-5, wr, top)
+    assert got is not None
+    y1, _, (tw, ids) = got
+    tw0, ids0 = torch.empty_like(tw), torch.empty_like(ids)
+    i32 = lambda c: torch.empty(c, dtype=torch.int32, device="cuda")     # noqa: E731
+    c0, o0, s0, v0, c1, o1, s1, v1 = (i32(m) for m in (8, 9, t * top, t * top) * 2)
+    st = torch.cuda.current_stream().cuda_stream
+    _ext.kernels().moe_router_route(y0.data_ptr(), wr.data_ptr(), t, n, 8, top, tw0.data_ptr(), ids0.data_ptr(), c0.data_ptr(), o0.data_ptr(),
+                                    s0.data_ptr(), v0.data_ptr(), st)
+    _ext.kernels().moe_scatter(ids.data_ptr(), t, 8, top, c1.data_ptr(), o1.data_ptr(), s1.data_ptr(), v1.data_ptr(), st)
+    for a, b in ((y0, y1), (r0, r1), (ids0, ids), (tw0, tw), (c0, c1), (o0, o1)):
+        assert torch.equal(a, b)
+    assert torch.equal(s1[v1.long()], torch.arange(t * top, device="cuda", dtype=torch.int32) // top)
+    want = (y0.double() @ wr.double().T).bfloat16().double().softmax(-1).topk(top, -1).values
+    assert (tw.double() - want / want.sum(-1, keepdim=True)).abs().max() <= 2.0 ** -6       # (logits of up to 4 with an ulp of 2^-6)
+
+
+@pytest.mark.parametrize("t", [1, 3, 64, 300])
+@pytest.mark.parametrize("h", [8, 2048, 2056, 4096, 8200, 16384])
+@pytest.mark.parametrize("top", [1, 2, 3, 8])
+def test_combine_and_norm_in_one_launch(cuda, t, h, top):
+    """The weighted sum of the experts' rows in the launch of the add + norm behind it: the bits of the two."""
+    ys, inv = _bf(t * top, h), torch.randperm(t * top, device="cuda").to(torch.int32)
+    tw = torch.rand(t, top, device="cuda")
+    res, nw, like = _bf(t + 1, h), _bf(h), torch.empty(t, h, device="cuda", dtype=torch.bfloat16)
+    c = moe.Combine(ys, tw, inv, top, like)
+    r0, r1 = res.clone(), res.clone()
+    y0, _ = ops.fused_add_rms_norm(c.materialize(), r0[:t], nw, 1e-5)
+    y1, _ = ops.fused_add_rms_norm(c, r1[:t], nw, 1e-5)
+    assert torch.equal(y0, y1) and torch.equal(r0, r1)
+
+
+def test_norm_and_choice_refuse(cuda):
+    """Other slabs, widths and experts keep their launches."""
+    from distributed_llms_amd.ops import gemm
+    nw, res = _bf(4096), _bf(2, 4096)
+    part = gemm.linear_wide(_bf(2, 4096), _bf(4096, 4096), splits=2, defer=True)
+    assert moe.norm_route(part, res, nw, 1e-5, _bf(8, 4096), 2) is None
+    part = gemm.linear_wide(_bf(2, 4096), _bf(4096, 4096), splits=8, defer=True)
+    assert moe.norm_route(part, res, nw, 1e-5, _bf(16, 4096), 2) is None
+    assert moe.norm_route(part.materialize(), res, nw, 1e-5, _bf(8, 4096), 2) is None
+    assert moe.norm_route(part, res, nw, 1e-5, _bf(8, 4096).T.contiguous().T, 2) is None
