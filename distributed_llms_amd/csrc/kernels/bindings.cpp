@@ -20,7 +20,7 @@ PYBIND11_MODULE(_C_kernels, m) {
   m.def("add_inplace", &dllm::add_inplace);
   m.def("moe_route", &dllm::moe_route);
   m.def("moe_grouped_gemm", &dllm::moe_grouped_gemm, py::arg("y"), py::arg("x"), py::arg("gather"), py::arg("w"), py::arg("counts"), py::arg("offsets"), py::arg("experts"), py::arg("n"), py::arg("k"), py::arg("mode"), py::arg("rows_hint"), py::arg("variant"), py::arg("stream"),
-        py::arg("limit") = 0.f);
+        py::arg("limit") = 0.f, py::arg("pairs") = 0, py::arg("top") = 1, py::arg("e0") = 0);
   m.def("splitk_add_rms_norm", &dllm::splitk_add_rms_norm);
   m.def("splitk_reduce", &dllm::splitk_reduce);
   m.def("splitk_reduce_clipped", &dllm::splitk_reduce_clipped);
@@ -42,12 +42,13 @@ PYBIND11_MODULE(_C_kernels, m) {
   m.def("gemm_pf", &dllm::gemm_pf, py::arg("c"), py::arg("a"), py::arg("b"), py::arg("m"), py::arg("n"), py::arg("k"),
         py::arg("mode"), py::arg("variant"), py::arg("stream"), py::arg("limit") = 0.f, py::arg("bm") = 256, py::arg("bias") = 0, py::arg("wgs") = 0);
   m.def("gemm_pf8", &dllm::gemm_pf8);
-  m.def("moe_combine", &dllm::moe_combine);
+  m.def("moe_combine", &dllm::moe_combine, py::arg("out"), py::arg("ysorted"), py::arg("topk_w"), py::arg("inv"), py::arg("tokens"),
+        py::arg("h"), py::arg("k"), py::arg("stream"), py::arg("ids") = (uintptr_t)0);
   m.def("moe_combine_norm", &dllm::moe_combine_norm);
   m.def("moe_scatter", &dllm::moe_scatter);
   m.def("splitk_norm_route", &dllm::splitk_norm_route);
   m.def("moe_wide_gemm", &dllm::moe_wide_gemm, py::arg("y"), py::arg("x"), py::arg("gather"), py::arg("w"), py::arg("counts"), py::arg("offsets"), py::arg("experts"), py::arg("n"), py::arg("k"), py::arg("mode"), py::arg("stream"),
-        py::arg("limit") = 0.f);
+        py::arg("limit") = 0.f, py::arg("pairs") = 0, py::arg("top") = 1, py::arg("e0") = 0);
   m.def("moe_router_route", &dllm::moe_router_route);
   m.def("paged_attention_decode", &dllm::paged_attention_decode);
   m.def("paged_attention_decode_rope", &dllm::paged_attention_decode_rope);

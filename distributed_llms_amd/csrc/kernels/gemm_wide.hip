@@ -37,6 +37,7 @@
 // by the load pipeline with a ~50 %-busy MFMA phase behind it.
 #include "common.h"
 #include "launchers.h"
+#include "moe_top.h"
 
 #include <type_traits>
 
@@ -572,12 +573,13 @@ __global__ void __launch_bounds__(512, 1) gemm_wide_fp8_kernel(const uint8_t* __
 // the decode regime of Mixtral at B >= 128 (32-128 rows per expert), where the weight-streaming
 // grouped kernel (moe.hip) runs its MFMAs at a fraction of the rate.
 // ---------------------------------------------------------------------------------------------
-template <int BM, bool SWIGLU, int VAR, bool FP8 = false, int NBUF = 3, bool CLIPPED = false>
+// PICK: `list` instead of what `gather` points to (MoePick)
+template <int BM, bool SWIGLU, int VAR, bool FP8 = false, int NBUF = 3, bool CLIPPED = false, bool PICK = false>
 __device__ __forceinline__ void moe_wide_rows(bf16* smem, bf16* __restrict__ Y, const bf16* __restrict__ X,
                                               const int* __restrict__ gather, const bf16* __restrict__ We, int cnt,
                                               int off, int N, int K, int n_t, int wv, int lane,
                                               const float* __restrict__ sa = nullptr,
-                                              const float* __restrict__ sb = nullptr, float limit = 0.f) {
+                                              const float* __restrict__ sb = nullptr, float limit = 0.f, int list = 0) {
   // FP8: X / We hold e4m3 bytes addressed in 2-byte units (K / 2 per row); sa: per-slot activation
   // scales (slot order), sb: this expert's per-channel weight scales
   constexpr int AI = BM / 64, BI = 2, RT = BM / 64;
@@ -592,7 +594,11 @@ __device__ __forceinline__ void moe_wide_rows(bf16* smem, bf16* __restrict__ Y, 
     for (int j = 0; j < AI; ++j) {
       const int r = 8 * (wv * AI + j) + (lane >> 3);
       const int slot = off + r0 + min(r, rows - 1);
-      const int src = gather ? gather[slot] : slot;
+      int src = slot;
+      if (gather) {
+        if constexpr (PICK) src = __builtin_amdgcn_ds_bpermute(4 * (r0 + min(r, rows - 1)), list);
+        else src = gather[slot];
+      }
       srcA[j] = X + (size_t)src * KU + wswz(r, lane & 7) * 8;
     }
 #pragma unroll
@@ -621,21 +627,30 @@ constexpr int moe_nbuf() {
   return NBUF_SEL == 0 ? 3 : (BM == 64 ? 6 : 5);
 }
 
-template <bool SWIGLU, bool FP8 = false, int NBUF_SEL = 1, bool CLIPPED = false>
+// PICK: `counts` are the choices of `pairs` (token, choice) pairs, `top` a token, `e0` the first expert's number (moe_pick)
+template <bool SWIGLU, bool FP8 = false, int NBUF_SEL = 1, bool CLIPPED = false, bool PICK = false>
 __global__ void __launch_bounds__(512, 1) moe_wide_kernel(bf16* __restrict__ Y, const bf16* __restrict__ X,
                                                           const int* __restrict__ gather, const bf16* __restrict__ W,
                                                           const int* __restrict__ counts,
                                                           const int* __restrict__ offsets, int N, int K, int nt,
                                                           const float* __restrict__ sa = nullptr,
-                                                          const float* __restrict__ wscale = nullptr, float limit = 0.f) {
+                                                          const float* __restrict__ wscale = nullptr, float limit = 0.f,
+                                                          int pairs = 0, int top = 1, int e0 = 0) {
   static_assert(moe_nbuf<64, NBUF_SEL>() * (64 + WBN) * WBK <= MOE_LDS &&
                 moe_nbuf<128, NBUF_SEL>() * (128 + WBN) * WBK <= MOE_LDS, "LDS");
   __shared__ __attribute__((aligned(16))) bf16 smem[MOE_LDS];
   const int e = blockIdx.y;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  if constexpr (PICK) {
+    const MoePick mp = moe_pick(counts, pairs, top, e0 + e, lane);
+    if (mp.cnt == 0) return;
+    moe_wide_rows<64, SWIGLU, 256 + 2, FP8, moe_nbuf<64, NBUF_SEL>(), CLIPPED, true>(smem, Y, X, gather, W + (size_t)e * N * K, mp.cnt, mp.off, N, K,
+                                                                                     blockIdx.x, wv, lane, nullptr, nullptr, limit, mp.list);
+    return;
+  }
   const int cnt = counts[e];
   if (cnt == 0) return;                       // uniform across the workgroup
   const int off = offsets[e];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const bf16* We = W + (size_t)e * N * (FP8 ? K / 2 : K);
   const float* sb = FP8 ? wscale + (size_t)e * N : nullptr;
   constexpr int NB64 = moe_nbuf<64, NBUF_SEL>(), NB128 = moe_nbuf<128, NBUF_SEL>();
@@ -656,12 +671,13 @@ __global__ void __launch_bounds__(512, 1) moe_wide_kernel(bf16* __restrict__ Y, 
 }
 
 // mode 1 (SwiGLU): W [E, 2I, K] -> Y [slots, I]; mode 0: W [E, N, K] -> Y [slots, N]; mode 3: as 1 with the clipped GLU
-// of `limit`
+// of `limit`.  pairs > 0: `counts` are the choices of that many pairs (moe_wide_kernel's PICK), `gather` says by being there that x holds tokens
 void moe_wide_gemm(uintptr_t y, uintptr_t x, uintptr_t gather, uintptr_t w, uintptr_t counts, uintptr_t offsets,
-                   int E, int N, int K, int mode, uintptr_t stream, float limit) {
+                   int E, int N, int K, int mode, uintptr_t stream, float limit, int pairs, int top, int e0) {
   DLLM_HOST_CHECK(E >= 1, "experts >= 1");
   DLLM_HOST_CHECK(K % WBK == 0, "K must be a multiple of 64");
   DLLM_HOST_CHECK(N % 128 == 0, "N must be a multiple of 128");
+  DLLM_HOST_CHECK(pairs >= 0 && pairs <= kPickPairs && top >= 1 && e0 >= 0 && (pairs == 0 || mode == 0 || mode == 1), "up to 64 pairs, the deep ring");
   // mode bit 2: the 3-slot ring instead of the deep one (A/B runs)
   const bool shallow = (mode & 4) != 0;
   mode &= 3;
@@ -672,11 +688,17 @@ void moe_wide_gemm(uintptr_t y, uintptr_t x, uintptr_t gather, uintptr_t w, uint
 #define DLLM_MOE_GO(SW_, SEL_, CL_)                                                                                   \
   hipLaunchKernelGGL((moe_wide_kernel<SW_, false, SEL_, CL_>), dim3(ntiles, E), dim3(512), 0, s, (bf16*)y,            \
                      (const bf16*)x, (const int*)gather, (const bf16*)w, (const int*)counts, (const int*)offsets, N, \
-                     K, nt, (const float*)nullptr, (const float*)nullptr, limit)
-  if (mode == 3) DLLM_MOE_GO(true, 1, true);
+                     K, nt, (const float*)nullptr, (const float*)nullptr, limit, 0, 1, 0)
+#define DLLM_MOE_PICK(SW_)                                                                                               \
+  hipLaunchKernelGGL((moe_wide_kernel<SW_, false, 1, false, true>), dim3(ntiles, E), dim3(512), 0, s, (bf16*)y, (const bf16*)x, \
+                     (const int*)gather, (const bf16*)w, (const int*)counts, (const int*)nullptr, N, K, nt, (const float*)nullptr, \
+                     (const float*)nullptr, limit, pairs, top, e0)
+  if (pairs > 0) { if (mode == 1) DLLM_MOE_PICK(true); else DLLM_MOE_PICK(false); }
+  else if (mode == 3) DLLM_MOE_GO(true, 1, true);
   else if (mode == 1) { if (shallow) DLLM_MOE_GO(true, 0, false); else DLLM_MOE_GO(true, 1, false); }
   else { if (shallow) DLLM_MOE_GO(false, 0, false); else DLLM_MOE_GO(false, 1, false); }
 #undef DLLM_MOE_GO
+#undef DLLM_MOE_PICK
   DLLM_HIP_CHECK(hipGetLastError());
 }
 
@@ -695,11 +717,11 @@ void moe_wide_gemm_fp8(uintptr_t y, uintptr_t x, uintptr_t gather, uintptr_t w, 
   if (mode == 1)
     hipLaunchKernelGGL((moe_wide_kernel<true, true>), dim3(ntiles, E), dim3(512), 0, s, (bf16*)y, (const bf16*)x,
                        (const int*)gather, (const bf16*)w, (const int*)counts, (const int*)offsets, N, K, nt,
-                       (const float*)sa, (const float*)wscale, 0.f);
+                       (const float*)sa, (const float*)wscale, 0.f, 0, 1, 0);
   else
     hipLaunchKernelGGL((moe_wide_kernel<false, true>), dim3(ntiles, E), dim3(512), 0, s, (bf16*)y, (const bf16*)x,
                        (const int*)gather, (const bf16*)w, (const int*)counts, (const int*)offsets, N, K, nt,
-                       (const float*)sa, (const float*)wscale, 0.f);
+                       (const float*)sa, (const float*)wscale, 0.f, 0, 1, 0);
   DLLM_HIP_CHECK(hipGetLastError());
 }
 

@@ -57,21 +57,21 @@ int gemm_sq(uintptr_t c, uintptr_t a, uintptr_t b, uintptr_t ws, long ws_floats,
 void moe_route(uintptr_t logits, int T, int E, int k, uintptr_t topk_w, uintptr_t topk_ids, uintptr_t counts,
                uintptr_t offsets, uintptr_t sorted_tok, uintptr_t inv, uintptr_t stream);
 void moe_grouped_gemm(uintptr_t y, uintptr_t x, uintptr_t gather, uintptr_t w, uintptr_t counts, uintptr_t offsets,
-                      int E, int N, int K, int mode, int rows_hint, int variant, uintptr_t stream, float limit);
+                      int E, int N, int K, int mode, int rows_hint, int variant, uintptr_t stream, float limit, int pairs, int top, int e0);
 void moe_router_route(uintptr_t x, uintptr_t w, int T, int H, int E, int k, uintptr_t topk_w, uintptr_t topk_ids,
                       uintptr_t counts, uintptr_t offsets, uintptr_t sorted_tok, uintptr_t inv, uintptr_t stream);
 void moe_wide_gemm(uintptr_t y, uintptr_t x, uintptr_t gather, uintptr_t w, uintptr_t counts, uintptr_t offsets,
-                   int E, int N, int K, int mode, uintptr_t stream, float limit);
+                   int E, int N, int K, int mode, uintptr_t stream, float limit, int pairs, int top, int e0);
 void moe_wide_gemm_fp8(uintptr_t y, uintptr_t x, uintptr_t gather, uintptr_t w, uintptr_t counts, uintptr_t offsets,
                        int E, int N, int K, int mode, uintptr_t sa, uintptr_t wscale, uintptr_t stream);
 void moe_scatter(uintptr_t topk_ids, int T, int E, int k, uintptr_t counts, uintptr_t offsets, uintptr_t sorted_tok, uintptr_t inv,
                  uintptr_t stream);
-void moe_combine_norm(uintptr_t y, uintptr_t residual, uintptr_t ysorted, uintptr_t topk_w, uintptr_t inv, uintptr_t w, int T, int H, int k,
-                      float eps, uintptr_t stream);
+void moe_combine_norm(uintptr_t y, uintptr_t residual, uintptr_t ysorted, uintptr_t topk_w, uintptr_t inv, uintptr_t ids, uintptr_t w, int T, int H,
+                      int k, float eps, uintptr_t stream);
 void splitk_norm_route(uintptr_t y, uintptr_t residual, uintptr_t ws, int S, int M, int N, uintptr_t w, float eps, uintptr_t router, int E,
                        int k, uintptr_t topk_w, uintptr_t topk_ids, uintptr_t stream);
 void moe_combine(uintptr_t out, uintptr_t ysorted, uintptr_t topk_w, uintptr_t inv, int T, int H, int k,
-                 uintptr_t stream);
+                 uintptr_t stream, uintptr_t ids);
 
 void paged_attention_decode(uintptr_t out, uintptr_t q, uintptr_t k_cache, uintptr_t v_cache,
                             uintptr_t block_tables, uintptr_t seq_lens, uintptr_t part_o, uintptr_t part_ml,

@@ -155,10 +155,11 @@ constexpr int MOE_EPI_RELU2 = 2;          // store max(v, 0)^2: the activation o
 
 // Rows [0, cnt) of one expert in chunks of MT*16 rows; every chunk streams the WG's W column
 // tile once (K split over the WAVES waves, partial tiles summed through LDS).
-template <int MT, int NT, int WAVES, int EPI>
+// PICK: `list` instead of what `gather` points to (MoePick)
+template <int MT, int NT, int WAVES, int EPI, bool PICK = false>
 __device__ __forceinline__ void moe_rows(float* red, bf16* __restrict__ y, const bf16* __restrict__ x,
                                          const int* __restrict__ gather, const bf16* const (&wrow)[NT], int cnt,
-                                         int off, int K, int ldy, int g0, int g1, int lane, float limit) {
+                                         int off, int K, int ldy, int g0, int g1, int lane, float limit, int list = 0) {
   constexpr int BM = MT * 16, BN = NT * 16, NTHR = WAVES * 64;
   const int r = lane & 15, g = lane >> 4;
   for (int r0 = 0; r0 < cnt; r0 += BM) {
@@ -168,7 +169,11 @@ __device__ __forceinline__ void moe_rows(float* red, bf16* __restrict__ y, const
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       const int slot = off + r0 + min(mt * 16 + r, rows - 1);
-      const int src = gather ? gather[slot] : slot;
+      int src = slot;
+      if (gather) {
+        if constexpr (PICK) src = __builtin_amdgcn_ds_bpermute(4 * (r0 + min(mt * 16 + r, rows - 1)), list);
+        else src = gather[slot];
+      }
       xrow[mt] = x + (size_t)src * K + 8 * g;
     }
     f32x4 acc[MT][NT];
@@ -199,20 +204,24 @@ __device__ __forceinline__ void moe_rows(float* red, bf16* __restrict__ y, const
 // actual count (a workgroup-uniform branch): 16-row tiles for <= 16 rows, 32 for <= 32, else
 // MTMAX*16-row chunks -- so routing imbalance never makes an expert re-stream its weights
 // while it fits one chunk, and a decode expert with 10 rows does not gather 64.
-template <int MTMAX, int NT, int WAVES, int EPI>
+// PICK: as moe_wide_kernel's
+template <int MTMAX, int NT, int WAVES, int EPI, bool PICK = false>
 __global__ void __launch_bounds__(WAVES * 64, 1) moe_grouped_kernel(bf16* __restrict__ y, const bf16* __restrict__ x,
                                                                     const int* __restrict__ gather,
                                                                     const bf16* __restrict__ w,
                                                                     const int* __restrict__ counts,
                                                                     const int* __restrict__ offsets, int N, int K,
-                                                                    int ldy, float limit) {
+                                                                    int ldy, float limit, int pairs, int top, int e0) {
   constexpr int BN = NT * 16;
   __shared__ __attribute__((aligned(16))) float red[MTMAX * 16 * BN];
   const int e = blockIdx.y;
-  const int cnt = counts[e];
-  if (cnt == 0) return;                       // uniform across the workgroup
-  const int off = offsets[e];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  MoePick mp{0, 0, 0};
+  if constexpr (PICK) mp = moe_pick(counts, pairs, top, e0 + e, lane);
+  else mp.cnt = counts[e];
+  const int cnt = mp.cnt;
+  if (cnt == 0) return;                       // uniform across the workgroup
+  const int off = PICK ? mp.off : offsets[e];
   const int r = lane & 15, g = lane >> 4;
   const bf16* we = w + (size_t)e * N * K;
   const bf16* wrow[NT];
@@ -227,29 +236,31 @@ __global__ void __launch_bounds__(WAVES * 64, 1) moe_grouped_kernel(bf16* __rest
   const int per = (ngroups + WAVES - 1) / WAVES;
   const int g0 = wv * per, g1 = min(ngroups, g0 + per);
   if (MTMAX == 1 || cnt <= 16) {
-    moe_rows<1, NT, WAVES, EPI>(red, y, x, gather, wrow, cnt, off, K, ldy, g0, g1, lane, limit);
+    moe_rows<1, NT, WAVES, EPI, PICK>(red, y, x, gather, wrow, cnt, off, K, ldy, g0, g1, lane, limit, mp.list);
   } else if constexpr (MTMAX >= 2) {
-    if (MTMAX == 2 || cnt <= 32) moe_rows<2, NT, WAVES, EPI>(red, y, x, gather, wrow, cnt, off, K, ldy, g0, g1, lane, limit);
-    else if constexpr (MTMAX >= 4) moe_rows<4, NT, WAVES, EPI>(red, y, x, gather, wrow, cnt, off, K, ldy, g0, g1, lane, limit);
+    if (MTMAX == 2 || cnt <= 32) moe_rows<2, NT, WAVES, EPI, PICK>(red, y, x, gather, wrow, cnt, off, K, ldy, g0, g1, lane, limit, mp.list);
+    else if constexpr (MTMAX >= 4) moe_rows<4, NT, WAVES, EPI, PICK>(red, y, x, gather, wrow, cnt, off, K, ldy, g0, g1, lane, limit, mp.list);
   }
 }
 
+// ids: the choices of up to 64 pairs (moe_slot) in place of inv
 __global__ void __launch_bounds__(256) moe_combine_kernel(bf16* __restrict__ out, const bf16* __restrict__ ysorted,
                                                           const float* __restrict__ topk_w,
-                                                          const int* __restrict__ inv, int H, int k) {
-  const int t = blockIdx.x;
-  for (int v = threadIdx.x; v < (H >> 3); v += 256) {
+                                                          const int* __restrict__ inv, const int* __restrict__ ids, int H, int k) {
+  const int t = blockIdx.x, id = ids ? moe_pair(ids, gridDim.x * k, threadIdx.x & 63) : 0;
+  for (int v0 = 0; v0 < (H >> 3); v0 += 256) {         // (whole waves: moe_slot votes)
+    const int v = v0 + threadIdx.x, vc = min(v, (H >> 3) - 1);
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     for (int j = 0; j < k; ++j) {
       const float wj = topk_w[t * k + j];
-      const bf16x8 yv = *reinterpret_cast<const bf16x8*>(ysorted + (size_t)inv[t * k + j] * H + v * 8);
+      const bf16x8 yv = *reinterpret_cast<const bf16x8*>(ysorted + (size_t)(ids ? moe_slot(id, t * k + j) : inv[t * k + j]) * H + vc * 8);
 #pragma unroll
       for (int i = 0; i < 8; ++i) acc[i] += wj * bf2f(yv[i]);
     }
     bf16x8 o;
 #pragma unroll
     for (int i = 0; i < 8; ++i) o[i] = f2bf(acc[i]);
-    *reinterpret_cast<bf16x8*>(out + (size_t)t * H + v * 8) = o;
+    if (v == vc) *reinterpret_cast<bf16x8*>(out + (size_t)t * H + v * 8) = o;
   }
 }
 
@@ -260,10 +271,12 @@ __global__ void __launch_bounds__(256) moe_combine_kernel(bf16* __restrict__ out
 template <int MAXV>
 __global__ void __launch_bounds__(256) moe_combine_norm_kernel(bf16* __restrict__ y, bf16* __restrict__ residual,
                                                                const bf16* __restrict__ ysorted, const float* __restrict__ topk_w,
-                                                               const int* __restrict__ inv_slot, const bf16* __restrict__ w, int H, int k,
-                                                               float eps) {
+                                                               const int* __restrict__ inv_slot, const int* __restrict__ ids,
+                                                               const bf16* __restrict__ w, int H, int k, float eps) {
   __shared__ float red[16];
   const int t = blockIdx.x, nvec = H >> 3;
+  const int id = ids ? moe_pair(ids, gridDim.x * k, threadIdx.x & 63) : 0;
+  auto slot = [&](int j) { return ids ? moe_slot(id, t * k + j) : inv_slot[t * k + j]; };
   bf16x8* rr = reinterpret_cast<bf16x8*>(residual + (size_t)t * H);
   bf16x8 b[MAXV], g[MAXV], a[MAXV];
   float v[MAXV][8];
@@ -278,8 +291,8 @@ __global__ void __launch_bounds__(256) moe_combine_norm_kernel(bf16* __restrict_
   for (int j = 0; j < k; j += 2) {                       // two experts' rows under way
     const int j1 = min(j + 1, k - 1);
     const float w0 = topk_w[t * k + j], w1 = topk_w[t * k + j1];
-    const bf16x8* y0 = reinterpret_cast<const bf16x8*>(ysorted + (size_t)inv_slot[t * k + j] * H);
-    const bf16x8* y1 = reinterpret_cast<const bf16x8*>(ysorted + (size_t)inv_slot[t * k + j1] * H);
+    const bf16x8* y0 = reinterpret_cast<const bf16x8*>(ysorted + (size_t)slot(j) * H);
+    const bf16x8* y1 = reinterpret_cast<const bf16x8*>(ysorted + (size_t)slot(j1) * H);
     bf16x8 e0[MAXV], e1[MAXV];
 #pragma unroll
     for (int i = 0; i < MAXV; ++i) {
@@ -369,16 +382,17 @@ void moe_scatter(uintptr_t topk_ids, int T, int E, int k, uintptr_t counts, uint
   DLLM_HIP_CHECK(hipGetLastError());
 }
 
-// y [T, H], residual [T, H] (updated), ysorted [T k, H], topk_w / inv [T, k], w [H]
-void moe_combine_norm(uintptr_t y, uintptr_t residual, uintptr_t ysorted, uintptr_t topk_w, uintptr_t inv, uintptr_t w, int T, int H, int k,
-                      float eps, uintptr_t stream) {
+// y [T, H], residual [T, H] (updated), ysorted [T k, H], topk_w / inv or ids [T, k], w [H]
+void moe_combine_norm(uintptr_t y, uintptr_t residual, uintptr_t ysorted, uintptr_t topk_w, uintptr_t inv, uintptr_t ids, uintptr_t w, int T, int H,
+                      int k, float eps, uintptr_t stream) {
   DLLM_HOST_CHECK(H % 8 == 0 && H > 0 && H <= 8 * 256 * 8, "hidden must be a multiple of 8 and <= 16384");
   DLLM_HOST_CHECK(T >= 0 && k >= 1 && k <= 8, "1 <= top_k <= 8");
+  DLLM_HOST_CHECK(inv != 0 || (ids != 0 && (long)T * k <= kPickPairs), "slots, or the choices of up to 64 pairs");
   DLLM_HOST_CHECK((y | residual | ysorted | w) % 16 == 0, "alignment");
   if (T == 0) return;
   auto go = [&](auto kern) {
     hipLaunchKernelGGL(kern, dim3(T), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), (bf16*)y, (bf16*)residual, (const bf16*)ysorted,
-                       (const float*)topk_w, (const int*)inv, (const bf16*)w, H, k, eps);
+                       (const float*)topk_w, (const int*)inv, (const int*)ids, (const bf16*)w, H, k, eps);
   };
   const int nvec = H / 8;
   if (nvec <= 256) go(moe_combine_norm_kernel<1>);
@@ -395,19 +409,19 @@ static void launch_grouped(hipStream_t s, bf16* y, const bf16* x, const int* gat
   if (mode == 1) {
     DLLM_HOST_CHECK(N % BN == 0, "moe grouped: 2I must be a multiple of the column tile");
     hipLaunchKernelGGL((moe_grouped_kernel<MTMAX, NT, WAVES, MOE_EPI_SWIGLU>), dim3(N / BN, E), dim3(WAVES * 64), 0,
-                       s, y, x, gather, w, counts, offsets, N, K, N / 2, 0.f);
+                       s, y, x, gather, w, counts, offsets, N, K, N / 2, 0.f, 0, 1, 0);
   } else if (mode == 3) {
     DLLM_HOST_CHECK(N % BN == 0, "moe grouped: 2I must be a multiple of the column tile");
     hipLaunchKernelGGL((moe_grouped_kernel<MTMAX, NT, WAVES, MOE_EPI_CLIPPED>), dim3(N / BN, E), dim3(WAVES * 64), 0,
-                       s, y, x, gather, w, counts, offsets, N, K, N / 2, limit);
+                       s, y, x, gather, w, counts, offsets, N, K, N / 2, limit, 0, 1, 0);
   } else if (mode == 2) {
     DLLM_HOST_CHECK(N % BN == 0, "moe grouped: N must be a multiple of the column tile");
     hipLaunchKernelGGL((moe_grouped_kernel<MTMAX, NT, WAVES, MOE_EPI_RELU2>), dim3(N / BN, E), dim3(WAVES * 64), 0, s,
-                       y, x, gather, w, counts, offsets, N, K, N, 0.f);
+                       y, x, gather, w, counts, offsets, N, K, N, 0.f, 0, 1, 0);
   } else {
     DLLM_HOST_CHECK(N % BN == 0, "moe grouped: N must be a multiple of the column tile");
     hipLaunchKernelGGL((moe_grouped_kernel<MTMAX, NT, WAVES, MOE_EPI_STORE>), dim3(N / BN, E), dim3(WAVES * 64), 0, s,
-                       y, x, gather, w, counts, offsets, N, K, N, 0.f);
+                       y, x, gather, w, counts, offsets, N, K, N, 0.f, 0, 1, 0);
   }
 }
 
@@ -416,10 +430,22 @@ static void launch_grouped(hipStream_t s, bf16* y, const bf16* x, const int* gat
 // rows_hint = expected rows per expert (T*k/E) picks the kernel family; variant > 0 forces one
 // (benchmarking: 1 = <1,4,8>, 2 = <2,4,8>, 3 = <4,2,8>, 4 = <2,4,4>, 5 = <4,4,4>, 6 = <2,2,8>).
 void moe_grouped_gemm(uintptr_t y, uintptr_t x, uintptr_t gather, uintptr_t w, uintptr_t counts, uintptr_t offsets,
-                      int E, int N, int K, int mode, int rows_hint, int variant, uintptr_t stream, float limit) {
+                      int E, int N, int K, int mode, int rows_hint, int variant, uintptr_t stream, float limit, int pairs, int top, int e0) {
   DLLM_HOST_CHECK(K % 128 == 0, "K % 128");
   DLLM_HOST_CHECK(N % 64 == 0, "N % 64");   // every column tile (32 or 64) divides N
+  DLLM_HOST_CHECK(pairs >= 0 && pairs <= kPickPairs && top >= 1 && e0 >= 0, "up to 64 pairs");
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  if (pairs > 0) {          // (`counts`: the choices; variant 5's tile)
+    DLLM_HOST_CHECK(mode == 0 || mode == 1, "mode");
+    auto go = [&](auto kern, int ldy) {
+      hipLaunchKernelGGL(kern, dim3(N / 64, E), dim3(256), 0, s, (bf16*)y, (const bf16*)x, (const int*)gather, (const bf16*)w, (const int*)counts,
+                         (const int*)nullptr, N, K, ldy, 0.f, pairs, top, e0);
+    };
+    if (mode == 1) go(moe_grouped_kernel<4, 4, 4, MOE_EPI_SWIGLU, true>, N / 2);
+    else go(moe_grouped_kernel<4, 4, 4, MOE_EPI_STORE, true>, N);
+    DLLM_HIP_CHECK(hipGetLastError());
+    return;
+  }
   auto args = [&](auto f) {
     f(s, (bf16*)y, (const bf16*)x, (const int*)gather, (const bf16*)w, (const int*)counts, (const int*)offsets, E, N,
       K, mode, limit);
@@ -442,11 +468,12 @@ void moe_grouped_gemm(uintptr_t y, uintptr_t x, uintptr_t gather, uintptr_t w, u
 }
 
 void moe_combine(uintptr_t out, uintptr_t ysorted, uintptr_t topk_w, uintptr_t inv, int T, int H, int k,
-                 uintptr_t stream) {
+                 uintptr_t stream, uintptr_t ids) {
   DLLM_HOST_CHECK(H % 8 == 0, "H % 8");
+  DLLM_HOST_CHECK(ids == 0 || (long)T * k <= kPickPairs, "the choices of up to 64 pairs");
   if (T == 0) return;
   hipLaunchKernelGGL(moe_combine_kernel, dim3(T), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), (bf16*)out,
-                     (const bf16*)ysorted, (const float*)topk_w, (const int*)inv, H, k);
+                     (const bf16*)ysorted, (const float*)topk_w, (const int*)inv, (const int*)ids, H, k);
   DLLM_HIP_CHECK(hipGetLastError());
 }
 

@@ -24,6 +24,7 @@ from .. import _ext, knobs
 from . import reference as ref
 from .stream import current_stream
 
+PICK_PAIRS = 64               # (csrc/kernels/moe_top.h: a pair per lane)
 GROUPED_MAX_TOKENS = 256      # beyond this the per-expert row count makes library GEMMs cheaper
 ROUTER_FUSED_MAX_TOKENS = 64  # up to this many tokens the grouped-choice router product runs inside the selection kernel
 # knobs.moe_variant: 0 = pick by expected rows per expert; 1..6 force a kernel variant
@@ -45,27 +46,27 @@ def mlp(x, w_gate_up, w_down, topk_w, topk_ids):
 
 class Combine:
     """A mixture's output whose experts' rows are not summed yet (``forward(..., defer=True)``): for ``ops.fused_add_rms_norm``, which sums them
-    in its launch, or :meth:`materialize`."""
+    in its launch, or :meth:`materialize`.  ``inv``: the slot of every (token, choice) pair; or None and ``ids``: the choices, of up to 64 pairs."""
 
-    __slots__ = ("ys", "topk_w", "inv", "top_k", "shape", "dtype", "device")
+    __slots__ = ("ys", "topk_w", "inv", "ids", "top_k", "shape", "dtype", "device")
 
-    def __init__(self, ys, topk_w, inv, top_k, like):
-        self.ys, self.topk_w, self.inv, self.top_k = ys, topk_w, inv, top_k
+    def __init__(self, ys, topk_w, inv, top_k, like, ids=None):
+        self.ys, self.topk_w, self.inv, self.ids, self.top_k = ys, topk_w, inv, ids, top_k
         self.shape, self.dtype, self.device = like.shape, like.dtype, like.device
 
     def materialize(self) -> torch.Tensor:
         t, h = self.shape
         out = torch.empty(t, h, dtype=self.dtype, device=self.device)
-        _ext.kernels().moe_combine(out.data_ptr(), self.ys.data_ptr(), self.topk_w.data_ptr(), self.inv.data_ptr(), t, h, self.top_k,
-                                   current_stream())
+        _ext.kernels().moe_combine(out.data_ptr(), self.ys.data_ptr(), self.topk_w.data_ptr(), 0 if self.inv is None else self.inv.data_ptr(), t, h,
+                                   self.top_k, current_stream(), 0 if self.inv is not None else self.ids.data_ptr())
         return out
 
     def add_norm(self, residual: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
         """residual <- residual + output; rms_norm(residual) * w."""
         t, h = self.shape
         y = torch.empty_like(residual)
-        _ext.kernels().moe_combine_norm(y.data_ptr(), residual.data_ptr(), self.ys.data_ptr(), self.topk_w.data_ptr(), self.inv.data_ptr(),
-                                        w.data_ptr(), t, h, self.top_k, float(eps), current_stream())
+        _ext.kernels().moe_combine_norm(y.data_ptr(), residual.data_ptr(), self.ys.data_ptr(), self.topk_w.data_ptr(),
+                                        0 if self.inv is None else self.inv.data_ptr(), 0 if self.inv is not None else self.ids.data_ptr(), w.data_ptr(), t, h, self.top_k, float(eps), current_stream())
         return y
 
 
@@ -120,6 +121,22 @@ def forward(x: torch.Tensor, w_router: torch.Tensor, w_gate_up: torch.Tensor, w_
     dev = x.device
     topk_w, topk_ids = choice or (torch.empty(t, top_k, dtype=torch.float32, device=dev),
                                   torch.empty(t, top_k, dtype=torch.int32, device=dev))
+    # few pairs whose choice is there: the experts' launches find their rows themselves (moe_top.h), no launch for counts and slots
+    wide = 0 < knobs.K.moe_wide_min_pairs <= t * top_k and x.dtype == torch.bfloat16 and two_i % 128 == 0 and h % 128 == 0 \
+        and h % 64 == 0 and inter % 64 == 0
+    if choice and not fp8 and t * top_k <= PICK_PAIRS and t <= GROUPED_MAX_TOKENS and knobs.K.moe_deep_ring and knobs.K.moe_variant <= 0 \
+            and (wide or (two_i % 64 == 0 and h % 128 == 0 and inter % 128 == 0)):
+        ys = (torch.zeros if ep else torch.empty)(t * top_k, h, dtype=x.dtype, device=dev)
+        act = torch.empty(t * top_k, inter, dtype=x.dtype, device=dev)
+        ids, pick = topk_ids.data_ptr(), (0.0, t * top_k, top_k, expert_offset)
+        if wide:
+            k.moe_wide_gemm(act.data_ptr(), x.data_ptr(), ids, w_gate_up.data_ptr(), ids, 0, e_loc, two_i, h, 1, st, *pick)
+            k.moe_wide_gemm(ys.data_ptr(), act.data_ptr(), 0, w_down.data_ptr(), ids, 0, e_loc, h, inter, 0, st, *pick)
+        else:
+            k.moe_grouped_gemm(act.data_ptr(), x.data_ptr(), ids, w_gate_up.data_ptr(), ids, 0, e_loc, two_i, h, 1, 0, 0, st, *pick)
+            k.moe_grouped_gemm(ys.data_ptr(), act.data_ptr(), 0, w_down.data_ptr(), ids, 0, e_loc, h, inter, 0, 0, 0, st, *pick)
+        out = Combine(ys, topk_w, None, top_k, x, topk_ids)
+        return out if defer else out.materialize()
     counts = torch.empty(e, dtype=torch.int32, device=dev)
     offsets = torch.empty(e + 1, dtype=torch.int32, device=dev)
     sorted_tok = torch.empty(t * top_k, dtype=torch.int32, device=dev)
@@ -159,8 +176,7 @@ def forward(x: torch.Tensor, w_router: torch.Tensor, w_gate_up: torch.Tensor, w_
     elif t <= GROUPED_MAX_TOKENS:
         act = torch.empty(t * top_k, inter, dtype=x.dtype, device=dev)
         rows = -(-t * top_k // e)        # expected rows per expert picks the kernel's row tile
-        if 0 < knobs.K.moe_wide_min_pairs <= t * top_k and x.dtype == torch.bfloat16 and two_i % 128 == 0 and h % 128 == 0 \
-                and h % 64 == 0 and inter % 64 == 0:
+        if wide:
             ring = 0 if knobs.K.moe_deep_ring else 4          # mode bit 2: the 3-slot LDS ring
             k.moe_wide_gemm(act.data_ptr(), x.data_ptr(), sorted_tok.data_ptr(), w_gate_up.data_ptr(),
                             cnt_p, off_p, e_loc, two_i, h, 1 | ring, st)

@@ -361,3 +361,34 @@ def test_norm_and_choice_refuse(cuda):
     assert moe.norm_route(part, res, nw, 1e-5, _bf(16, 4096), 2) is None
     assert moe.norm_route(part.materialize(), res, nw, 1e-5, _bf(8, 4096), 2) is None
     assert moe.norm_route(part, res, nw, 1e-5, _bf(8, 4096).T.contiguous().T, 2) is None
+
+
+@pytest.mark.parametrize("t,top", [(1, 1), (1, 2), (3, 2), (4, 2), (7, 8), (8, 8), (21, 3), (32, 2), (64, 1)])
+@pytest.mark.parametrize("skew", [False, True])
+@pytest.mark.parametrize("first,local", [(0, 8), (2, 4)])
+def test_experts_find_few_rows_themselves(cuda, t, top, skew, first, local):
+    """Up to 64 pairs of a choice that is there: the bits of the launches behind counts and slot lists (all experts, or a range of them)."""
+    h, i = 256, 256
+    x, gu, dn = _bf(t, h), _bf(8, 2 * i, h, scale=0.05), _bf(8, h, i, scale=0.05)
+    wr = _bf(8, h, scale=0.1)
+    ids = torch.stack([torch.randperm(8, device="cuda")[:top] for _ in range(t)]).to(torch.int32)
+    if skew:
+        ids[:] = torch.arange(8, device="cuda", dtype=torch.int32).flip(0)[:top]
+    tw = torch.rand(t, top, device="cuda")
+    gu, dn = gu[first:first + local].contiguous(), dn[first:first + local].contiguous()
+    res, nw = _bf(t, h), _bf(h)
+    out = moe.forward(x, wr, gu, dn, top, first, choice=(tw, ids))
+    part = moe.forward(x, wr, gu, dn, top, first, choice=(tw, ids), defer=True)
+    assert part.inv is None
+    pairs, moe.PICK_PAIRS = moe.PICK_PAIRS, 0
+    try:
+        want = moe.forward(x, wr, gu, dn, top, first, choice=(tw, ids))
+    finally:
+        moe.PICK_PAIRS = pairs
+    assert torch.equal(out, want)
+    r0, r1 = res.clone(), res.clone()
+    assert torch.equal(ops.fused_add_rms_norm(part, r0, nw, 1e-5)[0], ops.fused_add_rms_norm(want, r1, nw, 1e-5)[0]) and torch.equal(r0, r1)
+    local_ids = ids - first
+    mine = (local_ids >= 0) & (local_ids < local)
+    ref_out = ref.moe_mlp(x.float(), gu.float(), dn.float(), tw * mine, local_ids.clamp(0, local - 1))
+    torch.testing.assert_close(out.float(), ref_out, atol=3e-2, rtol=3e-2)
