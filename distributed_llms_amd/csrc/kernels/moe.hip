@@ -435,14 +435,17 @@ void moe_grouped_gemm(uintptr_t y, uintptr_t x, uintptr_t gather, uintptr_t w, u
   DLLM_HOST_CHECK(N % 64 == 0, "N % 64");   // every column tile (32 or 64) divides N
   DLLM_HOST_CHECK(pairs >= 0 && pairs <= kPickPairs && top >= 1 && e0 >= 0, "up to 64 pairs");
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (pairs > 0) {          // (`counts`: the choices; variant 5's tile)
+  if (pairs > 0) {          // (`counts`: the choices)
     DLLM_HOST_CHECK(mode == 0 || mode == 1, "mode");
-    auto go = [&](auto kern, int ldy) {
-      hipLaunchKernelGGL(kern, dim3(N / 64, E), dim3(256), 0, s, (bf16*)y, (const bf16*)x, (const int*)gather, (const bf16*)w, (const int*)counts,
-                         (const int*)nullptr, N, K, ldy, 0.f, pairs, top, e0);
+    auto go = [&](auto kern, int bn, int threads, int ldy) {
+      hipLaunchKernelGGL(kern, dim3(N / bn, E), dim3(threads), 0, s, (bf16*)y, (const bf16*)x, (const int*)gather, (const bf16*)w,
+                         (const int*)counts, (const int*)nullptr, N, K, ldy, 0.f, pairs, top, e0);
     };
-    if (mode == 1) go(moe_grouped_kernel<4, 4, 4, MOE_EPI_SWIGLU, true>, N / 2);
-    else go(moe_grouped_kernel<4, 4, 4, MOE_EPI_STORE, true>, N);
+    // variant 5's tile; one or two pairs of a product of few columns in tiles of 32, with K over eight waves, so that two experts' tiles are a
+    // workgroup per CU: 4096 x 14336 of two experts 79.5 -> 48.2 us (of three 85.0, here 92.3)
+    if (mode == 1) go(moe_grouped_kernel<4, 4, 4, MOE_EPI_SWIGLU, true>, 64, 256, N / 2);
+    else if (pairs <= 2) go(moe_grouped_kernel<1, 2, 8, MOE_EPI_STORE, true>, 32, 512, N);
+    else go(moe_grouped_kernel<4, 4, 4, MOE_EPI_STORE, true>, 64, 256, N);
     DLLM_HIP_CHECK(hipGetLastError());
     return;
   }

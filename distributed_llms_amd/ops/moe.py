@@ -129,11 +129,19 @@ def forward(x: torch.Tensor, w_router: torch.Tensor, w_gate_up: torch.Tensor, w_
         ys = (torch.zeros if ep else torch.empty)(t * top_k, h, dtype=x.dtype, device=dev)
         act = torch.empty(t * top_k, inter, dtype=x.dtype, device=dev)
         ids, pick = topk_ids.data_ptr(), (0.0, t * top_k, top_k, expert_offset)
+        # Fewer pairs than the line take the tiled kernel all the same where its workgroups of gate|up are a round of the CUs, and one or two the other
+        # one for the down projection, whose tiles of 32 columns are.  us, gate|up / down of 8 experts of 4096 and 14336, two a token, tiled / other
+        # kernel: one token 76 / 83, 98 / 48; two with three experts 111 / 86, 144 / 85; three with four 147 / 91, 174 / 90, with six 223 / 108,
+        # 264 / 164.
+        wide = wide or (0 < knobs.K.moe_wide_min_pairs and two_i % 128 == 0 and h % 128 == 0 and inter % 128 == 0
+                        and two_i // 128 * min(t * top_k, e_loc) >= 256)
         if wide:
             k.moe_wide_gemm(act.data_ptr(), x.data_ptr(), ids, w_gate_up.data_ptr(), ids, 0, e_loc, two_i, h, 1, st, *pick)
-            k.moe_wide_gemm(ys.data_ptr(), act.data_ptr(), 0, w_down.data_ptr(), ids, 0, e_loc, h, inter, 0, st, *pick)
         else:
             k.moe_grouped_gemm(act.data_ptr(), x.data_ptr(), ids, w_gate_up.data_ptr(), ids, 0, e_loc, two_i, h, 1, 0, 0, st, *pick)
+        if wide and not (t * top_k <= 2 and inter % 128 == 0):
+            k.moe_wide_gemm(ys.data_ptr(), act.data_ptr(), 0, w_down.data_ptr(), ids, 0, e_loc, h, inter, 0, st, *pick)
+        else:
             k.moe_grouped_gemm(ys.data_ptr(), act.data_ptr(), 0, w_down.data_ptr(), ids, 0, e_loc, h, inter, 0, 0, 0, st, *pick)
         out = Combine(ys, topk_w, None, top_k, x, topk_ids)
         return out if defer else out.materialize()

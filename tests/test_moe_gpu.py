@@ -385,10 +385,28 @@ def test_experts_find_few_rows_themselves(cuda, t, top, skew, first, local):
         want = moe.forward(x, wr, gu, dn, top, first, choice=(tw, ids))
     finally:
         moe.PICK_PAIRS = pairs
-    assert torch.equal(out, want)
+    if t * top > 2:
+        assert torch.equal(out, want)
     r0, r1 = res.clone(), res.clone()
-    assert torch.equal(ops.fused_add_rms_norm(part, r0, nw, 1e-5)[0], ops.fused_add_rms_norm(want, r1, nw, 1e-5)[0]) and torch.equal(r0, r1)
+    assert torch.equal(ops.fused_add_rms_norm(part, r0, nw, 1e-5)[0], ops.fused_add_rms_norm(out, r1, nw, 1e-5)[0]) and torch.equal(r0, r1)
     local_ids = ids - first
     mine = (local_ids >= 0) & (local_ids < local)
     ref_out = ref.moe_mlp(x.float(), gu.float(), dn.float(), tw * mine, local_ids.clamp(0, local - 1))
     torch.testing.assert_close(out.float(), ref_out, atol=3e-2, rtol=3e-2)
+
+
+@pytest.mark.parametrize("t,top", [(1, 1), (1, 2), (2, 2), (3, 2)])
+def test_few_pairs_of_large_experts(cuda, t, top):
+    """Fewer pairs than the tiled kernel's line, on it where its workgroups fill the CUs; the down projection of one or two in narrow tiles. """
+    h, i = 256, 16384
+    x, gu, dn = _bf(t, h), _bf(8, 2 * i, h, scale=h ** -0.5), _bf(8, h, i, scale=i ** -0.5)
+    ids = torch.stack([torch.randperm(8, device="cuda")[:top] for _ in range(t)]).to(torch.int32)
+    tw = torch.rand(t, top, device="cuda")
+    out = moe.forward(x, _bf(8, h), gu, dn, top, choice=(tw, ids))
+    want = torch.zeros(t, h, device="cuda", dtype=torch.float64)
+    for a in range(t):
+        for j in range(top):
+            z = gu[ids[a, j].item()].double() @ x[a].double()
+            want[a] += tw[a, j].double() * (dn[ids[a, j].item()].double() @ (F.silu(z[:i]) * z[i:]))
+    # 2^-9 for each of the activation, the expert's row and the result, rounded to bf16
+    assert (out.double() - want).norm() <= 3 * 2.0 ** -9 * want.norm()
