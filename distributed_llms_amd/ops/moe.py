@@ -119,6 +119,9 @@ def forward(x: torch.Tensor, w_router: torch.Tensor, w_gate_up: torch.Tensor, w_
     if not (x.is_contiguous() and w_gate_up.is_contiguous() and w_down.is_contiguous()):
         raise ValueError("moe: operands must be contiguous")
     dev = x.device
+    if choice and not all(c.shape == (t, top_k) and c.dtype == d and c.is_contiguous() and c.device == dev
+                          for c, d in zip(choice, (torch.float32, torch.int32))):
+        raise ValueError("moe: choice is ([T, top_k] float32 weights, [T, top_k] int32 experts)")
     topk_w, topk_ids = choice or (torch.empty(t, top_k, dtype=torch.float32, device=dev),
                                   torch.empty(t, top_k, dtype=torch.int32, device=dev))
     # few pairs whose choice is there: the experts' launches find their rows themselves (moe_top.h), no launch for counts and slots
