@@ -583,11 +583,13 @@ def _wide_plan(m: int, n: int, k: int, swiglu: bool, splits: int, variant: int, 
 
 def duo_fits(m: int, n: int, k: int, s: int, bm: int, swiglu: bool = False) -> bool:
     """Does gemm_duo serve an [m, k] x [n, k]^T product in ``s`` K slices on row tiles of ``bm`` (gemm_wide's plan, whose bits it has)?  GLUs from 65
-    rows on, slabs from 129 (up to 128 rows they are equal: 4096 x 14336 with its norm 29.8 / 29.8 us, 6144 x 4096 16.6 / 16.6), where
+    rows on, slabs from 129, or 65 where a slice is 32 K-tiles and more (us with the norm behind them, gemm_wide / this at 65 and 128 rows: 8192 x 28672
+    in slices of 112 93.1 / 87.9 and 103.7 / 100.6, 10240 x 8192 of 43 40.7 / 40.2 and 46.2 / 44.5, 8192 x 8192 of 32 39.4 / 39.7 and 42.4 / 42.2,
+    4096 x 14336 of 28 29.1 / 28.0 and 33.0 / 32.8, 6144 x 4096 of 13 17.5 / 18.1 and 19.9 / 21.0, 2560 x 7680 of 10 22.8 / 24.1 at 128), where
     the workgroups keep three quarters of the CUs busy: its four waves take twice as long over a K-tile as gemm_wide's eight where
     nothing else bounds them.  us, gemm_wide / this at 256 rows: 2048 x 2048 (64 workgroups) 12.0 / 14.1, 2560 x 2560 (100) 13.8 / 15.6,
     4096 x 2048 (128) 15.0 / 15.5, 8192 x 8192 (256) 45.4 / 43.6."""
-    rows = 64 < m <= 256 and s == 1 if swiglu else 128 < m <= 512 and s > 1
+    rows = 64 < m <= 256 and s == 1 if swiglu else (128 < m <= 512 or 64 < m <= 128 and k >= 2048 * s) and s > 1
     return (knobs.K.duo and rows and bm in (128, 192, 256) and n % 128 == 0 and k % 64 == 0 and n // 128 * s * -(-m // bm) >= 192
             and m * k * 2 < 1 << 32 and n * k * 2 < 1 << 32)
 

@@ -50,7 +50,7 @@ def test_swiglu_bits(cuda, bm, m, n, k):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,n,k,glu", [(96, 28672, 4096, True), (160, 28672, 4096, True), (200, 28672, 4096, True), (256, 28672, 4096, True),
-                                       (160, 4096, 4096, False), (256, 4096, 4096, False), (320, 4096, 4096, False), (512, 4096, 4096, False),
+                                       (65, 8192, 28672, False), (128, 10240, 8192, False), (160, 4096, 4096, False), (256, 4096, 4096, False), (320, 4096, 4096, False), (512, 4096, 4096, False),
                                        (200, 6144, 4096, False), (256, 4096, 14336, False), (384, 4096, 14336, False)])
 def test_reached_by_the_products(cuda, m, n, k, glu, monkeypatch):
     """The calls that are meant to take this kernel take it, and give what gemm_wide gives."""
@@ -104,6 +104,7 @@ def test_rule():
     assert f(128, 28672, 4096, 1, 128, True) and f(256, 28672, 4096, 1, 256, True) and not f(64, 28672, 4096, 1, 64, True)
     assert not f(256, 16384, 4096, 1, 256, True) and not f(300, 28672, 4096, 1, 192, True)
     assert f(256, 4096, 14336, 8, 256) and f(129, 4096, 4096, 4, 128) and not f(128, 4096, 14336, 8, 128)
+    assert f(128, 8192, 28672, 4, 128) and f(65, 8192, 8192, 4, 128) and not f(64, 8192, 28672, 4, 128) and not f(96, 6144, 4096, 5, 128)
     assert not f(256, 2048, 2048, 4, 256) and not f(256, 65536, 4096, 1, 256)
     with knobs.override(duo=False):
         assert not f(256, 4096, 14336, 8, 256)
