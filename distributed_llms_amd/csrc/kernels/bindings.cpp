@@ -26,7 +26,8 @@ PYBIND11_MODULE(_C_kernels, m) {
   m.def("splitk_reduce_clipped", &dllm::splitk_reduce_clipped);
   m.def("splitk_reduce_gelu", &dllm::splitk_reduce_gelu);
   m.def("gemm_one", &dllm::gemm_one);
-  m.def("gemm_duo", &dllm::gemm_duo);
+  m.def("gemm_duo", &dllm::gemm_duo, py::arg("c"), py::arg("a"), py::arg("b"), py::arg("ws"), py::arg("ws_floats"), py::arg("m"), py::arg("n"),
+        py::arg("k"), py::arg("splits"), py::arg("glu"), py::arg("bm"), py::arg("stream"), py::arg("like_pp") = false);
   m.def("gemm_wide", &dllm::gemm_wide);
   m.def("gemm_wide_fp8", &dllm::gemm_wide_fp8);
   m.def("quant_fp8_rows", &dllm::quant_fp8_rows);

@@ -7,8 +7,8 @@
 // stage, took 62-69 us for it: a wave that waits for room to issue a load issues no products either, and loads strewn among
 // products come as activations and weights in turn, which alone makes the staging 56 us instead of 50.  Here the waves that stage
 // issue a K-tile's activations, then its weights, as soon as a slot is free, and those that multiply wait for nothing but
-// the K-tile's one barrier: 57-62 us.  us, gemm_wide (or gemm_pp) / this, slabs with the sum and norm behind them:
-//   28672 x 4096, SwiGLU   M = 96 / 128 / 192 / 256   46.3 / 46.8 / 53.6 / 61.9 -> 44.5 / 45.8 / 52.8 / 57.5
+// the K-tile's one barrier: 57-62 us.  us, gemm_wide / this, slabs with the sum and norm behind them:
+//   28672 x 4096, SwiGLU   M = 96 / 128 / 192         46.3 / 46.8 / 53.6 -> 44.5 / 45.8 / 52.8
 //   4096 x 14336           192 / 256                  35.3 / 40.1 -> 34.4 / 38.6
 //   4096 x 4096            160 / 256 / 300 / 512      16.0 / 18.4 / 31.9 / 28.5 -> 15.1 / 17.6 / 23.6 / 27.4
 //   6144 x 4096            160 / 200 / 256            18.5 / 22.2 / 23.4 -> 18.2 / 19.7 / 21.5
@@ -24,7 +24,10 @@
 // kernel's end writes back otherwise (6144 x 4096 at 256 rows with its sum 22.6 -> 21.5, 4096 x 4096 18.0 -> 17.6), and leave
 // the weights in the caches' default policy; in longer ones the stores are a smaller part and nontemporal weights gain more (4096 x 14336
 // 41.4 -> 38.6).
-// The sums have gemm_wide's order: equal bits.
+// The sums have gemm_wide's order: equal bits.  A SwiGLU that gemm_pp would run (like_pp) has that kernel's instead: K from its start on every
+// XCD, gate and up rounded to bf16 in front of the SiLU.  us, gemm_pp / this / with gemm_wide's bits, 200 and 256 rows: 28672 x 4096
+// 60.9 / 58.2 / 58.1 and 62.1 / 60.6 / 59.5, 32768 x 4096 71.3 / 65.6 / 58.6 and 68.7 / 66.6 / 61.8, 28672 x 3072 52.9 / 51.6 / 51.7 and 49.4 / 48.1 / 48.6,
+// 27648 x 5120 74.5 / 72.0 / 72.8 and 77.8 / 76.3 / 76.9.
 //
 // An XCD has the column tiles of a slice next to each other: its L2 then holds one slice of the activations, where the slices of a column tile
 // beside each other had every XCD fetch all of them (7 MiB of 4096 x 14336 at 256 rows, eight times, beside 112 MiB of weights).  With the sum
@@ -38,7 +41,7 @@ namespace dllm {
 // Row tile 32 RT.  GLU: SwiGLU C [M, N / 2] of B = [gate; up] in alternating 16-row groups (pp_b_row), else slabs P [S, M, N].  LONG: long slices.
 template <int RT, bool GLU, bool LONG>
 __global__ void __launch_bounds__(512, 1) gemm_duo_kernel(const bf16* __restrict__ B, const bf16* __restrict__ A, int M, int N, int K,
-                                                          int kts, int nsplit, bf16* __restrict__ C, float* __restrict__ P) {
+                                                          int kts, int nsplit, bool like_pp, bf16* __restrict__ C, float* __restrict__ P) {
   constexpr int BM = 32 * RT, BN = 128, CT = 4, TM = 16 * RT, TN = 64, NB = 3;   // waves that multiply: 2 x 2 of TM x TN
   constexpr int SLOT = (BM + BN) * PBK;
   constexpr int GA = BM / 32, GB = BN / 32, G = GA + GB;       // pieces of 8 rows per staging wave and K-tile
@@ -57,7 +60,7 @@ __global__ void __launch_bounds__(512, 1) gemm_duo_kernel(const bf16* __restrict
   if (wv >= 4) {
     const int lw = wv - 4;
     // (unsplit: K from another place on each XCD, gemm_wide's rotation)
-    const int rot = nsplit == 1 && mtiles == 1 && nt >= 16 ? ((int)(blockIdx.x & 7) * nt) >> 3 : 0;
+    const int rot = !like_pp && nsplit == 1 && mtiles == 1 && nt >= 16 ? ((int)(blockIdx.x & 7) * nt) >> 3 : 0;
     uint32_t off[G];
 #pragma unroll
     for (int j = 0; j < G; ++j) {
@@ -181,7 +184,11 @@ __global__ void __launch_bounds__(512, 1) gemm_duo_kernel(const bf16* __restrict
       if constexpr (GLU) {
         bf16x4 h;
 #pragma unroll
-        for (int v = 0; v < 4; ++v) h[v] = f2bf(silu_f(acc[r][2 * i][v]) * acc[r][2 * i + 1][v]);
+        for (int v = 0; v < 4; ++v) {
+          float g = acc[r][2 * i][v], u = acc[r][2 * i + 1][v];
+          if (like_pp) g = bf2f(f2bf(g)), u = bf2f(f2bf(u));
+          h[v] = f2bf(silu_f(g) * u);
+        }
         q[i] = __builtin_bit_cast(u32x2, h);
       } else {
         f16x4 h;
@@ -211,9 +218,9 @@ __global__ void __launch_bounds__(512, 1) gemm_duo_kernel(const bf16* __restrict
 }
 
 // glu: SwiGLU c [m, n / 2] of b = [gate; up], unsplit; else slabs [S, m, n] of `splits` K slices in ws (S > 1).  bm: row tile 128, 192 or 256.
-// Returns the number of slices S.
+// like_pp: a SwiGLU with gemm_pp's bits, else with gemm_wide's.  Returns the number of slices S.
 int gemm_duo(uintptr_t c, uintptr_t a, uintptr_t b, uintptr_t ws, long ws_floats, int M, int N, int K, int splits, bool glu, int bm,
-             uintptr_t stream) {
+             uintptr_t stream, bool like_pp) {
   DLLM_HOST_CHECK(M >= 1 && N > 0 && N % 128 == 0 && K % PBK == 0 && K >= PBK && splits >= 1, "N a multiple of 128, K of 64");
   DLLM_HOST_CHECK((long)M * K * 2 < (1L << 32) && (long)N * K * 2 < (1L << 32), "operands must be < 4 GiB");
   DLLM_HOST_CHECK(bm == 128 || bm == 192 || bm == 256, "row tile 128, 192 or 256");
@@ -225,7 +232,7 @@ int gemm_duo(uintptr_t c, uintptr_t a, uintptr_t b, uintptr_t ws, long ws_floats
   DLLM_HOST_CHECK(grid < (1L << 31), "grid");
   auto go = [&](auto kern) {
     hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(512), 0, reinterpret_cast<hipStream_t>(stream), (const bf16*)b, (const bf16*)a, M,
-                       N, K, kts, S, (bf16*)c, (float*)ws);
+                       N, K, kts, S, like_pp, (bf16*)c, (float*)ws);
   };
 #define DLLM_DUO(RT_)                                     \
   do {                                                    \

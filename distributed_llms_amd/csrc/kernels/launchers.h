@@ -32,7 +32,7 @@ void splitk_reduce_gelu(uintptr_t out, uintptr_t ws, int S, int M, int N, uintpt
 int gemm_one(uintptr_t c, uintptr_t slabs, uintptr_t b, int n, int k, int splits, int mode, int nt, uintptr_t x, uintptr_t res,
              uintptr_t part, int nslabs, uintptr_t w, uintptr_t res_out, float eps, uintptr_t stream);
 int gemm_duo(uintptr_t c, uintptr_t a, uintptr_t b, uintptr_t ws, long ws_floats, int M, int N, int K, int splits, bool glu, int bm,
-             uintptr_t stream);
+             uintptr_t stream, bool like_pp);
 int gemm_wide(uintptr_t c, uintptr_t a, uintptr_t b, uintptr_t ws, long ws_floats, int M, int N, int K, int splits,
               int mode, int variant, uintptr_t stream);
 int gemm_wide_fp8(uintptr_t c, uintptr_t a, uintptr_t a_scale, uintptr_t b, uintptr_t b_scale, uintptr_t ws,

@@ -609,12 +609,14 @@ def duo_row_tile(m: int, n: int, k: int, s: int, bm: int, swiglu: bool = False) 
     return (one or fits or [0])[0]
 
 
-def _duo(x: torch.Tensor, w: torch.Tensor, m: int, n: int, k: int, s: int, bm: int, swiglu: bool, defer: bool):
-    """gemm_duo's launch: the SwiGLU, or the slabs' :class:`SplitKPartial` (summed without ``defer``)."""
+def _duo(x: torch.Tensor, w: torch.Tensor, m: int, n: int, k: int, s: int, bm: int, swiglu: bool, defer: bool,
+         like_pp: bool = False):
+    """gemm_duo's launch: the SwiGLU (gemm_wide's bits, ``like_pp``: gemm_pp's), or the slabs' :class:`SplitKPartial` (summed without
+    ``defer``)."""
     ws = _workspace(x.device)
     y = torch.empty(*x.shape[:-1], n // 2, dtype=x.dtype, device=x.device) if swiglu else None
     se = _ext.kernels().gemm_duo(y.data_ptr() if swiglu else 0, x.data_ptr(), w.data_ptr(), ws.data_ptr(), ws.numel(), m, n, k, s,
-                                 swiglu, bm, current_stream())
+                                 swiglu, bm, current_stream(), like_pp)
     if swiglu:
         return y
     part = SplitKPartial(ws, se, m, n, (*x.shape[:-1], n), x.dtype, x.device)
@@ -707,7 +709,7 @@ def linear_pp(x: torch.Tensor, w: torch.Tensor, splits: int = 0, swiglu: bool = 
         s = max(1, ws.numel() // (m * n))
     if swiglu and variant == PP_GATE_UP_VARIANT and s == 1 and duo_fits(m, n, k, s, wide_bm(m), True) and x.data_ptr() % 16 == 0 \
             and w.data_ptr() % 16 == 0:
-        return _duo(x, w, m, n, k, s, wide_bm(m), True, False)
+        return _duo(x, w, m, n, k, s, wide_bm(m), True, False, True)
     stream = current_stream()
     if defer and not swiglu and s > 1:
         se = _ext.kernels().gemm_pp(0, x.data_ptr(), w.data_ptr(), ws.data_ptr(), ws.numel(), m, n, k, s, 2, variant,
@@ -870,7 +872,7 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor) -> Optional[torch.Te
         return _stream(m, n, k, x, w_gate_up, glu="silu")
     if 0 < kn.pp_gate_up_min_m <= m <= 256 and not _comm_cus and _use_pp(m, n, k, x, w_gate_up, 1):
         # decode gate|up on gemm_pp, unsplit, weights nontemporal, on the column tile that gives one
-        # round of CUs / 2 .. CUs tiles: 8B (224 x 128 columns) 62.1 vs 64.1 us for gemm_wide (57.5 on gemm_duo, which
+        # round of CUs / 2 .. CUs tiles: 8B (224 x 128 columns) 62.1 vs 64.1 us for gemm_wide (60.6 on gemm_duo with its bits, which
         # linear_pp takes for these), 70B (224 x 256 columns) 204 vs 259 us for gemm_sq (bench/debug/medium_m_sweep.py --pp)
         cus = _cus(x.device)
         if n % 128 == 0 and cus // 2 <= n // 128 <= cus:

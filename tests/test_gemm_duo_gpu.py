@@ -48,19 +48,33 @@ def test_swiglu_bits(cuda, bm, m, n, k):
     assert (y.double() - ref).norm() <= 2.0 ** -8 * ref.norm()                  # (one rounding to bf16 and f32 sums)
 
 
+# one row tile's edges in each of the three; K-tiles fewer than the ring holds and more than gemm_wide's rotation needs
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [1, 65, 128, 129, 192, 193, 255, 256])
+@pytest.mark.parametrize("n,k", [(256, 64), (512, 192), (384, 1088), (24576, 4096)])
+def test_swiglu_bits_of_gemm_pp(cuda, m, n, k):
+    """In gemm_pp's place: its sums from K's start, its gate and up rounded to bf16 in front of the SiLU."""
+    x, w = _xw(m, n, k)
+    want = torch.empty(m, n // 2, device="cuda", dtype=torch.bfloat16)
+    _ext.kernels().gemm_pp(want.data_ptr(), x.data_ptr(), w.data_ptr(), 0, 0, m, n, k, 1, 1, gemm.PP_GATE_UP_VARIANT,
+                           torch.cuda.current_stream().cuda_stream)
+    assert torch.equal(gemm._duo(x, w, m, n, k, 1, 128 if m <= 128 else 192 if m <= 192 else 256, True, False, like_pp=True), want)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,n,k,glu", [(96, 28672, 4096, True), (160, 28672, 4096, True), (200, 28672, 4096, True), (256, 28672, 4096, True),
                                        (65, 8192, 28672, False), (128, 10240, 8192, False), (160, 4096, 4096, False), (256, 4096, 4096, False), (320, 4096, 4096, False), (512, 4096, 4096, False),
                                        (200, 6144, 4096, False), (256, 4096, 14336, False), (384, 4096, 14336, False)])
 def test_reached_by_the_products(cuda, m, n, k, glu, monkeypatch):
-    """The calls that are meant to take this kernel take it, and give what gemm_wide gives."""
+    """The calls that are meant to take this kernel take it, and give what the kernel gives that they would take (gemm_wide; a SwiGLU of 200
+    rows and more gemm_pp)."""
     x, w = _xw(m, n, k)
     calls, duo = [], gemm._duo
     monkeypatch.setattr(gemm, "_duo", lambda *a: calls.append(1) or duo(*a))
     go = (lambda: ops.linear_swiglu(x, w)) if glu else (lambda: ops.linear(x, w))
     y = go()
     assert calls
-    with knobs.override(duo=False, pp_gate_up_min_m=0):
+    with knobs.override(duo=False):
         assert torch.equal(y, go())
 
 
