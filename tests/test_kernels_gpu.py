@@ -275,6 +275,43 @@ def test_decode_reads_no_key_behind_the_last(cuda, hq, hkv, d, most):
         assert torch.equal(x, y)
 
 
+@pytest.mark.parametrize("hq,hkv,d", [(32, 8, 128), (12, 12, 64), (4, 1, 128)])
+@pytest.mark.parametrize("left", [float("inf"), float("nan")])
+def test_decode_overwrites_what_its_slot_held(cuda, hq, hkv, d, left):
+    """The slot of the new key may hold anything, and so may its block behind it: K rows of all later keys, V^T tiles of the later groups of eight."""
+    lens = list(range(1, 67))
+    k, v, bt = _fill_paged(lens, hkv, d)
+    b, sl = len(lens), torch.tensor(lens, dtype=torch.int32, device="cuda")
+    qkv, scale = _bf(b, (hq + 2 * hkv) * d), 1 / math.sqrt(d)
+    slots = torch.stack([bt[i, (n - 1) // 32] * 32 + (n - 1) % 32 for i, n in enumerate(lens)]).to(torch.int32)
+    cs = ref.rope_cos_sin(d, 4096, 500000.0, device="cuda")
+    outs = []
+    for fill in (0.0, left):
+        k1, v1 = k.clone(), v.clone()
+        for i, n in enumerate(lens):
+            blk, at = bt[i, (n - 1) // 32].item(), (n - 1) % 32
+            tiles = v1[blk].view(hkv, 4, d, 8)
+            tiles[:, at // 8, :, at % 8] = fill
+            tiles[:, at // 8 + 1:] = fill
+            for j in range(at, 32):
+                k1[blk, :, ((j & 4) << 2) + ((j >> 3) << 2) + (j & 3)] = fill
+        outs.append(ops.paged_attention_decode_rope(qkv, sl - 1, cs, k1, v1, slots, bt, sl, hq, hkv, d, scale))
+    assert torch.equal(*outs) and bool(torch.isfinite(outs[0]).all())
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(32, 8, 128), (12, 12, 64)])
+@pytest.mark.parametrize("at", [0, 5, 31])
+def test_decode_of_infinite_values(cuda, hq, hkv, d, at):
+    """A value that is infinite makes its channel infinite, and not NaN through lanes of keys behind the last one."""
+    lens = list(range(at + 1, 67))
+    k, v, bt = _fill_paged(lens, hkv, d)
+    b, sl = len(lens), torch.tensor(lens, dtype=torch.int32, device="cuda")
+    for i in range(b):
+        v[bt[i, 0].item()].view(hkv, 4, d, 8)[:, at // 8, 3, at % 8] = float("inf")
+    got = ops.paged_attention_decode(_bf(b, hq, d), k, v, bt, sl, 1 / math.sqrt(d))
+    assert bool((got[..., 3] == float("inf")).all()) and bool(torch.isfinite(got[..., :3]).all()) and bool(torch.isfinite(got[..., 4:]).all())
+
+
 @pytest.mark.parametrize("version", ["3", "4", "6", "7", "9"])
 @pytest.mark.parametrize("hq,hkv,d", [(32, 8, 128), (64, 8, 128), (12, 12, 64), (8, 4, 64), (16, 16, 128),
                                       (32, 2, 128)])
