@@ -397,9 +397,11 @@ def _decode_rope(qkv, positions, cos_sin, k_cache, v_cache, slot_mapping, block_
 
 def _o_by_heads(hq: int, hkv: int, d: int, n: int) -> bool:
     """Can the o-projection's K slices be the kv heads' (csrc/kernels/attention.hip, attn_o_kernel and join_o_kernel)?  Slices of at most 512 inputs,
-    whose weights fill the LDS, and one round of workgroups that keeps three quarters of the CUs busy."""
+    whose weights fill the LDS, one round of workgroups that keeps three quarters of the CUs busy, and as many slices as the projection has by itself
+    (of 512 inputs, so heads in groups of four): more slabs of 16 bits would cost precision (results around 0.01: 16 for 4 of 2048 inputs 4.4e-4
+    off for 2.6e-4, 8 for 2 of 1024 3.2e-4 for 2.3e-4), the same ones have the projection's bits."""
     return (knobs.K.one and d == 128 and hq % hkv == 0 and hq // hkv <= 4 and n % 128 == 0 and 192 <= n // 128 * hkv <= 256
-            and not gemm._comm_cus)
+            and not gemm._comm_cus and gemm.wide_splits(1, n, hq * d) == hkv)
 
 
 def attn_o_splits(batch: int, max_ctx: int, hq: int, hkv: int, d: int, n: int) -> int:
@@ -432,7 +434,7 @@ def paged_attention_decode_o(qkv, positions, cos_sin, k_cache, v_cache, slot_map
             or width != (hq + 2 * hkv) * d or (part is not None and len(part.shape) != 2):
         return None
     if not (wo.dim() == 2 and wo.shape[1] == hq * d and wo.dtype == torch.bfloat16 and wo.is_contiguous() and wo.data_ptr() % 16 == 0
-            and wo.device == k_cache.device):
+            and wo.device == k_cache.device and gemm._use_wide(b, n, hq * d, wo, wo)):
         return None
     ns = attn_o_splits(b, max_ctx, hq, hkv, d, n)
     ws = gemm.slab_space(k_cache.device, part)
