@@ -103,8 +103,11 @@ def forward(x: torch.Tensor, w_router: torch.Tensor, w_gate_up: torch.Tensor, w_
     fp8 = isinstance(w_gate_up, quant.Fp8Experts)
     if fp8 != isinstance(w_down, quant.Fp8Experts):
         raise TypeError("moe: gate|up and down experts must both be fp8 or both not")
+    if choice and not all(c.shape == (x.shape[0], top_k) and c.dtype == d and c.is_contiguous() and c.device == x.device
+                          for c, d in zip(choice, (torch.float32, torch.int32))):
+        raise ValueError("moe: choice is ([T, top_k] float32 weights, [T, top_k] int32 experts)")
     if not x.is_cuda:
-        tw, tid = ref.moe_route(ref.linear(x, w_router), top_k)
+        tw, tid = choice or ref.moe_route(ref.linear(x, w_router), top_k)
         if fp8:
             return quant.moe_mlp_ref(x, w_gate_up, w_down, tw, tid - expert_offset)
         return ref.moe_mlp(x, w_gate_up, w_down, tw, tid - expert_offset)
@@ -119,9 +122,6 @@ def forward(x: torch.Tensor, w_router: torch.Tensor, w_gate_up: torch.Tensor, w_
     if not (x.is_contiguous() and w_gate_up.is_contiguous() and w_down.is_contiguous()):
         raise ValueError("moe: operands must be contiguous")
     dev = x.device
-    if choice and not all(c.shape == (t, top_k) and c.dtype == d and c.is_contiguous() and c.device == dev
-                          for c, d in zip(choice, (torch.float32, torch.int32))):
-        raise ValueError("moe: choice is ([T, top_k] float32 weights, [T, top_k] int32 experts)")
     topk_w, topk_ids = choice or (torch.empty(t, top_k, dtype=torch.float32, device=dev),
                                   torch.empty(t, top_k, dtype=torch.int32, device=dev))
     # few pairs whose choice is there: the experts' launches find their rows themselves (moe_top.h), no launch for counts and slots

@@ -1,0 +1,32 @@
+"""A mixture whose choice of experts is given (ops.moe.forward's ``choice``)."""
+import pytest
+import torch
+
+from distributed_llms_amd.ops import moe, quant
+from distributed_llms_amd.ops import reference as ref
+
+
+def _case(t, top, h=128, i=128, device="cpu", dtype=torch.bfloat16):
+    g = torch.Generator().manual_seed(t + top)
+    r = lambda *s, scale=1.0: (torch.randn(*s, generator=g) * scale).to(dtype).to(device)     # noqa: E731
+    ids = torch.stack([torch.randperm(8, generator=g)[:top] for _ in range(t)]).to(torch.int32).to(device)
+    return r(t, h), r(8, h, scale=0.1), r(8, 2 * i, h, scale=0.05), r(8, h, i, scale=0.05), torch.rand(t, top, generator=g).to(device), ids
+
+
+@pytest.mark.parametrize("t,top", [(1, 1), (3, 2), (40, 2)])
+def test_taken_on_the_cpu(t, top):
+    x, wr, gu, dn, tw, ids = _case(t, top)
+    want = ref.moe_mlp(x, gu, dn, tw, ids)
+    assert torch.equal(moe.forward(x, wr, gu, dn, top, choice=(tw, ids)), want)
+    assert not torch.equal(moe.forward(x, wr, gu, dn, top), want)
+    half = moe.forward(x, wr, gu[4:], dn[4:], top, 4, choice=(tw, ids))
+    assert torch.equal(half, ref.moe_mlp(x, gu[4:], dn[4:], tw, ids - 4))
+    q = quant.quantize_experts(gu), quant.quantize_experts(dn)
+    assert torch.equal(moe.forward(x, wr, *q, top, choice=(tw, ids)), quant.moe_mlp_ref(x, *q, tw, ids))
+
+
+def test_forms_refused():
+    x, wr, gu, dn, tw, ids = _case(3, 2)
+    for choice in ((tw[:2], ids), (tw, ids.long()), (tw.bfloat16(), ids), (tw[:, :1], ids[:, :1]), (tw.T.contiguous().T, ids)):
+        with pytest.raises(ValueError, match="choice"):
+            moe.forward(x, wr, gu, dn, 2, choice=choice)
