@@ -122,6 +122,8 @@ def forward(x: torch.Tensor, w_router: torch.Tensor, w_gate_up: torch.Tensor, w_
     if not (x.is_contiguous() and w_gate_up.is_contiguous() and w_down.is_contiguous()):
         raise ValueError("moe: operands must be contiguous")
     dev = x.device
+    if choice and x.dtype != torch.bfloat16:
+        raise ValueError("moe: a given choice is for bf16 activations")
     topk_w, topk_ids = choice or (torch.empty(t, top_k, dtype=torch.float32, device=dev),
                                   torch.empty(t, top_k, dtype=torch.int32, device=dev))
     # few pairs whose choice is there: the experts' launches find their rows themselves (moe_top.h), no launch for counts and slots

@@ -30,3 +30,13 @@ def test_forms_refused():
     for choice in ((tw[:2], ids), (tw, ids.long()), (tw.bfloat16(), ids), (tw[:, :1], ids[:, :1]), (tw.T.contiguous().T, ids)):
         with pytest.raises(ValueError, match="choice"):
             moe.forward(x, wr, gu, dn, 2, choice=choice)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("t", [1, 40])
+def test_other_activations_refused(cuda, dtype, t):
+    """The launches behind a choice are bf16 ones; nothing is launched for other activations."""
+    x, wr, gu, dn, tw, ids = _case(t, 2, device="cuda", dtype=dtype)
+    with pytest.raises(ValueError, match="bf16"):
+        moe.forward(x, wr, gu, dn, 2, choice=(tw, ids))
