@@ -473,7 +473,7 @@ void moe_grouped_gemm(uintptr_t y, uintptr_t x, uintptr_t gather, uintptr_t w, u
 void moe_combine(uintptr_t out, uintptr_t ysorted, uintptr_t topk_w, uintptr_t inv, int T, int H, int k,
                  uintptr_t stream, uintptr_t ids) {
   DLLM_HOST_CHECK(H % 8 == 0, "H % 8");
-  DLLM_HOST_CHECK(ids == 0 || (long)T * k <= kPickPairs, "the choices of up to 64 pairs");
+  DLLM_HOST_CHECK((inv != 0 || ids != 0) && (ids == 0 || (long)T * k <= kPickPairs), "slots, or the choices of up to 64 pairs");
   if (T == 0) return;
   hipLaunchKernelGGL(moe_combine_kernel, dim3(T), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), (bf16*)out,
                      (const bf16*)ysorted, (const float*)topk_w, (const int*)inv, (const int*)ids, H, k);

@@ -2,6 +2,7 @@
 import pytest
 import torch
 
+from distributed_llms_amd import _ext
 from distributed_llms_amd.ops import moe, quant
 from distributed_llms_amd.ops import reference as ref
 
@@ -40,3 +41,15 @@ def test_other_activations_refused(cuda, dtype, t):
     x, wr, gu, dn, tw, ids = _case(t, 2, device="cuda", dtype=dtype)
     with pytest.raises(ValueError, match="bf16"):
         moe.forward(x, wr, gu, dn, 2, choice=(tw, ids))
+
+
+@pytest.mark.parametrize("call", ["combine", "combine_norm"])
+def test_combine_needs_slots_or_choices(call):
+    """Neither slots nor choices, or choices of more pairs than a wave has lanes: an error in front of the launch."""
+    k = _ext.kernels()
+    for inv, ids, t in ((0, 0, 4), (0, 64, 33)):
+        with pytest.raises(RuntimeError, match="pairs"):
+            if call == "combine":
+                k.moe_combine(64, 64, 64, inv, t, 64, 2, 0, ids)
+            else:
+                k.moe_combine_norm(64, 64, 64, 64, inv, ids, 64, t, 64, 2, 1e-5, 0)
