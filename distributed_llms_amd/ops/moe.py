@@ -124,6 +124,8 @@ def forward(x: torch.Tensor, w_router: torch.Tensor, w_gate_up: torch.Tensor, w_
     dev = x.device
     if choice and x.dtype != torch.bfloat16:
         raise ValueError("moe: a given choice is for bf16 activations")
+    if t == 0:
+        return torch.empty_like(x)       # (no choice, no counts: nothing that the experts' launches could read)
     topk_w, topk_ids = choice or (torch.empty(t, top_k, dtype=torch.float32, device=dev),
                                   torch.empty(t, top_k, dtype=torch.int32, device=dev))
     # few pairs whose choice is there: the experts' launches find their rows themselves (moe_top.h), no launch for counts and slots

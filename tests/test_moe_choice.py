@@ -53,3 +53,12 @@ def test_combine_needs_slots_or_choices(call):
                 k.moe_combine(64, 64, 64, inv, t, 64, 2, 0, ids)
             else:
                 k.moe_combine_norm(64, 64, 64, 64, inv, ids, 64, t, 64, 2, 1e-5, 0)
+
+
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("given", [False, True])
+def test_no_tokens(device, given):
+    x, wr, gu, dn, tw, ids = _case(1, 2, device=device)
+    for defer in (False, True):
+        out = moe.forward(x[:0], wr, gu, dn, 2, choice=(tw[:0], ids[:0]) if given else None, defer=defer)
+        assert out.shape == (0, 128) and out.dtype == x.dtype
