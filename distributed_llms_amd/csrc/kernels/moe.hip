@@ -14,6 +14,8 @@
 #include "stream_common.h"
 #include "moe_top.h"
 
+#include <algorithm>
+
 namespace dllm {
 
 constexpr int kMaxExperts = 64;
@@ -441,10 +443,12 @@ void moe_grouped_gemm(uintptr_t y, uintptr_t x, uintptr_t gather, uintptr_t w, u
       hipLaunchKernelGGL(kern, dim3(N / bn, E), dim3(threads), 0, s, (bf16*)y, (const bf16*)x, (const int*)gather, (const bf16*)w,
                          (const int*)counts, (const int*)nullptr, N, K, ldy, 0.f, pairs, top, e0);
     };
-    // variant 5's tile; one or two pairs of a product of few columns in tiles of 32, with K over eight waves, so that two experts' tiles are a
-    // workgroup per CU: 4096 x 14336 of two experts 79.5 -> 48.2 us (of three 85.0, here 92.3)
+    // variant 5's tile; one or two pairs of a product of few columns in tiles of 32, with K over eight waves, as long as their tiles are one round
+    // of the CUs.  us, tiles of 64 / of 32, 4096 and 14336 inputs, of two experts: 4096 columns 27.4 / 20.2 and 84.6 / 54.7, 6144 31.0 / 32.2 and 95.8 /
+    // 95.5, 8192 32.5 / 37.9 and 97.5 / 109.1; of one: 8192 29.2 / 23.1 and 84.4 / 58.9, 12288 32.7 / 35.4 and 96.2 / 98.1, 16384 32.3 / 38.5 and
+    // 98.1 / 108.4 (of three, 4096 x 14336, 85.0 / 92.3)
     if (mode == 1) go(moe_grouped_kernel<4, 4, 4, MOE_EPI_SWIGLU, true>, 64, 256, N / 2);
-    else if (pairs <= 2) go(moe_grouped_kernel<1, 2, 8, MOE_EPI_STORE, true>, 32, 512, N);
+    else if (pairs <= 2 && N / 32 * std::min(pairs, E) <= 256) go(moe_grouped_kernel<1, 2, 8, MOE_EPI_STORE, true>, 32, 512, N);
     else go(moe_grouped_kernel<4, 4, 4, MOE_EPI_STORE, true>, 64, 256, N);
     DLLM_HIP_CHECK(hipGetLastError());
     return;

@@ -137,7 +137,7 @@ def forward(x: torch.Tensor, w_router: torch.Tensor, w_gate_up: torch.Tensor, w_
         act = torch.empty(t * top_k, inter, dtype=x.dtype, device=dev)
         ids, pick = topk_ids.data_ptr(), (0.0, t * top_k, top_k, expert_offset)
         # Fewer pairs than the line take the tiled kernel all the same where its workgroups of gate|up are a round of the CUs, and one or two the other
-        # one for the down projection, whose tiles of 32 columns are.  us, gate|up / down of 8 experts of 4096 and 14336, two a token, tiled / other
+        # one for the down projection, whose tiles of 32 columns are (moe.hip).  us, gate|up / down of 8 experts of 4096 and 14336, two a token, tiled / other
         # kernel: one token 76 / 83, 98 / 48; two with three experts 111 / 86, 144 / 85; three with four 147 / 91, 174 / 90, with six 223 / 108,
         # 264 / 164.
         wide = wide or (0 < knobs.K.moe_wide_min_pairs and two_i % 128 == 0 and h % 128 == 0 and inter % 128 == 0

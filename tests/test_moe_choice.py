@@ -62,3 +62,18 @@ def test_no_tokens(device, given):
     for defer in (False, True):
         out = moe.forward(x[:0], wr, gu, dn, 2, choice=(tw[:0], ids[:0]) if given else None, defer=defer)
         assert out.shape == (0, 128) and out.dtype == x.dtype
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("t,top,h", [(1, 1, 8320), (1, 2, 4224), (2, 1, 8192)])
+def test_wide_down_projections_of_few_pairs(cuda, t, top, h):
+    """One or two pairs whose tiles of 32 columns are more than a round of the CUs keep the launches behind a slot list."""
+    x, wr, gu, dn, tw, ids = _case(t, top, h=h, i=1024, device="cuda")
+    if t == 2:
+        ids[:, 0] = torch.tensor([5, 2], dtype=torch.int32)
+    out = moe.forward(x, wr, gu, dn, top, choice=(tw, ids))
+    pairs, moe.PICK_PAIRS = moe.PICK_PAIRS, 0
+    try:
+        assert torch.equal(out, moe.forward(x, wr, gu, dn, top, choice=(tw, ids)))
+    finally:
+        moe.PICK_PAIRS = pairs
