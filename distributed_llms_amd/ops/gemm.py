@@ -690,11 +690,12 @@ def pp_splits(m: int, n: int, k: int, bn: int = 256, target_wgs: int = 256) -> i
 
 
 def linear_pp(x: torch.Tensor, w: torch.Tensor, splits: int = 0, swiglu: bool = False, defer: bool = False,
-              variant: int = 0):
+              variant: int = 0, duo: bool = False):
     """Ping-pong 256-row-tile GEMM (csrc/kernels/gemm_pp.hip).  ``variant``: bit 0 = 128-column tile
     (else 256), bit 1 = weights nontemporal, bit 2 = grouped row-tile order (large M).  Split-K
     partials are reduced by splitk_reduce(_swiglu), or returned as a :class:`SplitKPartial` with
-    ``defer`` (no SwiGLU)."""
+    ``defer`` (no SwiGLU).  ``duo``: an unsplit SwiGLU on 128-column tiles, weights nontemporal, on gemm_duo where that serves it
+    (:func:`duo_fits`), with the same bits."""
     k = x.shape[-1]
     n = w.shape[0]
     m = x.numel() // k
@@ -707,7 +708,7 @@ def linear_pp(x: torch.Tensor, w: torch.Tensor, splits: int = 0, swiglu: bool = 
     ws = _workspace(x.device)
     if s > 1 and s * m * n > ws.numel():
         s = max(1, ws.numel() // (m * n))
-    if swiglu and variant == PP_GATE_UP_VARIANT and s == 1 and duo_fits(m, n, k, s, wide_bm(m), True) and x.data_ptr() % 16 == 0 \
+    if duo and swiglu and variant == PP_GATE_UP_VARIANT and s == 1 and duo_fits(m, n, k, s, wide_bm(m), True) and x.data_ptr() % 16 == 0 \
             and w.data_ptr() % 16 == 0:
         return _duo(x, w, m, n, k, s, wide_bm(m), True, False, True)
     stream = current_stream()
@@ -873,10 +874,10 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor) -> Optional[torch.Te
     if 0 < kn.pp_gate_up_min_m <= m <= 256 and not _comm_cus and _use_pp(m, n, k, x, w_gate_up, 1):
         # decode gate|up on gemm_pp, unsplit, weights nontemporal, on the column tile that gives one
         # round of CUs / 2 .. CUs tiles: 8B (224 x 128 columns) 62.1 vs 64.1 us for gemm_wide (60.6 on gemm_duo with its bits, which
-        # linear_pp takes for these), 70B (224 x 256 columns) 204 vs 259 us for gemm_sq (bench/debug/medium_m_sweep.py --pp)
+        # takes these), 70B (224 x 256 columns) 204 vs 259 us for gemm_sq (bench/debug/medium_m_sweep.py --pp)
         cus = _cus(x.device)
         if n % 128 == 0 and cus // 2 <= n // 128 <= cus:
-            return linear_pp(x, w_gate_up, splits=1, swiglu=True, variant=PP_GATE_UP_VARIANT)
+            return linear_pp(x, w_gate_up, splits=1, swiglu=True, variant=PP_GATE_UP_VARIANT, duo=True)
         if n % 256 == 0 and cus // 2 <= n // 256 <= cus:
             return linear_pp(x, w_gate_up, splits=1, swiglu=True, variant=PP_GATE_UP_VARIANT & ~1)
     if _use_wide(m, n, k, x, w_gate_up, swiglu=True):

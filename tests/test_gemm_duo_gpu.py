@@ -79,6 +79,17 @@ def test_reached_by_the_products(cuda, m, n, k, glu, monkeypatch):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("variant", [gemm.PP_GATE_UP_VARIANT, 64 | 2, 64])
+def test_a_caller_that_asks_for_gemm_pp_gets_it(cuda, variant, monkeypatch):
+    x, w = _xw(256, 28672, 4096)
+    monkeypatch.setattr(gemm, "_duo", lambda *a: pytest.fail("gemm_duo"))
+    y = gemm.linear_pp(x, w, splits=1, swiglu=True, variant=variant)
+    z = x.double() @ w.double().T
+    want = F.silu(z[:, :14336]) * z[:, 14336:]
+    assert (y.double() - want).norm() <= 3 * 2.0 ** -9 * want.norm()            # (gate, up and the result rounded to bf16)
+
+
+@pytest.mark.gpu
 def test_replays_into_the_norm(cuda):
     """Slabs that are stored past the L2, and the launch that sums them, in a graph replayed between eager work."""
     m, n, k = 256, 4096, 4096
