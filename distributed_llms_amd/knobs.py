@@ -124,7 +124,10 @@ class Knobs:
     standin_channels: int = 4
     # ---- MoE (ops/moe.py)
     moe_variant: int = 0
-    moe_wide_min_pairs: int = 8       # token-expert pairs per expert from which the tiled GEMM serves
+    moe_wide_min_pairs: int = 8       # (token, expert) pairs of a step, all experts together, from which the tiled GEMM serves; 0: never
+    # fewer pairs than that on the tiled GEMM all the same where its gate|up workgroups are a round of the CUs, with a choice that the
+    # norm's launch has made (False, and a line behind the step's pairs: the grouped kernel)
+    moe_wide_fill: bool = True
     moe_fused_router: bool = True
     # prefill V append eight tokens per workgroup, 16-byte stores into the transposed V cache
     # (norm_elementwise.hip qkv_append_kernel); False = the per-token 2-byte scatter (not of a projection in split-K

@@ -140,7 +140,7 @@ def forward(x: torch.Tensor, w_router: torch.Tensor, w_gate_up: torch.Tensor, w_
         # one for the down projection, whose tiles of 32 columns are (moe.hip).  us, gate|up / down of 8 experts of 4096 and 14336, two a token, tiled / other
         # kernel: one token 76 / 83, 98 / 48; two with three experts 111 / 86, 144 / 85; three with four 147 / 91, 174 / 90, with six 223 / 108,
         # 264 / 164.
-        wide = wide or (0 < knobs.K.moe_wide_min_pairs and two_i % 128 == 0 and h % 128 == 0 and inter % 128 == 0
+        wide = wide or (knobs.K.moe_wide_fill and 0 < knobs.K.moe_wide_min_pairs and two_i % 128 == 0 and h % 128 == 0 and inter % 128 == 0
                         and two_i // 128 * min(t * top_k, e_loc) >= 256)
         if wide:
             k.moe_wide_gemm(act.data_ptr(), x.data_ptr(), ids, w_gate_up.data_ptr(), ids, 0, e_loc, two_i, h, 1, st, *pick)

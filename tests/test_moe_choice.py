@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from distributed_llms_amd import _ext
+from distributed_llms_amd import _ext, knobs
 from distributed_llms_amd.ops import moe, quant
 from distributed_llms_amd.ops import reference as ref
 
@@ -62,6 +62,36 @@ def test_no_tokens(device, given):
     for defer in (False, True):
         out = moe.forward(x[:0], wr, gu, dn, 2, choice=(tw[:0], ids[:0]) if given else None, defer=defer)
         assert out.shape == (0, 128) and out.dtype == x.dtype
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("t,top", [(1, 2), (3, 2), (8, 1)])
+def test_either_kernel_can_be_forced(cuda, t, top, monkeypatch):
+    """Which kernel serves the experts' products of few pairs: by the line, by the line alone, and by knobs that put it behind or in front of them."""
+    x, wr, gu, dn, tw, ids = _case(t, top, h=128, i=16384, device="cuda")
+
+    class Spy:
+        def __init__(self, k, calls):
+            self.k, self.calls = k, calls
+
+        def __getattr__(self, name):
+            f = getattr(self.k, name)
+            if name.startswith("moe_") and name.endswith("_gemm"):
+                return lambda *a: self.calls.append(name) or f(*a)
+            return f
+
+    k, calls = _ext.kernels(), []
+    monkeypatch.setattr(_ext, "kernels", lambda: Spy(k, calls))
+    want = None
+    for kn, first in (({}, "moe_wide_gemm"), ({"moe_wide_fill": False}, "moe_wide_gemm" if t * top >= 8 else "moe_grouped_gemm"),
+                      ({"moe_wide_fill": False, "moe_wide_min_pairs": 1000}, "moe_grouped_gemm"), ({"moe_wide_min_pairs": 0}, "moe_grouped_gemm"),
+                      ({"moe_wide_min_pairs": 1}, "moe_wide_gemm")):
+        calls.clear()
+        with knobs.override(**kn):
+            out = moe.forward(x, wr, gu, dn, top, choice=(tw, ids)).float()
+        assert calls[0] == first and len(calls) == 2
+        want = out if want is None else want
+        assert (out - want).norm() <= 2 * 2.0 ** -8 * want.norm()
 
 
 @pytest.mark.gpu
