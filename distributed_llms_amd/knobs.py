@@ -35,6 +35,8 @@ class Knobs:
     stream: bool = True
     # one row of a large weight, with the add + RMS norm in front of it, on gemm_one.hip (ops/gemm.one_fits)
     one: bool = True
+    # decode attention of few sequences, or the join of its splits, in the launch of the o-projection behind it (ops._o_by_heads)
+    attn_o: bool = True
     # 65 to 512 rows on gemm_duo.hip, waves that multiply beside waves that stage (ops/gemm.duo_fits)
     duo: bool = True
     # gemm_wide variant for unsplit grids (33: LDS-DMA interleaved + asm fragment reads with one

@@ -400,7 +400,7 @@ def _o_by_heads(hq: int, hkv: int, d: int, n: int) -> bool:
     whose weights fill the LDS, one round of workgroups that keeps three quarters of the CUs busy, and as many slices as the projection has by itself
     (of 512 inputs, so heads in groups of four): more slabs of 16 bits would cost precision (results around 0.01: 16 for 4 of 2048 inputs 4.4e-4
     off for 2.6e-4, 8 for 2 of 1024 3.2e-4 for 2.3e-4), the same ones have the projection's bits."""
-    return (knobs.K.one and d == 128 and hq % hkv == 0 and hq // hkv <= 4 and n % 128 == 0 and 192 <= n // 128 * hkv <= 256
+    return (knobs.K.attn_o and d == 128 and hq % hkv == 0 and hq // hkv <= 4 and n % 128 == 0 and 192 <= n // 128 * hkv <= 256
             and not gemm._comm_cus and gemm.wide_splits(1, n, hq * d) == hkv)
 
 

@@ -125,5 +125,7 @@ def test_rule():
         assert not f(1, 37, 32, 8, 128, 4096)
     finally:
         gemm.release_cus_for_comm()
-    with knobs.override(one=False):
+    with knobs.override(attn_o=False):
         assert not f(1, 37, 32, 8, 128, 4096)
+    with knobs.override(one=False):
+        assert f(1, 37, 32, 8, 128, 4096)
