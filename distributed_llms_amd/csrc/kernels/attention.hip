@@ -543,8 +543,9 @@ __global__ void __launch_bounds__(JOIN ? 512 : 64, 2) attn_decode_kernel(   // 2
 // that part of its input itself -- as the 31 other workgroups of the head do, out of the same XCD's L2 -- while its whole weight
 // slice is on its way into LDS.  Four waves attend, a (sequence, split of its keys) at a time, and four fetch the weights (loads
 // return in order: a wave that waits for keys would wait for its weights too), 0.9 us later, so that the first round trips of the
-// others are not behind 128 KiB (at once 11.3 us, 0.4 us later 10.5, now 10.2); all eight multiply.  The slices are left as split-K
-// slabs for the next norm.
+// others are not behind 128 KiB (at once 11.3 us, 0.4 us later 10.5, now 10.2); all eight multiply.  (Behind a barrier at the first keys' requests
+// in place of that time, with the norm, 37 / 150 / 256 / 400 keys 12.5 / 13.3 / 15.2 / 16.5 -> 12.6 / 13.4 / 15.8 / 16.9.)  The slices are left as
+// split-K slabs for the next norm.
 // us, attention and projection / this, 32 / 8 heads of 128, 4096 x 4096: one sequence of 37 / 69 / 150 / 256 / 400 / 500 keys 14.6 / 14.1 /
 // 14.0 / 14.7 / 14.3 / 14.9 -> 10.2 / 9.7 / 10.5 / 12.9 / 13.8 / 15.0, two of 30 / 60 / 120 / 200 15.2 / 15.8 / 15.6 / 14.9 -> 10.0 / 11.1 / 12.2 /
 // 14.6.  Every CU reads all keys and values of its head at some 16 KiB per 0.3 us, so that is where it ends: one of 1000 16.0 ->
